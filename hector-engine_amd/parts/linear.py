@@ -288,8 +288,8 @@ class Linear:
         constants of another gated activation ({alpha, limit, up_shift, cubic} as ops.silu_mul takes them)."""
         act = act or {}
         consts = (act.get("alpha", 1.0), act.get("limit", 0.0), act.get("up_shift", 0.0), act.get("cubic", 0.0))
-        act, a, scale, pieces = _operand(x)
-        if not self.gated_silu_rows(rows, ctx, act):
+        act_dtype, a, scale, pieces = _operand(x)
+        if not self.gated_silu_rows(rows, ctx, act_dtype):
             raise ValueError("Linear.gated_silu: not for these rows (ask gated_silu_rows)")
         if rows <= ops.BLOCKSPLIT_PIECES_MAX_M:
             ops.gemm_blocksplit(out, a, self.weight, None, rows, gated=True, row_scale=scale,
