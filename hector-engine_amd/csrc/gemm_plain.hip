@@ -7,15 +7,14 @@
 // The order: K is cut into segments of GP_SEG (128) consecutive k. The sum of a segment is one
 // chain of FMAs over its k in ascending order, begun at zero; the element is the segment
 // sums added one after the other in segment order, begun at zero; then the bias.
-// Three kernels keep this order and give the same bits:
-//   tiles   64 x 64 outputs a workgroup, staged through LDS, every thread 4 x 4 outputs
-//           (128 x 128 and 8 x 8 for fp32 steps of 128 rows or more);
-//   rows    for up to GP_ROWS_MAX_M rows (the one-token steps): a thread owns one weight
+// These kernels keep this order and give the same bits:
+//   mfma    fp32 operands, many rows: tiles of up to 128 x 128 outputs on the matrix cores;
+//   stream  fp32 operands, up to 64 rows, K in whole segments: matrix cores, a workgroup per 16 weight rows;
+//   tiles   bf16 operands: 64 x 64 outputs a workgroup, staged through LDS, every thread 4 x 4 outputs;
+//   rows    what the other two do not take of up to GP_ROWS_MAX_M rows: a thread owns one weight
 //           row and one segment and walks it with all M activation rows at once, so a product
 //           has N * ceil(K / GP_SEG) threads however few its rows are; the segment sums go
-//           to a workspace and a second kernel adds them in order. (With few rows the tile
-//           kernel is a grid of N / 64 workgroups walking all of K one after the other:
-//           the Qwen2.5-7B shape's one-token step took 190 ms with it.)
+//           to a workspace and a second kernel adds them in order.
 // No multiply and add of this file is fused unless it is written as an fma: the same lines are
 // compiled into several kernels that must give the same bits.
 #pragma clang fp contract(off)
@@ -49,31 +48,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = 0.f, total[i][j] = 0.f;
 
-  // a tile that lies inside both matrices is fetched four values a load
-  const bool a_vec = sizeof(TA) == 4 && m0 + GP_BM <= M && (lda & 3) == 0 && (((uintptr_t)A) & 15) == 0;
-  const bool w_vec = sizeof(TW) == 4 && n0 + GP_BN <= N && (ldw & 3) == 0 && (((uintptr_t)W) & 15) == 0;
   for (int k0 = 0; k0 < K; k0 += GP_BK) {
-    const bool whole = k0 + GP_BK <= K;
     const int am = m0 + lrow, wn = n0 + lrow;
-    if (a_vec && whole) {
-      const float4 v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(A) + am * lda + k0 + lk);
-      As[lk][lrow] = v.x, As[lk + 1][lrow] = v.y, As[lk + 2][lrow] = v.z, As[lk + 3][lrow] = v.w;
-    } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int k = k0 + lk + j;
-        As[lk + j][lrow] = (am < M && k < K) ? to_float(A[am * lda + k]) : 0.f;
-      }
-    }
-    if (w_vec && whole) {
-      const float4 v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(W) + wn * ldw + k0 + lk);
-      Ws[lk][lrow] = v.x, Ws[lk + 1][lrow] = v.y, Ws[lk + 2][lrow] = v.z, Ws[lk + 3][lrow] = v.w;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int k = k0 + lk + j;
-        Ws[lk + j][lrow] = (wn < N && k < K) ? to_float(W[wn * ldw + k]) : 0.f;
-      }
+    for (int j = 0; j < 4; ++j) {
+      const int k = k0 + lk + j;
+      As[lk + j][lrow] = (am < M && k < K) ? to_float(A[am * lda + k]) : 0.f;
+      Ws[lk + j][lrow] = (wn < N && k < K) ? to_float(W[wn * ldw + k]) : 0.f;
     }
     __syncthreads();
     // the chain of a segment holds its own k only: the last tile of K may be short
@@ -115,98 +96,256 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
   }
 }
 
-// The same product and order in tiles of 128 x 128 outputs, every thread 8 x 8 of them (two
-// groups of four rows by two groups of four columns, 64 apart, so that the operand reads from LDS
-// are whole 16-byte reads of neighbouring lanes): four times the products per LDS read of the
-// 64 x 64 kernel. For fp32 operands and steps of 128 rows or more (whole prompts).
-#define GPW_BM 128
-#define GPW_BN 128
-__global__ __launch_bounds__(256) void gemm_plain_wide_kernel(
+// The 32-bit product of more than GP_MROWS_MAX_M rows on the matrix cores, in the same order: a chain of
+// v_mfma_f32_32x32x2_f32 on one accumulator gives bit for bit the chain of FMAs over ascending k (measured
+// over normal, tiny, denormal, huge and non-finite operands), so a segment is 64 instructions begun at zero and
+// the segment sums are added as everywhere. A lane's operand for four instructions is one 16-byte LDS read: a row's
+// even k of a stage lie before its odd k (lanes 0..31 feed the even k of an instruction, lanes 32..63 the odd
+// one). Four wavefronts, two by two, each with BM/2 x BN/2 outputs; a stage of 32 k in LDS while the next one is on
+// its way in registers, one barrier a stage. Bound by the matrix cores (the loop reaches 139 TFLOP/s without
+// memory): the gate||up of the 7B shape (37888 x 3584) at 1003 rows takes 2.42 ms (112 TFLOP/s), its down projection
+// 1.38 ms; tiles on the vector ALU, which has half as many products a clock, took 4.80 and 5.20 ms. Columns of tiles go to an XCD in stretches: the row tiles that read one stretch of
+// weights run behind one L2.
+typedef float gp_f32x16 __attribute__((ext_vector_type(16)));
+typedef float gp_f32x4 __attribute__((ext_vector_type(4)));
+#define GPM_BK 32
+#define GPM_LD 36           // floats a row of a stage: 16 even k, 16 odd k, 4 of padding (reads without bank conflicts)
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_plain_mfma_kernel(
     float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W,
     const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int64_t lda, int64_t ldw,
-    int64_t ldc) {
-  __shared__ __attribute__((aligned(16))) float As[GP_BK][GPW_BM + 4];
-  __shared__ __attribute__((aligned(16))) float Ws[GP_BK][GPW_BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid & 15;  // along N
-  const int ty = tid >> 4;  // along M
-  const int m0 = blockIdx.y * GPW_BM;
-  const int n0 = blockIdx.x * GPW_BN;
-  const int lrow = tid >> 2;       // 0..63 (and + 64)
-  const int lk = (tid & 3) * 4;    // 0,4,8,12
-  float acc[8][8], total[8][8];
+    int64_t ldc, int mtiles, int ntiles, int vec) {
+  constexpr int TM = BM / 64, TN = BN / 64;      // 32 x 32 tiles of a wavefront
+  constexpr int LA = BM / 32, LW = BN / 32;      // 16-byte loads of a thread and stage
+  __shared__ __attribute__((aligned(16))) float stage[2][(BM + BN) * GPM_LD];
+  const int per_xcd = (mtiles * ntiles + HE_XCDS - 1) / HE_XCDS;
+  const int tile = (blockIdx.x % HE_XCDS) * per_xcd + blockIdx.x / HE_XCDS;
+  if (tile >= mtiles * ntiles) return;           // (the whole workgroup)
+  const int m0 = (tile % mtiles) * BM, n0 = (tile / mtiles) * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r32 = lane & 31, half = lane >> 5;
+  const int lrow = tid >> 3, lk = (tid & 7) * 4;
+  // rows beyond the matrices are the last row again: their outputs are not stored
+  const float* asrc[LA];
+  const float* wsrc[LW];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < LA; ++i) asrc[i] = A + (int64_t)min(m0 + lrow + 32 * i, M - 1) * lda;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f, total[i][j] = 0.f;
-  const bool a_vec = m0 + GPW_BM <= M && (lda & 3) == 0 && (((uintptr_t)A) & 15) == 0;
-  const bool w_vec = n0 + GPW_BN <= N && (ldw & 3) == 0 && (((uintptr_t)W) & 15) == 0;
-  for (int k0 = 0; k0 < K; k0 += GP_BK) {
-    const bool whole = k0 + GP_BK <= K;
+  for (int i = 0; i < LW; ++i) wsrc[i] = W + (int64_t)min(n0 + lrow + 32 * i, N - 1) * ldw;
+  gp_f32x4 av[LA], wv[LW];
+  auto fetch = [&](int k0) {
+    if (vec && k0 + GPM_BK <= K) {
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int r = lrow + 64 * half;
-      const int am = m0 + r, wn = n0 + r;
-      if (a_vec && whole) {
-        const float4 v = *reinterpret_cast<const float4*>(A + am * lda + k0 + lk);
-        As[lk][r] = v.x, As[lk + 1][r] = v.y, As[lk + 2][r] = v.z, As[lk + 3][r] = v.w;
-      } else {
+      for (int i = 0; i < LA; ++i) av[i] = *reinterpret_cast<const gp_f32x4*>(asrc[i] + k0 + lk);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = k0 + lk + j;
-          As[lk + j][r] = (am < M && k < K) ? A[am * lda + k] : 0.f;
-        }
-      }
-      if (w_vec && whole) {
-        const float4 v = *reinterpret_cast<const float4*>(W + wn * ldw + k0 + lk);
-        Ws[lk][r] = v.x, Ws[lk + 1][r] = v.y, Ws[lk + 2][r] = v.z, Ws[lk + 3][r] = v.w;
-      } else {
+      for (int i = 0; i < LW; ++i) wv[i] = *reinterpret_cast<const gp_f32x4*>(wsrc[i] + k0 + lk);
+    } else {      // K's end, or rows that are not 16-byte aligned: zeros beyond K leave a chain as it is
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = k0 + lk + j;
-          Ws[lk + j][r] = (wn < N && k < K) ? W[wn * ldw + k] : 0.f;
-        }
+      for (int e = 0; e < 4; ++e) {
+        const int k = k0 + lk + e;
+#pragma unroll
+        for (int i = 0; i < LA; ++i) av[i][e] = k < K ? asrc[i][k] : 0.f;
+#pragma unroll
+        for (int i = 0; i < LW; ++i) wv[i][e] = k < K ? wsrc[i][k] : 0.f;
       }
     }
+  };
+  auto put = [&](float* to) {
+#pragma unroll
+    for (int i = 0; i < LA + LW; ++i) {
+      const gp_f32x4 v = i < LA ? av[i < LA ? i : 0] : wv[i < LA ? 0 : i - LA];
+      float* row = to + (lrow + 32 * i) * GPM_LD + lk / 2;
+      *reinterpret_cast<float2*>(row) = make_float2(v[0], v[2]);
+      *reinterpret_cast<float2*>(row + 16) = make_float2(v[1], v[3]);
+    }
+  };
+  gp_f32x16 acc[TM][TN], total[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f, total[i][j][e] = 0.f;
+  const int arow = ((wave >> 1) * (BM / 2) + r32) * GPM_LD + half * 16;
+  const int wrow = (BM + (wave & 1) * (BN / 2) + r32) * GPM_LD + half * 16;
+  fetch(0);
+  put(stage[0]);
+  __syncthreads();
+  int cur = 0;
+  for (int k0 = 0; k0 < K; k0 += GPM_BK, cur ^= 1) {
+    const bool more = k0 + GPM_BK < K;
+    if (more) fetch(k0 + GPM_BK);
+    const float* at = stage[cur];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {                // eight k
+      gp_f32x4 a[TM], b[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const gp_f32x4*>(at + arow + i * 32 * GPM_LD + 4 * j);
+#pragma unroll
+      for (int i = 0; i < TN; ++i) b[i] = *reinterpret_cast<const gp_f32x4*>(at + wrow + i * 32 * GPM_LD + 4 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < TM; ++x)
+#pragma unroll
+          for (int y = 0; y < TN; ++y)
+            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x][e], b[y][e], acc[x][y], 0, 0, 0);
+    }
+    if ((k0 + GPM_BK) % GP_SEG == 0 || !more) {  // the segment ends here
+#pragma unroll
+      for (int x = 0; x < TM; ++x)
+#pragma unroll
+        for (int y = 0; y < TN; ++y)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) total[x][y][e] += acc[x][y][e], acc[x][y][e] = 0.f;
+    }
+    if (more) put(stage[cur ^ 1]);
     __syncthreads();
-#define GPW_STEP(kk)                                                                               \
-  {                                                                                                \
-    const float4 a0 = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);                           \
-    const float4 a1 = *reinterpret_cast<const float4*>(&As[kk][64 + ty * 4]);                      \
-    const float4 b0 = *reinterpret_cast<const float4*>(&Ws[kk][tx * 4]);                           \
-    const float4 b1 = *reinterpret_cast<const float4*>(&Ws[kk][64 + tx * 4]);                      \
-    const float a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};                           \
-    const float b[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};                           \
-    _Pragma("unroll") for (int i = 0; i < 8; ++i)                                                  \
-        _Pragma("unroll") for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);     \
-  }
-    if (whole) {
-#pragma unroll
-      for (int kk = 0; kk < GP_BK; ++kk) GPW_STEP(kk)
-    } else {
-      for (int kk = 0; kk < K - k0; ++kk) GPW_STEP(kk)
-    }
-#undef GPW_STEP
-    __syncthreads();
-    if ((k0 + GP_BK) % GP_SEG == 0 || k0 + GP_BK >= K) {   // the segment ends here
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) total[i][j] += acc[i][j], acc[i][j] = 0.f;
-    }
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + (i >> 2) * 64 + ty * 4 + (i & 3);
-    if (m >= M) continue;
+  for (int x = 0; x < TM; ++x)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int n = n0 + (j >> 2) * 64 + tx * 4 + (j & 3);
-      if (n >= N) continue;
-      float v = total[i][j];
-      if (bias != nullptr) v += load_param(bias, n, bias_dtype);
-      C[m * ldc + n] = v;
+    for (int y = 0; y < TN; ++y) {
+      const int n = n0 + (wave & 1) * (BN / 2) + 32 * y + r32;
+      const float b = bias != nullptr && n < N ? load_param(bias, n, bias_dtype) : 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + (wave >> 1) * (BM / 2) + 32 * x + (e >> 2) * 8 + half * 4 + (e & 3);
+        if (m < M && n < N) C[m * ldc + n] = bias != nullptr ? total[x][y][e] + b : total[x][y][e];
+      }
     }
+}
+
+// The 32-bit product of up to GP_MROWS_MAX_M rows in the same order, bound by the weights' way from memory. A
+// workgroup owns 16 weight rows and all activation rows (MT tiles of 16) and walks K with NW wavefronts, each
+// a segment of its own at a time: v_mfma_f32_16x16x4_f32 chains, whose sums go to LDS; after FLUSH rounds of
+// segments the workgroup adds them to its totals in segment order. So a weight of 3,584 rows still has 224 workgroups
+// with 16 wavefronts' loads in flight, and nothing goes through a workspace. (7B gate||up, 543 MB: 1 row 97 us, 4 rows
+// 98, 16 rows 128, 64 rows 308; a lane a weight row on the vector ALU and a second kernel for the segment sums, up to 8
+// rows, 104 and 114; 64 x 64 tiles, which more rows went through, 657 at 16 rows and, for the down projection's 3,584
+// weight rows of 18,944, 2479 where this takes 53.) A wavefront fetches a stage of KS k
+// of its 16 weight rows (and activation rows) whole lines at a time, two stages ahead, into its own LDS region, the
+// 16-byte pieces of row r at their index xor r, from which the operand of lane (row, k mod 4) is read a float at a
+// time without bank conflicts. For weights of whole segments in aligned rows.
+#define GP_MROWS_MAX_M 64
+template <int MT, int NW, int KS>
+__global__ __launch_bounds__(NW * 64) void gemm_plain_stream_kernel(
+    float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, const void* __restrict__ bias,
+    int bias_dtype, int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc) {
+  constexpr int FLUSH = NW * MT < 16 ? 16 / (NW * MT) : 1;   // rounds whose segment sums LDS holds
+  constexpr int P = KS / 4;                      // 16-byte pieces of a row and stage
+  constexpr int LD = KS / 16;                    // loads of a lane for 16 rows of a stage
+  constexpr int SPS = GP_SEG / KS;               // stages of a segment
+  __shared__ gp_f32x4 tiles[NW][(1 + MT) * 16 * P];
+  __shared__ float sums[FLUSH * NW][MT * 256];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16;
+  const int segments = K / GP_SEG;
+  A += (int64_t)blockIdx.y * (16 * MT) * lda;    // (more activation rows than a workgroup takes: the next ones along y)
+  C += (int64_t)blockIdx.y * (16 * MT) * ldc;
+  M -= blockIdx.y * (16 * MT);
+  // load t of a stage: row t * (64 / P) + lane / P of the 16, piece lane % P
+  const int lrow = lane / P, piece = lane % P;
+  const float* wsrc[LD];
+  const float* asrc[MT][LD];
+  bool real[MT][LD];
+#pragma unroll
+  for (int t = 0; t < LD; ++t) {
+    const int r = t * (64 / P) + lrow;
+    wsrc[t] = W + (int64_t)min(n0 + r, N - 1) * ldw + 4 * piece;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      real[i][t] = 16 * i + r < M;               // (rows beyond M stay zero: nothing is fetched for them)
+      asrc[i][t] = A + (int64_t)min(16 * i + r, M - 1) * lda + 4 * piece;
+    }
+  }
+  gp_f32x4* mine = tiles[wave];
+  const int rounds = (segments + NW - 1) / NW;
+  const int stages = rounds * SPS;               // of every wavefront; a stage of no segment does nothing
+  gp_f32x4 wv[2][LD], av[2][MT][LD];
+  const gp_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < LD; ++t) av[b][i][t] = zero;
+#define GPS_FETCH(B_, ST_)                                                                           \
+  {                                                                                                  \
+    const int seg_ = wave + NW * ((ST_) / SPS);                                                      \
+    if (seg_ < segments) {                                                                           \
+      const int64_t k_ = (int64_t)seg_ * GP_SEG + ((ST_) % SPS) * KS;                                \
+      _Pragma("unroll") for (int t = 0; t < LD; ++t) wv[B_][t] = *reinterpret_cast<const gp_f32x4*>(wsrc[t] + k_); \
+      _Pragma("unroll") for (int i = 0; i < MT; ++i)                                                 \
+        _Pragma("unroll") for (int t = 0; t < LD; ++t)                                               \
+          if (real[i][t]) av[B_][i][t] = *reinterpret_cast<const gp_f32x4*>(asrc[i][t] + k_);        \
+    }                                                                                                \
+  }
+  gp_f32x4 acc[MT];
+  float total[MT * 256 / (NW * 64) > 0 ? MT * 256 / (NW * 64) : 1];
+  constexpr int OWN = sizeof(total) / sizeof(float);   // outputs a thread adds up (threads beyond MT * 256: none)
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) total[i] = 0.f;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = zero;
+  const int r16 = lane & 15, h = lane >> 4;
+#define GPS_STAGE(B_, ST_)                                                                           \
+  {                                                                                                  \
+    const int seg_ = wave + NW * ((ST_) / SPS);                                                      \
+    if (seg_ < segments) {                                                                           \
+      _Pragma("unroll") for (int t = 0; t < LD; ++t) {                                               \
+        const int r = t * (64 / P) + lrow;                                                           \
+        mine[r * P + (piece ^ (r % P))] = wv[B_][t];                                                 \
+        _Pragma("unroll") for (int i = 0; i < MT; ++i)                                               \
+          mine[(16 * (1 + i) + r) * P + (piece ^ (r % P))] = av[B_][i][t];                           \
+      }                                                                                              \
+      __builtin_amdgcn_wave_barrier();                                                               \
+    }                                                                                                \
+    GPS_FETCH(B_, (ST_) + 2)                                                                         \
+    if (seg_ < segments) {                                                                           \
+      const float* f = reinterpret_cast<const float*>(mine) + r16 * KS + h;                          \
+      _Pragma("unroll") for (int j = 0; j < P; ++j) {                                                \
+        const int o = 4 * (j ^ (r16 % P));                                                           \
+        const float w = f[o];                                                                        \
+        _Pragma("unroll") for (int i = 0; i < MT; ++i)                                               \
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[16 * (1 + i) * KS + o], w, acc[i], 0, 0, 0); \
+      }                                                                                              \
+      __builtin_amdgcn_wave_barrier();                                                               \
+      if ((ST_) % SPS == SPS - 1) {                                                                  \
+        float* to = sums[((ST_) / SPS % FLUSH) * NW + wave];                                         \
+        _Pragma("unroll") for (int i = 0; i < MT; ++i) {                                             \
+          _Pragma("unroll") for (int e = 0; e < 4; ++e) to[i * 256 + (4 * h + e) * 16 + r16] = acc[i][e]; \
+          acc[i] = zero;                                                                             \
+        }                                                                                            \
+      }                                                                                              \
+    }                                                                                                \
+  }
+  GPS_FETCH(0, 0)
+  GPS_FETCH(1, 1)
+  for (int st = 0; st < stages; st += 2) {       // (SPS is even)
+    GPS_STAGE(0, st)
+    GPS_STAGE(1, st + 1)
+    const int round = (st + 2) / SPS;            // rounds done, where a round ends here
+    if ((st + 2) % SPS == 0 && (round % FLUSH == 0 || round == rounds)) {
+      __syncthreads();
+      const int first = (round - 1) / FLUSH * FLUSH * NW, count = min(segments - first, FLUSH * NW);
+#pragma unroll
+      for (int i = 0; i < OWN; ++i) {
+        const int o = tid + i * NW * 64;
+        if (o < MT * 256)
+          for (int s = 0; s < count; ++s) total[i] += sums[s][o];
+      }
+      __syncthreads();
+    }
+  }
+#undef GPS_FETCH
+#undef GPS_STAGE
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int o = tid + i * NW * 64, m = o >> 4, n = n0 + (o & 15);
+    if (o >= MT * 256 || m >= M || n >= N) continue;
+    C[m * ldc + n] = bias != nullptr ? total[i] + load_param(bias, n, bias_dtype) : total[i];
   }
 }
 
@@ -267,83 +406,6 @@ __global__ __launch_bounds__(256) void gemm_plain_rows_kernel(
   }
 }
 
-// The same sums for 32-bit weights whose K is whole segments, with the weights fetched line by
-// line: in the kernel above the 64 lanes of a load touch 64 cache lines (each lane its own row), and
-// the rate at which a compute unit looks lines up bounds it (3.6 TB/s at the Qwen2.5-7B shape). Here
-// eight neighbouring lanes fetch the 128 bytes of one row, a load touches eight lines, and the
-// wavefront turns the tile round in LDS: 32 k of its 64 rows at a time (two such chunks on their
-// way while one is multiplied), the values go into the wavefront's own LDS region as
-// [16-byte piece][row, 65 to a piece][4], from which lane n reads the pieces of row n one after the
-// other (a read of 64 lanes is one KiB on end) and extends its chain of FMAs in ascending k. The
-// region is the wavefront's own: LDS runs a wavefront's writes and reads in program order, so no
-// barrier is needed, and the compiler keeps stores and loads that may name the same address in
-// order. (A wavefront-scope fence here kept the staging registers in scratch memory.) grid and
-// block as above.
-#define GP_TURN_ROWS 65
-template <int MT>
-__global__ __launch_bounds__(256) void gemm_plain_rows_turned_kernel(
-    float* __restrict__ partial, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K,
-    int64_t lda, int64_t ldw, int segments) {
-  __shared__ float4 turned[4][8 * GP_TURN_ROWS];
-  const int lane = threadIdx.x;
-  const int n0 = blockIdx.x * 64;
-  const int seg = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + threadIdx.y);
-  if (seg >= segments) return;
-  const int k_begin = seg * GP_SEG;
-  // load i of a chunk of 32 k: row 8 i + lane / 8 of the tile, piece lane % 8 of its 128 bytes
-  const int lrow = lane >> 3, piece = lane & 7;
-  const float* src[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) src[i] = W + (int64_t)min(n0 + 8 * i + lrow, N - 1) * ldw + k_begin + 4 * piece;
-  float4 w0[8], w1[8];   // two chunks of 32 k on their way while a third is multiplied
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w0[i] = *reinterpret_cast<const float4*>(src[i]);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w1[i] = *reinterpret_cast<const float4*>(src[i] + 32);
-  float acc[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = 0.f;
-  const float* arow[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) arow[m] = A + (int64_t)min(m, M - 1) * lda + k_begin;
-  float4* mine = turned[threadIdx.y];
-#define GP_TURN(WV_, C_)                                                                          \
-  {                                                                                               \
-    _Pragma("unroll") for (int i = 0; i < 8; ++i) mine[piece * GP_TURN_ROWS + 8 * i + lrow] = WV_[i]; \
-    __builtin_amdgcn_wave_barrier();                                                              \
-    _Pragma("unroll") for (int p = 0; p < 8; ++p) {                                               \
-      const float4 w4 = mine[p * GP_TURN_ROWS + lane];                                            \
-      const float w[4] = {w4.x, w4.y, w4.z, w4.w};                                                \
-      _Pragma("unroll") for (int e = 0; e < 4; ++e)                                               \
-        _Pragma("unroll") for (int m = 0; m < MT; ++m)                                            \
-          acc[m] = fmaf(arow[m][32 * (C_) + 4 * p + e], w[e], acc[m]);                            \
-    }                                                                                             \
-    __builtin_amdgcn_wave_barrier();                                                              \
-  }
-  // (the scheduler would ask for all four chunks at once and then spill two of them: each
-  // sched_barrier keeps a group of loads where it is written)
-  __builtin_amdgcn_sched_barrier(0);
-  GP_TURN(w0, 0)
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w0[i] = *reinterpret_cast<const float4*>(src[i] + 64);
-  __builtin_amdgcn_sched_barrier(0);
-  GP_TURN(w1, 1)
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w1[i] = *reinterpret_cast<const float4*>(src[i] + 96);
-  __builtin_amdgcn_sched_barrier(0);
-  GP_TURN(w0, 2)
-  GP_TURN(w1, 3)
-#undef GP_TURN
-  const int n = n0 + lane;
-  if (n < N) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m < M) partial[((int64_t)seg * M + m) * N + n] = acc[m];
-  }
-}
-
 template <typename TC>
 __global__ __launch_bounds__(256) void gemm_plain_rows_sum_kernel(
     TC* __restrict__ C, const float* __restrict__ partial, const void* __restrict__ bias, int bias_dtype,
@@ -377,16 +439,9 @@ static int launch_rows(void* C, const void* A, const void* W, const void* bias, 
   const int segments = (K + GP_SEG - 1) / GP_SEG;
   dim3 grid((N + 63) / 64, (segments + 3) / 4), block(64, 4);
   HE_REQUIRE(grid.y <= 65535, "he_gemm_plain: K=%d too long for one launch", K);
-  // 32-bit weights in whole segments, rows 16-byte aligned: fetched line by line and turned round in LDS
-  constexpr bool f32 = sizeof(TA) == 4 && sizeof(TW) == 4;
-  const bool turned = f32 && K % GP_SEG == 0 && (ldw & 3) == 0 && (((uintptr_t)W) & 15) == 0;
 #define GP_ROWS(MT_)                                                                                  \
-  if (turned)                                                                                         \
-    gemm_plain_rows_turned_kernel<MT_><<<grid, block, 0, s>>>(ws, (const float*)A, (const float*)W, M, N, K, \
-                                                              lda, ldw, segments);                    \
-  else                                                                                                \
-    gemm_plain_rows_kernel<MT_, TA, TW><<<grid, block, 0, s>>>(ws, (const TA*)A, (const TW*)W, M, N, K, \
-                                                               lda, ldw, segments)
+  gemm_plain_rows_kernel<MT_, TA, TW><<<grid, block, 0, s>>>(ws, (const TA*)A, (const TW*)W, M, N, K, \
+                                                             lda, ldw, segments)
   if (M == 1) GP_ROWS(1);
   else if (M == 2) GP_ROWS(2);
   else if (M <= 4) GP_ROWS(4);
@@ -399,9 +454,52 @@ static int launch_rows(void* C, const void* A, const void* W, const void* bias, 
   return he_check_launch("he_gemm_plain");
 }
 
+// The kernel that streams the weights: up to GP_MROWS_MAX_M rows, and up to twice as many where tiles of 64 x 64 would
+// leave half of the units idle (3584 x 18944 at 128 rows: 458 us in tiles, 4608 x 3584, whose tiles fill the chip, 86). 16 wavefronts a workgroup where the weight's rows
+// give a compute unit one workgroup or less, else 8 (two workgroups share a unit).
+static int launch_stream(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K,
+                         int64_t lda, int64_t ldw, int64_t ldc, hipStream_t s) {
+  const dim3 grid((N + 15) / 16, (M + GP_MROWS_MAX_M - 1) / GP_MROWS_MAX_M);
+#define GP_STREAM(MT_, NW_, KS_) \
+  gemm_plain_stream_kernel<MT_, NW_, KS_><<<grid, NW_ * 64, 0, s>>>(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc)
+  if (M <= 16) {
+    if ((int)grid.x <= he_cus()) GP_STREAM(1, 16, 64);
+    else GP_STREAM(1, 8, 64);
+  } else if (M <= 32) {
+    GP_STREAM(2, 8, 32);
+  } else {
+    GP_STREAM(4, 8, 32);
+  }
+#undef GP_STREAM
+  return he_check_launch("he_gemm_plain");
+}
+
+// More rows: tiles on the matrix cores. Of the tile sizes the one whose fullest compute unit has the least to do
+// (a unit's workgroups share its matrix cores, so its time is the outputs dealt to it); the larger tile where
+// they tie, as it reads fewer operands an output.
+static int launch_mfma(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K,
+                       int64_t lda, int64_t ldw, int64_t ldc, hipStream_t s) {
+  const int vec = (lda & 3) == 0 && (ldw & 3) == 0 && (((uintptr_t)A) & 15) == 0 && (((uintptr_t)W) & 15) == 0;
+  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto most = [&](int bm, int bn) { return (tiles(bm, bn) + he_cus() - 1) / he_cus() * bm * bn; };
+  int bm = 128, bn = 128;
+  if (most(128, 64) < most(bm, bn)) bn = 64;
+  if (most(64, 64) < most(bm, bn)) bm = 64, bn = 64;
+  HE_REQUIRE(tiles(bm, bn) < (1 << 30), "he_gemm_plain: M=%d N=%d too large for one launch", M, N);
+  const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
+  const int grid = (int)((tiles(bm, bn) + HE_XCDS - 1) / HE_XCDS * HE_XCDS);
+#define GP_MFMA(BM_, BN_) \
+  gemm_plain_mfma_kernel<BM_, BN_><<<grid, 256, 0, s>>>(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc, mt, nt, vec)
+  if (bn == 128) GP_MFMA(128, 128);
+  else if (bm == 128) GP_MFMA(128, 64);
+  else GP_MFMA(64, 64);
+#undef GP_MFMA
+  return he_check_launch("he_gemm_plain");
+}
+
 // workspace_f32 (may be null) of workspace_floats floats: with he_gemm_plain_workspace_floats(M, N, K)
-// or more of them a product of few rows runs through the kernels made for it. The result is the
-// same bit for bit either way.
+// or more of them a product of few rows whose weight the streaming kernel does not take runs through the
+// kernels made for it. The result is the same bit for bit either way.
 extern "C" int he_gemm_plain(void* C, const void* A, const void* W, const void* bias, int M, int N,
                              int K, int64_t lda, int64_t ldw, int64_t ldc, int in_dtype,
                              int out_dtype, int bias_dtype, void* workspace_f32,
@@ -410,6 +508,11 @@ extern "C" int he_gemm_plain(void* C, const void* A, const void* W, const void* 
   HE_REQUIRE(lda >= K && ldw >= K && ldc >= N, "he_gemm_plain: bad leading dimensions");
   if (M == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  const bool f32 = in_dtype == HE_F32 && out_dtype == HE_F32;
+  const bool few = M <= GP_MROWS_MAX_M || (M <= 2 * GP_MROWS_MAX_M && 4 * ((N + 63) / 64) <= he_cus());
+  if (f32 && few && K % GP_SEG == 0 && (lda & 3) == 0 && (ldw & 3) == 0 && (((uintptr_t)A) & 15) == 0 &&
+      (((uintptr_t)W) & 15) == 0)
+    return launch_stream((float*)C, (const float*)A, (const float*)W, bias, bias_dtype, M, N, K, lda, ldw, ldc, s);
   const int64_t need = he_gemm_plain_workspace_floats(M, N, K);
   if (need > 0 && workspace_f32 != nullptr && workspace_floats >= need) {
     float* ws = (float*)workspace_f32;
@@ -421,16 +524,11 @@ extern "C" int he_gemm_plain(void* C, const void* A, const void* W, const void* 
       return launch_rows<bf16_t, bf16_t, float>(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc, ws, s);
     HE_REQUIRE(false, "he_gemm_plain: unsupported dtypes in=%d out=%d", in_dtype, out_dtype);
   }
+  if (f32)
+    return launch_mfma((float*)C, (const float*)A, (const float*)W, bias, bias_dtype, M, N, K, lda, ldw, ldc, s);
   dim3 grid((N + GP_BN - 1) / GP_BN, (M + GP_BM - 1) / GP_BM);
   HE_REQUIRE(grid.y <= 65535, "he_gemm_plain: M=%d too large for one launch", M);
-  if (in_dtype == HE_F32 && out_dtype == HE_F32 && M >= GPW_BM) {
-    dim3 wide((N + GPW_BN - 1) / GPW_BN, (M + GPW_BM - 1) / GPW_BM);
-    gemm_plain_wide_kernel<<<wide, 256, 0, s>>>((float*)C, (const float*)A, (const float*)W, bias, bias_dtype, M, N,
-                                                K, lda, ldw, ldc);
-  } else if (in_dtype == HE_F32 && out_dtype == HE_F32)
-    gemm_plain_kernel<float, float, float><<<grid, 256, 0, s>>>(
-        (float*)C, (const float*)A, (const float*)W, bias, bias_dtype, M, N, K, lda, ldw, ldc);
-  else if (in_dtype == HE_BF16 && out_dtype == HE_BF16)
+  if (in_dtype == HE_BF16 && out_dtype == HE_BF16)
     gemm_plain_kernel<bf16_t, bf16_t, bf16_t><<<grid, 256, 0, s>>>(
         (bf16_t*)C, (const bf16_t*)A, (const bf16_t*)W, bias, bias_dtype, M, N, K, lda, ldw, ldc);
   else if (in_dtype == HE_BF16 && out_dtype == HE_F32)
