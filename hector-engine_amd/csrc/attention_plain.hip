@@ -15,6 +15,8 @@
 // capped and then shifted by a table a head over the distance (ap_shape). gate (one number a row and head, or null): the
 // head's output is multiplied by sigmoid(gate) before it is stored.
 //
+// (32-bit caches with head sizes of 32, 64, 96 or 128 have an order of their own, on the matrix cores: further down.)
+//
 // Three launches keep that order and give the same bits: one wavefront per (query, head) that walks
 // the pages itself (or, in a step of many queries, per four neighbouring queries, which share what
 // they fetch); or, for steps of few queries over many keys (one-token steps), a wavefront
@@ -154,7 +156,7 @@ __device__ __forceinline__ void ap_page(ApState<NPL>& st, const float (&qv)[NPL]
 // total <- total joined with the result of the next page (one that had keys).
 template <int NPL>
 __device__ __forceinline__ void ap_join(ApState<NPL>& total, const ApState<NPL>& st) {
-  if (!(st.m > -INFINITY)) return;
+  if (!(st.m > -INFINITY) && st.l == 0.f) return;      // (scores that are no numbers leave a sum that is none)
   const float m_new = fmaxf(total.m, st.m);
   const float a = total.m > -INFINITY ? expf(total.m - m_new) : 0.f;
   const float b = expf(st.m - m_new);
@@ -192,6 +194,394 @@ __device__ __forceinline__ float ap_finish(ApState<NPL>& total, const ApExtras& 
   if (ex.gate == nullptr) return 1.f;
   const float g = to_float(((const T*)ex.gate)[row * ex.gate_stride + h]);
   return 1.f / (1.f + expf(-g));
+}
+
+// ---- 32-bit caches with head sizes of 32, 64, 96 or 128: both products on the matrix cores -------------------------
+//
+// A chain of v_mfma_f32_16x16x4_f32 on one accumulator is, bit for bit, a chain of FMAs over its k, so a fixed order
+// of the products costs nothing there. The order of a (query, head), the same in every launch: a score is the sum,
+// over ks, of (c0 + c1) + (c2 + c3), c the chain of the 8 dims 32 ks + 8 g + 2 c + e in the order of (e, g) (one chain of 128
+// would round more often than sums across a wavefront's lanes do: against 64 bits it is off by 3.1e-7 of the output's norm instead of
+// 2.8e-7, as such sums gave, at 1003 keys); a page's scores are taken off their maximum together, the sum of
+// the exponentials is, for each g, that of the keys 32 h + 8 g + 4 t + i in the order of (h, t, i), then (0 + 1) + (2 + 3)
+// over g; a value dim is one chain over the keys 32 h + 8 g + e in the order of (h, e, g); the pages are joined one
+// after the other as above. These orders are the pages' own layout (cache_layout.h): a lane's operands are the eight
+// consecutive elements it fetches, and the scores a lane holds (S^T = K Q^T: its column is a query, its rows are keys)
+// are the operand of O^T = V^T P^T as they are. Nothing goes through LDS.
+//
+// A key a query does not see has weight zero; where some value of the page is not finite and some query of the tile
+// does not see all of the page (or the page is not held, never for an admitted batch), the page's values are added key by key without the keys a query does not see (0 times
+// infinity would reach it). Values of keys beyond the tile's last position are taken as zero (nothing was written there).
+typedef float ap_f4 __attribute__((ext_vector_type(4)));
+template <int KS>
+struct ApPage32 {      // one page's operands as fetched: [half][key tile][k step][two pieces], [half][dim tile][two pieces]
+  ap_f4 k[2][2][KS][2];
+  ap_f4 v[2][2 * KS][2];
+};
+// A page is fetched through a buffer descriptor of its own: the address is one register, a scalar offset and an immediate
+// (as 64-bit pointers the addresses of a page's 64 loads took registers that its elements need).
+__device__ __forceinline__ ap_f4 ap32_load(__amdgpu_buffer_rsrc_t page, int lane, int piece) {
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  const u4 r = __builtin_amdgcn_raw_buffer_load_b128(page, lane * 32, piece * 16, 0);
+  return __builtin_bit_cast(ap_f4, r);
+}
+template <int KS>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ap32_rsrc(const float* page) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)page, 0, HE_PAGE_TOKENS * 32 * KS * 4, 0x00027000);
+}
+template <int KS>
+__device__ __forceinline__ void ap32_fetch_k(ApPage32<KS>& pg, __amdgpu_buffer_rsrc_t kpage, int h, int lane) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) pg.k[h][t][ks][b] = ap32_load(kpage, lane, ((h * 2 + t) * KS + ks) * 128 + b);
+}
+template <int KS>
+__device__ __forceinline__ void ap32_fetch_v(ApPage32<KS>& pg, __amdgpu_buffer_rsrc_t vpage, int h, int lane) {
+#pragma unroll
+  for (int dt = 0; dt < 2 * KS; ++dt)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) pg.v[h][dt][b] = ap32_load(vpage, lane, (h * 2 * KS + dt) * 128 + b);
+}
+// 16 queries: the lane's column is query lane % 16
+template <int KS>
+struct ApTile32 {
+  ap_f4* q;              // LDS: the lane's dims 32 ks + 8 g + 4 b .. + 3 of its query at (2 ks + b) 64
+  ap_f4* total;          // LDS: dims 16 dt + 4 g .. + 3 of the sums so far at 64 dt
+  float m, l;
+  int p, first;          // the keys the column sees: [first, p] (p < first: no query)
+  ApShape sh;
+};
+// The page whose first key is j0 joins the tile; pg holds its keys on entry and, with NEXT, those of next_k on return (not
+// under a condition: registers that may keep their old keys would be held through the page). last: no key beyond it has been
+// written. whole: every column sees all of it. With NEXT a page's halves of 32 keys take turns in the registers, so that
+// two wavefronts fit a SIMD (one's products beside the other's softmax and waits): a half's values are asked for
+// behind its scores, a half of the next page's keys behind its value products. Without it all values come before the scores.
+template <int KS, bool NEXT, bool SHAPED>
+__device__ __forceinline__ void ap32_page(ApTile32<KS>& t, ApPage32<KS>& pg, const float* vpage_at, const float* next_k_at,
+                                          bool held, int j0, int last, bool whole, float scale, int lane) {
+  const int g = lane >> 4;
+  const __amdgpu_buffer_rsrc_t vpage = ap32_rsrc<KS>(vpage_at), next_k = ap32_rsrc<KS>(next_k_at);
+  ap_f4 s[2][2];
+  if (!NEXT) ap32_fetch_v<KS>(pg, vpage, 0, lane), ap32_fetch_v<KS>(pg, vpage, 1, lane);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      ap_f4 part[4][2];
+      const ap_f4 qv[2] = {t.q[2 * ks * HE_WAVE], t.q[(2 * ks + 1) * HE_WAVE]};
+#pragma unroll
+      for (int e = 0; e < 2; ++e)      // (the eight chains in turn: an instruction does not wait for the one before it)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const int d = 2 * (c & 1) + e;
+            part[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(pg.k[h][x][ks][c >> 1][d], qv[c >> 1][d],
+                                                              e == 0 ? ap_f4{0.f, 0.f, 0.f, 0.f} : part[c][x], 0, 0, 0);
+          }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float all = (part[0][x][i] + part[1][x][i]) + (part[2][x][i] + part[3][x][i]);
+          s[h][x][i] = ks == 0 ? all : s[h][x][i] + all;
+        }
+      __builtin_amdgcn_sched_barrier(0);      // (the parts of several k steps at once would not fit the registers)
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (NEXT) ap32_fetch_v<KS>(pg, vpage, h, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float top = -INFINITY;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = j0 + 32 * h + 8 * g + 4 * x + i;
+        const float v = SHAPED ? ap_shape(t.sh, s[h][x][i] * scale, t.p - j) : s[h][x][i] * scale;
+        s[h][x][i] = held && j >= t.first && j <= t.p ? v : -INFINITY;
+        top = fmaxf(top, s[h][x][i]);
+      }
+  top = fmaxf(top, __shfl_xor(top, 16));
+  top = fmaxf(top, __shfl_xor(top, 32));
+  const float off = top > -INFINITY ? top : 0.f;
+  float sum = 0.f;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = s[h][x][i];
+        const float w = v == top && top > -INFINITY ? 1.f : expf(v - off);
+        s[h][x][i] = w;
+        sum += w;
+      }
+  const float l = xor32_sum(xor16_sum(sum));
+  ap_f4 acc[2 * KS];
+#pragma unroll
+  for (int dt = 0; dt < 2 * KS; ++dt) acc[dt] = ap_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    bool by_key = false;
+    if (!whole) {
+      float none = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int dt = 0; dt < 2 * KS; ++dt) {
+          const float v = j0 + 32 * h + 8 * g + e > last ? 0.f : pg.v[h][dt][e >> 2][e & 3];
+          pg.v[h][dt][e >> 2][e & 3] = v;
+          none = fmaf(v, 0.f, none);
+        }
+      by_key = __any(none != 0.f);
+    }
+    if (!by_key) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int dt = 0; dt < 2 * KS; ++dt)
+          acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(pg.v[h][dt][e >> 2][e & 3], s[h][e >> 2][e & 3], acc[dt], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma nounroll
+        for (int gg = 0; gg < 4; ++gg) {
+          int own = g;
+          asm volatile("" : "+v"(own));      // (the addresses of this rare path are not kept in registers all along)
+          const int key = 32 * h + 8 * gg + e;
+          const float w = __shfl(s[h][e >> 2][e & 3], (lane & 15) + 16 * gg);
+          if (held && j0 + key >= t.first && j0 + key <= t.p) {
+#pragma unroll
+            for (int dt = 0; dt < 2 * KS; ++dt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                acc[dt][i] = fmaf(vpage_at[he_v_index(key, 16 * dt + 4 * own + i, 2 * KS)], w, acc[dt][i]);
+          }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (NEXT) ap32_fetch_k<KS>(pg, next_k, h, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (top > -INFINITY || l != 0.f) {                // as ap_join
+    const float m_new = fmaxf(t.m, top);
+    const float a = t.m > -INFINITY ? expf(t.m - m_new) : 0.f;
+    const float b = expf(top - m_new);
+    t.l = fmaf(t.l, a, l * b);
+#pragma unroll
+    for (int dt = 0; dt < 2 * KS; ++dt) {
+      ap_f4 v = t.total[dt * HE_WAVE];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = fmaf(v[i], a, acc[dt][i] * b);
+      t.total[dt * HE_WAVE] = v;
+    }
+    t.m = m_new;
+  }
+}
+template <int KS>
+__device__ __forceinline__ void ap32_begin(ApTile32<KS>& t, const float* qrow, bool has, int lane) {
+  const int g = lane >> 4;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+      t.q[(2 * ks + b) * HE_WAVE] = has ? *reinterpret_cast<const ap_f4*>(qrow + 32 * ks + 8 * g + 4 * b) : ap_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int dt = 0; dt < 2 * KS; ++dt) t.total[dt * HE_WAVE] = ap_f4{0.f, 0.f, 0.f, 0.f};
+  t.m = -INFINITY;
+  t.l = 0.f;
+}
+template <int KS>
+__device__ __forceinline__ void ap32_store(ApTile32<KS>& t, float* o, const ApExtras& ex, int64_t row, int h, int lane) {
+  // the sink joins last; the gate scales what is stored
+  float gf = 1.f, a = 1.f;
+  if (ex.sinks != nullptr) {
+    const float sink = load_param(ex.sinks, h, ex.sinks_dtype), m_new = fmaxf(t.m, sink);
+    a = t.m > -INFINITY ? expf(t.m - m_new) : 0.f;
+    t.l = fmaf(t.l, a, expf(sink - m_new));
+  }
+  if (ex.gate != nullptr) gf = 1.f / (1.f + expf(-((const float*)ex.gate)[row * ex.gate_stride + h]));
+  const float inv = t.l > 0.f ? 1.f / t.l : 0.f;
+#pragma unroll
+  for (int dt = 0; dt < 2 * KS; ++dt) {
+    ap_f4 v = t.total[dt * HE_WAVE];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (ex.sinks != nullptr) v[i] = fmaf(v[i], a, 0.f);
+      v[i] = ex.gate ? v[i] * inv * gf : v[i] * inv;
+    }
+    *reinterpret_cast<ap_f4*>(o + 16 * dt + 4 * (lane >> 4)) = v;
+  }
+}
+
+// Rows of an aligned group of 16 that are neighbours in one sequence are a run; runs of at least AP32_RUN rows go through
+// the kernel for many queries, the others through the kernel for one.
+#define AP32_TILE 16
+#define AP32_RUN 8
+// bit i: row r0 + i begins a run (r0 the group's first row; rows beyond the step begin one each)
+__device__ __forceinline__ uint32_t ap32_runs(const int32_t* row_seq, const int32_t* positions, int r0, int rows, int lane) {
+  const int r = r0 + (lane & 15);
+  const int seq = r < rows ? row_seq[r] : -1, p = r < rows ? positions[r] : 0;
+  const int seq_before = __shfl_up(seq, 1), p_before = __shfl_up(p, 1);
+  const bool begins = (lane & 15) == 0 || seq < 0 || seq != seq_before || p != p_before + 1;
+  return (uint32_t)__ballot(begins) & 0xffffu;
+}
+__device__ __forceinline__ int ap32_run_end(uint32_t begins, int i) {      // the first row behind the run that row i is in
+  const uint32_t later = begins & ~((2u << i) - 1u);
+  return later ? __ffs(later) - 1 : AP32_TILE;
+}
+__device__ __forceinline__ int ap32_run_begin(uint32_t begins, int i) { return 31 - __clz(begins & ((2u << i) - 1u)); }
+
+// Many queries: a wavefront takes 16 rows of one head, run by run. grid (ceil(rows / 16), ceil(H / 4)), the last rows (the most
+// keys) first; a workgroup's wavefronts walk the same pages for neighbouring heads. Per page 256 instructions of 32 cycles
+// on the matrix cores (head size 128) beside the softmax of the other wavefront of the SIMD. 1003 tokens, 28 heads of 128:
+// 202 us a layer; 1850 with a wavefront's lanes along the dims and a sum across the wavefront for every score.
+template <int KS, bool SHAPED>
+__global__ __launch_bounds__(256, SHAPED ? 1 : 2) void attention_f32_rows_kernel(
+    float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ kpool, const float* __restrict__ vpool,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ row_seq, const int32_t* __restrict__ seq_slot,
+    const int32_t* __restrict__ page_table, int max_blocks, int num_pages, int rows, int H, int KVH, int window, int chunk,
+    float scale, ApExtras ex) {
+  constexpr int hd = 32 * KS;
+  const int lane = threadIdx.x & (HE_WAVE - 1);
+  const int h = blockIdx.y * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (h >= H) return;
+  const int r0 = (gridDim.x - 1 - blockIdx.x) * AP32_TILE;
+  const int kvh = h / (H / KVH);
+  __shared__ ap_f4 own[4][KS * 4 * HE_WAVE];    // queries and sums (each wavefront's own, each lane its own places of it)
+  const uint32_t begins = ap32_runs(row_seq, positions, r0, rows, lane);
+  for (int i0 = 0; i0 < AP32_TILE && r0 + i0 < rows;) {
+    const int i1 = ap32_run_end(begins, i0);
+    const int seq = row_seq[r0 + i0];
+    const int begin = i0;
+    i0 = i1;
+    if (seq < 0 || i1 - begin < AP32_RUN) continue;
+    const int p0 = positions[r0 + begin], p_last = p0 + (i1 - begin) - 1;
+    ApTile32<KS> t;
+    t.q = own[threadIdx.x >> 6] + lane;
+    t.total = t.q + 2 * KS * HE_WAVE;
+    const int c = lane & 15;
+    const bool has = c >= begin && c < i1;
+    t.p = has ? p0 + c - begin : -1;
+    t.first = has ? ap_first(t.p, window, chunk) : 0;
+    t.sh = ap_shape_of(ex, h);
+    ap32_begin<KS>(t, q + ((int64_t)(r0 + (has ? c : begin)) * H + h) * hd, has, lane);
+    const int32_t* pt = page_table + (int64_t)seq_slot[seq] * max_blocks;
+    const int first = ap_first(p0, window, chunk);      // (first never falls along a run)
+    const int first_last = ap_first(p_last, window, chunk);
+    const int c0 = first >> HE_PAGE_SHIFT, c1 = p_last >> HE_PAGE_SHIFT;
+    ApPage32<KS> pg;
+    int page = __builtin_amdgcn_readfirstlane(pt[c0]);
+    bool held = page >= 0 && page < num_pages;          // always, for an admitted batch
+    const int64_t elems = 32 * KS * HE_PAGE_TOKENS;
+    for (int half = 0; half < 2; ++half)
+      ap32_fetch_k<KS>(pg, ap32_rsrc<KS>(kpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems), half, lane);
+    for (int b = c0; b <= c1; ++b) {
+      const float* vpage = vpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems;
+      const int next = __builtin_amdgcn_readfirstlane(pt[min(b + 1, c1)]);
+      const bool next_held = next >= 0 && next < num_pages;
+      const float* next_k = kpool + ((next_held ? next : 0) * (int64_t)KVH + kvh) * elems;
+      const int j0 = b << HE_PAGE_SHIFT;
+      // (a column without a query sees nothing of any page: the sums it takes part in are not stored)
+      const bool whole = held && j0 >= first_last && j0 + HE_PAGE_TOKENS - 1 <= p0;
+      ap32_page<KS, true, SHAPED>(t, pg, vpage, next_k, held, j0, p_last, whole, scale, lane);
+      page = next;
+      held = next_held;
+    }
+    if (has) ap32_store<KS>(t, out + ((int64_t)(r0 + c) * H + h) * hd, ex, r0 + c, h, lane);
+  }
+}
+
+// One query: a wavefront takes one row and up to 16 heads of one kv head (its columns), and one page (pages > 1: the result
+// goes to ws as attention_plain_kernel's does) or all of them. Rows of long runs are left out where the kernel above takes them
+// (runs_elsewhere). A unit is a wavefront: rows x kv heads x tiles of 16 heads x pages, pages fastest.
+// 4 sequences of about 700 keys, 28 heads of 128 on 4: 16.5 us, 38 with a wavefront a head.
+template <int KS, bool SPLIT, bool SHAPED>
+__global__ __launch_bounds__(256, SPLIT || SHAPED ? 1 : 2) void attention_f32_one_kernel(
+    float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ q, const float* __restrict__ kpool,
+    const float* __restrict__ vpool, const int32_t* __restrict__ positions, const int32_t* __restrict__ row_seq,
+    const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ page_table, int max_blocks, int num_pages, int rows,
+    int H, int KVH, int window, int chunk, float scale, int pages, int runs_elsewhere, ApExtras ex) {
+  constexpr int hd = 32 * KS;
+  const int lane = threadIdx.x & (HE_WAVE - 1);
+  const int group = H / KVH, tiles = (group + 15) / 16;
+  int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int z = (int)(unit % pages);
+  unit /= pages;
+  const int tile = (int)(unit % tiles);
+  unit /= tiles;
+  const int kvh = (int)(unit % KVH);
+  unit /= KVH;
+  if (unit >= rows) return;
+  const int row = (int)unit;
+  const int col = 16 * tile + (lane & 15);
+  const bool has = col < group;
+  const int h = kvh * group + min(col, group - 1);
+  float* o = out + ((int64_t)row * H + h) * hd;
+  const int seq = row_seq[row];
+  if (seq < 0) {
+    if (!SPLIT && has)
+#pragma unroll
+      for (int dt = 0; dt < 2 * KS; ++dt) *reinterpret_cast<ap_f4*>(o + 16 * dt + 4 * (lane >> 4)) = ap_f4{0.f, 0.f, 0.f, 0.f};
+    return;
+  }
+  if (runs_elsewhere) {
+    const int r0 = row & ~(AP32_TILE - 1);
+    const uint32_t begins = ap32_runs(row_seq, positions, r0, rows, lane);
+    if (ap32_run_end(begins, row - r0) - ap32_run_begin(begins, row - r0) >= AP32_RUN) return;
+  }
+  const int p = positions[row];
+  const int first = ap_first(p, window, chunk);
+  int c0 = first >> HE_PAGE_SHIFT, c1 = p >> HE_PAGE_SHIFT;
+  if (SPLIT) {
+    if (c0 + z > c1) return;
+    c0 += z;
+    c1 = c0;
+  }
+  const int32_t* pt = page_table + (int64_t)seq_slot[seq] * max_blocks;
+  __shared__ ap_f4 own[4][KS * 4 * HE_WAVE];
+  ApTile32<KS> t;
+  t.q = own[threadIdx.x >> 6] + lane;
+  t.total = t.q + 2 * KS * HE_WAVE;
+  t.p = has ? p : -1;
+  t.first = has ? first : 0;
+  t.sh = ap_shape_of(ex, h);
+  ApPage32<KS> pg;
+  const int64_t elems = 32 * KS * HE_PAGE_TOKENS;
+  int page = __builtin_amdgcn_readfirstlane(pt[c0]);
+  bool held = page >= 0 && page < num_pages;
+  for (int half = 0; half < 2; ++half)
+    ap32_fetch_k<KS>(pg, ap32_rsrc<KS>(kpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems), half, lane);
+  ap32_begin<KS>(t, q + ((int64_t)row * H + h) * hd, has, lane);
+  for (int c = c0; c <= c1; ++c) {
+    const float* vpage = vpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems;
+    const int next = __builtin_amdgcn_readfirstlane(pt[min(c + 1, c1)]);
+    const bool next_held = next >= 0 && next < num_pages;
+    const float* next_k = kpool + ((next_held ? next : 0) * (int64_t)KVH + kvh) * elems;
+    const int j0 = c << HE_PAGE_SHIFT;
+    const bool whole = held && j0 >= first && j0 + HE_PAGE_TOKENS - 1 <= p;
+    ap32_page<KS, !SPLIT, SHAPED>(t, pg, vpage, next_k, held, j0, p, whole, scale, lane);
+    page = next;
+    held = next_held;
+  }
+  if (!has) return;
+  if (SPLIT) {
+    float* w = ws + (((int64_t)row * H + h) * pages + z) * (hd + 2);
+#pragma unroll
+    for (int dt = 0; dt < 2 * KS; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[16 * dt + 4 * (lane >> 4) + i] = t.total[dt * HE_WAVE][i];
+    if (lane < 16) w[hd] = t.m, w[hd + 1] = t.l;
+    return;
+  }
+  ap32_store<KS>(t, o, ex, row, h, lane);
 }
 
 // grid (rows, ceil(H / 4), pages): pages == 1: the wavefront walks all pages of its query and stores
@@ -516,6 +906,32 @@ extern "C" int he_attention_plain(void* out, const void* q, const void* kpool, c
   dim3 grid(rows, (H + 3) / 4, pages);
   float* ws = (float*)workspace_f32;
   hipStream_t s = (hipStream_t)stream;
+  // 32-bit caches whose head size is whole steps of the matrix cores' operands
+  const bool mfma = dtype == HE_F32 && hd % 32 == 0 && hd <= 128 && (((uintptr_t)q | (uintptr_t)kpool | (uintptr_t)vpool | (uintptr_t)out) & 15) == 0;
+  const bool by_runs = mfma && !split && rows >= AP32_TILE;
+  const int64_t units = (int64_t)rows * KVH * ((H / KVH + 15) / 16) * pages;
+  HE_REQUIRE(!mfma || units < (1ll << 32), "he_attention_plain: %d rows are too many for one launch", rows);
+  const bool shaped = slopes_f32 != nullptr || table_f32 != nullptr || cap > 0.f;
+#define AP32_ONE(KS_, SPLIT_, SHAPED_)                                                                               \
+  attention_f32_one_kernel<KS_, SPLIT_, SHAPED_><<<(unsigned)((units + 3) / 4), 256, 0, s>>>(                        \
+      (float*)out, ws, (const float*)q, (const float*)kpool, (const float*)vpool, (const int32_t*)positions,         \
+      (const int32_t*)row_seq, (const int32_t*)seq_slot, (const int32_t*)page_table, max_blocks, num_pages, rows, H, KVH, \
+      window, chunk, scale, pages, by_runs ? 1 : 0, ex)
+#define AP32_SHAPED(KS_, SHAPED_)                                                                                    \
+  {                                                                                                                  \
+    if (by_runs)                                                                                                     \
+      attention_f32_rows_kernel<KS_, SHAPED_><<<dim3((rows + AP32_TILE - 1) / AP32_TILE, (H + 3) / 4), 256, 0, s>>>( \
+          (float*)out, (const float*)q, (const float*)kpool, (const float*)vpool, (const int32_t*)positions,         \
+          (const int32_t*)row_seq, (const int32_t*)seq_slot, (const int32_t*)page_table, max_blocks, num_pages, rows, H, \
+          KVH, window, chunk, scale, ex);                                                                            \
+    if (split) AP32_ONE(KS_, true, SHAPED_);                                                                         \
+    else AP32_ONE(KS_, false, SHAPED_);                                                                              \
+  }
+#define AP32_LAUNCH(KS_)                                                                                             \
+  {                                                                                                                  \
+    if (shaped) AP32_SHAPED(KS_, true)                                                                               \
+    else AP32_SHAPED(KS_, false)                                                                                     \
+  }
 #define AP_LAUNCH(T, NPL)                                                                      \
   attention_plain_kernel<T, NPL><<<grid, 256, 0, s>>>(                                         \
       (T*)out, ws, (const T*)q, (const T*)kpool, (const T*)vpool, (const int32_t*)positions,   \
@@ -544,6 +960,16 @@ extern "C" int he_attention_plain(void* out, const void* q, const void* kpool, c
       (T*)out, (const T*)q, (const T*)kpool, (const T*)vpool, (const int32_t*)positions,               \
       (const int32_t*)row_seq, (const int32_t*)seq_slot, (const int32_t*)page_table, max_blocks,       \
       num_pages, rows, H, KVH, hd, window, chunk, scale, ex)
+  if (mfma) {
+    if (hd == 32) AP32_LAUNCH(1)
+    else if (hd == 64) AP32_LAUNCH(2)
+    else if (hd == 96) AP32_LAUNCH(3)
+    else AP32_LAUNCH(4)
+    int rc = he_check_launch("he_attention_plain");
+    if (rc || !split) return rc;
+    AP_BY_SIZE(AP_JOIN)
+    return he_check_launch("he_attention_plain");
+  }
   if (!split && rows >= 64) {      // a step of many queries: four neighbours a wavefront share their keys
     AP_BY_SIZE(AP_ROWS_LAUNCH)
     return he_check_launch("he_attention_plain");
@@ -555,6 +981,9 @@ extern "C" int he_attention_plain(void* out, const void* q, const void* kpool, c
 #undef AP_BY_SIZE
 #undef AP_ROWS_LAUNCH
 #undef AP_LAUNCH
+#undef AP32_LAUNCH
+#undef AP32_SHAPED
+#undef AP32_ONE
 #undef AP_JOIN
   return he_check_launch("he_attention_plain");
 }
