@@ -269,6 +269,20 @@ int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32, const voi
                     const void* correction, int c_dtype, int rows, int E, int real, int groups, int keep,
                     int top, float scale, int normalize, const void* bias, int bias_dtype, int x_pieces, void* stream);
 // bias (or null): [E], added to the logits before anything else; x_pieces: the bf16 rows x lie piece-major for exactly `rows` rows.
+// bf16 products of many rows: out[m][n] = x[m] . w[n] (+ bias). epilogue 0: bf16 results; 1: the weight's rows alternate gate and
+// up, out[m][n / 2] = the gated activation (constants as he_gated_act); 2: fp32 results. bm: rows a tile, 128 or 256.
+// K a multiple of 64, N of 4.
+int he_gemm_tall_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
+                      int64_t ldx, int64_t ldw, int64_t ldo, int epilogue, int bm, float alpha, float limit, float up_shift,
+                      float cubic, void* stream);
+// The experts of a routed feed-forward over the rows that chose them (gemm_tall.hip): scratch sizes, and the whole
+// (down null: the activations alone).
+int he_group_rows_most_tiles(int rows, int top, int groups, int bm);
+int64_t he_routed_groups_ints(int rows, int top, int real, int bm);
+int he_routed_groups(void* out, void* lists_i32, void* h_bf16, void* partial_f32, const void* x, const void* gate_up,
+                     const void* down, int64_t ldw, const void* ids_i32, const void* weights_f32, const void* dense_f32,
+                     int rows, int top, int real, int I, int D, int identity, int bm, float alpha, float limit, float up_shift,
+                     float cubic, void* stream);
 // he_routed_act: `shared` more columns behind the experts' (an expert every row uses): weight 1.
 int he_routed_act(void* out, const void* gate_up, const void* dense_f32, const void* h, int rows, int real,
                   int I, int shared, int extra, int dtype, float alpha, float limit, float up_shift, float cubic,

@@ -99,6 +99,12 @@ _SIGNATURES = {
                         c_int, c_int, c_ptr, c_int, c_f32, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_ptr],
     "he_routed_act": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_int, c_f32, c_f32, c_f32, c_f32,
                       c_ptr],
+    "he_gemm_tall_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_int, c_int,
+                          c_f32, c_f32, c_f32, c_f32, c_ptr],
+    "he_group_rows_most_tiles": [c_int, c_int, c_int, c_int],
+    "he_routed_groups_ints": [c_int, c_int, c_int, c_int],
+    "he_routed_groups": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int,
+                         c_int, c_int, c_int, c_f32, c_f32, c_f32, c_f32, c_ptr],
     "he_chosen_experts": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_f32, c_f32, c_f32, c_f32, c_int, c_ptr],
     "he_diff_heads": [c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_f32, c_f32, c_f32, c_int, c_ptr],
@@ -139,6 +145,7 @@ _RESTYPES = {
     "he_delta_state_floats": c_i64,
     "he_delta_workspace_floats": c_i64,
     "he_gemm_plain_workspace_floats": c_i64,
+    "he_routed_groups_ints": c_i64,
     "he_attention_decode_workspace_floats": c_i64,
     "he_attention_decode_fused_workspace_floats": c_i64,
     "he_attention_prefill_workspace_floats": c_i64,

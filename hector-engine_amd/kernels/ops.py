@@ -1179,6 +1179,83 @@ def routed_act(out, gate_up, dense, h, rows: int, real: int, inter: int, *, shar
                                _stream()))
 
 
+@_op("gemm_tall")
+def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
+    """out[M, N] = x[M, K] . w[N, K]^T (+ bias) for many bf16 rows (bf16 or fp32 results); with act, the constants (alpha,
+    limit, up_shift, cubic) of a gated activation, w's rows alternate gate and up and out is [M, N / 2]. K a multiple
+    of 64, N of 4. bm: rows of a tile, 128 or 256."""
+    N, K = w.shape
+    cols = N // 2 if act is not None else N
+    _need(out, "out", None, (None, cols))
+    _need(x, "x", torch.bfloat16, (None, K))
+    _need(w, "w", torch.bfloat16)
+    if bias is not None:
+        _need(bias, "bias", None, (N,))
+    if min(out.shape[0], x.shape[0]) < M or out.dtype not in ((torch.bfloat16,) if act is not None else (torch.bfloat16, torch.float32)):
+        raise ValueError("gemm_tall: buffers smaller than the row count, or results of an unknown type")
+    epilogue = 1 if act is not None else 2 if out.dtype == torch.float32 else 0
+    alpha, limit, up_shift, cubic = act or (1.0, 0.0, 0.0, 0.0)
+    _lib.check(_lib.load().he_gemm_tall_bf16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias),
+                                             dtype_code(bias.dtype) if bias is not None else F32, M, N, K, K, K, cols, epilogue,
+                                             bm, float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+
+
+def routed_groups_sizes(rows: int, top: int, real: int, bm: int) -> tuple[int, int]:
+    """(ints of lists, slots) of routed_groups' scratch."""
+    L = _lib.load()
+    return int(L.he_routed_groups_ints(rows, top, real, bm)), bm * int(L.he_group_rows_most_tiles(rows, top, real, bm))
+
+
+@_op("routed_groups")
+def routed_groups(out, lists, h, partial, x, gate_up, down, ids, weights, dense, rows: int, real: int, inter: int, *,
+                  bm: int, alpha: float = 1.0, limit: float = 0.0, up_shift: float = 0.0, cubic: float = 0.0) -> None:
+    """out[rows, D] = the weighted sum of the chosen experts' results (ids, weights [rows, top] and dense [rows, real + 1] as
+    route_tokens leaves them): the rows are sorted by expert and each expert's gate, up and down products run over its own
+    rows, in tiles of bm (128 or 256). gate_up [2 real inter, D] (gate and up alternating), down [D, real inter (+ D)]; with
+    the last D columns the identity experts' share dense[row, real] * x is added. lists int32, h bf16 [slots, inter] and
+    partial fp32 [slots, D]: scratch, routed_groups_sizes()."""
+    D, top = gate_up.shape[1], ids.shape[1]
+    for name, t in (("out", out), ("h", h), ("x", x), ("gate_up", gate_up), ("down", down)):
+        _need(t, name, torch.bfloat16)
+    _need(ids, "ids", torch.int32, (None, top))
+    _need(weights, "weights", torch.float32, (None, top))
+    _need(dense, "dense", torch.float32, (None, real + 1))
+    _need(lists, "lists", torch.int32)
+    _need(partial, "partial", torch.float32)
+    ints, slots = routed_groups_sizes(rows, top, real, bm)
+    if tuple(gate_up.shape) != (2 * real * inter, D) or down.shape[0] != D or down.shape[1] not in (real * inter, real * inter + D):
+        raise ValueError("routed_groups: the fused matrices do not match the sizes")
+    if min(out.shape[0], x.shape[0], ids.shape[0], weights.shape[0], dense.shape[0]) < rows or out.shape[1] != D \
+            or x.shape[1] != D or lists.numel() < ints or h.numel() < slots * inter or partial.numel() < slots * D:
+        raise ValueError("routed_groups: buffers smaller than the row count")
+    L = _lib.load()
+    _lib.check(L.he_routed_groups(out.data_ptr(), lists.data_ptr(), h.data_ptr(), partial.data_ptr(), x.data_ptr(),
+                                  gate_up.data_ptr(), down.data_ptr(), down.stride(0), ids.data_ptr(), weights.data_ptr(),
+                                  dense.data_ptr(), rows, top, real, inter, D, int(down.shape[1] > real * inter), bm,
+                                  float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+
+
+@_op("routed_groups_act")
+def routed_groups_act(h, lists, x, gate_up, ids, weights, rows: int, real: int, inter: int, *, bm: int, alpha: float = 1.0,
+                      limit: float = 0.0, up_shift: float = 0.0, cubic: float = 0.0) -> None:
+    """The first half of routed_groups in the layout of the product over all experts: h [rows, real inter], cleared by the
+    caller, gets weight * act(gate x, up x) in the columns of the experts a row chose."""
+    D, top = gate_up.shape[1], ids.shape[1]
+    for name, t in (("h", h), ("x", x), ("gate_up", gate_up)):
+        _need(t, name, torch.bfloat16)
+    _need(ids, "ids", torch.int32, (None, top))
+    _need(weights, "weights", torch.float32, (None, top))
+    _need(lists, "lists", torch.int32)
+    if tuple(gate_up.shape) != (2 * real * inter, D) or h.shape[1] != real * inter or x.shape[1] != D \
+            or min(h.shape[0], x.shape[0], ids.shape[0], weights.shape[0]) < rows \
+            or lists.numel() < routed_groups_sizes(rows, top, real, bm)[0]:
+        raise ValueError("routed_groups_act: the buffers do not match the sizes")
+    L = _lib.load()
+    _lib.check(L.he_routed_groups(None, lists.data_ptr(), h.data_ptr(), None, x.data_ptr(), gate_up.data_ptr(), None, 0,
+                                  ids.data_ptr(), weights.data_ptr(), None, rows, top, real, inter, D, 0, bm,
+                                  float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+
+
 @_op("chosen_experts")
 def chosen_experts(out, h_scratch, x, gate_up, down, ids, weights, dense, rows: int, real: int, inter: int, *,
                    shared: int = 0, x_pieces: bool = False, alpha: float = 1.0, limit: float = 0.0, up_shift: float = 0.0,

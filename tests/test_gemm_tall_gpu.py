@@ -1,0 +1,99 @@
+"""bf16 products of many rows in tiles, and the experts of a routed feed-forward over the rows that chose them."""
+import pytest
+import torch
+
+from hector_engine_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def rnd(*shape, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale).to(BF16)
+
+
+# fp32 sums of bf16 products in another order: a few ulp of 32 bits of the sum of magnitudes, then one rounding to bf16
+def near(got, want, size, bf16):
+    tol = 1e-6 * size + (2 ** -8 * want.abs() if bf16 else 0)
+    assert ((got.double().cpu() - want).abs() <= tol + 1e-30).all()
+
+
+@pytest.mark.parametrize("bm", [128, 256])
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (128, 256, 128), (127, 260, 192), (257, 516, 64), (300, 12, 320), (2200, 300, 64)])
+def test_products_in_tiles(bm, M, N, K):
+    x, w, b = rnd(M, K, seed=1), rnd(N, K, seed=2), rnd(N, seed=3)
+    want = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    out = torch.full((M + 1, N), 7.0, dtype=BF16, device="cuda")
+    ops.gemm_tall(out, x.cuda(), w.cuda(), b.cuda(), M, bm=bm)
+    near(out[:M], want + b.double(), size + b.double().abs(), True)
+    assert (out[M] == 7).all()
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    ops.gemm_tall(out, x.cuda(), w.cuda(), None, M, bm=bm)
+    near(out[:M], want, size, False)
+    assert (out[M] == 7).all()
+    for act in ((1.0, 0.0, 0.0, 0.0), (1.702, 2.0, 1.0, 0.0)):
+        out = torch.full((M + 1, N // 2), 7.0, dtype=BF16, device="cuda")
+        ops.gemm_tall(out, x.cuda(), w.cuda(), None, M, bm=bm, act=act)
+        g, u = want[:, 0::2], want[:, 1::2]
+        if act[1]:
+            g, u = g.clamp(max=act[1]), u.clamp(-act[1], act[1])
+        gated = g * torch.sigmoid(act[0] * g) * (u + act[2])
+        # the derivatives of the activation are at most 1.2 (|u| + 1) and |g| + 1
+        # and gate and up are rounded to bf16 before it
+        slack = 2 ** -8 * (want[:, 0::2].abs() * 1.2 * (u.abs() + 1) + want[:, 1::2].abs() * (g.abs() + 1))
+        got, bound = out[:M].double().cpu(), 1e-6 * (size[:, 0::2] * 1.2 * (u.abs() + 1) + size[:, 1::2] * (g.abs() + 1))
+        assert ((got - gated).abs() <= bound + slack + 2 ** -8 * gated.abs()).all()
+        assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("bm", [128, 256])
+@pytest.mark.parametrize("rows,real,identity,top", [(1, 3, 0, 1), (130, 5, 1, 2), (300, 16, 2, 4), (513, 1, 0, 1), (700, 40, 0, 8)])
+def test_experts_over_the_rows_that_chose_them(bm, rows, real, identity, top):
+    D, I = 128, 192
+    x = rnd(rows, D, seed=5)
+    gate_up, down = rnd(2 * real * I, D, seed=6, scale=0.2), rnd(D, real * I + (D if identity else 0), seed=7, scale=0.2)
+    g = torch.Generator().manual_seed(8)
+    ids = torch.stack([torch.randperm(real + identity, generator=g)[:top] for _ in range(rows)]).int()
+    ids[rows // 2:, 0] = 0 if real > 1 and top == 1 else ids[rows // 2:, 0]          # an expert with many rows, others with few
+    ids[0, top - 1] = -1                                                             # a choice that found nothing
+    weights = torch.rand(rows, top, generator=g)
+    weights[ids < 0] = 0
+    dense = torch.zeros(rows, real + 1)
+    for k in range(top):
+        for e in range(real):
+            dense[:, e] += weights[:, k] * (ids[:, k] == e)
+        dense[:, real] += weights[:, k] * (ids[:, k] >= real)
+    ints, slots = ops.routed_groups_sizes(rows, top, real, bm)
+    out = torch.full((rows, D), 7.0, dtype=BF16, device="cuda")
+    h = torch.full((slots, I), float("nan"), dtype=BF16, device="cuda")
+    ops.routed_groups(out, torch.full((ints,), -5, dtype=torch.int32, device="cuda"), h,
+                      torch.full((slots, D), float("nan"), device="cuda"), x.cuda(), gate_up.cuda(), down.cuda(), ids.cuda(),
+                      weights.cuda(), dense.cuda(), rows, real, I, bm=bm)
+    want, size = torch.zeros(rows, D, dtype=torch.float64), torch.zeros(rows, D, dtype=torch.float64)
+    for e in range(real):
+        gu = x.double() @ gate_up[2 * e * I:2 * (e + 1) * I].double().T
+        a = gu[:, 0::2] * torch.sigmoid(gu[:, 0::2]) * gu[:, 1::2] * dense[:, e:e + 1].double()
+        d = down[:, e * I:(e + 1) * I].double()
+        want += a @ d.T
+        size += a.abs() @ d.abs().T
+    if identity:
+        want += dense[:, real:].double() * x.double()
+        size += dense[:, real:].double() * x.double().abs()
+    # gates and ups are rounded to bf16 (which moves an activation by 2.2 times its rounding at most here), the activations and the result too
+    assert ((out.double().cpu() - want).abs() <= 2 ** -8 * 3.2 * size + 2 ** -8 * want.abs() + 1e-3).all()
+    if not identity:
+        # the activations alone, spread over the columns of all experts: what the second half read, zeros elsewhere
+        wide = torch.zeros(rows, real * I, dtype=BF16, device="cuda")
+        lists = torch.full((ints,), -5, dtype=torch.int32, device="cuda")
+        ops.routed_groups_act(wide, lists, x.cuda(), gate_up.cuda(), ids.cuda(), weights.cuda(), rows, real, I, bm=bm)
+        tile_rows = (real + 1 + 3) // 4 * 4
+        rows_of = lists[tile_rows:tile_rows + slots].cpu()
+        begin = lists[:real + 1].cpu()
+        for e in range(real):
+            for slot in range(int(begin[e]) * bm, int(begin[e + 1]) * bm):
+                if rows_of[slot] >= 0:
+                    assert torch.equal(wide[rows_of[slot], e * I:(e + 1) * I], h[slot])
+                    wide[rows_of[slot], e * I:(e + 1) * I] = 0
+        assert (wide == 0).all()
