@@ -13,7 +13,8 @@ registers:
                               are cut along K across workgroups and leave fp32 slices, which a
                               small kernel adds (into the result, or straight into the residual)
   bfloat16, M > 64         -> the library matrix product (the reference calls its BLAS
-                              library for every product: kernels/matmul_cublas.cu:240-277)
+                              library for every product: kernels/matmul_cublas.cu:240-277), or
+                              the tiles of kernels.ops.gemm_tall where they are faster (_tall, tall_gated)
   fp32 results (logits)    -> the MFMA kernels up to 64 rows, above that the library,
                               which writes fp32 from bf16 operands
 
@@ -67,6 +68,7 @@ class Linear:
         self.weight = weight
         self.bias = bias
         self.out_features, self.in_features = weight.shape
+        self.one_round_tiles = False        # set by a part: _tall's products may run in tiles of this library's own
         self._plans: dict[bool, tuple[int, int]] = {}
         self._chosen: dict[tuple, routes.Route] = {}     # (rows, activations, fast) -> route, for one version of the table
         self._chosen_version = -1
@@ -218,10 +220,25 @@ class Linear:
             slices //= 2
         return slices
 
+    def _tall(self, rows: int, x, out, out_dtype) -> bool:
+        """Whether a product of long K runs in tiles of 128 x 256 outputs (kernels.ops.gemm_tall): where these are one round on
+        the chip, at least 0.6 of it (2048 x 3584 x 18944 265 us, the library 354; 1536 rows 254, 275). Fewer tiles leave units
+        idle, and with more the library's choices are as good (kernel against kernel 0.8 to 1.3). Only where a part allows
+        it: the library adds some tiles of such a product in two halves, so 6 results in 10,000 differ in their last bit, which
+        a router over rows that no norm has evened out turns into other choices."""
+        N, K = self.weight.shape
+        if not (self.one_round_tiles and out_dtype == BF16 and K >= 8192 and K % 64 == 0 and N % 4 == 0 and x.is_contiguous() and out.is_contiguous()):
+            return False
+        tiles = -(-rows // 128) * -(-N // 256)
+        return 0.6 * 256 <= tiles <= 256
+
     def _library(self, x, bias, rows, out, out_dtype, ctx):
         """More than 64 rows: the library's product; it also writes fp32 results (the logits) from
         bf16 operands (the head of the Qwen2.5-7B shape at 64 rows: 217 us)."""
         w = self.weight
+        if self._tall(rows, x, out, out_dtype):
+            ops.gemm_tall(out, x, w, bias, rows, bm=128)
+            return out
         slices = self._library_slices(rows) if out_dtype == torch.bfloat16 and x.is_contiguous() else 1
         if slices > 1:
             N, K = w.shape
@@ -306,6 +323,20 @@ class Linear:
         partial = ctx.alloc((splits, rows, self.weight.shape[0]), torch.float32)
         ops.gemm_rows(None, partial, a, self.weight, None, rows, row_scale=scale, x_pieces=pieces)
         ops.silu_mul(out, partial, rows, True, splits, **act)
+
+    def tall_gated(self, rows: int, ctx: StepContext, x) -> int:
+        """The rows of a tile where the gated product of this many bf16 rows runs as one kernel (kernels.ops.gemm_tall), 0 where it
+        is the library's product and an activation kernel. Where the two were slower: K up to 1024 (9728 x 896: 128 rows 19 us
+        against 42, 2048 60 against 73, 12001 235 against 339; tiles of 128 rows up to 1024 rows) and 2048 to 3072 rows
+        (37888 x 3584: 2048 rows 499 us beside 560 + 40, 3072 707 beside 753; 1536 395 beside 357, and beyond 4096 the library's
+        product is as fast as this one)."""
+        N, K = self.weight.shape
+        if not (ctx.env.fast_kernels and rows > ops.ROWS_MAX_M and self.weight.dtype == BF16 and isinstance(x, torch.Tensor)
+                and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0):
+            return 0
+        if K <= 1024:
+            return 128 if rows <= 1024 else 256
+        return 256 if 2048 <= rows <= 3072 else 0
 
     def gated_pieces(self, rows: int) -> bool:
         """Whether gated_silu can write its result piece-major at this many rows."""

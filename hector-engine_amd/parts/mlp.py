@@ -75,6 +75,18 @@ class GatedMLP(FeedForward):
         self.gate_up = Linear(w.contiguous())
         del g, u, w
         self.down = Linear(tensors[n["down"]])
+        self.down.one_round_tiles = True
+
+    def _gate(self, h, x, rows: int, ctx: StepContext) -> None:
+        """h[rows, inter] = act(gate x, up x) of many rows: one kernel where the product takes the activation along."""
+        bm = self.gate_up.tall_gated(rows, ctx, x)
+        if bm:
+            a = self.act
+            ops.gemm_tall(h, x, self.gate_up.weight, None, rows, bm=bm,
+                          act=(a.get("alpha", 1.0), a.get("limit", 0.0), a.get("up_shift", 0.0), a.get("cubic", 0.0)))
+            return
+        gu = self.gate_up(x, rows, ctx)
+        ops.silu_mul(h, gu, rows, True, **self.act)
 
     def forward(self, x, ctx: StepContext):
         rows = ctx.rows
@@ -88,8 +100,7 @@ class GatedMLP(FeedForward):
                 self.gate_up.gated_silu(x, rows, ctx, h, out_pieces=pieces, act=self.act)
                 return self.down(PieceRows(h) if pieces else h, rows, ctx, sink=ctx.take_sink())
             h = ctx.alloc((rows, self.inter))
-            gu = self.gate_up(x, rows, ctx)
-            ops.silu_mul(h, gu, rows, True, **self.act)
+            self._gate(h, x.tensor(ctx) if isinstance(x, NormedRows) else x, rows, ctx)
             return self.down(h, rows, ctx, sink=ctx.take_sink())
         if not isinstance(x, torch.Tensor):
             x = x.tensor(ctx)
@@ -98,8 +109,7 @@ class GatedMLP(FeedForward):
             n = min(_ROW_CHUNK, rows - r0)
             turn = ctx.scratch.mark()
             h = ctx.alloc((n, self.inter))
-            gu = self.gate_up(x[r0:r0 + n], n, ctx)
-            ops.silu_mul(h, gu, n, True, **self.act)
+            self._gate(h, x[r0:r0 + n], n, ctx)
             self.down(h, n, ctx, out=out[r0:r0 + n])
             ctx.scratch.release(turn)       # the next turn reuses h and gate||up
         return out
