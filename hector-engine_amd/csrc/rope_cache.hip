@@ -491,7 +491,7 @@ extern "C" int he_qkv_rope_cache(void* q_out, void* kpool, void* vpool, const vo
     const int vec_threads = min(1024, max(64, (items + 63) / 64 * 64));
     // A row's own workgroup for its v in steps that may mix one-token sequences with a prompt: eight rows of one workgroup are a
     // chain of eight times three dependent loads where each begins a run (200 tokens beside seven one-token sequences, 7B shape:
-    // 25 us a launch with a workgroup per eight rows, the step of 28 layers 9.16 ms; 8.67 so); in a longer prompt a
+    // 25 us a launch with a workgroup per eight rows, 7.6 so; the step of 28 layers 9.16 ms, 8.67); in a longer prompt a
     // workgroup per eight rows is one run.
     const int v_span = rows <= 1024 ? 1 : 8;
     const int v_blocks = k_in ? (rows + v_span - 1) / v_span : 0;
