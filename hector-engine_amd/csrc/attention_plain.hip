@@ -68,7 +68,7 @@ __device__ __forceinline__ void ap_update(ApState<NPL>& st, float s, const float
   const float m_new = up ? s : st.m;
   const float e = expf(up ? st.m - s : s - st.m);
   const float alpha = up ? e : 1.f;
-  const float w = up ? 1.f : e;
+  const float w = up ? 1.f : s == -INFINITY ? 0.f : e;      // (also where no key had weight yet: there e is exp(-inf + inf))
   st.l = fmaf(st.l, alpha, w);
 #pragma unroll
   for (int i = 0; i < NPL; ++i) {
@@ -153,10 +153,11 @@ __device__ __forceinline__ void ap_page(ApState<NPL>& st, const float (&qv)[NPL]
   }
 }
 
-// total <- total joined with the result of the next page (one that had keys).
+// total <- total joined with the result of the next page (one that had keys). A page whose scores are all -inf has a sum of 0 and
+// is passed over; scores that are no numbers leave a sum that is none, which joins and stays visible.
 template <int NPL>
 __device__ __forceinline__ void ap_join(ApState<NPL>& total, const ApState<NPL>& st) {
-  if (!(st.m > -INFINITY) && st.l == 0.f) return;      // (scores that are no numbers leave a sum that is none)
+  if (!(st.m > -INFINITY) && st.l == 0.f) return;
   const float m_new = fmaxf(total.m, st.m);
   const float a = total.m > -INFINITY ? expf(total.m - m_new) : 0.f;
   const float b = expf(st.m - m_new);
@@ -186,7 +187,7 @@ __device__ __forceinline__ float ap_finish(ApState<NPL>& total, const ApExtras& 
   if (ex.sinks != nullptr) {
     ApState<NPL> sk;
     sk.m = load_param(ex.sinks, h, ex.sinks_dtype);
-    sk.l = 1.f;
+    sk.l = sk.m > -INFINITY ? 1.f : 0.f;         // a sink of -inf (or none that is a number) is passed over
 #pragma unroll
     for (int i = 0; i < NPL; ++i) sk.acc[i] = 0.f;
     ap_join(total, sk);
@@ -402,8 +403,10 @@ template <int KS>
 __device__ __forceinline__ void ap32_store(ApTile32<KS>& t, float* o, const ApExtras& ex, int64_t row, int h, int lane) {
   // the sink joins last; the gate scales what is stored
   float gf = 1.f, a = 1.f;
-  if (ex.sinks != nullptr) {
-    const float sink = load_param(ex.sinks, h, ex.sinks_dtype), m_new = fmaxf(t.m, sink);
+  const float sink = ex.sinks != nullptr ? load_param(ex.sinks, h, ex.sinks_dtype) : -INFINITY;
+  const bool sinks = sink > -INFINITY;            // (as ap_finish)
+  if (sinks) {
+    const float m_new = fmaxf(t.m, sink);
     a = t.m > -INFINITY ? expf(t.m - m_new) : 0.f;
     t.l = fmaf(t.l, a, expf(sink - m_new));
   }
@@ -414,7 +417,7 @@ __device__ __forceinline__ void ap32_store(ApTile32<KS>& t, float* o, const ApEx
     ap_f4 v = t.total[dt * HE_WAVE];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (ex.sinks != nullptr) v[i] = fmaf(v[i], a, 0.f);
+      if (sinks) v[i] = fmaf(v[i], a, 0.f);
       v[i] = ex.gate ? v[i] * inv * gf : v[i] * inv;
     }
     *reinterpret_cast<ap_f4*>(o + 16 * dt + 4 * (lane >> 4)) = v;
