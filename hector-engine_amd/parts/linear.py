@@ -87,6 +87,11 @@ class Linear:
             self._chosen[key] = route
         return route
 
+    def own_tiles(self, rows: int, ctx: StepContext, act: torch.dtype = BF16) -> bool:
+        """Whether a part may run this many rows through the tile kernels itself (kernels.ops.gemm_tall, routed_groups): where
+        the library's route would, so that a route registered in front of it still gets its products."""
+        return self._has("tiles", rows, ctx, act)
+
     def _has(self, trait: str, rows: int, ctx: StepContext, act: torch.dtype) -> bool:
         if not routes.routes_of("linear", (self.weight.dtype, act)):
             return False
@@ -331,8 +336,8 @@ class Linear:
         (37888 x 3584: 2048 rows 499 us beside 560 + 40, 3072 707 beside 753; 1536 395 beside 357, and beyond 4096 the library's
         product is as fast as this one)."""
         N, K = self.weight.shape
-        if not (ctx.env.fast_kernels and rows > ops.ROWS_MAX_M and self.weight.dtype == BF16 and isinstance(x, torch.Tensor)
-                and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0) or library_tuning.enabled():
+        if not (isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0
+                and self.own_tiles(rows, ctx)) or library_tuning.enabled():
             return 0             # (the library's tuned choice is faster still: 386 + 42 us at 2048 rows of 37888 x 3584)
         if K <= 1024:
             return 128 if rows <= 1024 else 256
@@ -351,6 +356,6 @@ def _mfma_takes(case: ProductCase) -> bool:
 routes.register_route("linear", (BF16, BF16), "mfma", _mfma_takes, Linear._run_mfma,
                       traits=("pieces", "gated", "k_slices"))
 routes.register_route("linear", (BF16, BF16), "plain", lambda c: not c.fast or c.K % 8 != 0, Linear._run_plain)
-routes.register_route("linear", (BF16, BF16), "library", lambda c: True, Linear._run_library)
+routes.register_route("linear", (BF16, BF16), "library", lambda c: True, Linear._run_library, traits=("tiles",))
 routes.register_route("linear", (F32, F32), "plain", lambda c: True, Linear._run_plain)
 routes.register_route("linear", (F32, BF16), "plain_widened", lambda c: True, Linear._run_plain_widened)

@@ -79,6 +79,8 @@ class GatedMLP(FeedForward):
 
     def _gate(self, h, x, rows: int, ctx: StepContext) -> None:
         """h[rows, inter] = act(gate x, up x) of many rows: one kernel where the product takes the activation along."""
+        if isinstance(x, NormedRows) and self.gate_up.own_tiles(rows, ctx, x.scaled.dtype):
+            x = x.tensor(ctx)
         bm = self.gate_up.tall_gated(rows, ctx, x)
         if bm:
             a = self.act
@@ -100,7 +102,7 @@ class GatedMLP(FeedForward):
                 self.gate_up.gated_silu(x, rows, ctx, h, out_pieces=pieces, act=self.act)
                 return self.down(PieceRows(h) if pieces else h, rows, ctx, sink=ctx.take_sink())
             h = ctx.alloc((rows, self.inter))
-            self._gate(h, x.tensor(ctx) if isinstance(x, NormedRows) else x, rows, ctx)
+            self._gate(h, x, rows, ctx)
             return self.down(h, rows, ctx, sink=ctx.take_sink())
         if not isinstance(x, torch.Tensor):
             x = x.tensor(ctx)

@@ -156,10 +156,11 @@ class RoutedExperts(FeedForward):
         that carry norms): an expert's tiles over its own rows are never more than over all rows, so the sorting is all
         that could cost. 16 experts of 2048 over rows of 2048, 4 chosen: 65 rows 196 -> 145 us, 512 330 -> 163, 2048 849 -> 228.
         Tiles of 256 rows from 112 rows an expert on (384 rows there: 144 us in tiles of 128, 160 of 256; 512: 181, 163)."""
-        if not (ctx.env.fast_kernels and ctx.env.dtype == torch.bfloat16 and isinstance(x, torch.Tensor) and rows > ops.ROWS_MAX_M
-                and self.gate_up.weight.dtype == torch.bfloat16 and not self.shared_cols and 2 * self.top <= self.real <= 1024
-                and self.inter % 64 == 0 and self.hidden % 64 == 0
-                and not (self.shared is not None and self.identity)):
+        turn = min(rows, _ROW_CHUNK)
+        if not (ctx.env.dtype == torch.bfloat16 and isinstance(x, torch.Tensor) and not self.shared_cols
+                and 2 * self.top <= self.real <= 1024 and self.inter % 64 == 0 and self.hidden % 64 == 0
+                and not (self.shared is not None and self.identity)
+                and self.gate_up.own_tiles(turn, ctx) and (self.shared is not None or self.down.own_tiles(turn, ctx))):
             return 0
         return 256 if rows * self.top >= 112 * self.real else 128
 
