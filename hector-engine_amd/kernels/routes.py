@@ -12,8 +12,7 @@ part is edited for it.
 
 ``dtypes`` is a tuple of torch dtypes whose meaning belongs to the operation ("linear":
 (weight, activations); "attention": (cache,)). ``traits`` are names a part may ask a route
-for without running it ("pieces": reads piece-major rows, "gated": has the gated epilogue, "tiles": a part may run such
-products through the tile kernels in its place).
+for without running it ("pieces": reads piece-major rows, "gated": has the gated epilogue).
 """
 from __future__ import annotations
 

@@ -90,7 +90,7 @@ class Linear:
     def own_tiles(self, rows: int, ctx: StepContext, act: torch.dtype = BF16) -> bool:
         """Whether a part may run this many rows through the tile kernels itself (kernels.ops.gemm_tall, routed_groups): where
         the library's route would, so that a route registered in front of it still gets its products."""
-        return self._has("tiles", rows, ctx, act)
+        return bool(routes.routes_of("linear", (self.weight.dtype, act))) and self.route(rows, ctx, act).run is Linear._run_library
 
     def _has(self, trait: str, rows: int, ctx: StepContext, act: torch.dtype) -> bool:
         if not routes.routes_of("linear", (self.weight.dtype, act)):
@@ -356,6 +356,6 @@ def _mfma_takes(case: ProductCase) -> bool:
 routes.register_route("linear", (BF16, BF16), "mfma", _mfma_takes, Linear._run_mfma,
                       traits=("pieces", "gated", "k_slices"))
 routes.register_route("linear", (BF16, BF16), "plain", lambda c: not c.fast or c.K % 8 != 0, Linear._run_plain)
-routes.register_route("linear", (BF16, BF16), "library", lambda c: True, Linear._run_library, traits=("tiles",))
+routes.register_route("linear", (BF16, BF16), "library", lambda c: True, Linear._run_library)
 routes.register_route("linear", (F32, F32), "plain", lambda c: True, Linear._run_plain)
 routes.register_route("linear", (F32, BF16), "plain_widened", lambda c: True, Linear._run_plain_widened)
