@@ -46,4 +46,6 @@ int he_cus() {
   return n;
 }
 
+extern "C" int he_compute_units(void) { return he_cus(); }
+
 extern "C" int he_abi_version(void) { return HE_ABI_VERSION; }

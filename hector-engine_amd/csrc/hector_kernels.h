@@ -13,6 +13,7 @@ extern "C" {
 #endif
 
 const char* he_last_error(void);
+int he_compute_units(void);      // of the current device
 int he_abi_version(void);
 
 // ---- weight preparation ----------------------------------------------------

@@ -1179,6 +1179,11 @@ def routed_act(out, gate_up, dense, h, rows: int, real: int, inter: int, *, shar
                                _stream()))
 
 
+def compute_units() -> int:
+    """Compute units of the current device: what the plans of grids count in."""
+    return int(_lib.load().he_compute_units())
+
+
 @_op("gemm_tall")
 def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
     """out[M, N] = x[M, K] . w[N, K]^T (+ bias) for many bf16 rows (bf16 or fp32 results); with act, the constants (alpha,

@@ -329,19 +329,26 @@ class Linear:
         ops.gemm_rows(None, partial, a, self.weight, None, rows, row_scale=scale, x_pieces=pieces)
         ops.silu_mul(out, partial, rows, True, splits, **act)
 
+    def _rounds(self, rows: int, bm: int) -> float:
+        """The tiles of bm x 256 outputs of this product, in rounds of the chip's units."""
+        return -(-rows // bm) * -(-self.weight.shape[0] // 256) / ops.compute_units()
+
     def tall_gated(self, rows: int, ctx: StepContext, x) -> int:
         """The rows of a tile where the gated product of this many bf16 rows runs as one kernel (kernels.ops.gemm_tall), 0 where it
-        is the library's product and an activation kernel. Where the two were slower: K up to 1024 (9728 x 896: 128 rows 19 us
-        against 42, 2048 60 against 73, 12001 235 against 339; tiles of 128 rows up to 1024 rows) and 2048 to 3072 rows
-        (37888 x 3584: 2048 rows 499 us beside 560 + 40, 3072 707 beside 753; 1536 395 beside 357, and beyond 4096 the library's
-        product is as fast as this one)."""
+        is the library's product and an activation kernel. One kernel for K up to 1024 where its tiles are one round on the
+        chip: of 128 rows from 0.6 of a round on, of 256 where those are more than a round and 0.7 of the round's outputs are
+        real. Over 220 random weights and row counts that this takes, 0.34 to 1.01 of the time of the two, 0.72 in the geometric mean
+        (8192 x 1024 at 1000 rows 24.8 us beside 28.1, 9728 x 896 at 768 rows 23.7 beside 27.0, at 1400 38.8 beside 40.3). With fewer
+        tiles units idle (1024 x 256 at 1000 rows 13.0, 9.1); with more, or a longer K, the two come out ahead as often as not,
+        by the library's choice of a kernel alone: over 420 random weights of K 1536 to 8192 and 1000 to 6000 rows the one
+        kernel took 0.66 to 1.31 of their time, in no relation to rows, columns or rounds."""
         N, K = self.weight.shape
-        if not (isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0
+        if not (K <= 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0
                 and self.own_tiles(rows, ctx)) or library_tuning.enabled():
-            return 0             # (the library's tuned choice is faster still: 386 + 42 us at 2048 rows of 37888 x 3584)
-        if K <= 1024:
-            return 128 if rows <= 1024 else 256
-        return 256 if 2048 <= rows <= 3072 else 0
+            return 0             # (a tuned choice of the library has not been measured against)
+        if self._rounds(rows, 128) <= 1:
+            return 128 if self._rounds(rows, 128) >= 0.6 else 0
+        return 256 if self._rounds(rows, 256) <= 1 and rows * N >= 0.7 * 256 * 256 * ops.compute_units() else 0
 
     def gated_pieces(self, rows: int) -> bool:
         """Whether gated_silu can write its result piece-major at this many rows."""

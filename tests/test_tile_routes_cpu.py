@@ -49,3 +49,15 @@ def test_a_registered_route_gets_the_experts_products_it_takes(N):
     assert part._many_rows(2048, x, CTX)
     with route_before_the_library(lambda c: c.N == N):
         assert not part._many_rows(2048, x, CTX)
+
+
+@pytest.mark.parametrize("N,K,tiles", [
+    (9728, 896, {65: 0, 512: 0, 513: 128, 768: 128, 769: 0, 1207: 0, 1208: 256, 1536: 256, 1537: 0, 2048: 0, 12001: 0}),
+    (8192, 1024, {512: 0, 640: 128, 1024: 128, 1025: 0, 1434: 256, 2048: 256, 2049: 0}),
+    (1024, 256, {1000: 0, 4096: 0, 4992: 128, 8192: 128}),                # a few columns of tiles: units idle below
+    (37888, 3584, {1024: 0, 1536: 0, 2048: 0, 2560: 0, 3072: 0}),         # a longer K: no relation to the sizes
+    (4096, 2048, {2048: 0, 4096: 0}), (9728, 880, {600: 0}), (9724, 896, {600: 0})])
+def test_which_gated_products_run_as_one_kernel(N, K, tiles):
+    """At 256 units: tiles of 128 rows from 0.6 to 1 round of the chip, of 256 above that up to a round with 0.7 of it real."""
+    lin = Linear(empty(N, K))
+    assert {rows: lin.tall_gated(rows, CTX, empty(rows, K)) for rows in tiles} == tiles
