@@ -226,16 +226,19 @@ class Linear:
         return slices
 
     def _tall(self, rows: int, x, out, out_dtype) -> bool:
-        """Whether a product of long K runs in tiles of 128 x 256 outputs (kernels.ops.gemm_tall): where these are one round on
-        the chip, at least 0.6 of it (2048 x 3584 x 18944 265 us, the library 354; 1536 rows 254, 275). Fewer tiles leave units
-        idle, and with more the library's choices are as good (kernel against kernel 0.8 to 1.3). Only where a part allows
-        it: the library adds some tiles of such a product in two halves, so 6 results in 10,000 differ in their last bit, which
-        a router over rows that no norm has evened out turns into other choices."""
+        """Whether a product of long K runs in tiles of 128 x 256 outputs (kernels.ops.gemm_tall): for K from 16448 to 27648, where
+        the library's default choice drops to 0.75 PFLOP/s (from 1.0 to 1.4 at shorter K), and tiles that are at most 0.94 of a
+        round on the chip, 0.72 of it real outputs. 2048 x 3584 x 18944 takes 256 us, the library 358; over 149 random products of
+        this range 0.55 to 1.07 of the library's time, 0.78 in the geometric mean. Fewer tiles leave units idle; beyond 0.94 the
+        library's choice is another one for some widths (3072 x 18944: the tiles take 1.09 of its time), and beyond K 27648 for others (8192 x
+        29568 1.24 of it). Up to K 16384 the tiles lost on nearly every width (4096 x 14336 at 1019 rows 197 us, 132). Only where a part
+        allows it: the library adds some tiles of such a product in two halves, so 6 results in 10,000 differ in their last bit,
+        which a router over rows that no norm has evened out turns into other choices."""
         N, K = self.weight.shape
-        if library_tuning.enabled() or not (self.one_round_tiles and out_dtype == BF16 and K >= 8192 and K % 64 == 0 and N % 4 == 0 and x.is_contiguous() and out.is_contiguous()):
+        if library_tuning.enabled() or not (self.one_round_tiles and out_dtype == BF16 and 16384 < K <= 27648 and K % 64 == 0
+                                            and N % 4 == 0 and x.is_contiguous() and out.is_contiguous()):
             return False
-        tiles = -(-rows // 128) * -(-N // 256)
-        return 0.6 * 256 <= tiles <= 256
+        return self._rounds(rows, 128) <= 0.94 and rows * N >= 0.72 * 128 * 256 * ops.compute_units()
 
     def _library(self, x, bias, rows, out, out_dtype, ctx):
         """More than 64 rows: the library's product; it also writes fp32 results (the logits) from

@@ -61,3 +61,17 @@ def test_which_gated_products_run_as_one_kernel(N, K, tiles):
     """At 256 units: tiles of 128 rows from 0.6 to 1 round of the chip, of 256 above that up to a round with 0.7 of it real."""
     lin = Linear(empty(N, K))
     assert {rows: lin.tall_gated(rows, CTX, empty(rows, K)) for rows in tiles} == tiles
+
+
+@pytest.mark.parametrize("N,K,rows", [
+    (3584, 18944, {1408: False, 1684: False, 1686: True, 2048: True, 2176: True, 2177: False}),
+    (5120, 27648, {1179: False, 1180: True, 1536: True, 1537: False}),
+    (8192, 29568, {768: False, 896: False, 1024: False}), (4096, 14336, {1664: False, 2048: False}), (2048, 8192, {4000: False}),
+    (3586, 18944, {2048: False}), (3584, 18912, {2048: False})])
+def test_which_products_of_long_k_run_in_tiles(N, K, rows):
+    """At 256 units: K from 16448 to 27648, at most 0.94 of a round of 128 x 256 tiles, 0.72 of one real."""
+    lin = Linear(empty(N, K))
+    assert not any(lin._tall(r, empty(r, K), empty(r, N), BF16) for r in rows)      # no part has allowed it
+    lin.one_round_tiles = True
+    assert {r: lin._tall(r, empty(r, K), empty(r, N), BF16) for r in rows} == rows
+    assert not any(lin._tall(r, empty(r, K), empty(r, N, dtype=torch.float32), torch.float32) for r in rows)
