@@ -139,6 +139,8 @@ class RoutedExperts(FeedForward):
         self.down = Linear(torch.cat(downs, 1).contiguous())
         if self.shared is not None and not self.shared_cols:
             self.shared.bind(tensors)
+            if isinstance(self.shared, GatedMLP):
+                self.shared.down.one_round_tiles = False      # (the router may read rows no norm has evened out)
         if self._shared_gate:
             self.shared_gate = tensors[self._shared_gate].reshape(-1).contiguous()
 

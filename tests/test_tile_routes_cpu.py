@@ -75,3 +75,16 @@ def test_which_products_of_long_k_run_in_tiles(N, K, rows):
     lin.one_round_tiles = True
     assert {r: lin._tall(r, empty(r, K), empty(r, N), BF16) for r in rows} == rows
     assert not any(lin._tall(r, empty(r, K), empty(r, N, dtype=torch.float32), torch.float32) for r in rows)
+
+
+def test_a_shared_expert_keeps_the_library_s_sums():
+    """A router over rows that no norm has evened out turns last bits into other choices: a feed-forward beside it stays out."""
+    def bound(kind, params):
+        part = build_part("feed_forward", PartSpec(kind, params), "m.", CTX.env)
+        part.bind({k: torch.zeros(v.shape, dtype=BF16) for k, v in part.tensor_specs().items()})
+        return part
+    mlp = {"hidden_size": 8, "intermediate_size": 16}
+    assert bound("gated_mlp", mlp).down.one_round_tiles
+    routed = bound("routed_experts", {**mlp, "experts": 4, "top": 2, "correction": False,
+                                      "shared": {"gate": "sg", "feed_forward": PartSpec("gated_mlp", mlp)}})
+    assert not routed.shared.down.one_round_tiles and not routed.down.one_round_tiles
