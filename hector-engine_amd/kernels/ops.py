@@ -1184,6 +1184,11 @@ def compute_units() -> int:
     return int(_lib.load().he_compute_units())
 
 
+def tiles_read(*tensors) -> bool:
+    """Whether the tile kernels (gemm_tall, routed_groups) read and write these where they lie: from 16-byte boundaries on."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 @_op("gemm_tall")
 def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
     """out[M, N] = x[M, K] . w[N, K]^T (+ bias) for many bf16 rows (bf16 or fp32 results); with act, the constants (alpha,

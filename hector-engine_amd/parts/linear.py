@@ -236,7 +236,8 @@ class Linear:
         which a router over rows that no norm has evened out turns into other choices."""
         N, K = self.weight.shape
         if library_tuning.enabled() or not (self.one_round_tiles and out_dtype == BF16 and 16384 < K <= 27648 and K % 64 == 0
-                                            and N % 4 == 0 and x.is_contiguous() and out.is_contiguous()):
+                                            and N % 4 == 0 and x.is_contiguous() and out.is_contiguous()
+                                            and ops.tiles_read(x, self.weight, out)):
             return False
         return self._rounds(rows, 128) <= 0.94 and rows * N >= 0.72 * 128 * 256 * ops.compute_units()
 
@@ -347,7 +348,7 @@ class Linear:
         kernel took 0.66 to 1.31 of their time, in no relation to rows, columns or rounds."""
         N, K = self.weight.shape
         if not (K <= 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0
-                and self.own_tiles(rows, ctx)) or library_tuning.enabled():
+                and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) or library_tuning.enabled():
             return 0             # (a tuned choice of the library has not been measured against)
         if self._rounds(rows, 128) <= 1:
             return 128 if self._rounds(rows, 128) >= 0.6 else 0

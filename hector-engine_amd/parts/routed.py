@@ -161,7 +161,9 @@ class RoutedExperts(FeedForward):
         turn = min(rows, _ROW_CHUNK)
         if not (ctx.env.dtype == torch.bfloat16 and isinstance(x, torch.Tensor) and not self.shared_cols
                 and 2 * self.top <= self.real <= 1024 and self.inter % 64 == 0 and self.hidden % 64 == 0
-                and not (self.shared is not None and self.identity)
+                and not (self.shared is not None and self.identity) and ops.tiles_read(x)
+                # (a lane's offsets into the rows and into 256 rows of a weight are 32-bit)
+                and 2 * max(turn * self.hidden, 256 * (self.real * self.inter + self.hidden)) < 1 << 32
                 and self.gate_up.own_tiles(turn, ctx) and (self.shared is not None or self.down.own_tiles(turn, ctx))):
             return 0
         return 256 if rows * self.top >= 112 * self.real else 128

@@ -1,5 +1,6 @@
 """Which products of many rows run through the tile kernels: the rules alone, over tensors without storage."""
 import contextlib
+import math
 from types import SimpleNamespace
 
 import pytest
@@ -88,3 +89,22 @@ def test_a_shared_expert_keeps_the_library_s_sums():
     routed = bound("routed_experts", {**mlp, "experts": 4, "top": 2, "correction": False,
                                       "shared": {"gate": "sg", "feed_forward": PartSpec("gated_mlp", mlp)}})
     assert not routed.shared.down.one_round_tiles and not routed.down.one_round_tiles
+
+
+def test_operands_the_tiles_do_not_read_stay_with_the_library():
+    def shifted(*shape):
+        return torch.empty(math.prod(shape) + 1, dtype=BF16)[1:].view(shape)
+    for w, x in ((shifted(9728, 896), empty(600, 896)), (empty(9728, 896), shifted(600, 896))):
+        assert Linear(w).tall_gated(600, CTX, x) == 0
+    N, K, rows = 384, 16448, 12000
+    for w, x, out in ((shifted(N, K), empty(rows, K), empty(rows, N)), (empty(N, K), empty(rows, K), shifted(rows, N)),
+                      (empty(N, K), empty(rows, K), empty(rows, N))):
+        lin = Linear(w)
+        lin.one_round_tiles = True
+        assert lin._tall(rows, x, out, BF16) == (w.is_meta and out.is_meta)
+    assert not experts()._many_rows(300, shifted(300, 2048), CTX)
+
+
+def test_experts_beyond_the_tiles_offsets_stay_with_the_product_over_all():
+    assert experts(real=512, inter=16320, hidden=64)._many_rows(4000, empty(4000, 64), CTX)
+    assert not experts(real=512, inter=16384, hidden=64)._many_rows(4000, empty(4000, 64), CTX)
