@@ -96,7 +96,7 @@ def test_operands_the_tiles_do_not_read_stay_with_the_library():
         return torch.empty(math.prod(shape) + 1, dtype=BF16)[1:].view(shape)
     for w, x in ((shifted(9728, 896), empty(600, 896)), (empty(9728, 896), shifted(600, 896))):
         assert Linear(w).tall_gated(600, CTX, x) == 0
-    N, K, rows = 384, 16448, 12000
+    N, K, rows = 512, 16448, 12000
     for w, x, out in ((shifted(N, K), empty(rows, K), empty(rows, N)), (empty(N, K), empty(rows, K), shifted(rows, N)),
                       (empty(N, K), empty(rows, K), empty(rows, N))):
         lin = Linear(w)
