@@ -141,6 +141,7 @@ int he_qkv_rope_cache(void* q_out, void* kpool, void* vpool, const void* q_in, c
                       int H, int KVH, int hd, int hd_in, int vd_in, int interleaved, float mscale,
                       float q_coef, int q_every, int unit, float unit_eps, const void* v_first,
                       int64_t v_stride, float v_lambda, int dtype, void* stream);
+int he_rope_value_rows(int rows, int v_cols);      // rows of v a workgroup of that launch takes
 // unit: every head of q and k is divided by sqrt(mean(x^2) + unit_eps) as well (bias and rotation as before). v_first
 // (rows of KVH * vd_in values, v_stride elements apart, or null): v <- (1 - v_lambda) v + v_lambda v_first.
 // hd: head size of q_out and of the cache pages. hd_in, vd_in (0: hd): head sizes of the q/k rows and

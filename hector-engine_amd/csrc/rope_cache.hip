@@ -189,7 +189,7 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// grid: one workgroup per 8 rows (per row in a step of up to 1024 rows) for v, then one per row for q and k.
+// grid: one workgroup per 8 rows (or per row: he_rope_value_rows) for v, then one per row for q and k.
 // V lies transposed in a page (8 keys of one dim are 16 contiguous bytes), so the v values of
 // a run of tokens that share such a group are gathered dim by dim and stored together: 16
 // bytes a store when the run is a whole group (a prompt), 2 bytes a token otherwise.
@@ -432,6 +432,16 @@ __global__ __launch_bounds__(1024) void qkv_rope_cache_vec_kernel(
   }
 }
 
+// Rows whose v a workgroup of the launch above takes. One in steps that may mix one-token sequences with a prompt: eight rows of one
+// workgroup are a chain of eight times three dependent loads where each begins a run (200 tokens beside seven one-token
+// sequences, 7B shape: 25 us a launch with a workgroup per eight rows, 7.6 so). In a prompt seven of eight such workgroups find no
+// run of theirs and leave, which costs more than the shorter chain gives once there are many, and large ones: one prompt of 512
+// rows of 512 columns 7.0 us by eight, 6.6 by one, of 768 rows 7.6 and 8.1, of 400 rows of 1024 columns 7.9 and 8.4,
+// of 1000 10.4 and 17.7.
+extern "C" int he_rope_value_rows(int rows, int v_cols) {
+  return rows <= 128 || (rows <= 1024 && (int64_t)rows * v_cols <= 262144) ? 1 : 8;
+}
+
 extern "C" int he_qkv_rope_cache(void* q_out, void* kpool, void* vpool, const void* q_in,
                                  const void* k_in, const void* v_in, int64_t in_stride,
                                  const void* q_bias, const void* k_bias, const void* v_bias,
@@ -489,11 +499,7 @@ extern "C" int he_qkv_rope_cache(void* q_out, void* kpool, void* vpool, const vo
     const int items = H * (rot8 + ((hd - rotary_dim) >> 3)) + (k_in ? KVH * (rot8 + ((hd_in - rotary_dim) >> 3)) : 0);
     HE_REQUIRE(!unit || items <= 12288, "he_qkv_rope_cache: %d heads are too many to norm", H + KVH);
     const int vec_threads = min(1024, max(64, (items + 63) / 64 * 64));
-    // A row's own workgroup for its v in steps that may mix one-token sequences with a prompt: eight rows of one workgroup are a
-    // chain of eight times three dependent loads where each begins a run (200 tokens beside seven one-token sequences, 7B shape:
-    // 25 us a launch with a workgroup per eight rows, 7.6 so; the step of 28 layers 9.16 ms, 8.67); in a longer prompt a
-    // workgroup per eight rows is one run.
-    const int v_span = rows <= 1024 ? 1 : 8;
+    const int v_span = he_rope_value_rows(rows, KVH * vd_in);
     const int v_blocks = k_in ? (rows + v_span - 1) / v_span : 0;
     qkv_rope_cache_vec_kernel<<<rows + v_blocks, vec_threads, unit ? sizeof(float) * items : 0, s>>>(
         (uint16_t*)q_out, (uint16_t*)kpool, (uint16_t*)vpool, (const uint16_t*)q_in,

@@ -54,6 +54,7 @@ _SIGNATURES = {
     "he_splitk_reduce_residual_blocks": [c_int],
     "he_splitk_reduce_residual": [c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_int, c_ptr, c_ptr, c_int, c_int, c_int,
                                   c_int, c_int, c_f32, c_ptr, c_ptr, c_ptr],
+    "he_rope_value_rows": [c_int, c_int],
     "he_qkv_rope_cache": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr,
                           c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_ptr, c_int, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_f32, c_f32, c_int, c_int, c_f32, c_ptr, c_i64, c_f32, c_int,

@@ -164,3 +164,13 @@ def test_profiler_reads_its_oldest_events_on_the_way(monkeypatch):
         assert len(prof._pending) < 8
     rows = {name: (calls, ms) for name, calls, ms, _, _ in prof.rows()}
     assert rows == {"a": (15, 7.5), "b": (15, 7.5)} and prof._pending == []
+
+
+def test_how_many_rows_of_v_a_workgroup_of_the_rotation_takes():
+    """One up to 128 rows, and up to 1024 where the step has at most 262,144 values; else eight."""
+    from hector_engine_amd.kernels import lib
+    rows_of = lib.load().he_rope_value_rows
+    taken = {(rows, cols): rows_of(rows, cols) for rows, cols in (
+        (1, 4096), (128, 4096), (129, 1024), (256, 1024), (257, 1024), (512, 512), (768, 512), (1000, 1024), (1024, 128), (1025, 128))}
+    assert taken == {(1, 4096): 1, (128, 4096): 1, (129, 1024): 1, (256, 1024): 1, (257, 1024): 8, (512, 512): 1, (768, 512): 8,
+                     (1000, 1024): 8, (1024, 128): 1, (1025, 128): 8}
