@@ -11,7 +11,7 @@
 //   mfma    fp32 operands, many rows: tiles of up to 128 x 128 outputs on the matrix cores;
 //   stream  fp32 operands, up to 64 rows, K in whole segments: matrix cores, a workgroup per 16 weight rows;
 //   tiles   bf16 operands: 64 x 64 outputs a workgroup, staged through LDS, every thread 4 x 4 outputs;
-//   rows    what the other two do not take of up to GP_ROWS_MAX_M rows: a thread owns one weight
+//   rows    up to GP_ROWS_MAX_M rows that stream does not take (gp_streams), with a workspace: a thread owns one weight
 //           row and one segment and walks it with all M activation rows at once, so a product
 //           has N * ceil(K / GP_SEG) threads however few its rows are; the segment sums go
 //           to a workspace and a second kernel adds them in order.
@@ -406,6 +406,83 @@ __global__ __launch_bounds__(256) void gemm_plain_rows_kernel(
   }
 }
 
+// The same sums for 32-bit weights whose K is whole segments, with the weights fetched line by
+// line: in the kernel above the 64 lanes of a load touch 64 cache lines (each lane its own row), and
+// the rate at which a compute unit looks lines up bounds it (3.6 TB/s at the Qwen2.5-7B shape). Here
+// eight neighbouring lanes fetch the 128 bytes of one row, a load touches eight lines, and the
+// wavefront turns the tile round in LDS: 32 k of its 64 rows at a time (two such chunks on their
+// way while one is multiplied), the values go into the wavefront's own LDS region as
+// [16-byte piece][row, 65 to a piece][4], from which lane n reads the pieces of row n one after the
+// other (a read of 64 lanes is one KiB on end) and extends its chain of FMAs in ascending k. The
+// region is the wavefront's own: LDS runs a wavefront's writes and reads in program order, so no
+// barrier is needed, and the compiler keeps stores and loads that may name the same address in
+// order. (A wavefront-scope fence here kept the staging registers in scratch memory.) grid and
+// block as above.
+#define GP_TURN_ROWS 65
+template <int MT>
+__global__ __launch_bounds__(256) void gemm_plain_rows_turned_kernel(
+    float* __restrict__ partial, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K,
+    int64_t lda, int64_t ldw, int segments) {
+  __shared__ float4 turned[4][8 * GP_TURN_ROWS];
+  const int lane = threadIdx.x;
+  const int n0 = blockIdx.x * 64;
+  const int seg = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + threadIdx.y);
+  if (seg >= segments) return;
+  const int k_begin = seg * GP_SEG;
+  // load i of a chunk of 32 k: row 8 i + lane / 8 of the tile, piece lane % 8 of its 128 bytes
+  const int lrow = lane >> 3, piece = lane & 7;
+  const float* src[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) src[i] = W + (int64_t)min(n0 + 8 * i + lrow, N - 1) * ldw + k_begin + 4 * piece;
+  float4 w0[8], w1[8];   // two chunks of 32 k on their way while a third is multiplied
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w0[i] = *reinterpret_cast<const float4*>(src[i]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w1[i] = *reinterpret_cast<const float4*>(src[i] + 32);
+  float acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = 0.f;
+  const float* arow[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) arow[m] = A + (int64_t)min(m, M - 1) * lda + k_begin;
+  float4* mine = turned[threadIdx.y];
+#define GP_TURN(WV_, C_)                                                                          \
+  {                                                                                               \
+    _Pragma("unroll") for (int i = 0; i < 8; ++i) mine[piece * GP_TURN_ROWS + 8 * i + lrow] = WV_[i]; \
+    __builtin_amdgcn_wave_barrier();                                                              \
+    _Pragma("unroll") for (int p = 0; p < 8; ++p) {                                               \
+      const float4 w4 = mine[p * GP_TURN_ROWS + lane];                                            \
+      const float w[4] = {w4.x, w4.y, w4.z, w4.w};                                                \
+      _Pragma("unroll") for (int e = 0; e < 4; ++e)                                               \
+        _Pragma("unroll") for (int m = 0; m < MT; ++m)                                            \
+          acc[m] = fmaf(arow[m][32 * (C_) + 4 * p + e], w[e], acc[m]);                            \
+    }                                                                                             \
+    __builtin_amdgcn_wave_barrier();                                                              \
+  }
+  // (the scheduler would ask for all four chunks at once and then spill two of them: each
+  // sched_barrier keeps a group of loads where it is written)
+  __builtin_amdgcn_sched_barrier(0);
+  GP_TURN(w0, 0)
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w0[i] = *reinterpret_cast<const float4*>(src[i] + 64);
+  __builtin_amdgcn_sched_barrier(0);
+  GP_TURN(w1, 1)
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w1[i] = *reinterpret_cast<const float4*>(src[i] + 96);
+  __builtin_amdgcn_sched_barrier(0);
+  GP_TURN(w0, 2)
+  GP_TURN(w1, 3)
+#undef GP_TURN
+  const int n = n0 + lane;
+  if (n < N) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      if (m < M) partial[((int64_t)seg * M + m) * N + n] = acc[m];
+  }
+}
+
 template <typename TC>
 __global__ __launch_bounds__(256) void gemm_plain_rows_sum_kernel(
     TC* __restrict__ C, const float* __restrict__ partial, const void* __restrict__ bias, int bias_dtype,
@@ -426,10 +503,30 @@ __global__ __launch_bounds__(256) void gemm_plain_rows_sum_kernel(
   C[(int64_t)m * ldc + n] = from_float<TC>(total);
 }
 
-// Floats of workspace with which a product of M rows runs through the kernels for few rows (0: it
-// runs through the tile kernel, which needs none).
-extern "C" int64_t he_gemm_plain_workspace_floats(int M, int N, int K) {
+// Whether a 32-bit product runs through the streaming kernel: up to GP_MROWS_MAX_M rows, and up to twice as many where tiles of 64 x 64
+// would leave half of the units idle (3584 x 18944 at 128 rows: 458 us in tiles, 4608 x 3584, whose tiles fill the chip, 86);
+// weights of whole segments in aligned rows. Its workgroups are 16 weight rows and its wavefronts a segment each, so it is
+// left where these do not fill the chip. K in few segments against many weight rows, whose wavefronts mostly idle: up to 8
+// rows the rows kernel (32000 x 256 at 1 row 10.4 us, streamed 14.0; 65536 x 128 at 8 rows 19.8, 22.1), above that tiles
+// (151936 x 128 at 64 rows 44, 182; 16384 x 512 at 64 rows 20, 28; but 16384 x 256 at 16 rows 11.6, 8.6, and 8192 x 256
+// at 64 even). Long K against few weight rows, a unit's own rate of about 30 bytes a ns: the rows kernel (512 x 12288
+// at 1 row 13.6, 26.6, at 8 rows 20, 29; 1024 x 4864 at 4 rows 13.5, 14.1; 2048 x 8192 at 1 row 20.1, 22.7, at 4 rows 23.8, 22.2).
+static bool gp_streams(int M, int N, int K, bool aligned) {
+  const int segments = K / GP_SEG, cus = he_cus();
+  if (!aligned || K % GP_SEG != 0) return false;
+  if (M > GP_MROWS_MAX_M) return M <= 2 * GP_MROWS_MAX_M && 4 * ((N + 63) / 64) <= cus;
+  if (segments <= (M + 15) / 16 && N >= (M <= 16 ? 96 : 64) * cus) return false;
+  if (M > GP_ROWS_MAX_M) return true;
+  if (segments <= 4 && N >= 96 * cus) return M > 4 && M * segments > (N >= 192 * cus ? 16 : 8);
+  if (segments >= 24 && N <= 4 * cus) return 4 * M > segments - 16;
+  return segments < 24 || N > 8 * cus || M > 2;
+}
+
+// Floats of workspace with which a product of M rows runs through the kernels for few rows (0: another kernel takes it, which
+// needs none). in_dtype, out_dtype below 0: the most that any operands of these sizes take.
+extern "C" int64_t he_gemm_plain_workspace_floats(int M, int N, int K, int in_dtype, int out_dtype, int aligned) {
   if (M <= 0 || M > GP_ROWS_MAX_M || N <= 0 || K <= 0) return 0;
+  if (in_dtype == HE_F32 && out_dtype == HE_F32 && gp_streams(M, N, K, aligned != 0)) return 0;
   return (int64_t)((K + GP_SEG - 1) / GP_SEG) * M * N;
 }
 
@@ -439,9 +536,16 @@ static int launch_rows(void* C, const void* A, const void* W, const void* bias, 
   const int segments = (K + GP_SEG - 1) / GP_SEG;
   dim3 grid((N + 63) / 64, (segments + 3) / 4), block(64, 4);
   HE_REQUIRE(grid.y <= 65535, "he_gemm_plain: K=%d too long for one launch", K);
+  // 32-bit weights in whole segments, rows 16-byte aligned: fetched line by line and turned round in LDS
+  constexpr bool f32 = sizeof(TA) == 4 && sizeof(TW) == 4;
+  const bool turned = f32 && K % GP_SEG == 0 && (ldw & 3) == 0 && (((uintptr_t)W) & 15) == 0;
 #define GP_ROWS(MT_)                                                                                  \
-  gemm_plain_rows_kernel<MT_, TA, TW><<<grid, block, 0, s>>>(ws, (const TA*)A, (const TW*)W, M, N, K, \
-                                                             lda, ldw, segments)
+  if (turned)                                                                                         \
+    gemm_plain_rows_turned_kernel<MT_><<<grid, block, 0, s>>>(ws, (const float*)A, (const float*)W, M, N, K, \
+                                                              lda, ldw, segments);                    \
+  else                                                                                                \
+    gemm_plain_rows_kernel<MT_, TA, TW><<<grid, block, 0, s>>>(ws, (const TA*)A, (const TW*)W, M, N, K, \
+                                                               lda, ldw, segments)
   if (M == 1) GP_ROWS(1);
   else if (M == 2) GP_ROWS(2);
   else if (M <= 4) GP_ROWS(4);
@@ -454,8 +558,7 @@ static int launch_rows(void* C, const void* A, const void* W, const void* bias, 
   return he_check_launch("he_gemm_plain");
 }
 
-// The kernel that streams the weights: up to GP_MROWS_MAX_M rows, and up to twice as many where tiles of 64 x 64 would
-// leave half of the units idle (3584 x 18944 at 128 rows: 458 us in tiles, 4608 x 3584, whose tiles fill the chip, 86). 16 wavefronts a workgroup where the weight's rows
+// The kernel that streams the weights. 16 wavefronts a workgroup where the weight's rows
 // give a compute unit one workgroup or less, else 8 (two workgroups share a unit).
 static int launch_stream(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K,
                          int64_t lda, int64_t ldw, int64_t ldc, hipStream_t s) {
@@ -497,8 +600,8 @@ static int launch_mfma(float* C, const float* A, const float* W, const void* bia
   return he_check_launch("he_gemm_plain");
 }
 
-// workspace_f32 (may be null) of workspace_floats floats: with he_gemm_plain_workspace_floats(M, N, K)
-// or more of them a product of few rows whose weight the streaming kernel does not take runs through the
+// workspace_f32 (may be null) of workspace_floats floats: with as many as he_gemm_plain_workspace_floats names for
+// these operands, or more, a product of few rows that is not streamed runs through the
 // kernels made for it. The result is the same bit for bit either way.
 extern "C" int he_gemm_plain(void* C, const void* A, const void* W, const void* bias, int M, int N,
                              int K, int64_t lda, int64_t ldw, int64_t ldc, int in_dtype,
@@ -509,11 +612,10 @@ extern "C" int he_gemm_plain(void* C, const void* A, const void* W, const void* 
   if (M == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool f32 = in_dtype == HE_F32 && out_dtype == HE_F32;
-  const bool few = M <= GP_MROWS_MAX_M || (M <= 2 * GP_MROWS_MAX_M && 4 * ((N + 63) / 64) <= he_cus());
-  if (f32 && few && K % GP_SEG == 0 && (lda & 3) == 0 && (ldw & 3) == 0 && (((uintptr_t)A) & 15) == 0 &&
-      (((uintptr_t)W) & 15) == 0)
+  const bool aligned = (lda & 3) == 0 && (ldw & 3) == 0 && (((uintptr_t)A) & 15) == 0 && (((uintptr_t)W) & 15) == 0;
+  if (f32 && gp_streams(M, N, K, aligned))
     return launch_stream((float*)C, (const float*)A, (const float*)W, bias, bias_dtype, M, N, K, lda, ldw, ldc, s);
-  const int64_t need = he_gemm_plain_workspace_floats(M, N, K);
+  const int64_t need = he_gemm_plain_workspace_floats(M, N, K, in_dtype, out_dtype, aligned);
   if (need > 0 && workspace_f32 != nullptr && workspace_floats >= need) {
     float* ws = (float*)workspace_f32;
     if (in_dtype == HE_F32 && out_dtype == HE_F32)

@@ -65,10 +65,11 @@ int he_rmsnorm_row_pair(void* x, const void* w1, int D1, const void* w2, int D2,
 
 // ---- matrix products: C[M,N] = A[M,K] * W[N,K]^T (+ bias) -------------------
 // he_gemm_plain: fp32 FMA sums in one fixed order per element (segments of 128 k, each a chain in
-// ascending k, added in segment order). With a workspace of he_gemm_plain_workspace_floats(M, N, K)
-// floats (0 for more than 8 rows) a product of few rows runs through kernels made for it; the
-// result is the same bit for bit.
-int64_t he_gemm_plain_workspace_floats(int M, int N, int K);
+// ascending k, added in segment order). With a workspace of he_gemm_plain_workspace_floats
+// floats (0 for more than 8 rows, and where a kernel that needs none takes these operands; aligned: rows of A and W begin
+// at 16 bytes) a product of few rows runs through kernels made for it; the
+// result is the same bit for bit. in_dtype, out_dtype < 0: the most that any operands take.
+int64_t he_gemm_plain_workspace_floats(int M, int N, int K, int in_dtype, int out_dtype, int aligned);
 int he_gemm_plain(void* C, const void* A, const void* W, const void* bias, int M, int N, int K,
                   int64_t lda, int64_t ldw, int64_t ldc, int in_dtype, int out_dtype,
                   int bias_dtype, void* workspace_f32, int64_t workspace_floats, void* stream);

@@ -234,16 +234,20 @@ def rmsnorm_row_pair(x, w1, D1: int, w2, D2: int, col2: int, rows: int, eps: flo
                                      float(eps), dtype_code(x.dtype), dtype_code(w1.dtype), _stream()))
 
 
-def gemm_plain_workspace_floats(M: int, N: int, K: int) -> int:
+def gemm_plain_workspace_floats(M: int, N: int, K: int, *, a=None, w=None, out=None) -> int:
     """Floats of workspace with which gemm_plain runs a product of few rows through the kernels made
-    for it (0: none needed)."""
-    return int(_lib.load().he_gemm_plain_workspace_floats(M, N, K))
+    for it. Without the operands: the most that any of these sizes take; with them: 0 also where a kernel that needs none
+    takes them (most 32-bit products)."""
+    if a is None:
+        return int(_lib.load().he_gemm_plain_workspace_floats(M, N, K, -1, -1, 0))
+    aligned = K % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    return int(_lib.load().he_gemm_plain_workspace_floats(M, N, K, dtype_code(a.dtype), dtype_code(out.dtype), int(aligned)))
 
 
 @_op("gemm_plain")
 def gemm_plain(out, a, w, bias, M: int, workspace=None) -> None:
     """out[M,N] = a[M,K] . w[N,K]^T (+ bias), fixed summation order. workspace: fp32, of
-    gemm_plain_workspace_floats(M, N, K) elements or more, for a product of few rows (the result
+    gemm_plain_workspace_floats(M, N, K, a=a, w=w, out=out) elements or more, for a product of few rows (the result
     is the same bit for bit without it, and slower)."""
     N, K = w.shape
     _need(a, "a")

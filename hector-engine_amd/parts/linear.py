@@ -201,9 +201,8 @@ class Linear:
         return self._library(x, bias, rows, out, out_dtype, ctx)
 
     def _plain(self, out, x, bias, rows: int, ctx: StepContext) -> None:
-        """The plain product (fixed summation order); with few rows through its kernels for them,
-        which want a workspace for their segment sums."""
-        floats = ops.gemm_plain_workspace_floats(rows, *self.weight.shape)
+        """The plain product (fixed summation order); some products of few rows want a workspace for their segment sums."""
+        floats = ops.gemm_plain_workspace_floats(rows, *self.weight.shape, a=x, w=self.weight, out=out)
         ws = ctx.alloc((floats,), torch.float32) if floats else None
         ops.gemm_plain(out, x, self.weight, bias, rows, workspace=ws)
 

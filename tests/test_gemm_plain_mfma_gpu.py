@@ -62,3 +62,16 @@ def test_what_is_not_finite_stays_in_its_row_and_column():
         out = torch.empty(M, 40, device="cuda")
         ops.gemm_plain(out, a[:M], w, None, M)
         assert torch.equal(out.isnan(), want[:M].isnan()) and torch.equal(out.nan_to_num(1.0, 2.0, 3.0), want[:M].nan_to_num(1.0, 2.0, 3.0))
+
+
+@pytest.mark.parametrize("M", [1, 3, 4, 8, 9, 33, 64])
+@pytest.mark.parametrize("N,K", [(24580, 128), (24576, 256), (16400, 512), (300, 3072), (1500, 4096)])
+def test_few_segments_and_few_weight_rows_give_the_same_bits_with_and_without_a_workspace(M, N, K):
+    a, w, bias = operands(M, N, K, M + N + K)
+    want = by_fma(a, w, bias)
+    out = torch.full((M, N), 7.0, device="cuda")
+    floats = ops.gemm_plain_workspace_floats(M, N, K, a=a, w=w, out=out)
+    for workspace in ({None, floats} if floats else {None}):
+        out.fill_(7.0)
+        ops.gemm_plain(out, a, w, bias, M, workspace=workspace and torch.full((workspace,), float("nan"), device="cuda"))
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))

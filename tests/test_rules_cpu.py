@@ -174,3 +174,26 @@ def test_how_many_rows_of_v_a_workgroup_of_the_rotation_takes():
         (1, 4096), (128, 4096), (129, 1024), (256, 1024), (257, 1024), (512, 512), (768, 512), (1000, 1024), (1024, 128), (1025, 128))}
     assert taken == {(1, 4096): 1, (128, 4096): 1, (129, 1024): 1, (256, 1024): 1, (257, 1024): 8, (512, 512): 1, (768, 512): 8,
                      (1000, 1024): 8, (1024, 128): 1, (1025, 128): 8}
+
+
+def test_which_products_of_few_rows_want_a_workspace():
+    """At 256 units: 32-bit products are streamed without one, but for K in few segments of 128 against many weight rows and for a
+    long K against few; bfloat16, other K and unaligned weights go by segments and want one up to 8 rows."""
+    from hector_engine_amd.kernels import ops
+
+    def wants(M, N, K, dtype=torch.float32, shift=0):
+        a, out = (torch.empty(s, dtype=dtype, device="meta") for s in ((M, K), (M, N)))
+        w = torch.empty(8 * K + shift, dtype=dtype)[shift:].view(8, K) if shift else torch.empty(N, K, dtype=dtype, device="meta")
+        floats = ops.gemm_plain_workspace_floats(M, N, K, a=a, w=w, out=out)
+        assert floats in (0, -(-K // 128) * M * N)
+        return floats > 0
+    assert not any(wants(M, N, K) for M in (1, 8) for N, K in ((152064, 3584), (37888, 3584), (4608, 3584), (3584, 18944), (1152, 896), (4096, 128)))
+    assert [M for M in range(1, 10) if wants(M, 32000, 128)] == list(range(1, 9))
+    assert [M for M in range(1, 10) if wants(M, 32000, 256)] == [1, 2, 3, 4]
+    assert [M for M in range(1, 10) if wants(M, 32000, 512)] == [1, 2, 3, 4]
+    assert [M for M in range(1, 10) if wants(M, 65536, 256)] == list(range(1, 9))
+    assert [M for M in range(1, 10) if wants(M, 32000, 640)] == []
+    assert [M for M in range(1, 10) if wants(M, 896, 4864)] == [1, 2, 3, 4, 5]
+    assert [M for M in range(1, 10) if wants(M, 512, 12288)] == list(range(1, 9))
+    assert [M for M in range(1, 10) if wants(M, 2048, 8192)] == [1, 2] and not wants(1, 2049, 8192)
+    assert wants(8, 37888, 3584, torch.bfloat16) and wants(8, 100, 1000) and not wants(9, 100, 1000) and wants(8, 8, 256, shift=1)
