@@ -297,6 +297,24 @@ __device__ __forceinline__ void ap32_page(ApTile32<KS>& t, ApPage32<KS>& pg, con
     if (NEXT) ap32_fetch_v<KS>(pg, vpage, h, lane);
     __builtin_amdgcn_sched_barrier(0);
   }
+  if (SHAPED) {      // (as ap_shape, a kind at a time and a score at a time: what all of them would need at once does not fit the registers)
+#define AP32_EACH(V_, ...)                                               \
+  _Pragma("unroll") for (int h = 0; h < 2; ++h)                          \
+      _Pragma("unroll") for (int x = 0; x < 2; ++x)                      \
+          _Pragma("unroll") for (int i = 0; i < 4; ++i) {                \
+    const int back = t.p - (j0 + 32 * h + 8 * g + 4 * x + i);            \
+    (void)back;                                                          \
+    float V_ = s[h][x][i];                                               \
+    __VA_ARGS__;                                                         \
+    s[h][x][i] = V_;                                                     \
+    __builtin_amdgcn_sched_barrier(0);                                   \
+  }
+    AP32_EACH(v, v = v * scale)
+    if (t.sh.cap > 0.f) AP32_EACH(v, v = t.sh.cap * tanhf(v / t.sh.cap))
+    if (t.sh.table != nullptr) AP32_EACH(v, v = v + t.sh.table[min(max(back, 0), t.sh.last)])
+    else AP32_EACH(v, v = fmaf(t.sh.slope, (float)-back, v))
+#undef AP32_EACH
+  }
   float top = -INFINITY;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -305,7 +323,7 @@ __device__ __forceinline__ void ap32_page(ApTile32<KS>& t, ApPage32<KS>& pg, con
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int j = j0 + 32 * h + 8 * g + 4 * x + i;
-        const float v = SHAPED ? ap_shape(t.sh, s[h][x][i] * scale, t.p - j) : s[h][x][i] * scale;
+        const float v = SHAPED ? s[h][x][i] : s[h][x][i] * scale;
         s[h][x][i] = held && j >= t.first && j <= t.p ? v : -INFINITY;
         top = fmaxf(top, s[h][x][i]);
       }
@@ -447,7 +465,7 @@ __device__ __forceinline__ int ap32_run_begin(uint32_t begins, int i) { return 3
 // on the matrix cores (head size 128) beside the softmax of the other wavefront of the SIMD. 1003 tokens, 28 heads of 128:
 // 202 us a layer; 1850 with a wavefront's lanes along the dims and a sum across the wavefront for every score.
 template <int KS, bool SHAPED>
-__global__ __launch_bounds__(256, SHAPED ? 1 : 2) void attention_f32_rows_kernel(
+__global__ __launch_bounds__(256, 2) void attention_f32_rows_kernel(
     float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ kpool, const float* __restrict__ vpool,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ row_seq, const int32_t* __restrict__ seq_slot,
     const int32_t* __restrict__ page_table, int max_blocks, int num_pages, int rows, int H, int KVH, int window, int chunk,
@@ -502,28 +520,31 @@ __global__ __launch_bounds__(256, SHAPED ? 1 : 2) void attention_f32_rows_kernel
   }
 }
 
-// One query: a wavefront takes one row and up to 16 heads of one kv head (its columns), and one page (pages > 1: the result
-// goes to ws as attention_plain_kernel's does) or all of them. Rows of long runs are left out where the kernel above takes them
-// (runs_elsewhere). A unit is a wavefront: rows x kv heads x tiles of 16 heads x pages, pages fastest.
+// One query: a wavefront takes one row and up to 16 heads of one kv head (its columns), and all pages or (SPLIT: a page's result
+// goes to ws as attention_plain_kernel's does) every parts-th of them. Rows of long runs are left out where the kernel above takes
+// them (runs_elsewhere). A unit is a wavefront: rows x kv heads x tiles of 16 heads x parts, the parts in the outermost order, so that the units with pages
+// come first and lie on all L2 domains (parts innermost, 64 of them: four of eight domains had work). Units without
+// a page of their own leave at once, but each holds its registers and LDS through three dependent loads: a step that
+// replays a graph is launched for the most keys it may have, and a unit a page of those took 58 us where 32 sequences of 8
+// keys, 16 heads on 16, may have 4200; parts that fill the chip take 18, and at 1000 keys
+// 130 where those took 188.
 // 4 sequences of about 700 keys, 28 heads of 128 on 4: 16.5 us, 38 with a wavefront a head.
 template <int KS, bool SPLIT, bool SHAPED>
-__global__ __launch_bounds__(256, SPLIT || SHAPED ? 1 : 2) void attention_f32_one_kernel(
+__global__ __launch_bounds__(256, SPLIT && KS >= 3 ? 1 : 2) void attention_f32_one_kernel(
     float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ q, const float* __restrict__ kpool,
     const float* __restrict__ vpool, const int32_t* __restrict__ positions, const int32_t* __restrict__ row_seq,
     const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ page_table, int max_blocks, int num_pages, int rows,
-    int H, int KVH, int window, int chunk, float scale, int pages, int runs_elsewhere, ApExtras ex) {
+    int H, int KVH, int window, int chunk, float scale, int pages, int parts, int runs_elsewhere, ApExtras ex) {
   constexpr int hd = 32 * KS;
   const int lane = threadIdx.x & (HE_WAVE - 1);
   const int group = H / KVH, tiles = (group + 15) / 16;
-  int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int z = (int)(unit % pages);
-  unit /= pages;
+  int64_t unit = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = (int)(unit % tiles);
   unit /= tiles;
   const int kvh = (int)(unit % KVH);
   unit /= KVH;
-  if (unit >= rows) return;
-  const int row = (int)unit;
+  const int row = (int)(unit % rows), z = (int)(unit / rows);
+  if (z >= parts) return;
   const int col = 16 * tile + (lane & 15);
   const bool has = col < group;
   const int h = kvh * group + min(col, group - 1);
@@ -542,30 +563,30 @@ __global__ __launch_bounds__(256, SPLIT || SHAPED ? 1 : 2) void attention_f32_on
   }
   const int p = positions[row];
   const int first = ap_first(p, window, chunk);
-  int c0 = first >> HE_PAGE_SHIFT, c1 = p >> HE_PAGE_SHIFT;
-  if (SPLIT) {
-    if (c0 + z > c1) return;
-    c0 += z;
-    c1 = c0;
-  }
+  const int c0 = first >> HE_PAGE_SHIFT, c1 = min(p >> HE_PAGE_SHIFT, SPLIT ? c0 + pages - 1 : 0x7fffffff);
+  if (SPLIT && c0 + z > c1) return;
   const int32_t* pt = page_table + (int64_t)seq_slot[seq] * max_blocks;
-  __shared__ ap_f4 own[4][KS * 4 * HE_WAVE];
+  extern __shared__ ap_f4 own_of_each[];         // [wavefronts][KS * 4 * HE_WAVE]
   ApTile32<KS> t;
-  t.q = own[threadIdx.x >> 6] + lane;
+  t.q = own_of_each + (threadIdx.x >> 6) * (KS * 4 * HE_WAVE) + lane;
   t.total = t.q + 2 * KS * HE_WAVE;
   t.p = has ? p : -1;
   t.first = has ? first : 0;
   t.sh = ap_shape_of(ex, h);
   ApPage32<KS> pg;
   const int64_t elems = 32 * KS * HE_PAGE_TOKENS;
-  int page = __builtin_amdgcn_readfirstlane(pt[c0]);
+  const int step = SPLIT ? parts : 1;
+  int page = __builtin_amdgcn_readfirstlane(pt[c0 + z]);
   bool held = page >= 0 && page < num_pages;
-  for (int half = 0; half < 2; ++half)
-    ap32_fetch_k<KS>(pg, ap32_rsrc<KS>(kpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems), half, lane);
+  auto fetch_k = [&] {
+    for (int half = 0; half < 2; ++half)
+      ap32_fetch_k<KS>(pg, ap32_rsrc<KS>(kpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems), half, lane);
+  };
+  fetch_k();
   ap32_begin<KS>(t, q + ((int64_t)row * H + h) * hd, has, lane);
-  for (int c = c0; c <= c1; ++c) {
+  for (int c = c0 + z;;) {
     const float* vpage = vpool + ((held ? page : 0) * (int64_t)KVH + kvh) * elems;
-    const int next = __builtin_amdgcn_readfirstlane(pt[min(c + 1, c1)]);
+    const int next = __builtin_amdgcn_readfirstlane(pt[min(c + step, c1)]);
     const bool next_held = next >= 0 && next < num_pages;
     const float* next_k = kpool + ((next_held ? next : 0) * (int64_t)KVH + kvh) * elems;
     const int j0 = c << HE_PAGE_SHIFT;
@@ -573,17 +594,24 @@ __global__ __launch_bounds__(256, SPLIT || SHAPED ? 1 : 2) void attention_f32_on
     ap32_page<KS, !SPLIT, SHAPED>(t, pg, vpage, next_k, held, j0, p, whole, scale, lane);
     page = next;
     held = next_held;
-  }
-  if (!has) return;
-  if (SPLIT) {
-    float* w = ws + (((int64_t)row * H + h) * pages + z) * (hd + 2);
+    if (SPLIT) {
+      float* w = ws + (((int64_t)row * H + h) * pages + (c - c0)) * (hd + 2);
 #pragma unroll
-    for (int dt = 0; dt < 2 * KS; ++dt)
+      for (int dt = 0; dt < 2 * KS; ++dt) {
+        if (has)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) w[16 * dt + 4 * (lane >> 4) + i] = t.total[dt * HE_WAVE][i];
-    if (lane < 16) w[hd] = t.m, w[hd + 1] = t.l;
-    return;
+          for (int i = 0; i < 4; ++i) w[16 * dt + 4 * (lane >> 4) + i] = t.total[dt * HE_WAVE][i];
+        t.total[dt * HE_WAVE] = ap_f4{0.f, 0.f, 0.f, 0.f};
+      }
+      if (has && lane < 16) w[hd] = t.m, w[hd + 1] = t.l;
+      t.m = -INFINITY;
+      t.l = 0.f;
+    }
+    c += step;
+    if (c > c1) break;
+    if (SPLIT) fetch_k();
   }
+  if (SPLIT || !has) return;
   ap32_store<KS>(t, o, ex, row, h, lane);
 }
 
@@ -912,14 +940,21 @@ extern "C" int he_attention_plain(void* out, const void* q, const void* kpool, c
   // 32-bit caches whose head size is whole steps of the matrix cores' operands
   const bool mfma = dtype == HE_F32 && hd % 32 == 0 && hd <= 128 && (((uintptr_t)q | (uintptr_t)kpool | (uintptr_t)vpool | (uintptr_t)out) & 15) == 0;
   const bool by_runs = mfma && !split && rows >= AP32_TILE;
-  const int64_t units = (int64_t)rows * KVH * ((H / KVH + 15) / 16) * pages;
-  HE_REQUIRE(!mfma || units < (1ll << 32), "he_attention_plain: %d rows are too many for one launch", rows);
+  const int64_t columns = (int64_t)rows * KVH * ((H / KVH + 15) / 16);
+  // (parts a query: as many wavefronts as the chip holds of this kernel, one a SIMD at head sizes of 96 and 128, two below)
+  const int parts = (int)max((int64_t)1, min((int64_t)pages, (hd > 64 ? 4 : 8) * he_cus() / columns));
+  const int64_t units = columns * parts;
+  // The launch of single queries: four units a workgroup, or one where compute units would stay without any (16 sequences of 16
+  // keys, 28 heads on 4: 17.5 us by fours, 16.8 by one).
+  const int ones_waves = units <= 2 * he_cus() ? 1 : 4;
+  const int64_t ones = (units + ones_waves - 1) / ones_waves;
+  const dim3 ones_grid((unsigned)(ones < (1 << 22) ? ones : 1 << 22), (unsigned)((ones + (1 << 22) - 1) >> 22));
   const bool shaped = slopes_f32 != nullptr || table_f32 != nullptr || cap > 0.f;
 #define AP32_ONE(KS_, SPLIT_, SHAPED_)                                                                               \
-  attention_f32_one_kernel<KS_, SPLIT_, SHAPED_><<<(unsigned)((units + 3) / 4), 256, 0, s>>>(                        \
+  attention_f32_one_kernel<KS_, SPLIT_, SHAPED_><<<ones_grid, ones_waves * HE_WAVE, ones_waves * KS_ * 4096, s>>>(  \
       (float*)out, ws, (const float*)q, (const float*)kpool, (const float*)vpool, (const int32_t*)positions,         \
       (const int32_t*)row_seq, (const int32_t*)seq_slot, (const int32_t*)page_table, max_blocks, num_pages, rows, H, KVH, \
-      window, chunk, scale, pages, by_runs ? 1 : 0, ex)
+      window, chunk, scale, pages, parts, by_runs ? 1 : 0, ex)
 #define AP32_SHAPED(KS_, SHAPED_)                                                                                    \
   {                                                                                                                  \
     if (by_runs)                                                                                                     \

@@ -81,3 +81,12 @@ def test_a_value_that_is_not_finite_reaches_only_the_queries_that_see_it(what):
         assert not got[seen:, 2:, 3].isfinite().any()
         keep = torch.arange(64) != 3
         assert torch.equal(got[:, :, keep.cuda()], want[:, :, keep.cuda()])
+
+
+@pytest.mark.parametrize("hd,window", [(128, 0), (128, 300), (64, 0), (32, 0)])
+def test_a_wavefront_takes_several_pages_of_a_query(hd, window):
+    """32 queries of 8 heads of their own, of 1 to 16 pages, in more units than the chip holds at once when each is a page."""
+    lengths = [1 + 33 * i for i in range(31)] + [1000]
+    step = Step(16, 16, hd, lengths, [1] * 32, 700)
+    split = step.run(0, 32, window, split=True)
+    assert torch.equal(split, step.run(0, 32, window)) and torch.equal(split[31:], step.run(31, 32, window, split=True))
