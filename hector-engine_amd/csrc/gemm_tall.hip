@@ -40,6 +40,7 @@ struct GtCase {
   const int32_t* tile_begin;  // [groups + 1] or null: one group of all rows
   const int32_t* rows_of;     // a slot's row of x, -1: none; null: the slot itself
   const float* scale;         // a slot's factor (GT_GATED) or null
+  const int32_t* out_of;      // GT_F32: a slot's row of out, -1: none; null: the slot itself
   int groups;
   int spread;                 // GT_GATED: the result goes to row rows_of[slot], columns from group * N / 2 on
   GatedAct act;
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 2) void gemm_tall_kernel(GtCase c) {
     const int m = m0 + wm * (BM / 2) + 16 * i + r16;
     if (!c.tile_begin && m >= c.M) continue;
     const float f = EPI == GT_GATED && c.scale ? c.scale[m] : 1.f;
-    const int to = EPI == GT_GATED && c.spread ? c.rows_of[m] : m;
+    const int to = EPI == GT_GATED && c.spread ? c.rows_of[m] : EPI == GT_F32 && c.out_of ? c.out_of[m] : m;
     if (to < 0) continue;
     const int64_t at0 = to * c.ldo + (EPI == GT_GATED && c.spread ? (int64_t)group * (c.N / 2) : 0);
 #pragma unroll
@@ -221,7 +222,7 @@ extern "C" int he_gemm_tall_bf16(void* out, const void* x, const void* w, const 
   HE_REQUIRE((int64_t)GT_BN * ldx * 2 < (1ll << 32) && (int64_t)GT_BN * ldw * 2 < (1ll << 32), "he_gemm_tall: rows too long");
   if (M == 0) return 0;
   GtCase c = {(const uint16_t*)x, (const uint16_t*)w, out, bias, bias_dtype, M, N, K, ldx, ldw, ldo, 0, nullptr, nullptr,
-              nullptr, 1, 0, {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic}};
+              nullptr, nullptr, 1, 0, {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic}};
   return bm == 256 ? gt_launch<256>(c, (M + 255) / 256, epilogue, (hipStream_t)stream)
                    : gt_launch<128>(c, (M + 127) / 128, epilogue, (hipStream_t)stream);
 }
@@ -229,14 +230,15 @@ extern "C" int he_gemm_tall_bf16(void* out, const void* x, const void* w, const 
 // ---- rows in groups: a token's choice of experts -----------------------------------------------
 // ids [rows][top] (an expert, or what has none: below 0 or from `groups` on). Every expert gets whole tiles of BM slots;
 // its tokens take them in the order of the rows. tile_begin [groups + 1]: an expert's first tile; rows_of / scale: a
-// slot's row (-1: none) and the weight of that choice; slot_of [rows][top]: where a choice went (-1: nowhere).
+// slot's row (-1: none) and the weight of that choice; choice_of: its place in ids (-1: none); slot_of [rows][top]: where a
+// choice went (-1: nowhere).
 // grid: an expert a workgroup, each counts all of them (a few thousand ids from L2) and writes its own.
 #define GR_THREADS 1024
 #define GR_MAX_GROUPS 1024
 __global__ __launch_bounds__(GR_THREADS) void group_rows_kernel(int32_t* __restrict__ tile_begin, int32_t* __restrict__ rows_of,
                                                                 float* __restrict__ scale, int32_t* __restrict__ slot_of,
-                                                                const int32_t* __restrict__ ids, const float* __restrict__ weights,
-                                                                int n, int top, int groups, int bm) {
+                                                                int32_t* __restrict__ choice_of, const int32_t* __restrict__ ids,
+                                                                const float* __restrict__ weights, int n, int top, int groups, int bm) {
   __shared__ int hist[GR_MAX_GROUPS];
   __shared__ int wave_sums[GR_THREADS / 64];
   __shared__ int begin_sh;
@@ -272,9 +274,10 @@ __global__ __launch_bounds__(GR_THREADS) void group_rows_kernel(int32_t* __restr
     if (ids[i] != e) continue;
     rows_of[slot] = i / top;
     scale[slot] = weights[i];
+    choice_of[slot] = i;
     slot_of[i] = slot++;
   }
-  for (int s = begin * bm + hist[e] + tid; s < (begin + tiles) * bm; s += GR_THREADS) rows_of[s] = -1, scale[s] = 0.f;
+  for (int s = begin * bm + hist[e] + tid; s < (begin + tiles) * bm; s += GR_THREADS) rows_of[s] = choice_of[s] = -1, scale[s] = 0.f;
   if (tid == 0) tile_begin[e] = begin;
   if (tid == 0 && e == groups - 1) tile_begin[groups] = begin + tiles;
 }
@@ -287,7 +290,7 @@ extern "C" int he_group_rows_most_tiles(int rows, int top, int groups, int bm) {
   return rows <= 0 || top <= 0 || groups <= 0 || bm <= 0 ? 0 : gr_most_tiles((int64_t)rows * top, groups, bm);
 }
 
-// out[row][d] = the sum over the row's choices of partial[slot][d], in the order of the choices, + dense[row][groups] * x[row][d]
+// out[row][d] = the sum over the row's choices that an expert took (slot_of) of partial[row][choice][d], in their order, + dense[row][groups] * x[row][d]
 // (x null: without).
 __global__ __launch_bounds__(256) void combine_groups_kernel(uint16_t* __restrict__ out, const float* __restrict__ partial,
                                                              const int32_t* __restrict__ slot_of, const float* __restrict__ dense,
@@ -297,8 +300,8 @@ __global__ __launch_bounds__(256) void combine_groups_kernel(uint16_t* __restric
   if (d >= D) return;
   gt_f32x4 sum = {0.f, 0.f, 0.f, 0.f};
   for (int k = 0; k < top; ++k) {
-    const int slot = slot_of[row * top + k];
-    if (slot >= 0) sum += *reinterpret_cast<const gt_f32x4*>(partial + (int64_t)slot * D + d);
+    const int64_t choice = row * top + k;
+    if (slot_of[choice] >= 0) sum += *reinterpret_cast<const gt_f32x4*>(partial + choice * D + d);
   }
   if (x != nullptr) {
     const float w = dense[row * (groups + 1) + groups];
@@ -316,12 +319,13 @@ __global__ __launch_bounds__(256) void combine_groups_kernel(uint16_t* __restric
 
 // The experts of a routed feed-forward, each over the rows that chose it: out[row] = the sum over the row's choices e of
 // weight * down_e (act(gate_e x, up_e x)) + dense[row][real] * x (identity). Fused matrices as he_chosen_experts takes them
-// (without shared columns). Scratch: lists int32 (he_routed_groups_ints), h bf16 [slots][I], partial fp32 [slots][D], slots
-// = bm * he_group_rows_most_tiles(rows, top, real, bm).
+// (without shared columns). Scratch: lists int32 (he_routed_groups_ints), h bf16 [slots][I], slots
+// = bm * he_group_rows_most_tiles(rows, top, real, bm), partial fp32 [rows][top][D]: by choice, since with few rows and many experts
+// nearly all slots are padding (65 rows, 8 of 256 experts, D 7168: 33,280 slots for 520 choices, 954 MB against 15).
 // down null: the activations alone, h_bf16 [rows][real I] with expert e's columns from e I on, the chosen ones written (the
 // caller has cleared it); out, partial and dense are not used.
 extern "C" int64_t he_routed_groups_ints(int rows, int top, int real, int bm) {
-  return (real + 1 + 3) / 4 * 4 + 2ll * bm * he_group_rows_most_tiles(rows, top, real, bm) + (int64_t)rows * top;
+  return (real + 1 + 3) / 4 * 4 + 3ll * bm * he_group_rows_most_tiles(rows, top, real, bm) + (int64_t)rows * top;
 }
 extern "C" int he_routed_groups(void* out, void* lists_i32, void* h_bf16, void* partial_f32, const void* x, const void* gate_up,
                                 const void* down, int64_t ldw, const void* ids_i32, const void* weights_f32,
@@ -342,16 +346,17 @@ extern "C" int he_routed_groups(void* out, void* lists_i32, void* h_bf16, void* 
   int32_t* tile_begin = (int32_t*)lists_i32;
   int32_t* rows_of = tile_begin + (real + 1 + 3) / 4 * 4;
   float* scale = (float*)(rows_of + slots);
-  int32_t* slot_of = (int32_t*)(scale + slots);
-  group_rows_kernel<<<real, GR_THREADS, 0, s>>>(tile_begin, rows_of, scale, slot_of, (const int32_t*)ids_i32,
+  int32_t* choice_of = (int32_t*)(scale + slots);
+  int32_t* slot_of = choice_of + slots;
+  group_rows_kernel<<<real, GR_THREADS, 0, s>>>(tile_begin, rows_of, scale, slot_of, choice_of, (const int32_t*)ids_i32,
                                                 (const float*)weights_f32, rows * top, top, real, bm);
   int rc = he_check_launch("he_routed_groups (lists)");
   if (rc) return rc;
   const GatedAct act = {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic};
   GtCase up = {(const uint16_t*)x, (const uint16_t*)gate_up, h_bf16, nullptr, 0, slots, 2 * I, D, D, D, spread ? (int64_t)real * I : I, (int64_t)2 * I * D,
-               tile_begin, rows_of, scale, real, spread, act};
+               tile_begin, rows_of, scale, nullptr, real, spread, act};
   GtCase dn = {(const uint16_t*)h_bf16, (const uint16_t*)down, partial_f32, nullptr, 0, slots, D, I, I, ldw, D, I, tile_begin,
-               nullptr, nullptr, real, 0, act};
+               nullptr, nullptr, choice_of, real, 0, act};
   rc = bm == 256 ? gt_launch<256>(up, mtiles, GT_GATED, s) : gt_launch<128>(up, mtiles, GT_GATED, s);
   if (rc || spread) return rc;
   rc = bm == 256 ? gt_launch<256>(dn, mtiles, GT_F32, s) : gt_launch<128>(dn, mtiles, GT_F32, s);

@@ -1215,7 +1215,7 @@ def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
 
 
 def routed_groups_sizes(rows: int, top: int, real: int, bm: int) -> tuple[int, int]:
-    """(ints of lists, slots) of routed_groups' scratch."""
+    """(ints of lists, slots) of routed_groups' scratch: h has a row a slot, partial one a choice."""
     L = _lib.load()
     return int(L.he_routed_groups_ints(rows, top, real, bm)), bm * int(L.he_group_rows_most_tiles(rows, top, real, bm))
 
@@ -1226,8 +1226,8 @@ def routed_groups(out, lists, h, partial, x, gate_up, down, ids, weights, dense,
     """out[rows, D] = the weighted sum of the chosen experts' results (ids, weights [rows, top] and dense [rows, real + 1] as
     route_tokens leaves them): the rows are sorted by expert and each expert's gate, up and down products run over its own
     rows, in tiles of bm (128 or 256). gate_up [2 real inter, D] (gate and up alternating), down [D, real inter (+ D)]; with
-    the last D columns the identity experts' share dense[row, real] * x is added. lists int32, h bf16 [slots, inter] and
-    partial fp32 [slots, D]: scratch, routed_groups_sizes()."""
+    the last D columns the identity experts' share dense[row, real] * x is added. lists int32, h bf16 [slots, inter]
+    (routed_groups_sizes()) and partial fp32 [rows * top, D]: scratch."""
     D, top = gate_up.shape[1], ids.shape[1]
     for name, t in (("out", out), ("h", h), ("x", x), ("gate_up", gate_up), ("down", down)):
         _need(t, name, torch.bfloat16)
@@ -1240,7 +1240,7 @@ def routed_groups(out, lists, h, partial, x, gate_up, down, ids, weights, dense,
     if tuple(gate_up.shape) != (2 * real * inter, D) or down.shape[0] != D or down.shape[1] not in (real * inter, real * inter + D):
         raise ValueError("routed_groups: the fused matrices do not match the sizes")
     if min(out.shape[0], x.shape[0], ids.shape[0], weights.shape[0], dense.shape[0]) < rows or out.shape[1] != D \
-            or x.shape[1] != D or lists.numel() < ints or h.numel() < slots * inter or partial.numel() < slots * D:
+            or x.shape[1] != D or lists.numel() < ints or h.numel() < slots * inter or partial.numel() < rows * top * D:
         raise ValueError("routed_groups: buffers smaller than the row count")
     L = _lib.load()
     _lib.check(L.he_routed_groups(out.data_ptr(), lists.data_ptr(), h.data_ptr(), partial.data_ptr(), x.data_ptr(),

@@ -186,7 +186,7 @@ class RoutedExperts(FeedForward):
                 ctx.scratch.release(turn)
                 continue
             h = ctx.alloc((slots, self.inter))
-            partial = ctx.alloc((slots, self.hidden), torch.float32)
+            partial = ctx.alloc((n * self.top, self.hidden), torch.float32)
             ops.routed_groups(out[r0:r0 + n], lists, h, partial, x[r0:r0 + n], self.gate_up.weight, self.down.weight,
                               ids[r0:r0 + n], weights[r0:r0 + n], dense[r0:r0 + n], n, self.real, self.inter, bm=bm, **act)
             ctx.scratch.release(turn)

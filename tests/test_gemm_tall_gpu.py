@@ -97,3 +97,23 @@ def test_experts_over_the_rows_that_chose_them(bm, rows, real, identity, top):
                     assert torch.equal(wide[rows_of[slot], e * I:(e + 1) * I], h[slot])
                     wide[rows_of[slot], e * I:(e + 1) * I] = 0
         assert (wide == 0).all()
+
+
+def test_experts_sums_lie_by_choice():
+    """partial holds a row a choice, whatever the slots of the tiles: nothing is written behind it, and the two sizes give the same bits."""
+    rows, real, top, D, I, bm = 70, 40, 2, 128, 64, 128
+    x, gate_up, down = rnd(rows, D, seed=1).cuda(), rnd(2 * real * I, D, seed=2, scale=0.2).cuda(), rnd(D, real * I, seed=3, scale=0.2).cuda()
+    g = torch.Generator().manual_seed(4)
+    ids = torch.stack([torch.randperm(real, generator=g)[:top] for _ in range(rows)]).int().cuda()
+    weights = torch.rand(rows, top, generator=g).cuda()
+    dense = torch.zeros(rows, real + 1, device="cuda").scatter_(1, ids.long(), weights)
+    ints, slots = ops.routed_groups_sizes(rows, top, real, bm)
+    assert slots > 20 * rows * top
+    h = torch.empty(slots, I, dtype=BF16, device="cuda")
+    room = torch.full((rows * top + 1, D), 7.0, device="cuda")
+    outs = []
+    for partial in (room[:rows * top], torch.full((slots, D), float("nan"), device="cuda")):
+        outs.append(torch.empty(rows, D, dtype=BF16, device="cuda"))
+        ops.routed_groups(outs[-1], torch.empty(ints, dtype=torch.int32, device="cuda"), h, partial, x, gate_up, down, ids, weights,
+                          dense, rows, real, I, bm=bm)
+    assert torch.equal(*outs) and (room[-1] == 7).all() and not (room[:-1] == 7).all(1).any()

@@ -6,7 +6,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-from hector_engine_amd.kernels import routes
+from hector_engine_amd.kernels import ops, routes
 from hector_engine_amd.parts.base import BuildEnv, PartSpec, build_part
 from hector_engine_amd.parts.linear import Linear
 
@@ -108,3 +108,20 @@ def test_operands_the_tiles_do_not_read_stay_with_the_library():
 def test_experts_beyond_the_tiles_offsets_stay_with_the_product_over_all():
     assert experts(real=512, inter=16320, hidden=64)._many_rows(4000, empty(4000, 64), CTX)
     assert not experts(real=512, inter=16384, hidden=64)._many_rows(4000, empty(4000, 64), CTX)
+
+
+def test_many_experts_of_few_rows_take_no_more_scratch_than_the_product_over_all(monkeypatch):
+    """An expert's tiles are mostly padding there: 65 rows that choose 8 of 256 experts, 33,280 slots for 520 choices."""
+    part, rows, taken = experts(real=256, top=8, inter=2048, hidden=7168), 65, []
+
+    def alloc(shape, dtype=BF16):
+        taken.append(math.prod(shape) * dtype.itemsize)
+        return empty(*shape, dtype=dtype)
+    ctx = SimpleNamespace(env=CTX.env, alloc=alloc, scratch=SimpleNamespace(mark=lambda: None, release=lambda turn: None))
+    x = empty(rows, 7168)
+    bm = part._many_rows(rows, x, ctx)
+    assert bm == 128
+    monkeypatch.setattr(ops, "routed_groups", lambda *a, **k: None)
+    part._by_expert(x, empty(rows, 257, dtype=torch.float32), empty(rows, 8, dtype=torch.int32), empty(rows, 8, dtype=torch.float32),
+                    rows, bm, {}, ctx)
+    assert sum(taken) <= rows * 3 * 256 * 2048 * 2       # gate and up of every expert, and their activations
