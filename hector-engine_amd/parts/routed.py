@@ -155,9 +155,7 @@ class RoutedExperts(FeedForward):
         """The rows a tile has where the step runs expert by expert over the rows that chose it (kernels.ops.routed_groups),
         0 where it runs through the products over all experts. For bfloat16 with the fast kernels, sizes in multiples
         of 64, no shared columns, and a choice of half of the experts at most, from 65 rows on (fewer go through the kernels
-        that carry norms): an expert's tiles over its own rows are never more than over all rows, so the sorting is all
-        that could cost. 16 experts of 2048 over rows of 2048, 4 chosen: 65 rows 196 -> 145 us, 512 330 -> 163, 2048 849 -> 228.
-        Tiles of 256 rows from 112 rows an expert on (384 rows there: 144 us in tiles of 128, 160 of 256; 512: 181, 163)."""
+        that carry norms), where _by_expert_times expects the faster of the two tile heights in 0.8 of the other form's time."""
         turn = min(rows, _ROW_CHUNK)
         if not (ctx.env.dtype == torch.bfloat16 and isinstance(x, torch.Tensor) and not self.shared_cols
                 and 2 * self.top <= self.real <= 1024 and self.inter % 64 == 0 and self.hidden % 64 == 0
@@ -166,7 +164,35 @@ class RoutedExperts(FeedForward):
                 and 2 * max(turn * self.hidden, 256 * (self.real * self.inter + self.hidden)) < 1 << 32
                 and self.gate_up.own_tiles(turn, ctx) and (self.shared is not None or self.down.own_tiles(turn, ctx))):
             return 0
-        return 256 if rows * self.top >= 112 * self.real else 128
+        low, high, over_all = self._by_expert_times(turn)
+        return 0 if min(low, high) > 0.8 * over_all else 128 if low <= high else 256
+
+    def _by_expert_times(self, rows: int) -> tuple[float, float, float]:
+        """Microseconds the experts of so many rows are expected to take: by expert in tiles of 128 and of 256 rows, and as products over
+        all experts. A round of tiles on the chip costs a start and its stages of 64 k, an expert has whole tiles however few rows
+        chose it, every choice's part of the sum is written and read in 32 bits, and sorting takes a nanosecond a choice; the
+        library's products cost their operations or their weights' bytes. Fitted to 7116 random sizes (2 to 256 experts of 64 to
+        4096, 65 to 4096 rows of 256 to 7168), on which the three are off by a sixth (standard deviation). With the factor 0.8 the 2586
+        of these that go by expert take 0.38 of the other form's time in the geometric mean (0.68 beside a shared expert), 15 of them 1.03
+        to 1.14 of it: 16 experts of 2048 over rows of 2048, 4 chosen, 65 rows 120 us beside 114, 512 153 beside 211, 2048 354 beside 851.
+        Few or small experts are left to the other form: 2 of 64 over 224 rows of 1728, 1 chosen, 13 us beside 43."""
+        D, I, real = self.hidden, self.inter, self.real
+        choices, cus = rows * self.top, ops.compute_units()
+
+        def library(cols: int, k: int) -> float:
+            return max(2 * rows * cols * k / 1300e6, 2 * cols * k / 4e6)
+
+        def by_expert(bm: int, start: float, begin: float, stage: float) -> float:
+            tiles = min(min(real, choices) * -(-choices // (real * bm)), choices // bm + min(choices, real))
+
+            def rounds(cols: int, k: int) -> float:
+                return -(-tiles * -(-cols // 256) // cus) * (begin + k // 64 * stage)
+            first = start + choices / 1000 + rounds(2 * I, D)
+            if self.shared is not None:      # (the second product stays one over all experts, over rows cleared first)
+                return first + 2 * rows * real * I / 0.8e6 + library(D, real * I)
+            return first + rounds(D, I) + 4 * choices * D / 2e6
+        over_all = 14 + library(2 * real * I, D) + library(D, real * I) + 6 * rows * real * I / 1.5e6
+        return by_expert(128, 9, 7.5, 0.9), by_expert(256, 11, 10.5, 1.33), over_all
 
     def _by_expert(self, x, dense, ids, weights, rows: int, bm: int, act: dict, ctx: StepContext):
         out = ctx.alloc((rows, self.hidden))
@@ -178,7 +204,7 @@ class RoutedExperts(FeedForward):
             if self.shared is not None:
                 # Beside a shared expert the sum over the experts stays one product over all of them, with its order of
                 # sums: a design that routes rows as they are, without a norm, turns near ties over at any change of it
-                # (Domorax: 3 to 6 % of the logits). The first product's sums are the same in both forms.
+                # (Domorax: 3 to 6 % of the logits; with the first product alone by expert they stay bit for bit what they were).
                 h = ctx.alloc((n, self.real * self.inter)).zero_()
                 ops.routed_groups_act(h, lists, x[r0:r0 + n], self.gate_up.weight, ids[r0:r0 + n], weights[r0:r0 + n], n,
                                       self.real, self.inter, bm=bm, **act)

@@ -125,3 +125,15 @@ def test_many_experts_of_few_rows_take_no_more_scratch_than_the_product_over_all
     part._by_expert(x, empty(rows, 257, dtype=torch.float32), empty(rows, 8, dtype=torch.int32), empty(rows, 8, dtype=torch.float32),
                     rows, bm, {}, ctx)
     assert sum(taken) <= rows * 3 * 256 * 2048 * 2       # gate and up of every expert, and their activations
+
+
+@pytest.mark.parametrize("sizes,tiles", [
+    (dict(real=16, top=4, inter=2048, hidden=2048), {65: 128, 512: 128, 768: 256, 2048: 256, 9000: 256}),
+    (dict(real=64, top=4, inter=512, hidden=1024), {65: 128, 2048: 128, 4096: 256}),
+    (dict(real=2, top=1, inter=64, hidden=1728), {65: 0, 224: 0, 1212: 0, 4096: 0}),      # small experts: two launches beat four
+    (dict(real=256, top=128, inter=64, hidden=1152), {300: 0, 2948: 0, 4096: 0}),         # half of the experts, narrow tiles
+    (dict(real=8, top=1, inter=4096, hidden=2048), {65: 0, 128: 0, 256: 128, 4096: 256})])  # few tiles of a long K
+def test_which_routed_steps_run_expert_by_expert(sizes, tiles):
+    """At 256 units: where the estimate of four launches over chosen rows is below 0.8 of the products over all experts."""
+    part = experts(**sizes)
+    assert {rows: part._many_rows(rows, empty(rows, sizes["hidden"]), CTX) for rows in tiles} == tiles

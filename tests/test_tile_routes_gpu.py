@@ -117,27 +117,28 @@ def test_products_of_long_k_in_tiles(monkeypatch, rows, tall):
         assert ((out[tall[0]:].double() - want).abs() <= err + 2 ** -8 * (want.abs() + err)).all()
 
 
-MLP = {"hidden_size": 128, "intermediate_size": 192}
+D = 1024
+MLP = {"hidden_size": D, "intermediate_size": 192}
 
 
 @pytest.mark.parametrize("turns", [(65,), (300,), (4096, 70), (4096, 9)])
 @pytest.mark.parametrize("form", ["plain", "identity_limited", "beside_a_shared_expert"])
 def test_experts_over_the_rows_that_chose_them(monkeypatch, form, turns):
-    rows, real, top, I = sum(turns), 16, 4, 64
+    rows, real, top, I = sum(turns), 64, 4, 512
     more = {"plain": {}, "identity_limited": {"identity_experts": 3, "limit": 1.5},
             "beside_a_shared_expert": {"shared": {"gate": "sg", "feed_forward": PartSpec("gated_mlp", MLP)}}}[form]
-    part = bound_part("routed_experts", {"hidden_size": 128, "intermediate_size": I, "experts": real, "top": top,
-                                         "correction": False, **more}, 128 ** -0.5)
+    part = bound_part("routed_experts", {"hidden_size": D, "intermediate_size": I, "experts": real, "top": top,
+                                         "correction": False, **more}, D ** -0.5)
     name, n_at = ("routed_groups_act", 6) if form == "beside_a_shared_expert" else ("routed_groups", 10)
-    x, calls, ctx = rnd(rows, 128, seed=92), spied(monkeypatch, name), context(rows)
+    x, calls, ctx = rnd(rows, D, seed=92), spied(monkeypatch, name), context(rows)
     routed = part._routed(x, ctx, False)
     assert [c.args[n_at] for c in calls] == list(turns)
-    assert {c.kw["bm"] for c in calls} == {256 if rows * top >= 112 * real else 128}
+    assert {c.kw["bm"] for c in calls} == {part._many_rows(rows, x, ctx)} == {256 if rows > 4096 else 128}
     dense, ids = torch.empty(rows, real + 1, device="cuda"), torch.empty(rows, top, dtype=torch.int32, device="cuda")
     ops.route_tokens(dense, ids, torch.empty(rows, top, device="cuda"), None, None, rows, real, 1, 1, top, part.scale, x=x,
                      router=part.router)
     fn, shift, limit = (lambda g: g * torch.sigmoid(1.702 * g), 1.0, 1.5) if "limit" in more else SILU
-    want = torch.zeros(rows, 128, dtype=torch.float64, device="cuda")
+    want = torch.zeros(rows, D, dtype=torch.float64, device="cuda")
     err = torch.zeros_like(want)
     wide = torch.zeros(rows, real * I, dtype=torch.float64, device="cuda")
     wide_off = torch.zeros_like(wide)
@@ -158,6 +159,6 @@ def test_experts_over_the_rows_that_chose_them(monkeypatch, form, turns):
     if form == "beside_a_shared_expert":
         got = torch.cat([c.args[0][:n] for c, n in zip(calls, turns)]).double()
         assert ((got - wide).abs() <= wide_off).all()                    # exact zeros where an expert was not chosen
-        both = torch.empty(rows, 128, dtype=BF16, device="cuda")
+        both = torch.empty(rows, D, dtype=BF16, device="cuda")
         ops.gated_add(both, routed, part.shared.forward(x, context(rows)), x, part.shared_gate, rows)
         assert torch.equal(part.forward(x, context(rows)), both)
