@@ -511,6 +511,10 @@ __global__ __launch_bounds__(256) void gemm_plain_rows_sum_kernel(
 // (151936 x 128 at 64 rows 44, 182; 16384 x 512 at 64 rows 20, 28; but 16384 x 256 at 16 rows 11.6, 8.6, and 8192 x 256
 // at 64 even). Long K against few weight rows, a unit's own rate of about 30 bytes a ns: the rows kernel (512 x 12288
 // at 1 row 13.6, 26.6, at 8 rows 20, 29; 1024 x 4864 at 4 rows 13.5, 14.1; 2048 x 8192 at 1 row 20.1, 22.7, at 4 rows 23.8, 22.2).
+// Workgroups that fill part of their last round (a unit with one more than the others takes that much longer), the less of it
+// the more rows: 4608 x 3584 at 1 row 17.0, 20.1, at 4 rows 20.8, 20.6; 4160 x 8192 at 4 rows 37.4, 43.8; 5120 x 5120 at 1 row
+// 24.7, 27.8 (weights from memory; over 7758 random sizes of 1 to 8 rows the choice takes 0.69 of the rows kernel's time in the
+// geometric mean, 24 of them 1.1 to 1.17 of it).
 static bool gp_streams(int M, int N, int K, bool aligned) {
   const int segments = K / GP_SEG, cus = he_cus();
   if (!aligned || K % GP_SEG != 0) return false;
@@ -518,8 +522,13 @@ static bool gp_streams(int M, int N, int K, bool aligned) {
   if (segments <= (M + 15) / 16 && N >= (M <= 16 ? 96 : 64) * cus) return false;
   if (M > GP_ROWS_MAX_M) return true;
   if (segments <= 4 && N >= 96 * cus) return M > 4 && M * segments > (N >= 192 * cus ? 16 : 8);
+  if (segments <= 4 && N >= 66 * cus) return M * segments > (N >= 82 * cus ? 4 : 2);
   if (segments >= 24 && N <= 4 * cus) return 4 * M > segments - 16;
-  return segments < 24 || N > 8 * cus || M > 2;
+  if (segments >= 24 && 2 * N <= 13 * cus) return M > 2 && 8 * M > segments - 8;
+  if (segments >= 24 && N <= 8 * cus) return M > 2;
+  const int workgroups = (N + 15) / 16, held = (workgroups + cus - 1) / cus * cus;       // held: what whole rounds have room for
+  const bool idle = workgroups > cus && N <= 40 * cus && 10ll * M * held <= 108ll * held - 120ll * workgroups;
+  return !idle || segments < 16 || (segments < 24 && M > 1);
 }
 
 // Floats of workspace with which a product of M rows runs through the kernels for few rows (0: another kernel takes it, which

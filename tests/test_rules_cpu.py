@@ -187,12 +187,17 @@ def test_which_products_of_few_rows_want_a_workspace():
         floats = ops.gemm_plain_workspace_floats(M, N, K, a=a, w=w, out=out)
         assert floats in (0, -(-K // 128) * M * N)
         return floats > 0
-    assert not any(wants(M, N, K) for M in (1, 8) for N, K in ((152064, 3584), (37888, 3584), (4608, 3584), (3584, 18944), (1152, 896), (4096, 128)))
+    assert not any(wants(M, N, K) for M in (1, 8) for N, K in ((152064, 3584), (37888, 3584), (3584, 3584), (3584, 18944), (1152, 896), (4096, 128)))
     assert [M for M in range(1, 10) if wants(M, 32000, 128)] == list(range(1, 9))
     assert [M for M in range(1, 10) if wants(M, 32000, 256)] == [1, 2, 3, 4]
     assert [M for M in range(1, 10) if wants(M, 32000, 512)] == [1, 2, 3, 4]
     assert [M for M in range(1, 10) if wants(M, 65536, 256)] == list(range(1, 9))
     assert [M for M in range(1, 10) if wants(M, 32000, 640)] == []
+    assert [M for M in range(1, 10) if wants(M, 20480, 128)] == [1, 2]
+    assert [M for M in range(1, 10) if wants(M, 1280, 8192)] == [1, 2, 3, 4, 5, 6, 7]
+    # workgroups that fill part of a last round of the chip: 288 of 512, 320, 520 of 768, 576, 448 of 512
+    assert [[M for M in range(1, 10) if wants(M, N, K)] for N, K in ((4608, 3584), (5120, 5120), (8320, 4096), (9216, 4096), (7168, 5120), (4608, 2048), (4608, 1920))] \
+        == [[1, 2, 3, 4], [1, 2, 3], [1, 2], [1], [], [1], []]
     assert [M for M in range(1, 10) if wants(M, 896, 4864)] == [1, 2, 3, 4, 5]
     assert [M for M in range(1, 10) if wants(M, 512, 12288)] == list(range(1, 9))
     assert [M for M in range(1, 10) if wants(M, 2048, 8192)] == [1, 2] and not wants(1, 2049, 8192)
