@@ -528,7 +528,7 @@ __global__ __launch_bounds__(256, 2) void attention_f32_rows_kernel(
 // replays a graph is launched for the most keys it may have, and a unit a page of those took 58 us where 32 sequences of 8
 // keys, 16 heads on 16, may have 4200; parts that fill the chip take 18, and at 1000 keys
 // 130 where those took 188.
-// 4 sequences of about 700 keys, 28 heads of 128 on 4: 16.5 us, 38 with a wavefront a head.
+// 4 sequences of about 700 keys, 28 heads of 128 on 4: 14.1 us, 38 with a wavefront a head.
 template <int KS, bool SPLIT, bool SHAPED>
 __global__ __launch_bounds__(256, SPLIT && KS >= 3 ? 1 : 2) void attention_f32_one_kernel(
     float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ q, const float* __restrict__ kpool,

@@ -9,7 +9,7 @@
 // sixteen rows of an operand read hit different banks. The product is formed as W X^T: a lane then holds four
 // neighbouring outputs of one row, two (gate, up) pairs where the weight's rows alternate.
 // Groups: a row of tiles belongs to one group (`tile_begin`: the first tile row of each), its rows are the slots of a list
-// (he_group_rows), their sources named by `rows_of`. The grid is sized by what the host knows; workgroups beyond the tiles
+// (group_rows_kernel), their sources named by `rows_of`. The grid is sized by what the host knows; workgroups beyond the tiles
 // there are leave at once. Tiles go to an XCD in stretches, eight row tiles by column after column: the 32 workgroups an XCD
 // has at once read about 8 + 4 tiles of operands (12001 x 3584 x 18944: 1087 TFLOP/s without, 1176 with).
 // The wavefronts work in two groups, one phase apart: while the four of one group (one a SIMD) multiply, the other four

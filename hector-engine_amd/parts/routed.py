@@ -19,7 +19,8 @@ product with the down matrices side by side (and an identity block) adds everyth
 has the same launches whatever the tokens choose, so it replays as a graph, and a token's sums do
 not depend on the rest of the batch. A bfloat16 step of so few rows that they cannot choose more than
 half of the experts reads only the chosen experts' rows of the same matrices (ops.chosen_experts). A bfloat16 step of
-more than 64 rows sorts its rows by expert and multiplies each expert's matrices with the rows that chose it (ops.routed_groups).
+more than 64 rows sorts its rows by expert and multiplies each expert's matrices with the rows that chose it
+(ops.routed_groups) where that is the faster form (_by_expert_times).
 Options: `normalize` divides the chosen outputs' weights by their sum (the softmax over the chosen logits
 alone; the choice itself is the same, the softmax being monotone); `shared` = {"feed_forward": PartSpec, "name":
 suffix of its prefix, "gate": suffix of a stored vector of hidden_size or None} adds an expert that every token
