@@ -363,13 +363,18 @@ extern "C" int he_attention_decode_bf16(void* out, const void* q, const void* kp
 
 // The same join for many rows (the parts of a prompt step): one wavefront per (row, head), four
 // of them a workgroup, no LDS and no barrier; a lane has the dims 2 lane, 2 lane + 1 (+ 128, ...).
-// Parts are added in their order. Every part was stored; out is row-major.
+// Parts are added in their order. Every part of the rows below *rows_end was stored; the rows from there on get zeros; out is row-major.
 __global__ __launch_bounds__(256) void attention_merge_rows_kernel(
     uint16_t* __restrict__ out, const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-    int64_t pairs, int HD, int nsplit, int H, AttnExtras ex) {
+    int64_t pairs, int HD, int nsplit, int H, const int32_t* __restrict__ rows_end, AttnExtras ex) {
   const int lane = threadIdx.x & 63;
   const int64_t pair = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // row * H + h
   if (pair >= pairs) return;
+  if (pair >= (int64_t)*rows_end * H) {
+    // a row of no sequence (they end the step): nothing has stored its parts
+    for (int d0 = 2 * lane; d0 < HD; d0 += 128) *reinterpret_cast<uint32_t*>(out + pair * HD + d0) = 0;
+    return;
+  }
   const int64_t base = pair * nsplit;
   const float2 ml = lane < nsplit ? *reinterpret_cast<const float2*>(ws_ml + 2 * (base + lane))
                                   : make_float2(-INFINITY, 0.f);
@@ -404,13 +409,13 @@ __global__ __launch_bounds__(256) void attention_merge_rows_kernel(
 }
 
 int he_attention_merge_rows(void* out, const float* ws_o, const float* ws_ml, int rows, int H, int hd,
-                            int parts, const AttnExtras& ex, void* stream) {
+                            int parts, const int32_t* rows_end, const AttnExtras& ex, void* stream) {
   HE_REQUIRE(parts >= 1 && parts <= 64 && hd % 2 == 0, "he_attention_merge_rows: %d parts (at most 64), head_dim %d", parts, hd);
   const int64_t pairs = (int64_t)rows * H;
   HE_REQUIRE((pairs + 3) / 4 < (1ll << 31), "he_attention_merge_rows: too many rows for one launch");
   if (pairs == 0) return 0;
   attention_merge_rows_kernel<<<(unsigned)((pairs + 3) / 4), 256, 0, (hipStream_t)stream>>>(
-      (uint16_t*)out, ws_o, ws_ml, pairs, hd, parts, H, ex);
+      (uint16_t*)out, ws_o, ws_ml, pairs, hd, parts, H, rows_end, ex);
   return he_check_launch("he_attention_merge_rows");
 }
 
@@ -433,14 +438,23 @@ int he_attention_merge_parts(void* out, const float* ws_o, const float* ws_ml, c
 // has (or a bound). Measured at 28 heads of 128, 4 kv heads (us without parts -> with, join included):
 // 8 tokens after 8000 108 -> 18, 64 after 8000 114 -> 27, 200 after 8000 129 -> 45, 512 after 7680 130 -> 76,
 // 4 x 128 after 4000 74 -> 51, 512 after 30000 457 -> 233, 1024 after 7168 144 -> 134.
-extern "C" int he_attention_prefill_parts(int num_seqs, int max_q_len, int H, int hd, int most_keys) {
+// total_rows, KVH (0: not known, every sequence may be as long as the longest): the other sequences are taken to share the rows that
+// the longest leaves; one of so few queries that the heads of a kv group share a workgroup
+// (attention_prefill_wide.hip) counts once a kv head. Where all do, the parts may be 32: the launch stays small.
+extern "C" int he_attention_prefill_parts(int num_seqs, int max_q_len, int H, int hd, int most_keys, int total_rows, int KVH) {
   if (num_seqs <= 0 || H <= 0 || hd <= 0 || hd > 128 || hd % 16 || max_q_len <= 0) return 1;
   if ((int64_t)most_keys < 4 * (int64_t)max_q_len) return 1;
-  const int64_t blocks = (int64_t)((max_q_len + 127) / 128) * H * num_seqs;
-  int64_t parts = 2 * he_cus() / blocks;
+  int64_t groups = (int64_t)((max_q_len + 127) / 128) * H * num_seqs, most_parts = 16;
+  if (total_rows > 0 && KVH > 0 && H % KVH == 0) {
+    const int64_t G = H / KVH, others = num_seqs - 1, left = std::max(0, total_rows - max_q_len);
+    const bool longest_folds = max_q_len * G <= 128, others_fold = left * G <= 128 * others;
+    groups = (longest_folds ? KVH : (int64_t)((max_q_len + 127) / 128) * H) +
+             (others_fold ? others * KVH : others * ((left / others + 127) / 128) * H);
+    if (longest_folds && others_fold) most_parts = 32;
+  }
+  int64_t parts = 2 * he_cus() / groups;
   const int pages = (most_keys + HE_PAGE_TOKENS - 1) / HE_PAGE_TOKENS;
-  if (parts > pages / 4) parts = pages / 4;
-  if (parts > 16) parts = 16;
+  parts = std::min(std::min<int64_t>(parts, pages / 4), most_parts);
   return parts < 1 ? 1 : (int)parts;
 }
 
@@ -497,10 +511,10 @@ extern "C" int he_attention_prefill_bf16(void* out, const void* q, const void* k
                  parts, (long long)need, (long long)workspace_floats);
     }
     int rc = he_attention_prefill_wide(out, q, kpool, vpool, cu_seqlens, seq_slot, seq_start, page_table,
-                                       max_blocks, num_pages, num_seqs, max_q_len, H, KVH, hd, window, scale,
+                                       max_blocks, num_pages, num_seqs, max_q_len, total_rows, H, KVH, hd, window, scale,
                                        parts, ws_o, ws_ml, ex, stream);
     if (rc || parts == 1) return rc;
-    return he_attention_merge_rows(out, ws_o, ws_ml, total_rows, H, hd, parts, ex, stream);
+    return he_attention_merge_rows(out, ws_o, ws_ml, total_rows, H, hd, parts, (const int32_t*)cu_seqlens + num_seqs, ex, stream);
   }
   dim3 grid((max_q_len + 63) / 64, H, num_seqs);
 #define PREFILL_ARGS                                                                                   \

@@ -1,7 +1,7 @@
 // Prompt attention over the paged cache with 32 queries a wavefront as one 32x32 MFMA tile,
 // the softmax of one step of 32 keys running beside the matrix products of its neighbours.
 //
-// grid (ceil(max_q_len / 128), H, num_seqs), 256 threads. A workgroup takes 128 consecutive
+// grid (ceil(max_q_len / 128), H, num_seqs), or one row of workgroups where the keys are cut into parts, 256 threads. A workgroup takes 128 consecutive
 // queries of one sequence and head, wavefront w the 32 queries 32w..32w+31. Tiles are
 // transposed as in the other MFMA attention kernels (attention_mfma.hip): keys are the rows
 // of the score tile and queries its columns, so a lane holds, for the one query of its
@@ -38,11 +38,16 @@
 // fits on the chip at once puts its lightest beside its heaviest); an XCD sees neighbouring
 // heads. Head sizes up to 128.
 //
-// parts > 1: grid.x counts (block of queries, part). The pages of a block are dealt out evenly to its
-// parts; a part runs the same loops over its own pages and leaves unnormalised sums, reference
-// point and sum of weights per query and head (ws_o, ws_ml) for attention_merge_rows_kernel
-// (attention_mfma.hip). For steps of few queries against many keys, which would otherwise keep
-// a fraction of the chip busy.
+// parts > 1: the pages of a block are dealt out evenly to its parts; a part runs the same loops over
+// its own pages and leaves unnormalised sums, reference point and sum of weights per query and head
+// (ws_o, ws_ml) for attention_merge_rows_kernel (attention_mfma.hip). For steps of few queries against
+// many keys, which would otherwise keep a fraction of the chip busy. Such steps often hold one-token
+// sequences beside the longer ones, so the workgroups are counted through the sequences (pw_find), with no grid
+// of the longest one's size for all; and a sequence of up to 128 queries over all heads of a kv group
+// is folded: column c of the workgroup is query c / G under head c % G of the group, G = H / KVH, and the
+// group's keys are read once. What bounds such a step is the walk of the longest share of pages. (203 tokens after 2500 beside seven
+// one-token sequences of as many keys, 28 heads, 4 kv heads: a block of 128 columns a head and all keys of a sequence in one
+// workgroup, PW_BEFORE; folded and in six parts PW_AFTER us, join included.)
 //
 // Measured at 28 heads of 128, 4 kv heads (causal flops): 0.61 PFLOP/s at 2048 tokens,
 // 0.94 at 8192, 1.1 at 16384, 0.85 for eight prompts of 2048. In the long runs the shader
@@ -364,6 +369,53 @@ __device__ __forceinline__ void pw_fast_step(WideTile<NT>& t, floatx16& s_pend, 
   s_pend = s_next;
 }
 
+// Whether all heads of a kv group share a workgroup's columns. (Not with a distance table: LDS holds that of one head.)
+template <int MODE>
+__device__ __forceinline__ bool pw_folds(int q_len, int G) { return MODE != ATTN_SHAPED && q_len * G <= PW_QUERIES; }
+
+// A step in parts: workgroup t counted through the sequences, each with (kv heads) x (its blocks, for every head of the group unless it
+// is folded) x parts of them. Every wavefront finds its own for itself (64 sequences a turn); neighbouring
+// workgroups, which go to different XCDs, differ in the kv head first, so an XCD's L2 keeps few kv heads' pages.
+// False: the step has no workgroup t.
+struct PwItem {
+  int seq, h, bx, part;
+};
+template <int MODE>
+__device__ __forceinline__ bool pw_find(PwItem& item, int t, const int32_t* __restrict__ cu, const int32_t* __restrict__ seq_slot,
+                                        int num_seqs, int H, int KVH, int parts, int most_blocks) {
+  const int lane = threadIdx.x & 63, G = H / KVH;
+  int base = 0;
+  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
+    const int s = min(s0 + lane, num_seqs - 1);
+    const int q_len = cu[s + 1] - cu[s], slot = seq_slot[s];
+    const int blocks = min((q_len + PW_QUERIES - 1) / PW_QUERIES, most_blocks);
+    const int each = s0 + lane >= num_seqs || slot < 0 || q_len <= 0 ? 0 : pw_folds<MODE>(q_len, G) ? 1 : G * blocks;
+    const int n = each * KVH * parts;
+    int upto = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(upto, o);
+      if (lane >= o) upto += u;
+    }
+    const unsigned long long hit = __ballot(t < base + upto);
+    if (hit != 0) {
+      const int f = __ffsll((long long)hit) - 1;
+      int local = __builtin_amdgcn_readfirstlane(t - base - __shfl(upto - n, f));
+      const int per = __builtin_amdgcn_readfirstlane(__shfl(each, f));
+      item.seq = s0 + f;
+      const int kvh = local % KVH;
+      local /= KVH;
+      const int i = local % per;
+      item.part = local / per;
+      item.h = kvh * G + i % G;          // (folded: i is 0, the group's first head)
+      item.bx = i / G;
+      return true;
+    }
+    base += __shfl(upto, 63);
+  }
+  return false;
+}
+
 template <int NT, int MODE>
 __global__ __launch_bounds__(64 * PW_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 attention_prefill_wide_kernel(
@@ -371,8 +423,8 @@ attention_prefill_wide_kernel(
     const uint16_t* __restrict__ kpool, const uint16_t* __restrict__ vpool,
     const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_slot,
     const int32_t* __restrict__ seq_start, const int32_t* __restrict__ page_table, int max_blocks,
-    int num_pages, int H, int KVH, int window, float scale, int parts, float* __restrict__ ws_o,
-    float* __restrict__ ws_ml, AttnExtras ex) {
+    int num_pages, int H, int KVH, int window, float scale, int parts, int num_seqs, int most_blocks,
+    float* __restrict__ ws_o, float* __restrict__ ws_ml, AttnExtras ex) {
   constexpr int HD = Pw<NT>::HD, KS = Pw<NT>::KS, DT = Pw<NT>::DT;
   constexpr int KP = Pw<NT>::K_PIECES, VP = Pw<NT>::V_PIECES;
   __shared__ uint4 k_lds[2 * KP];
@@ -387,25 +439,29 @@ attention_prefill_wide_kernel(
   // Of the rows (head, sequence) an XCD then sees every (HE_XCDS / g)-th, g = gcd(HE_XCDS,
   // rows); the rows are numbered so that these are neighbours, i.e. few kv heads, whose pages
   // the XCD's own L2 keeps.
-  const int rows = gridDim.y * gridDim.z;
-  const int launched = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-  int gcd = HE_XCDS;
-  while (rows % gcd) gcd >>= 1;               // HE_XCDS is a power of two
-  // When the whole launch is on the chip at once (two workgroups a compute unit), a unit's second
-  // workgroup is the one launched HE_CUS after its first (the 33rd of its XCD): the heaviest gets
-  // the lightest beside it, and so on, and every unit has about the same to do (2048 tokens,
-  // 28 heads: 52.1 -> 49.6 us).
-  int rank = launched;
-  if ((int)(gridDim.x * rows) <= 2 * HE_CUS) {
-    const int x = launched % HE_XCDS, j = launched / HE_XCDS;
-    const int of_xcd = ((int)(gridDim.x * rows) - x + HE_XCDS - 1) / HE_XCDS;
-    rank = x + HE_XCDS * (j < HE_CUS / HE_XCDS ? j : of_xcd - 1 - (j - HE_CUS / HE_XCDS));
+  PwItem item;
+  if (parts > 1) {
+    if (!pw_find<MODE>(item, blockIdx.x, cu_seqlens, seq_slot, num_seqs, H, KVH, parts, most_blocks)) return;
+  } else {
+    const int rows = gridDim.y * gridDim.z;
+    const int launched = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    int gcd = HE_XCDS;
+    while (rows % gcd) gcd >>= 1;               // HE_XCDS is a power of two
+    // When the whole launch is on the chip at once (two workgroups a compute unit), a unit's second
+    // workgroup is the one launched HE_CUS after its first (the 33rd of its XCD): the heaviest gets
+    // the lightest beside it, and so on, and every unit has about the same to do (2048 tokens,
+    // 28 heads: 52.1 -> 49.6 us).
+    int rank = launched;
+    if ((int)(gridDim.x * rows) <= 2 * HE_CUS) {
+      const int x = launched % HE_XCDS, j = launched / HE_XCDS;
+      const int of_xcd = ((int)(gridDim.x * rows) - x + HE_XCDS - 1) / HE_XCDS;
+      rank = x + HE_XCDS * (j < HE_CUS / HE_XCDS ? j : of_xcd - 1 - (j - HE_CUS / HE_XCDS));
+    }
+    const int rho = rank % rows;
+    const int row = (rho % gcd) * (rows / gcd) + rho / gcd;
+    item = {row % (int)gridDim.z, row / (int)gridDim.z, (int)gridDim.x - 1 - rank / rows, 0};
   }
-  const int rho = rank % rows;
-  const int row = (rho % gcd) * (rows / gcd) + rho / gcd;
-  const int gx = gridDim.x - 1 - rank / rows;   // gridDim.x = query blocks x parts
-  const int bx = gx / parts, part = gx - bx * parts;
-  const int seq = row % gridDim.z, h = row / gridDim.z;
+  const int seq = item.seq, h = item.h, bx = item.bx, part = item.part;
   const int slot = seq_slot[seq];
   if (slot < 0) return;
   const int row0 = cu_seqlens[seq];
@@ -413,7 +469,10 @@ attention_prefill_wide_kernel(
   const int q0 = PW_QUERIES * bx;
   if (q0 >= q_len) return;
   const int start = seq_start[seq];
-  const int kvh = h / (H / KVH);
+  const int G = H / KVH, kvh = h / G;
+  // the workgroup's columns: queries of one head, or (query, head of the group) pairs
+  const int fold = parts > 1 && pw_folds<MODE>(q_len, G) ? G : 1;
+  const int cols = q_len * fold;
   const int32_t* pt = page_table + (int64_t)slot * max_blocks;
   const int64_t k_stride = (int64_t)KVH * he_k_page_elems(HD), v_stride = (int64_t)KVH * he_v_page_elems(HD);
   const uint16_t* kp = kpool + (int64_t)kvh * he_k_page_elems(HD);
@@ -421,9 +480,10 @@ attention_prefill_wide_kernel(
   const float scale_log2 = MODE >= ATTN_SHAPED ? 1.f : scale * PW_LOG2E;
 
   // the workgroup's pages: from the first key its first query sees to its last query
-  const int blk_last = start + min(q0 + PW_QUERIES, q_len) - 1;
-  const int blk_first = attn_first(start + q0, window, ex.chunk);
+  const int blk_last = start + (min(q0 + PW_QUERIES, cols) - 1) / fold;
+  const int blk_first = attn_first(start + q0 / fold, window, ex.chunk);
   int pbA = blk_first >> HE_PAGE_SHIFT, pbB = blk_last >> HE_PAGE_SHIFT;
+  const int pb0 = pbA;
   if (parts > 1) {
     // this workgroup's share of the block's pages; one without pages leaves empty parts
     const int per = (pbB - pbA + parts) / parts;
@@ -431,14 +491,15 @@ attention_prefill_wide_kernel(
     pbB = min(pbB, pbA + per - 1);
   }
 
-  // the wavefront's tile; a query beyond the sequence doubles the last one and is not stored
+  // the wavefront's tile; a column beyond the sequence doubles the last one and is not stored
   const int qt = q0 + 32 * wave;
-  const bool tile = qt < q_len;
-  const int qi = min(qt + col, q_len - 1);
+  const bool tile = qt < cols;
+  const int ci = min(qt + col, cols - 1);
+  const int qi = fold > 1 ? ci / fold : ci, hq = fold > 1 ? h + ci - qi * fold : h;
   if (pbA > pbB) {
     // a part without pages (more parts than the block has pages): empty parts for its queries
-    if (tile && qt + col < q_len) {
-      const int64_t idx = ((int64_t)(row0 + qi) * H + h) * parts + part;
+    if (tile && qt + col < cols) {
+      const int64_t idx = ((int64_t)(row0 + qi) * H + hq) * parts + part;
       if (g == 0) *reinterpret_cast<float2*>(ws_ml + 2 * idx) = make_float2(-INFINITY, 0.f);
       for (int d = 4 * g; d < HD; d += 8) *reinterpret_cast<float4*>(ws_o + idx * HD + d) = make_float4(0.f, 0.f, 0.f, 0.f);
     }
@@ -449,8 +510,8 @@ attention_prefill_wide_kernel(
   t.lo = attn_first(t.hi, window, ex.chunk);
   t.m = -INFINITY;
   t.l = 0.f;
-  t.bias = MODE == ATTN_SLOPES ? ex.slopes[h] / scale : 0.f;
-  if (MODE == ATTN_CAPPED) t.sh = attn_shape_of(ex, h, scale);
+  t.bias = MODE == ATTN_SLOPES ? ex.slopes[hq] / scale : 0.f;
+  if (MODE == ATTN_CAPPED) t.sh = attn_shape_of(ex, h, scale);   // (the cap: the same for all heads)
   if (MODE == ATTN_SHAPED) {
     t.sh = attn_shape_of(ex, h, scale);
     const int entries = t.sh.table != nullptr ? ex.table_len : 1;
@@ -463,12 +524,12 @@ attention_prefill_wide_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) t.o[dt][i] = 0.f;
   {
-    const uint16_t* qrow = q + ((int64_t)(row0 + qi) * H + h) * HD + 8 * g;
+    const uint16_t* qrow = q + ((int64_t)(row0 + qi) * H + hq) * HD + 8 * g;
 #pragma unroll
     for (int kk = 0; kk < NT; ++kk) t.qf[kk] = ld8(qrow + 16 * kk, true);
   }
   // steps of 32 keys (hs: keys 32hs..32hs+31) of the tile: hsA..hsB; without a mask: hsI0..hsI1-1
-  const int first_pos = start + qt, last_pos = start + min(qt + 31, q_len - 1);
+  const int first_pos = start + qt / fold, last_pos = start + min(qt + 31, cols - 1) / fold;
   const int lo_min = attn_first(first_pos, window, ex.chunk);
   const int lo_max = attn_first(last_pos, window, ex.chunk);
   // (a part has the steps of its own pages only)
@@ -490,10 +551,26 @@ attention_prefill_wide_kernel(
   p_pend[0] = p_pend[1] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
 
   pw_stage<Pw<NT>::K_CHUNKS>(k_base + (pbA & 1) * KP * 16, pw_page(kp, pt[pbA], num_pages, k_stride, lane), wave);
+  // A part that begins behind the first page takes its reference point from the tile's first step too, as one walk over all
+  // keys would (it follows later keys only where they exceed it by 2^PW_SLACK): the probabilities are then rounded alike
+  // however the keys are cut, and what the cut changes is the order of fp32 sums.
+  if (parts > 1 && pbA > pb0)
+    pw_stage<Pw<NT>::K_CHUNKS>(k_base + ((pbA + 1) & 1) * KP * 16, pw_page(kp, pt[pb0], num_pages, k_stride, lane), wave);
   pw_epoch_end();
   // Q has arrived before the loops begin: a wait for it inside them would also wait for the page on its way
 #pragma unroll
   for (int kk = 0; kk < NT; ++kk) asm volatile("" : "+v"(t.qf[kk]));
+  if (parts > 1 && pbA > pb0) {
+    const int hs = lo_min >> 5;
+    if (tile && hs >> 1 == pb0) {
+      const floatx16 s = pw_scores<NT>(t.qf, k_lds + ((pbA + 1) & 1) * KP, kl, hs & 1, pw_score_start<MODE>(t.bias, t.hi, 32 * hs, g));
+      float alpha;
+      pw_softmax<NT, MODE>(t, s, 32 * hs, g, scale_log2, p_pend, alpha);
+      t.l = 0.f;
+      p_pend[0] = p_pend[1] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+    }
+    __syncthreads();     // the buffer is filled again in the first epoch
+  }
   int j = pbA;
   for (; j < jF0; ++j) {
     if (j + 1 <= pbB) pw_stage<Pw<NT>::K_CHUNKS>(k_base + ((j + 1) & 1) * KP * 16, pw_page(kp, pt[j + 1], num_pages, k_stride, lane), wave);
@@ -537,11 +614,11 @@ attention_prefill_wide_kernel(
   }
 
   const float l = xor32_sum(t.l);
-  if (!tile || qt + col >= q_len) return;
+  if (!tile || qt + col >= cols) return;
   if (parts > 1) {
     // one of several parts of the keys: the sums as they stand, with their reference point, for
-    // attention_merge_kernel (O fp32 [hd], then (m, l) with m in the base-2 domain)
-    const int64_t idx = ((int64_t)(row0 + qi) * H + h) * parts + part;
+    // attention_merge_rows_kernel (O fp32 [hd], then (m, l) with m in the base-2 domain)
+    const int64_t idx = ((int64_t)(row0 + qi) * H + hq) * parts + part;
     if (g == 0) *reinterpret_cast<float2*>(ws_ml + 2 * idx) = make_float2(t.m, l);
     float* orow = ws_o + idx * HD + 4 * g;
 #pragma unroll
@@ -573,20 +650,24 @@ attention_prefill_wide_kernel(
 int he_attention_prefill_wide(void* out, const void* q, const void* kpool, const void* vpool,
                               const void* cu_seqlens, const void* seq_slot, const void* seq_start,
                               const void* page_table, int max_blocks, int num_pages, int num_seqs,
-                              int max_q_len, int H, int KVH, int hd, int window, float scale,
+                              int max_q_len, int total_rows, int H, int KVH, int hd, int window, float scale,
                               int parts, float* ws_o, float* ws_ml, const AttnExtras& ex, void* stream) {
   HE_REQUIRE(hd % 16 == 0 && hd >= 16 && hd <= 128,
              "he_attention_prefill_wide: head_dim %d must be a multiple of 16 up to 128", hd);
   HE_REQUIRE(parts >= 1 && parts <= 64 && (parts == 1 || (ws_o != nullptr && ws_ml != nullptr)),
              "he_attention_prefill_wide: %d parts (1 to 64, with room for them)", parts);
-  const int64_t gx = (int64_t)((max_q_len + PW_QUERIES - 1) / PW_QUERIES) * parts;
-  HE_REQUIRE(gx * H * num_seqs < (1ll << 31), "he_attention_prefill_wide: grid too large");
-  dim3 grid((unsigned)gx, H, num_seqs);
+  const int64_t most_blocks = (max_q_len + PW_QUERIES - 1) / PW_QUERIES;
+  // in parts: the blocks of any lengths that sum up to the step's rows (a sequence's last block may hold one query)
+  const int64_t blocks = std::min(num_seqs * most_blocks, (total_rows + (int64_t)num_seqs * (PW_QUERIES - 1)) / PW_QUERIES);
+  HE_REQUIRE((parts > 1 ? blocks * parts : most_blocks * num_seqs) * H < (1ll << 31), "he_attention_prefill_wide: grid too large");
+  if (parts > 1 && blocks == 0) return 0;
+  const dim3 grid = parts > 1 ? dim3((unsigned)(blocks * H * parts)) : dim3((unsigned)most_blocks, H, num_seqs);
   hipStream_t s = (hipStream_t)stream;
 #define PREFILL_WIDE_ARGS                                                                      \
   (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kpool, (const uint16_t*)vpool,           \
       (const int32_t*)cu_seqlens, (const int32_t*)seq_slot, (const int32_t*)seq_start,          \
-      (const int32_t*)page_table, max_blocks, num_pages, H, KVH, window, scale, parts, ws_o, ws_ml, ex
+      (const int32_t*)page_table, max_blocks, num_pages, H, KVH, window, scale, parts, num_seqs, (int)most_blocks, ws_o, \
+      ws_ml, ex
 #define PREFILL_WIDE(NTV)                                                                       \
   case NTV:                                                                                     \
     if (mode == ATTN_SLOPES)                                                                    \

@@ -242,7 +242,7 @@ int he_attention_merge_parts(void* out, const float* ws_o, const float* ws_ml, c
 int he_attention_prefill_wide(void* out, const void* q, const void* kpool, const void* vpool,
                               const void* cu_seqlens, const void* seq_slot, const void* seq_start,
                               const void* page_table, int max_blocks, int num_pages, int num_seqs,
-                              int max_q_len, int H, int KVH, int hd, int window, float scale,
+                              int max_q_len, int total_rows, int H, int KVH, int hd, int window, float scale,
                               int parts, float* ws_o, float* ws_ml, const AttnExtras& ex, void* stream);
 
 #define HE_REQUIRE(cond, ...)      \

@@ -214,7 +214,7 @@ int he_attention_decode_fused_bf16(void* out, const void* qkv, const void* qkv_p
 // block of queries are cut into that many parts that run side by side and are joined by a
 // second launch; the workspace holds he_attention_prefill_workspace_floats() floats.
 // he_attention_prefill_parts() is the number the library would take for a step.
-int he_attention_prefill_parts(int num_seqs, int max_q_len, int H, int hd, int most_keys);
+int he_attention_prefill_parts(int num_seqs, int max_q_len, int H, int hd, int most_keys, int total_rows, int KVH);
 int64_t he_attention_prefill_workspace_floats(int total_rows, int H, int hd, int parts);
 int he_attention_prefill_bf16(void* out, const void* q, const void* kpool, const void* vpool,
                               const void* cu_seqlens, const void* seq_slot, const void* seq_start,

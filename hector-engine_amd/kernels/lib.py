@@ -126,7 +126,7 @@ _SIGNATURES = {
     "he_attention_prefill_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_int,
                                   c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_f32, c_int,
                                   c_int, c_int, c_ptr, c_i64, c_int, c_ptr, c_int, c_ptr, c_i64, c_ptr, c_ptr, c_int, c_f32, c_ptr],
-    "he_attention_prefill_parts": [c_int, c_int, c_int, c_int, c_int],
+    "he_attention_prefill_parts": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "he_attention_prefill_workspace_floats": [c_int, c_int, c_int, c_int],
     "he_argmax_workspace_bytes": [c_int, c_int],
     "he_argmax_rows": [c_ptr, c_ptr, c_int, c_int, c_i64, c_ptr, c_i64, c_ptr],

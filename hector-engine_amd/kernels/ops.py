@@ -1494,10 +1494,12 @@ def attention_decode_fused(out, qkv, bias, kpool, vpool, positions, row_seq, seq
         workspace.numel() if workspace is not None else 0, _stream()))
 
 
-def attention_prefill_parts(num_seqs: int, max_q_len: int, H: int, hd: int, most_keys: int) -> int:
+def attention_prefill_parts(num_seqs: int, max_q_len: int, H: int, hd: int, most_keys: int, total_rows: int = 0,
+                            KVH: int = 0) -> int:
     """Parts the library would cut the keys of this prompt step into (1: none): more than one
-    for a step of few queries against many keys, which would otherwise leave most of the chip idle."""
-    return int(_lib.load().he_attention_prefill_parts(num_seqs, max_q_len, H, hd, most_keys))
+    for a step of few queries against many keys, which would otherwise leave most of the chip idle.
+    total_rows, KVH: the step's rows and kv heads (0: every sequence may be as long as the longest, no kv heads shared)."""
+    return int(_lib.load().he_attention_prefill_parts(num_seqs, max_q_len, H, hd, most_keys, total_rows, KVH))
 
 
 def attention_prefill_workspace_floats(total_rows: int, H: int, hd: int, parts: int) -> int:

@@ -529,15 +529,15 @@ class Attention(Mixer):
             most = min(most, self.window + ctx.max_q_len)
         if self.chunk > 0:
             most = min(most, self.chunk + ctx.max_q_len)
-        parts = ops.attention_prefill_parts(ctx.num_seqs, ctx.max_q_len, H, hd, most)
+        parts = ops.attention_prefill_parts(ctx.num_seqs, ctx.max_q_len, H, hd, most, rows, KVH if self.table is None else 0)
         if self.table is not None and self.table.shape[1] > ops.ATTENTION_TABLE_LDS:
             parts = 1                     # the kernel that cuts the keys keeps the head's table in LDS
         ws = ctx.alloc((ops.attention_prefill_workspace_floats(rows, H, hd, parts),), torch.float32) \
             if parts > 1 else None
-        if ctx.padded:
-            # the prompt kernels write the rows of sequences only: padding rows hold zeros (their
-            # parts too, whose join then gives zeros), never what the buffer held before
-            (ws if ws is not None else out).zero_()
+        if ctx.padded and ws is None:
+            # the prompt kernels write the rows of sequences only: padding rows hold zeros, never what
+            # the buffer held before (the join of parts writes them itself)
+            out.zero_()
         ops.attention_prefill(out, q, cache.kpool, cache.vpool, ctx.cu_seqlens, ctx.seq_slot,
                               ctx.seq_start, cache.page_table, ctx.num_seqs, ctx.max_q_len,
                               rows, H, KVH, hd, self.window, self.scale, parts=parts, workspace=ws,
