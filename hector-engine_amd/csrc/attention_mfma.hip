@@ -446,7 +446,8 @@ extern "C" int he_attention_prefill_parts(int num_seqs, int max_q_len, int H, in
   if ((int64_t)most_keys < 4 * (int64_t)max_q_len) return 1;
   int64_t groups = (int64_t)((max_q_len + 127) / 128) * H * num_seqs, most_parts = 16;
   if (total_rows > 0 && KVH > 0 && H % KVH == 0) {
-    const int64_t G = H / KVH, others = num_seqs - 1, left = std::max(0, total_rows - max_q_len);
+    const int64_t G = H / KVH, others = num_seqs - 1;
+    const int64_t left = others > 0 ? std::max(0, total_rows - max_q_len) : 0;      // (one sequence: padding rows)
     const bool longest_folds = max_q_len * G <= 128, others_fold = left * G <= 128 * others;
     groups = (longest_folds ? KVH : (int64_t)((max_q_len + 127) / 128) * H) +
              (others_fold ? others * KVH : others * ((left / others + 127) / 128) * H);

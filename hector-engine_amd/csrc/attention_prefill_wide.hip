@@ -47,7 +47,7 @@
 // is folded: column c of the workgroup is query c / G under head c % G of the group, G = H / KVH, and the
 // group's keys are read once. What bounds such a step is the walk of the longest share of pages. (203 tokens after 2500 beside seven
 // one-token sequences of as many keys, 28 heads, 4 kv heads: a block of 128 columns a head and all keys of a sequence in one
-// workgroup, PW_BEFORE; folded and in six parts PW_AFTER us, join included.)
+// workgroup 59 us and a fill of 4.7; folded and in six parts 25, and a join of 6.3.)
 //
 // Measured at 28 heads of 128, 4 kv heads (causal flops): 0.61 PFLOP/s at 2048 tokens,
 // 0.94 at 8192, 1.1 at 16384, 0.85 for eight prompts of 2048. In the long runs the shader

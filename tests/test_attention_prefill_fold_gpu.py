@@ -51,3 +51,5 @@ def test_parts_of_steps_whose_other_sequences_are_short(ops):
     assert ops.attention_prefill_parts(8, 256, 28, 128, 1000, 256, 4) == 1       # fewer than four keys a query
     assert ops.attention_prefill_parts(1, 8, 28, 128, 8064, 8, 4) == 31          # one folded sequence: four pages a part
     assert ops.attention_prefill_parts(4, 128, 28, 128, 4096, 512, 4) == ops.attention_prefill_parts(4, 128, 28, 128, 4096) == 4
+    # one sequence and padding rows behind it
+    assert ops.attention_prefill_parts(1, 200, 28, 128, 8200, 256, 4) == ops.attention_prefill_parts(1, 200, 28, 128, 8200) == 9
