@@ -16,10 +16,10 @@
 // rows (all at once). A chunk begins at the first row
 // a step brings, every power of the decay is at most the decay's own, and no exponent is ever positive: how the rows
 // were cut shows in rounding only. The powers come from a table [H][DM_C + 1] formed in double precision on the host.
-#include "common.h"
+#include "chunks.h"
 #include "hector_kernels.h"
 
-#define DM_C 64       // rows of a chunk
+#define DM_C CK_ROWS
 #define DM_B 64       // dims of a block of keys or of values
 #define DM_LD 68      // floats between rows in LDS (a multiple of 4, and four banks on from row to row)
 #define DM_WALK 8     // steps of at most so many rows a sequence are walked
@@ -59,35 +59,6 @@ __device__ __forceinline__ void dm_vec4(float* x, const bf16_t* p) {
   const uint2 v = *reinterpret_cast<const uint2*>(p);
   x[0] = __uint_as_float(v.x << 16); x[1] = __uint_as_float(v.x & 0xffff0000u);
   x[2] = __uint_as_float(v.y << 16); x[3] = __uint_as_float(v.y & 0xffff0000u);
-}
-
-// ---- which chunk is whose ------------------------------------------------------------------------------
-__device__ __forceinline__ int dm_chunks(const int32_t* cu, int s) { return (cu[s + 1] - cu[s] + DM_C - 1) / DM_C; }
-
-// Chunk t of the step, counted through its sequences: the sequence and the chunk inside it. Every wavefront finds it
-// for itself (64 sequences a turn). False: the step has no chunk t.
-__device__ __forceinline__ bool dm_find(int t, const int32_t* __restrict__ cu, int num_seqs, int& seq, int& chunk) {
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
-    const int s = s0 + lane;
-    const int n = s < num_seqs ? dm_chunks(cu, s) : 0;
-    int upto = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int u = __shfl_up(upto, o);
-      if (lane >= o) upto += u;
-    }
-    const unsigned long long hit = __ballot(t < base + upto);
-    if (hit != 0) {
-      const int f = __ffsll((long long)hit) - 1;
-      seq = s0 + f;
-      chunk = t - base - __shfl(upto - n, f);
-      return true;
-    }
-    base += __shfl(upto, 63);
-  }
-  return false;
 }
 
 // what every kernel of a scan reads
@@ -180,7 +151,7 @@ __global__ __launch_bounds__(256) void dm_share_kernel(DmArgs<T> a, int t0) {
   __shared__ __attribute__((aligned(16))) float ks[DM_C * DM_LD], vs[DM_C * DM_LD];
   const int h = blockIdx.y;
   int seq, chunk;
-  if (!dm_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
   if (a.slot[seq] < 0) return;
   const int vb = (a.dvp + DM_B - 1) / DM_B;
   const int d0 = ((int)blockIdx.x / vb) * DM_B, c0 = ((int)blockIdx.x % vb) * DM_B;
@@ -238,12 +209,12 @@ __global__ __launch_bounds__(256) void dm_carry_kernel(DmArgs<T> a, int t0, int 
   int before = 0;
   for (int s0 = 0; s0 < seq; s0 += 64) {
     const int s = s0 + (int)(threadIdx.x & 63);
-    int n = s < seq ? dm_chunks(a.cu, s) : 0;
+    int n = s < seq ? ck_chunks(a.cu, s) : 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
     before += n;
   }
-  const int chunks = dm_chunks(a.cu, seq);
+  const int chunks = ck_chunks(a.cu, seq);
   const int first = max(0, t0 - before), end = min(chunks, t0 + nt - before);
   if (first >= end) return;
   const int64_t memory = (int64_t)a.dk * a.dvp;
@@ -305,7 +276,7 @@ __global__ __launch_bounds__(256, 4) void dm_rows_kernel(float* __restrict__ y, 
     return;
   }
   int seq, chunk;
-  if (!dm_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
   if (a.slot[seq] < 0) return;
   const int64_t r0 = a.cu[seq] + (int64_t)chunk * DM_C;
   const int n = min(DM_C, (int)(a.cu[seq + 1] - r0));

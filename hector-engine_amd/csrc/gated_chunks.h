@@ -1,0 +1,429 @@
+// A memory per head whose rows have gates of their own, by chunks of CK_ROWS rows on the fp32 matrix cores:
+//   S_t = exp(f_t) S_(t-1) + w_t v_t k_t^T  (dv x dk),  y_t = S_t q_t
+// with a logarithm f_t <= 0 of what is kept and a weight w_t >= 0 of what is written a row. One after the other the
+// rows are a chain of multiply-adds that leaves the chip waiting (the matrix memory of 14 heads of 128 x 256: 0.52 us a
+// row, a prompt of 2,048 rows 1,003 us; the state space of 64 heads of 128 x 64: 665 us). In a chunk, with F_i the sum of f over its first i rows and S
+// the memory before it,
+//   y_i = exp(F_i) S q_i + sum over j <= i of exp(F_i - F_j) w_j (k_j . q_i) v_j
+//   S'  = exp(F_n) S + sum over j of exp(F_n - F_j) w_j v_j k_j^T
+// are matrix products, in three launches: every chunk's own share of S' (all chunks at once), the memory before every
+// chunk (one walk over the chunks of a sequence, element by element), every chunk's rows (all at once). (The same two prompts of
+// 2,048 rows: 125 and 136 us alone.)
+// F is summed in 64 bits and no exponent is positive, so the powers are as exact as the
+// walk's; everything else is fp32 arithmetic as there. What bounds the three: the share and the rows kernel the fp32
+// products, the walk over chunks the memories it reads and writes (two passes over 4 (dv + 1) dk bytes a head and chunk).
+//
+// NORMED (the matrix memory): w_t = exp(i_t), S carries a factor exp(-m_t), m_t = max(f_t + m_(t-1), i_t), and
+// y is divided by max(|n_t . q_t|, exp(-m_t)) + 1e-6 with n the same recurrence over k alone: n is one more column of S. In a chunk
+// m_i = F_i + max(m before it, the largest i_j - F_j up to j = i); a chunk's own share is kept relative to its own G = the
+// largest F_n - F_j + i_j until the walk knows m.
+//
+// The policy P gives what differs: static NORMED; gate(row, h, f, in): f, and in = i_t (NORMED) or w_t; place(st, h, c, d): where
+// four neighbouring key dims from d on of column c (dv: n) of S lie in a sequence's state; keep(...) puts them back (n into every copy of it);
+// m(st, h) and keep_m(...): NORMED's m and its copies; result(y, x, h): what follows the products.
+#pragma once
+#include "chunks.h"
+
+#define GC_LD 68      // floats between rows of 64 in LDS (four banks on from row to row)
+#define GC_KB 32      // key dims of a block of the rows kernel
+#define GC_KLD 36
+#define GC_WINDOW_FLOATS (64 << 20)   // memories held between the launches at once (256 MiB)
+// Steps whose longest sequence has more rows than this go by chunks. One sequence, walked and by chunks: matrix memory of 14 heads 48
+// rows 29 and 27 us, 64 rows 35 and 27, 128 rows 65 and 29; state space of 64 heads 48 rows 22 and 27, 64 rows 27 and 28, 128 rows 48 and 30;
+// four sequences of 32 rows of 128 heads 54 and 55.
+#define GC_FROM 64
+
+typedef float gc_acc __attribute__((ext_vector_type(16)));
+
+template <typename T>
+struct GcArgs {
+  const T* q;              // head h's at (h / per) dk
+  const T* k;
+  const T* v;              // at h dv
+  int64_t stride;          // elements between rows
+  int per;                 // heads that share q and k
+  float q_scale;
+  const int32_t* cu;
+  const int32_t* slot;
+  int num_seqs, H, dk, dv, dkp;      // dkp: key dims with the state's padding, a multiple of 4
+  uint8_t* state;
+  int64_t state_stride, state_offset;
+  float* ws;               // [chunk of the window][H][cols][dkp]: first the chunks' shares, then the memories before them
+  float* ends;             // [chunk of the window][H][2]: F_n and G of a chunk; then the m before it
+};
+template <typename T, class P>
+__host__ __device__ constexpr int gc_cols(int dv) { return dv + (P::NORMED ? 1 : 0); }
+
+__device__ __forceinline__ float4 gc_load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 gc_load4(const bf16_t* p) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                     __uint_as_float(v.y & 0xffff0000u));
+}
+// Four numbers at dim d of a row of a chunk of n rows from `first` on; zeros beyond the chunk or the head. The load itself
+// stands behind no condition, so that a tile's loads go out together.
+template <typename T>
+__device__ __forceinline__ float4 gc_tile4(const T* first, int64_t stride, int row, int n, int d, int width) {
+  const float4 v = gc_load4(first + min(row, n - 1) * stride + (d < width ? d : 0));
+  return row < n && d < width ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// Sums of many products are formed sixteen at a time and then added: a chain of all of them would lose more in rounding than the
+// walk's sums, which are spread over the lanes of a value dim.
+__device__ __forceinline__ void gc_add(gc_acc& a, const gc_acc& b) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) a[r] += b[r];
+}
+
+// F of the lane's row (lane < 64: the rows of the chunk, summed up to and with it) and in; rows beyond the chunk keep everything and
+// write nothing. NORMED: peak = the largest in - F up to and with the lane's row.
+template <class P>
+__device__ __forceinline__ void gc_gates(const P& p, int64_t r0, int n, int h, int lane, double& F, float& in, double& peak) {
+  float f;
+  p.gate(r0 + min(lane, n - 1), h, f, in);
+  if (lane >= n) f = 0.f, in = P::NORMED ? -INFINITY : 0.f;
+  F = (double)f;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double u = __shfl_up(F, o);
+    if (lane >= o) F += u;
+  }
+  peak = 0.;
+  if (P::NORMED) {
+    peak = (double)in - F;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double u = __shfl_up(peak, o);
+      if (lane >= o) peak = fmax(peak, u);
+    }
+  }
+}
+
+// ---- every chunk's own share of the memory behind it -----------------------------------------------------
+// One workgroup of four wavefronts a (64 key dims x 64 columns, head, chunk), a wavefront 32 x 32 of it, two rows of the
+// chunk an instruction (v_mfma_f32_32x32x2_f32: A lane l holds A[l % 32][l / 32], B likewise, D register r of lane l is
+// D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]).
+template <typename T, class P>
+__global__ __launch_bounds__(256) void gc_share_kernel(GcArgs<T> a, P p, int t0) {
+  __shared__ __attribute__((aligned(16))) float ks[CK_ROWS * GC_LD], vs[CK_ROWS * GC_LD];
+  __shared__ float weight[CK_ROWS], part[4][64];
+  const int h = blockIdx.y;
+  int seq, chunk;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (a.slot[seq] < 0) return;
+  const int vb = (a.dv + 63) / 64;
+  const int d0 = ((int)blockIdx.x / vb) * 64, c0 = ((int)blockIdx.x % vb) * 64;
+  const int64_t r0 = a.cu[seq] + (int64_t)chunk * CK_ROWS;
+  const int n = min(CK_ROWS, (int)(a.cu[seq + 1] - r0));
+  const int t = threadIdx.x, d = 4 * (t & 15);
+  const T* kr = a.k + r0 * a.stride + (int64_t)(h / a.per) * a.dk;
+  const T* vr = a.v + r0 * a.stride + (int64_t)h * a.dv;
+  float4 kx[4], vx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    kx[i] = gc_tile4(kr, a.stride, (t >> 4) + 16 * i, n, d0 + d, a.dk);
+    vx[i] = gc_tile4(vr, a.stride, (t >> 4) + 16 * i, n, c0 + d, a.dv);
+  }
+  if (t < 64) {
+    double F, peak;
+    float in;
+    gc_gates(p, r0, n, h, t, F, in, peak);
+    const double Fn = __shfl(F, 63), G = P::NORMED ? Fn + __shfl(peak, 63) : 0.;
+    weight[t] = P::NORMED ? expf((float)(Fn - F + (double)in - G)) : in * expf((float)(Fn - F));
+    if (t == 0 && blockIdx.x == 0) *reinterpret_cast<float2*>(a.ends + 2 * ((int64_t)blockIdx.z * a.H + h)) = make_float2((float)Fn, (float)G);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = (t >> 4) + 16 * i;
+    const float w = weight[row];
+    *reinterpret_cast<float4*>(ks + row * GC_LD + d) = make_float4(kx[i].x * w, kx[i].y * w, kx[i].z * w, kx[i].w * w);
+    *reinterpret_cast<float4*>(vs + row * GC_LD + d) = vx[i];
+  }
+  __syncthreads();
+  const int cols = gc_cols<T, P>(a.dv);
+  float* out = a.ws + ((int64_t)blockIdx.z * a.H + h) * cols * a.dkp;
+  const int wave = t >> 6, l32 = t & 31, hl = (t >> 5) & 1;
+  const int i0 = (wave >> 1) * 32, j0 = (wave & 1) * 32;       // columns of S, key dims
+  gc_acc acc = {0.f};
+  for (int g0 = 0; g0 < n; g0 += 16) {
+    gc_acc some = {0.f};
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int row = g0 + 8 * hl + m;
+      some = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[row * GC_LD + i0 + l32], ks[row * GC_LD + j0 + l32], some, 0, 0, 0);
+    }
+    gc_add(acc, some);
+  }
+  const int od = d0 + j0 + l32;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int c = c0 + i0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+    if (c < a.dv && od < a.dkp) out[(int64_t)c * a.dkp + od] = acc[r];
+  }
+  if (P::NORMED && c0 == 0) {      // n's share: the weighted rows of k alone
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sum += ks[(16 * wave + e) * GC_LD + (t & 63)];
+    part[wave][t & 63] = sum;
+    __syncthreads();
+    if (t < 64 && d0 + t < a.dkp) out[(int64_t)a.dv * a.dkp + d0 + t] = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
+  }
+}
+
+// ---- the memory before every chunk ---------------------------------------------------------------------
+// A thread holds four neighbouring key dims of a column of a sequence's S and walks its chunks in the window
+// [t0, t0 + nt): the chunk's share is taken out, the memory before the chunk put in its place.
+template <typename T, class P>
+__global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0, int nt, float* __restrict__ before_m) {
+  const int seq = blockIdx.z, h = blockIdx.y;
+  const int slot = a.slot[seq];
+  if (slot < 0 || a.cu[seq + 1] <= a.cu[seq]) return;
+  int before = 0;
+  for (int s0 = 0; s0 < seq; s0 += 64) {
+    const int s = s0 + (int)(threadIdx.x & 63);
+    int n = s < seq ? ck_chunks(a.cu, s) : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    before += n;
+  }
+  const int first = max(0, t0 - before), end = min(ck_chunks(a.cu, seq), t0 + nt - before);
+  if (first >= end) return;
+  const int cols = gc_cols<T, P>(a.dv);
+  const int64_t memory = (int64_t)cols * a.dkp, step = (int64_t)a.H * memory;
+  const int64_t id = blockIdx.x * 256ll + threadIdx.x, at = 4 * id;
+  const bool own = at < memory;
+  const int c = own ? (int)(at / a.dkp) : 0, d = own ? (int)(at % a.dkp) : 0;
+  float* st = reinterpret_cast<float*>(a.state + (int64_t)slot * a.state_stride + a.state_offset);
+  float* place = p.place(st, h, c, d);
+  const int64_t base = (int64_t)(before + first - t0) * a.H + h;
+  float* w = a.ws + base * memory + (own ? at : 0);
+  const float2* ends = reinterpret_cast<const float2*>(a.ends) + base;
+  float m = p.m(st, h);
+  float4 S = *reinterpret_cast<const float4*>(place);
+  constexpr int AHEAD = 8;
+  for (int i = first; i < end; i += AHEAD) {
+    float4 mine[AHEAD];
+    float2 e[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int k = min(u, end - 1 - i);
+      mine[u] = *reinterpret_cast<const float4*>(w + k * step);
+      e[u] = ends[(int64_t)k * a.H];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (i + u < end) {
+        if (own) *reinterpret_cast<float4*>(w + u * step) = S;
+        if (P::NORMED && id == 0) before_m[base + (int64_t)(i + u - first) * a.H] = m;
+        const float next = P::NORMED ? fmaxf(e[u].x + m, e[u].y) : 0.f;
+        const float keep = expf(e[u].x + m - next), take = P::NORMED ? expf(e[u].y - next) : 1.f;
+        S.x = fmaf(keep, S.x, take * mine[u].x);
+        S.y = fmaf(keep, S.y, take * mine[u].y);
+        S.z = fmaf(keep, S.z, take * mine[u].z);
+        S.w = fmaf(keep, S.w, take * mine[u].w);
+        m = next;
+      }
+    }
+    w += AHEAD * step;
+    ends += (int64_t)AHEAD * a.H;
+  }
+  if (own) p.keep(st, h, c, d, S);            // (m is kept by the rows kernel: every workgroup here reads it)
+}
+
+// ---- every chunk's rows --------------------------------------------------------------------------------
+// One workgroup of four wavefronts a (64 columns, head, chunk), a wavefront 32 rows x 32 columns: the rows' products with the
+// keys of the chunk (a square of which the part behind the diagonal is left out) and with the memory before it, block
+// by block of 32 key dims; then the square, weighted, on the values.
+template <typename T, class P>
+__global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, GcArgs<T> a, P p, int t0, const float* __restrict__ before_m) {
+  // rows of q, rows of k, columns of the memory; later the square and the values
+  __shared__ __attribute__((aligned(16))) float lds[2 * CK_ROWS * GC_LD];
+  static_assert(3 * CK_ROWS * GC_KLD <= 2 * CK_ROWS * GC_LD, "the blocks fit where the square and the values will be");
+  float* qs = lds;
+  float* ks = qs + CK_ROWS * GC_KLD;
+  float* ss = ks + CK_ROWS * GC_KLD;
+  float* square_s = lds;
+  float* vs = lds + CK_ROWS * GC_LD;
+  __shared__ double Fs[CK_ROWS];
+  __shared__ float ins[CK_ROWS], ms[CK_ROWS], olds[CK_ROWS], dens[CK_ROWS];
+  __shared__ __attribute__((aligned(16))) float ns[GC_KB];
+  const int h = blockIdx.y, c0 = (int)blockIdx.x * 64;
+  const int t = threadIdx.x, wave = t >> 6, l32 = t & 31, hl = (t >> 5) & 1;
+  int seq, chunk;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (a.slot[seq] < 0) return;
+  const int64_t r0 = a.cu[seq] + (int64_t)chunk * CK_ROWS;
+  const int n = min(CK_ROWS, (int)(a.cu[seq + 1] - r0));
+  const int i0 = (wave >> 1) * 32, j0 = (wave & 1) * 32;
+  const int cols = gc_cols<T, P>(a.dv);
+  const int64_t item = (int64_t)blockIdx.z * a.H + h;
+  const float* S = a.ws + item * cols * a.dkp;
+  const T* qr = a.q + r0 * a.stride + (int64_t)(h / a.per) * a.dk;
+  const T* kr = a.k + r0 * a.stride + (int64_t)(h / a.per) * a.dk;
+  const T* vr = a.v + r0 * a.stride + (int64_t)h * a.dv;
+  if (t < 64) {
+    double F, peak;
+    float in;
+    gc_gates(p, r0, n, h, t, F, in, peak);
+    const double m0 = P::NORMED ? (double)before_m[item] : 0.;
+    const float m = P::NORMED ? (float)(F + fmax(m0, peak)) : 0.f;
+    Fs[t] = F;
+    ins[t] = in;
+    ms[t] = m;
+    olds[t] = expf((float)(F + m0 - (double)m));
+  }
+  if (P::NORMED && blockIdx.x == 0 && (chunk + 1) * CK_ROWS >= a.cu[seq + 1] - a.cu[seq]) {
+    const float2 e = *reinterpret_cast<const float2*>(a.ends + 2 * item);
+    p.keep_m(reinterpret_cast<float*>(a.state + (int64_t)a.slot[seq] * a.state_stride + a.state_offset), h, fmaxf(e.x + before_m[item], e.y), t);
+  }
+  gc_acc square = {0.f}, out = {0.f};
+  float den = 0.f;                            // NORMED: n . q of row t / 4, this thread's share
+  for (int d0 = 0; d0 < a.dkp; d0 += GC_KB) {
+    const int d = 4 * (t & 7);
+    float4 qx[2], kx[2], sx[2], nx = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = (t >> 3) + 32 * i;
+      qx[i] = gc_tile4(qr, a.stride, row, n, d0 + d, a.dk);
+      kx[i] = gc_tile4(kr, a.stride, row, n, d0 + d, a.dk);
+      sx[i] = gc_tile4(S + (int64_t)c0 * a.dkp, a.dkp, row, a.dv - c0, d0 + d, a.dkp);
+    }
+    if (P::NORMED) nx = gc_tile4(S + (int64_t)a.dv * a.dkp, 0, 0, 1, d0 + d, a.dkp);
+    __syncthreads();                          // (the block before has been read)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int at = ((t >> 3) + 32 * i) * GC_KLD + d;
+      *reinterpret_cast<float4*>(qs + at) = make_float4(qx[i].x * a.q_scale, qx[i].y * a.q_scale, qx[i].z * a.q_scale, qx[i].w * a.q_scale);
+      *reinterpret_cast<float4*>(ks + at) = kx[i];
+      *reinterpret_cast<float4*>(ss + at) = sx[i];
+    }
+    if (P::NORMED && t < 8) *reinterpret_cast<float4*>(ns + d) = nx;
+    __syncthreads();
+#pragma unroll
+    for (int g0 = 0; g0 < GC_KB; g0 += 16) {
+      gc_acc some = {0.f}, dots = {0.f};
+#pragma unroll
+      for (int g = g0; g < g0 + 16; g += 8) {
+        const float4 qv = *reinterpret_cast<const float4*>(qs + (i0 + l32) * GC_KLD + g + 4 * hl);
+        const float4 kv = *reinterpret_cast<const float4*>(ks + (j0 + l32) * GC_KLD + g + 4 * hl);
+        const float4 sv = *reinterpret_cast<const float4*>(ss + (j0 + l32) * GC_KLD + g + 4 * hl);
+        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.x, sv.x, some, 0, 0, 0);
+        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.y, sv.y, some, 0, 0, 0);
+        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.z, sv.z, some, 0, 0, 0);
+        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.w, sv.w, some, 0, 0, 0);
+        if (j0 <= i0) {                       // (the same in the wavefront)
+          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.x, kv.x, dots, 0, 0, 0);
+          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.y, kv.y, dots, 0, 0, 0);
+          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.z, kv.z, dots, 0, 0, 0);
+          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.w, kv.w, dots, 0, 0, 0);
+        }
+      }
+      gc_add(out, some);
+      gc_add(square, dots);
+    }
+    if (P::NORMED) {
+      float some = 0.f;
+#pragma unroll
+      for (int e = 0; e < GC_KB / 4; e += 4) {
+        const float4 qv = *reinterpret_cast<const float4*>(qs + (t >> 2) * GC_KLD + 8 * (t & 3) + e);
+        const float4 nv = *reinterpret_cast<const float4*>(ns + 8 * (t & 3) + e);
+        some = fmaf(qv.x, nv.x, fmaf(qv.y, nv.y, fmaf(qv.z, nv.z, fmaf(qv.w, nv.w, some))));
+      }
+      den += some;
+    }
+  }
+  float4 vx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) vx[i] = gc_tile4(vr, a.stride, (t >> 4) + 16 * i, n, c0 + 4 * (t & 15), a.dv);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(vs + ((t >> 4) + 16 * i) * GC_LD + 4 * (t & 15)) = vx[i];
+  {
+    const int j = j0 + l32;
+    const double Fj = Fs[j];
+    const float inj = ins[j];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int i = i0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+      out[r] *= olds[i];
+      const float e = P::NORMED ? expf((float)(Fs[i] - Fj + (double)inj - (double)ms[i])) : inj * expf((float)(Fs[i] - Fj));
+      square_s[i * GC_LD + j] = j <= i && j < n ? e * square[r] : 0.f;
+    }
+  }
+  __syncthreads();
+  if (P::NORMED) {
+    float some = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      const float4 s = *reinterpret_cast<const float4*>(square_s + (t >> 2) * GC_LD + 16 * (t & 3) + e);
+      some += (s.x + s.y) + (s.z + s.w);
+    }
+    den = fmaf(den, olds[t >> 2], some);
+    den += __shfl_xor(den, 1);
+    den += __shfl_xor(den, 2);
+    if ((t & 3) == 0) dens[t >> 2] = fmaxf(fabsf(den), expf(-ms[t >> 2])) + 1e-6f;
+  }
+#pragma unroll
+  for (int g0 = 0; g0 < CK_ROWS; g0 += 16) {
+    if (g0 >= i0 + 32 || g0 >= n) break;      // (the same in the wavefront)
+    gc_acc some = {0.f};
+#pragma unroll
+    for (int g = g0; g < g0 + 16; g += 8) {
+      const float4 s = *reinterpret_cast<const float4*>(square_s + (i0 + l32) * GC_LD + g + 4 * hl);
+      const float* v = vs + (g + 4 * hl) * GC_LD + j0 + l32;
+      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.x, v[0], some, 0, 0, 0);
+      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.y, v[GC_LD], some, 0, 0, 0);
+      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.z, v[2 * GC_LD], some, 0, 0, 0);
+      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.w, v[3 * GC_LD], some, 0, 0, 0);
+    }
+    gc_add(out, some);
+  }
+  if (P::NORMED) __syncthreads();
+  const int c = c0 + j0 + l32;
+  if (c < a.dv) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int i = i0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+      if (i < n) y[(r0 + i) * a.H * a.dv + (int64_t)h * a.dv + c] = P::NORMED ? out[r] / dens[i] : p.result(out[r], vs[i * GC_LD + j0 + l32], h);
+    }
+  }
+}
+
+// Chunks whose memories are held at once, and the floats of workspace for them: memories, ends and the m before them.
+static inline int64_t gc_window(int rows, int num_seqs, int64_t memory) {
+  const int64_t chunks = (int64_t)rows / CK_ROWS + num_seqs;      // no fewer than the sequences' chunks
+  int64_t most = GC_WINDOW_FLOATS / memory;
+  if (most > 32768) most = 32768;
+  return chunks < most ? chunks : (most < 1 ? 1 : most);
+}
+static inline int64_t gc_floats(int rows, int num_seqs, int max_q_len, int H, int cols, int dkp) {
+  if (rows <= 0 || num_seqs <= 0 || max_q_len <= GC_FROM) return 0;
+  const int64_t memory = (int64_t)H * cols * dkp;
+  return gc_window(rows, num_seqs, memory) * (memory + 4ll * H);
+}
+
+template <typename T, class P>
+static int gc_run(float* y, GcArgs<T> a, const P& p, int rows, float* workspace, const char* name, hipStream_t s) {
+  const int cols = gc_cols<T, P>(a.dv);
+  const int64_t memory = (int64_t)a.H * cols * a.dkp;
+  const int window = (int)gc_window(rows, a.num_seqs, memory), chunks = rows / CK_ROWS + a.num_seqs;
+  a.ws = workspace;
+  a.ends = a.ws + window * memory;
+  float* before_m = a.ends + 2ll * window * a.H;
+  const int kb = (a.dkp + 63) / 64, vb = (a.dv + 63) / 64;
+  for (int t0 = 0; t0 < chunks; t0 += window) {
+    const int nt = chunks - t0 < window ? chunks - t0 : window;
+    gc_share_kernel<T, P><<<dim3(kb * vb, a.H, nt), 256, 0, s>>>(a, p, t0);
+    gc_carry_kernel<T, P><<<dim3((unsigned)((memory / a.H / 4 + 255) / 256), a.H, a.num_seqs), 256, 0, s>>>(a, p, t0, nt, before_m);
+    gc_rows_kernel<T, P><<<dim3(vb, a.H, nt), 256, 0, s>>>(y, a, p, t0, before_m);
+  }
+  return he_check_launch(name);
+}
+
+// Whole fours of every row and head, which the kernels above load at once.
+template <typename T>
+static inline bool gc_takes(const GcArgs<T>& a) {
+  return a.dk % 4 == 0 && a.dv % 4 == 0 && a.stride % 4 == 0 && a.H <= 65535 && a.num_seqs <= 65535 &&
+         (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & (4 * sizeof(T) - 1)) == 0;
+}

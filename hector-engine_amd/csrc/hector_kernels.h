@@ -240,10 +240,12 @@ int he_conv_state(void* out, const void* x, int64_t x_stride, const void* taps, 
 int64_t he_ssm_state_floats(int R, int P, int N);
 // xbc [rows][R P + 2 Q N]: x, then the Q groups' B vectors, then their C vectors; dt_in[row * dt_stride + r].
 // y [rows][R P] fp32 (rows without a sequence are not written). max_q_len: a bound on the rows a sequence brings (0: none).
+// workspace of he_ssm_workspace_floats() floats: sequences of many rows go by chunks (bf16 activations); null: row by row.
+int64_t he_ssm_workspace_floats(int rows, int num_seqs, int max_q_len, int R, int N, int P, int dtype);
 int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int64_t dt_stride, const void* dt_bias,
                 const void* a_log, const void* d_skip, int w_dtype, void* state, int64_t state_stride,
                 int64_t state_offset, const void* cu_seqlens, const void* seq_slot, int rows, int num_seqs,
-                int max_q_len, int R, int Q, int N, int P, int dtype, void* stream);
+                int max_q_len, int R, int Q, int N, int P, int dtype, void* workspace_f32, int64_t workspace_floats, void* stream);
 // out = rms over each of `parts` stretches of (y * silu(z)) * weight; z[row * z_stride + c]. gate_after 1: out =
 // rms over each stretch of y, * weight * sigmoid(z) * out_scale (the gate behind the norm).
 int he_gated_group_norm(void* out, const void* y_f32, const void* z, int64_t z_stride, const void* weight,
@@ -256,14 +258,17 @@ int he_gated_group_norm(void* out, const void* y_f32, const void* z, int64_t z_s
 // he_mlstm_scan: y_f32 [rows, H dv] from q, k [rows, H dk] and v [rows, H dv] (views of rows in_stride elements
 // apart) and the gates' logarithms (raw_gates: their pre-activations, with gate_bias and cap as he_mlstm_gates takes
 // them, and the logarithms are formed inside); S, n and m of a sequence live at state_offset of its row of `state`,
-// he_mlstm_state_floats(H, dk, dv) floats, zeros at a sequence's start. dk up to 512.
+// he_mlstm_state_floats(H, dk, dv) floats, zeros at a sequence's start. dk up to 512. max_q_len: a bound on the rows a
+// sequence brings (0: none); workspace of he_mlstm_workspace_floats() floats: sequences of many rows go by chunks (bf16 activations); null: row by row.
+int64_t he_mlstm_workspace_floats(int rows, int num_seqs, int max_q_len, int H, int dk, int dv, int dtype);
 int64_t he_mlstm_state_floats(int H, int dk, int dv);
 int he_mlstm_gates(void* out_f32, const void* x_f32, const void* bias, int bias_dtype, int rows, int H, float cap,
                    void* stream);
 int he_mlstm_scan(void* y_f32, const void* q, const void* k, const void* v, int64_t in_stride, const void* gates_f32,
                   void* state, int64_t state_stride, int64_t state_offset, const void* cu_seqlens,
                   const void* seq_slot, int rows, int num_seqs, int H, int dk, int dv, float q_scale, int dtype,
-                  int raw_gates, const void* gate_bias, int bias_dtype, float cap, void* stream);
+                  int raw_gates, const void* gate_bias, int bias_dtype, float cap, int max_q_len, void* workspace_f32,
+                  int64_t workspace_floats, void* stream);
 
 // ---- routing and head combination (routing.hip) ---------------------------------
 // logits_f32 [rows][E], or null and x [rows][D] (x_dtype) with router_f32 [E][D]: the kernel forms the logits itself.

@@ -5,8 +5,9 @@
 //   y_t = S_t^T q_t / (max(|n_t . q_t|, exp(-m_t)) + 1e-6)
 // with i_t and f_t the logarithms of the input and forget gates. S, n and m start at zero and live in
 // 32-bit floats in the sequence's row of the cache's state area; everything here is fp32 arithmetic, only
-// q, k and v are read in the activation dtype.
-#include "common.h"
+// q, k and v are read in the activation dtype. Sequences of up to GC_FROM rows are walked row by row, longer ones of
+// bf16 activations go by chunks (gated_chunks.h); with 32-bit activations results do not depend on how the rows were cut into steps.
+#include "gated_chunks.h"
 #include "hector_kernels.h"
 
 #define MM_NPT 8   // key dims of S a thread holds for its value dim
@@ -452,11 +453,49 @@ __global__ void __launch_bounds__(256) mlstm_step_kernel(float* __restrict__ y, 
   }
 }
 
+// The matrix memory by chunks: a head's S as [dv][dkp], n and m once a workgroup of the walks.
+struct MmChunks {
+  static constexpr bool NORMED = true;
+  const float* gates;
+  const void* bias;
+  int bias_dtype, raw, H, dv, dkp, tiles;
+  float cap;
+  __device__ __forceinline__ void gate(int64_t row, int h, float& f, float& in) const {
+    in = gates[row * 2 * H + h];
+    f = gates[row * 2 * H + H + h];
+    if (!raw) return;
+    in = mm_gate_log(in + (bias ? load_param(bias, h, bias_dtype) : 0.f), cap, false);
+    f = mm_gate_log(f + (bias ? load_param(bias, H + h, bias_dtype) : 0.f), cap, true);
+  }
+  __device__ __forceinline__ float* aux(float* st, int h, int tile) const {
+    return st + (int64_t)H * dv * dkp + ((int64_t)h * tiles + tile) * (dkp + 4);
+  }
+  __device__ __forceinline__ float* place(float* st, int h, int c, int d) const {
+    return c < dv ? st + ((int64_t)h * dv + c) * dkp + d : aux(st, h, 0) + d;
+  }
+  __device__ __forceinline__ float m(float* st, int h) const { return aux(st, h, 0)[dkp]; }
+  __device__ __forceinline__ void keep(float* st, int h, int c, int d, const float4& S) const {
+    if (c < dv) *reinterpret_cast<float4*>(place(st, h, c, d)) = S;
+    else
+      for (int i = 0; i < tiles; ++i) *reinterpret_cast<float4*>(aux(st, h, i) + d) = S;
+  }
+  __device__ __forceinline__ void keep_m(float* st, int h, float m, int t) const {
+    for (int i = t; i < tiles; i += 256) aux(st, h, i)[dkp] = m;
+  }
+  __device__ __forceinline__ float result(float y, float, int) const { return y; }
+};
+
+// Floats of workspace he_mlstm_scan wants to go by chunks (0: it walks the rows). max_q_len: the most rows of a sequence, 0: not known.
+extern "C" int64_t he_mlstm_workspace_floats(int rows, int num_seqs, int max_q_len, int H, int dk, int dv, int dtype) {
+  if (H <= 0 || dk <= 0 || dv <= 0 || dtype != HE_BF16) return 0;
+  return gc_floats(rows, num_seqs, max_q_len, H, dv + 1, mm_groups(dk) * MM_NPT);
+}
+
 extern "C" int he_mlstm_scan(void* y_f32, const void* q, const void* k, const void* v, int64_t in_stride,
                              const void* gates_f32, void* state, int64_t state_stride, int64_t state_offset,
                              const void* cu_seqlens, const void* seq_slot, int rows, int num_seqs, int H, int dk, int dv,
                              float q_scale, int dtype, int raw_gates, const void* gate_bias, int bias_dtype, float cap,
-                             void* stream) {
+                             int max_q_len, void* workspace_f32, int64_t workspace_floats, void* stream) {
   HE_REQUIRE(rows >= 0 && num_seqs >= 0 && H > 0 && dk > 0 && dv > 0, "he_mlstm_scan: bad sizes H=%d dk=%d dv=%d", H, dk, dv);
   HE_REQUIRE(dk <= 512, "he_mlstm_scan: key size %d above 512", dk);
   HE_REQUIRE(dtype == HE_BF16 || dtype == HE_F32, "he_mlstm_scan: unknown dtype %d", dtype);
@@ -472,6 +511,16 @@ extern "C" int he_mlstm_scan(void* y_f32, const void* q, const void* k, const vo
   const bool vec = dk % ve == 0 && in_stride < (1 << 24) && (in_stride * esz) % 16 == 0 && (((uintptr_t)q | (uintptr_t)k) & 15) == 0;
   const dim3 grid((dv + PB - 1) / PB, H, num_seqs);
   hipStream_t s = (hipStream_t)stream;
+  const int64_t need = he_mlstm_workspace_floats(rows, num_seqs, max_q_len, H, dk, dv, dtype);
+  if (need > 0 && workspace_f32 != nullptr) {
+    HE_REQUIRE(workspace_floats >= need && ((uintptr_t)workspace_f32 & 15) == 0,
+               "he_mlstm_scan: the workspace has %lld floats of %lld, or is not aligned", (long long)workspace_floats, (long long)need);
+    const MmChunks p = {(const float*)gates_f32, gate_bias, bias_dtype, raw_gates, H, dv, NG * MM_NPT, (int)grid.x, cap};
+    const GcArgs<bf16_t> a = {(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, in_stride, 1, q_scale, (const int32_t*)cu_seqlens,
+                              (const int32_t*)seq_slot, num_seqs, H, dk, dv, NG * MM_NPT, (uint8_t*)state, state_stride,
+                              state_offset, nullptr, nullptr};
+    if (gc_takes(a)) return gc_run((float*)y_f32, a, p, rows, (float*)workspace_f32, "he_mlstm_scan", s);
+  }
   if (rows <= num_seqs) {       // no sequence brings more than a row, or the few that do are walked row by row
 #define MM_STEP(T)                                                                                                       \
   mlstm_step_kernel<T><<<grid, threads, 0, s>>>((float*)y_f32, (const T*)q, (const T*)k, (const T*)v, in_stride,          \

@@ -3,7 +3,7 @@
 // to step lives in its row of the cache's state area, in fp32: the last K-1 inputs of the
 // convolution, [K-1][C], and then the state of the scan, he_ssm_state_floats() floats in the order the
 // scan's threads hold them. Everything that enters the recurrence is fp32.
-#include "common.h"
+#include "gated_chunks.h"
 #include "hector_kernels.h"
 
 __device__ __forceinline__ float ss_silu(float z) { return z / (1.f + expf(-z)); }
@@ -116,7 +116,8 @@ extern "C" int he_conv_state(void* out, const void* x, int64_t x_stride, const v
 // does not depend on the step. A workgroup takes PB value dims of one (sequence, head) and walks the
 // sequence's rows in order; what a token brings (its B and C, the x of the workgroup's value dims,
 // its step size and decay, which one thread a token computes) is staged through LDS a tile of tokens
-// at a time, the next tile's loads in flight while this one is computed. In the state area the
+// at a time, the next tile's loads in flight while this one is computed. Sequences of more than GC_FROM rows of
+// bf16 activations go by chunks (gated_chunks.h); with 32-bit ones results do not depend on how the rows were cut into steps. In the state area the
 // workgroup's share of S lies in the order its threads load it, 16 bytes a lane: [i / 4][thread][i % 4].
 #define SS_PRE 16      // values a thread fetches for the next tile
 // state dims a thread holds. Measured at 64 heads of 64 with a state of 128, one prompt of 2,048 tokens: 0.93 ms
@@ -305,10 +306,40 @@ extern "C" int64_t he_ssm_state_floats(int R, int P, int N) {
   return (int64_t)R * ((P + PB - 1) / PB) * PB * ss_groups(N) * ss_npt(N);
 }
 
+// The scan by chunks: C asks, B is written with weight dt, the state lies as the walk's threads hold it.
+struct SsChunks {
+  static constexpr bool NORMED = false;
+  const bf16_t* dt_in;
+  int64_t dt_stride;
+  const void* dt_bias;
+  const void* a_log;
+  const void* d_skip;
+  int w_dtype, NG, PB, npt, tiles;
+  __device__ __forceinline__ void gate(int64_t row, int h, float& f, float& in) const {
+    in = ss_softplus(to_float(dt_in[row * dt_stride + h]) + load_param(dt_bias, h, w_dtype));
+    f = -expf(load_param(a_log, h, w_dtype)) * in;
+  }
+  __device__ __forceinline__ float* place(float* st, int h, int c, int d) const {
+    const int tile = c / PB, pl = c - tile * PB, ng = d / npt, i4 = (d - ng * npt) / 4;
+    return st + ((int64_t)h * tiles + tile) * PB * NG * npt + ((int64_t)i4 * PB * NG + pl * NG + ng) * 4;
+  }
+  __device__ __forceinline__ void keep(float* st, int h, int c, int d, const float4& S) const { *reinterpret_cast<float4*>(place(st, h, c, d)) = S; }
+  __device__ __forceinline__ float m(float*, int) const { return 0.f; }
+  __device__ __forceinline__ void keep_m(float*, int, float, int) const {}
+  __device__ __forceinline__ float result(float y, float x, int h) const { return fmaf(load_param(d_skip, h, w_dtype), x, y); }
+};
+
+// Floats of workspace he_ssm_scan wants to go by chunks (0: it walks the rows). max_q_len: the most rows of a sequence, 0: not known.
+extern "C" int64_t he_ssm_workspace_floats(int rows, int num_seqs, int max_q_len, int R, int N, int P, int dtype) {
+  if (R <= 0 || N <= 0 || P <= 0 || dtype != HE_BF16) return 0;
+  return gc_floats(rows, num_seqs, max_q_len, R, P, ss_groups(N) * ss_npt(N));
+}
+
 extern "C" int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int64_t dt_stride, const void* dt_bias,
                            const void* a_log, const void* d_skip, int w_dtype, void* state, int64_t state_stride,
                            int64_t state_offset, const void* cu_seqlens, const void* seq_slot, int rows, int num_seqs,
-                           int max_q_len, int R, int Q, int N, int P, int dtype, void* stream) {
+                           int max_q_len, int R, int Q, int N, int P, int dtype, void* workspace_f32, int64_t workspace_floats,
+                           void* stream) {
   HE_REQUIRE(rows >= 0 && num_seqs >= 0 && R > 0 && Q > 0 && N > 0 && P > 0 && R % Q == 0,
              "he_ssm_scan: bad sizes R=%d Q=%d N=%d P=%d", R, Q, N, P);
   HE_REQUIRE(N <= 1024, "he_ssm_scan: state size %d above 1024", N);
@@ -321,6 +352,18 @@ extern "C" int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int6
   const int PB = ss_pb(N, P);
   const int threads = (PB * NG + 63) / 64 * 64;
   const int W = (2 * NG * ss_npt(N) + PB + 2 + 3) & ~3;
+  const int64_t need = he_ssm_workspace_floats(rows, num_seqs, max_q_len, R, N, P, dtype);
+  if (need > 0 && workspace_f32 != nullptr) {
+    HE_REQUIRE(workspace_floats >= need && ((uintptr_t)workspace_f32 & 15) == 0,
+               "he_ssm_scan: the workspace has %lld floats of %lld, or is not aligned", (long long)workspace_floats, (long long)need);
+    const int inner = R * P;
+    const bf16_t* at = (const bf16_t*)xbc;
+    const SsChunks p = {(const bf16_t*)dt_in, dt_stride, dt_bias, a_log, d_skip, w_dtype, NG, PB, ss_npt(N), (P + PB - 1) / PB};
+    const GcArgs<bf16_t> a = {at + inner + Q * N, at + inner, at, inner + 2 * Q * N, R / Q, 1.f, (const int32_t*)cu_seqlens,
+                              (const int32_t*)seq_slot, num_seqs, R, N, P, NG * ss_npt(N), (uint8_t*)state, state_stride,
+                              state_offset, nullptr, nullptr};
+    if (gc_takes(a)) return gc_run((float*)y_f32, a, p, rows, (float*)workspace_f32, "he_ssm_scan", (hipStream_t)stream);
+  }
   int TT = SS_PRE * threads / W;
   TT = TT < 1 ? 1 : (TT > 16 ? 16 : TT);
   if (max_q_len > 0 && TT > max_q_len) TT = max_q_len;      // no sequence brings more rows than that

@@ -62,15 +62,17 @@ _SIGNATURES = {
     "he_conv_state": [c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_int, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr,
                       c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_ptr],
     "he_ssm_state_floats": [c_int, c_int, c_int],
+    "he_ssm_workspace_floats": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "he_ssm_scan": [c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_i64, c_i64, c_ptr, c_ptr,
-                    c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_ptr],
+                    c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_ptr, c_i64, c_ptr],
     "he_gated_group_norm": [c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_int, c_int, c_int, c_int, c_f32, c_int, c_f32,
                             c_int, c_ptr],
     "he_rmsnorm_row_pair": [c_ptr, c_ptr, c_int, c_ptr, c_int, c_int, c_int, c_i64, c_f32, c_int, c_int, c_ptr],
     "he_mlstm_state_floats": [c_int, c_int, c_int],
+    "he_mlstm_workspace_floats": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "he_mlstm_gates": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_f32, c_ptr],
     "he_mlstm_scan": [c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr, c_int, c_int,
-                      c_int, c_int, c_int, c_f32, c_int, c_int, c_ptr, c_int, c_f32, c_ptr],
+                      c_int, c_int, c_int, c_f32, c_int, c_int, c_ptr, c_int, c_f32, c_int, c_ptr, c_i64, c_ptr],
     "he_add_normed": [c_ptr, c_ptr, c_int, c_ptr, c_f32, c_ptr, c_f32, c_int, c_ptr, c_int, c_int, c_int, c_ptr],
     "he_add_normed_pair": [c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_ptr, c_int, c_f32, c_f32, c_ptr, c_f32, c_ptr, c_f32, c_int,
                            c_ptr, c_int, c_int, c_int, c_ptr],
@@ -141,7 +143,9 @@ _SIGNATURES = {
 _RESTYPES = {
     "he_attention_plain_workspace_floats": c_i64,
     "he_ssm_state_floats": c_i64,
+    "he_ssm_workspace_floats": c_i64,
     "he_mlstm_state_floats": c_i64,
+    "he_mlstm_workspace_floats": c_i64,
     "he_decay_state_floats": c_i64,
     "he_decay_workspace_floats": c_i64,
     "he_delta_state_floats": c_i64,

@@ -626,18 +626,32 @@ def conv_state(out, x, taps, bias, state, positions, row_seq, seq_slot, seq_star
                                rows, num_seqs, C, K, int(all_single), int(act), dtype_code(x.dtype), _stream()))
 
 
+def _workspace(t):
+    """(address, floats) of a workspace that may be None."""
+    if t is None:
+        return None, 0
+    _need(t, "workspace", torch.float32)
+    return t.data_ptr(), t.numel()
+
+
 def ssm_state_floats(R: int, P: int, N: int) -> int:
     """Floats of a sequence's scan state (the state dims padded to the threads' share)."""
     return int(_lib.load().he_ssm_state_floats(R, P, N))
 
 
+def ssm_workspace_floats(rows: int, num_seqs: int, max_q_len: int, R: int, N: int, P: int, dtype: torch.dtype) -> int:
+    """Floats of workspace ssm_scan wants to take a step of these sizes and activations by chunks (0: it walks the rows)."""
+    return int(_lib.load().he_ssm_workspace_floats(rows, num_seqs, max_q_len, R, N, P, dtype_code(dtype)))
+
+
 @_op("ssm_scan")
 def ssm_scan(y, xbc, dt, dt_bias, a_log, d_skip, state, state_offset: int, cu_seqlens, seq_slot,
-             rows: int, num_seqs: int, R: int, Q: int, N: int, P: int, max_q_len: int = 0) -> None:
+             rows: int, num_seqs: int, R: int, Q: int, N: int, P: int, max_q_len: int = 0, workspace=None) -> None:
     """y (fp32 [rows, R P]) = the selective scan of xbc [rows, R P + 2 Q N] (x, then B, then C) with step
     sizes softplus(dt + dt_bias) (dt: a view [rows, R] of wider rows), per head r the decay
     exp(-exp(a_log_r) dt) and the skip d_skip_r; the state [R][P][N'] lives at byte state_offset of a
-    sequence's row of `state` and is carried on. max_q_len: a bound on the rows a sequence brings (0: none)."""
+    sequence's row of `state` and is carried on. max_q_len: a bound on the rows a sequence brings (0: none).
+    workspace: fp32, ssm_workspace_floats elements or more: long sequences go by chunks (None: row by row)."""
     C = R * P + 2 * Q * N
     _need(y, "y", torch.float32, (None, R * P))
     _need(xbc, "xbc", None, (None, C))
@@ -658,7 +672,7 @@ def ssm_scan(y, xbc, dt, dt_bias, a_log, d_skip, state, state_offset: int, cu_se
     _lib.check(L.he_ssm_scan(y.data_ptr(), xbc.data_ptr(), dt.data_ptr(), dt.stride(0), dt_bias.data_ptr(),
                              a_log.data_ptr(), d_skip.data_ptr(), dtype_code(dt_bias.dtype), state.data_ptr(),
                              state.stride(0), state_offset, cu_seqlens.data_ptr(), seq_slot.data_ptr(), rows,
-                             num_seqs, int(max_q_len), R, Q, N, P, dtype_code(xbc.dtype), _stream()))
+                             num_seqs, int(max_q_len), R, Q, N, P, dtype_code(xbc.dtype), *_workspace(workspace), _stream()))
 
 
 @_op("gated_group_norm")
@@ -1080,14 +1094,21 @@ def mlstm_gates(out, x, bias, rows: int, H: int, cap: float) -> None:
                                 rows, H, float(cap), _stream()))
 
 
+def mlstm_workspace_floats(rows: int, num_seqs: int, max_q_len: int, H: int, dk: int, dv: int, dtype: torch.dtype) -> int:
+    """Floats of workspace mlstm_scan wants to take a step of these sizes and activations by chunks (0: it walks the rows)."""
+    return int(_lib.load().he_mlstm_workspace_floats(rows, num_seqs, max_q_len, H, dk, dv, dtype_code(dtype)))
+
+
 @_op("mlstm_scan")
 def mlstm_scan(y, q, k, v, gates, state, state_offset: int, cu_seqlens, seq_slot, rows: int, num_seqs: int,
-               H: int, dk: int, dv: int, q_scale: float, raw_gates: bool = False, gate_bias=None, cap: float = 0.0) -> None:
+               H: int, dk: int, dv: int, q_scale: float, raw_gates: bool = False, gate_bias=None, cap: float = 0.0,
+               max_q_len: int = 0, workspace=None) -> None:
     """y (fp32 [rows, H dv]) = the matrix memory's answers to q, after each row's k and v went in under the
     row's gates (gates: fp32 [rows, 2 H], the logarithms). q, k [rows, H dk] and v [rows, H dv] are views of
     the same wider rows; the memory lives at byte state_offset of a sequence's row of `state` and is carried on.
     raw_gates: `gates` holds the pre-activations, and the kernel forms the logarithms itself from them, gate_bias
-    ([2 H] or None) and cap, with mlstm_gates' arithmetic."""
+    ([2 H] or None) and cap, with mlstm_gates' arithmetic. max_q_len: a bound on the rows a sequence brings (0: none);
+    workspace: fp32, mlstm_workspace_floats elements or more: long sequences go by chunks (None: row by row)."""
     _need(y, "y", torch.float32, (None, H * dv))
     _need(gates, "gates", torch.float32, (None, 2 * H))
     stride = q.stride(0)
@@ -1111,7 +1132,7 @@ def mlstm_scan(y, q, k, v, gates, state, state_offset: int, cu_seqlens, seq_slot
                                state.data_ptr(), state.stride(0), state_offset, cu_seqlens.data_ptr(),
                                seq_slot.data_ptr(), rows, num_seqs, H, dk, dv, float(q_scale), dtype_code(q.dtype),
                                int(raw_gates), _ptr(gate_bias), dtype_code(gate_bias.dtype) if gate_bias is not None else F32,
-                               float(cap), _stream()))
+                               float(cap), int(max_q_len), *_workspace(workspace), _stream()))
 
 
 @_op("route_tokens")

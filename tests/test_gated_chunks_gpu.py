@@ -1,0 +1,144 @@
+"""The matrix memory and the state-space scan by chunks of rows: against the recurrences in 64 bits and beside the walk row by
+row, over edges of chunks, of blocks of key and value dims, and gates from keeping everything to forgetting at once."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from hector_engine_amd.kernels import ops
+    return ops
+
+
+def rnd(*shape, seed, scale=1.0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed), dtype=F64) * scale
+
+
+def i32(*v):
+    return torch.tensor(v, dtype=torch.int32, device="cuda")
+
+
+def cu_of(lengths):
+    return i32(0, *torch.tensor(lengths).cumsum(0).tolist())
+
+
+def rel(got, want):
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+# first a step of these lengths, then one of those that goes on from its states (both have a sequence of more than 64 rows)
+STEPS = [[130, 1, 64, 260, 65], [3, 200, 128, 1, 97]]
+
+
+def mlstm_plain(q, k, v, i, f, state):
+    """One head: q, k [T, dk], v [T, dv], logarithms i, f [T]; state (S, n, m) or None."""
+    S, n, m = state or (torch.zeros(q.shape[1], v.shape[1], dtype=F64), torch.zeros(q.shape[1], dtype=F64), torch.zeros((), dtype=F64))
+    y = []
+    for t in range(len(q)):
+        new = torch.maximum(f[t] + m, i[t])
+        a, b = torch.exp(f[t] + m - new), torch.exp(i[t] - new)
+        S, n, m = a * S + b * torch.outer(k[t], v[t]), a * n + b * k[t], new
+        y.append(S.t() @ q[t] / (torch.maximum((n @ q[t]).abs(), torch.exp(-m)) + 1e-6))
+    return torch.stack(y), (S, n, m)
+
+
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 256), (3, 20, 36), (1, 8, 4), (2, 132, 68)])
+@pytest.mark.parametrize("keep,write", [(3.0, -1.0), (-20.0, 0.0), (30.0, 12.0)])
+def test_matrix_memory_by_chunks(ops, H, dk, dv, keep, write):
+    slots, room = i32(2, 0, 4, 1, 3), 5
+    state = {way: torch.zeros((room, 4 * ops.mlstm_state_floats(H, dk, dv)), dtype=torch.uint8, device="cuda") for way in ("chunks", "walk")}
+    plain = [[None] * H for _ in range(5)]
+    for s, lengths in enumerate(STEPS):
+        rows = sum(lengths)
+        x = rnd(rows, H * (2 * dk + dv), seed=s)
+        if write > 1:                        # (every row is remembered: with signs of their own n . q would be a small difference)
+            x[:, :2 * H * dk] = x[:, :2 * H * dk].abs()
+        x = x.bfloat16()
+        gates = torch.cat([rnd(rows, H, seed=10 + s, scale=2.0) + write, -torch.nn.functional.softplus(-(rnd(rows, H, seed=20 + s, scale=2.0) + keep))], 1).float()
+        xd, gd, cu = x.cuda(), gates.cuda(), cu_of(lengths)
+        q, k, v = xd[:, :H * dk], xd[:, H * dk:2 * H * dk], xd[:, 2 * H * dk:]
+        floats = ops.mlstm_workspace_floats(rows, 5, max(lengths), H, dk, dv, torch.bfloat16)
+        assert floats > 0
+        got = {}
+        for way in state:
+            got[way] = torch.full((rows, H * dv), float("nan"), device="cuda")
+            ws = torch.full((floats,), float("nan"), device="cuda") if way == "chunks" else None
+            ops.mlstm_scan(got[way], q, k, v, gd, state[way], 0, cu, slots, rows, 5, H, dk, dv, dk ** -0.5, max_q_len=max(lengths), workspace=ws)
+        want, r = torch.empty(rows, H * dv, dtype=F64), 0
+        xq, g64 = x.double(), gates.double()
+        for b, n in enumerate(lengths):
+            at = slice(r, r + n)
+            for h in range(H):
+                cols = slice(h * dk, (h + 1) * dk)
+                want[at, h * dv:(h + 1) * dv], plain[b][h] = mlstm_plain(
+                    xq[at, :H * dk][:, cols] * dk ** -0.5, xq[at, H * dk:2 * H * dk][:, cols], xq[at, 2 * H * dk + h * dv:2 * H * dk + (h + 1) * dv],
+                    g64[at, h], g64[at, H + h], plain[b][h])
+            r += n
+        e = {way: rel(got[way].cpu(), want) for way in got}
+        # 32-bit sums and exponentials: a few 2^-24
+        assert e["chunks"] <= max(2e-6, 1.5 * e["walk"])
+
+
+def ssm_plain(C, B, x, f, dt, S):
+    y = []
+    for t in range(len(x)):
+        S = torch.exp(f[t]) * S + dt[t] * torch.outer(B[t], x[t])
+        y.append(S.t() @ C[t])
+    return torch.stack(y), S
+
+
+@pytest.mark.parametrize("R,Q,N,P", [(8, 2, 128, 64), (3, 1, 20, 36), (2, 2, 4, 8), (4, 2, 260, 132)])
+@pytest.mark.parametrize("decay", [-3.0, 1.0, 5.0])
+def test_state_space_by_chunks(ops, R, Q, N, P, decay):
+    slots, room, C = i32(2, 0, 4, 1, 3), 5, R * P + 2 * Q * N
+    state = {way: torch.zeros((room, 64 + 4 * ops.ssm_state_floats(R, P, N)), dtype=torch.uint8, device="cuda") for way in ("chunks", "walk")}
+    a_log, bias, skip = (rnd(R, seed=i).float() for i in (1, 2, 3))
+    a_log += decay
+    plain = [[torch.zeros(N, P, dtype=F64) for _ in range(R)] for _ in range(5)]
+    for s, lengths in enumerate(STEPS):
+        rows = sum(lengths)
+        xbc, dt_in = rnd(rows, C, seed=30 + s).bfloat16(), rnd(rows, R + 3, seed=40 + s).bfloat16()
+        xd, dd, cu = xbc.cuda(), dt_in.cuda(), cu_of(lengths)
+        floats = ops.ssm_workspace_floats(rows, 5, max(lengths), R, N, P, torch.bfloat16)
+        assert floats > 0
+        got = {}
+        for way in state:
+            got[way] = torch.full((rows, R * P), float("nan"), device="cuda")
+            ws = torch.full((floats,), float("nan"), device="cuda") if way == "chunks" else None
+            ops.ssm_scan(got[way], xd, dd[:, 2:2 + R], bias.cuda(), a_log.cuda(), skip.cuda(), state[way], 64, cu, slots, rows, 5, R, Q, N, P,
+                         max_q_len=max(lengths), workspace=ws)
+        dt = torch.nn.functional.softplus(dt_in[:, 2:2 + R].double() + bias.double())
+        f = -torch.exp(a_log.double()) * dt
+        x64, want, r = xbc.double(), torch.empty(rows, R * P, dtype=F64), 0
+        for b, n in enumerate(lengths):
+            at = slice(r, r + n)
+            for h in range(R):
+                g = h // (R // Q)
+                x = x64[at, h * P:(h + 1) * P]
+                y, plain[b][h] = ssm_plain(x64[at, R * P + (Q + g) * N:R * P + (Q + g + 1) * N], x64[at, R * P + g * N:R * P + (g + 1) * N],
+                                           x, f[at, h], dt[at, h], plain[b][h])
+                want[at, h * P:(h + 1) * P] = y + skip[h].double() * x
+            r += n
+        e = {way: rel(got[way].cpu(), want) for way in got}
+        assert e["chunks"] <= max(2e-6, 1.5 * e["walk"])
+
+
+def test_what_goes_by_chunks(ops):
+    """Short or unknown lengths and 32-bit activations are walked, and so are heads that are no whole fours, whatever workspace is given."""
+    bf16 = torch.bfloat16
+    assert ops.mlstm_workspace_floats(1000, 2, 64, 4, 64, 64, bf16) == ops.ssm_workspace_floats(1000, 2, 0, 4, 64, 64, bf16) == 0
+    assert ops.mlstm_workspace_floats(1000, 2, 65, 4, 64, 64, torch.float32) == ops.ssm_workspace_floats(1000, 2, 65, 4, 64, 64, torch.float32) == 0
+    assert ops.mlstm_workspace_floats(1000, 2, 65, 4, 64, 64, bf16) > 0 and ops.ssm_workspace_floats(1000, 2, 65, 4, 64, 64, bf16) > 0
+    H, dk, dv, rows = 2, 6, 10, 150
+    x, gates = rnd(rows, H * (2 * dk + dv), seed=5).bfloat16().cuda(), (-rnd(rows, 2 * H, seed=6).abs()).float().cuda()
+    got = []
+    for ws in (None, torch.empty(ops.mlstm_workspace_floats(rows, 1, rows, H, dk, dv, bf16), device="cuda")):
+        y = torch.empty(rows, H * dv, device="cuda")
+        state = torch.zeros((1, 4 * ops.mlstm_state_floats(H, dk, dv)), dtype=torch.uint8, device="cuda")
+        ops.mlstm_scan(y, x[:, :H * dk], x[:, H * dk:2 * H * dk], x[:, 2 * H * dk:], gates, state, 0, i32(0, rows), i32(0), rows, 1, H, dk, dv, 1.0,
+                       max_q_len=rows, workspace=ws)
+        got.append(y)
+    assert torch.equal(*got)
