@@ -17,7 +17,11 @@
 // them in wavefront order: O = sum_w O_w 2^(m_w - M), L = sum_w l_w 2^(m_w - M). With
 // Z = 1 the workgroup stores O / L; with more (few sequences: one workgroup per sequence
 // and kv head would leave most of the chip, and its memory bandwidth, idle) it stores
-// (M, L, O) and attention_merge_kernel joins the Z parts in a second launch.
+// (M, L, O), and the Z parts are joined by the workgroup that leaves the last of them (fused_join), told by a counter, or,
+// without counters, by attention_merge_kernel in a second launch: the same operations in the same order. What such
+// a step pays is the start and end of launches: the second one 3.7 to 4.9 us a layer and the gap before it, the way of the parts to memory
+// and back inside the first one about 1 us less (eight steps of 24 layers of a 0.5B model 7.21 -> 7.01 ms, of the 7B shape at batch 8
+// 27.67 -> 27.31).
 #include "attention_tiles.h"
 #include "hector_kernels.h"
 
@@ -137,18 +141,76 @@ __device__ __forceinline__ void rotate_q(bf16x8* qf, float (&x)[NT / 2][8], int 
                            pack2_bf16(x[ks][4], x[ks][5]), pack2_bf16(x[ks][6], x[ks][7])));
 }
 
+// Parts that another workgroup of the launch will read: stored through to what all XCDs share, and read from there, as
+// atomics of the whole chip are. (Ordinary stores and a release by every workgroup cost more than the second launch:
+// each writes back all that its XCD's L2 holds; 8 sequences, 256 workgroups, 28.2 ms a pass of 8 steps and 28 layers, with the
+// second launch 27.6, so 27.3.)
+__device__ __forceinline__ void shared_store2(float* p, float a, float b) {
+  const uint64_t v = (uint64_t)__float_as_uint(a) | (uint64_t)__float_as_uint(b) << 32;
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 shared_load2(const float* p) {
+  const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+}
+
+// The join of the Z parts (Z <= 64) of GT heads by one workgroup of 256 threads, with the bits attention_merge_kernel gives: the
+// weights and their sum by a wavefront a head, lane s part s; then four sums a dim, of the parts s % 4 = 0 .. 3 in order, added in that order.
+// store(hg, d, v): the four results of head hg of the tile from dim d on. lds: 65 floats a head.
+template <int NT, typename Store>
+__device__ __forceinline__ void fused_join(const float* ws_o, const float* ws_ml, int64_t head0, int GT, int Z, float* lds, Store store) {
+  constexpr int HD = 16 * NT, PER = 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float* inv = lds + 64 * GT;
+  for (int hg = wave; hg < GT; hg += 4) {
+    const float2 ml = lane < Z ? shared_load2(ws_ml + 2 * ((head0 + hg) * Z + lane)) : make_float2(-INFINITY, 0.f);
+    const float M = wave_max(ml.x);
+    const float w = ml.x > -INFINITY ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
+    const float L = wave_sum(ml.y * w);
+    lds[64 * hg + lane] = w;
+    if (lane == 0) inv[hg] = L > 0.f ? 1.f / L : 0.f;
+  }
+  __syncthreads();
+  for (int item = threadIdx.x; item < GT * (HD / 4); item += 256) {
+    const int hg = item / (HD / 4), d = 4 * (item % (HD / 4));
+    const float* o = ws_o + (head0 + hg) * Z * HD + d;
+    float4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < Z; s0 += PER) {
+      float4 v[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const float* at = o + (int64_t)min(s0 + i, Z - 1) * HD;
+        const float2 lo = shared_load2(at), hi = shared_load2(at + 2);
+        v[i] = make_float4(lo.x, lo.y, hi.x, hi.y);
+      }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        if (s0 + i >= Z) break;
+        const float w = lds[64 * hg + s0 + i];
+        float4& a = acc[i & 3];
+        a.x = fmaf(v[i].x, w, a.x), a.y = fmaf(v[i].y, w, a.y), a.z = fmaf(v[i].z, w, a.z), a.w = fmaf(v[i].w, w, a.w);
+      }
+    }
+    const float f = inv[hg];
+    store(hg, d, make_float4((((acc[0].x + acc[1].x) + acc[2].x) + acc[3].x) * f, (((acc[0].y + acc[1].y) + acc[2].y) + acc[3].y) * f,
+                             (((acc[0].z + acc[1].z) + acc[2].z) + acc[3].z) * f, (((acc[0].w + acc[1].w) + acc[2].w) + acc[3].w) * f));
+  }
+}
+
 // SLICED: qkv is null and the projection row comes as the fp32 sums of its K slices,
 // qkv_part [qkv_slices][.][qkv_stride], slice_stride elements from slice to slice.
 template <int NT, bool SLICED>
 __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
-    uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml,
+    uint16_t* __restrict__ out, float* ws_o, float* ws_ml,      // (other workgroups' parts are read back: no __restrict__)
     const uint16_t* __restrict__ qkv, const float* __restrict__ qkv_part, int qkv_slices,
     int64_t slice_stride, int64_t qkv_stride,
     const void* __restrict__ bias, int bias_dtype, uint16_t* kpool, uint16_t* vpool,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ row_seq,
     const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ page_table, int max_blocks,
     int num_pages, const float* __restrict__ inv_freq, int rotary_dim, int H, int KVH,
-    int head_tiles, int window, float scale, int write_kv, int out_pieces) {
+    int head_tiles, int window, float scale, int write_kv, int out_pieces, int32_t* counters) {
   constexpr int HD = 16 * NT;
   constexpr int KS = (HD + 31) / 32;
   extern __shared__ __attribute__((aligned(16))) float lds[];   // [NW][GT][HD] O, then [NW][GT][2] (m, l)
@@ -198,7 +260,7 @@ __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
     return out_pieces ? out + ((c >> 3) * gridDim.y + row) * 8 + (c & 7) : out + (int64_t)row * H * HD + c;
   };
   if (seq < 0) {                           // padding row: zeros (from the merge kernel if there is one)
-    if (Z == 1)
+    if (Z == 1 || (counters != nullptr && z == 0))
       for (int i = threadIdx.x; i < GT * HD; i += blockDim.x) *out_at(i / HD, i % HD) = 0;
     return;
   }
@@ -392,13 +454,38 @@ __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
       w2.x = pack2_bf16(acc.x * inv, acc.y * inv);
       w2.y = pack2_bf16(acc.z * inv, acc.w * inv);
       *reinterpret_cast<uint2*>(out_at(hg, d)) = w2;
-    } else {                               // a part without keys stores (-inf, 0, zeros)
+    } else if (counters != nullptr) {      // a part without keys stores (-inf, 0, zeros)
+      float* o = ws_o + (head * Z + z) * HD + d;
+      shared_store2(o, acc.x, acc.y);
+      shared_store2(o + 2, acc.z, acc.w);
+      if (d == 0) shared_store2(ws_ml + 2 * (head * Z + z), M, L);
+    } else {
       *reinterpret_cast<float4*>(ws_o + (head * Z + z) * HD + d) = acc;
       if (d == 0) {
         ws_ml[2 * (head * Z + z)] = M;
         ws_ml[2 * (head * Z + z) + 1] = L;
       }
     }
+  }
+  if (Z > 1 && counters != nullptr) {
+    // Every wavefront's part has arrived (the wait; a barrier alone does not say so of stores), then one thread counts the
+    // workgroup in; the last one puts the counter back for the next launch and reads all parts.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(lds);
+    if (threadIdx.x == 0) {
+      int32_t* counter = counters + (int64_t)row * gridDim.x + blockIdx.x;
+      const int before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (before == Z - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *last = before == Z - 1;
+    }
+    __syncthreads();
+    const bool joins = *last;
+    __syncthreads();
+    if (joins)
+      fused_join<NT>(ws_o, ws_ml, (int64_t)row * H + kvh * G + 16 * ht, GT, Z, lds, [&](int hg, int d, const float4& v) {
+        *reinterpret_cast<uint2*>(out_at(hg, d)) = make_uint2(pack2_bf16(v.x, v.y), pack2_bf16(v.z, v.w));
+      });
   }
   asm volatile("" :: "v"(touched));
 }
@@ -466,7 +553,8 @@ extern "C" int he_attention_decode_fused_bf16(void* out, const void* qkv, const 
                                               int rows, int H, int KVH, int hd, int window,
                                               float scale, int max_keys, int spread, int write_kv,
                                               int out_pieces, void* workspace_f32,
-                                              int64_t workspace_floats, void* stream) {
+                                              int64_t workspace_floats, void* counters_i32,
+                                              int64_t num_counters, void* stream) {
   HE_REQUIRE(rows >= 0 && H > 0 && KVH > 0 && hd > 0 && max_keys > 0,
              "he_attention_decode_fused_bf16: bad sizes");
   HE_REQUIRE(scale > 0.f, "he_attention_decode_fused_bf16: the score scale must be positive");
@@ -499,6 +587,8 @@ extern "C" int he_attention_decode_fused_bf16(void* out, const void* qkv, const 
   float* ws_o = (float*)workspace_f32;
   float* ws_ml = ws_o ? ws_o + (int64_t)rows * H * Z * hd : nullptr;
   const size_t lds = (size_t)nw * gt * (hd + 2) * sizeof(float);
+  // parts are cut for four wavefronts a workgroup (fused_shape); a counter per (row, kv head, head tile)
+  int32_t* counters = Z > 1 && nw == 4 && (int64_t)rows * KVH * head_tiles <= num_counters ? (int32_t*)counters_i32 : nullptr;
   hipStream_t s = (hipStream_t)stream;
   dim3 grid(KVH * head_tiles, rows, Z);
 #define FUSED_LAUNCH(NTV, SL)                                                                   \
@@ -509,7 +599,7 @@ extern "C" int he_attention_decode_fused_bf16(void* out, const void* qkv, const 
         (uint16_t*)vpool, (const int32_t*)positions, (const int32_t*)row_seq,                   \
         (const int32_t*)seq_slot, (const int32_t*)page_table, max_blocks, num_pages,            \
         (const float*)inv_freq, rotary_dim, H, KVH, head_tiles, window, scale, write_kv,        \
-        out_pieces)
+        out_pieces, counters)
 #define FUSED(NTV)                                                                              \
   case NTV:                                                                                     \
     if (qkv_part != nullptr) FUSED_LAUNCH(NTV, true); else FUSED_LAUNCH(NTV, false);            \
@@ -522,6 +612,6 @@ extern "C" int he_attention_decode_fused_bf16(void* out, const void* qkv, const 
 #undef FUSED
 #undef FUSED_LAUNCH
   const int rc = he_check_launch("he_attention_decode_fused_bf16");
-  if (rc || Z == 1) return rc;
+  if (rc || Z == 1 || counters != nullptr) return rc;
   return he_attention_merge_parts(out, ws_o, ws_ml, row_seq, rows, H, hd, Z, out_pieces, stream);
 }

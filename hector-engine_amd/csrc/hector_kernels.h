@@ -184,7 +184,9 @@ int he_attention_decode_bf16(void* out, const void* q, const void* kpool, const 
                              const void* slopes_f32, const void* table_f32, int table_len, float cap, void* stream);
 int64_t he_attention_decode_workspace_floats(int rows, int H, int KVH, int hd, int max_keys);
 // bf16, one query row per sequence, one launch for bias + rotary + cache write + attention +
-// merge (a second launch joins the parts where few sequences are cut across workgroups).
+// merge. Where few sequences are cut across workgroups, the last workgroup of a (row, kv head, tile of 16 heads) joins the
+// parts, counted by counters_i32: zeros before the first launch that uses them and again after every one, for one launch at a
+// time; without them, or with fewer than the launch has such groups, a second launch joins the parts. The results are the same bits.
 // qkv: the un-biased projection rows [rows, (H + 2 KVH) hd]. he_attention_decode_fused_ok: 1
 // when the sizes are taken (head_dim 64 or 128, rotated whole). out_pieces: out lies piece-major
 // (as he_gemm_blocksplit_fused_bf16 reads it with x_pieces). spread: one sequence of the step has
@@ -205,7 +207,7 @@ int he_attention_decode_fused_bf16(void* out, const void* qkv, const void* qkv_p
                                    const void* inv_freq, int rotary_dim, int rows, int H, int KVH,
                                    int hd, int window, float scale, int max_keys, int spread,
                                    int write_kv, int out_pieces, void* workspace_f32,
-                                   int64_t workspace_floats,
+                                   int64_t workspace_floats, void* counters_i32, int64_t num_counters,
                                    void* stream);
 // bf16, prompt steps: tiles of queries of one sequence against its cache rows. kernel: 0 leaves
 // the choice to the library; 1: 16 queries a wavefront, operands straight from global memory

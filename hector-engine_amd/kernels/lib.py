@@ -124,7 +124,7 @@ _SIGNATURES = {
     "he_attention_decode_fused_workspace_floats": [c_int, c_int, c_int, c_int, c_int, c_int],
     "he_attention_decode_fused_bf16": [c_ptr, c_ptr, c_ptr, c_int, c_i64, c_i64, c_ptr, c_int, c_ptr, c_ptr, c_ptr, c_ptr,
                                        c_ptr, c_ptr, c_int, c_int, c_ptr, c_int, c_int, c_int, c_int,
-                                       c_int, c_int, c_f32, c_int, c_int, c_int, c_int, c_ptr, c_i64, c_ptr],
+                                       c_int, c_int, c_f32, c_int, c_int, c_int, c_int, c_ptr, c_i64, c_ptr, c_i64, c_ptr],
     "he_attention_prefill_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_int,
                                   c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_f32, c_int,
                                   c_int, c_int, c_ptr, c_i64, c_int, c_ptr, c_int, c_ptr, c_i64, c_ptr, c_ptr, c_int, c_f32, c_ptr],

@@ -1462,7 +1462,7 @@ def attention_decode_fused_workspace_floats(rows: int, H: int, KVH: int, hd: int
 def attention_decode_fused(out, qkv, bias, kpool, vpool, positions, row_seq, seq_slot, page_table,
                            inv_freq, rotary_dim: int, rows: int, H: int, KVH: int, hd: int,
                            window: int, scale: float, max_keys: int, write_kv: bool,
-                           workspace, out_pieces: bool = False, spread: bool = False) -> None:
+                           workspace, out_pieces: bool = False, spread: bool = False, counters=None) -> None:
     """One-token steps in one launch: bias, rotation of q and of the new key, cache write,
     attention over the cache, merge. spread: one sequence has several times the keys of the
     others (every sequence's keys are then cut across more workgroups; the workspace is asked for
@@ -1471,7 +1471,10 @@ def attention_decode_fused(out, qkv, bias, kpool, vpool, positions, row_seq, seq
     alone where the run reads another run's cache (write_kv False). out_pieces: out is written
     piece-major for exactly `rows` rows (see :func:`to_pieces`). seq_slot None: page_table has a row
     per row of the step ([rows or more, blocks]: the page numbers of the row's sequence), not a
-    row per slot; the kernel then asks for them at its start, without the chain through the slot."""
+    row per slot; the kernel then asks for them at its start, without the chain through the slot.
+    counters: int32 zeros, left as zeros, for one launch at a time (a caller's own): where the keys are cut across workgroups
+    the last one to finish then joins the parts and no second launch does; as many as rows x kv heads x tiles of 16
+    heads of a group, fewer are not used."""
     width = (H + 2 * KVH) * hd if write_kv else H * hd
     _need(out, "out", torch.bfloat16)
     slices, slice_stride = 0, 0
@@ -1504,6 +1507,8 @@ def attention_decode_fused(out, qkv, bias, kpool, vpool, positions, row_seq, seq
     _need(inv_freq, "inv_freq", torch.float32, (rotary_dim // 2,))
     if workspace is not None:
         _need(workspace, "workspace", torch.float32)
+    if counters is not None:
+        _need(counters, "counters", torch.int32)
     L = _lib.load()
     _lib.check(L.he_attention_decode_fused_bf16(
         out.data_ptr(), qkv.data_ptr() if not slices else None, qkv.data_ptr() if slices else None, slices,
@@ -1512,7 +1517,8 @@ def attention_decode_fused(out, qkv, bias, kpool, vpool, positions, row_seq, seq
         positions.data_ptr(), row_seq.data_ptr(), _ptr(seq_slot), page_table.data_ptr(),
         page_table.shape[1], kpool.shape[0], inv_freq.data_ptr(), rotary_dim, rows, H, KVH, hd,
         window, float(scale), max_keys, int(spread), int(write_kv), int(out_pieces), _ptr(workspace),
-        workspace.numel() if workspace is not None else 0, _stream()))
+        workspace.numel() if workspace is not None else 0, _ptr(counters), counters.numel() if counters is not None else 0,
+        _stream()))
 
 
 def attention_prefill_parts(num_seqs: int, max_q_len: int, H: int, hd: int, most_keys: int, total_rows: int = 0,

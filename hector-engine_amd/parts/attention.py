@@ -87,6 +87,9 @@ class AttentionCase:
     fusable: bool       # head size and position encoding are ones the fused one-token kernel takes
 
 
+JOIN_COUNTERS = 1024
+
+
 def keys_uneven(lengths: list[int], before=None) -> bool:
     """Whether one sequence of a one-token step has several times the keys of the others (and
     thousands of them): the one-token attention then cuts every sequence's keys across more
@@ -336,6 +339,9 @@ class Attention(Mixer):
                                 device=wo.device)
             self.table = stored.float()[rows].t().contiguous()
         self.position.bind(tensors)
+        # the fused one-token kernel's counters of finished workgroups (zeros between launches): its launches that cut the
+        # keys across workgroups have few rows, as a rule fewer than a workgroup a compute unit
+        self._arrived = torch.zeros(JOIN_COUNTERS, dtype=torch.int32, device=wo.device)
 
     def _by_map(self, which: str, t: torch.Tensor) -> torch.Tensor:
         """A differential attention's stored rows (or bias) as the kernels' heads read them: q from
@@ -404,7 +410,7 @@ class Attention(Mixer):
                                    ctx.row_seq, None if by_row is not None else ctx.seq_slot,
                                    by_row if by_row is not None else cache.page_table, rot[0], rot[1],
                                    rows, H, KVH, hd, self.window, self.scale, ctx.max_keys,
-                                   cache.writes, ws, out_pieces=pieces, spread=uneven)
+                                   cache.writes, ws, out_pieces=pieces, spread=uneven, counters=self._arrived)
         return self.o_proj(PieceRows(out) if pieces else out, rows, ctx, sink=ctx.take_sink())
 
     def _encoded_q(self, x, ctx: StepContext, cache: LayerCache):
