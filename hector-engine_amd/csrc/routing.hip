@@ -5,19 +5,7 @@
 
 #define ROUTE_MAX_EXPERTS 1024
 
-// (value, index) maximum over the wavefront; among equal values the lowest index wins
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(v, m);
-    const int oi = __shfl_xor(i, m);
-    if (ov > v || (ov == v && oi < i)) {
-      v = ov;
-      i = oi;
-    }
-  }
-}
-
-// One wavefront a row. logits [rows][E] fp32, or, with x and router given, the router's product itself:
+// One workgroup a row. logits [rows][E] fp32, or, with x and router given, the router's product itself:
 // logits[e] = sum_i x[row][i] * router[e][i] in fp32 (router fp32 [E][D]; a lane adds its elements i = lane,
 // lane + 64, ... in that order, the lanes' sums meet in the wavefront's butterfly: one fixed order a row,
 // whatever else the step holds). bias (or null): a stored number an output, added to its logit first. x_pieces: the bf16
@@ -28,158 +16,200 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
 // to one). The last E - real outputs are experts without weights whose result is the input
 // itself: their weights are added up in column `real` of dense. dense [rows][real + 1] holds the
 // weight of every expert (0 where not chosen); ids / weights [rows][top] list the chosen ones.
+//
+// What bounds a step of few rows is the chain: the router's rows come from memory, so a wavefront asks for those of up to four
+// outputs together; the choice is made by the first wavefront alone, PL outputs a lane in registers, without a barrier or a
+// walk through LDS a choice. (2 rows of 2048, 18 outputs in 3 groups, 4 chosen: 14.5 us with eight wavefronts that meet at two barriers a choice and
+// ask for one output at a time, 9 so; 2048 rows 41 us and 31; one row of 300 outputs in 5 groups, 8 chosen, 89 and 36.)
 #define ROUTE_WAVES 8
+
+// The dot products of row x with the router's rows e0, e0 + ROUTE_WAVES, ... (OUT of them, those beyond E repeat the last): four elements
+// a lane and turn, four sums a lane that meet in index order.
+template <int OUT>
+__device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x_dtype, const float* router, int64_t row, int D, int E, int e0,
+                                           int x_pieces) {
+  const int lane = threadIdx.x & 63;
+  const bool vec = (D & 3) == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)router & 15) == 0;
+  const float* w[OUT];
+  float a[OUT][4];
+#pragma unroll
+  for (int o = 0; o < OUT; ++o) {
+    w[o] = router + (int64_t)min(e0 + o * ROUTE_WAVES, E - 1) * D;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[o][j] = 0.f;
+  }
+  if (vec) {
+    // row-major: four elements i at 4 i; piece-major [D / 8][rows][8]: half i & 1 of the row's piece i / 2
+    const uint2* xh = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * row : row * (D >> 2));
+    const float4* xf = reinterpret_cast<const float4*>((const float*)x + row * D);
+    const int64_t piece = 2 * (int64_t)gridDim.x;
+#pragma unroll 4
+    for (int i = lane; i < (D >> 2); i += 64) {
+      float4 xv;
+      if (x_dtype == HE_BF16) {
+        const uint2 b = x_pieces ? xh[(i >> 1) * piece + (i & 1)] : xh[i];
+        xv = make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16),
+                         __uint_as_float(b.y & 0xffff0000u));
+      } else {
+        xv = xf[i];
+      }
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) {
+        const float4 wv = reinterpret_cast<const float4*>(w[o])[i];
+        a[o][0] = fmaf(xv.x, wv.x, a[o][0]);
+        a[o][1] = fmaf(xv.y, wv.y, a[o][1]);
+        a[o][2] = fmaf(xv.z, wv.z, a[o][2]);
+        a[o][3] = fmaf(xv.w, wv.w, a[o][3]);
+      }
+    }
+  } else {
+    for (int i = lane; i < D; i += 64) {
+      const float xv = x_dtype == HE_BF16 ? bf16_bits_to_float(((const uint16_t*)x)[row * D + i])
+                                          : ((const float*)x)[row * D + i];
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) a[o][0] = fmaf(xv, w[o][i], a[o][0]);
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < OUT; ++o) z[o] = wave_sum((a[o][0] + a[o][1]) + (a[o][2] + a[o][3]));
+}
+
+// The lowest index among the largest of the lanes' values (lane, lane + 64, ...), NaN never; `none` if all are NaN.
+template <int PL>
+__device__ __forceinline__ int route_argmax(const float (&c)[PL], int none) {
+  float v = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) v = fmaxf(v, c[j]);
+  v = wave_max(v);
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(c[j] == v);
+    if (hit != 0) return 64 * j + __ffsll((long long)hit) - 1;       // (the same in all lanes)
+  }
+  return none;
+}
+
+template <int PL>
 __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
     float* __restrict__ dense, int32_t* __restrict__ ids, float* __restrict__ weights, const float* __restrict__ logits,
     const void* __restrict__ x, int x_dtype, const float* __restrict__ router, int D,
     const void* __restrict__ correction, int c_dtype, int E, int real, int groups, int keep, int top, float scale,
     int normalize, const void* __restrict__ bias, int bias_dtype, int x_pieces) {
-  __shared__ float s_sh[ROUTE_MAX_EXPERTS];
-  __shared__ float c_sh[ROUTE_MAX_EXPERTS];
-  __shared__ float d_sh[ROUTE_MAX_EXPERTS + 1];
-  __shared__ float g_sh[ROUTE_MAX_EXPERTS];
-  __shared__ float z[ROUTE_MAX_EXPERTS];
+  __shared__ float z_sh[64 * PL], c_sh[64 * PL];
   const int64_t row = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  // The first wavefront makes the choice; with x given, all of them form the logits first, each the outputs
-  // e = wave, wave + 8, ...: four elements a lane and turn, four sums a lane that meet in index order.
-  const bool lead = wave == 0;
   if (x != nullptr) {
-    const bool vec = (D & 3) == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)router & 15) == 0;
-    for (int e = wave; e < E; e += ROUTE_WAVES) {
-      const float* w = router + (int64_t)e * D;
-      float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-      if (vec && x_dtype == HE_BF16) {
-        // row-major: four elements i at 4 i; piece-major [D / 8][rows][8]: half i & 1 of the row's piece i / 2
-        const uint2* xr = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * row : row * (D >> 2));
-        const int64_t piece = 2 * (int64_t)gridDim.x;
-#pragma unroll 4
-        for (int i = lane; i < (D >> 2); i += 64) {
-          const uint2 xv = x_pieces ? xr[(i >> 1) * piece + (i & 1)] : xr[i];
-          const float4 wv = reinterpret_cast<const float4*>(w)[i];
-          a0 = fmaf(__uint_as_float(xv.x << 16), wv.x, a0);
-          a1 = fmaf(__uint_as_float(xv.x & 0xffff0000u), wv.y, a1);
-          a2 = fmaf(__uint_as_float(xv.y << 16), wv.z, a2);
-          a3 = fmaf(__uint_as_float(xv.y & 0xffff0000u), wv.w, a3);
-        }
-      } else if (vec) {
-        const float4* xr = reinterpret_cast<const float4*>((const float*)x + row * D);
-#pragma unroll 4
-        for (int i = lane; i < (D >> 2); i += 64) {
-          const float4 xv = xr[i];
-          const float4 wv = reinterpret_cast<const float4*>(w)[i];
-          a0 = fmaf(xv.x, wv.x, a0);
-          a1 = fmaf(xv.y, wv.y, a1);
-          a2 = fmaf(xv.z, wv.z, a2);
-          a3 = fmaf(xv.w, wv.w, a3);
-        }
+    for (int e0 = wave; e0 < E; e0 += 4 * ROUTE_WAVES) {
+      if (e0 + 2 * ROUTE_WAVES < E) {
+        float z[4];
+        route_dots<4>(z, x, x_dtype, router, row, D, E, e0, x_pieces);
+#pragma unroll
+        for (int o = 0; o < 4; ++o)
+          if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_sh[e0 + o * ROUTE_WAVES] = z[o];
       } else {
-        for (int i = lane; i < D; i += 64) {
-          const float xv = x_dtype == HE_BF16 ? bf16_bits_to_float(((const uint16_t*)x)[row * D + i])
-                                              : ((const float*)x)[row * D + i];
-          a0 = fmaf(xv, w[i], a0);
-        }
+        float z[2];
+        route_dots<2>(z, x, x_dtype, router, row, D, E, e0, x_pieces);
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+          if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_sh[e0 + o * ROUTE_WAVES] = z[o];
       }
-      const float acc = wave_sum((a0 + a1) + (a2 + a3));
-      if (lane == 0) z[e] = bias ? acc + load_param(bias, e, bias_dtype) : acc;
     }
-  } else if (lead) {
-    for (int e = lane; e < E; e += 64) z[e] = logits[row * E + e] + (bias ? load_param(bias, e, bias_dtype) : 0.f);
+    __syncthreads();
   }
-  __syncthreads();
-  // from here on the first wavefront works; the others only keep the barriers' count
-  if (lead) {
-    float mx = -INFINITY;
-    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
-    mx = wave_max(mx);
-    float sum = 0.f;
-    for (int e = lane; e < E; e += 64) {
-      const float v = expf(z[e] - mx);
-      s_sh[e] = v;
-      sum += v;
-    }
-    sum = wave_sum(sum);
-    const float inv = 1.f / sum;
-    for (int e = lane; e < E; e += 64) {
-      const float s = s_sh[e] * inv;
-      s_sh[e] = s;
-      // (without a correction the choice is made on the logits themselves: the same order, and no two meet at zero)
-      c_sh[e] = correction ? s + load_param(correction, e, c_dtype) : z[e];
-    }
-    for (int e = lane; e <= real; e += 64) d_sh[e] = 0.f;
+  if (wave != 0) return;
+  // element j of a lane's arrays is output lane + 64 j; those beyond E are NaN to the choice
+  float z[PL], s[PL], c[PL], d[PL];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    const int e = lane + 64 * j;
+    z[j] = s[j] = d[j] = 0.f;
+    if (e >= E) continue;
+    z[j] = (x != nullptr ? z_sh[e] : logits[row * E + e]) + (bias ? load_param(bias, e, bias_dtype) : 0.f);
+    mx = fmaxf(mx, z[j]);
   }
-  __syncthreads();
-  const int size = E / groups;
+  mx = wave_max(mx);
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    if (lane + 64 * j >= E) continue;
+    s[j] = expf(z[j] - mx);
+    sum += s[j];
+  }
+  sum = wave_sum(sum);
+  const float inv = 1.f / sum;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    const int e = lane + 64 * j;
+    s[j] *= inv;
+    // (without a correction the choice is made on the logits themselves: the same order, and no two meet at zero)
+    c[j] = e >= E ? NAN : correction ? s[j] + load_param(correction, e, c_dtype) : z[j];
+  }
   if (keep < groups) {
-    if (lead) {
-      for (int g = lane; g < groups; g += 64) {
-        float best = -INFINITY;
-        for (int i = 0; i < size; ++i) best = fmaxf(best, c_sh[g * size + i]);
-        g_sh[g] = best;
-      }
+    // a lane ranks whole groups; the kept ones are marked by NaN, then the others' outputs are masked
+    const int size = E / groups;
+#pragma unroll
+    for (int j = 0; j < PL; ++j) c_sh[lane + 64 * j] = c[j];
+    __builtin_amdgcn_wave_barrier();
+    float g[PL];
+#pragma unroll
+    for (int j = 0; j < PL; ++j) {
+      const int group = lane + 64 * j;
+      g[j] = NAN;
+      if (group >= groups) continue;
+      float best = -INFINITY;
+      for (int i = 0; i < size; ++i) best = fmaxf(best, c_sh[group * size + i]);
+      g[j] = best == INFINITY ? NAN : best;      // (such a group is kept beside the `keep` best)
     }
-    __syncthreads();
-    // the `keep` best groups are marked by +inf in g_sh, then the others' outputs are masked
     for (int k = 0; k < keep; ++k) {
-      float v = -INFINITY;
-      int idx = 0x7fffffff;
-      if (lead) {
-        for (int g = lane; g < groups; g += 64) {
-          const float gv = g_sh[g];
-          if (gv != INFINITY && (gv > v || (gv == v && g < idx))) {
-            v = gv;
-            idx = g;
-          }
-        }
-        wave_argmax(v, idx);
-      }
-      __syncthreads();
-      if (lead && lane == 0 && idx < groups) g_sh[idx] = INFINITY;
-      __syncthreads();
+      const int best = route_argmax<PL>(g, E);
+#pragma unroll
+      for (int j = 0; j < PL; ++j)
+        if (best == lane + 64 * j) g[j] = NAN;
     }
-    if (lead) {
-      for (int e = lane; e < E; e += 64)
-        if (g_sh[e / size] != INFINITY) c_sh[e] = -INFINITY;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < PL; ++j) c_sh[lane + 64 * j] = g[j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < PL; ++j) {
+      const int e = lane + 64 * j;
+      if (e < E && !isnan(c_sh[e / size])) c[j] = -INFINITY;
     }
-    __syncthreads();
   }
-  float chosen_sum = 0.f;     // lane 0 of the first wavefront: the chosen outputs' scores, added in the order of the choice
+  float chosen_sum = 0.f, rest = 0.f;      // the chosen outputs' scores; the weights of those from `real` on: both in the order of the choice
   for (int k = 0; k < top; ++k) {
-    float v = -INFINITY;
-    int idx = 0x7fffffff;
-    if (lead) {
-      for (int e = lane; e < E; e += 64) {
-        const float cv = c_sh[e];
-        // a chosen output is marked by NaN, which no comparison takes
-        if (cv > v || (cv == v && e < idx)) {
-          v = cv;
-          idx = e;
-        }
-      }
-      wave_argmax(v, idx);
+    const int e = route_argmax<PL>(c, E);
+    const bool found = e < E;
+    float score = 0.f;
+#pragma unroll
+    for (int j = 0; j < PL; ++j)
+      if (e >> 6 == j) score = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[j]), e & 63));
+    const float w = found ? score * scale : 0.f;
+    if (found) {
+      chosen_sum += score;
+      if (e >= real) rest += w;
+#pragma unroll
+      for (int j = 0; j < PL; ++j)
+        if (e == lane + 64 * j) c[j] = NAN, d[j] = w;
     }
-    __syncthreads();
-    if (lead && lane == 0) {
-      const bool found = idx < E;
-      const int e = found ? idx : 0;
-      const float w = found ? s_sh[e] * scale : 0.f;
-      if (found) {
-        c_sh[e] = NAN;
-        d_sh[e < real ? e : real] += w;
-        chosen_sum += s_sh[e];
-      }
+    if (lane == 0) {
       ids[row * top + k] = found ? e : -1;
+      // normalize: the chosen outputs' weights are made to sum to `scale` (the softmax over the chosen logits alone), below
       weights[row * top + k] = w;
     }
-    __syncthreads();
   }
-  if (lead) {
-    // normalize: the chosen outputs' weights are made to sum to `scale` (the softmax over the chosen logits alone)
-    const float norm = normalize ? 1.f / __shfl(chosen_sum, 0) : 1.f;
-    for (int e = lane; e <= real; e += 64) dense[row * (real + 1) + e] = normalize ? d_sh[e] * norm : d_sh[e];
+  const float norm = normalize ? 1.f / chosen_sum : 1.f;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    const int e = lane + 64 * j;
+    if (e < real) dense[row * (real + 1) + e] = normalize ? d[j] * norm : d[j];
+  }
+  if (lane == 0) {
+    dense[row * (real + 1) + real] = normalize ? rest * norm : rest;
     if (normalize)
-      for (int k = lane; k < top; k += 64) weights[row * top + k] *= norm;
+      for (int k = 0; k < top; ++k) weights[row * top + k] *= norm;
   }
 }
 
@@ -200,10 +230,14 @@ extern "C" int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32
   HE_REQUIRE(!x_pieces || (x != nullptr && x_dtype == HE_BF16 && (D & 7) == 0 && (((uintptr_t)x | (uintptr_t)router_f32) & 15) == 0),
              "he_route_tokens: piece-major rows are bf16, 16-byte aligned and a multiple of 8 wide");
   if (rows == 0) return 0;
-  route_kernel<<<rows, 64 * ROUTE_WAVES, 0, (hipStream_t)stream>>>((float*)dense_f32, (int32_t*)ids_i32, (float*)weights_f32,
-                                                     (const float*)logits_f32, x, x_dtype, (const float*)router_f32, D,
-                                                     correction, c_dtype, E, real, groups, keep, top, scale, normalize, bias, bias_dtype,
-                                                     x_pieces);
+#define ROUTE_LAUNCH(PL)                                                                                                       \
+  route_kernel<PL><<<rows, 64 * ROUTE_WAVES, 0, (hipStream_t)stream>>>(                                                         \
+      (float*)dense_f32, (int32_t*)ids_i32, (float*)weights_f32, (const float*)logits_f32, x, x_dtype, (const float*)router_f32, D, \
+      correction, c_dtype, E, real, groups, keep, top, scale, normalize, bias, bias_dtype, x_pieces)
+  if (E <= 64) ROUTE_LAUNCH(1);
+  else if (E <= 256) ROUTE_LAUNCH(4);
+  else ROUTE_LAUNCH(16);
+#undef ROUTE_LAUNCH
   return he_check_launch("he_route_tokens");
 }
 
