@@ -285,6 +285,11 @@ int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32, const voi
 int he_gemm_tall_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
                       int64_t ldx, int64_t ldw, int64_t ldo, int epilogue, int bm, float alpha, float limit, float up_shift,
                       float cubic, void* stream);
+// gemm_few_tiles.hip: out bf16 [M][ldo] = x [M][ldx] w [N][ldw]^T (+ bias) in tiles of he_gemm_few_tiles_tile(M, N) (0: no tile makes the
+// product one round of the chip). K a multiple of 64, N of 4, operands 16-byte aligned.
+int he_gemm_few_tiles_tile(int M, int N);
+int he_gemm_few_tiles_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
+                           int64_t ldx, int64_t ldw, int64_t ldo, int tile, void* stream);
 // The experts of a routed feed-forward over the rows that chose them (gemm_tall.hip): scratch sizes, and the whole
 // (down null: the activations alone).
 int he_group_rows_most_tiles(int rows, int top, int groups, int bm);

@@ -3,6 +3,7 @@ the host, then launch on torch's current stream. Tensors are torch tensors on
 the GPU; nothing here computes in torch."""
 from __future__ import annotations
 
+import functools
 import torch
 
 from . import kv_layout as layout
@@ -1233,6 +1234,27 @@ def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
     _lib.check(_lib.load().he_gemm_tall_bf16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias),
                                              dtype_code(bias.dtype) if bias is not None else F32, M, N, K, K, K, cols, epilogue,
                                              bm, float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+
+
+@functools.lru_cache(maxsize=4096)
+def few_tiles_tile(M: int, N: int) -> int:
+    """The tile gemm_few_tiles would take (BM << 16 | BN), 0 where no tile makes the product one round of the chip."""
+    return int(_lib.load().he_gemm_few_tiles_tile(M, N))
+
+
+@_op("gemm_few_tiles")
+def gemm_few_tiles(out, x, w, bias, M: int, tile: int) -> None:
+    """out[M, N] = x[M, K] . w[N, K]^T (+ bias), bf16, in tiles as few_tiles_tile gives them. K a multiple of 64, N of 4."""
+    N, K = w.shape
+    _need(out, "out", torch.bfloat16, (None, N))
+    _need(x, "x", torch.bfloat16, (None, K))
+    _need(w, "w", torch.bfloat16)
+    if bias is not None:
+        _need(bias, "bias", None, (N,))
+    if min(out.shape[0], x.shape[0]) < M:
+        raise ValueError("gemm_few_tiles: buffers smaller than the row count")
+    _lib.check(_lib.load().he_gemm_few_tiles_bf16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias),
+                                                  dtype_code(bias.dtype) if bias is not None else F32, M, N, K, K, K, N, tile, _stream()))
 
 
 def routed_groups_sizes(rows: int, top: int, real: int, bm: int) -> tuple[int, int]:
