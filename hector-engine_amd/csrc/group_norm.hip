@@ -56,6 +56,59 @@ __global__ __launch_bounds__(256) void add_group_normed_kernel(
   }
 }
 
+// The same, bit for bit, where a lane's elements of a group (lane, lane + 64, ...: at most PER) fit its registers and both norms have
+// the same groups, so that a lane norms again what it has just added: every element is read once, all of a
+// group's loads are out before the first sum, and nothing is waited for between the two norms. The kernel above reads a row
+// three times, each time behind the sum before it: 4 rows of 2048 in 4 groups, a branch added and normed on
+// 7.1 us, so 5.4; 3,001 rows 27 and 21.
+template <typename TD, typename TO, int PER>
+__global__ __launch_bounds__(256) void add_group_normed_regs_kernel(
+    float* __restrict__ resid, const TD* __restrict__ delta, const void* __restrict__ weight, int w_dtype, int groups,
+    float eps, float delta_scale, TO* __restrict__ out, const void* __restrict__ next_weight, float next_eps, int D) {
+  const int64_t row = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int width = D / groups;
+  for (int g = wave; g < groups; g += waves) {
+    const int c0 = g * width;
+    float* r = resid + row * D + c0;
+    float x[PER], v[PER], w[PER], nw[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = min(lane + 64 * k, width - 1);      // (no load behind a condition)
+      v[k] = r[i];
+      if (delta != nullptr) {
+        x[k] = to_float(delta[row * D + c0 + i]);
+        w[k] = load_param(weight, c0 + i, w_dtype);
+      }
+      if (next_weight != nullptr) nw[k] = load_param(next_weight, c0 + i, w_dtype);
+    }
+    if (delta != nullptr) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < PER; ++k)
+        if (lane + 64 * k < width) ss = fmaf(x[k], x[k], ss);
+      const float inv = delta_scale / sqrtf(wave_sum(ss) / (float)width + eps);
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        v[k] = fmaf(x[k] * inv, w[k], v[k]);
+        if (lane + 64 * k < width) r[lane + 64 * k] = v[k];
+      }
+    }
+    if (out == nullptr) continue;
+    float inv = 1.f;
+    if (next_weight != nullptr) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < PER; ++k)
+        if (lane + 64 * k < width) ss = fmaf(v[k], v[k], ss);
+      inv = 1.f / sqrtf(wave_sum(ss) / (float)width + next_eps);
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if (lane + 64 * k < width) out[row * D + c0 + lane + 64 * k] = from_float<TO>(next_weight != nullptr ? v[k] * inv * nw[k] : v[k]);
+  }
+}
+
 extern "C" int he_add_group_normed(void* resid_f32, const void* delta, int delta_dtype, const void* weight,
                                    int w_dtype, int groups, float eps, float delta_scale, void* out, int out_dtype,
                                    const void* next_weight, int next_groups, float next_eps, int rows, int D,
@@ -72,48 +125,74 @@ extern "C" int he_add_group_normed(void* resid_f32, const void* delta, int delta
   if (rows == 0 || (delta == nullptr && out == nullptr)) return 0;
   hipStream_t s = (hipStream_t)stream;
   const int threads = D / (groups > 0 ? groups : 1) >= 256 || groups >= 4 ? 256 : (groups >= 2 ? 128 : 64);
+  // (a branch is added, or a norm taken; of both the groups must be the same)
+  const int parts = delta != nullptr ? groups : next_weight != nullptr ? next_groups : 1;
+  const int per = (D / parts + 63) / 64;
+  // (more than 16 elements a lane of many rows: 3,001 rows of 8192 in 4 groups 77 us, 95 in registers; 4 rows 12.7 and 9.3)
+  const bool regs = per <= (rows <= 64 ? 32 : 16) && (delta == nullptr ? next_weight != nullptr : next_weight == nullptr || out == nullptr || next_groups == groups);
+#define GN_REGS(TD, TO, PER)                                                                                       \
+  add_group_normed_regs_kernel<TD, TO, PER><<<rows, threads, 0, s>>>((float*)resid_f32, (const TD*)delta, weight, w_dtype,  \
+                                                                     parts, eps, delta_scale, (TO*)out,             \
+                                                                     out != nullptr ? next_weight : nullptr, next_eps, D)
 #define GN_LAUNCH(TD, TO)                                                                                          \
-  add_group_normed_kernel<TD, TO><<<rows, threads, 0, s>>>((float*)resid_f32, (const TD*)delta, weight, w_dtype,  \
+  if (regs && per <= 1) GN_REGS(TD, TO, 1);                                                                        \
+  else if (regs && per <= 2) GN_REGS(TD, TO, 2);                                                                   \
+  else if (regs && per <= 4) GN_REGS(TD, TO, 4);                                                                   \
+  else if (regs && per <= 8) GN_REGS(TD, TO, 8);                                                                   \
+  else if (regs && per <= 16) GN_REGS(TD, TO, 16);                                                                 \
+  else if (regs) GN_REGS(TD, TO, 32);                                                                              \
+  else add_group_normed_kernel<TD, TO><<<rows, threads, 0, s>>>((float*)resid_f32, (const TD*)delta, weight, w_dtype,  \
                                                            groups, eps, delta_scale, (TO*)out, next_weight,        \
                                                            next_groups, next_eps, D)
   const bool db = delta != nullptr && delta_dtype == HE_BF16, ob = out != nullptr && out_dtype == HE_BF16;
-  if (db && ob) GN_LAUNCH(bf16_t, bf16_t);
-  else if (db) GN_LAUNCH(bf16_t, float);
-  else if (ob) GN_LAUNCH(float, bf16_t);
-  else GN_LAUNCH(float, float);
+  if (db && ob) { GN_LAUNCH(bf16_t, bf16_t); }
+  else if (db) { GN_LAUNCH(bf16_t, float); }
+  else if (ob) { GN_LAUNCH(float, bf16_t); }
+  else { GN_LAUNCH(float, float); }
 #undef GN_LAUNCH
+#undef GN_REGS
   return he_check_launch("he_add_group_normed");
 }
 
 // out[r, i] = a z / rms(z) + b z^2 / rms(z^2) + c z^3 / rms(z^3) + e over the W values z of row r, with
 // rms(x) = sqrt(mean(x^2) + eps) and the four numbers (a, b, c, e) in `numbers`. out may be x itself.
+#define PN_KEPT 8      // elements a thread reads once (4 rows of 8192: 6.5 us with two passes and a sum after the other, 4.4)
 template <typename T>
 __global__ __launch_bounds__(1024) void polynorm_kernel(T* out, const T* x,
                                                         const void* __restrict__ numbers, int n_dtype, int W, float eps) {
-  __shared__ float scratch[16];
+  __shared__ float scratch[48];
   const int64_t row = blockIdx.x;
   const T* z = x + row * W;
   float s2 = 0.f, s4 = 0.f, s6 = 0.f;
-  for (int i = threadIdx.x; i < W; i += blockDim.x) {
-    const float v = to_float(z[i]);
+  float keep[PN_KEPT];      // a thread's first elements: read once
+#pragma unroll
+  for (int k = 0; k < PN_KEPT; ++k) keep[k] = to_float(z[min((int)(threadIdx.x + k * blockDim.x), W - 1)]);
+  auto add = [&](float v) {
     const float v2 = v * v;
     s2 += v2;
     s4 = fmaf(v2, v2, s4);
     s6 = fmaf(v2 * v, v2 * v, s6);
-  }
-  s2 = block_sum(s2, scratch);
+  };
+#pragma unroll
+  for (int k = 0; k < PN_KEPT; ++k)
+    if ((int)(threadIdx.x + k * blockDim.x) < W) add(keep[k]);
+  for (int i = threadIdx.x + PN_KEPT * blockDim.x; i < W; i += blockDim.x) add(to_float(z[i]));
+  // the three sums side by side, each as block_sum forms it
+  s2 = wave_sum(s2), s4 = wave_sum(s4), s6 = wave_sum(s6);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = (blockDim.x + 63) >> 6;
+  if (lane == 0) scratch[wave] = s2, scratch[16 + wave] = s4, scratch[32 + wave] = s6;
   __syncthreads();
-  s4 = block_sum(s4, scratch);
-  __syncthreads();
-  s6 = block_sum(s6, scratch);
+  s2 = s4 = s6 = 0.f;
+  for (int w = 0; w < waves; ++w) s2 += scratch[w], s4 += scratch[16 + w], s6 += scratch[32 + w];
   const float a = load_param(numbers, 0, n_dtype) / sqrtf(s2 / (float)W + eps);
   const float b = load_param(numbers, 1, n_dtype) / sqrtf(s4 / (float)W + eps);
   const float c = load_param(numbers, 2, n_dtype) / sqrtf(s6 / (float)W + eps);
   const float e = load_param(numbers, 3, n_dtype);
-  for (int i = threadIdx.x; i < W; i += blockDim.x) {
-    const float v = to_float(z[i]);
-    out[row * W + i] = from_float<T>(fmaf(a, v, fmaf(b, v * v, fmaf(c, v * v * v, e))));
-  }
+  auto value = [&](float v) { return fmaf(a, v, fmaf(b, v * v, fmaf(c, v * v * v, e))); };
+#pragma unroll
+  for (int k = 0; k < PN_KEPT; ++k)
+    if ((int)(threadIdx.x + k * blockDim.x) < W) out[row * W + threadIdx.x + k * blockDim.x] = from_float<T>(value(keep[k]));
+  for (int i = threadIdx.x + PN_KEPT * blockDim.x; i < W; i += blockDim.x) out[row * W + i] = from_float<T>(value(to_float(z[i])));
 }
 
 extern "C" int he_polynorm(void* out, const void* x, const void* numbers, int n_dtype, int rows, int W, float eps,

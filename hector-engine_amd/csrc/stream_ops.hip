@@ -32,17 +32,35 @@ extern "C" int he_depth_mix(void* resid_f32, void* kept_f32, int64_t plane, cons
 }
 
 // out[r, :] = a[r, :] + sigmoid(sum_i x[r, i] * g[i]) * b[r, :]; x [rows, Dx], a, b, out [rows, D]; the sum in fp32.
-template <typename T>
+// KEPT: a thread's first elements, asked for together, a and b beside the sum they wait for (4 rows of 2048: 4.9 us with a load at a time, 4.1).
+template <typename T, int KEPT>
 __global__ __launch_bounds__(256) void gated_add_kernel(T* __restrict__ out, const T* __restrict__ a,
                                                         const T* __restrict__ b, const T* __restrict__ x,
                                                         const void* __restrict__ g, int g_dtype, int D, int Dx) {
   __shared__ float scratch[16];
   const int64_t row = blockIdx.x;
+  float xv[KEPT], gv[KEPT], av[KEPT], bv[KEPT];
+#pragma unroll
+  for (int k = 0; k < KEPT; ++k) {
+    const int i = min((int)(threadIdx.x + k * blockDim.x), Dx - 1), j = min((int)(threadIdx.x + k * blockDim.x), D - 1);
+    xv[k] = to_float(x[row * Dx + i]);
+    gv[k] = load_param(g, i, g_dtype);
+    av[k] = to_float(a[row * D + j]);
+    bv[k] = to_float(b[row * D + j]);
+  }
   float dot = 0.f;
-  for (int i = threadIdx.x; i < Dx; i += blockDim.x) dot = fmaf(to_float(x[row * Dx + i]), load_param(g, i, g_dtype), dot);
+#pragma unroll
+  for (int k = 0; k < KEPT; ++k)
+    if ((int)(threadIdx.x + k * blockDim.x) < Dx) dot = fmaf(xv[k], gv[k], dot);
+  for (int i = threadIdx.x + KEPT * blockDim.x; i < Dx; i += blockDim.x) dot = fmaf(to_float(x[row * Dx + i]), load_param(g, i, g_dtype), dot);
   dot = block_sum(dot, scratch);
   const float w = 1.f / (1.f + expf(-dot));
-  for (int i = threadIdx.x; i < D; i += blockDim.x)
+#pragma unroll
+  for (int k = 0; k < KEPT; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i < D) out[row * D + i] = from_float<T>(fmaf(w, bv[k], av[k]));
+  }
+  for (int i = threadIdx.x + KEPT * blockDim.x; i < D; i += blockDim.x)
     out[row * D + i] = from_float<T>(fmaf(w, to_float(b[row * D + i]), to_float(a[row * D + i])));
 }
 
@@ -53,9 +71,13 @@ extern "C" int he_gated_add(void* out, const void* a, const void* b, const void*
   if (rows == 0) return 0;
   const int threads = D >= 1024 ? 256 : (D >= 256 ? 128 : 64);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == HE_BF16)
-    gated_add_kernel<bf16_t><<<rows, threads, 0, s>>>((bf16_t*)out, (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)x, g, g_dtype, D, Dx);
-  else
-    gated_add_kernel<float><<<rows, threads, 0, s>>>((float*)out, (const float*)a, (const float*)b, (const float*)x, g, g_dtype, D, Dx);
+#define GA_LAUNCH(T, KEPT) \
+  gated_add_kernel<T, KEPT><<<rows, threads, 0, s>>>((T*)out, (const T*)a, (const T*)b, (const T*)x, g, g_dtype, D, Dx)
+  const bool few = D <= 2 * threads && Dx <= 2 * threads;
+  if (dtype == HE_BF16 && few) GA_LAUNCH(bf16_t, 2);
+  else if (dtype == HE_BF16) GA_LAUNCH(bf16_t, 8);
+  else if (few) GA_LAUNCH(float, 2);
+  else GA_LAUNCH(float, 8);
+#undef GA_LAUNCH
   return he_check_launch("he_gated_add");
 }
