@@ -33,6 +33,7 @@
 // four sequences of 32 rows of 128 heads 54 and 55.
 #define GC_FROM 64
 
+#define GC_FORGETS -1e7f
 typedef float gc_acc __attribute__((ext_vector_type(16)));
 
 template <typename T>
@@ -82,6 +83,9 @@ __device__ __forceinline__ void gc_gates(const P& p, int64_t r0, int n, int h, i
   float f;
   p.gate(r0 + min(lane, n - 1), h, f, in);
   if (lane >= n) f = 0.f, in = P::NORMED ? -INFINITY : 0.f;
+  // (a row that forgets everything has f = -inf, and differences of sums with it would be no numbers: exp of what stands in its place is 0 too, and
+  // 64 of them are known to 1e-7 in 64 bits; NaN stays)
+  if (f < GC_FORGETS) f = GC_FORGETS;
   F = (double)f;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -129,7 +133,8 @@ __global__ __launch_bounds__(256) void gc_share_kernel(GcArgs<T> a, P p, int t0)
     float in;
     gc_gates(p, r0, n, h, t, F, in, peak);
     const double Fn = __shfl(F, 63), G = P::NORMED ? Fn + __shfl(peak, 63) : 0.;
-    weight[t] = P::NORMED ? expf((float)(Fn - F + (double)in - G)) : in * expf((float)(Fn - F));
+    // (in = -inf writes nothing, also where all of a chunk's rows have it and G is -inf)
+    weight[t] = !P::NORMED ? in * expf((float)(Fn - F)) : in == -INFINITY ? 0.f : expf((float)(Fn - F + (double)in - G));
     if (t == 0 && blockIdx.x == 0) *reinterpret_cast<float2*>(a.ends + 2 * ((int64_t)blockIdx.z * a.H + h)) = make_float2((float)Fn, (float)G);
   }
   __syncthreads();

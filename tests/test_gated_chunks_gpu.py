@@ -82,6 +82,44 @@ def test_matrix_memory_by_chunks(ops, H, dk, dv, keep, write):
         assert e["chunks"] <= max(2e-6, 1.5 * e["walk"])
 
 
+def test_matrix_memory_of_closed_gates(ops):
+    """Input gates closed (-inf) for the first chunk and a half, then here and there; rows that forget everything (-inf) on either side of a
+    chunk's edge: finite, and as the walk has it."""
+    H, dk, dv, rows = 2, 32, 64, 200
+    x = rnd(rows, H * (2 * dk + dv), seed=7).bfloat16().cuda()
+    gates = torch.cat([rnd(rows, H, seed=8), -rnd(rows, H, seed=9).abs()], 1)
+    gates[:96, 0] = -torch.inf
+    gates[100:110, 1] = -torch.inf
+    gates[[127, 128, 150], H] = -torch.inf
+    gates[[20, 64], H + 1] = -torch.inf
+    got = []
+    for ws in (None, torch.full((ops.mlstm_workspace_floats(rows, 1, rows, H, dk, dv, torch.bfloat16),), float("nan"), device="cuda")):
+        y = torch.empty(rows, H * dv, device="cuda")
+        state = torch.zeros((1, 4 * ops.mlstm_state_floats(H, dk, dv)), dtype=torch.uint8, device="cuda")
+        for at in (slice(0, 130), slice(130, rows)):
+            n = at.stop - at.start
+            ops.mlstm_scan(y[at], x[at, :H * dk], x[at, H * dk:2 * H * dk], x[at, 2 * H * dk:], gates[at].float().cuda(), state, 0, i32(0, n), i32(0), n, 1,
+                           H, dk, dv, dk ** -0.5, max_q_len=n, workspace=ws)
+        got.append(y.cpu().double())
+    assert bool(torch.isfinite(got[0]).all()) and bool(torch.isfinite(got[1]).all())
+    # both are fp32 sums; rows whose n . q is a small difference carry a few 2^-24 of what it is a difference of
+    assert rel(got[1], got[0]) < 1e-4
+
+
+def test_state_space_that_forgets_at_once(ops):
+    """A decay of exp(-exp(a_log) dt) with exp(a_log) beyond the floats: every row forgets the ones before it."""
+    R, Q, N, P, rows = 2, 1, 16, 8, 130
+    xbc, dt = rnd(rows, R * P + 2 * Q * N, seed=3).bfloat16().cuda(), rnd(rows, R, seed=4).bfloat16().cuda()
+    one = torch.ones(R, device="cuda")
+    got = []
+    for ws in (None, torch.full((ops.ssm_workspace_floats(rows, 1, rows, R, N, P, torch.bfloat16),), float("nan"), device="cuda")):
+        y = torch.empty(rows, R * P, device="cuda")
+        state = torch.zeros((1, 4 * ops.ssm_state_floats(R, P, N)), dtype=torch.uint8, device="cuda")
+        ops.ssm_scan(y, xbc, dt, one, 100 * one, one, state, 0, i32(0, rows), i32(0), rows, 1, R, Q, N, P, max_q_len=rows, workspace=ws)
+        got.append(y.cpu().double())
+    assert bool(torch.isfinite(got[0]).all()) and rel(got[1], got[0]) < 2e-6
+
+
 def ssm_plain(C, B, x, f, dt, S):
     y = []
     for t in range(len(x)):
