@@ -178,7 +178,8 @@ __global__ __launch_bounds__(256) void gc_share_kernel(GcArgs<T> a, P p, int t0)
 
 // ---- the memory before every chunk ---------------------------------------------------------------------
 // A thread holds four neighbouring key dims of a column of a sequence's S and walks its chunks in the window
-// [t0, t0 + nt): the chunk's share is taken out, the memory before the chunk put in its place.
+// [t0, t0 + nt): the chunk's share is taken out, the memory before the chunk put in its place. Behind them S goes back to the state: the
+// next window's walk takes it from there.
 template <typename T, class P>
 __global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0, int nt, float* __restrict__ before_m) {
   const int seq = blockIdx.z, h = blockIdx.y;
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0,
 // keys of the chunk (a square of which the part behind the diagonal is left out) and with the memory before it, block
 // by block of 32 key dims; then the square, weighted, on the values.
 template <typename T, class P>
-__global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, GcArgs<T> a, P p, int t0, const float* __restrict__ before_m) {
+__global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, GcArgs<T> a, P p, int t0, int nt, const float* __restrict__ before_m) {
   // rows of q, rows of k, columns of the memory; later the square and the values
   __shared__ __attribute__((aligned(16))) float lds[2 * CK_ROWS * GC_LD];
   static_assert(3 * CK_ROWS * GC_KLD <= 2 * CK_ROWS * GC_LD, "the blocks fit where the square and the values will be");
@@ -278,7 +279,9 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
     ms[t] = m;
     olds[t] = expf((float)(F + m0 - (double)m));
   }
-  if (P::NORMED && blockIdx.x == 0 && (chunk + 1) * CK_ROWS >= a.cu[seq + 1] - a.cu[seq]) {
+  // the sequence's last chunk in the window: its m goes with the S and n that the walk over the chunks has kept, also where the sequence goes
+  // on in the next window, whose walk begins with all three
+  if (P::NORMED && blockIdx.x == 0 && ((int)blockIdx.z == nt - 1 || (chunk + 1) * CK_ROWS >= a.cu[seq + 1] - a.cu[seq])) {
     const float2 e = *reinterpret_cast<const float2*>(a.ends + 2 * item);
     p.keep_m(reinterpret_cast<float*>(a.state + (int64_t)a.slot[seq] * a.state_stride + a.state_offset), h, fmaxf(e.x + before_m[item], e.y), t);
   }
@@ -421,7 +424,7 @@ static int gc_run(float* y, GcArgs<T> a, const P& p, int rows, float* workspace,
     const int nt = chunks - t0 < window ? chunks - t0 : window;
     gc_share_kernel<T, P><<<dim3(kb * vb, a.H, nt), 256, 0, s>>>(a, p, t0);
     gc_carry_kernel<T, P><<<dim3((unsigned)((memory / a.H / 4 + 255) / 256), a.H, a.num_seqs), 256, 0, s>>>(a, p, t0, nt, before_m);
-    gc_rows_kernel<T, P><<<dim3(vb, a.H, nt), 256, 0, s>>>(y, a, p, t0, before_m);
+    gc_rows_kernel<T, P><<<dim3(vb, a.H, nt), 256, 0, s>>>(y, a, p, t0, nt, before_m);
   }
   return he_check_launch(name);
 }

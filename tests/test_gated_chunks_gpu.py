@@ -164,6 +164,90 @@ def test_state_space_by_chunks(ops, R, Q, N, P, decay):
         assert e["chunks"] <= max(2e-6, 1.5 * e["walk"])
 
 
+def chunks_of(lengths):
+    return sum(-(-n // 64) for n in lengths)
+
+
+def mlstm_plain_heads(q, k, v, i, f, state):
+    """All heads of a sequence on the device: q, k [T, H, dk], v [T, H, dv], i, f [T, H]; state (S, n, m) is carried on in place."""
+    S, n, m = state
+    y = torch.empty_like(v)
+    for t in range(len(q)):
+        new = torch.maximum(f[t] + m, i[t])
+        a, b = torch.exp(f[t] + m - new), torch.exp(i[t] - new)
+        kt = k[t] * b[:, None]
+        S.mul_(a[:, None, None]).baddbmm_(kt[:, :, None], v[t][:, None, :])
+        n.mul_(a[:, None]).add_(kt)
+        m.copy_(new)
+        y[t] = torch.bmm(q[t][:, None, :], S)[:, 0] / (torch.maximum((n * q[t]).sum(-1).abs(), torch.exp(-m)) + 1e-6)[:, None]
+    return y
+
+
+@pytest.mark.parametrize("H,dk,dv,lengths", [(64, 512, 256, [130, 500, 900, 70]), (4, 512, 1024, [2100])])
+def test_matrix_memory_over_several_windows(ops, H, dk, dv, lengths):
+    """More chunks than the workspace holds at once: sequences cut by the edge of a window once, twice and not at all, and a second step
+    that goes on from the states. Every row against the recurrence in 64 bits, beside the walk."""
+    B, room = len(lengths), 4 * ops.mlstm_state_floats(H, dk, dv)
+    slots = i32(*reversed(range(B)))
+    state = {way: torch.zeros((B, room), dtype=torch.uint8, device="cuda") for way in ("chunks", "walk")}
+    plain = [[torch.zeros(*shape, dtype=F64, device="cuda") for shape in ((H, dk, dv), (H, dk), (H,))] for _ in lengths]
+    for s, lens in enumerate((lengths, [70] * B)):
+        rows = sum(lens)
+        x = rnd(rows, H * (2 * dk + dv), seed=50 + s).bfloat16().cuda()
+        gates = torch.cat([rnd(rows, H, seed=60 + s, scale=2.0) - 1.0, -torch.nn.functional.softplus(-(rnd(rows, H, seed=70 + s, scale=2.0) + 3.0))], 1).float().cuda()
+        q, k, v = x[:, :H * dk], x[:, H * dk:2 * H * dk], x[:, 2 * H * dk:]
+        floats = ops.mlstm_workspace_floats(rows, B, max(lens), H, dk, dv, torch.bfloat16)
+        assert s or floats // (H * ((dv + 1) * dk + 4)) < chunks_of(lens)
+        got = {}
+        for way in state:
+            got[way] = torch.full((rows, H * dv), float("nan"), device="cuda")
+            ws = torch.full((floats,), float("nan"), device="cuda") if way == "chunks" else None
+            ops.mlstm_scan(got[way], q, k, v, gates, state[way], 0, cu_of(lens), slots, rows, B, H, dk, dv, dk ** -0.5, max_q_len=max(lens), workspace=ws)
+        x64, g64, r = x.double(), gates.double(), 0
+        for b, n in enumerate(lens):
+            at = slice(r, r + n)
+            want = mlstm_plain_heads(x64[at, :H * dk].reshape(n, H, dk) * dk ** -0.5, x64[at, H * dk:2 * H * dk].reshape(n, H, dk),
+                                     x64[at, 2 * H * dk:].reshape(n, H, dv), g64[at, :H], g64[at, H:], plain[b]).reshape(n, H * dv)
+            e = {way: rel(got[way][at], want) for way in got}
+            # 32-bit sums and exponentials: a few 2^-24
+            assert e["chunks"] <= max(2e-6, 1.5 * e["walk"]), (s, b)
+            r += n
+
+
+@pytest.mark.parametrize("R,Q,N,P,lengths", [(64, 8, 256, 256, [130, 1100, 2300, 70])])
+def test_state_space_over_several_windows(ops, R, Q, N, P, lengths):
+    """The same for the state space, whose chunks hand on S alone."""
+    B, C = len(lengths), R * P + 2 * Q * N
+    slots, room = i32(*reversed(range(B))), 4 * ops.ssm_state_floats(R, P, N)
+    state = {way: torch.zeros((B, room), dtype=torch.uint8, device="cuda") for way in ("chunks", "walk")}
+    a_log, bias, skip = (rnd(R, seed=i).float().cuda() for i in (1, 2, 3))
+    plain = [torch.zeros(R, N, P, dtype=F64, device="cuda") for _ in lengths]
+    for s, lens in enumerate((lengths, [70] * B)):
+        rows = sum(lens)
+        xbc, dt_in = rnd(rows, C, seed=80 + s).bfloat16().cuda(), rnd(rows, R, seed=90 + s).bfloat16().cuda()
+        floats = ops.ssm_workspace_floats(rows, B, max(lens), R, N, P, torch.bfloat16)
+        assert s or floats // (R * (P * N + 4)) < chunks_of(lens)
+        got = {}
+        for way in state:
+            got[way] = torch.full((rows, R * P), float("nan"), device="cuda")
+            ws = torch.full((floats,), float("nan"), device="cuda") if way == "chunks" else None
+            ops.ssm_scan(got[way], xbc, dt_in, bias, a_log, skip, state[way], 0, cu_of(lens), slots, rows, B, R, Q, N, P, max_q_len=max(lens), workspace=ws)
+        dt = torch.nn.functional.softplus(dt_in.double() + bias.double())
+        keep, x64, r = torch.exp(-torch.exp(a_log.double()) * dt), xbc.double(), 0
+        for b, n in enumerate(lens):
+            at = slice(r, r + n)
+            x = x64[at, :R * P].reshape(n, R, P)
+            Bs, Cs = (x64[at, R * P + i * Q * N:R * P + (i + 1) * Q * N].reshape(n, Q, N).repeat_interleave(R // Q, 1) for i in (0, 1))
+            S, want = plain[b], torch.empty_like(x)
+            for t in range(n):
+                S.mul_(keep[r + t][:, None, None]).baddbmm_((Bs[t] * dt[r + t][:, None])[:, :, None], x[t][:, None, :])
+                want[t] = torch.bmm(Cs[t][:, None, :], S)[:, 0]
+            want += skip.double()[:, None] * x
+            e = {way: rel(got[way][at], want.reshape(n, R * P)) for way in got}
+            assert e["chunks"] <= max(2e-6, 1.5 * e["walk"]), (s, b)
+            r += n
+
+
 def test_what_goes_by_chunks(ops):
     """Short or unknown lengths and 32-bit activations are walked, and so are heads that are no whole fours, whatever workspace is given."""
     bf16 = torch.bfloat16
