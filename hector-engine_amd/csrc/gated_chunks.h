@@ -50,7 +50,7 @@ struct GcArgs {
   uint8_t* state;
   int64_t state_stride, state_offset;
   float* ws;               // [chunk of the window][H][cols][dkp]: first the chunks' shares, then the memories before them
-  float* ends;             // [chunk of the window][H][2]: F_n and G of a chunk; then the m before it
+  double* ends;            // [chunk of the window][H][2]: F_n and G of a chunk
 };
 template <typename T, class P>
 __host__ __device__ constexpr int gc_cols(int dv) { return dv + (P::NORMED ? 1 : 0); }
@@ -69,11 +69,37 @@ __device__ __forceinline__ float4 gc_tile4(const T* first, int64_t stride, int r
   return row < n && d < width ? v : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Sums of many products are formed sixteen at a time and then added: a chain of all of them would lose more in rounding than the
-// walk's sums, which are spread over the lanes of a value dim.
-__device__ __forceinline__ void gc_add(gc_acc& a, const gc_acc& b) {
+// exp(x) of an x <= 0 that is a difference of sums in 64 bits: what x loses as a 32-bit number would show in the power times |x|
+__device__ __forceinline__ float gc_exp(double x) {
+  const float hi = (float)x;
+  if (hi < -104.f) return 0.f;      // (below half of the smallest number; -inf among them)
+  const float e = expf(hi);
+  return fmaf(e, (float)(x - (double)hi), e);
+}
+
+// Sums of many products are formed sixteen at a time, as two chains of eight, and then added: a chain of all of them would lose more in
+// rounding than the walk's sums, which are spread over the lanes of a value dim. KEEP: what an addition loses is carried along to the next (NORMED,
+// whose results are quotients of two such sums: keys of 512 dims and one sign were 1.15 times as far from 64 bits as the walk without it, and are 0.91 so;
+// 2,048 rows of 14 heads of 128 x 256 take 141 us for it, 130 before).
+template <bool KEEP>
+__device__ __forceinline__ void gc_add(gc_acc& a, gc_acc& lost, const gc_acc& b, const gc_acc& c) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) a[r] += b[r];
+  for (int r = 0; r < 16; ++r) {
+    if (KEEP) {
+      const float more = b[r] + c[r] - lost[r], sum = a[r] + more;
+      lost[r] = (sum - a[r]) - more;
+      a[r] = sum;
+    } else {
+      a[r] += b[r] + c[r];
+    }
+  }
+}
+__device__ __forceinline__ gc_acc gc_mfma4(const float4& a, const float4& b) {
+  gc_acc s = {0.f};
+  s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, s, 0, 0, 0);
+  s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, s, 0, 0, 0);
+  s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, s, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, s, 0, 0, 0);
 }
 
 // F of the lane's row (lane < 64: the rows of the chunk, summed up to and with it) and in; rows beyond the chunk keep everything and
@@ -102,6 +128,9 @@ __device__ __forceinline__ void gc_gates(const P& p, int64_t r0, int n, int h, i
     }
   }
 }
+
+// The m behind a chunk of those ends.
+__device__ __forceinline__ float gc_next_m(const double2& e, float m) { return (float)fmax(e.x + (double)m, e.y); }
 
 // ---- every chunk's own share of the memory behind it -----------------------------------------------------
 // One workgroup of four wavefronts a (64 key dims x 64 columns, head, chunk), a wavefront 32 x 32 of it, two rows of the
@@ -132,10 +161,11 @@ __global__ __launch_bounds__(256) void gc_share_kernel(GcArgs<T> a, P p, int t0)
     double F, peak;
     float in;
     gc_gates(p, r0, n, h, t, F, in, peak);
-    const double Fn = __shfl(F, 63), G = P::NORMED ? Fn + __shfl(peak, 63) : 0.;
+    // (G as a 32-bit number: where it becomes the m behind the chunk, the share is taken as it is)
+    const double Fn = __shfl(F, 63), G = P::NORMED ? (float)(Fn + __shfl(peak, 63)) : 0.;
     // (in = -inf writes nothing, also where all of a chunk's rows have it and G is -inf)
-    weight[t] = !P::NORMED ? in * expf((float)(Fn - F)) : in == -INFINITY ? 0.f : expf((float)(Fn - F + (double)in - G));
-    if (t == 0 && blockIdx.x == 0) *reinterpret_cast<float2*>(a.ends + 2 * ((int64_t)blockIdx.z * a.H + h)) = make_float2((float)Fn, (float)G);
+    weight[t] = !P::NORMED ? in * gc_exp(Fn - F) : in == -INFINITY ? 0.f : gc_exp(Fn - F + (double)in - G);
+    if (t == 0 && blockIdx.x == 0) *reinterpret_cast<double2*>(a.ends + 2 * ((int64_t)blockIdx.z * a.H + h)) = make_double2(Fn, G);
   }
   __syncthreads();
 #pragma unroll
@@ -152,13 +182,13 @@ __global__ __launch_bounds__(256) void gc_share_kernel(GcArgs<T> a, P p, int t0)
   const int i0 = (wave >> 1) * 32, j0 = (wave & 1) * 32;       // columns of S, key dims
   gc_acc acc = {0.f};
   for (int g0 = 0; g0 < n; g0 += 16) {
-    gc_acc some = {0.f};
+    gc_acc some[2] = {{0.f}, {0.f}};
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
       const int row = g0 + 8 * hl + m;
-      some = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[row * GC_LD + i0 + l32], ks[row * GC_LD + j0 + l32], some, 0, 0, 0);
+      some[m & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[row * GC_LD + i0 + l32], ks[row * GC_LD + j0 + l32], some[m & 1], 0, 0, 0);
     }
-    gc_add(acc, some);
+    gc_add<false>(acc, acc, some[0], some[1]);
   }
   const int od = d0 + j0 + l32;
 #pragma unroll
@@ -204,13 +234,13 @@ __global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0,
   float* place = p.place(st, h, c, d);
   const int64_t base = (int64_t)(before + first - t0) * a.H + h;
   float* w = a.ws + base * memory + (own ? at : 0);
-  const float2* ends = reinterpret_cast<const float2*>(a.ends) + base;
+  const double2* ends = reinterpret_cast<const double2*>(a.ends) + base;
   float m = p.m(st, h);
   float4 S = *reinterpret_cast<const float4*>(place);
   constexpr int AHEAD = 8;
   for (int i = first; i < end; i += AHEAD) {
     float4 mine[AHEAD];
-    float2 e[AHEAD];
+    double2 e[AHEAD];
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
       const int k = min(u, end - 1 - i);
@@ -222,8 +252,8 @@ __global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0,
       if (i + u < end) {
         if (own) *reinterpret_cast<float4*>(w + u * step) = S;
         if (P::NORMED && id == 0) before_m[base + (int64_t)(i + u - first) * a.H] = m;
-        const float next = P::NORMED ? fmaxf(e[u].x + m, e[u].y) : 0.f;
-        const float keep = expf(e[u].x + m - next), take = P::NORMED ? expf(e[u].y - next) : 1.f;
+        const float next = P::NORMED ? gc_next_m(e[u], m) : 0.f;
+        const float keep = gc_exp(e[u].x + (double)m - (double)next), take = P::NORMED ? gc_exp(e[u].y - (double)next) : 1.f;
         S.x = fmaf(keep, S.x, take * mine[u].x);
         S.y = fmaf(keep, S.y, take * mine[u].y);
         S.z = fmaf(keep, S.z, take * mine[u].z);
@@ -242,7 +272,7 @@ __global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0,
 // keys of the chunk (a square of which the part behind the diagonal is left out) and with the memory before it, block
 // by block of 32 key dims; then the square, weighted, on the values.
 template <typename T, class P>
-__global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, GcArgs<T> a, P p, int t0, int nt, const float* __restrict__ before_m) {
+__global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* __restrict__ y, GcArgs<T> a, P p, int t0, int nt, const float* __restrict__ before_m) {
   // rows of q, rows of k, columns of the memory; later the square and the values
   __shared__ __attribute__((aligned(16))) float lds[2 * CK_ROWS * GC_LD];
   static_assert(3 * CK_ROWS * GC_KLD <= 2 * CK_ROWS * GC_LD, "the blocks fit where the square and the values will be");
@@ -277,16 +307,16 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
     Fs[t] = F;
     ins[t] = in;
     ms[t] = m;
-    olds[t] = expf((float)(F + m0 - (double)m));
+    olds[t] = gc_exp(F + m0 - (double)m);
   }
   // the sequence's last chunk in the window: its m goes with the S and n that the walk over the chunks has kept, also where the sequence goes
   // on in the next window, whose walk begins with all three
   if (P::NORMED && blockIdx.x == 0 && ((int)blockIdx.z == nt - 1 || (chunk + 1) * CK_ROWS >= a.cu[seq + 1] - a.cu[seq])) {
-    const float2 e = *reinterpret_cast<const float2*>(a.ends + 2 * item);
-    p.keep_m(reinterpret_cast<float*>(a.state + (int64_t)a.slot[seq] * a.state_stride + a.state_offset), h, fmaxf(e.x + before_m[item], e.y), t);
+    const double2 e = *reinterpret_cast<const double2*>(a.ends + 2 * item);
+    p.keep_m(reinterpret_cast<float*>(a.state + (int64_t)a.slot[seq] * a.state_stride + a.state_offset), h, gc_next_m(e, before_m[item]), t);
   }
-  gc_acc square = {0.f}, out = {0.f};
-  float den = 0.f;                            // NORMED: n . q of row t / 4, this thread's share
+  gc_acc square = {0.f}, out = {0.f}, lost_s = {0.f}, lost_o = {0.f};
+  float den = 0.f, lost_d = 0.f;              // NORMED: n . q of row t / 4, this thread's share
   for (int d0 = 0; d0 < a.dkp; d0 += GC_KB) {
     const int d = 4 * (t & 7);
     float4 qx[2], kx[2], sx[2], nx = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -308,27 +338,19 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
     }
     if (P::NORMED && t < 8) *reinterpret_cast<float4*>(ns + d) = nx;
     __syncthreads();
-#pragma unroll
+#pragma unroll 1
     for (int g0 = 0; g0 < GC_KB; g0 += 16) {
-      gc_acc some = {0.f}, dots = {0.f};
+      float4 qv[2], kv[2], sv[2];
 #pragma unroll
-      for (int g = g0; g < g0 + 16; g += 8) {
-        const float4 qv = *reinterpret_cast<const float4*>(qs + (i0 + l32) * GC_KLD + g + 4 * hl);
-        const float4 kv = *reinterpret_cast<const float4*>(ks + (j0 + l32) * GC_KLD + g + 4 * hl);
-        const float4 sv = *reinterpret_cast<const float4*>(ss + (j0 + l32) * GC_KLD + g + 4 * hl);
-        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.x, sv.x, some, 0, 0, 0);
-        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.y, sv.y, some, 0, 0, 0);
-        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.z, sv.z, some, 0, 0, 0);
-        some = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.w, sv.w, some, 0, 0, 0);
-        if (j0 <= i0) {                       // (the same in the wavefront)
-          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.x, kv.x, dots, 0, 0, 0);
-          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.y, kv.y, dots, 0, 0, 0);
-          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.z, kv.z, dots, 0, 0, 0);
-          dots = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.w, kv.w, dots, 0, 0, 0);
-        }
+      for (int u = 0; u < 2; ++u) {
+        const int g = g0 + 8 * u + 4 * hl;
+        qv[u] = *reinterpret_cast<const float4*>(qs + (i0 + l32) * GC_KLD + g);
+        kv[u] = *reinterpret_cast<const float4*>(ks + (j0 + l32) * GC_KLD + g);
+        sv[u] = *reinterpret_cast<const float4*>(ss + (j0 + l32) * GC_KLD + g);
       }
-      gc_add(out, some);
-      gc_add(square, dots);
+      gc_add<P::NORMED>(out, lost_o, gc_mfma4(qv[0], sv[0]), gc_mfma4(qv[1], sv[1]));
+      __builtin_amdgcn_sched_barrier(0);
+      if (j0 <= i0) gc_add<P::NORMED>(square, lost_s, gc_mfma4(qv[0], kv[0]), gc_mfma4(qv[1], kv[1]));      // (the same in the wavefront)
     }
     if (P::NORMED) {
       float some = 0.f;
@@ -338,7 +360,9 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
         const float4 nv = *reinterpret_cast<const float4*>(ns + 8 * (t & 3) + e);
         some = fmaf(qv.x, nv.x, fmaf(qv.y, nv.y, fmaf(qv.z, nv.z, fmaf(qv.w, nv.w, some))));
       }
-      den += some;
+      const float more = some - lost_d, sum = den + more;
+      lost_d = (sum - den) - more;
+      den = sum;
     }
   }
   float4 vx[4];
@@ -354,8 +378,7 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int i = i0 + 8 * (r >> 2) + 4 * hl + (r & 3);
-      out[r] *= olds[i];
-      const float e = P::NORMED ? expf((float)(Fs[i] - Fj + (double)inj - (double)ms[i])) : inj * expf((float)(Fs[i] - Fj));
+      const float e = P::NORMED ? gc_exp(Fs[i] - Fj + (double)inj - (double)ms[i]) : inj * gc_exp(Fs[i] - Fj);
       square_s[i * GC_LD + j] = j <= i && j < n ? e * square[r] : 0.f;
     }
   }
@@ -373,19 +396,18 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
     if ((t & 3) == 0) dens[t >> 2] = fmaxf(fabsf(den), expf(-ms[t >> 2])) + 1e-6f;
   }
 #pragma unroll
+  for (int r = 0; r < 16; ++r) square[r] = lost_s[r] = 0.f;      // (from here on the square's share of the result)
+#pragma unroll
   for (int g0 = 0; g0 < CK_ROWS; g0 += 16) {
     if (g0 >= i0 + 32 || g0 >= n) break;      // (the same in the wavefront)
-    gc_acc some = {0.f};
+    gc_acc some[2];
 #pragma unroll
-    for (int g = g0; g < g0 + 16; g += 8) {
-      const float4 s = *reinterpret_cast<const float4*>(square_s + (i0 + l32) * GC_LD + g + 4 * hl);
-      const float* v = vs + (g + 4 * hl) * GC_LD + j0 + l32;
-      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.x, v[0], some, 0, 0, 0);
-      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.y, v[GC_LD], some, 0, 0, 0);
-      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.z, v[2 * GC_LD], some, 0, 0, 0);
-      some = __builtin_amdgcn_mfma_f32_32x32x2f32(s.w, v[3 * GC_LD], some, 0, 0, 0);
+    for (int u = 0; u < 2; ++u) {
+      const int g = g0 + 8 * u + 4 * hl;
+      const float* v = vs + g * GC_LD + j0 + l32;
+      some[u] = gc_mfma4(*reinterpret_cast<const float4*>(square_s + (i0 + l32) * GC_LD + g), make_float4(v[0], v[GC_LD], v[2 * GC_LD], v[3 * GC_LD]));
     }
-    gc_add(out, some);
+    gc_add<P::NORMED>(square, lost_s, some[0], some[1]);
   }
   if (P::NORMED) __syncthreads();
   const int c = c0 + j0 + l32;
@@ -393,7 +415,8 @@ __global__ __launch_bounds__(256, 4) void gc_rows_kernel(float* __restrict__ y, 
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int i = i0 + 8 * (r >> 2) + 4 * hl + (r & 3);
-      if (i < n) y[(r0 + i) * a.H * a.dv + (int64_t)h * a.dv + c] = P::NORMED ? out[r] / dens[i] : p.result(out[r], vs[i * GC_LD + j0 + l32], h);
+      const float sum = fmaf(out[r], olds[i], square[r]);
+      if (i < n) y[(r0 + i) * a.H * a.dv + (int64_t)h * a.dv + c] = P::NORMED ? sum / dens[i] : p.result(sum, vs[i * GC_LD + j0 + l32], h);
     }
   }
 }
@@ -408,7 +431,7 @@ static inline int64_t gc_window(int rows, int num_seqs, int64_t memory) {
 static inline int64_t gc_floats(int rows, int num_seqs, int max_q_len, int H, int cols, int dkp) {
   if (rows <= 0 || num_seqs <= 0 || max_q_len <= GC_FROM) return 0;
   const int64_t memory = (int64_t)H * cols * dkp;
-  return gc_window(rows, num_seqs, memory) * (memory + 4ll * H);
+  return gc_window(rows, num_seqs, memory) * (memory + 6ll * H);
 }
 
 template <typename T, class P>
@@ -417,8 +440,8 @@ static int gc_run(float* y, GcArgs<T> a, const P& p, int rows, float* workspace,
   const int64_t memory = (int64_t)a.H * cols * a.dkp;
   const int window = (int)gc_window(rows, a.num_seqs, memory), chunks = rows / CK_ROWS + a.num_seqs;
   a.ws = workspace;
-  a.ends = a.ws + window * memory;
-  float* before_m = a.ends + 2ll * window * a.H;
+  a.ends = reinterpret_cast<double*>(a.ws + window * memory);      // (a memory is whole fours)
+  float* before_m = reinterpret_cast<float*>(a.ends + 2ll * window * a.H);
   const int kb = (a.dkp + 63) / 64, vb = (a.dv + 63) / 64;
   for (int t0 = 0; t0 < chunks; t0 += window) {
     const int nt = chunks - t0 < window ? chunks - t0 : window;
