@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void dm_share_kernel(DmArgs<T> a, int t0) {
   __shared__ __attribute__((aligned(16))) float ks[DM_C * DM_LD], vs[DM_C * DM_LD];
   const int h = blockIdx.y;
   int seq, chunk;
-  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, 0, seq, chunk)) return;
   if (a.slot[seq] < 0) return;
   const int vb = (a.dvp + DM_B - 1) / DM_B;
   const int d0 = ((int)blockIdx.x / vb) * DM_B, c0 = ((int)blockIdx.x % vb) * DM_B;
@@ -209,12 +209,12 @@ __global__ __launch_bounds__(256) void dm_carry_kernel(DmArgs<T> a, int t0, int 
   int before = 0;
   for (int s0 = 0; s0 < seq; s0 += 64) {
     const int s = s0 + (int)(threadIdx.x & 63);
-    int n = s < seq ? ck_chunks(a.cu, s) : 0;
+    int n = s < seq ? ck_chunks(a.cu, s, 0) : 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
     before += n;
   }
-  const int chunks = ck_chunks(a.cu, seq);
+  const int chunks = ck_chunks(a.cu, seq, 0);
   const int first = max(0, t0 - before), end = min(chunks, t0 + nt - before);
   if (first >= end) return;
   const int64_t memory = (int64_t)a.dk * a.dvp;
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256, 4) void dm_rows_kernel(float* __restrict__ y, 
     return;
   }
   int seq, chunk;
-  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, 0, seq, chunk)) return;
   if (a.slot[seq] < 0) return;
   const int64_t r0 = a.cu[seq] + (int64_t)chunk * DM_C;
   const int n = min(DM_C, (int)(a.cu[seq + 1] - r0));

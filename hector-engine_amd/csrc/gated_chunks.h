@@ -22,16 +22,29 @@
 // four neighbouring key dims from d on of column c (dv: n) of S lie in a sequence's state; keep(...) puts them back (n into every copy of it);
 // m(st, h) and keep_m(...): NORMED's m and its copies; result(y, x, h): what follows the products.
 #pragma once
+#include <algorithm>
+#include <climits>
+
 #include "chunks.h"
 
 #define GC_LD 68      // floats between rows of 64 in LDS (four banks on from row to row)
 #define GC_KB 32      // key dims of a block of the rows kernel
 #define GC_KLD 36
 #define GC_WINDOW_FLOATS (64 << 20)   // memories held between the launches at once (256 MiB)
-// Steps whose longest sequence has more rows than this go by chunks. One sequence, walked and by chunks: matrix memory of 14 heads 48
-// rows 29 and 27 us, 64 rows 35 and 27, 128 rows 65 and 29; state space of 64 heads 48 rows 22 and 27, 64 rows 27 and 28, 128 rows 48 and 30;
-// four sequences of 32 rows of 128 heads 54 and 55.
+// No step goes by chunks whose longest sequence has no more rows than this; from there on gc_pays says.
 #define GC_FROM 64
+// Of several sequences in such a step, those of up to GC_SHORT rows are walked, in launches of their own: a chunk costs what a whole one does (one of
+// 14 heads of 128 x 256 3.7 us in a step of many; a walk of one row 0.8, of 2 to 8 3.0 to 3.9, of 40 12; of 64 heads of 128 x 64 4.0 and 1.2, 1.4
+// to 2.5, 6.7) and moves the memory three times. Up to GC_FEW rows a walk stages nothing, or little.
+#define GC_SHORT 16
+#define GC_FEW 4
+static inline int gc_from(int num_seqs) { return num_seqs > 1 ? GC_SHORT : 0; }
+
+// Where chunks pay: the rows of one sequence alone, of the longest beside shorter ones, and the rows the others have on average where they pay
+// from GC_FROM on.
+struct GcLines {
+  int alone, beside, others;
+};
 
 #define GC_FORGETS -1e7f
 typedef float gc_acc __attribute__((ext_vector_type(16)));
@@ -47,6 +60,7 @@ struct GcArgs {
   const int32_t* cu;
   const int32_t* slot;
   int num_seqs, H, dk, dv, dkp;      // dkp: key dims with the state's padding, a multiple of 4
+  int from;                // sequences of up to so many rows are the walk's (gc_from)
   uint8_t* state;
   int64_t state_stride, state_offset;
   float* ws;               // [chunk of the window][H][cols][dkp]: first the chunks' shares, then the memories before them
@@ -142,7 +156,7 @@ __global__ __launch_bounds__(256) void gc_share_kernel(GcArgs<T> a, P p, int t0)
   __shared__ float weight[CK_ROWS], part[4][64];
   const int h = blockIdx.y;
   int seq, chunk;
-  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, a.from, seq, chunk)) return;
   if (a.slot[seq] < 0) return;
   const int vb = (a.dv + 63) / 64;
   const int d0 = ((int)blockIdx.x / vb) * 64, c0 = ((int)blockIdx.x % vb) * 64;
@@ -214,16 +228,16 @@ template <typename T, class P>
 __global__ __launch_bounds__(256) void gc_carry_kernel(GcArgs<T> a, P p, int t0, int nt, float* __restrict__ before_m) {
   const int seq = blockIdx.z, h = blockIdx.y;
   const int slot = a.slot[seq];
-  if (slot < 0 || a.cu[seq + 1] <= a.cu[seq]) return;
+  if (slot < 0 || a.cu[seq + 1] - a.cu[seq] <= a.from) return;
   int before = 0;
   for (int s0 = 0; s0 < seq; s0 += 64) {
     const int s = s0 + (int)(threadIdx.x & 63);
-    int n = s < seq ? ck_chunks(a.cu, s) : 0;
+    int n = s < seq ? ck_chunks(a.cu, s, a.from) : 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
     before += n;
   }
-  const int first = max(0, t0 - before), end = min(ck_chunks(a.cu, seq), t0 + nt - before);
+  const int first = max(0, t0 - before), end = min(ck_chunks(a.cu, seq, a.from), t0 + nt - before);
   if (first >= end) return;
   const int cols = gc_cols<T, P>(a.dv);
   const int64_t memory = (int64_t)cols * a.dkp, step = (int64_t)a.H * memory;
@@ -287,7 +301,7 @@ __global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* 
   const int h = blockIdx.y, c0 = (int)blockIdx.x * 64;
   const int t = threadIdx.x, wave = t >> 6, l32 = t & 31, hl = (t >> 5) & 1;
   int seq, chunk;
-  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, seq, chunk)) return;
+  if (!ck_find(t0 + (int)blockIdx.z, a.cu, a.num_seqs, a.from, seq, chunk)) return;
   if (a.slot[seq] < 0) return;
   const int64_t r0 = a.cu[seq] + (int64_t)chunk * CK_ROWS;
   const int n = min(CK_ROWS, (int)(a.cu[seq + 1] - r0));
@@ -421,24 +435,42 @@ __global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* 
   }
 }
 
+// Whether a step is faster by chunks. The walk of the longest sequence hides those of the others; behind the chunks these stand alone, and
+// sequences of GC_FEW to GC_SHORT rows cost there what memory / 65536 rows of the longest one's walk do. (us walked and by chunks, 14 heads of 128 x 256; 64 heads
+// of 128 x 64: 70 rows 42 and 34; 29 and 34. 140 rows 73 and 36; 51 and 36. 70 rows beside 7 of one row 46 and 45; 30 and 50. Beside 63 201 and 93; 140 and 144.
+// 200 beside 31 of one row 145 and 69; 93 and 92. 70 beside 15 of 40 195 and 106; 109 and 105. 70 beside 31 of 8 143 and 161; 91 and 122.)
+static inline bool gc_pays(int rows, int num_seqs, int max_q_len, int64_t memory, const GcLines& lines) {
+  const int longest = std::min(rows, max_q_len);
+  if (num_seqs == 1) return longest > lines.alone;
+  const int others = (rows - longest) / (num_seqs - 1);
+  if (others >= lines.others) return longest > GC_FROM;
+  return longest > lines.beside + (others > GC_FEW ? (num_seqs - 1) * memory / 65536 : 0);
+}
+
+// No fewer than the chunks of a step's sequences: whole ones, and one more of every sequence that has chunks.
+static inline int64_t gc_chunks(int rows, int num_seqs) {
+  return rows / CK_ROWS + std::min(num_seqs, rows / (gc_from(num_seqs) + 1));
+}
+
 // Chunks whose memories are held at once, and the floats of workspace for them: memories, ends and the m before them.
 static inline int64_t gc_window(int rows, int num_seqs, int64_t memory) {
-  const int64_t chunks = (int64_t)rows / CK_ROWS + num_seqs;      // no fewer than the sequences' chunks
+  const int64_t chunks = gc_chunks(rows, num_seqs);
   int64_t most = GC_WINDOW_FLOATS / memory;
   if (most > 32768) most = 32768;
   return chunks < most ? chunks : (most < 1 ? 1 : most);
 }
-static inline int64_t gc_floats(int rows, int num_seqs, int max_q_len, int H, int cols, int dkp) {
-  if (rows <= 0 || num_seqs <= 0 || max_q_len <= GC_FROM) return 0;
+static inline int64_t gc_floats(int rows, int num_seqs, int max_q_len, int H, int cols, int dkp, const GcLines& lines) {
   const int64_t memory = (int64_t)H * cols * dkp;
+  if (num_seqs <= 0 || !gc_pays(rows, num_seqs, max_q_len, memory, lines)) return 0;
   return gc_window(rows, num_seqs, memory) * (memory + 6ll * H);
 }
 
 template <typename T, class P>
-static int gc_run(float* y, GcArgs<T> a, const P& p, int rows, float* workspace, const char* name, hipStream_t s) {
+static int gc_run(float* y, const GcArgs<T>& args, const P& p, int rows, float* workspace, const char* name, hipStream_t s) {
+  GcArgs<T> a = args;
   const int cols = gc_cols<T, P>(a.dv);
   const int64_t memory = (int64_t)a.H * cols * a.dkp;
-  const int window = (int)gc_window(rows, a.num_seqs, memory), chunks = rows / CK_ROWS + a.num_seqs;
+  const int window = (int)gc_window(rows, a.num_seqs, memory), chunks = (int)gc_chunks(rows, a.num_seqs);
   a.ws = workspace;
   a.ends = reinterpret_cast<double*>(a.ws + window * memory);      // (a memory is whole fours)
   float* before_m = reinterpret_cast<float*>(a.ends + 2ll * window * a.H);

@@ -242,7 +242,8 @@ int he_conv_state(void* out, const void* x, int64_t x_stride, const void* taps, 
 int64_t he_ssm_state_floats(int R, int P, int N);
 // xbc [rows][R P + 2 Q N]: x, then the Q groups' B vectors, then their C vectors; dt_in[row * dt_stride + r].
 // y [rows][R P] fp32 (rows without a sequence are not written). max_q_len: a bound on the rows a sequence brings (0: none).
-// workspace of he_ssm_workspace_floats() floats: sequences of many rows go by chunks (bf16 activations); null: row by row.
+// workspace of he_ssm_workspace_floats() floats, where these are more than none: by chunks, all but the step's short sequences (bf16
+// activations); null: row by row.
 int64_t he_ssm_workspace_floats(int rows, int num_seqs, int max_q_len, int R, int N, int P, int dtype);
 int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int64_t dt_stride, const void* dt_bias,
                 const void* a_log, const void* d_skip, int w_dtype, void* state, int64_t state_stride,
@@ -261,7 +262,8 @@ int he_gated_group_norm(void* out, const void* y_f32, const void* z, int64_t z_s
 // apart) and the gates' logarithms (raw_gates: their pre-activations, with gate_bias and cap as he_mlstm_gates takes
 // them, and the logarithms are formed inside); S, n and m of a sequence live at state_offset of its row of `state`,
 // he_mlstm_state_floats(H, dk, dv) floats, zeros at a sequence's start. dk up to 512. max_q_len: a bound on the rows a
-// sequence brings (0: none); workspace of he_mlstm_workspace_floats() floats: sequences of many rows go by chunks (bf16 activations); null: row by row.
+// sequence brings (0: none); workspace of he_mlstm_workspace_floats() floats, where these are more than none: by chunks, all but the step's short
+// sequences (bf16 activations); null: row by row.
 int64_t he_mlstm_workspace_floats(int rows, int num_seqs, int max_q_len, int H, int dk, int dv, int dtype);
 int64_t he_mlstm_state_floats(int H, int dk, int dv);
 int he_mlstm_gates(void* out_f32, const void* x_f32, const void* bias, int bias_dtype, int rows, int H, float cap,

@@ -5,8 +5,9 @@
 //   y_t = S_t^T q_t / (max(|n_t . q_t|, exp(-m_t)) + 1e-6)
 // with i_t and f_t the logarithms of the input and forget gates. S, n and m start at zero and live in
 // 32-bit floats in the sequence's row of the cache's state area; everything here is fp32 arithmetic, only
-// q, k and v are read in the activation dtype. Sequences of up to GC_FROM rows are walked row by row, longer ones of
-// bf16 activations go by chunks (gated_chunks.h); with 32-bit activations results do not depend on how the rows were cut into steps.
+// q, k and v are read in the activation dtype. Steps of long sequences of bf16 activations go by chunks, all but their short
+// sequences (gated_chunks.h: gc_pays, gc_from), others are walked row by row; with 32-bit activations results do not depend on
+// how the rows were cut into steps.
 #include "gated_chunks.h"
 #include "hector_kernels.h"
 
@@ -125,13 +126,13 @@ __global__ void __launch_bounds__(256) mlstm_scan_kernel(float* __restrict__ y, 
                                   uint8_t* __restrict__ state, int64_t state_stride, int64_t state_offset,
                                   const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_slot, int H,
                                   int dk, int dv, int NG, int PB, int TB, float q_scale, int raw_gates,
-                                  const void* __restrict__ gate_bias, int bias_dtype, float cap) {
+                                  const void* __restrict__ gate_bias, int bias_dtype, float cap, int least, int most) {
   extern __shared__ float mm_lds[];
   constexpr int VE = 16 / sizeof(T);            // elements of a 16-byte piece
   const int seq = blockIdx.z, h = blockIdx.y;
   const int slot = seq_slot[seq];
   const int r0 = cu_seqlens[seq], r1 = cu_seqlens[seq + 1];
-  if (slot < 0 || r0 >= r1) return;
+  if (slot < 0 || r1 - r0 < least || r1 - r0 > most) return;       // (sequences of least to most rows; least is 1 or more)
   const int t = threadIdx.x, threads = blockDim.x;
   const int c = t / NG, j = t % NG;
   const int col0 = blockIdx.x * PB;
@@ -380,11 +381,12 @@ __global__ void __launch_bounds__(256) mlstm_step_kernel(float* __restrict__ y, 
                                                          const int32_t* __restrict__ cu_seqlens,
                                                          const int32_t* __restrict__ seq_slot, int H, int dk, int dv, int NG,
                                                          int PB, float q_scale, int vec, int raw_gates,
-                                                         const void* __restrict__ gate_bias, int bias_dtype, float cap) {
+                                                         const void* __restrict__ gate_bias, int bias_dtype, float cap, int least,
+                                                         int most) {
   const int seq = blockIdx.z, h = blockIdx.y;
   const int slot = seq_slot[seq];
   const int r0 = cu_seqlens[seq], r1 = cu_seqlens[seq + 1];
-  if (slot < 0 || r0 >= r1) return;
+  if (slot < 0 || r1 - r0 < least || r1 - r0 > most) return;       // (sequences of least to most rows; least is 1 or more)
   const int c = threadIdx.x / NG, j = threadIdx.x % NG;
   const int col = blockIdx.x * PB + c;
   const bool active = c < PB && col < dv;
@@ -488,7 +490,7 @@ struct MmChunks {
 // Floats of workspace he_mlstm_scan wants to go by chunks (0: it walks the rows). max_q_len: the most rows of a sequence, 0: not known.
 extern "C" int64_t he_mlstm_workspace_floats(int rows, int num_seqs, int max_q_len, int H, int dk, int dv, int dtype) {
   if (H <= 0 || dk <= 0 || dv <= 0 || dtype != HE_BF16) return 0;
-  return gc_floats(rows, num_seqs, max_q_len, H, dv + 1, mm_groups(dk) * MM_NPT);
+  return gc_floats(rows, num_seqs, max_q_len, H, dv + 1, mm_groups(dk) * MM_NPT, {64, 64, 16});
 }
 
 extern "C" int he_mlstm_scan(void* y_f32, const void* q, const void* k, const void* v, int64_t in_stride,
@@ -511,30 +513,38 @@ extern "C" int he_mlstm_scan(void* y_f32, const void* q, const void* k, const vo
   const bool vec = dk % ve == 0 && in_stride < (1 << 24) && (in_stride * esz) % 16 == 0 && (((uintptr_t)q | (uintptr_t)k) & 15) == 0;
   const dim3 grid((dv + PB - 1) / PB, H, num_seqs);
   hipStream_t s = (hipStream_t)stream;
+  bool chunked = false;
   const int64_t need = he_mlstm_workspace_floats(rows, num_seqs, max_q_len, H, dk, dv, dtype);
   if (need > 0 && workspace_f32 != nullptr) {
     HE_REQUIRE(workspace_floats >= need && ((uintptr_t)workspace_f32 & 15) == 0,
                "he_mlstm_scan: the workspace has %lld floats of %lld, or is not aligned", (long long)workspace_floats, (long long)need);
     const MmChunks p = {(const float*)gates_f32, gate_bias, bias_dtype, raw_gates, H, dv, NG * MM_NPT, (int)grid.x, cap};
     const GcArgs<bf16_t> a = {(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, in_stride, 1, q_scale, (const int32_t*)cu_seqlens,
-                              (const int32_t*)seq_slot, num_seqs, H, dk, dv, NG * MM_NPT, (uint8_t*)state, state_stride,
+                              (const int32_t*)seq_slot, num_seqs, H, dk, dv, NG * MM_NPT, gc_from(num_seqs), (uint8_t*)state, state_stride,
                               state_offset, nullptr, nullptr};
-    if (gc_takes(a)) return gc_run((float*)y_f32, a, p, rows, (float*)workspace_f32, "he_mlstm_scan", s);
+    if (gc_takes(a)) {
+      const int rc = gc_run((float*)y_f32, a, p, rows, (float*)workspace_f32, "he_mlstm_scan", s);
+      if (rc || num_seqs == 1) return rc;
+      chunked = true;
+    }
   }
-  if (rows <= num_seqs) {       // no sequence brings more than a row, or the few that do are walked row by row
+  // behind the chunks: the sequences of a few rows by the first of the two, those up to GC_SHORT by the second
+  const int most = chunked ? GC_FEW : INT_MAX;
+  if (chunked || rows <= num_seqs) {       // no sequence brings more than a row, or the few that do are walked row by row
 #define MM_STEP(T)                                                                                                       \
   mlstm_step_kernel<T><<<grid, threads, 0, s>>>((float*)y_f32, (const T*)q, (const T*)k, (const T*)v, in_stride,          \
                                                 (const float*)gates_f32, (uint8_t*)state, state_stride, state_offset,    \
                                                 (const int32_t*)cu_seqlens, (const int32_t*)seq_slot, H, dk, dv, NG, PB,  \
-                                                q_scale, (int)vec, raw_gates, gate_bias, bias_dtype, cap)
+                                                q_scale, (int)vec, raw_gates, gate_bias, bias_dtype, cap, 1, most)
     if (dtype == HE_BF16) MM_STEP(bf16_t); else MM_STEP(float);
 #undef MM_STEP
-    return he_check_launch("he_mlstm_scan");
+    const int rc = he_check_launch("he_mlstm_scan");
+    if (rc || !chunked) return rc;
   }
   int TB = vec ? mm_block_rows(dk, dv, threads, 2 * dk / ve) : 0;
   const bool ahead = TB > 0;
   if (!ahead) TB = mm_block_rows(dk, dv, threads, 0);
-  if (rows < TB) TB = rows;        // a step of few rows stages no more than it has
+  TB = std::min(TB, chunked ? GC_SHORT : rows);        // a step of few rows stages no more than it has
   const size_t lds = sizeof(float) * ((size_t)2 * TB * NG * MM_NPT + (size_t)2 * TB * PB + 6 * TB + 4);
   HE_REQUIRE(TB >= 1 && lds <= 64 * 1024, "he_mlstm_scan: a block of %d rows needs %zu bytes of LDS", TB, lds);
 #define MM_LAUNCH(T, AHEAD)                                                                                              \
@@ -542,7 +552,8 @@ extern "C" int he_mlstm_scan(void* y_f32, const void* q, const void* k, const vo
                                                          (const float*)gates_f32, (uint8_t*)state, state_stride,         \
                                                          state_offset, (const int32_t*)cu_seqlens,                       \
                                                          (const int32_t*)seq_slot, H, dk, dv, NG, PB, TB, q_scale, \
-                                                         raw_gates, gate_bias, bias_dtype, cap)
+                                                         raw_gates, gate_bias, bias_dtype, cap, chunked ? GC_FEW + 1 : 1, \
+                                                         chunked ? GC_SHORT : INT_MAX)
   if (dtype == HE_BF16) {
     if (ahead) MM_LAUNCH(bf16_t, true); else MM_LAUNCH(bf16_t, false);
   } else {

@@ -216,8 +216,9 @@ extern "C" int he_conv_state(void* out, const void* x, int64_t x_stride, const v
 // does not depend on the step. A workgroup takes PB value dims of one (sequence, head) and walks the
 // sequence's rows in order; what a token brings (its B and C, the x of the workgroup's value dims,
 // its step size and decay, which one thread a token computes) is staged through LDS a tile of tokens
-// at a time, the next tile's loads in flight while this one is computed. Sequences of more than GC_FROM rows of
-// bf16 activations go by chunks (gated_chunks.h); with 32-bit ones results do not depend on how the rows were cut into steps. In the state area the
+// at a time, the next tile's loads in flight while this one is computed. Steps of long sequences of bf16 activations go by
+// chunks, all but their short sequences (gated_chunks.h: gc_pays, gc_from); with 32-bit ones results do not depend on how the rows were cut
+// into steps. In the state area the
 // workgroup's share of S lies in the order its threads load it, 16 bytes a lane: [i / 4][thread][i % 4].
 #define SS_PRE 16      // values a thread fetches for the next tile
 // state dims a thread holds. Measured at 64 heads of 64 with a state of 128, one prompt of 2,048 tokens: 0.93 ms
@@ -243,14 +244,14 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(
     float* __restrict__ y, const T* __restrict__ xbc, const T* __restrict__ dt_in, int64_t dt_stride,
     const void* __restrict__ dt_bias, const void* __restrict__ a_log, const void* __restrict__ d_skip, int w_dtype,
     uint8_t* __restrict__ state, int64_t state_stride, int64_t state_offset, const int32_t* __restrict__ cu_seqlens,
-    const int32_t* __restrict__ seq_slot, int R, int Q, int N, int P, int NG, int PB, int TT) {
+    const int32_t* __restrict__ seq_slot, int R, int Q, int N, int P, int NG, int PB, int TT, int least, int most) {
   extern __shared__ float4 ss_lds4[];
   float* lds = reinterpret_cast<float*>(ss_lds4);
   const int seq = blockIdx.z, r = blockIdx.y;
   const int slot = seq_slot[seq];
   if (slot < 0) return;
   const int t0 = cu_seqlens[seq], t1 = cu_seqlens[seq + 1];
-  if (t1 <= t0) return;
+  if (t1 - t0 < least || t1 - t0 > most) return;        // (sequences of least to most rows; least is 1 or more)
   const int tid = threadIdx.x, threads = blockDim.x;
   const int ng = tid % NG;
   const bool own = tid < PB * NG;                       // the thread holds a share of the state
@@ -432,7 +433,7 @@ struct SsChunks {
 // Floats of workspace he_ssm_scan wants to go by chunks (0: it walks the rows). max_q_len: the most rows of a sequence, 0: not known.
 extern "C" int64_t he_ssm_workspace_floats(int rows, int num_seqs, int max_q_len, int R, int N, int P, int dtype) {
   if (R <= 0 || N <= 0 || P <= 0 || dtype != HE_BF16) return 0;
-  return gc_floats(rows, num_seqs, max_q_len, R, P, ss_groups(N) * ss_npt(N));
+  return gc_floats(rows, num_seqs, max_q_len, R, P, ss_groups(N) * ss_npt(N), {96, 128, 32});
 }
 
 extern "C" int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int64_t dt_stride, const void* dt_bias,
@@ -452,6 +453,8 @@ extern "C" int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int6
   const int PB = ss_pb(N, P);
   const int threads = (PB * NG + 63) / 64 * 64;
   const int W = (2 * NG * ss_npt(N) + PB + 2 + 3) & ~3;
+  HE_REQUIRE(W <= SS_PRE * threads, "he_ssm_scan: a token's %d values do not fit a tile", W);
+  bool chunked = false;
   const int64_t need = he_ssm_workspace_floats(rows, num_seqs, max_q_len, R, N, P, dtype);
   if (need > 0 && workspace_f32 != nullptr) {
     HE_REQUIRE(workspace_floats >= need && ((uintptr_t)workspace_f32 & 15) == 0,
@@ -460,34 +463,42 @@ extern "C" int he_ssm_scan(void* y_f32, const void* xbc, const void* dt_in, int6
     const bf16_t* at = (const bf16_t*)xbc;
     const SsChunks p = {(const bf16_t*)dt_in, dt_stride, dt_bias, a_log, d_skip, w_dtype, NG, PB, ss_npt(N), (P + PB - 1) / PB};
     const GcArgs<bf16_t> a = {at + inner + Q * N, at + inner, at, inner + 2 * Q * N, R / Q, 1.f, (const int32_t*)cu_seqlens,
-                              (const int32_t*)seq_slot, num_seqs, R, N, P, NG * ss_npt(N), (uint8_t*)state, state_stride,
+                              (const int32_t*)seq_slot, num_seqs, R, N, P, NG * ss_npt(N), gc_from(num_seqs), (uint8_t*)state, state_stride,
                               state_offset, nullptr, nullptr};
-    if (gc_takes(a)) return gc_run((float*)y_f32, a, p, rows, (float*)workspace_f32, "he_ssm_scan", (hipStream_t)stream);
+    if (gc_takes(a)) {
+      const int rc = gc_run((float*)y_f32, a, p, rows, (float*)workspace_f32, "he_ssm_scan", (hipStream_t)stream);
+      if (rc || num_seqs == 1) return rc;
+      chunked = true;
+    }
   }
-  int TT = SS_PRE * threads / W;
-  TT = TT < 1 ? 1 : (TT > 16 ? 16 : TT);
-  if (max_q_len > 0 && TT > max_q_len) TT = max_q_len;      // no sequence brings more rows than that
-  HE_REQUIRE(W <= SS_PRE * threads, "he_ssm_scan: a token's %d values do not fit a tile", W);
-  if (2 * TT > threads) TT = threads / 2;               // a thread a token brings its step size, another its decay
-  const size_t lds_bytes = (size_t)2 * TT * W * sizeof(float);
   const dim3 grid((P + PB - 1) / PB, R, num_seqs);
   hipStream_t s = (hipStream_t)stream;
-  const bool trim = TT * W <= (SS_PRE / 2) * threads;
+  const int npt = ss_npt(N);
+  // the sequences of least to most rows, in tiles of no more tokens than they bring
+  auto walk = [&](int least, int most, int bound) {
+    int TT = SS_PRE * threads / W;
+    TT = std::min(TT < 1 ? 1 : (TT > 16 ? 16 : TT), bound);
+    if (2 * TT > threads) TT = threads / 2;               // a thread a token brings its step size, another its decay
+    const size_t lds_bytes = (size_t)2 * TT * W * sizeof(float);
+    const bool trim = TT * W <= (SS_PRE / 2) * threads;
 #define SCAN_LAUNCH(T, NPT)                                                                                       \
   if (trim) SCAN_LAUNCH_(T, NPT, true); else SCAN_LAUNCH_(T, NPT, false)
 #define SCAN_LAUNCH_(T, NPT, TRIM)                                                                                \
   ssm_scan_kernel<T, NPT, TRIM><<<grid, threads, lds_bytes, s>>>(                                                       \
       (float*)y_f32, (const T*)xbc, (const T*)dt_in, dt_stride, dt_bias, a_log, d_skip, w_dtype, (uint8_t*)state, \
-      state_stride, state_offset, (const int32_t*)cu_seqlens, (const int32_t*)seq_slot, R, Q, N, P, NG, PB, TT)
-  const int npt = ss_npt(N);
-  if (dtype == HE_BF16) {
-    if (npt == 8) { SCAN_LAUNCH(bf16_t, 8); } else { SCAN_LAUNCH(bf16_t, 16); }
-  } else {
-    if (npt == 8) { SCAN_LAUNCH(float, 8); } else { SCAN_LAUNCH(float, 16); }
-  }
+      state_stride, state_offset, (const int32_t*)cu_seqlens, (const int32_t*)seq_slot, R, Q, N, P, NG, PB, TT, least, most)
+    if (dtype == HE_BF16) {
+      if (npt == 8) { SCAN_LAUNCH(bf16_t, 8); } else { SCAN_LAUNCH(bf16_t, 16); }
+    } else {
+      if (npt == 8) { SCAN_LAUNCH(float, 8); } else { SCAN_LAUNCH(float, 16); }
+    }
 #undef SCAN_LAUNCH
 #undef SCAN_LAUNCH_
-  return he_check_launch("he_ssm_scan");
+    return he_check_launch("he_ssm_scan");
+  };
+  if (!chunked) return walk(1, INT_MAX, max_q_len > 0 ? max_q_len : INT_MAX);
+  const int rc = walk(1, GC_FEW, GC_FEW);
+  return rc ? rc : walk(GC_FEW + 1, GC_SHORT, GC_SHORT);
 }
 
 // ---- gated, grouped RMS norm ------------------------------------------------------------------

@@ -652,7 +652,7 @@ def ssm_scan(y, xbc, dt, dt_bias, a_log, d_skip, state, state_offset: int, cu_se
     sizes softplus(dt + dt_bias) (dt: a view [rows, R] of wider rows), per head r the decay
     exp(-exp(a_log_r) dt) and the skip d_skip_r; the state [R][P][N'] lives at byte state_offset of a
     sequence's row of `state` and is carried on. max_q_len: a bound on the rows a sequence brings (0: none).
-    workspace: fp32, ssm_workspace_floats elements or more: long sequences go by chunks (None: row by row)."""
+    workspace: fp32, ssm_workspace_floats elements or more: by chunks, all but the step's short sequences (None: row by row)."""
     C = R * P + 2 * Q * N
     _need(y, "y", torch.float32, (None, R * P))
     _need(xbc, "xbc", None, (None, C))
@@ -1109,7 +1109,7 @@ def mlstm_scan(y, q, k, v, gates, state, state_offset: int, cu_seqlens, seq_slot
     the same wider rows; the memory lives at byte state_offset of a sequence's row of `state` and is carried on.
     raw_gates: `gates` holds the pre-activations, and the kernel forms the logarithms itself from them, gate_bias
     ([2 H] or None) and cap, with mlstm_gates' arithmetic. max_q_len: a bound on the rows a sequence brings (0: none);
-    workspace: fp32, mlstm_workspace_floats elements or more: long sequences go by chunks (None: row by row)."""
+    workspace: fp32, mlstm_workspace_floats elements or more: by chunks, all but the step's short sequences (None: row by row)."""
     _need(y, "y", torch.float32, (None, H * dv))
     _need(gates, "gates", torch.float32, (None, 2 * H))
     stride = q.stride(0)

@@ -272,6 +272,54 @@ def test_state_space_over_several_windows(ops, R, Q, N, P, lengths):
             r += n
 
 
+@pytest.mark.parametrize("which", ["mlstm", "ssm"])
+def test_short_sequences_of_a_long_step_are_walked(ops, which):
+    """Sequences of up to 16 rows beside longer ones have the bits they have alone, rows and states, and no chunk of the workspace; the longer
+    ones are the chunks', whatever walks beside them. 70 sequences: the search for a chunk's sequence goes through two turns of 64."""
+    bf16, lengths = torch.bfloat16, ([1, 4, 5, 16, 17, 200, 2, 64, 65, 3] * 7)
+    B, rows = len(lengths), sum(lengths)
+    cu = [0] + torch.tensor(lengths).cumsum(0).tolist()
+    if which == "mlstm":
+        H, dk, dv = 2, 24, 36
+        x, gates = rnd(rows, H * (2 * dk + dv), seed=1).bfloat16().cuda(), (-rnd(rows, 2 * H, seed=2).abs()).float().cuda()
+        start = torch.rand((B, ops.mlstm_state_floats(H, dk, dv)), generator=torch.Generator().manual_seed(3)).cuda()
+        width, floats = H * dv, lambda *a: ops.mlstm_workspace_floats(*a, H, dk, dv, bf16)
+
+        def scan(at, lens, state, ws):
+            y, v = torch.full((sum(lens), width), float("nan"), device="cuda"), x[at]
+            ops.mlstm_scan(y, v[:, :H * dk], v[:, H * dk:2 * H * dk], v[:, 2 * H * dk:], gates[at], state, 0, cu_of(lens), i32(*range(len(lens))), sum(lens),
+                           len(lens), H, dk, dv, 0.2, max_q_len=max(lens), workspace=ws)
+            return y
+    else:
+        R, Q, N, P = 4, 2, 20, 36
+        x, dt = rnd(rows, R * P + 2 * Q * N, seed=1).bfloat16().cuda(), rnd(rows, R, seed=2).bfloat16().cuda()
+        one = torch.ones(R, device="cuda")
+        start = torch.rand((B, ops.ssm_state_floats(R, P, N)), generator=torch.Generator().manual_seed(3)).cuda()
+        width, floats = R * P, lambda *a: ops.ssm_workspace_floats(*a, R, N, P, bf16)
+
+        def scan(at, lens, state, ws):
+            y = torch.full((sum(lens), width), float("nan"), device="cuda")
+            ops.ssm_scan(y, x[at], dt[at], one, -one, one, state, 0, cu_of(lens), i32(*range(len(lens))), sum(lens), len(lens), R, Q, N, P,
+                         max_q_len=max(lens), workspace=ws)
+            return y
+    bytes_of = lambda t: t.clone().view(torch.uint8)
+    state = bytes_of(start)
+    room = floats(rows, B, max(lengths))
+    assert room > 0
+    got = scan(slice(0, rows), lengths, state, torch.full((room,), float("nan"), device="cuda"))
+    for b, n in enumerate(lengths[:20]):
+        at, alone = slice(cu[b], cu[b + 1]), bytes_of(start[b:b + 1])
+        ws = torch.full((floats(n, 1, n),), float("nan"), device="cuda") if n > 96 else None
+        y = scan(at, [n], alone, ws)
+        if n <= 16 or n > 96:
+            assert torch.equal(got[at], y) and torch.equal(state[b], alone[0]), n
+        else:
+            assert rel(got[at], y.double()) < 2e-6 and rel(state[b].view(torch.float32), alone[0].view(torch.float32).double()) < 2e-6, n
+    assert bool(torch.isfinite(got).all())
+    # one sequence of 200 rows among 63 of one row: room for its chunks and for those 63 rows could have, not for 63 memories more
+    assert 0 < floats(263, 64, 200) <= 5 * floats(200, 1, 200)
+
+
 def test_what_goes_by_chunks(ops):
     """Short or unknown lengths and 32-bit activations are walked, and so are heads that are no whole fours, whatever workspace is given."""
     bf16 = torch.bfloat16
