@@ -484,9 +484,10 @@ static int gc_run(float* y, const GcArgs<T>& args, const P& p, int rows, float* 
   return he_check_launch(name);
 }
 
-// Whole fours of every row and head, which the kernels above load at once.
+// Whole fours of every row and head, which the kernels above load at once. (Head sizes that are none are not given a workspace either.)
+static inline bool gc_heads(int dk, int dv) { return dk % 4 == 0 && dv % 4 == 0; }
 template <typename T>
 static inline bool gc_takes(const GcArgs<T>& a) {
-  return a.dk % 4 == 0 && a.dv % 4 == 0 && a.stride % 4 == 0 && a.H <= 65535 && a.num_seqs <= 65535 &&
+  return gc_heads(a.dk, a.dv) && a.stride % 4 == 0 && a.H <= 65535 && a.num_seqs <= 65535 &&
          (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & (4 * sizeof(T) - 1)) == 0;
 }

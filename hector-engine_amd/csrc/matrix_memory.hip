@@ -489,7 +489,7 @@ struct MmChunks {
 
 // Floats of workspace he_mlstm_scan wants to go by chunks (0: it walks the rows). max_q_len: the most rows of a sequence, 0: not known.
 extern "C" int64_t he_mlstm_workspace_floats(int rows, int num_seqs, int max_q_len, int H, int dk, int dv, int dtype) {
-  if (H <= 0 || dk <= 0 || dv <= 0 || dtype != HE_BF16) return 0;
+  if (H <= 0 || dk <= 0 || dv <= 0 || dtype != HE_BF16 || !gc_heads(dk, dv)) return 0;
   return gc_floats(rows, num_seqs, max_q_len, H, dv + 1, mm_groups(dk) * MM_NPT, {64, 64, 16});
 }
 

@@ -432,7 +432,7 @@ struct SsChunks {
 
 // Floats of workspace he_ssm_scan wants to go by chunks (0: it walks the rows). max_q_len: the most rows of a sequence, 0: not known.
 extern "C" int64_t he_ssm_workspace_floats(int rows, int num_seqs, int max_q_len, int R, int N, int P, int dtype) {
-  if (R <= 0 || N <= 0 || P <= 0 || dtype != HE_BF16) return 0;
+  if (R <= 0 || N <= 0 || P <= 0 || dtype != HE_BF16 || !gc_heads(N, P)) return 0;
   return gc_floats(rows, num_seqs, max_q_len, R, P, ss_groups(N) * ss_npt(N), {96, 128, 32});
 }
 

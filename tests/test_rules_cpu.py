@@ -202,3 +202,21 @@ def test_which_products_of_few_rows_want_a_workspace():
     assert [M for M in range(1, 10) if wants(M, 512, 12288)] == list(range(1, 9))
     assert [M for M in range(1, 10) if wants(M, 2048, 8192)] == [1, 2] and not wants(1, 2049, 8192)
     assert wants(8, 37888, 3584, torch.bfloat16) and wants(8, 100, 1000) and not wants(9, 100, 1000) and wants(8, 8, 256, shift=1)
+
+
+def test_scans_ask_for_a_workspace_where_they_go_by_chunks_alone():
+    """Heads of whole fours of bf16 activations whose longest sequence is long enough beside the others; of several sequences room for
+    the chunks of those of more than 16 rows."""
+    from hector_engine_amd.kernels import ops
+    bf16, f32 = torch.bfloat16, torch.float32
+    mlstm = lambda rows, n, most, dtype=bf16, dk=128, dv=256: ops.mlstm_workspace_floats(rows, n, most, 14, dk, dv, dtype)
+    ssm = lambda rows, n, most, dtype=bf16, N=128, P=64: ops.ssm_workspace_floats(rows, n, most, 64, N, P, dtype)
+    assert mlstm(2048, 1, 2048) and ssm(2048, 1, 2048)
+    for scan in (mlstm, ssm):
+        assert not scan(2048, 1, 2048, f32) and not scan(2048, 1, 2048, bf16, 126, 64) and not scan(2048, 1, 2048, bf16, 64, 66)
+        assert not scan(64, 1, 2048) and not scan(2048, 40, 64) and not scan(2048, 1, 0)        # a bound above what the step has; no bound
+    assert mlstm(65, 1, 65) and not ssm(96, 1, 96) and ssm(97, 1, 97)
+    assert mlstm(133, 64, 70) and not ssm(133, 64, 70) and not ssm(135, 8, 128) and ssm(136, 8, 129)      # beside sequences of one row
+    assert ssm(280, 4, 70) and not mlstm(318, 32, 70) and mlstm(2296, 32, 2048)                           # of 70 rows, of 8
+    one = mlstm(200, 1, 200) // 4                                                                         # 200 rows: four chunks
+    assert mlstm(263, 64, 200) == 19 * one                                                                # 263 / 64, and 263 / 17 sequences
