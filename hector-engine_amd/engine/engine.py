@@ -30,7 +30,7 @@ from ..parts.base import BuildEnv, StepContext
 from ..registry import build_model, load_config
 from ..weights.loader import load_tensors
 from ..weights.random_init import random_tensors
-from .scratch import ScratchPool
+from .scratch import ScratchPool, SharedScratch
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32,
            "fp32": torch.float32}
@@ -91,12 +91,12 @@ def _pow2(n: int, least: int = 1) -> int:
 
 class _GraphBucket:
     def __init__(self, size: int, device, seqs: int | None = None, wants: int | None = None,
-                 row_tables: int = 0):
+                 row_tables: int = 0, shared: SharedScratch | None = None):
         self.size = size
         self.meta = _Meta(size, size if seqs is None else seqs, size if wants is None else wants, row_tables)
         self.dev = torch.zeros(self.meta.total, dtype=torch.int32, device=device)
         self.views = self.meta.views(self.dev)
-        self.pool = ScratchPool(device)
+        self.pool = ScratchPool(device, shared=shared)
         self.graph: torch.cuda.CUDAGraph | None = None
         self.logits: torch.Tensor | None = None
         self.uses = 0
@@ -170,7 +170,8 @@ class Engine:
         # the cache counts in whole pages; the engine holds sequences to the length asked for
         self._max_seq_len = min(max_seq_len, self.cache.max_seq_len)
         self.caches = [self.cache.layer_cache(r) for r in range(len(self.model.schedule))]
-        self.scratch = ScratchPool(self.device)
+        self.shared = SharedScratch(self.device)
+        self.scratch = ScratchPool(self.device, shared=self.shared)
         self.profiler = profiler.OpProfiler() if profile else None
         self.sync_each_launch = sync_each_launch
         self.use_graphs = use_graphs and self.model.graph_safe() and not profile and not sync_each_launch
@@ -390,7 +391,7 @@ class Engine:
         # are there 1.8 us after the kernel's start instead of 3.0).
         by_row = groups * size * blocks if groups * size * blocks * 4 <= ROW_TABLES_MAX_BYTES else 0
         if bucket is None:
-            bucket = self._buckets[(size, hints)] = _GraphBucket(size, self.device, row_tables=by_row)
+            bucket = self._buckets[(size, hints)] = _GraphBucket(size, self.device, row_tables=by_row, shared=self.shared)
         # every row of the bucket gets logits; padding rows are inert (row_seq -1)
         padded = [StepEntry(e.slot, e.tokens, [0]) for e in entries]
         host, idx, _ = self._pack(padded, bucket.meta, size, size)
@@ -477,7 +478,7 @@ class Engine:
         if bucket is None:
             if len(self._plans) >= GRAPH_MAX_STEP_PLANS:
                 self._plans.popitem(last=False)          # the least recently used graph and its buffers
-            bucket = self._plans[plan] = _GraphBucket(R, self.device, S, max(W, 1))
+            bucket = self._plans[plan] = _GraphBucket(R, self.device, S, max(W, 1), shared=self.shared)
         self._plans.move_to_end(plan)
         host, idx, nw = self._pack(entries, bucket.meta, R, S)
         self._upload(host, idx, bucket.dev)

@@ -6,7 +6,8 @@ the logits), and two that the layers take in turn. A layer's arena is reset when
 layer after the next begins, so what a layer hands to its successor (a branch output
 not yet added, the rows prepared for the next norm) stays valid while that one runs,
 and a step holds the activations of two layers, not of all of them. Inside a layer,
-mark() / release() give back the temporaries of a loop's turn.
+mark() / release() give back the temporaries of a loop's turn. What one operation alone reads
+and writes comes from transient(): one buffer for all pools of an engine.
 
 Tensors handed out are views into an arena and are valid until it is reset. When an
 arena is too small, a larger one replaces it (views of the old one stay valid through
@@ -52,9 +53,30 @@ class _Arena:
         self.spilled = 0
 
 
-class ScratchPool:
-    def __init__(self, device, initial_bytes: int = 1 << 20):
+class SharedScratch:
+    """A buffer that all pools of an engine hand out, one operation at a time: an engine's steps follow each other on one
+    stream, so plans captured for many sizes need not keep a workspace each. It grows by half at least and never shrinks;
+    a pool that backs a captured graph keeps the buffer its graph was captured with."""
+
+    def __init__(self, device):
         self.device = device
+        self.buffer: torch.Tensor | None = None
+
+    def take(self, nbytes: int, may_grow: bool) -> torch.Tensor:
+        have = 0 if self.buffer is None else self.buffer.numel()
+        if nbytes > have:
+            if not may_grow:
+                raise RuntimeError("scratch pool of a captured graph cannot grow")
+            self.buffer = torch.empty(max(nbytes, have + have // 2), dtype=torch.uint8, device=self.device)
+        return self.buffer
+
+
+class ScratchPool:
+    def __init__(self, device, initial_bytes: int = 1 << 20, shared: SharedScratch | None = None):
+        """shared: the engine's buffer for transient(); a pool by itself has one of its own."""
+        self.device = device
+        self.shared = shared or SharedScratch(device)
+        self._held: torch.Tensor | None = None      # the shared buffer this step's operations used last
         self.frozen = False
         self.peak = 0
         self._arenas = [_Arena(device, initial_bytes) for _ in range(3)]   # step, layers in turn
@@ -93,6 +115,16 @@ class ScratchPool:
         a = self._arenas[index]
         if index == self._current and a.generation == generation:
             a.offset = offset
+
+    def transient(self, shape, dtype: torch.dtype) -> torch.Tensor:
+        """Memory of one operation: valid until transient() is called again, by whatever pool of the engine."""
+        numel = 1
+        for s in shape:
+            numel *= int(s)
+        nbytes = numel * torch.empty((), dtype=dtype).element_size()
+        self._held = self.shared.take(nbytes, not self.frozen)
+        self.peak = max(self.peak, sum(x.high + x.spilled for x in self._arenas) + nbytes)
+        return self._held[:nbytes].view(dtype).view(*shape)
 
     def alloc(self, shape, dtype: torch.dtype) -> torch.Tensor:
         numel = 1

@@ -100,13 +100,11 @@ class MatrixMemory(Mixer):
         y = ctx.alloc((rows, H * dv), torch.float32)
         if ctx.padded:
             y.zero_()           # the scan writes the rows of sequences only
-        turn = ctx.scratch.mark()           # (the chunks' memories are the scan's own)
         floats = ops.mlstm_workspace_floats(rows, ctx.num_seqs, ctx.max_q_len, H, dk, dv, proj.dtype)
-        ws = ctx.alloc((floats,), torch.float32) if floats else None
+        ws = ctx.scratch.transient((floats,), torch.float32) if floats else None
         ops.mlstm_scan(y, proj[:, :H * dk], proj[:, H * dk:2 * H * dk], proj[:, 2 * H * dk:2 * H * dk + H * dv], pre,
                        cache.state, 0, ctx.cu_seqlens, ctx.seq_slot, rows, ctx.num_seqs, H, dk, dv, self.q_scale,
                        raw_gates=True, gate_bias=self.gate_bias, cap=self.cap, max_q_len=ctx.max_q_len, workspace=ws)
-        ctx.scratch.release(turn)
         g = ctx.alloc((rows, H * dv))
         ops.gated_group_norm(g, y, proj[:, 2 * H * dk + H * dv:], self.norm, rows, H, self.eps, gate_after=True,
                              out_scale=self.out_scale * out_scale)

@@ -117,13 +117,11 @@ class SelectiveScanMixer(Mixer):
         y = ctx.alloc((rows, inner), torch.float32)
         if ctx.padded:
             y.zero_()           # the scan writes the rows of sequences only
-        turn = ctx.scratch.mark()           # (the chunks' memories are the scan's own)
         floats = ops.ssm_workspace_floats(rows, ctx.num_seqs, ctx.max_q_len, self.R, self.N, self.P, xbc.dtype)
-        ws = ctx.alloc((floats,), torch.float32) if floats else None
+        ws = ctx.scratch.transient((floats,), torch.float32) if floats else None
         ops.ssm_scan(y, xbc, proj[:, inner + self.C:], self.dt_bias, self.a_log, self.d_skip, cache.state,
                      self._conv_bytes(), ctx.cu_seqlens, ctx.seq_slot, rows, ctx.num_seqs,
                      self.R, self.Q, self.N, self.P, max_q_len=ctx.max_q_len, workspace=ws)
-        ctx.scratch.release(turn)
         g = ctx.alloc((rows, inner))
         ops.gated_group_norm(g, y, proj[:, :inner], self.norm, rows, self.parts, self.eps)
         return self.o_proj(g, rows, ctx, sink=ctx.take_sink())

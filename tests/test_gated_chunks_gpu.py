@@ -336,3 +336,25 @@ def test_what_goes_by_chunks(ops):
                        max_q_len=rows, workspace=ws)
         got.append(y)
     assert torch.equal(*got)
+
+
+def test_captured_steps_share_the_workspace():
+    """Steps of several sizes as graphs, whose chunks lie in one buffer of the engine: it grows between a graph's capture and its replays,
+    and every replay gives the logits the step's first, eager run gave."""
+    import hector_engine_amd as he
+    from hector_engine_amd.registry import config_from_dict
+    from tests.test_butolorn_cpu import attn, layer, memory, model, pair
+    H, dk, dv = 4, 64, 96
+    layers = [layer("parallel", pair(attn(2, 1, 16, 16, 0.25, 8), memory(H, dk, dv, 15.0)), 64)] * 2
+    engine = he.Engine(config=config_from_dict(model(layers, 50, 32, 8)), seed=3, dtype="bfloat16", max_tokens=4096, max_slots=2, max_seq_len=1024)
+    first, sizes = {}, []
+    for n in (100, 100, 300, 100, 500, 300, 200, 100, 500, 300, 200, 100, 500, 200):
+        slot = engine.acquire()
+        logits = engine.step([he.StepEntry(slot, [(7 * i + n) % 50 for i in range(n)], [0, n // 2, n - 1])]).clone()
+        engine.release(slot)
+        assert torch.equal(logits, first.setdefault(n, logits)) and bool(torch.isfinite(logits).all())
+        sizes.append(engine.shared.buffer.numel())
+        engine.scratch.transient((sizes[-1] // 4,), torch.float32).fill_(float("nan"))       # what a graph finds there is not its own
+    # 300 and 500 rows run as 512 rows, 200 as 256
+    assert engine.stats["step_graph_captures"] == 3 and engine.stats["step_graph_replays"] == 11 and not engine.capture_failures
+    assert sizes[1] < sizes[2] == sizes[-1] >= 4 * (512 // 64 + 1) * H * dk * (dv + 1)

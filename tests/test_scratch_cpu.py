@@ -2,7 +2,7 @@
 import torch
 
 import hector_engine_amd  # noqa: F401
-from hector_engine_amd.engine.scratch import ScratchPool
+from hector_engine_amd.engine.scratch import ScratchPool, SharedScratch
 
 
 def test_a_layers_tensors_outlive_the_next_layer_but_not_the_one_after():
@@ -68,3 +68,28 @@ def test_an_arena_that_was_too_small_is_made_whole_at_the_next_step_and_a_frozen
     else:
         raise AssertionError("a frozen pool grew")
 
+
+
+def test_pools_share_the_memory_of_single_operations():
+    """One buffer for all pools, whatever each asks for; a frozen pool keeps the one it was given last and does not make it grow; a pool by
+    itself has its own."""
+    shared = SharedScratch("cpu")
+    one, two, alone = ScratchPool("cpu", 256, shared), ScratchPool("cpu", 256, shared), ScratchPool("cpu", 256)
+    a = one.transient((100, 10), torch.float32)
+    assert a.shape == (100, 10) and one.peak >= 4000 and one.capacity == 3 * 256
+    assert two.transient((10,), torch.float32).data_ptr() == a.data_ptr() != alone.transient((10,), torch.float32).data_ptr()
+    one.frozen = True
+    one.reset()
+    assert one.transient((1000,), torch.float32).data_ptr() == a.data_ptr()
+    try:
+        one.transient((1001,), torch.float32)
+    except RuntimeError as e:
+        assert "cannot grow" in str(e)
+    else:
+        raise AssertionError("a frozen pool grew")
+    a.fill_(3.0)
+    b = two.transient((1001,), torch.float32)
+    assert shared.buffer.numel() == 6000 and b.data_ptr() != a.data_ptr()       # by half, and not by four bytes
+    b.fill_(5.0)
+    assert one._held.data_ptr() == a.data_ptr() and a.eq(3.0).all()             # as a graph captured with it would find it
+    assert one.transient((1000,), torch.float32).data_ptr() == b.data_ptr()
