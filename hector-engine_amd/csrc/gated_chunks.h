@@ -382,6 +382,9 @@ __global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* 
   float4 vx[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) vx[i] = gc_tile4(vr, a.stride, (t >> 4) + 16 * i, n, c0 + 4 * (t & 15), a.dv);
+  float zero = 0.f;                           // (what is not finite shows as NaN)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) zero = fmaf(vx[i].x, 0.f, fmaf(vx[i].y, 0.f, fmaf(vx[i].z, 0.f, fmaf(vx[i].w, 0.f, zero))));
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(vs + ((t >> 4) + 16 * i) * GC_LD + 4 * (t & 15)) = vx[i];
@@ -396,7 +399,7 @@ __global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* 
       square_s[i * GC_LD + j] = j <= i && j < n ? e * square[r] : 0.f;
     }
   }
-  __syncthreads();
+  const bool finite = !__syncthreads_or(!(zero == 0.f));
   if (P::NORMED) {
     float some = 0.f;
 #pragma unroll
@@ -413,7 +416,7 @@ __global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* 
   for (int r = 0; r < 16; ++r) square[r] = lost_s[r] = 0.f;      // (from here on the square's share of the result)
 #pragma unroll
   for (int g0 = 0; g0 < CK_ROWS; g0 += 16) {
-    if (g0 >= i0 + 32 || g0 >= n) break;      // (the same in the wavefront)
+    if (g0 >= i0 + 32 || g0 >= n || !finite) break;      // (the same in the wavefront)
     gc_acc some[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -422,6 +425,15 @@ __global__ __launch_bounds__(256, P::NORMED ? 3 : 4) void gc_rows_kernel(float* 
       some[u] = gc_mfma4(*reinterpret_cast<const float4*>(square_s + (i0 + l32) * GC_LD + g), make_float4(v[0], v[GC_LD], v[2 * GC_LD], v[3 * GC_LD]));
     }
     gc_add<P::NORMED>(square, lost_s, some[0], some[1]);
+  }
+  if (!finite) {      // a row sees the values up to its own: an infinity behind it, times the square's zero, would be NaN
+    for (int j = 0; j < n; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = i0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+        if (j <= i) square[r] = fmaf(square_s[i * GC_LD + j], vs[j * GC_LD + j0 + l32], square[r]);
+      }
+    }
   }
   if (P::NORMED) __syncthreads();
   const int c = c0 + j0 + l32;

@@ -130,6 +130,38 @@ def test_matrix_memory_of_closed_gates(ops):
     assert rel(got[1], got[0]) < 1e-4
 
 
+@pytest.mark.parametrize("which", ["mlstm", "ssm"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_rows_before_one_that_is_not_finite(ops, which, bad):
+    """A value that is no number, in the middle of a chunk: the rows before it are what they are without it, those behind it are no numbers
+    in its column, as the walk has them, and the other columns never see it."""
+    rows, at, col, bf16 = 200, 90, 5, torch.bfloat16
+    got = []
+    for value, way in ((0.5, "chunks"), (bad, "chunks"), (bad, "walk")):
+        if which == "mlstm":
+            H, dk, dv = 2, 32, 64
+            x, gates = rnd(rows, H * (2 * dk + dv), seed=1).bfloat16().cuda(), (-rnd(rows, 2 * H, seed=2).abs()).float().cuda()
+            x[at, 2 * H * dk + col] = value
+            y, state = torch.empty(rows, H * dv, device="cuda"), torch.zeros((1, 4 * ops.mlstm_state_floats(H, dk, dv)), dtype=torch.uint8, device="cuda")
+            ws = torch.empty(ops.mlstm_workspace_floats(rows, 1, rows, H, dk, dv, bf16), device="cuda") if way == "chunks" else None
+            ops.mlstm_scan(y, x[:, :H * dk], x[:, H * dk:2 * H * dk], x[:, 2 * H * dk:], gates, state, 0, i32(0, rows), i32(0), rows, 1, H, dk, dv, 1.0,
+                           max_q_len=rows, workspace=ws)
+        else:
+            R, Q, N, P = 2, 1, 16, 68
+            x, dt, one = rnd(rows, R * P + 2 * Q * N, seed=1).bfloat16().cuda(), rnd(rows, R, seed=2).bfloat16().cuda(), torch.ones(R, device="cuda")
+            x[at, col] = value
+            y, state = torch.empty(rows, R * P, device="cuda"), torch.zeros((1, 4 * ops.ssm_state_floats(R, P, N)), dtype=torch.uint8, device="cuda")
+            ws = torch.empty(ops.ssm_workspace_floats(rows, 1, rows, R, N, P, bf16), device="cuda") if way == "chunks" else None
+            ops.ssm_scan(y, x, dt, one, one, one, state, 0, i32(0, rows), i32(0), rows, 1, R, Q, N, P, max_q_len=rows, workspace=ws)
+        got.append(y)
+    good, chunks, walk = got
+    # (the column's chunk goes through another loop: the same products, summed one after the other)
+    assert rel(chunks[:at], good[:at].double()) < 2e-6
+    assert torch.equal(chunks.isfinite(), walk.isfinite()) and not chunks[at:, col].isfinite().any()
+    others = torch.arange(y.shape[1], device="cuda") != col
+    assert rel(chunks[:, others], good[:, others].double()) < 2e-6
+
+
 def test_state_space_that_forgets_at_once(ops):
     """A decay of exp(-exp(a_log) dt) with exp(a_log) beyond the floats: every row forgets the ones before it."""
     R, Q, N, P, rows = 2, 1, 16, 8, 130
