@@ -128,7 +128,9 @@ extern "C" int he_add_group_normed(void* resid_f32, const void* delta, int delta
   // (a branch is added, or a norm taken; of both the groups must be the same)
   const int parts = delta != nullptr ? groups : next_weight != nullptr ? next_groups : 1;
   const int per = (D / parts + 63) / 64;
-  // (more than 16 elements a lane of many rows: 3,001 rows of 8192 in 4 groups 77 us, 95 in registers; 4 rows 12.7 and 9.3)
+  // (us of the kernel above and in registers, a branch of bf16 added and normed on. Up to 16 elements a lane, 1 to 3,001 rows: 0.61 to 0.85 of it. 20 to 32
+  // elements: up to 512 rows 0.55 to 0.84 of it, 1,024 rows 0.60 to 1.13, 3,001 rows 1.05 to 1.50: 8192 in 4 groups, 64 rows 22.6 and 12.9, 3,001 rows 117 and 150. The line
+  // for these is far on the safe side. The bits are the same.)
   const bool regs = per <= (rows <= 64 ? 32 : 16) && (delta == nullptr ? next_weight != nullptr : next_weight == nullptr || out == nullptr || next_groups == groups);
 #define GN_REGS(TD, TO, PER)                                                                                       \
   add_group_normed_regs_kernel<TD, TO, PER><<<rows, threads, 0, s>>>((float*)resid_f32, (const TD*)delta, weight, w_dtype,  \

@@ -180,8 +180,9 @@ extern "C" int he_conv_state(void* out, const void* x, int64_t x_stride, const v
   conv_rows_kernel<T, K_><<<dim3((C / 4 + 255) / 256, (rows + CV_ROWS - 1) / CV_ROWS), 256, 0, s>>>(    \
       (T*)out, (const T*)x, x_stride, taps, bias, w_dtype, (const uint8_t*)state, state_stride,         \
       (const int32_t*)positions, (const int32_t*)row_seq, (const int32_t*)seq_slot, (const int32_t*)seq_start, rows, C, act)
-  // runs of rows: two to four taps, channels in whole fours, and work for the whole chip (24 rows of 2048 channels 5 us above, 10 here;
-  // 2,048 rows of 2048 23 and 16)
+  // runs of rows: two to four taps, channels in whole fours, and work for the whole chip. (us above and here, four taps of 512, 2048 and 6144 channels,
+  // one sequence or four: 2^18 values 5.4 to 5.8 and 9.6 to 10.4; 2^20 8.5 to 8.9 and 9.9 to 10.7; 2^21 13 and 11 to 12; 2^22 21 to 34 and 14 to 16; 2^24 87 to 117
+  // and 37 to 42. The line is where it is faster for all of them by a third.)
   const int esz = dtype == HE_BF16 ? 2 : 4;
   const bool runs = !all_single && (int64_t)rows * C >= 1 << 22 && K >= 2 && K <= 4 && C % 4 == 0 && x_stride % 4 == 0 &&
                     (((uintptr_t)x | (uintptr_t)out) & (4 * esz - 1)) == 0 && ((uintptr_t)state & 15) == 0 && state_stride % 16 == 0;

@@ -37,6 +37,24 @@ def test_add_group_normed(width, rows, groups, next_groups):
             close(out, gn(want, next_groups, 1e-2) * follow.to(F64) if norm else want, ot)
 
 
+@pytest.mark.parametrize("width,groups", [(1025, 1), (1537, 2), (2048, 1), (2048, 4)])
+@pytest.mark.parametrize("dt,ot", [(BF16, BF16), (F32, F32), (None, BF16)])
+def test_rows_have_the_same_bits_in_any_company(width, groups, dt, ot):
+    """More than 16 elements a lane are held in registers up to 64 rows and read again beyond: the same rows in a step of 64 and in one of 130."""
+    from hector_engine_amd.kernels import ops
+    D = width * groups
+    g = torch.Generator().manual_seed(D)
+    resid, weight, follow = torch.randn(130, D, generator=g), torch.randn(D, generator=g).cuda(), torch.randn(D, generator=g).cuda()
+    delta = None if dt is None else torch.randn(130, D, generator=g).to(dt)
+    got = {}
+    for rows in (64, 130):
+        r, out = resid[:rows].cuda(), torch.empty(rows, D, dtype=ot, device="cuda")
+        ops.add_group_normed(r, None if delta is None else delta[:rows].cuda(), None if delta is None else weight, groups, 1e-3, 0.5, out, rows,
+                             next_weight=follow, next_groups=groups, next_eps=1e-2)
+        got[rows] = r[:64].cpu(), out[:64].cpu()
+    assert torch.equal(got[64][0], got[130][0]) and torch.equal(got[64][1], got[130][1])
+
+
 @pytest.mark.parametrize("rows,D,Dx", [(3, 100, 129), (70, 2048, 2049), (3, 511, 4100), (1, 1, 1)])
 @pytest.mark.parametrize("dtype", [BF16, F32])
 def test_gated_add(rows, D, Dx, dtype):
