@@ -8,7 +8,7 @@
 //   S'  = exp(F_n) S + sum over j of exp(F_n - F_j) w_j v_j k_j^T
 // are matrix products, in three launches: every chunk's own share of S' (all chunks at once), the memory before every
 // chunk (one walk over the chunks of a sequence, element by element), every chunk's rows (all at once). (The same two prompts of
-// 2,048 rows: 125 and 136 us alone.)
+// 2,048 rows: 141 and 138 us alone.)
 // F is summed in 64 bits and no exponent is positive, so the powers are as exact as the
 // walk's; everything else is fp32 arithmetic as there. What bounds the three: the share and the rows kernel the fp32
 // products, the walk over chunks the memories it reads and writes (two passes over 4 (dv + 1) dk bytes a head and chunk).
