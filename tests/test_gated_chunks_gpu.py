@@ -78,8 +78,8 @@ def test_matrix_memory_by_chunks(ops, H, dk, dv, keep, write):
                     g64[at, h], g64[at, H + h], plain[b][h])
             r += n
         e = {way: rel(got[way].cpu(), want) for way in got}
-        # 32-bit sums and exponentials: a few 2^-24
-        assert e["chunks"] <= max(2e-6, 1.5 * e["walk"])
+        # 32-bit sums and exponentials: a few 2^-24, the two about as far from 64 bits as each other (single inputs: a third either way)
+        assert e["chunks"] <= 1.3 * e["walk"] < 1e-5
 
 
 @pytest.mark.parametrize("rows,keep,positive", [(500, 0.0, False), (500, 3.0, True), (2048, 0.0, False)])
@@ -217,7 +217,7 @@ def test_state_space_by_chunks(ops, R, Q, N, P, decay):
                 want[at, h * P:(h + 1) * P] = y + skip[h].double() * x
             r += n
         e = {way: rel(got[way].cpu(), want) for way in got}
-        assert e["chunks"] <= max(2e-6, 1.5 * e["walk"])
+        assert e["chunks"] <= 1.3 * e["walk"] < 1e-5
 
 
 def chunks_of(lengths):
