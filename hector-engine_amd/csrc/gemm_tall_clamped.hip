@@ -1,0 +1,8 @@
+// Products of many rows (gemm_tall_tiles.h): results of the other gated activations.
+#include "gemm_tall_tiles.h"
+
+int gt_run_clamped(const GtCase& c, int tile, int mtiles, hipStream_t s) {
+#define GT_CASE(BM, BN, NX, NW) if (tile == ((BM) << 16 | (BN))) return gt_run<BM, BN, NX, NW, GT_GATED, true>(c, mtiles, s);
+  GT_TILES(GT_CASE)
+  return -1;
+}

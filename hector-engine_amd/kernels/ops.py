@@ -1216,10 +1216,10 @@ def tiles_read(*tensors) -> bool:
 
 
 @_op("gemm_tall")
-def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
+def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, bn: int = 256, act=None) -> None:
     """out[M, N] = x[M, K] . w[N, K]^T (+ bias) for many bf16 rows (bf16 or fp32 results); with act, the constants (alpha,
     limit, up_shift, cubic) of a gated activation, w's rows alternate gate and up and out is [M, N / 2]. K a multiple
-    of 64, N of 4. bm: rows of a tile, 128 or 256."""
+    of 64, N of 4. bm, bn: the outputs of a tile (gemm_tall_tile)."""
     N, K = w.shape
     cols = N // 2 if act is not None else N
     _need(out, "out", None, (None, cols))
@@ -1233,7 +1233,14 @@ def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, act=None) -> None:
     alpha, limit, up_shift, cubic = act or (1.0, 0.0, 0.0, 0.0)
     _lib.check(_lib.load().he_gemm_tall_bf16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias),
                                              dtype_code(bias.dtype) if bias is not None else F32, M, N, K, K, K, cols, epilogue,
-                                             bm, float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+                                             bm << 16 | bn, float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_tall_tile(M: int, N: int, K: int) -> tuple[int, int]:
+    """(bm, bn) of the tile gemm_tall is fastest with, by estimate."""
+    tile = int(_lib.load().he_gemm_tall_tile(M, N, K))
+    return tile >> 16, tile & 0xffff
 
 
 @functools.lru_cache(maxsize=4096)

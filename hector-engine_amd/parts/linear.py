@@ -226,10 +226,10 @@ class Linear:
         return slices
 
     def _tall(self, rows: int, x, out, out_dtype) -> bool:
-        """Whether a product of long K runs in tiles of 128 x 256 outputs (kernels.ops.gemm_tall): for K from 16448 to 27648, where
+        """Whether a product of long K runs in tiles (kernels.ops.gemm_tall) by the rule for tiles of 128 x 256: for K from 16448 to 27648, where
         the library's default choice drops to 0.75 PFLOP/s (from 1.0 to 1.4 at shorter K), and tiles that are at most 0.94 of a
-        round on the chip, 0.72 of it real outputs. 2048 x 3584 x 18944 takes 256 us, the library 358; over 149 random products of
-        this range 0.55 to 1.07 of the library's time, 0.78 in the geometric mean. Fewer tiles leave units idle; beyond 0.94 the
+        round on the chip, 0.72 of it real outputs. 2048 x 3584 x 18944 takes 225 us (in tiles of 128 x 224), the library 355; over 149 random products of
+        this range 0.55 to 1.07 of the library's time, 0.78 in the geometric mean, with an earlier kernel that took 256 us there. Fewer tiles leave units idle; beyond 0.94 the
         library's choice is another one for some widths (3072 x 18944: the tiles take 1.09 of its time), and beyond K 27648 for others (8192 x
         29568 1.24 of it). Up to K 16384 the tiles lost on nearly every width (4096 x 14336 at 1019 rows 197 us, 132). Only where a part
         allows it: the library adds some tiles of such a product in two halves, so 6 results in 10,000 differ in their last bit,
@@ -264,7 +264,8 @@ class Linear:
         bf16 operands (the head of the Qwen2.5-7B shape at 64 rows: 217 us)."""
         w = self.weight
         if self._tall(rows, x, out, out_dtype):
-            ops.gemm_tall(out, x, w, bias, rows, bm=128)
+            bm, bn = ops.gemm_tall_tile(rows, *w.shape)
+            ops.gemm_tall(out, x, w, bias, rows, bm=bm, bn=bn)
             return out
         tile = self._few_tiles(rows, x, out, out_dtype)
         if tile:

@@ -48,6 +48,33 @@ def test_products_in_tiles(bm, M, N, K):
         assert (out[M] == 7).all()
 
 
+TILES = [(256, 256), (256, 224), (256, 192), (256, 160), (128, 288), (128, 256), (128, 224), (128, 160)]
+
+
+# one stage and fewer stages than the rings hold; a single output, edges of tiles, rows of results that begin at no 16-byte boundary,
+# more tiles than the chip has units (a workgroup goes from tile to tile), rows and columns of tiles that do not divide by the band
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (255, 156, 64), (257, 452, 128), (130, 300, 320), (1300, 4600, 64), (2500, 6404, 192)])
+@pytest.mark.parametrize("bm,bn", TILES)
+def test_every_tile(bm, bn, M, N, K):
+    x, w, b = rnd(M, K, seed=1).cuda(), rnd(N, K, seed=2).cuda(), rnd(N, seed=3).cuda()
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    out = torch.full((M + 1, N), 7.0, dtype=BF16, device="cuda")
+    for bias in (None, b):
+        ops.gemm_tall(out, x, w, bias, M, bm=bm, bn=bn)
+        plus = 0 if bias is None else bias.double()
+        near(out[:M], (want + plus).cpu(), (size + abs(plus)).cpu(), True)
+        assert (out[M] == 7).all()
+    act = (1.0, 0.0, 0.0, 0.0)
+    gated = torch.full((M + 1, N // 2), 7.0, dtype=BF16, device="cuda")
+    ops.gemm_tall(gated, x, w, None, M, bm=bm, bn=bn, act=act)
+    ops.gemm_tall(out, x, w, None, M, bm=bm, bn=bn)
+    two = torch.empty(M, N // 2, dtype=BF16, device="cuda")
+    ops.silu_mul(two, out, M, True)            # the activation of the rounded products, by the kernel that reads them from memory
+    # (the same function of the same bf16 gates and ups: one rounding apart at most)
+    assert ((gated[:M].double() - two.double()).abs() <= 2 ** -8 * two.double().abs()).all()
+    assert (gated[M] == 7).all()
+
+
 @pytest.mark.parametrize("bm", [128, 256])
 @pytest.mark.parametrize("rows,real,identity,top", [(1, 3, 0, 1), (130, 5, 1, 2), (300, 16, 2, 4), (513, 1, 0, 1), (700, 40, 0, 8)])
 def test_experts_over_the_rows_that_chose_them(bm, rows, real, identity, top):

@@ -137,3 +137,11 @@ def test_which_routed_steps_run_expert_by_expert(sizes, tiles):
     """At 256 units: where the estimate of four launches over chosen rows is below 0.8 of the products over all experts."""
     part = experts(**sizes)
     assert {rows: part._many_rows(rows, empty(rows, sizes["hidden"]), CTX) for rows in tiles} == tiles
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (2048, 3584, 18944, (128, 224)), (12001, 3584, 18944, (256, 224)),        # 256 tiles, 752: one round, three of the shorter ones
+    (2048, 37888, 3584, (256, 256)), (203, 37888, 3584, (256, 160)), (100, 37888, 3584, (128, 160)),
+    (2048, 4608, 3584, (128, 288)), (1, 4, 64, (128, 160))])
+def test_which_tile_a_product_of_many_rows_takes(M, N, K, tile):
+    assert ops.gemm_tall_tile(M, N, K) == tile
