@@ -15,7 +15,7 @@ registers:
   bfloat16, M > 64         -> the library matrix product (the reference calls its BLAS
                               library for every product: kernels/matmul_cublas.cu:240-277), or
                               the tiles of kernels.ops.gemm_tall or gemm_few_tiles where they are faster
-                              (_tall, tall_gated, _few_tiles)
+                              (_tall, _long, tall_gated, gated_tile, _few_tiles)
   fp32 results (logits)    -> the MFMA kernels up to 64 rows, above that the library,
                               which writes fp32 from bf16 operands
 
@@ -69,7 +69,7 @@ class Linear:
         self.weight = weight
         self.bias = bias
         self.out_features, self.in_features = weight.shape
-        self.one_round_tiles = False        # set by a part: _tall's products may run in tiles of this library's own
+        self.one_round_tiles = False        # set by a part: _tall's, _long's and gated_tile's products may run in tiles of this library's own
         self._plans: dict[bool, tuple[int, int]] = {}
         self._chosen: dict[tuple, routes.Route] = {}     # (rows, activations, fast) -> route, for one version of the table
         self._chosen_version = -1
@@ -241,6 +241,25 @@ class Linear:
             return False
         return self._rounds(rows, 128) <= 0.94 and rows * N >= 0.72 * 128 * 256 * ops.compute_units()
 
+    def _tile_fill(self, rows: int) -> tuple[float, float]:
+        """Of the tile gemm_tall_tile chooses: the share of its rounds of the chip that has tiles, and that has real outputs."""
+        N, K = self.weight.shape
+        bm, bn = ops.gemm_tall_tile(rows, N, K)
+        tiles, cus = -(-rows // bm) * -(-N // bn), ops.compute_units()
+        places = -(-tiles // cus) * cus
+        return tiles / places, rows * N / (places * bm * bn)
+
+    def _long(self, rows: int, x, out, out_dtype) -> bool:
+        """Whether a product of long K runs in tiles of this library's own whatever their number: for K from 16448 to 27648 again, where
+        the tiles of gemm_tall_tile's choice leave at most 0.3 of their rounds without real outputs. Over 53 products of 70 to
+        12001 rows and 320 to 20864 columns 0.55 to 1.10 of the library's time, 0.79 in the geometric mean, three above 1.03 (12001 x 3584 x
+        18944 1144 us, the library 1528); with 0.4 to 0.6 of the rounds real up to 1.27. At K up to 16384 the library's choice is as often
+        as not the faster one (0.57 to 1.24 of its time over 300 products of whole rounds, 0.98 in the geometric mean)."""
+        N, K = self.weight.shape
+        return not library_tuning.enabled() and self.one_round_tiles and out_dtype == BF16 and 16384 < K <= 27648 and K % 64 == 0 \
+            and N % 4 == 0 and x.is_contiguous() and out.is_contiguous() and self.weight.is_contiguous() and ops.tiles_read(x, self.weight, out) \
+            and self._tile_fill(rows)[1] >= 0.7
+
     def _few_tiles(self, rows: int, x, out, out_dtype) -> int:
         """The tile (kernels.ops.few_tiles_tile) of a product whose tiles are one round of the chip, 0 where the library runs it: tiles of
         at most 208 rows and columns together, for half of the chip's units or more, of K up to 5120; of K up to 1024
@@ -263,7 +282,7 @@ class Linear:
         """More than 64 rows: the library's product, or tiles of this one's own; it also writes fp32 results (the logits) from
         bf16 operands (the head of the Qwen2.5-7B shape at 64 rows: 217 us)."""
         w = self.weight
-        if self._tall(rows, x, out, out_dtype):
+        if self._tall(rows, x, out, out_dtype) or self._long(rows, x, out, out_dtype):
             bm, bn = ops.gemm_tall_tile(rows, *w.shape)
             ops.gemm_tall(out, x, w, bias, rows, bm=bm, bn=bn)
             return out
@@ -376,6 +395,18 @@ class Linear:
         if self._rounds(rows, 128) <= 1:
             return 128 if self._rounds(rows, 128) >= 0.6 else 0
         return 256 if self._rounds(rows, 256) <= 1 and rows * N >= 0.7 * 256 * 256 * ops.compute_units() else 0
+
+    def gated_tile(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
+        """The tile (ops.gemm_tall's bm, bn) where the gated product of this many bf16 rows with K above 1024 runs as one kernel,
+        None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
+        0.8 of their rounds or more. Over 229 products of 70 to 12001 rows, 256 to 55296 columns and K up to 27648 it took 0.55 to
+        1.10 of the time of the two, 0.91 in the geometric mean, 15 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
+        beside 84, 100 rows 57 beside 69); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _tall."""
+        N, K = self.weight.shape
+        if not (self.one_round_tiles and K > 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0
+                and N % 8 == 0 and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) or library_tuning.enabled():
+            return None
+        return ops.gemm_tall_tile(rows, N, K) if self._tile_fill(rows)[0] >= 0.8 else None
 
     def gated_pieces(self, rows: int) -> bool:
         """Whether gated_silu can write its result piece-major at this many rows."""

@@ -75,16 +75,17 @@ class GatedMLP(FeedForward):
         self.gate_up = Linear(w.contiguous())
         del g, u, w
         self.down = Linear(tensors[n["down"]])
-        self.down.one_round_tiles = True
+        self.gate_up.one_round_tiles = self.down.one_round_tiles = True
 
     def _gate(self, h, x, rows: int, ctx: StepContext) -> None:
         """h[rows, inter] = act(gate x, up x) of many rows: one kernel where the product takes the activation along."""
         if isinstance(x, NormedRows) and self.gate_up.own_tiles(rows, ctx, x.scaled.dtype):
             x = x.tensor(ctx)
         bm = self.gate_up.tall_gated(rows, ctx, x)
-        if bm:
+        tile = (bm, 256) if bm else self.gate_up.gated_tile(rows, ctx, x)
+        if tile:
             a = self.act
-            ops.gemm_tall(h, x, self.gate_up.weight, None, rows, bm=bm,
+            ops.gemm_tall(h, x, self.gate_up.weight, None, rows, bm=tile[0], bn=tile[1],
                           act=(a.get("alpha", 1.0), a.get("limit", 0.0), a.get("up_shift", 0.0), a.get("cubic", 0.0)))
             return
         gu = self.gate_up(x, rows, ctx)

@@ -141,7 +141,7 @@ class RoutedExperts(FeedForward):
         if self.shared is not None and not self.shared_cols:
             self.shared.bind(tensors)
             if isinstance(self.shared, GatedMLP):
-                self.shared.down.one_round_tiles = False      # (the router may read rows no norm has evened out)
+                self.shared.gate_up.one_round_tiles = self.shared.down.one_round_tiles = False      # (the router may read rows no norm has evened out)
         if self._shared_gate:
             self.shared_gate = tensors[self._shared_gate].reshape(-1).contiguous()
 

@@ -145,3 +145,29 @@ def test_which_routed_steps_run_expert_by_expert(sizes, tiles):
     (2048, 4608, 3584, (128, 288)), (1, 4, 64, (128, 160))])
 def test_which_tile_a_product_of_many_rows_takes(M, N, K, tile):
     assert ops.gemm_tall_tile(M, N, K) == tile
+
+
+@pytest.mark.parametrize("N,K,tiles", [
+    (37888, 3584, {70: (128, 160), 203: (256, 160), 300: (128, 224), 2048: (256, 256), 12001: (256, 256)}),
+    (14336, 4096, {175: None, 512: (128, 224)}),        # 0.70 of a round; a whole one
+    (9728, 896, {2048: None}), (37888, 3600, {2048: None}), (37884, 3584, {2048: None})])      # short K (tall_gated's), no multiples
+def test_which_gated_products_of_longer_k_run_as_one_kernel(N, K, tiles):
+    """At 256 units: where the tiles are 0.8 of their rounds or more."""
+    lin = Linear(empty(N, K))
+    assert not any(lin.gated_tile(r, CTX, empty(r, K)) for r in tiles)      # no part has allowed it
+    lin.one_round_tiles = True
+    assert {r: lin.gated_tile(r, CTX, empty(r, K)) for r in tiles} == tiles
+    with route_before_the_library(lambda c: c.N == N):
+        assert not any(lin.gated_tile(r, CTX, empty(r, K)) for r in tiles)
+
+
+@pytest.mark.parametrize("N,K,rows", [(3584, 18944, {768: False, 900: False, 1300: True, 3001: True, 12001: True}),
+                                      (5120, 27648, {900: True, 8192: True}), (4096, 14336, {10000: False}), (3584, 29568, {12001: False}),
+                                      (3584, 18912, {12001: False}), (3586, 18944, {12001: False})])
+def test_which_products_of_long_k_run_in_tiles_of_many_rounds(N, K, rows):
+    """At 256 units: K from 16448 to 27648, 0.7 of the rounds real outputs."""
+    lin = Linear(empty(N, K))
+    assert not any(lin._long(r, empty(r, K), empty(r, N), BF16) for r in rows)
+    lin.one_round_tiles = True
+    assert {r: lin._long(r, empty(r, K), empty(r, N), BF16) for r in rows} == rows
+    assert not any(lin._long(r, empty(r, K), empty(r, N, dtype=torch.float32), torch.float32) for r in rows)

@@ -162,3 +162,20 @@ def test_experts_over_the_rows_that_chose_them(monkeypatch, form, turns):
         both = torch.empty(rows, D, dtype=BF16, device="cuda")
         ops.gated_add(both, routed, part.shared.forward(x, context(rows)), x, part.shared_gate, rows)
         assert torch.equal(part.forward(x, context(rows)), both)
+
+
+@pytest.mark.parametrize("act,params,fn,shift,limit,consts", [
+    ("silu", {}, *SILU, (1.0, 0.0, 0.0, 0.0)),
+    ("clamped_swiglu", {"limit": 1.5}, lambda g: g * torch.sigmoid(1.702 * g), 1.0, 1.5, (1.702, 1.5, 1.0, 0.0))])
+@pytest.mark.parametrize("inter,rows,tile", [(20000, 70, (128, 160)), (12200, 250, (128, 224)), (2872, 1900, (256, 192))])
+def test_gated_products_of_longer_k_as_one_kernel(monkeypatch, act, params, fn, shift, limit, consts, inter, rows, tile):
+    """K of 1088, above the rule for short ones; columns and rows that end inside a tile."""
+    hidden = 1088
+    part = bound_part("gated_mlp", {"hidden_size": hidden, "intermediate_size": inter, "activation": act, **params}, hidden ** -0.5)
+    x, calls = rnd(rows, hidden, seed=92), spied(monkeypatch, "gemm_tall")
+    part.forward(x, context(rows))
+    assert [(c.args[4], (c.kw["bm"], c.kw["bn"])) for c in calls] == [(rows, tile)]
+    assert calls[0].kw["act"] == pytest.approx(consts)
+    w = part.gate_up.weight
+    want, off = gated(x, w[0::2], w[1::2], fn, shift, limit)
+    assert ((calls[0].args[0][:rows].double() - want).abs() <= off + 2 ** -8 * (want.abs() + off)).all()
