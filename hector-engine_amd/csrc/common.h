@@ -195,6 +195,21 @@ __device__ __forceinline__ float he_gated_act(float g, float u, const GatedAct& 
   return g / (1.f + expf(-fmaf(a.cubic, g * g, a.alpha) * g)) * (u + a.shift);
 }
 
+// An activation of one input. kind 0: relu(x)^2; 1: gelu with tanh, 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))); 2: silu; 3: relu
+#define HE_ACT_RELU2 0
+#define HE_ACT_GELU_TANH 1
+#define HE_ACT_SILU 2
+#define HE_ACT_RELU 3
+__device__ __forceinline__ float he_unary(float x, int kind) {
+  if (kind == HE_ACT_RELU2) {
+    const float r = fmaxf(x, 0.f);
+    return r * r;
+  }
+  if (kind == HE_ACT_GELU_TANH) return 0.5f * x * (1.f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
+  if (kind == HE_ACT_SILU) return x / (1.f + expf(-x));
+  return fmaxf(x, 0.f);
+}
+
 // tanh for a result that is rounded to bfloat16: (1 - t) / (1 + t) with t = exp(-2 |z|), the sign put back
 // (relative error below 1e-4 from |z| = 1e-3 on, far inside a bfloat16's half ulp of 2e-3).
 __device__ __forceinline__ float he_tanh_bf16(float z) {

@@ -317,21 +317,6 @@ extern "C" int he_silu_mul(void* out, const void* gate_up, int rows, int I, int 
 }
 
 // ---- activations and gates of one input -----------------------------------------------------------
-// kind 0: relu(x)^2; 1: gelu with tanh, 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))); 2: silu; 3: relu
-#define HE_ACT_RELU2 0
-#define HE_ACT_GELU_TANH 1
-#define HE_ACT_SILU 2
-#define HE_ACT_RELU 3
-__device__ __forceinline__ float he_unary(float x, int kind) {
-  if (kind == HE_ACT_RELU2) {
-    const float r = fmaxf(x, 0.f);
-    return r * r;
-  }
-  if (kind == HE_ACT_GELU_TANH) return 0.5f * x * (1.f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
-  if (kind == HE_ACT_SILU) return x / (1.f + expf(-x));
-  return fmaxf(x, 0.f);
-}
-
 // out[i] = act(x[i]), in place when out == x
 template <typename T>
 __global__ void unary_act_kernel(T* out, const T* x, int64_t n, int kind) {

@@ -116,7 +116,9 @@ extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
 
 // R, U, NW <= 0 choose the heuristic tiling (NW wavefronts = K slices per workgroup).
 // scale_partials: sums of squares of the input rows (the rows are then scaled before
-// bias or gate); resid: the residual epilogue (C is not written; gain, xg, sq_out needed).
+// bias or gate); resid: the residual epilogue (C is not written; gain, xg, sq_out needed). unary: an activation of one input
+// (he_unary's kinds) of the bf16 results, -1: none: a feed-forward without a gate writes its activations at once (a launch of its
+// own for 18944 of them took 4.7 us beside the product's 26).
 extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W,
                                              const void* bias, int M, int N, int K, int out_dtype,
                                              int bias_dtype, int gated, int R, int U, int NW,
@@ -126,7 +128,7 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
                                              int sq_count, int x_pieces, int out_pieces,
                                              float act_alpha, float act_limit, float act_shift, float act_cubic,
                                              float resid_scale, const void* dyt_bias,
-                                             const void* dyt_alpha, void* stream) {
+                                             const void* dyt_alpha, int unary, void* stream) {
   HE_REQUIRE((dyt_alpha == nullptr) == (dyt_bias == nullptr), "he_gemm_blocksplit_bf16: Dynamic Tanh needs alpha and bias");
   HE_REQUIRE(M > 0 && M <= HE_BLOCKSPLIT_MAX_M, "he_gemm_blocksplit_bf16: M=%d outside [1, %d]", M,
              HE_BLOCKSPLIT_MAX_M);
@@ -143,6 +145,8 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
              "he_gemm_blocksplit_bf16: piece-major activations are for up to 16 rows, not %d", M);
   HE_REQUIRE(!out_pieces || ((resid != nullptr || out_dtype == HE_BF16) && ((gated ? N / 2 : N) & 7) == 0),
              "he_gemm_blocksplit_bf16: a piece-major output is bf16 and a multiple of 8 wide");
+  HE_REQUIRE(unary < 0 || (unary <= HE_ACT_RELU && !gated && resid == nullptr && out_dtype == HE_BF16),
+             "he_gemm_blocksplit_bf16: an activation of one input goes with plain bf16 results");
   const BlockSplitPlan p = blocksplit_plan(M, N, K, gated, R, U, NW);
   HE_REQUIRE(p.NW >= 1 && p.NW <= 16, "he_gemm_blocksplit_bf16: %d wavefronts outside [1, 16]",
              p.NW);
@@ -173,6 +177,7 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
   fu.act.limit = act_limit > 0.f ? act_limit : INFINITY;
   fu.act.shift = act_shift;
   fu.act.cubic = act_cubic;
+  fu.unary = unary;
   fu.resid_scale = resid_scale;
   fu.dyt_bias = dyt_bias;
   fu.dyt_alpha = dyt_alpha;
@@ -191,5 +196,5 @@ extern "C" int he_gemm_blocksplit_bf16(void* C, const void* A, const void* W, co
                                        int gated, int R, int U, int NW, void* stream) {
   return he_gemm_blocksplit_fused_bf16(C, A, W, bias, M, N, K, out_dtype, bias_dtype, gated, R, U,
                                        NW, nullptr, 0, 0.f, nullptr, nullptr, HE_F32, nullptr,
-                                       nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, stream);
+                                       nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, -1, stream);
 }

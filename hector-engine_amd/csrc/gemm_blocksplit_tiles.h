@@ -154,6 +154,7 @@ struct BsFusion {
   int out_pieces;                // the bf16 output (C, or xg) is written piece-major
   int act_clamped;               // the gated epilogue runs he_gated_act with `act`, not SiLU(gate) * up
   GatedAct act;
+  int unary;                     // >= 0: the bf16 output is he_unary of the result rounded to bf16
   float resid_scale;             // the residual epilogue adds resid_scale * result
   const void* dyt_bias;          // with dyt_alpha: xg = tanh(alpha * resid) * gain + dyt_bias (Dynamic Tanh; both of
   const void* dyt_alpha;         // gain's dtype; alpha one stored number), and sq_out = 0: nothing is owed
@@ -378,6 +379,9 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, R, U)) void gemm_blocksplit_k
       if (bias != nullptr)
         for (int i = 0; i < valid; ++i) v[i] += load_param(bias, n + i, bias_dtype);
       if (!to_resid) {
+        if (fu.unary >= 0)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = he_unary(bf16_bits_to_float(float_to_bf16_bits(v[i])), fu.unary);
         if (valid > 0) {
           if (fu.out_pieces)
             bs_store_pieces(reinterpret_cast<uint16_t*>(C), M, m, n, v, 4, valid);

@@ -15,7 +15,7 @@ static int gt_launch(GtCase c, int tile, int mtiles, int epi, hipStream_t s) {
 
 extern "C" int he_gemm_tall_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
                                  int64_t ldx, int64_t ldw, int64_t ldo, int epilogue, int tile, float alpha, float limit,
-                                 float up_shift, float cubic, void* stream) {
+                                 float up_shift, float cubic, int unary, void* stream) {
   HE_REQUIRE(M >= 0 && N > 0 && K > 0 && N % 4 == 0 && K % GT_BK == 0, "he_gemm_tall: bad sizes M=%d N=%d K=%d", M, N, K);
   HE_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && ldo % (epilogue == GT_GATED ? 2 : 4) == 0 &&
                  ldo >= (epilogue == GT_GATED ? N / 2 : N),
@@ -27,10 +27,12 @@ extern "C" int he_gemm_tall_bf16(void* out, const void* x, const void* w, const 
   GT_TILES(GT_KNOWN)
   HE_REQUIRE(epilogue >= GT_BF16 && epilogue <= GT_F32 && known && (epilogue != GT_F32 || bn == 256), "he_gemm_tall: unknown form");
   HE_REQUIRE(bias == nullptr || epilogue == GT_BF16, "he_gemm_tall: a bias goes with plain bf16 results");
+  HE_REQUIRE(unary < 0 || (epilogue == GT_BF16 && (unary == HE_ACT_RELU2 || unary == HE_ACT_RELU)),
+             "he_gemm_tall: no such activation of one input, or not of plain bf16 results");
   HE_REQUIRE((int64_t)288 * ldx * 2 < (1ll << 32) && (int64_t)288 * ldw * 2 < (1ll << 32), "he_gemm_tall: rows too long");
   if (M == 0) return 0;
   const GtCase c = {(const uint16_t*)x, (const uint16_t*)w, out, bias, bias_dtype, M, N, K, ldx, ldw, ldo, 0, nullptr, nullptr,
-                    nullptr, nullptr, 1, 0, {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic}, false};
+                    nullptr, nullptr, 1, 0, {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic}, unary, false};
   return gt_launch(c, tile, (M + bm - 1) / bm, epilogue, (hipStream_t)stream);
 }
 
@@ -184,9 +186,9 @@ extern "C" int he_routed_groups(void* out, void* lists_i32, void* h_bf16, void* 
   if (rc) return rc;
   const GatedAct act = {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic};
   const GtCase up = {(const uint16_t*)x, (const uint16_t*)gate_up, h_bf16, nullptr, 0, slots, 2 * I, D, D, D, spread ? (int64_t)real * I : I, (int64_t)2 * I * D,
-               tile_begin, rows_of, scale, nullptr, real, spread, act, false};
+               tile_begin, rows_of, scale, nullptr, real, spread, act, -1, false};
   const GtCase dn = {(const uint16_t*)h_bf16, (const uint16_t*)down, partial_f32, nullptr, 0, slots, D, I, I, ldw, D, I, tile_begin,
-               nullptr, nullptr, choice_of, real, 0, act, false};
+               nullptr, nullptr, choice_of, real, 0, act, -1, false};
   rc = gt_launch(up, bm << 16 | 256, mtiles, GT_GATED, s);
   if (rc || spread) return rc;
   rc = gt_launch(dn, bm << 16 | 256, mtiles, GT_F32, s);

@@ -52,6 +52,7 @@ struct GtCase {
   int groups;
   int spread;                 // GT_GATED: the result goes to row rows_of[slot], columns from group * N / 2 on
   GatedAct act;
+  int unary;                  // GT_BF16: HE_ACT_RELU2 or HE_ACT_RELU of the result rounded to bf16; -1: none
   bool wide;                  // every row of out begins at a 16-byte boundary
 };
 
@@ -295,7 +296,16 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
         if (c.bias)
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] += load_param(c.bias, n + e, c.bias_dtype);
-        return make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        uint2 p = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        if (c.unary >= 0) {
+          auto relu = [&](uint32_t bits) {
+            const float r = fmaxf(__uint_as_float(bits), 0.f);
+            return c.unary == HE_ACT_RELU2 ? r * r : r;
+          };
+          p.x = pack2_bf16(relu(p.x << 16), relu(p.x & 0xffff0000u));
+          p.y = pack2_bf16(relu(p.y << 16), relu(p.y & 0xffff0000u));
+        }
+        return p;
       };
 #pragma unroll
       for (int j = 0; j < WI; j += j < W16 ? 4 : j < W8 ? 2 : 1) {

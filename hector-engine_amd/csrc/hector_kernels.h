@@ -92,7 +92,7 @@ int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W, const v
                                   float scale_eps, void* resid, const void* gain, int gain_dtype,
                                   void* xg, void* sq_out, int sq_count, int x_pieces, int out_pieces,
                                   float act_alpha, float act_limit, float act_shift, float act_cubic, float resid_scale,
-                                  const void* dyt_bias, const void* dyt_alpha, void* stream);
+                                  const void* dyt_bias, const void* dyt_alpha, int unary, void* stream);
 // resid_scale: the residual epilogue adds resid_scale * result. dyt_alpha, dyt_bias (both null, or both
 // of gain's dtype; alpha one stored number): the norm that follows is Dynamic Tanh, and the epilogue
 // leaves it finished, xg = tanh(alpha * resid) * gain + dyt_bias, with sq_out = 0 (a reader that
@@ -283,11 +283,11 @@ int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32, const voi
 // bias (or null): [E], added to the logits before anything else; x_pieces: the bf16 rows x lie piece-major for exactly `rows` rows.
 // bf16 products of many rows: out[m][n] = x[m] . w[n] (+ bias). epilogue 0: bf16 results; 1: the weight's rows alternate gate and
 // up, out[m][n / 2] = the gated activation (constants as he_gated_act); 2: fp32 results. tile: BM << 16 | BN, one of those of
-// gemm_tall_tiles.h (fp32 results: BN 256), as he_gemm_tall_tile chooses.
+// gemm_tall_tiles.h (fp32 results: BN 256), as he_gemm_tall_tile chooses. unary: relu squared (0) or relu (3) of the bf16 results, -1: none.
 // K a multiple of 64, N of 4.
 int he_gemm_tall_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
                       int64_t ldx, int64_t ldw, int64_t ldo, int epilogue, int tile, float alpha, float limit, float up_shift,
-                      float cubic, void* stream);
+                      float cubic, int unary, void* stream);
 int he_gemm_tall_tile(int M, int N, int K);
 // gemm_few_tiles.hip: out bf16 [M][ldo] = x [M][ldx] w [N][ldw]^T (+ bias) in tiles of he_gemm_few_tiles_tile(M, N) (0: no tile makes the
 // product one round of the chip). K a multiple of 64, N of 4, operands 16-byte aligned.

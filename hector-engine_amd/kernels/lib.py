@@ -43,7 +43,7 @@ _SIGNATURES = {
     "he_gemm_blocksplit_fused_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_int,
                                       c_int, c_int, c_int, c_ptr, c_int, c_f32, c_ptr, c_ptr, c_int,
                                       c_ptr, c_ptr, c_int, c_int, c_int, c_f32, c_f32, c_f32, c_f32, c_f32, c_ptr, c_ptr,
-                                      c_ptr],
+                                      c_int, c_ptr],
     "he_scale_rows_bf16": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_f32, c_int, c_ptr],
     "he_splitk_reduce": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_ptr],
     "he_compute_units": [],
@@ -106,7 +106,7 @@ _SIGNATURES = {
     "he_gemm_few_tiles_tile": [c_int, c_int],
     "he_gemm_few_tiles_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_int, c_ptr],
     "he_gemm_tall_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_int, c_int,
-                          c_f32, c_f32, c_f32, c_f32, c_ptr],
+                          c_f32, c_f32, c_f32, c_f32, c_int, c_ptr],
     "he_gemm_tall_tile": [c_int, c_int, c_int],
     "he_group_rows_most_tiles": [c_int, c_int, c_int, c_int],
     "he_routed_groups_ints": [c_int, c_int, c_int, c_int],

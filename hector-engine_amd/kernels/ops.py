@@ -298,7 +298,7 @@ def _act4(act) -> tuple:
 @_op("gemm_blocksplit")
 def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0), *,
                     row_scale=None, residual=None, x_pieces: bool = False, out_pieces: bool = False,
-                    act=(1.0, 0.0, 0.0)) -> None:
+                    act=(1.0, 0.0, 0.0), unary: str | None = None) -> None:
     """bf16 MFMA product for M <= 32 with K cut inside the workgroup; one launch, complete
     result (bf16 or fp32), with bias or, gated, as [M, N/2] = silu(gate) * up for a weight
     that alternates gate and up rows (gate i at row 2i, its up at 2i + 1). plan = (R, U, NW),
@@ -314,7 +314,8 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
     (a vector [N] and a one-element tensor of gain's dtype) the rows left are those of a Dynamic Tanh in
     full, xg = tanh(alpha * resid) * gain + dyt_bias, and sq = 0 (with eps 1 nothing is owed).
     x_pieces: `a` is piece-major, shaped pieces_shape(M, K). out_pieces: the bf16 output (`out`,
-    or xg of the residual epilogue) is written piece-major, shaped pieces_shape(M, its width)."""
+    or xg of the residual epilogue) is written piece-major, shaped pieces_shape(M, its width).
+    unary: an activation (ACT_KINDS) of the bf16 results, as unary_act gives it."""
     N, K = w.shape
     NO = N // 2 if gated else N
     _need(a, "a", torch.bfloat16)
@@ -372,7 +373,7 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
         dtype_code(bias.dtype) if bias is not None else F32, int(gated),
         int(plan[0]), int(plan[1]), int(plan[2]), sp, sc, float(se), rp, gp, gdt, xp, qp, qc,
         int(x_pieces), int(out_pieces), *_act4(act), float(rscale),
-        _ptr(dyt_bias), _ptr(dyt_alpha), _stream()))
+        _ptr(dyt_bias), _ptr(dyt_alpha), -1 if unary is None else ACT_KINDS[unary], _stream()))
 
 
 def gemm_rows_plan(M: int, N: int, K: int) -> tuple[int, int]:
@@ -1216,10 +1217,11 @@ def tiles_read(*tensors) -> bool:
 
 
 @_op("gemm_tall")
-def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, bn: int = 256, act=None) -> None:
+def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, bn: int = 256, act=None,
+              unary: str | None = None) -> None:
     """out[M, N] = x[M, K] . w[N, K]^T (+ bias) for many bf16 rows (bf16 or fp32 results); with act, the constants (alpha,
     limit, up_shift, cubic) of a gated activation, w's rows alternate gate and up and out is [M, N / 2]. K a multiple
-    of 64, N of 4. bm, bn: the outputs of a tile (gemm_tall_tile)."""
+    of 64, N of 4. bm, bn: the outputs of a tile (gemm_tall_tile). unary: "relu2" or "relu" of the bf16 results, as unary_act gives it."""
     N, K = w.shape
     cols = N // 2 if act is not None else N
     _need(out, "out", None, (None, cols))
@@ -1233,7 +1235,8 @@ def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, bn: int = 256, act=None
     alpha, limit, up_shift, cubic = act or (1.0, 0.0, 0.0, 0.0)
     _lib.check(_lib.load().he_gemm_tall_bf16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias),
                                              dtype_code(bias.dtype) if bias is not None else F32, M, N, K, K, K, cols, epilogue,
-                                             bm << 16 | bn, float(alpha), float(limit), float(up_shift), float(cubic), _stream()))
+                                             bm << 16 | bn, float(alpha), float(limit), float(up_shift), float(cubic),
+                                             -1 if unary is None else ACT_KINDS[unary], _stream()))
 
 
 @functools.lru_cache(maxsize=4096)

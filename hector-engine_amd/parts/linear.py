@@ -396,17 +396,39 @@ class Linear:
             return 128 if self._rounds(rows, 128) >= 0.6 else 0
         return 256 if self._rounds(rows, 256) <= 1 and rows * N >= 0.7 * 256 * 256 * ops.compute_units() else 0
 
-    def gated_tile(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
-        """The tile (ops.gemm_tall's bm, bn) where the gated product of this many bf16 rows with K above 1024 runs as one kernel,
-        None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
-        0.8 of their rounds or more. Over 229 products of 70 to 12001 rows, 256 to 55296 columns and K up to 27648 it took 0.55 to
+    def _tile_with_activation(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
+        """The tile (ops.gemm_tall's bm, bn) where a product of this many bf16 rows with K above 1024 takes the activation of its results
+        along, None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
+        0.8 of their rounds or more. Over 229 gated products of 70 to 12001 rows, 256 to 55296 columns and K up to 27648 it took 0.55 to
         1.10 of the time of the two, 0.91 in the geometric mean, 15 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
         beside 84, 100 rows 57 beside 69); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _tall."""
         N, K = self.weight.shape
         if not (self.one_round_tiles and K > 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0
-                and N % 8 == 0 and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) or library_tuning.enabled():
+                and N % 8 == 0 and self.weight.is_contiguous() and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) \
+                or library_tuning.enabled():
             return None
         return ops.gemm_tall_tile(rows, N, K) if self._tile_fill(rows)[0] >= 0.8 else None
+
+    def gated_tile(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
+        """The tile where the gated product of this many rows runs as one kernel, None where it does not (K up to 1024: tall_gated)."""
+        return self._tile_with_activation(rows, ctx, x)
+
+    def activated(self, x, rows: int, ctx: StepContext, kind: str):
+        """unary_act(kind) of the product as one kernel, None where the caller runs the two: up to 16 rows for any kind, many rows
+        for the relu ones."""
+        act, a, scale, pieces = _operand(x)
+        if act != BF16 or not routes.routes_of("linear", (self.weight.dtype, act)):
+            return None
+        if 0 < rows <= ops.BLOCKSPLIT_PIECES_MAX_M and self.route(rows, ctx, act).run is Linear._run_mfma:
+            out = ctx.alloc((rows, self.weight.shape[0]), act)
+            ops.gemm_blocksplit(out, a, self.weight, self.bias, rows, row_scale=scale, x_pieces=pieces, unary=kind)
+            return out
+        tile = self._tile_with_activation(rows, ctx, x) if kind in ("relu2", "relu") else None
+        if tile is None:
+            return None
+        out = ctx.alloc((rows, self.weight.shape[0]), act)
+        ops.gemm_tall(out, x, self.weight, self.bias, rows, bm=tile[0], bn=tile[1], unary=kind)
+        return out
 
     def gated_pieces(self, rows: int) -> bool:
         """Whether gated_silu can write its result piece-major at this many rows."""

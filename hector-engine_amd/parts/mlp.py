@@ -154,20 +154,27 @@ class DenseMLP(FeedForward):
         n = self._names
         self.up = Linear(tensors[n["up"]])
         self.down = Linear(tensors[n["down"]])
+        # (polynorm stands beside routers that read rows no norm has evened out: the library's sums stay)
+        self.up.one_round_tiles = self.down.one_round_tiles = self.act != "polynorm"
         if self.act == "polynorm":
             self.numbers = tensors[n["act"]]
 
-    def _activate(self, h, rows: int) -> None:
+    def _activated(self, x, rows: int, ctx: StepContext):
+        """act(up x): one kernel where the product takes the activation along."""
+        h = self.up.activated(x, rows, ctx, self.act) if self.act != "polynorm" else None
+        if h is not None:
+            return h
+        h = self.up(x, rows, ctx)
         if self.act == "polynorm":
             ops.polynorm(h, h, self.numbers, rows, self.eps)
         else:
             ops.unary_act(h, h, rows, self.act)
+        return h
 
     def forward(self, x, ctx: StepContext):
         rows = ctx.rows
         if rows <= _ROW_CHUNK:
-            h = self.up(x, rows, ctx)
-            self._activate(h, rows)
+            h = self._activated(x, rows, ctx)
             return self.down(h, rows, ctx, sink=ctx.take_sink())
         if not isinstance(x, torch.Tensor):
             x = x.tensor(ctx)
@@ -175,8 +182,7 @@ class DenseMLP(FeedForward):
         for r0 in range(0, rows, _ROW_CHUNK):
             n = min(_ROW_CHUNK, rows - r0)
             turn = ctx.scratch.mark()
-            h = self.up(x[r0:r0 + n], n, ctx)
-            self._activate(h, n)
+            h = self._activated(x[r0:r0 + n], n, ctx)
             self.down(h, n, ctx, out=out[r0:r0 + n])
             ctx.scratch.release(turn)
         return out

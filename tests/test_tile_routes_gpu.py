@@ -179,3 +179,25 @@ def test_gated_products_of_longer_k_as_one_kernel(monkeypatch, act, params, fn, 
     w = part.gate_up.weight
     want, off = gated(x, w[0::2], w[1::2], fn, shift, limit)
     assert ((calls[0].args[0][:rows].double() - want).abs() <= off + 2 ** -8 * (want.abs() + off)).all()
+
+
+@pytest.mark.parametrize("rows,kernel", [(1, "gemm_blocksplit"), (5, "gemm_blocksplit"), (16, "gemm_blocksplit"), (17, None), (70, "gemm_tall"), (1900, "gemm_tall")])
+@pytest.mark.parametrize("kind", ["relu2", "relu", "gelu_tanh", "silu"])
+def test_activations_that_go_with_the_up_product(monkeypatch, rows, kernel, kind):
+    """The bits of the product and the activation one after the other; the relu ones also in steps of many rows."""
+    hidden, inter = 1088, 40000 if rows == 70 else 5744
+    part = bound_part("dense_mlp", {"hidden_size": hidden, "intermediate_size": inter, "activation": kind}, hidden ** -0.5)
+    x, w = rnd(rows, hidden, seed=93), part.up.weight
+    alone = torch.empty(rows, inter, dtype=BF16, device="cuda")
+    if rows <= 16:
+        ops.gemm_blocksplit(alone, x, w, None, rows)
+    elif kernel:
+        ops.gemm_tall(alone, x, w, None, rows)
+    if kernel:
+        ops.unary_act(alone, alone, rows, kind)
+    one, two = spied(monkeypatch, kernel or "gemm_tall"), spied(monkeypatch, "unary_act")
+    h = part._activated(x, rows, context(rows))
+    taken = kernel and (rows <= 16 or kind.startswith("relu"))
+    assert [c.kw.get("unary") for c in one] == ([kind] if taken or rows <= 16 else []) and len(two) == (0 if taken else 1)
+    if taken:
+        assert torch.equal(h[:rows], alone)
