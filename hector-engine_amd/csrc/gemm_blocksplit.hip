@@ -118,7 +118,8 @@ extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
 // scale_partials: sums of squares of the input rows (the rows are then scaled before
 // bias or gate); resid: the residual epilogue (C is not written; gain, xg, sq_out needed). unary: an activation of one input
 // (he_unary's kinds) of the bf16 results, -1: none: a feed-forward without a gate writes its activations at once (a launch of its
-// own for 18944 of them took 4.7 us beside the product's 26).
+// own for 18944 of them took 4.7 us beside the product's 26). used: groups of the weight that no row uses are not read (BsFusion):
+// the experts of a routed step that nobody chose.
 extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W,
                                              const void* bias, int M, int N, int K, int out_dtype,
                                              int bias_dtype, int gated, int R, int U, int NW,
@@ -128,7 +129,8 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
                                              int sq_count, int x_pieces, int out_pieces,
                                              float act_alpha, float act_limit, float act_shift, float act_cubic,
                                              float resid_scale, const void* dyt_bias,
-                                             const void* dyt_alpha, int unary, void* stream) {
+                                             const void* dyt_alpha, int unary, const void* used, int used_ld,
+                                             int used_count, int used_rows, int used_k, void* stream) {
   HE_REQUIRE((dyt_alpha == nullptr) == (dyt_bias == nullptr), "he_gemm_blocksplit_bf16: Dynamic Tanh needs alpha and bias");
   HE_REQUIRE(M > 0 && M <= HE_BLOCKSPLIT_MAX_M, "he_gemm_blocksplit_bf16: M=%d outside [1, %d]", M,
              HE_BLOCKSPLIT_MAX_M);
@@ -147,6 +149,10 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
              "he_gemm_blocksplit_bf16: a piece-major output is bf16 and a multiple of 8 wide");
   HE_REQUIRE(unary < 0 || (unary <= HE_ACT_RELU && !gated && resid == nullptr && out_dtype == HE_BF16),
              "he_gemm_blocksplit_bf16: an activation of one input goes with plain bf16 results");
+  HE_REQUIRE(used == nullptr || (M <= 16 && !gated && used_count >= 0 && used_ld >= used_count && used_rows >= 0 && used_k >= 0 &&
+                                 (used_rows > 0) != (used_k > 0) && (used_k == 0 || used_k >= 512) &&
+                                 (resid == nullptr || used_rows == 0) && (resid != nullptr || out_dtype == HE_BF16)),
+             "he_gemm_blocksplit_bf16: groups that are used: up to 16 rows, bf16 results, along the rows or in stretches of 512 k and more");
   const BlockSplitPlan p = blocksplit_plan(M, N, K, gated, R, U, NW);
   HE_REQUIRE(p.NW >= 1 && p.NW <= 16, "he_gemm_blocksplit_bf16: %d wavefronts outside [1, 16]",
              p.NW);
@@ -178,6 +184,8 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
   fu.act.shift = act_shift;
   fu.act.cubic = act_cubic;
   fu.unary = unary;
+  fu.used = (const float*)used;
+  fu.used_ld = used_ld, fu.used_count = used_count, fu.used_rows = used_rows, fu.used_k = used_k;
   fu.resid_scale = resid_scale;
   fu.dyt_bias = dyt_bias;
   fu.dyt_alpha = dyt_alpha;
@@ -186,7 +194,7 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
   static int (*const tiles[2][2])(HE_BS_DISPATCH_ARGS) = {
       {he_blocksplit_tiles_bf16, he_blocksplit_tiles_f32},
       {he_blocksplit_tiles_gated_bf16, he_blocksplit_tiles_gated_f32}};
-  rc = tiles[gated != 0][out_dtype != HE_BF16](p, C, A, W, bias, bias_dtype, M, N, K, fu, x_pieces != 0, s);
+  rc = (used ? he_blocksplit_tiles_used_bf16 : tiles[gated != 0][out_dtype != HE_BF16])(p, C, A, W, bias, bias_dtype, M, N, K, fu, x_pieces != 0, s);
   if (rc) return rc;
   return he_check_launch("he_gemm_blocksplit_bf16");
 }
@@ -196,5 +204,5 @@ extern "C" int he_gemm_blocksplit_bf16(void* C, const void* A, const void* W, co
                                        int gated, int R, int U, int NW, void* stream) {
   return he_gemm_blocksplit_fused_bf16(C, A, W, bias, M, N, K, out_dtype, bias_dtype, gated, R, U,
                                        NW, nullptr, 0, 0.f, nullptr, nullptr, HE_F32, nullptr,
-                                       nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, -1, stream);
+                                       nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, -1, nullptr, 0, 0, 0, 0, stream);
 }

@@ -298,7 +298,7 @@ def _act4(act) -> tuple:
 @_op("gemm_blocksplit")
 def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0), *,
                     row_scale=None, residual=None, x_pieces: bool = False, out_pieces: bool = False,
-                    act=(1.0, 0.0, 0.0), unary: str | None = None) -> None:
+                    act=(1.0, 0.0, 0.0), unary: str | None = None, used=None) -> None:
     """bf16 MFMA product for M <= 32 with K cut inside the workgroup; one launch, complete
     result (bf16 or fp32), with bias or, gated, as [M, N/2] = silu(gate) * up for a weight
     that alternates gate and up rows (gate i at row 2i, its up at 2i + 1). plan = (R, U, NW),
@@ -315,7 +315,10 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
     full, xg = tanh(alpha * resid) * gain + dyt_bias, and sq = 0 (with eps 1 nothing is owed).
     x_pieces: `a` is piece-major, shaped pieces_shape(M, K). out_pieces: the bf16 output (`out`,
     or xg of the residual epilogue) is written piece-major, shaped pieces_shape(M, its width).
-    unary: an activation (ACT_KINDS) of the bf16 results, as unary_act gives it."""
+    unary: an activation (ACT_KINDS) of the bf16 results, as unary_act gives it.
+    used = (weights fp32 [M, count + 1 or more], count, size, along_k): the weight's rows, or its k, come in groups of `size`, and of the
+    first `count` of them those are left out that no row has a weight for: their outputs are not written, or their products,
+    with zeros in `a`, not added (up to 16 rows)."""
     N, K = w.shape
     NO = N // 2 if gated else N
     _need(a, "a", torch.bfloat16)
@@ -366,6 +369,13 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
             raise ValueError("gemm_blocksplit: residual buffers do not match [M, N]")
         rp, gp, xp, qp = resid.data_ptr(), gain.data_ptr(), xg.data_ptr(), sq.data_ptr()
         gdt, qc = dtype_code(gain.dtype), sq.shape[1]
+    uargs = (None, 0, 0, 0, 0)
+    if used is not None:
+        weights, count, size, along_k = used
+        _need(weights, "used weights", torch.float32)
+        if weights.dim() != 2 or weights.shape[0] < M or weights.shape[1] < count or size <= 0:
+            raise ValueError("gemm_blocksplit: the weights that say what is used do not match the rows")
+        uargs = (weights.data_ptr(), weights.shape[1], count, 0 if along_k else size, size if along_k else 0)
     L = _lib.load()
     _lib.check(L.he_gemm_blocksplit_fused_bf16(
         _ptr(out), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K,
@@ -373,7 +383,7 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
         dtype_code(bias.dtype) if bias is not None else F32, int(gated),
         int(plan[0]), int(plan[1]), int(plan[2]), sp, sc, float(se), rp, gp, gdt, xp, qp, qc,
         int(x_pieces), int(out_pieces), *_act4(act), float(rscale),
-        _ptr(dyt_bias), _ptr(dyt_alpha), -1 if unary is None else ACT_KINDS[unary], _stream()))
+        _ptr(dyt_bias), _ptr(dyt_alpha), -1 if unary is None else ACT_KINDS[unary], *uargs, _stream()))
 
 
 def gemm_rows_plan(M: int, N: int, K: int) -> tuple[int, int]:

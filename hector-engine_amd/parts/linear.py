@@ -127,27 +127,31 @@ class Linear:
 
     def __call__(self, x, rows: int, ctx: StepContext, *, use_bias: bool = True,
                  out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None,
-                 sink: ResidualSink | None = None):
+                 sink: ResidualSink | None = None, used=None):
         """x: a tensor, NormedRows or PieceRows. With a sink the result may go into the
-        residual stream directly; the call then returns None."""
+        residual stream directly; the call then returns None. used: groups of the weight that may be left out
+        (ops.gemm_blocksplit), where the kernel can."""
         bias = self.bias if use_bias else None
         act = _operand(x)[0]
+        if used is not None and 0 < rows <= ops.BLOCKSPLIT_PIECES_MAX_M and self.route(rows, ctx, act).run is Linear._run_mfma \
+                and (out_dtype or act) == BF16:
+            return self._run_mfma(x, rows, ctx, bias, BF16, out, sink, used)
         return self.route(rows, ctx, act).run(self, x, rows, ctx, bias, out_dtype or act, out, sink)
 
     # ---- the routes' bodies ----
 
-    def _run_mfma(self, x, rows, ctx, bias, out_dtype, out, sink):
+    def _run_mfma(self, x, rows, ctx, bias, out_dtype, out, sink, used=None):
         """Up to 64 rows of bf16: the block-split kernel (up to 16 rows) or the rows kernel."""
         w = self.weight
         N = w.shape[0]
         act, a, scale, pieces = _operand(x)
         if sink is not None and out is None and out_dtype == act \
                 and sink.stream.rows == rows and sink.stream.resid.shape[-1] == N:
-            return self._into_residual(x, bias, rows, ctx, sink)
+            return self._into_residual(x, bias, rows, ctx, sink, used)
         if out is None:
             out = ctx.alloc((rows, N), out_dtype)
         if rows <= ops.BLOCKSPLIT_PIECES_MAX_M:
-            ops.gemm_blocksplit(out, a, w, bias, rows, row_scale=scale, x_pieces=pieces)
+            ops.gemm_blocksplit(out, a, w, bias, rows, row_scale=scale, x_pieces=pieces, used=used)
             return out
         splits = self._plan(rows)[1]
         if splits == 1:
@@ -312,7 +316,7 @@ class Linear:
                 torch.mm(x[:rows], w.t(), out=out[:rows])
         return out
 
-    def _into_residual(self, x, bias, rows, ctx, sink: ResidualSink):
+    def _into_residual(self, x, bias, rows, ctx, sink: ResidualSink, used=None):
         """The product added into the residual rows, and the rows of the norm that follows left as
         NormedRows: by the product's own epilogue, or, where it is cut along K, by the kernel
         that adds the slices."""
@@ -326,7 +330,7 @@ class Linear:
             sq = ctx.alloc((rows, ops.gemm_blocksplit_blocks(rows, N, K)), torch.float32)
             ops.gemm_blocksplit(None, a, self.weight, bias, rows, row_scale=scale,
                                 residual=(sink.stream.resid, gain, xg, sq, *more), x_pieces=pieces,
-                                out_pieces=out_pieces)
+                                out_pieces=out_pieces, used=used)
         else:
             groups, splits = self._plan(rows)
             if splits == 1:

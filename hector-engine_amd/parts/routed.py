@@ -260,10 +260,12 @@ class RoutedExperts(FeedForward):
         if bm:
             return self._by_expert(x, dense, ids, weights, rows, bm, act, ctx)
         if rows <= _ROW_CHUNK:
-            gu = self.gate_up(given, rows, ctx)
+            # up to 16 rows the products leave out the experts that nobody chose (routed_act gives exact zeros for those)
+            gu = self.gate_up(given, rows, ctx, used=(dense, real, 2 * I, False))
             h = ctx.alloc((rows, cols))
             ops.routed_act(h, gu, dense, x if self.identity else None, rows, real, I, shared=S, **act)
-            return self.down(h, rows, ctx, sink=ctx.take_sink() if may_sink else None)
+            return self.down(h, rows, ctx, sink=ctx.take_sink() if may_sink else None,
+                             used=(dense, real, I, True) if I >= 512 else None)
         out = ctx.alloc((rows, self.hidden))
         for r0 in range(0, rows, _ROW_CHUNK):
             n = min(_ROW_CHUNK, rows - r0)

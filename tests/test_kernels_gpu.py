@@ -1219,3 +1219,49 @@ def test_sample_frequencies(ops):
     p = torch.softmax(logits.double() / 0.8, 0)
     chi2 = (n * (freq - p) ** 2 / p).sum().item()
     assert chi2 < 30, chi2                        # 7 degrees of freedom; 30 is far in the tail
+
+
+# ------------------------------------------------------------------ groups of a weight that no row uses
+@pytest.mark.parametrize("M", [1, 4, 16])
+@pytest.mark.parametrize("pieces", [False, True])
+@pytest.mark.parametrize("N,count,size,extra", [(2048, 16, 2048, 0), (320, 5, 512, 192), (4608, 3, 640, 0), (96, 80, 512, 64), (1024, 6, 1000, 0), (70000, 2, 576, 0)])
+def test_blocksplit_leaves_out_groups_along_k(ops, M, pieces, N, count, size, extra):
+    """The bits of the whole product where x is zero along the groups nobody uses; their weights are not read (NaN here)."""
+    K = count * size + extra
+    g = torch.Generator().manual_seed(N + M)
+    used = torch.rand(M, count + 1, generator=g) * (torch.rand(M, count + 1, generator=g) < 1.5 / count)
+    used[0, count // 2], some = 0.5, None
+    some = (used[:, :count] != 0).any(0)
+    x, w = rnd(M, K, seed=3).to(torch.bfloat16), dev(rnd(N, K, seed=4, scale=0.05).to(torch.bfloat16))
+    for e in range(count):
+        x[:, e * size:(e + 1) * size] *= (used[:, e] != 0)[:, None]
+    given = dev(x.view(M, K // 8, 8).transpose(0, 1).contiguous() if pieces else x)
+    whole, out = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    ops.gemm_blocksplit(whole, given, w, None, M, x_pieces=pieces)
+    ops.gemm_blocksplit(out, given, w, None, M, x_pieces=pieces, used=(dev(used), count, size, True))
+    assert torch.equal(out, whole)
+    if size >= 1024:                                   # (no turn of a wavefront meets two groups there)
+        for e in range(count):
+            if not some[e]:
+                w[:, e * size:(e + 1) * size] = float("nan")
+        ops.gemm_blocksplit(out, given, w, None, M, x_pieces=pieces, used=(dev(used), count, size, True))
+        assert torch.equal(out, whole)
+
+
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("K,count,size,extra", [(2048, 16, 4096, 0), (520, 5, 300, 40), (64, 40, 16, 0), (1024, 3, 2, 6)])
+def test_blocksplit_leaves_out_groups_of_rows(ops, M, K, count, size, extra):
+    N = count * size + extra
+    g = torch.Generator().manual_seed(N + M)
+    used = torch.rand(M, count + 1, generator=g) * (torch.rand(M, count + 1, generator=g) < 1.5 / count)
+    some = (used[:, :count] != 0).any(0)
+    x, w = dev(rnd(M, K, seed=3).to(torch.bfloat16)), dev(rnd(N, K, seed=4, scale=0.05).to(torch.bfloat16))
+    whole, out = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    ops.gemm_blocksplit(whole, x, w, None, M)
+    ops.gemm_blocksplit(out, x, w, None, M, used=(dev(used), count, size, False))
+    for e in range(count):
+        cols = slice(e * size, (e + 1) * size)
+        assert torch.equal(out[:, cols], whole[:, cols]) if some[e] else ((out[:, cols] == whole[:, cols]) | (out[:, cols] == 7)).all()
+    assert torch.equal(out[:, count * size:], whole[:, count * size:])
+    if size >= 4096:
+        assert (out == 7).all(0).sum() >= 0.9 * size * int((~some).sum())      # (a workgroup at a border computes both sides)
