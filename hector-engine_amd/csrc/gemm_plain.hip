@@ -9,6 +9,7 @@
 // sums added one after the other in segment order, begun at zero; then the bias.
 // These kernels keep this order and give the same bits:
 //   mfma    fp32 operands, many rows: tiles of up to 128 x 128 outputs on the matrix cores;
+//   rounds  the same for aligned rows and K in 32s (gemm_plain_rounds.hip): tiles that are whole rounds of the chip;
 //   stream  fp32 operands, up to 64 rows, K in whole segments: matrix cores, a workgroup per 16 weight rows;
 //   tiles   bf16 operands: 64 x 64 outputs a workgroup, staged through LDS, every thread 4 x 4 outputs;
 //   rows    up to GP_ROWS_MAX_M rows that stream does not take (gp_streams), with a workspace: a thread owns one weight
@@ -586,7 +587,15 @@ static int launch_stream(float* C, const float* A, const float* W, const void* b
   return he_check_launch("he_gemm_plain");
 }
 
-// More rows: tiles on the matrix cores. Of the tile sizes the one whose fullest compute unit has the least to do
+// gemm_plain_rounds.hip
+int he_gemm_plain_rounds(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K, int64_t lda,
+                         int64_t ldw, int64_t ldc, hipStream_t s);
+float he_gemm_plain_rounds_estimate(int M, int N);
+
+// More rows: tiles on the matrix cores. Rows that begin at 16-byte boundaries with K in 32s go to gemm_plain_rounds.hip, whose tiles have
+// 128 rows, unless so many of those are padding that its estimate is above this kernel's time, 4.5 ps an output
+// and k of the fullest unit (130 rows of 37888 x 3584 602 us there, 470 here; over 12 weights and 65 to 3001 rows the kernel there takes
+// 0.56 to 1.06 of the time where it is taken, 0.85 in the geometric mean). Here, of the tile sizes the one whose fullest compute unit has the least to do
 // (a unit's workgroups share its matrix cores, so its time is the outputs dealt to it); the larger tile where
 // they tie, as it reads fewer operands an output.
 static int launch_mfma(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K,
@@ -597,6 +606,9 @@ static int launch_mfma(float* C, const float* A, const float* W, const void* bia
   int bm = 128, bn = 128;
   if (most(128, 64) < most(bm, bn)) bn = 64;
   if (most(64, 64) < most(bm, bn)) bm = 64, bn = 64;
+  // (lda, ldw: a lane's offsets into a tile's rows are 32-bit)
+  if (vec && K % 32 == 0 && lda < (1 << 22) && ldw < (1 << 22) && he_gemm_plain_rounds_estimate(M, N) <= 4.5e-6f * most(bm, bn))
+    return he_gemm_plain_rounds(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc, s);
   HE_REQUIRE(tiles(bm, bn) < (1 << 30), "he_gemm_plain: M=%d N=%d too large for one launch", M, N);
   const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
   const int grid = (int)((tiles(bm, bn) + HE_XCDS - 1) / HE_XCDS * HE_XCDS);

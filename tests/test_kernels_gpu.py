@@ -1265,3 +1265,24 @@ def test_blocksplit_leaves_out_groups_of_rows(ops, M, K, count, size, extra):
     assert torch.equal(out[:, count * size:], whole[:, count * size:])
     if size >= 4096:
         assert (out == 7).all(0).sum() >= 0.9 * size * int((~some).sum())      # (a workgroup at a border computes both sides)
+
+
+# ------------------------------------------------------------------ 32-bit products in whole rounds of the chip
+# (8 row tiles: every width from 16 to 144; columns that end inside a tile and inside four; several tiles a workgroup; a single stage, a
+# segment that ends early, more stages than are in flight; few rows, whose other kernel has tiles of 64)
+@pytest.mark.parametrize("M,N,K", [(1003, n, 160) for n in (512, 1024, 1533, 2048, 2560, 3070, 3584, 4096, 4607)] +
+                         [(65, 300, 32), (129, 9000, 96), (1003, 20001, 128), (2050, 5124, 384), (200, 4608, 3584), (66, 1, 256)])
+def test_plain_products_in_whole_rounds_give_the_bits_of_the_other_kernels(ops, M, N, K):
+    a, w, b = dev(rnd(M, K, seed=1)), dev(rnd(N, K, seed=2)), dev(rnd(N, seed=3))
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    apart = torch.empty(M * K + 1, device="cuda")[1:].view(M, K)       # rows that begin at no 16-byte boundary go through the other kernel
+    apart.copy_(a)
+    other = torch.empty(M, N, device="cuda")
+    for bias in (None, b):
+        ops.gemm_plain(out, a, w, bias, M)
+        ops.gemm_plain(other, apart, w, bias, M)
+        assert torch.equal(out[:M], other) and (out[M] == 7).all()
+    want = a.double() @ w.double().T + b.double()
+    size = a.double().abs() @ w.double().abs().T + b.double().abs()
+    # chains of 128 and the sums of segments: so many roundings of at most the sum of magnitudes
+    assert ((out[:M].double() - want).abs() <= (128 + K / 128 + 2) * 2 ** -24 * size).all()
