@@ -1,21 +1,17 @@
 // bf16 products of many rows (the kernel: gemm_tall_tiles.h), and the experts of a routed feed-forward over the rows that chose them.
 #include "gemm_tall_tiles.h"
 
-// fp32 results: the two tiles whose BM a group may have
-static int gt_run_f32(const GtCase& c, int bm, int mtiles, hipStream_t s) {
-  return bm == 256 ? gt_run<256, 256, 3, 2, GT_F32, false>(c, mtiles, s) : gt_run<128, 256, 4, 3, GT_F32, false>(c, mtiles, s);
-}
 static int gt_launch(GtCase c, int tile, int mtiles, int epi, hipStream_t s) {
   c.wide = ((uintptr_t)c.out & 15) == 0 && c.ldo * (epi == GT_F32 ? 4 : 2) % 16 == 0;
   const bool clamped = !(c.act.alpha == 1.f && !(c.act.limit < INFINITY) && c.act.shift == 0.f && c.act.cubic == 0.f);
-  if (epi == GT_F32) return gt_run_f32(c, tile >> 16, mtiles, s);
+  if (epi == GT_F32) return gt_run_f32(c, tile, mtiles, s);
   if (epi == GT_GATED) return clamped ? gt_run_clamped(c, tile, mtiles, s) : gt_run_gated(c, tile, mtiles, s);
   return gt_run_bf16(c, tile, mtiles, s);
 }
 
 extern "C" int he_gemm_tall_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
                                  int64_t ldx, int64_t ldw, int64_t ldo, int epilogue, int tile, float alpha, float limit,
-                                 float up_shift, float cubic, int unary, void* stream) {
+                                 float up_shift, float cubic, int unary, int slices, void* stream) {
   HE_REQUIRE(M >= 0 && N > 0 && K > 0 && N % 4 == 0 && K % GT_BK == 0, "he_gemm_tall: bad sizes M=%d N=%d K=%d", M, N, K);
   HE_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && ldo % (epilogue == GT_GATED ? 2 : 4) == 0 &&
                  ldo >= (epilogue == GT_GATED ? N / 2 : N),
@@ -25,14 +21,16 @@ extern "C" int he_gemm_tall_bf16(void* out, const void* x, const void* w, const 
   bool known = false;
 #define GT_KNOWN(BM, BN, NX, NW) known = known || (bm == BM && bn == BN);
   GT_TILES(GT_KNOWN)
-  HE_REQUIRE(epilogue >= GT_BF16 && epilogue <= GT_F32 && known && (epilogue != GT_F32 || bn == 256), "he_gemm_tall: unknown form");
+  HE_REQUIRE(epilogue >= GT_BF16 && epilogue <= GT_F32 && known, "he_gemm_tall: unknown form");
+  HE_REQUIRE(slices >= 1 && (slices == 1 || epilogue == GT_F32) && K % slices == 0 && K / slices % GT_BK == 0,
+             "he_gemm_tall: %d K slices: of fp32 results, each in whole stages", slices);
   HE_REQUIRE(bias == nullptr || epilogue == GT_BF16, "he_gemm_tall: a bias goes with plain bf16 results");
   HE_REQUIRE(unary < 0 || (epilogue == GT_BF16 && (unary == HE_ACT_RELU2 || unary == HE_ACT_RELU)),
              "he_gemm_tall: no such activation of one input, or not of plain bf16 results");
   HE_REQUIRE((int64_t)288 * ldx * 2 < (1ll << 32) && (int64_t)288 * ldw * 2 < (1ll << 32), "he_gemm_tall: rows too long");
   if (M == 0) return 0;
-  const GtCase c = {(const uint16_t*)x, (const uint16_t*)w, out, bias, bias_dtype, M, N, K, ldx, ldw, ldo, 0, nullptr, nullptr,
-                    nullptr, nullptr, 1, 0, {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic}, unary, false};
+  const GtCase c = {(const uint16_t*)x, (const uint16_t*)w, out, bias, bias_dtype, M, N, K / slices, ldx, ldw, ldo, 0, nullptr, nullptr,
+                    nullptr, nullptr, 1, 0, {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic}, slices, unary, false};
   return gt_launch(c, tile, (M + bm - 1) / bm, epilogue, (hipStream_t)stream);
 }
 
@@ -47,13 +45,14 @@ struct GtCost {
 };
 static const GtCost gt_costs[] = {{256, 256, 1.40f}, {256, 224, 1.27f}, {256, 192, 1.13f}, {256, 160, 0.97f},
                                   {128, 288, 0.94f}, {128, 256, 0.83f}, {128, 224, 0.76f}, {128, 160, 0.65f}};
-extern "C" int he_gemm_tall_tile(int M, int N, int K) {
+// slices: K slices, each a product of K / slices.
+extern "C" int he_gemm_tall_tile(int M, int N, int K, int slices) {
   int best = 0;
   float least = INFINITY;
   for (const GtCost& t : gt_costs) {
-    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * slices;
     const int64_t rounds = (tiles + he_cus() - 1) / he_cus();
-    const float us = rounds * (5.f + K / GT_BK * t.stage);
+    const float us = rounds * (5.f + K / slices / GT_BK * t.stage);
     if (us < least) least = us, best = t.bm << 16 | t.bn;
   }
   return best;
@@ -186,9 +185,9 @@ extern "C" int he_routed_groups(void* out, void* lists_i32, void* h_bf16, void* 
   if (rc) return rc;
   const GatedAct act = {alpha, limit > 0.f ? limit : INFINITY, up_shift, cubic};
   const GtCase up = {(const uint16_t*)x, (const uint16_t*)gate_up, h_bf16, nullptr, 0, slots, 2 * I, D, D, D, spread ? (int64_t)real * I : I, (int64_t)2 * I * D,
-               tile_begin, rows_of, scale, nullptr, real, spread, act, -1, false};
+               tile_begin, rows_of, scale, nullptr, real, spread, act, 1, -1, false};
   const GtCase dn = {(const uint16_t*)h_bf16, (const uint16_t*)down, partial_f32, nullptr, 0, slots, D, I, I, ldw, D, I, tile_begin,
-               nullptr, nullptr, choice_of, real, 0, act, -1, false};
+               nullptr, nullptr, choice_of, real, 0, act, 1, -1, false};
   rc = gt_launch(up, bm << 16 | 256, mtiles, GT_GATED, s);
   if (rc || spread) return rc;
   rc = gt_launch(dn, bm << 16 | 256, mtiles, GT_F32, s);

@@ -52,6 +52,7 @@ struct GtCase {
   int groups;
   int spread;                 // GT_GATED: the result goes to row rows_of[slot], columns from group * N / 2 on
   GatedAct act;
+  int slices;                 // GT_F32: K slices, each K long: of x and w from slice * K on, sums to out + slice * M * ldo
   int unary;                  // GT_BF16: HE_ACT_RELU2 or HE_ACT_RELU of the result rounded to bf16; -1: none
   bool wide;                  // every row of out begins at a 16-byte boundary
 };
@@ -80,7 +81,7 @@ __device__ __forceinline__ int gt_at(const int32_t* list, int i) {
 }
 
 struct GtTile {
-  int m0, n0, group;
+  int m0, n0, group, slice;
 };
 
 template <int BM, int BN, int NX, int NW, int EPI, bool CLAMPED>
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntiles = (c.N + BN - 1) / BN;
   const int mtiles = c.tile_begin ? gt_at(c.tile_begin, c.groups) : (c.M + BM - 1) / BM;
-  const int total = mtiles * ntiles, per_xcd = (total + HE_XCDS - 1) / HE_XCDS;
+  const int of_slice = mtiles * ntiles, total = of_slice * (EPI == GT_F32 ? c.slices : 1), per_xcd = (total + HE_XCDS - 1) / HE_XCDS;
   // this XCD's tiles: `count` of them from `begin` on; this workgroup's: every `stride`th of these
   const int begin = blockIdx.x % HE_XCDS * per_xcd, count = min(per_xcd, total - begin), stride = gridDim.x / HE_XCDS;
   const int mine = blockIdx.x / HE_XCDS;
@@ -103,8 +104,9 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
   const int stages = c.K / GT_BK;
 
   auto tile_at = [&](int i) {
-    const int tile = begin + i;
-    GtTile t = {0, 0, 0};
+    int tile = begin + i;
+    GtTile t = {0, 0, 0, 0};
+    if (EPI == GT_F32 && c.slices > 1) t.slice = tile / of_slice, tile -= t.slice * of_slice;
     int first = 0, deep = mtiles;
     if (c.tile_begin) {
       int lo = 0, hi = c.groups;                           // the last group that begins at or before this tile
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
   int xi = mine, wi = mine, xs = 0, ws = 0;                // tile and stage
   auto aim_x = [&]() {
     const GtTile t = tile_at(xi);
-    xbase = (const uint8_t*)(c.x + (c.rows_of ? 0 : (int64_t)t.m0 * c.ldx));
+    xbase = (const uint8_t*)(c.x + (c.rows_of ? 0 : (int64_t)t.m0 * c.ldx) + (int64_t)t.slice * c.K);
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
       const int r = 8 * (wave * XL + i) + (lane >> 3);
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
   };
   auto aim_w = [&]() {
     const GtTile t = tile_at(wi);
-    wbase = (const uint8_t*)(c.w + t.group * c.w_group + (int64_t)t.n0 * c.ldw);
+    wbase = (const uint8_t*)(c.w + t.group * c.w_group + (int64_t)t.n0 * c.ldw + (int64_t)t.slice * c.K);
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
       const int r = 8 * (wave * WL + i) + (lane >> 3), in_wave = r % TN;
@@ -336,7 +338,7 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
             *reinterpret_cast<uint32_t*>(p) = gated(acc[i][j]);
           }
         } else if (EPI == GT_F32) {
-          float* p = (float*)c.out + row + n;
+          float* p = (float*)c.out + (int64_t)t.slice * c.M * c.ldo + row + n;
           *reinterpret_cast<gt_f32x4*>(p) = acc[i][j];
           if (j < W8 && (wide || n + 4 < c.N)) *reinterpret_cast<gt_f32x4*>(p + 4) = acc[i][(j + 1) % WI];
         } else {
@@ -365,7 +367,7 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
 
 template <int BM, int BN, int NX, int NW, int EPI, bool CLAMPED>
 int gt_run(const GtCase& c, int mtiles, hipStream_t s) {
-  const int64_t tiles = (int64_t)mtiles * ((c.N + BN - 1) / BN);
+  const int64_t tiles = (int64_t)mtiles * ((c.N + BN - 1) / BN) * c.slices;
   HE_REQUIRE(tiles < (1 << 28), "he_gemm_tall: %d x %d outputs are too many for one launch", c.M, c.N);
   const int units = he_cus() / HE_XCDS * HE_XCDS, grid = (int)(tiles < units ? (tiles + HE_XCDS - 1) / HE_XCDS * HE_XCDS : units);
   gemm_tall_kernel<BM, BN, NX, NW, EPI, CLAMPED><<<grid, GT_THREADS, 0, s>>>(c);
@@ -375,3 +377,4 @@ int gt_run(const GtCase& c, int mtiles, hipStream_t s) {
 int gt_run_bf16(const GtCase& c, int tile, int mtiles, hipStream_t s);
 int gt_run_gated(const GtCase& c, int tile, int mtiles, hipStream_t s);
 int gt_run_clamped(const GtCase& c, int tile, int mtiles, hipStream_t s);
+int gt_run_f32(const GtCase& c, int tile, int mtiles, hipStream_t s);

@@ -284,12 +284,12 @@ int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32, const voi
 // bias (or null): [E], added to the logits before anything else; x_pieces: the bf16 rows x lie piece-major for exactly `rows` rows.
 // bf16 products of many rows: out[m][n] = x[m] . w[n] (+ bias). epilogue 0: bf16 results; 1: the weight's rows alternate gate and
 // up, out[m][n / 2] = the gated activation (constants as he_gated_act); 2: fp32 results. tile: BM << 16 | BN, one of those of
-// gemm_tall_tiles.h (fp32 results: BN 256), as he_gemm_tall_tile chooses. unary: relu squared (0) or relu (3) of the bf16 results, -1: none.
+// gemm_tall_tiles.h, as he_gemm_tall_tile chooses. slices (fp32 results): out is [slices][M][ldo], each the sums of a K / slices stretch. unary: relu squared (0) or relu (3) of the bf16 results, -1: none.
 // K a multiple of 64, N of 4.
 int he_gemm_tall_bf16(void* out, const void* x, const void* w, const void* bias, int bias_dtype, int M, int N, int K,
                       int64_t ldx, int64_t ldw, int64_t ldo, int epilogue, int tile, float alpha, float limit, float up_shift,
-                      float cubic, int unary, void* stream);
-int he_gemm_tall_tile(int M, int N, int K);
+                      float cubic, int unary, int slices, void* stream);
+int he_gemm_tall_tile(int M, int N, int K, int slices);
 // gemm_few_tiles.hip: out bf16 [M][ldo] = x [M][ldx] w [N][ldw]^T (+ bias) in tiles of he_gemm_few_tiles_tile(M, N) (0: no tile makes the
 // product one round of the chip). K a multiple of 64, N of 4, operands 16-byte aligned.
 int he_gemm_few_tiles_tile(int M, int N);

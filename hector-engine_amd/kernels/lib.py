@@ -106,8 +106,8 @@ _SIGNATURES = {
     "he_gemm_few_tiles_tile": [c_int, c_int],
     "he_gemm_few_tiles_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_int, c_ptr],
     "he_gemm_tall_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_int, c_int,
-                          c_f32, c_f32, c_f32, c_f32, c_int, c_ptr],
-    "he_gemm_tall_tile": [c_int, c_int, c_int],
+                          c_f32, c_f32, c_f32, c_f32, c_int, c_int, c_ptr],
+    "he_gemm_tall_tile": [c_int, c_int, c_int, c_int],
     "he_group_rows_most_tiles": [c_int, c_int, c_int, c_int],
     "he_routed_groups_ints": [c_int, c_int, c_int, c_int],
     "he_routed_groups": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int,

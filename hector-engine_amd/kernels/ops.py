@@ -1228,31 +1228,32 @@ def tiles_read(*tensors) -> bool:
 
 @_op("gemm_tall")
 def gemm_tall(out, x, w, bias, M: int, *, bm: int = 256, bn: int = 256, act=None,
-              unary: str | None = None) -> None:
+              unary: str | None = None, slices: int = 1) -> None:
     """out[M, N] = x[M, K] . w[N, K]^T (+ bias) for many bf16 rows (bf16 or fp32 results); with act, the constants (alpha,
     limit, up_shift, cubic) of a gated activation, w's rows alternate gate and up and out is [M, N / 2]. K a multiple
-    of 64, N of 4. bm, bn: the outputs of a tile (gemm_tall_tile). unary: "relu2" or "relu" of the bf16 results, as unary_act gives it."""
+    of 64, N of 4. bm, bn: the outputs of a tile (gemm_tall_tile). unary: "relu2" or "relu" of the bf16 results, as unary_act gives it.
+    slices: out is fp32 [slices, M, N], each the sums of one of so many equal stretches of K (whole 64s), as splitk_reduce adds them."""
     N, K = w.shape
     cols = N // 2 if act is not None else N
-    _need(out, "out", None, (None, cols))
+    _need(out, "out", None if slices == 1 else torch.float32, (None, cols) if slices == 1 else (slices, M, cols))
     _need(x, "x", torch.bfloat16, (None, K))
     _need(w, "w", torch.bfloat16)
     if bias is not None:
         _need(bias, "bias", None, (N,))
-    if min(out.shape[0], x.shape[0]) < M or out.dtype not in ((torch.bfloat16,) if act is not None else (torch.bfloat16, torch.float32)):
+    if min(out.shape[0] if slices == 1 else M, x.shape[0]) < M or out.dtype not in ((torch.bfloat16,) if act is not None else (torch.bfloat16, torch.float32)):
         raise ValueError("gemm_tall: buffers smaller than the row count, or results of an unknown type")
     epilogue = 1 if act is not None else 2 if out.dtype == torch.float32 else 0
     alpha, limit, up_shift, cubic = act or (1.0, 0.0, 0.0, 0.0)
     _lib.check(_lib.load().he_gemm_tall_bf16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias),
                                              dtype_code(bias.dtype) if bias is not None else F32, M, N, K, K, K, cols, epilogue,
                                              bm << 16 | bn, float(alpha), float(limit), float(up_shift), float(cubic),
-                                             -1 if unary is None else ACT_KINDS[unary], _stream()))
+                                             -1 if unary is None else ACT_KINDS[unary], slices, _stream()))
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_tall_tile(M: int, N: int, K: int) -> tuple[int, int]:
+def gemm_tall_tile(M: int, N: int, K: int, slices: int = 1) -> tuple[int, int]:
     """(bm, bn) of the tile gemm_tall is fastest with, by estimate."""
-    tile = int(_lib.load().he_gemm_tall_tile(M, N, K))
+    tile = int(_lib.load().he_gemm_tall_tile(M, N, K, slices))
     return tile >> 16, tile & 0xffff
 
 

@@ -75,6 +75,19 @@ def test_every_tile(bm, bn, M, N, K):
     assert (gated[M] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K,slices", [(70, 300, 128, 2), (203, 460, 1536, 8), (257, 2052, 768, 4)])
+@pytest.mark.parametrize("bm,bn", TILES)
+def test_k_slices(bm, bn, M, N, K, slices):
+    """Each slice is the product of its stretch of K, bit for bit."""
+    x, w = rnd(M, K, seed=1).cuda(), rnd(N, K, seed=2).cuda()
+    out = torch.full((slices, M, N), 7.0, device="cuda")
+    ops.gemm_tall(out, x, w, None, M, bm=bm, bn=bn, slices=slices)
+    for s in range(slices):
+        part, alone = slice(s * K // slices, (s + 1) * K // slices), torch.empty(M, N, device="cuda")
+        ops.gemm_tall(alone, x[:, part].contiguous(), w[:, part].contiguous(), None, M, bm=bm, bn=bn)
+        assert torch.equal(out[s], alone)
+
+
 @pytest.mark.parametrize("bm", [128, 256])
 @pytest.mark.parametrize("rows,real,identity,top", [(1, 3, 0, 1), (130, 5, 1, 2), (300, 16, 2, 4), (513, 1, 0, 1), (700, 40, 0, 8)])
 def test_experts_over_the_rows_that_chose_them(bm, rows, real, identity, top):
