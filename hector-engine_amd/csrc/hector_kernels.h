@@ -277,10 +277,13 @@ int he_mlstm_scan(void* y_f32, const void* q, const void* k, const void* v, int6
 
 // ---- routing and head combination (routing.hip) ---------------------------------
 // logits_f32 [rows][E], or null and x [rows][D] (x_dtype) with router_f32 [E][D]: the kernel forms the logits itself.
+// partials_f32 [rows][count] (or null): x are bf16 rows whose norm's scale is still owed; scaled_out [rows][D] gets the rows he_scale_rows_bf16
+// makes of them, and those are what the router reads.
 int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32, const void* logits_f32,
                     const void* x, int x_dtype, const void* router_f32, int D,
                     const void* correction, int c_dtype, int rows, int E, int real, int groups, int keep,
-                    int top, float scale, int normalize, const void* bias, int bias_dtype, int x_pieces, void* stream);
+                    int top, float scale, int normalize, const void* bias, int bias_dtype, int x_pieces,
+                    const void* partials_f32, int count, float eps, void* scaled_out, void* stream);
 // bias (or null): [E], added to the logits before anything else; x_pieces: the bf16 rows x lie piece-major for exactly `rows` rows.
 // bf16 products of many rows: out[m][n] = x[m] . w[n] (+ bias). epilogue 0: bf16 results; 1: the weight's rows alternate gate and
 // up, out[m][n / 2] = the gated activation (constants as he_gated_act); 2: fp32 results. tile: BM << 16 | BN, one of those of

@@ -2,10 +2,11 @@
 // combination of the two score maps of a differential attention head.
 #include "common.h"
 #include "hector_kernels.h"
+#include <type_traits>
 
 #define ROUTE_MAX_EXPERTS 1024
 
-// One workgroup a row. logits [rows][E] fp32, or, with x and router given, the router's product itself:
+// One workgroup a row, or two rows. logits [rows][E] fp32, or, with x and router given, the router's product itself:
 // logits[e] = sum_i x[row][i] * router[e][i] in fp32 (router fp32 [E][D]; a lane adds its elements i = lane,
 // lane + 64, ... in that order, the lanes' sums meet in the wavefront's butterfly: one fixed order a row,
 // whatever else the step holds). bias (or null): a stored number an output, added to its logit first. x_pieces: the bf16
@@ -17,17 +18,39 @@
 // itself: their weights are added up in column `real` of dense. dense [rows][real + 1] holds the
 // weight of every expert (0 where not chosen); ids / weights [rows][top] list the chosen ones.
 //
+// A step of many rows is bound by the reads of the router's matrix from L2, D * E * 4 bytes a workgroup: two rows share them.
 // What bounds a step of few rows is the chain: the router's rows come from memory, so a wavefront asks for those of up to four
 // outputs together; the choice is made by the first wavefront alone, PL outputs a lane in registers, without a barrier or a
 // walk through LDS a choice. (2 rows of 2048, 18 outputs in 3 groups, 4 chosen: 14.5 us with eight wavefronts that meet at two barriers a choice and
 // ask for one output at a time, 9 so; 2048 rows 41 us and 31; one row of 300 outputs in 5 groups, 8 chosen, 89 and 36.)
 #define ROUTE_WAVES 8
 
+// Rows x whose norm's scale is still owed (partials null: none is): the rows are bf16(x * inv) with inv as scale_rows_kernel forms it, and
+// the workgroup leaves them, row-major, in `out`: a launch less (2 rows of 2048, 18 outputs: 8.0 us in two launches, 7.1 in one, warm; with
+// 128 outputs, whose rows' scaling is done again for every four outputs of a wavefront, 20.0 and 20.5: up to 64 outputs only).
+struct RouteOwed {
+  const float* partials;      // [rows][count]: the row's sum of squares in parts
+  int count;
+  float eps;
+  uint16_t* out;
+};
+
+__device__ __forceinline__ float4 route_four(const uint2 b) {
+  return make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16),
+                     __uint_as_float(b.y & 0xffff0000u));
+}
+
+__device__ __forceinline__ uint2 route_scaled(const uint2 b, float inv) {
+  const float4 v = route_four(b);
+  return make_uint2(float_to_bf16_bits(v.x * inv) | (uint32_t)float_to_bf16_bits(v.y * inv) << 16,
+                    float_to_bf16_bits(v.z * inv) | (uint32_t)float_to_bf16_bits(v.w * inv) << 16);
+}
+
 // The dot products of row x with the router's rows e0, e0 + ROUTE_WAVES, ... (OUT of them, those beyond E repeat the last): four elements
 // a lane and turn, four sums a lane that meet in index order.
-template <int OUT>
-__device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x_dtype, const float* router, int64_t row, int D, int E, int e0,
-                                           int x_pieces) {
+template <int OUT, bool OWED>
+__device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x_dtype, const float* router, int64_t row, int rows, int D, int E,
+                                           int e0, int x_pieces, float inv) {
   const int lane = threadIdx.x & 63;
   const bool vec = (D & 3) == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)router & 15) == 0;
   const float* w[OUT];
@@ -42,14 +65,13 @@ __device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x
     // row-major: four elements i at 4 i; piece-major [D / 8][rows][8]: half i & 1 of the row's piece i / 2
     const uint2* xh = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * row : row * (D >> 2));
     const float4* xf = reinterpret_cast<const float4*>((const float*)x + row * D);
-    const int64_t piece = 2 * (int64_t)gridDim.x;
+    const int64_t piece = 2 * (int64_t)rows;
 #pragma unroll 4
     for (int i = lane; i < (D >> 2); i += 64) {
       float4 xv;
-      if (x_dtype == HE_BF16) {
+      if (OWED || x_dtype == HE_BF16) {
         const uint2 b = x_pieces ? xh[(i >> 1) * piece + (i & 1)] : xh[i];
-        xv = make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16),
-                         __uint_as_float(b.y & 0xffff0000u));
+        xv = route_four(OWED ? route_scaled(b, inv) : b);
       } else {
         xv = xf[i];
       }
@@ -74,6 +96,55 @@ __device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x
   for (int o = 0; o < OUT; ++o) z[o] = wave_sum((a[o][0] + a[o][1]) + (a[o][2] + a[o][3]));
 }
 
+// The same for RW rows from row0 on (those beyond the last repeat it), row-major, so that a load of the router's rows serves RW of them: every
+// product and sum as above.
+template <int OUT, int RW>
+__device__ __forceinline__ void route_dots_rows(float (&z)[RW][OUT], const void* x, int x_dtype, const float* router, int row0, int rows,
+                                                int D, int E, int e0) {
+  const int lane = threadIdx.x & 63;
+  const float* w[OUT];
+  int64_t at[RW];
+  float a[RW][OUT][4];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) at[r] = (int64_t)min(row0 + r, rows - 1) * (D >> 2);
+#pragma unroll
+  for (int o = 0; o < OUT; ++o) {
+    w[o] = router + (int64_t)min(e0 + o * ROUTE_WAVES, E - 1) * D;
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[r][o][j] = 0.f;
+  }
+  const auto turns = [&](auto bf) {         // one loop a type, without a branch in it: a turn's loads are in flight together
+#pragma unroll 2
+    for (int i = lane; i < (D >> 2); i += 64) {
+      float4 xv[RW];
+#pragma unroll
+      for (int r = 0; r < RW; ++r) {
+        if constexpr (decltype(bf)::value) xv[r] = route_four(((const uint2*)x)[at[r] + i]);
+        else xv[r] = ((const float4*)x)[at[r] + i];
+      }
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) {
+        const float4 wv = reinterpret_cast<const float4*>(w[o])[i];
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+          a[r][o][0] = fmaf(xv[r].x, wv.x, a[r][o][0]);
+          a[r][o][1] = fmaf(xv[r].y, wv.y, a[r][o][1]);
+          a[r][o][2] = fmaf(xv[r].z, wv.z, a[r][o][2]);
+          a[r][o][3] = fmaf(xv[r].w, wv.w, a[r][o][3]);
+        }
+      }
+    }
+  };
+  if (x_dtype == HE_BF16) turns(std::true_type{});
+  else turns(std::false_type{});
+#pragma unroll
+  for (int r = 0; r < RW; ++r)
+#pragma unroll
+    for (int o = 0; o < OUT; ++o) z[r][o] = wave_sum((a[r][o][0] + a[r][o][1]) + (a[r][o][2] + a[r][o][3]));
+}
+
 // The lowest index among the largest of the lanes' values (lane, lane + 64, ...), NaN never; `none` if all are NaN.
 template <int PL>
 __device__ __forceinline__ int route_argmax(const float (&c)[PL], int none) {
@@ -89,35 +160,57 @@ __device__ __forceinline__ int route_argmax(const float (&c)[PL], int none) {
   return none;
 }
 
-template <int PL>
+template <int PL, int RW, bool OWED>
 __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
     float* __restrict__ dense, int32_t* __restrict__ ids, float* __restrict__ weights, const float* __restrict__ logits,
     const void* __restrict__ x, int x_dtype, const float* __restrict__ router, int D,
-    const void* __restrict__ correction, int c_dtype, int E, int real, int groups, int keep, int top, float scale,
-    int normalize, const void* __restrict__ bias, int bias_dtype, int x_pieces) {
-  __shared__ float z_sh[64 * PL], c_sh[64 * PL];
-  const int64_t row = blockIdx.x;
+    const void* __restrict__ correction, int c_dtype, int rows, int E, int real, int groups, int keep, int top, float scale,
+    int normalize, const void* __restrict__ bias, int bias_dtype, int x_pieces, RouteOwed owed) {
+  static_assert(RW <= ROUTE_WAVES && (RW == 1 || !OWED), "a wavefront chooses for a row");
+  __shared__ float z_all[RW][64 * PL], c_all[RW][64 * PL];
+  const int row0 = blockIdx.x * RW;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   if (x != nullptr) {
+    float inv = 1.f;
+    if (OWED) {
+      float part = 0.f;
+      for (int i = lane; i < owed.count; i += 64) part += owed.partials[(int64_t)row0 * owed.count + i];
+      inv = 1.0f / sqrtf(wave_sum(part) / (float)D + owed.eps);
+    }
     for (int e0 = wave; e0 < E; e0 += 4 * ROUTE_WAVES) {
       if (e0 + 2 * ROUTE_WAVES < E) {
-        float z[4];
-        route_dots<4>(z, x, x_dtype, router, row, D, E, e0, x_pieces);
+        float z[RW][4];
+        if constexpr (RW == 1) route_dots<4, OWED>(z[0], x, x_dtype, router, row0, rows, D, E, e0, x_pieces, inv);
+        else route_dots_rows<4, RW>(z, x, x_dtype, router, row0, rows, D, E, e0);
 #pragma unroll
-        for (int o = 0; o < 4; ++o)
-          if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_sh[e0 + o * ROUTE_WAVES] = z[o];
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+          for (int o = 0; o < 4; ++o)
+            if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_all[r][e0 + o * ROUTE_WAVES] = z[r][o];
       } else {
-        float z[2];
-        route_dots<2>(z, x, x_dtype, router, row, D, E, e0, x_pieces);
+        float z[RW][2];
+        if constexpr (RW == 1) route_dots<2, OWED>(z[0], x, x_dtype, router, row0, rows, D, E, e0, x_pieces, inv);
+        else route_dots_rows<2, RW>(z, x, x_dtype, router, row0, rows, D, E, e0);
 #pragma unroll
-        for (int o = 0; o < 2; ++o)
-          if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_sh[e0 + o * ROUTE_WAVES] = z[o];
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+          for (int o = 0; o < 2; ++o)
+            if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_all[r][e0 + o * ROUTE_WAVES] = z[r][o];
       }
+    }
+    if (OWED) {
+      const uint2* xh = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * (int64_t)row0 : (int64_t)row0 * (D >> 2));
+      uint2* to = reinterpret_cast<uint2*>(owed.out) + (int64_t)row0 * (D >> 2);
+      for (int i = threadIdx.x; i < (D >> 2); i += 64 * ROUTE_WAVES)
+        to[i] = route_scaled(x_pieces ? xh[(i >> 1) * (2 * (int64_t)rows) + (i & 1)] : xh[i], inv);
     }
     __syncthreads();
   }
-  if (wave != 0) return;
+  const int64_t row = row0 + wave;
+  if (wave >= RW || row >= rows) return;
+  float* z_sh = z_all[wave];
+  float* c_sh = c_all[wave];
   // element j of a lane's arrays is output lane + 64 j; those beyond E are NaN to the choice
   float z[PL], s[PL], c[PL], d[PL];
   float mx = -INFINITY;
@@ -217,7 +310,7 @@ extern "C" int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32
                                const void* x, int x_dtype, const void* router_f32, int D,
                                const void* correction, int c_dtype, int rows, int E, int real, int groups, int keep,
                                int top, float scale, int normalize, const void* bias, int bias_dtype, int x_pieces,
-                               void* stream) {
+                               const void* partials_f32, int count, float eps, void* scaled_out, void* stream) {
   HE_REQUIRE((logits_f32 != nullptr) != (x != nullptr), "he_route_tokens: give the logits, or the rows and the router");
   HE_REQUIRE(x == nullptr || (router_f32 != nullptr && D > 0 && (x_dtype == HE_BF16 || x_dtype == HE_F32)),
              "he_route_tokens: the router's matrix is missing");
@@ -229,14 +322,29 @@ extern "C" int he_route_tokens(void* dense_f32, void* ids_i32, void* weights_f32
              keep * (E / groups));
   HE_REQUIRE(!x_pieces || (x != nullptr && x_dtype == HE_BF16 && (D & 7) == 0 && (((uintptr_t)x | (uintptr_t)router_f32) & 15) == 0),
              "he_route_tokens: piece-major rows are bf16, 16-byte aligned and a multiple of 8 wide");
+  HE_REQUIRE(partials_f32 == nullptr ||
+                 (x != nullptr && x_dtype == HE_BF16 && E <= 64 && scaled_out != nullptr && count > 0 && (D & 7) == 0 &&
+                  (((uintptr_t)x | (uintptr_t)router_f32 | (uintptr_t)scaled_out) & 15) == 0),
+             "he_route_tokens: rows whose scale is owed are bf16, 16-byte aligned and a multiple of 8 wide, for at most 64 outputs");
   if (rows == 0) return 0;
-#define ROUTE_LAUNCH(PL)                                                                                                       \
-  route_kernel<PL><<<rows, 64 * ROUTE_WAVES, 0, (hipStream_t)stream>>>(                                                         \
+  const RouteOwed owed = {(const float*)partials_f32, count, eps, (uint16_t*)scaled_out};
+#define ROUTE_LAUNCH(PL, RW, OWED)                                                                                             \
+  route_kernel<PL, RW, OWED><<<(rows + (RW) - 1) / (RW), 64 * ROUTE_WAVES, 0, (hipStream_t)stream>>>(                               \
       (float*)dense_f32, (int32_t*)ids_i32, (float*)weights_f32, (const float*)logits_f32, x, x_dtype, (const float*)router_f32, D, \
-      correction, c_dtype, E, real, groups, keep, top, scale, normalize, bias, bias_dtype, x_pieces)
-  if (E <= 64) ROUTE_LAUNCH(1);
-  else if (E <= 256) ROUTE_LAUNCH(4);
-  else ROUTE_LAUNCH(16);
+      correction, c_dtype, rows, E, real, groups, keep, top, scale, normalize, bias, bias_dtype, x_pieces, owed)
+  // Two rows a workgroup where that leaves no compute unit idle: one load of the router's rows serves both, and two wavefronts choose at once.
+  // (us with one row a workgroup and two, bf16 rows of 2048: 18 outputs, 256 rows 6.3 and 5.8, 512 rows 9.7 and 6.0, 4096 rows
+  // 53.6 and 23.7; 128 outputs 20.1 and 18.2, 33.8 and 19.2, 222 and 96.5; 64 rows the same within 0.3. Four rows a workgroup: 7.2, 7.3 and
+  // 21.8 with 18 outputs, 27, 27 and 98 with 128.)
+  const bool shared = x != nullptr && !x_pieces && rows > 256 && (D & 3) == 0 && (((uintptr_t)x | (uintptr_t)router_f32) & 15) == 0;
+#define ROUTE_OUTPUTS(PL)                       \
+  if (shared) ROUTE_LAUNCH(PL, 2, false);       \
+  else ROUTE_LAUNCH(PL, 1, false)
+  if (partials_f32 != nullptr) ROUTE_LAUNCH(1, 1, true);
+  else if (E <= 64) { ROUTE_OUTPUTS(1); }
+  else if (E <= 256) { ROUTE_OUTPUTS(4); }
+  else { ROUTE_OUTPUTS(16); }
+#undef ROUTE_OUTPUTS
 #undef ROUTE_LAUNCH
   return he_check_launch("he_route_tokens");
 }

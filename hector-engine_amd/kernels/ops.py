@@ -1150,14 +1150,18 @@ def mlstm_scan(y, q, k, v, gates, state, state_offset: int, cu_seqlens, seq_slot
 @_op("route_tokens")
 def route_tokens(dense, ids, weights, logits, correction, rows: int, real: int, groups: int, keep: int,
                  top: int, scale: float, *, x=None, router=None, normalize: bool = False, bias=None,
-                 x_pieces: bool = False) -> None:
+                 x_pieces: bool = False, owed=None) -> None:
     """The choice of `top` of E router outputs per row (logits fp32 [rows, E]; or logits None and the kernel
     forms them in fp32 from the rows x [rows, D] and the router's matrix, fp32 [E, D]): softmax scores s, the
     choice on s + correction inside the `keep` best of `groups` equal groups, weights s * scale. dense (fp32
     [rows, real + 1]): each expert's weight or 0, the outputs from `real` on added up in the last column;
     ids (int32) and weights (fp32) [rows, top]: the chosen outputs. normalize: the chosen outputs' weights are divided
     by their sum (times scale): the softmax over the chosen logits alone. bias [E]: added to the logits first.
-    x_pieces: x lies piece-major, shaped pieces_shape(rows, D)."""
+    x_pieces: x lies piece-major, shaped pieces_shape(rows, D). owed: (partials, eps, out) where x are bf16 rows whose norm's
+    scale is owed (D a multiple of 8, at most 64 outputs): the launch leaves the rows scale_rows makes of them in out [rows, D], and those are the
+    ones the router reads."""
+    if owed is not None and logits is not None:
+        raise ValueError("route_tokens: the scale of rows the launch does not read")
     if logits is None:
         E, D = router.shape
         _need(router, "router", torch.float32)
@@ -1167,8 +1171,14 @@ def route_tokens(dense, ids, weights, logits, correction, rows: int, real: int, 
             _need(x, "x", None, (None, D))
             if x.shape[0] < rows:
                 raise ValueError("route_tokens: x has fewer rows than the step")
+        if owed is not None:
+            _need(x, "x", torch.bfloat16)
+            _need(owed[0], "partials", torch.float32)
+            _need(owed[2], "out", torch.bfloat16, (None, D))
+            if owed[0].dim() != 2 or min(owed[0].shape[0], owed[2].shape[0]) < rows:
+                raise ValueError("route_tokens: buffers smaller than the row count")
         return _route(dense, ids, weights, None, x, router, correction, rows, E, real, groups, keep, top, scale, normalize,
-                      bias, x_pieces)
+                      bias, x_pieces, owed)
     E = logits.shape[-1]
     _need(logits, "logits", torch.float32, (None, E))
     if logits.shape[0] < rows:
@@ -1177,7 +1187,7 @@ def route_tokens(dense, ids, weights, logits, correction, rows: int, real: int, 
 
 
 def _route(dense, ids, weights, logits, x, router, correction, rows, E, real, groups, keep, top, scale, normalize=False,
-           bias=None, x_pieces=False) -> None:
+           bias=None, x_pieces=False, owed=None) -> None:
     _need(dense, "dense", torch.float32, (None, real + 1))
     _need(ids, "ids", torch.int32, (None, top))
     _need(weights, "weights", torch.float32, (None, top))
@@ -1193,7 +1203,9 @@ def _route(dense, ids, weights, logits, x, router, correction, rows, E, real, gr
                                  router.shape[1] if router is not None else 0,
                                  _ptr(correction), dtype_code(correction.dtype) if correction is not None else F32,
                                  rows, E, real, groups, keep, top, float(scale), int(normalize), _ptr(bias),
-                                 dtype_code(bias.dtype) if bias is not None else F32, int(x_pieces), _stream()))
+                                 dtype_code(bias.dtype) if bias is not None else F32, int(x_pieces),
+                                 _ptr(owed[0]) if owed else 0, owed[0].shape[1] if owed else 0,
+                                 float(owed[1]) if owed else 0.0, _ptr(owed[2]) if owed else 0, _stream()))
 
 
 @_op("routed_act")

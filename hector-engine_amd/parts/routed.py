@@ -235,18 +235,28 @@ class RoutedExperts(FeedForward):
     def _routed(self, x, ctx: StepContext, may_sink: bool):
         rows, real, I, S = ctx.rows, self.real, self.inter, self.shared_cols
         # rows a product has left for this norm: read as they lie where they owe nothing (and no identity expert wants
-        # them row by row), else made into a tensor
+        # them row by row), else made into a tensor, by the router's launch where that pays and its reads are whole
         pieces = isinstance(x, NormedRows) and x.finished and x.pieces and not self.identity
-        given = x                                    # what the experts' first product reads
+        owed = None
+        given, read, read_pieces = x, x, pieces      # what the experts' first product reads, and the router
         if isinstance(x, NormedRows):
-            x = x.scaled if pieces else x.tensor(ctx)
-            given = given if pieces else x
+            read, read_pieces = x.scaled, x.pieces
+            if pieces:
+                x = x.scaled
+            elif self.router.shape[0] <= 64 and x.dim % 8 == 0 and read.data_ptr() % 16 == 0 and self.router.data_ptr() % 16 == 0:
+                given = ctx.alloc((rows, x.dim), read.dtype)
+                owed = (x.partials, x.eps, given)
+                x = given
+            else:
+                given = read = x = x.tensor(ctx)
+                read_pieces = False
         dense = ctx.alloc((rows, real + 1), torch.float32)
         ids = ctx.alloc((rows, self.top), torch.int32)
         weights = ctx.alloc((rows, self.top), torch.float32)
         # the router's product (fp32 sums over the rows as they are) and the choice, one launch
         ops.route_tokens(dense, ids, weights, None, self.correction, rows, real, self.groups, self.keep,
-                         self.top, self.scale, x=x, router=self.router, normalize=self.normalize, bias=self.bias, x_pieces=pieces)
+                         self.top, self.scale, x=read, router=self.router, normalize=self.normalize, bias=self.bias,
+                         x_pieces=read_pieces, owed=owed)
         cols = real * I + S + (self.hidden if self.identity else 0)
         act = {"alpha": self.alpha, "limit": self.limit, "up_shift": self.up_shift}
         if self._few_rows(rows, x, ctx):

@@ -52,3 +52,54 @@ def test_choice(E, real, groups, keep, top, normalize):
             for e, v in zip(got, w):
                 want[min(e, real)] += v
             assert torch.allclose(dense[r].cpu().double(), want, rtol=4e-6, atol=1e-9)
+
+
+def _routed(ops, x, router, rows, groups, keep, top, **more):
+    E = router.shape[0]
+    dense = torch.full((rows, E - 1), math.nan, device="cuda")
+    ids, weights = torch.full((rows, top), 77, dtype=torch.int32, device="cuda"), torch.full((rows, top), math.nan, device="cuda")
+    ops.route_tokens(dense, ids, weights, None, None, rows, E - 2, groups, keep, top, 1.5, x=x, router=router, **more)
+    return dense, ids, weights
+
+
+@pytest.mark.parametrize("E,D,groups,keep,top", [(3, 4, 1, 1, 2), (18, 2048, 3, 2, 4), (64, 260, 8, 2, 5), (100, 1028, 1, 1, 8), (300, 64, 5, 3, 9),
+                                                 (18, 42, 1, 1, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_that_share_a_workgroup(E, D, groups, keep, top, dtype):
+    """Steps of more than 256 rows read the router's rows once for two rows: each row's result has the bits it has alone."""
+    from hector_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(D)
+    for rows in (257, 518):
+        x = torch.randn(rows, D, generator=g).to(dtype).cuda()
+        router = torch.randn(E, D, generator=g).cuda()
+        got = _routed(ops, x, router, rows, groups, keep, top, normalize=True)
+        at = 0
+        for n in (1, 200, 56, rows - 257):
+            if n == 0:
+                continue
+            alone = _routed(ops, x[at:at + n].clone(), router, n, groups, keep, top, normalize=True)
+            for a, b in zip(got, alone):
+                assert torch.equal(a[at:at + n], b)
+            at += n
+        assert at == rows
+
+
+@pytest.mark.parametrize("rows,E,D,count,pieces", [(1, 18, 2048, 256, True), (3, 64, 8, 1, False), (16, 5, 520, 65, True), (300, 33, 264, 7, False)])
+def test_the_norms_scale_with_the_choice(rows, E, D, count, pieces):
+    """Rows whose norm's scale is owed: the launch gives the rows and the choice of the two launches it stands for, bit for bit."""
+    from hector_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, D, generator=g).bfloat16().cuda()
+    partials = (torch.rand(rows, count, generator=g) * D / count).cuda()
+    router = torch.randn(E, D, generator=g).cuda()
+    given = x.view(rows, D // 8, 8).transpose(0, 1).contiguous() if pieces else x
+    want_rows, got_rows = torch.empty_like(x), torch.full_like(x, math.nan)
+    ops.scale_rows(want_rows, given, partials, 1e-6, rows, pieces)
+    want = _routed(ops, want_rows, router, rows, 1, 1, 3)
+    got = _routed(ops, given, router, rows, 1, 1, 3, x_pieces=pieces, owed=(partials, 1e-6, got_rows))
+    assert torch.equal(got_rows, want_rows)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    with pytest.raises(RuntimeError):
+        ops.route_tokens(*want, None, None, rows, E - 2, 1, 1, 3, 1.5, x=given, router=torch.randn(65, D, device="cuda"), x_pieces=pieces,
+                         owed=(partials, 1e-6, got_rows))
