@@ -80,20 +80,6 @@ __device__ __forceinline__ int gt_at(const int32_t* list, int i) {
   return ((const __attribute__((address_space(4))) int32_t*)(uintptr_t)list)[i];
 }
 
-// silu(g) u for a result that is rounded to bfloat16, without the library's exp and the division's corrections: exp(-g) as a power of two with
-// what the rounding of its exponent loses put back, and the hardware's reciprocal, of a quarter of the denominator (so that it stays a
-// normal number wherever the exponential is finite). Its relative error is below 5e-7 (the bf16 rounding behind it 2e-3); infinities,
-// NaN and overflow of the exponential end as in g / (1 + exp(-g)) * u. (With that an epilogue took 4 us a tile of 256 x 256:
-// 2048 x 37888 x 3584 424 us beside 414 so, 12001 rows 2484 and 2364.)
-__device__ __forceinline__ float gt_silu_mul(float g, float u) {
-  const float e = g * -1.44269504088896341f;                      // -g log2(e)
-  const float lost = fmaf(g, -1.44269504088896341f, -e);          // exact: what the rounding of e lost
-  const float low = fmaf(g, 1.92596299112661746887e-8f, lost);    // and what log2(e) in 32 bits has too much
-  const float t = __builtin_amdgcn_exp2f(e);
-  const float power = fabsf(e) < 128.f ? fmaf(t * 0.693147180559945309f, low, t) : t;      // t 2^low (no NaN from an infinite t or g)
-  return (0.25f * g) * __builtin_amdgcn_rcpf(fmaf(power, 0.25f, 0.25f)) * u;
-}
-
 struct GtTile {
   int m0, n0, group, slice;
 };
@@ -301,12 +287,14 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
       if (to < 0) continue;
       const int64_t row = to * c.ldo + (EPI == GT_GATED && c.spread ? (int64_t)t.group * (c.N / 2) : 0);
       // gate and up are rounded to bf16 first, as where a kernel of its own reads them from memory: the two ways then
-      // differ by the order of fp32 sums alone (a choice of weight zero gives exact zeros, whatever its row holds)
+      // differ by the order of fp32 sums alone (a choice of weight zero gives exact zeros, whatever its row holds). The activation is the one
+      // those kernels have, bit for bit: beside a router over rows that no norm has evened out a last bit turns near ties into other
+      // choices (with an exponential and a reciprocal of fewer corrections, 12001 x 37888 x 3584 2364 us instead of 2484, one such
+      // design's logits moved by 7 % of their size)
       auto gated = [&](gt_f32x4 v) {
         const uint32_t p = pack2_bf16(v[0], v[1]), q = pack2_bf16(v[2], v[3]);
-        auto act = [&](float gate, float up) { return CLAMPED ? he_gated_act<true>(gate, up, c.act) : gt_silu_mul(gate, up); };
-        const float a = f == 0.f ? 0.f : act(__uint_as_float(p << 16), __uint_as_float(p & 0xffff0000u)) * f;
-        const float b = f == 0.f ? 0.f : act(__uint_as_float(q << 16), __uint_as_float(q & 0xffff0000u)) * f;
+        const float a = f == 0.f ? 0.f : he_gated_act<CLAMPED>(__uint_as_float(p << 16), __uint_as_float(p & 0xffff0000u), c.act) * f;
+        const float b = f == 0.f ? 0.f : he_gated_act<CLAMPED>(__uint_as_float(q << 16), __uint_as_float(q & 0xffff0000u), c.act) * f;
         return pack2_bf16(a, b);
       };
       auto plain = [&](gt_f32x4 v, int n) {

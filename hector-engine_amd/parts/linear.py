@@ -412,8 +412,8 @@ class Linear:
         """The tile (ops.gemm_tall's bm, bn) where a product of this many bf16 rows with K above 1024 takes the activation of its results
         along, None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
         0.8 of their rounds or more. Over 229 gated products of 70 to 12001 rows, 256 to 55296 columns and K up to 27648 it took 0.55 to
-        1.10 of the time of the two, 0.91 in the geometric mean, 15 of them above 1.03 (2048 x 37888 x 3584 414 us beside 546, 203 rows 73
-        beside 84, 100 rows 57 beside 69); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _tall."""
+        1.10 of the time of the two, 0.91 in the geometric mean, 15 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
+        beside 85, 100 rows 58 beside 71); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _tall."""
         N, K = self.weight.shape
         if not (self.one_round_tiles and K > 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0
                 and N % 8 == 0 and self.weight.is_contiguous() and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) \
