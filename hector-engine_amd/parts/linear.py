@@ -69,7 +69,7 @@ class Linear:
         self.weight = weight
         self.bias = bias
         self.out_features, self.in_features = weight.shape
-        self.one_round_tiles = False        # set by a part: _tall's, _long's and gated_tile's products may run in tiles of this library's own
+        self.one_round_tiles = False        # set by a part: _tall's, _long's, gated_tile's and K slices' products may run in tiles of this library's own
         self._plans: dict[bool, tuple[int, int]] = {}
         self._chosen: dict[tuple, routes.Route] = {}     # (rows, activations, fast) -> route, for one version of the table
         self._chosen_version = -1
@@ -298,10 +298,12 @@ class Linear:
         if slices > 1:
             N, K = w.shape
             partial = ctx.alloc((slices, rows, N), torch.float32)
-            if K % (64 * slices) == 0 and N % 4 == 0 and w.is_contiguous() and ops.tiles_read(x, w) and not library_tuning.enabled():
-                # the same slices in this library's own tiles, the same bits: over 35 products of 70 to 512 rows 0.57 to 1.03 of the
+            if self.one_round_tiles and K % (64 * slices) == 0 and N % 4 == 0 and w.is_contiguous() and ops.tiles_read(x, w) \
+                    and not library_tuning.enabled():
+                # the same slices in this library's own tiles, over 35 products of 70 to 512 rows 0.57 to 1.03 of the
                 # batched product's time, 0.89 in the geometric mean (203 x 3584 x 18944 45.9 us beside 48.8, 128 x 2048 x 8192 17.8 beside
-                # 31.1)
+                # 31.1). Only where a part allows it (see _tall): of 310 products of 65 to 512 rows 295 had the library's bits, 15 of some
+                # widths (768 x 16384 at 65 rows, 2192 x 28672 at 128) 3 results in 10,000 that differ in their last bit
                 bm, bn = ops.gemm_tall_tile(rows, N, K, slices)
                 ops.gemm_tall(partial, x, w, None, rows, bm=bm, bn=bn, slices=slices)
                 ops.splitk_reduce(out, partial, bias, rows, slices)

@@ -273,16 +273,18 @@ def test_a_kernel_route_registered_from_outside_is_the_one_that_runs(fw):
 
 @pytest.mark.parametrize("rows", [65, 200, 512, 513])
 @pytest.mark.parametrize("N,K,bias", [(72, 8192, True), (300, 9024, False), (40, 8200, True)])
-def test_a_long_k_product_in_slices_through_the_library(fw, rows, N, K, bias):
+@pytest.mark.parametrize("own", [False, True])
+def test_a_long_k_product_in_slices_through_the_library(fw, rows, N, K, bias, own):
     """More than 64 rows against a weight with a long K and few output columns (a down projection):
     up to 512 rows the library runs it as a batched product over K slices whose fp32 results are added
-    in slice order; above, or where K does not divide, as one product. Either way the double-precision
-    result, within bfloat16's rounding of the output."""
+    in slice order; above, or where K does not divide, as one product. Either way, and where a part allows the
+    slices this library's own tiles, the double-precision result, within bfloat16's rounding of the output."""
     from hector_engine_amd.parts.linear import Linear
     env = env_for(fw, torch.bfloat16)
     w = rnd(N, K, seed=11, scale=0.05).to(torch.bfloat16)
     b = rnd(N, seed=12).to(torch.bfloat16) if bias else None
     lin = Linear(w.cuda(), b.cuda() if bias else None)
+    lin.one_round_tiles = own
     slices = lin._library_slices(rows)
     want = 1 if rows > 512 else 8          # a handful of the library's tiles at these sizes
     while want > 1 and K % (8 * want):

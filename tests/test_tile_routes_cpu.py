@@ -91,6 +91,20 @@ def test_a_shared_expert_keeps_the_library_s_sums():
     assert not routed.shared.down.one_round_tiles and not routed.down.one_round_tiles
 
 
+def test_k_slices_in_tiles_are_for_parts_that_allow_them(monkeypatch):
+    """The experts' down product beside a shared expert is such a weight: its slices stay the library's, whose bits the tiles do not always give."""
+    ran, N, K, rows = [], 2048, 32768, 300
+    for module, name in ((ops, "gemm_tall"), (ops, "splitk_reduce"), (torch, "bmm")):
+        monkeypatch.setattr(module, name, lambda *a, name=name, **k: ran.append(name))
+    ctx = SimpleNamespace(env=CTX.env, alloc=lambda shape, dtype=BF16: empty(*shape, dtype=dtype))
+    lin = Linear(empty(N, K))
+    assert lin._library_slices(rows) == 8
+    for allowed in (False, True):
+        lin.one_round_tiles = allowed
+        lin._library(empty(rows, K), None, rows, empty(rows, N), BF16, ctx)
+    assert ran == ["bmm", "splitk_reduce", "gemm_tall", "splitk_reduce"]
+
+
 def test_operands_the_tiles_do_not_read_stay_with_the_library():
     def shifted(*shape):
         return torch.empty(math.prod(shape) + 1, dtype=BF16)[1:].view(shape)
