@@ -42,6 +42,12 @@ from .mlp import GatedMLP
 _ROW_CHUNK = 4096
 
 
+def _linears(part) -> list[Linear]:
+    """The linear layers of a bound part and of the parts it is made of."""
+    own = [v for v in vars(part).values() if isinstance(v, Linear)]
+    return own + [lin for child in part.children() for lin in _linears(child)]
+
+
 @register_part("feed_forward", "routed_experts")
 class RoutedExperts(FeedForward):
     def __init__(self, params: dict, prefix: str, env: BuildEnv):
@@ -140,8 +146,8 @@ class RoutedExperts(FeedForward):
         self.down = Linear(torch.cat(downs, 1).contiguous())
         if self.shared is not None and not self.shared_cols:
             self.shared.bind(tensors)
-            if isinstance(self.shared, GatedMLP):
-                self.shared.gate_up.one_round_tiles = self.shared.down.one_round_tiles = False      # (the router may read rows no norm has evened out)
+            for lin in _linears(self.shared):
+                lin.one_round_tiles = False                # (the router may read rows no norm has evened out)
         if self._shared_gate:
             self.shared_gate = tensors[self._shared_gate].reshape(-1).contiguous()
 

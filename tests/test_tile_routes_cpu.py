@@ -89,6 +89,14 @@ def test_a_shared_expert_keeps_the_library_s_sums():
     routed = bound("routed_experts", {**mlp, "experts": 4, "top": 2, "correction": False,
                                       "shared": {"gate": "sg", "feed_forward": PartSpec("gated_mlp", mlp)}})
     assert not routed.shared.down.one_round_tiles and not routed.down.one_round_tiles
+    # one without a gate, and one that is itself routed and has a shared expert
+    dense = PartSpec("dense_mlp", {**mlp, "activation": "relu2"})
+    assert bound("dense_mlp", dense.params).up.one_round_tiles
+    within = PartSpec("routed_experts", {**mlp, "experts": 4, "top": 2, "correction": False, "shared": {"gate": "sg", "feed_forward": dense}})
+    for shared in (dense, within):
+        part = bound("routed_experts", {**mlp, "experts": 4, "top": 2, "correction": False, "shared": {"feed_forward": shared}}).shared
+        mlp_of = getattr(part, "shared", part)
+        assert not mlp_of.up.one_round_tiles and not mlp_of.down.one_round_tiles
 
 
 def test_k_slices_in_tiles_are_for_parts_that_allow_them(monkeypatch):
