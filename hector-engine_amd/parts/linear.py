@@ -246,7 +246,9 @@ class Linear:
         return self._rounds(rows, 128) <= 0.94 and rows * N >= 0.72 * 128 * 256 * ops.compute_units()
 
     def _tile_fill(self, rows: int) -> tuple[float, float]:
-        """Of the tile gemm_tall_tile chooses: the share of its rounds of the chip that has tiles, and that has real outputs."""
+        """Of the tile gemm_tall_tile chooses: the share of its rounds of the chip that has tiles, and that has real outputs (none of no rows)."""
+        if rows == 0:
+            return 0.0, 0.0
         N, K = self.weight.shape
         bm, bn = ops.gemm_tall_tile(rows, N, K)
         tiles, cus = -(-rows // bm) * -(-N // bn), ops.compute_units()

@@ -183,6 +183,21 @@ def test_which_gated_products_of_longer_k_run_as_one_kernel(N, K, tiles):
         assert not any(lin.gated_tile(r, CTX, empty(r, K)) for r in tiles)
 
 
+@pytest.mark.parametrize("kind,names", [("gated_mlp", {"activation": "silu"}), ("dense_mlp", {"activation": "relu2"})])
+def test_no_rows_are_no_product_in_tiles(monkeypatch, kind, names):
+    """A part called with no rows answers with none, at a K and a width whose products of many rows run in tiles."""
+    def alloc(shape, dtype=BF16):
+        return empty(*shape, dtype=dtype)
+    ctx = SimpleNamespace(env=CTX.env, rows=0, alloc=alloc, take_sink=lambda: None)
+    part = build_part("feed_forward", PartSpec(kind, {"hidden_size": 2048, "intermediate_size": 16384, **names}), "m.", CTX.env)
+    part.bind({k: empty(*v.shape) for k, v in part.tensor_specs().items()})
+    for name in ("silu_mul", "unary_act"):
+        monkeypatch.setattr(ops, name, lambda *a, **k: None)
+    first = part.gate_up if kind == "gated_mlp" else part.up
+    assert first.gated_tile(0, ctx, empty(0, 2048)) is None
+    assert part.forward(empty(0, 2048), ctx).shape == (0, 2048)
+
+
 @pytest.mark.parametrize("N,K,rows", [(3584, 18944, {768: False, 900: False, 1300: True, 3001: True, 12001: True}),
                                       (5120, 27648, {900: True, 8192: True}), (4096, 14336, {10000: False}), (3584, 29568, {12001: False}),
                                       (3584, 18912, {12001: False}), (3586, 18944, {12001: False})])
