@@ -15,7 +15,7 @@ registers:
   bfloat16, M > 64         -> the library matrix product (the reference calls its BLAS
                               library for every product: kernels/matmul_cublas.cu:240-277), or
                               the tiles of kernels.ops.gemm_tall or gemm_few_tiles where they are faster
-                              (_tall, _long, tall_gated, gated_tile, _few_tiles)
+                              (_long, tall_gated, gated_tile, _few_tiles)
   fp32 results (logits)    -> the MFMA kernels up to 64 rows, above that the library,
                               which writes fp32 from bf16 operands
 
@@ -69,7 +69,7 @@ class Linear:
         self.weight = weight
         self.bias = bias
         self.out_features, self.in_features = weight.shape
-        self.one_round_tiles = False        # set by a part: _tall's, _long's, gated_tile's and K slices' products may run in tiles of this library's own
+        self.one_round_tiles = False        # set by a part: _long's, gated_tile's and K slices' products may run in tiles of this library's own
         self._plans: dict[bool, tuple[int, int]] = {}
         self._chosen: dict[tuple, routes.Route] = {}     # (rows, activations, fast) -> route, for one version of the table
         self._chosen_version = -1
@@ -229,22 +229,6 @@ class Linear:
             slices //= 2
         return slices
 
-    def _tall(self, rows: int, x, out, out_dtype) -> bool:
-        """Whether a product of long K runs in tiles (kernels.ops.gemm_tall) by the rule for tiles of 128 x 256: for K from 16448 to 27648, where
-        the library's default choice drops to 0.75 PFLOP/s (from 1.0 to 1.4 at shorter K), and tiles that are at most 0.94 of a
-        round on the chip, 0.72 of it real outputs. 2048 x 3584 x 18944 takes 225 us (in tiles of 128 x 224), the library 355; over 149 random products of
-        this range 0.55 to 1.07 of the library's time, 0.78 in the geometric mean, with an earlier kernel that took 256 us there. Fewer tiles leave units idle; beyond 0.94 the
-        library's choice is another one for some widths (3072 x 18944: the tiles take 1.09 of its time), and beyond K 27648 for others (8192 x
-        29568 1.24 of it). Up to K 16384 the tiles lost on nearly every width (4096 x 14336 at 1019 rows 197 us, 132). Only where a part
-        allows it: the library adds some tiles of such a product in two halves, so 6 results in 10,000 differ in their last bit,
-        which a router over rows that no norm has evened out turns into other choices."""
-        N, K = self.weight.shape
-        if library_tuning.enabled() or not (self.one_round_tiles and out_dtype == BF16 and 16384 < K <= 27648 and K % 64 == 0
-                                            and N % 4 == 0 and x.is_contiguous() and out.is_contiguous()
-                                            and ops.tiles_read(x, self.weight, out)):
-            return False
-        return self._rounds(rows, 128) <= 0.94 and rows * N >= 0.72 * 128 * 256 * ops.compute_units()
-
     def _tile_fill(self, rows: int) -> tuple[float, float]:
         """Of the tile gemm_tall_tile chooses: the share of its rounds of the chip that has tiles, and that has real outputs (none of no rows)."""
         if rows == 0:
@@ -256,11 +240,15 @@ class Linear:
         return tiles / places, rows * N / (places * bm * bn)
 
     def _long(self, rows: int, x, out, out_dtype) -> bool:
-        """Whether a product of long K runs in tiles of this library's own whatever their number: for K from 16448 to 27648 again, where
-        the tiles of gemm_tall_tile's choice leave at most 0.3 of their rounds without real outputs. Over 53 products of 70 to
-        12001 rows and 320 to 20864 columns 0.55 to 1.10 of the library's time, 0.79 in the geometric mean, three above 1.03 (12001 x 3584 x
-        18944 1144 us, the library 1528); with 0.4 to 0.6 of the rounds real up to 1.27. At K up to 16384 the library's choice is as often
-        as not the faster one (0.57 to 1.24 of its time over 300 products of whole rounds, 0.98 in the geometric mean)."""
+        """Whether a product of long K runs in tiles of this library's own (kernels.ops.gemm_tall): for K from 16448 to 27648, where
+        the library's default choice drops to 0.65 to 0.9 PFLOP/s at many sizes (from 1.0 to 1.4 at shorter K), and tiles of gemm_tall_tile's
+        choice that leave at most 0.3 of their rounds without real outputs. Over 522 products of 458 to 12032 rows and 480 to 12892
+        columns 0.53 to 1.19 of the library's time, 0.78 in the geometric mean, 70 of them above 1.03 (2048 x 3584 x 18944 230 us, the library 358; 12001 rows
+        1144, 1528); with 0.4 to 0.6 of the rounds real up to 1.19, with less up to 3. At K up to 16384 the library's choice is as often
+        as not the faster one (0.57 to 1.24 of its time over 300 products of whole rounds, 0.98 in the geometric mean), and beyond K 27648 too
+        (8192 x 29568 up to 1.24). Only where a part allows it (one_round_tiles): the library adds some tiles of such a product in
+        two halves, so 6 results in 10,000 differ in their last bit, which a router over rows that no norm has evened out turns into
+        other choices."""
         N, K = self.weight.shape
         return not library_tuning.enabled() and self.one_round_tiles and out_dtype == BF16 and 16384 < K <= 27648 and K % 64 == 0 \
             and N % 4 == 0 and x.is_contiguous() and out.is_contiguous() and self.weight.is_contiguous() and ops.tiles_read(x, self.weight, out) \
@@ -288,7 +276,7 @@ class Linear:
         """More than 64 rows: the library's product, or tiles of this one's own; it also writes fp32 results (the logits) from
         bf16 operands (the head of the Qwen2.5-7B shape at 64 rows: 217 us)."""
         w = self.weight
-        if self._tall(rows, x, out, out_dtype) or self._long(rows, x, out, out_dtype):
+        if self._long(rows, x, out, out_dtype):
             bm, bn = ops.gemm_tall_tile(rows, *w.shape)
             ops.gemm_tall(out, x, w, bias, rows, bm=bm, bn=bn)
             return out
@@ -304,7 +292,7 @@ class Linear:
                     and not library_tuning.enabled():
                 # the same slices in this library's own tiles, over 35 products of 70 to 512 rows 0.57 to 1.03 of the
                 # batched product's time, 0.89 in the geometric mean (203 x 3584 x 18944 45.9 us beside 48.8, 128 x 2048 x 8192 17.8 beside
-                # 31.1). Only where a part allows it (see _tall): of 310 products of 65 to 512 rows 295 had the library's bits, 15 of some
+                # 31.1). Only where a part allows it (see _long): of 310 products of 65 to 512 rows 295 had the library's bits, 15 of some
                 # widths (768 x 16384 at 65 rows, 2192 x 28672 at 128) 3 results in 10,000 that differ in their last bit
                 bm, bn = ops.gemm_tall_tile(rows, N, K, slices)
                 ops.gemm_tall(partial, x, w, None, rows, bm=bm, bn=bn, slices=slices)
@@ -417,7 +405,7 @@ class Linear:
         along, None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
         0.8 of their rounds or more. Over 229 gated products of 70 to 12001 rows, 256 to 55296 columns and K up to 27648 it took 0.55 to
         1.10 of the time of the two, 0.91 in the geometric mean, 15 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
-        beside 85, 100 rows 58 beside 71); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _tall."""
+        beside 85, 100 rows 58 beside 71); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _long."""
         N, K = self.weight.shape
         if not (self.one_round_tiles and K > 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0
                 and N % 8 == 0 and self.weight.is_contiguous() and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) \
