@@ -403,15 +403,18 @@ class Linear:
     def _tile_with_activation(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
         """The tile (ops.gemm_tall's bm, bn) where a product of this many bf16 rows with K above 1024 takes the activation of its results
         along, None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
-        0.8 of their rounds or more. Over 229 gated products of 70 to 12001 rows, 256 to 55296 columns and K up to 27648 it took 0.55 to
-        1.10 of the time of the two, 0.91 in the geometric mean, 15 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
-        beside 85, 100 rows 58 beside 71); below 0.8 up to 1.17. Only where a part allows it (one_round_tiles): see _long."""
+        0.8 of their rounds or more, and either one row of tiles, which read the weight once whatever of their rows is padding, or 0.72 of
+        the rounds real outputs. Over 198 gated products of 65 to 12001 rows, 256 to 55296 columns and K up to 20000 it took 0.71 to
+        1.09 of the time of the two, 0.90 in the geometric mean, 3 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
+        beside 85, 100 rows 58 beside 71); with several rows of tiles and less of them real 0.77 to 1.24 (259 x 28672 x 4096 100 us, the two 82,
+        541 x 37888 x 2048 106 and 98), with tiles for less than 0.8 of the rounds up to 1.48. Only where a part allows it (one_round_tiles): see _long."""
         N, K = self.weight.shape
         if not (self.one_round_tiles and K > 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0
                 and N % 8 == 0 and self.weight.is_contiguous() and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) \
                 or library_tuning.enabled():
             return None
-        return ops.gemm_tall_tile(rows, N, K) if self._tile_fill(rows)[0] >= 0.8 else None
+        tile, (tiles, real) = ops.gemm_tall_tile(rows, N, K), self._tile_fill(rows)
+        return tile if tiles >= 0.8 and (rows <= tile[0] or real >= 0.72) else None
 
     def gated_tile(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
         """The tile where the gated product of this many rows runs as one kernel, None where it does not (K up to 1024: tall_gated)."""
