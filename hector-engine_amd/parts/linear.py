@@ -242,9 +242,11 @@ class Linear:
     def _long(self, rows: int, x, out, out_dtype) -> bool:
         """Whether a product of long K runs in tiles of this library's own (kernels.ops.gemm_tall): for K from 16448 to 27648, where
         the library's default choice drops to 0.65 to 0.9 PFLOP/s at many sizes (from 1.0 to 1.4 at shorter K), and tiles of gemm_tall_tile's
-        choice that leave at most 0.3 of their rounds without real outputs. Over 522 products of 458 to 12032 rows and 480 to 12892
-        columns 0.53 to 1.19 of the library's time, 0.78 in the geometric mean, 70 of them above 1.03 (2048 x 3584 x 18944 230 us, the library 358; 12001 rows
-        1144, 1528); with 0.4 to 0.6 of the rounds real up to 1.19, with less up to 3. At K up to 16384 the library's choice is as often
+        choice that leave at most 0.3 of their rounds without real outputs. Over 468 products of 458 to 12032 rows and 480 to 12892
+        columns 0.53 to 1.11 of the library's time, 0.76 in the geometric mean, 25 of them above 1.03 (2048 x 3584 x 18944 230 us, the library 358; 12001 rows
+        1144, 1528). Not where the library's own tiles of 256 x 256 are one or two rounds all but whole, which it runs at 1.4 to 1.55 PFLOP/s (37 such
+        products, 1.07 of its time in the geometric mean: 4608 x 3584 x 18944 450 us, 404), nor several rounds of tiles of 128 x 256, which
+        reach 1.1 to 1.2 (17 products, 0.68 to 1.19: 6889 x 3584 x 18944 803 us, 692); with 0.4 to 0.6 of the rounds real up to 1.19, with less up to 3. At K up to 16384 the library's choice is as often
         as not the faster one (0.57 to 1.24 of its time over 300 products of whole rounds, 0.98 in the geometric mean), and beyond K 27648 too
         (8192 x 29568 up to 1.24). Only where a part allows it (one_round_tiles): the library adds some tiles of such a product in
         two halves, so 6 results in 10,000 differ in their last bit, which a router over rows that no norm has evened out turns into
@@ -252,7 +254,8 @@ class Linear:
         N, K = self.weight.shape
         return not library_tuning.enabled() and self.one_round_tiles and out_dtype == BF16 and 16384 < K <= 27648 and K % 64 == 0 \
             and N % 4 == 0 and x.is_contiguous() and out.is_contiguous() and self.weight.is_contiguous() and ops.tiles_read(x, self.weight, out) \
-            and self._tile_fill(rows)[1] >= 0.7
+            and self._tile_fill(rows)[1] >= 0.7 and not (0.925 <= self._rounds(rows, 256) <= 1 or 1.93 <= self._rounds(rows, 256) <= 2) \
+            and (self._rounds(rows, 128) <= 1 or ops.gemm_tall_tile(rows, N, K) != (128, 256))
 
     def _few_tiles(self, rows: int, x, out, out_dtype) -> int:
         """The tile (kernels.ops.few_tiles_tile) of a product whose tiles are one round of the chip, 0 where the library runs it: tiles of
