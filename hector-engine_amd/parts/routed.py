@@ -158,6 +158,19 @@ class RoutedExperts(FeedForward):
         return (ctx.env.fast_kernels and ctx.env.dtype == torch.bfloat16 and self.gate_up.weight.dtype == torch.bfloat16
                 and self.inter % 8 == 0 and self.shared_cols % 8 == 0 and self.hidden % 8 == 0 and 2 * rows * self.top <= self.real)
 
+    def _leaves_out(self, rows: int) -> tuple[bool, bool]:
+        """Whether the products over all experts of a step of up to 16 bfloat16 rows, the first and the second, leave out the experts that
+        nobody chose (routed_act gives exact zeros for those). Every workgroup asks for the choice before its weights, 2 us and more a
+        product: 1.04 to 1.3 of its time where every expert is chosen. So only where the experts expected without a row (`top` even among the
+        outputs) are a quarter and 80 MB of the first product's weights, in rows of 1024 and more, and a fifth of 50 MB and more of the
+        second's (whose groups of k are no shorter than 512, a turn of the kernel's walk). Over 13,700 random sizes with weights from
+        memory (4 to 64 experts of 256 to 4096, 2 to 16 rows of 512 to 4096) the 1731 first products that this takes need 0.78 of the time of
+        the whole ones in the geometric mean, 5 of them 1.03 to 1.07, the 3236 second ones 0.85, none above 1.03; all others 1.12 and 1.04 of it. 4 rows
+        of 2048, 4 chosen of 16 experts of 2048: 49.3 us and 41.5, 33.5 and 29.9."""
+        unused = (1 - self.top / (self.real + self.identity)) ** rows
+        mb = 2e-6 * self.real * self.inter * self.hidden
+        return (self.hidden >= 1024 and unused >= 0.25 and unused * 2 * mb >= 80, self.inter >= 512 and unused >= 0.2 and mb >= 50)
+
     def _many_rows(self, rows: int, x, ctx: StepContext) -> int:
         """The rows a tile has where the step runs expert by expert over the rows that chose it (kernels.ops.routed_groups),
         0 where it runs through the products over all experts. For bfloat16 with the fast kernels, sizes in multiples
@@ -276,12 +289,12 @@ class RoutedExperts(FeedForward):
         if bm:
             return self._by_expert(x, dense, ids, weights, rows, bm, act, ctx)
         if rows <= _ROW_CHUNK:
-            # up to 16 rows the products leave out the experts that nobody chose (routed_act gives exact zeros for those)
-            gu = self.gate_up(given, rows, ctx, used=(dense, real, 2 * I, False))
+            first, second = self._leaves_out(rows)
+            gu = self.gate_up(given, rows, ctx, used=(dense, real, 2 * I, False) if first else None)
             h = ctx.alloc((rows, cols))
             ops.routed_act(h, gu, dense, x if self.identity else None, rows, real, I, shared=S, **act)
             return self.down(h, rows, ctx, sink=ctx.take_sink() if may_sink else None,
-                             used=(dense, real, I, True) if I >= 512 else None)
+                             used=(dense, real, I, True) if second else None)
         out = ctx.alloc((rows, self.hidden))
         for r0 in range(0, rows, _ROW_CHUNK):
             n = min(_ROW_CHUNK, rows - r0)

@@ -147,6 +147,35 @@ def test_which_routed_steps_run_expert_by_expert(sizes, tiles):
     assert {rows: part._many_rows(rows, empty(rows, sizes["hidden"]), CTX) for rows in tiles} == tiles
 
 
+@pytest.mark.parametrize("sizes,left_out", [
+    (dict(real=16, top=4, inter=2048, hidden=2048), {3: (True, True), 4: (True, True), 5: (False, True), 6: (False, False), 16: (False, False)}),
+    (dict(real=16, top=4, inter=2048, hidden=768), {4: (False, True), 8: (False, False)}),       # short rows: the first product's check costs more
+    (dict(real=40, top=4, inter=448, hidden=3072), {7: (True, False), 16: (False, False)}),      # groups of k shorter than a turn of the walk
+    (dict(real=4, top=2, inter=1664, hidden=704), {2: (False, False), 11: (False, False)}),      # small weights; every expert chosen
+    (dict(real=14, top=4, inter=2048, hidden=2048, identity_experts=2), {4: (False, True)})])
+def test_which_steps_of_few_rows_leave_out_experts(monkeypatch, sizes, left_out):
+    """Where the experts that nobody is expected to choose are enough bytes for what the check costs."""
+    part, took = experts(**sizes), []
+
+    class Product:
+        weight = empty(8, 8)
+
+        def own_tiles(self, rows, ctx):
+            return False
+
+        def __call__(self, x, rows, ctx, sink=None, used=None):
+            took.append(used is not None and used[1:])
+    part.router, part.gate_up, part.down = empty(18, sizes["hidden"], dtype=torch.float32), Product(), Product()
+    for name in ("route_tokens", "routed_act"):
+        monkeypatch.setattr(ops, name, lambda *a, **k: None)
+    for rows, want in left_out.items():
+        took.clear()
+        ctx = SimpleNamespace(env=CTX.env, rows=rows, alloc=lambda shape, dtype=BF16: empty(*shape, dtype=dtype))
+        part._routed(empty(rows, sizes["hidden"]), ctx, False)
+        real, inter = sizes["real"], sizes["inter"]
+        assert took == [want[0] and (real, 2 * inter, False), want[1] and (real, inter, True)], rows
+
+
 @pytest.mark.parametrize("M,N,K,tile", [
     (2048, 3584, 18944, (128, 224)), (12001, 3584, 18944, (256, 224)),        # 256 tiles, 752: one round, three of the shorter ones
     (2048, 37888, 3584, (256, 256)), (203, 37888, 3584, (256, 160)), (100, 37888, 3584, (128, 160)),

@@ -164,6 +164,19 @@ def test_experts_over_the_rows_that_chose_them(monkeypatch, form, turns):
         assert torch.equal(part.forward(x, context(rows)), both)
 
 
+@pytest.mark.parametrize("form", [{}, {"identity_experts": 2}, {"shared": {"feed_forward": PartSpec("gated_mlp", {"hidden_size": 1024, "intermediate_size": 1088})}}])
+@pytest.mark.parametrize("rows", [3, 5])
+def test_experts_that_nobody_chose_are_left_out(monkeypatch, form, rows):
+    """A step of few rows at sizes whose rule leaves them out of both products: the bits of the products over all experts."""
+    part = bound_part("routed_experts", {"hidden_size": 1024, "intermediate_size": 1088, "experts": 64, "top": 12, "correction": False, **form},
+                      1024 ** -0.5)
+    x = rnd(rows, 1024, seed=94)
+    assert part._leaves_out(rows) == (True, True) and not part._few_rows(rows, x, context(rows))
+    out = part._routed(x, context(rows), False)
+    monkeypatch.setattr(part, "_leaves_out", lambda rows: (False, False))
+    assert torch.equal(out, part._routed(x, context(rows), False))
+
+
 @pytest.mark.parametrize("act,params,fn,shift,limit,consts", [
     ("silu", {}, *SILU, (1.0, 0.0, 0.0, 0.0)),
     ("clamped_swiglu", {"limit": 1.5}, lambda g: g * torch.sigmoid(1.702 * g), 1.0, 1.5, (1.702, 1.5, 1.0, 0.0))])
