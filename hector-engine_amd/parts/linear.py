@@ -229,15 +229,15 @@ class Linear:
             slices //= 2
         return slices
 
-    def _tile_fill(self, rows: int) -> tuple[float, float]:
-        """Of the tile gemm_tall_tile chooses: the share of its rounds of the chip that has tiles, and that has real outputs (none of no rows)."""
+    def _tile_fill(self, rows: int, slices: int = 1) -> tuple[float, float]:
+        """Of the tile gemm_tall_tile chooses (for so many K slices): the share of its rounds of the chip that has tiles, and that has real outputs (none of no rows)."""
         if rows == 0:
             return 0.0, 0.0
         N, K = self.weight.shape
-        bm, bn = ops.gemm_tall_tile(rows, N, K)
-        tiles, cus = -(-rows // bm) * -(-N // bn), ops.compute_units()
+        bm, bn = ops.gemm_tall_tile(rows, N, K, slices)
+        tiles, cus = -(-rows // bm) * -(-N // bn) * slices, ops.compute_units()
         places = -(-tiles // cus) * cus
-        return tiles / places, rows * N / (places * bm * bn)
+        return tiles / places, rows * N * slices / (places * bm * bn)
 
     def _long(self, rows: int, x, out, out_dtype) -> bool:
         """Whether a product of long K runs in tiles of this library's own (kernels.ops.gemm_tall): for K from 16448 to 27648, where
@@ -256,6 +256,17 @@ class Linear:
             and N % 4 == 0 and x.is_contiguous() and out.is_contiguous() and self.weight.is_contiguous() and ops.tiles_read(x, self.weight, out) \
             and self._tile_fill(rows)[1] >= 0.7 and not (0.925 <= self._rounds(rows, 256) <= 1 or 1.93 <= self._rounds(rows, 256) <= 2) \
             and (self._rounds(rows, 128) <= 1 or ops.gemm_tall_tile(rows, N, K) != (128, 256))
+
+    def _slices_in_tiles(self, rows: int, slices: int, x) -> bool:
+        """Whether the K slices of a product of up to 512 rows (_library_slices) run in this library's own tiles: more than 2048 columns, and
+        tiles for 0.7 of a round of the chip or more. Over 90 products that this takes 0.67 to 1.04 of the batched product's time and its sum,
+        0.89 in the geometric mean (203 x 3584 x 18944 45.9 us beside 48.8 without the sum); of 70 others 0.65 to 1.86, 1.06 in the
+        mean (128 x 2048 x 27648 49.7 and 38.3, 292 x 2048 x 8192 27.0 and 24.5, 78 x 496 x 27648 38.6 and 20.8). Only where a part allows it
+        (see _long): of 310 products of 65 to 512 rows 295 had the library's bits, 15 of some widths (768 x 16384 at 65 rows,
+        2192 x 28672 at 128) 3 results in 10,000 that differ in their last bit."""
+        N, K = self.weight.shape
+        return self.one_round_tiles and not library_tuning.enabled() and N > 2048 and N % 4 == 0 and K % (64 * slices) == 0 \
+            and self.weight.is_contiguous() and ops.tiles_read(x, self.weight) and self._tile_fill(rows, slices)[0] >= 0.7
 
     def _few_tiles(self, rows: int, x, out, out_dtype) -> int:
         """The tile (kernels.ops.few_tiles_tile) of a product whose tiles are one round of the chip, 0 where the library runs it: tiles of
@@ -291,12 +302,7 @@ class Linear:
         if slices > 1:
             N, K = w.shape
             partial = ctx.alloc((slices, rows, N), torch.float32)
-            if self.one_round_tiles and K % (64 * slices) == 0 and N % 4 == 0 and w.is_contiguous() and ops.tiles_read(x, w) \
-                    and not library_tuning.enabled():
-                # the same slices in this library's own tiles, over 35 products of 70 to 512 rows 0.57 to 1.03 of the
-                # batched product's time, 0.89 in the geometric mean (203 x 3584 x 18944 45.9 us beside 48.8, 128 x 2048 x 8192 17.8 beside
-                # 31.1). Only where a part allows it (see _long): of 310 products of 65 to 512 rows 295 had the library's bits, 15 of some
-                # widths (768 x 16384 at 65 rows, 2192 x 28672 at 128) 3 results in 10,000 that differ in their last bit
+            if self._slices_in_tiles(rows, slices, x):
                 bm, bn = ops.gemm_tall_tile(rows, N, K, slices)
                 ops.gemm_tall(partial, x, w, None, rows, bm=bm, bn=bn, slices=slices)
                 ops.splitk_reduce(out, partial, bias, rows, slices)

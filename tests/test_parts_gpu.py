@@ -272,7 +272,7 @@ def test_a_kernel_route_registered_from_outside_is_the_one_that_runs(fw):
 
 
 @pytest.mark.parametrize("rows", [65, 200, 512, 513])
-@pytest.mark.parametrize("N,K,bias", [(72, 8192, True), (300, 9024, False), (40, 8200, True)])
+@pytest.mark.parametrize("N,K,bias", [(72, 8192, True), (300, 9024, False), (40, 8200, True), (2120, 8192, True)])
 @pytest.mark.parametrize("own", [False, True])
 def test_a_long_k_product_in_slices_through_the_library(fw, rows, N, K, bias, own):
     """More than 64 rows against a weight with a long K and few output columns (a down projection):

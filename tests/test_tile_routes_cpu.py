@@ -87,7 +87,7 @@ def test_a_shared_expert_keeps_the_library_s_sums():
 
 def test_k_slices_in_tiles_are_for_parts_that_allow_them(monkeypatch):
     """The experts' down product beside a shared expert is such a weight: its slices stay the library's, whose bits the tiles do not always give."""
-    ran, N, K, rows = [], 2048, 32768, 300
+    ran, N, K, rows = [], 3584, 18944, 200
     for module, name in ((ops, "gemm_tall"), (ops, "splitk_reduce"), (torch, "bmm")):
         monkeypatch.setattr(module, name, lambda *a, name=name, **k: ran.append(name))
     ctx = SimpleNamespace(env=CTX.env, alloc=lambda shape, dtype=BF16: empty(*shape, dtype=dtype))
@@ -97,6 +97,17 @@ def test_k_slices_in_tiles_are_for_parts_that_allow_them(monkeypatch):
         lin.one_round_tiles = allowed
         lin._library(empty(rows, K), None, rows, empty(rows, N), BF16, ctx)
     assert ran == ["bmm", "splitk_reduce", "gemm_tall", "splitk_reduce"]
+
+
+@pytest.mark.parametrize("N,K,rows", [(3584, 18944, {65: True, 203: True, 257: True, 512: True}), (5120, 27648, {66: True, 380: True}),
+                                      (2560, 14336, {97: False, 139: True, 262: True}),                  # half of the units
+                                      (2048, 27648, {66: False, 128: False, 292: False}), (1024, 14336, {208: False}), (496, 27648, {78: False}),
+                                      (3584, 18912, {203: False}), (3586, 18944, {203: False})])
+def test_which_k_slices_run_in_tiles(N, K, rows):
+    """At 256 units: more than 2048 columns, tiles for 0.7 of a round or more."""
+    lin = Linear(empty(N, K))
+    lin.one_round_tiles = True
+    assert {r: lin._slices_in_tiles(r, lin._library_slices(r), empty(r, K)) for r in rows} == rows
 
 
 def test_operands_the_tiles_do_not_read_stay_with_the_library():
