@@ -592,26 +592,46 @@ int he_gemm_plain_rounds(float* C, const float* A, const float* W, const void* b
                          int64_t ldw, int64_t ldc, hipStream_t s);
 float he_gemm_plain_rounds_estimate(int M, int N);
 
-// More rows: tiles on the matrix cores. Rows that begin at 16-byte boundaries with K in 32s go to gemm_plain_rounds.hip, whose tiles have
-// 128 rows, unless so many of those are padding that its estimate is above this kernel's time, 4.5 ps an output
-// and k of the fullest unit (130 rows of 37888 x 3584 602 us there, 470 here; over 12 weights and 65 to 3001 rows the kernel there takes
-// 0.56 to 1.06 of the time where it is taken, 0.85 in the geometric mean). Here, of the tile sizes the one whose fullest compute unit has the least to do
-// (a unit's workgroups share its matrix cores, so its time is the outputs dealt to it); the larger tile where
-// they tie, as it reads fewer operands an output.
+// The tile of this file's kernel: of its sizes the one whose fullest compute unit has the least to do (a unit's workgroups share its
+// matrix cores, so its time is the outputs dealt to it); the larger tile where they tie, as it reads fewer operands an output.
+struct GpTile {
+  int bm, bn;
+  int64_t tiles, most;        // outputs of the fullest unit
+};
+static GpTile gp_tile(int M, int N) {
+  GpTile best = {};
+  const int sizes[3][2] = {{128, 128}, {128, 64}, {64, 64}};
+  for (auto& size : sizes) {
+    const int64_t tiles = (int64_t)((M + size[0] - 1) / size[0]) * ((N + size[1] - 1) / size[1]);
+    const int64_t most = (tiles + he_cus() - 1) / he_cus() * size[0] * size[1];
+    if (best.bm == 0 || most < best.most) best = {size[0], size[1], tiles, most};
+  }
+  return best;
+}
+
+// Whether the product of rows that begin at 16-byte boundaries goes to gemm_plain_rounds.hip: K in 32s and more than one of its stages (with
+// one 700 x 288 x 32 takes 5.4 us there, 4.5 here), unless so many rows of its tiles of 128 are padding that its estimate is above this file's
+// kernel's time, 4.5 ps an output and k of the fullest unit (130 rows of 37888 x 3584 602 us there, 470 here). wide: four outputs of a row are
+// stored at once; where they are not, single stores outlast the products of a K below 512 (532 x 14083 x 64 31.3 us and 20.5, 946 x 4567 x 160
+// 27.9 and 24.2, 559 x 3297 x 512 27.1 and 26.4). Over 227 products of 33 to 4000 rows, 16 to 30000 columns and K 32 to 20000 the 206 that are
+// not refused by these two lines take 0.62 to 1.04 of the time with this file's kernel alone.
+extern "C" int he_gemm_plain_in_rounds(int M, int N, int K, int wide) {
+  return K % 32 == 0 && K >= 64 && (wide || K >= 512) && he_gemm_plain_rounds_estimate(M, N) <= 4.5e-6f * gp_tile(M, N).most;
+}
+
+// More rows: tiles on the matrix cores.
 static int launch_mfma(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K,
                        int64_t lda, int64_t ldw, int64_t ldc, hipStream_t s) {
   const int vec = (lda & 3) == 0 && (ldw & 3) == 0 && (((uintptr_t)A) & 15) == 0 && (((uintptr_t)W) & 15) == 0;
-  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  auto most = [&](int bm, int bn) { return (tiles(bm, bn) + he_cus() - 1) / he_cus() * bm * bn; };
-  int bm = 128, bn = 128;
-  if (most(128, 64) < most(bm, bn)) bn = 64;
-  if (most(64, 64) < most(bm, bn)) bm = 64, bn = 64;
   // (lda, ldw: a lane's offsets into a tile's rows are 32-bit)
-  if (vec && K % 32 == 0 && lda < (1 << 22) && ldw < (1 << 22) && he_gemm_plain_rounds_estimate(M, N) <= 4.5e-6f * most(bm, bn))
+  if (vec && lda < (1 << 22) && ldw < (1 << 22) &&
+      he_gemm_plain_in_rounds(M, N, K, (ldc & 3) == 0 && (N & 3) == 0 && ((uintptr_t)C & 15) == 0))
     return he_gemm_plain_rounds(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc, s);
-  HE_REQUIRE(tiles(bm, bn) < (1 << 30), "he_gemm_plain: M=%d N=%d too large for one launch", M, N);
+  const GpTile tile = gp_tile(M, N);
+  const int bm = tile.bm, bn = tile.bn;
+  HE_REQUIRE(tile.tiles < (1 << 30), "he_gemm_plain: M=%d N=%d too large for one launch", M, N);
   const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
-  const int grid = (int)((tiles(bm, bn) + HE_XCDS - 1) / HE_XCDS * HE_XCDS);
+  const int grid = (int)((tile.tiles + HE_XCDS - 1) / HE_XCDS * HE_XCDS);
 #define GP_MFMA(BM_, BN_) \
   gemm_plain_mfma_kernel<BM_, BN_><<<grid, 256, 0, s>>>(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc, mt, nt, vec)
   if (bn == 128) GP_MFMA(128, 128);

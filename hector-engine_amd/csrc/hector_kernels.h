@@ -70,6 +70,8 @@ int he_rmsnorm_row_pair(void* x, const void* w1, int D1, const void* w2, int D2,
 // at 16 bytes) a product of few rows runs through kernels made for it; the
 // result is the same bit for bit. in_dtype, out_dtype < 0: the most that any operands take.
 int64_t he_gemm_plain_workspace_floats(int M, int N, int K, int in_dtype, int out_dtype, int aligned);
+// Whether a 32-bit product of many aligned rows runs in tiles that are whole rounds of the chip (wide: rows of results that are stored in fours).
+int he_gemm_plain_in_rounds(int M, int N, int K, int wide);
 int he_gemm_plain(void* C, const void* A, const void* W, const void* bias, int M, int N, int K,
                   int64_t lda, int64_t ldw, int64_t ldc, int in_dtype, int out_dtype,
                   int bias_dtype, void* workspace_f32, int64_t workspace_floats, void* stream);

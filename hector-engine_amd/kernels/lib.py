@@ -35,6 +35,7 @@ _SIGNATURES = {
     "he_add_rmsnorm": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_f32, c_int, c_int, c_ptr],
     "he_rmsnorm_rows": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_i64, c_i64, c_f32, c_int, c_int, c_ptr],
     "he_gemm_plain_workspace_floats": [c_int, c_int, c_int, c_int, c_int, c_int],
+    "he_gemm_plain_in_rounds": [c_int, c_int, c_int, c_int],
     "he_gemm_plain": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_i64, c_i64, c_i64,
                       c_int, c_int, c_int, c_ptr, c_i64, c_ptr],
     "he_gemm_blocksplit_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_int,

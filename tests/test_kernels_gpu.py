@@ -1271,7 +1271,8 @@ def test_blocksplit_leaves_out_groups_of_rows(ops, M, K, count, size, extra):
 # (8 row tiles: every width from 16 to 144; columns that end inside a tile and inside four; several tiles a workgroup; a single stage, a
 # segment that ends early, more stages than are in flight; few rows, whose other kernel has tiles of 64)
 @pytest.mark.parametrize("M,N,K", [(1003, n, 160) for n in (512, 1024, 1533, 2048, 2560, 3070, 3584, 4096, 4607)] +
-                         [(65, 300, 32), (129, 9000, 96), (1003, 20001, 128), (2050, 5124, 384), (200, 4608, 3584), (66, 1, 256)])
+                         [(65, 300, 32), (129, 9000, 96), (1003, 20001, 128), (2050, 5124, 384), (200, 4608, 3584), (66, 1, 256),
+                          (1003, 1533, 544), (700, 4607, 512), (66, 1, 640)])
 def test_plain_products_in_whole_rounds_give_the_bits_of_the_other_kernels(ops, M, N, K):
     a, w, b = dev(rnd(M, K, seed=1)), dev(rnd(N, K, seed=2)), dev(rnd(N, seed=3))
     out = torch.full((M + 1, N), 7.0, device="cuda")

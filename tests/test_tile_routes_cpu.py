@@ -240,3 +240,14 @@ def test_which_products_of_long_k_run_in_tiles_of_many_rounds(N, K, rows):
     lin.one_round_tiles = True
     assert {r: lin._long(r, empty(r, K), empty(r, N), BF16) for r in rows} == rows
     assert not any(lin._long(r, empty(r, K), empty(r, N, dtype=torch.float32), torch.float32) for r in rows)
+
+
+@pytest.mark.parametrize("M,N,K,taken", [
+    (1003, 3584, 18944, True), (2048, 37888, 3584, True), (130, 37888, 3584, False),      # 126 of the second row of tiles are padding
+    (700, 288, 32, False), (305, 3400, 64, True),                                         # one stage; two
+    (532, 14083, 64, False), (946, 4567, 160, False), (1096, 989, 544, True),             # rows of results that are stored one by one
+    (1003, 3584, 18948, False)])
+def test_which_32_bit_products_run_in_whole_rounds(M, N, K, taken):
+    """At 256 units, rows that begin at 16-byte boundaries."""
+    from hector_engine_amd.kernels import lib
+    assert lib.load().he_gemm_plain_in_rounds(M, N, K, int(N % 4 == 0)) == taken
