@@ -396,11 +396,10 @@ class Linear:
         """The rows of a tile where the gated product of this many bf16 rows runs as one kernel (kernels.ops.gemm_tall), 0 where it
         is the library's product and an activation kernel. One kernel for K up to 1024 where its tiles are one round on the
         chip: of 128 rows from 0.6 of a round on, of 256 where those are more than a round and 0.7 of the round's outputs are
-        real. Over 220 random weights and row counts that this takes, 0.34 to 1.01 of the time of the two, 0.72 in the geometric mean
-        (8192 x 1024 at 1000 rows 24.8 us beside 28.1, 9728 x 896 at 768 rows 23.7 beside 27.0, at 1400 38.8 beside 40.3). With fewer
-        tiles units idle (1024 x 256 at 1000 rows 13.0, 9.1); with more, or a longer K, the two come out ahead as often as not,
-        by the library's choice of a kernel alone: over 420 random weights of K 1536 to 8192 and 1000 to 6000 rows the one
-        kernel took 0.66 to 1.31 of their time, in no relation to rows, columns or rounds."""
+        real. Over 4879 random weights and row counts that this takes, 0.48 to 1.21 of the time of the two, 0.70 in the geometric mean, 22
+        above 1.03, those of some 150 to 320 rows whose second row of tiles is mostly padding (8192 x 1024 at 1000 rows 27.2 us beside 31.6,
+        9728 x 896 at 768 rows 22.5 beside 24.9, at 1400 36.4 beside 36.8; 29824 x 704 at 149 rows 1.21). With fewer tiles units idle (1024 x 256 at
+        1000 rows 12.7, 8.0)."""
         N, K = self.weight.shape
         if not (K <= 1024 and isinstance(x, torch.Tensor) and x.dtype == BF16 and x.is_contiguous() and K % 64 == 0 and N % 8 == 0
                 and ops.tiles_read(x, self.weight) and self.own_tiles(rows, ctx)) or library_tuning.enabled():
@@ -409,11 +408,11 @@ class Linear:
             return 128 if self._rounds(rows, 128) >= 0.6 else 0
         return 256 if self._rounds(rows, 256) <= 1 and rows * N >= 0.7 * 256 * 256 * ops.compute_units() else 0
 
-    def _tile_with_activation(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
-        """The tile (ops.gemm_tall's bm, bn) where a product of this many bf16 rows with K above 1024 takes the activation of its results
-        along, None where it is the library's product and an activation kernel: one kernel where the tiles of gemm_tall_tile's choice are
-        0.8 of their rounds or more, and either one row of tiles, which read the weight once whatever of their rows is padding, or 0.72 of
-        the rounds real outputs. Over 198 gated products of 65 to 12001 rows, 256 to 55296 columns and K up to 20000 it took 0.71 to
+    def gated_tile(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
+        """The tile (ops.gemm_tall's bm, bn) where a gated product of this many bf16 rows with K above 1024 (up to 1024: tall_gated), or one
+        with a relu, runs as one kernel, None where it is the library's product and an activation kernel: one kernel where the tiles of
+        gemm_tall_tile's choice are 0.8 of their rounds or more, and either one row of tiles, which read the weight once whatever of
+        their rows is padding, or 0.72 of the rounds real outputs. Over 198 gated products of 65 to 12001 rows, 256 to 55296 columns and K up to 20000 it took 0.71 to
         1.09 of the time of the two, 0.90 in the geometric mean, 3 of them above 1.03 (2048 x 37888 x 3584 424 us beside 546, 203 rows 73
         beside 85, 100 rows 58 beside 71); with several rows of tiles and less of them real 0.77 to 1.24 (259 x 28672 x 4096 100 us, the two 82,
         541 x 37888 x 2048 106 and 98), with tiles for less than 0.8 of the rounds up to 1.48. Only where a part allows it (one_round_tiles): see _long."""
@@ -425,10 +424,6 @@ class Linear:
         tile, (tiles, real) = ops.gemm_tall_tile(rows, N, K), self._tile_fill(rows)
         return tile if tiles >= 0.8 and (rows <= tile[0] or real >= 0.72) else None
 
-    def gated_tile(self, rows: int, ctx: StepContext, x) -> tuple[int, int] | None:
-        """The tile where the gated product of this many rows runs as one kernel, None where it does not (K up to 1024: tall_gated)."""
-        return self._tile_with_activation(rows, ctx, x)
-
     def activated(self, x, rows: int, ctx: StepContext, kind: str):
         """unary_act(kind) of the product as one kernel, None where the caller runs the two: up to 16 rows for any kind, many rows
         for the relu ones."""
@@ -439,7 +434,7 @@ class Linear:
             out = ctx.alloc((rows, self.weight.shape[0]), act)
             ops.gemm_blocksplit(out, a, self.weight, self.bias, rows, row_scale=scale, x_pieces=pieces, unary=kind)
             return out
-        tile = self._tile_with_activation(rows, ctx, x) if kind in ("relu2", "relu") else None
+        tile = self.gated_tile(rows, ctx, x) if kind in ("relu2", "relu") else None
         if tile is None:
             return None
         out = ctx.alloc((rows, self.weight.shape[0]), act)

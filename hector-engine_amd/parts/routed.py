@@ -191,11 +191,14 @@ class RoutedExperts(FeedForward):
         """Microseconds the experts of so many rows are expected to take: by expert in tiles of 128 and of 256 rows, and as products over
         all experts. A round of tiles on the chip costs a start and its stages of 64 k, an expert has whole tiles however few rows
         chose it, every choice's part of the sum is written and read in 32 bits, and sorting takes a nanosecond a choice; the
-        library's products cost their operations or their weights' bytes. Fitted to 7116 random sizes (2 to 256 experts of 64 to
-        4096, 65 to 4096 rows of 256 to 7168), on which the three are off by a sixth (standard deviation). With the factor 0.8 the 2586
-        of these that go by expert take 0.38 of the other form's time in the geometric mean (0.68 beside a shared expert), 15 of them 1.03
-        to 1.14 of it: 16 experts of 2048 over rows of 2048, 4 chosen, 65 rows 120 us beside 114, 512 153 beside 211, 2048 354 beside 851.
-        Few or small experts are left to the other form: 2 of 64 over 224 rows of 1728, 1 chosen, 13 us beside 43."""
+        library's products cost their operations or their weights' bytes. The numbers were fitted with the tile kernel that had eight
+        wavefronts; with the one there is they are 1.03 and 1.04 of what by-expert steps take (0.9 beside a shared expert) and 0.92 of the products
+        over all, each off by a fifth (standard deviation over 2709 random sizes, 2 to 256 experts of 64 to 4096, 65 to 4096 rows of 256
+        to 7168). With the factor 0.8 the 1403 of these that go by expert take 0.43 of the other form's time in the geometric mean, 5 of
+        them 1.03 to 1.05 (beside a shared expert 1323, 0.72, 4 of them 1.03 to 1.11), in tiles that are 1.006 of the better of the
+        two heights: 16 experts of 2048 over rows of 2048, 4 chosen, 65 rows 118 us beside 115, 512 150 beside 220, 2048 318 beside 874.
+        Few or small experts are left to the other form: 2 of 64 over 224 rows of 1728, 1 chosen, 13 us beside 44; 201 of the 1306 left would
+        be below 0.8 by expert."""
         D, I, real = self.hidden, self.inter, self.real
         choices, cus = rows * self.top, ops.compute_units()
 
