@@ -26,6 +26,14 @@ struct bf16_t {
   uint16_t v;
 };
 
+// 16 bytes that nothing else of the launch reads, in loads of whole lines: the caches may drop them first.
+typedef uint32_t he_uint4v __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ T he_load16_once(const void* p) {
+  static_assert(sizeof(T) == 16, "16 bytes");
+  return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const he_uint4v*>(p)));
+}
+
 __device__ __forceinline__ float bf16_bits_to_float(uint16_t b) {
   return __uint_as_float(((uint32_t)b) << 16);
 }

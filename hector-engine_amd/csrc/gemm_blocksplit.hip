@@ -1,14 +1,12 @@
 // bf16 matrix product for few rows (M <= 32) with K cut inside the workgroup:
 // C[M,N] = X[M,K] * W[N,K]^T (+ bias), or the gated activation of a gate||up
-// weight. One workgroup owns up to 16*R weight rows (the rows are dealt out evenly over the
-// compute units, see blocksplit_plan); its NW wavefronts take one K slice
-// each (operands straight from global memory into the MFMA registers, in the operand
-// layout gemm_rows.hip describes), leave their fp32
-// tiles in LDS, and the workgroup adds the slices in wavefront order and writes
+// weight. One workgroup owns up to 32 weight rows (blocksplit_plan); its NW wavefronts take one K slice
+// each (operands straight from global memory into the MFMA registers, laid out so that the weight is read in whole lines, see
+// BsLanes), leave their fp32 sums in LDS, and the workgroup adds the slices in wavefront order and writes
 // the result. The sum is complete inside one launch: no partial sums in global
 // memory, no second kernel, no atomics, and the order of the additions is fixed.
-// With 16 wavefronts a product as small as 3584 x 3584 still puts 3584
-// wavefronts on the chip.
+// What bounds it: the weight's way from memory (6.1 to 6.8 TB/s at 37888 x 3584 and more), and for small products the launch and one
+// trip to memory: nothing is read ahead of the first weights, and what the epilogue reads is asked for behind them.
 //
 // Gated epilogue: the weight alternates gate and up rows (gate i at row 2i, its up at
 // 2i + 1), so the four neighbouring weight rows whose sums a thread holds are two
@@ -26,9 +24,8 @@
 //
 // Activations between two such products may lie piece-major instead of row-major: a [M, D]
 // bf16 tensor as 16-byte pieces [D / 8][M][8], element (m, d) at ((d / 8) M + m) 8 + d % 8.
-// The 16 lanes of an activation operand load then read 16 neighbouring pieces (two lines)
-// instead of 16 rows (16 lines): the cost of the activation rows, which grows with their
-// number (gate||up 48 us at 1 row, 50 at 8, 59 at 16), all but goes (49 and 55 us). The
+// The lanes of an activation operand load then read neighbouring pieces (whole lines)
+// instead of one piece of a line in each row. The
 // producing epilogue writes the layout, the consuming product reads it (x_pieces / out_pieces).
 #include "common.h"
 //
@@ -37,80 +34,86 @@
 #include "gemm_blocksplit_tiles.h"
 
 
-// Tilings measured on MI355X (graph-timed sweeps over R, U and NW at the Qwen2.5-7B, Qwen2.5-32B
-// and Qwen2-72B shapes). The rule depends on the sizes only, so a product always runs the same way.
-// What counts is how many weight rows fall to a compute unit, so the bounds on N are written in
-// rows a unit (on the MI355X's 256 units: 256 a unit = 65536 rows, the output head; 64 a unit =
-// 16384, gate||up; 16 a unit = 4096); the bounds on K are lengths of a weight row.
-static BlockSplitPlan blocksplit_plan(int M, int N, int K, int gated, int R, int U, int NW) {
+// The tiling of a product, from its sizes only, so that it always runs the same way. Swept on MI355X over NA, S, NW and the rows of a
+// workgroup at 20 shapes (896 x 896 to 152064 x 3584 and 5120 x 27648) with 1, 4, 8 and 16 rows, weights from memory: this choice is within 4 % of the best of
+// some 60 tilings at all but the smallest.
+// Weight rows of a workgroup: the multiple of four (outputs are stored in fours; 3584 x 3584 in rows of 14 8.5 us, of 16 7.2) up to 16 or
+// 32 that costs least as rounds of the chip times rows and a start worth four rows, of equal ones the largest (each workgroup reads all of
+// X). 5120 x 27648 at 8 rows in rows of 20 52 us, of 8 or 10 55 to 58; 8512 x 2048 at 1 row in twelves 9.1, in sixteens
+// 9.8; 37888 x 3584 at 16 rows in thirty-twos 49, in eights 86.
+// NW = 8 wavefronts take a K slice each; 4 where that leaves a slice one instruction and the chip has other workgroups to run
+// (151936 x 896 at 4 rows 43 us, with eight 52). A wavefront with a single accumulator asks for two units a step (896 x 4864 at 8 rows 6.0 us, 6.8).
+// plan arguments NA, S, NW <= 0: this choice.
+static BlockSplitPlan blocksplit_plan(int M, int N, int K, int NA, int S, int NW) {
   BlockSplitPlan p;
   const int cus = he_cus();
-  p.MT = (M + 15) / 16;
+  p.SP = M <= 4 ? 2 : M <= 16 ? 1 : 0;
+  p.MT = M <= 8 ? 1 : 2;
+  const int rt = 16 >> p.SP, km = p.SP == 0 ? 64 : 32 << p.SP, units = (K + km - 1) / km;
+  int rows = 0, best = 0;
+  for (int r = p.SP == 2 ? 16 : 32; r >= 4; r -= 4) {
+    const int blocks = (N + r - 1) / r, cost = (blocks + cus - 1) / cus * (r + 4);
+    if (rows == 0 || cost < best) best = cost, rows = r;
+  }
+  p.NA = rows <= rt ? 1 : rows <= 2 * rt ? 2 : 4;
+  if (NA > 0) p.NA = NA, rows = rt * NA;
+  p.S = S > 0 ? (S > 1 ? 2 : 1) : p.NA == 1 ? 2 : 1;
+  p.rows_per_block = rows;
+  if (NW <= 0) {
+    NW = units < 16 && N >= 2 * cus * rows ? 4 : 8;
+    while (NW > 1 && 2 * units <= NW) NW >>= 1;
+  }
+  if (NW > bs_max_waves(p.MT, p.NA, p.S)) NW = bs_max_waves(p.MT, p.NA, p.S);
+  p.NW = NW;
+  p.units = (units + NW - 1) / NW;
+  p.turn = p.S;
+  return p;
+}
+
+// The tiling of the ordered sums of up to 16 rows: tiles, K slices and turns of 128 u k as this product had them before its lanes
+// were spread. For weights whose results reach a router over rows that no norm has evened out: there another order of sums turns
+// near ties over.
+static BlockSplitPlan ordered_plan(int M, int N, int K) {
+  BlockSplitPlan p;
+  const int cus = he_cus();
+  p.SP = 0, p.MT = 1;
   int r, u, nw;
-  if (N >= 256 * cus) {             // 256 rows or more a unit: the output head
+  if (N >= 256 * cus) {             // 256 rows or more a unit
     if (M <= 8) r = 2, u = 1, nw = 8;
-    else if (p.MT == 1) r = 4, u = 2, nw = 4;
-    else r = 2, u = 2, nw = 4;
+    else r = 4, u = 2, nw = 4;
   } else if (K >= 8192) {           // long K
     const int groups = (N + 31) / 32, last_round = groups % cus;   // with two tiles a workgroup
-    if (N < 16 * cus) {             // few weight rows: one tile a workgroup, or the chip is not filled
-      r = 1, u = 1, nw = p.MT == 1 ? 8 : 4;
-    } else if (p.MT == 2) {
-      r = 2, u = 2, nw = 4;
-    } else if (M > 8 && N >= 40 * cus) {
-      r = 4, u = 2, nw = 4;         // the activation rows are read half as often
-    } else if (groups < cus) {
-      r = 2, u = 1, nw = 8;         // under one workgroup a compute unit: more wavefronts each
-    } else if (groups < 4 * cus && last_round > 0 && last_round <= cus / 2) {
-      r = 1, u = 1, nw = 8;         // the last round of whole tiles would fill under half of the chip:
-                                    // the rows are dealt out below, 20 a workgroup for 10240
-    } else if (K >= 16384) {
-      r = 2, u = 2, nw = 8;         // 8192 x 29568 at 8 rows: 85.3 us against 89.2 us for the next line's tiling
-    } else {
-      r = 2, u = 4, nw = 4;
-    }
-  } else if (N >= 64 * cus) {       // wide N (gate||up)
-    r = 2, u = 1, nw = 8;
-    if (p.MT == 2 || K < 5120) u = 2, nw = 4;   // 37888 x 3584 at 8 rows: 47.7 us against 48.5 us
-    else if (M > 8) r = 4;
-  } else {                          // small products (q||k||v, o)
-    r = N >= 16 * cus ? 2 : 1;
-    u = p.MT == 1 && K < 5120 ? 4 : 1;   // 5120 x 5120 at 8 rows: 12.8 us unrolled once, 13.5 us four times
-    nw = 8;
+    if (N < 16 * cus) r = 1, u = 1, nw = 8;
+    else if (M > 8 && N >= 40 * cus) r = 4, u = 2, nw = 4;
+    else if (groups < cus) r = 2, u = 1, nw = 8;
+    else if (groups < 4 * cus && last_round > 0 && last_round <= cus / 2) r = 1, u = 1, nw = 8;
+    else if (K >= 16384) r = 2, u = 2, nw = 8;
+    else r = 2, u = 4, nw = 4;
+  } else if (N >= 64 * cus) {       // wide N
+    r = M > 8 ? 4 : 2, u = 1, nw = 8;
+    if (K < 5120) r = 2, u = 2, nw = 4;
+  } else {                          // small products
+    r = N >= 16 * cus ? 2 : 1, u = K < 5120 ? 4 : 1, nw = 8;
   }
-  // Weight rows are dealt out evenly over the compute units (256 of them: or twice, three times ... 256
-  // workgroups, at most 32 rows each) rather than in whole tiles of 16: 4608 rows as 256
-  // workgroups of 18 rows instead of 144 of 32, the 37888 rows of gate||up as 1280 of 30
-  // instead of 1184 of 32 (4.6 a compute unit). The last tile of such a workgroup is partly
-  // empty. A workgroup's rows are an even number: a gate stays with its up, and outputs can be
-  // stored in pairs. From two rows a unit on: the 896 rows of a small model's down projection as
-  // 224 workgroups of 4 rather than 56 of 16 (896 x 4864 at 8 rows 9.5 -> 7.4 us, 1536 x 8960
-  // 15.4 -> 12.5 us): a tile with four of its sixteen rows in use costs nothing that matters
-  // there, a compute unit without work does.
   int rows = 0;
-  if (R <= 0 && r <= 2 && N >= 2 * cus && N < 256 * cus) {
+  if (r <= 2 && N >= 2 * cus && N < 256 * cus) {      // dealt out evenly over the compute units, an even number each
     const int rounds = (N + cus * 32 - 1) / (cus * 32);
     rows = ((N + cus * rounds - 1) / (cus * rounds) + 1) & ~1;
     r = rows > 16 ? 2 : 1;
   }
-  p.R = R > 0 ? R : r;
-  p.U = U > 0 ? U : u;
-  if (NW <= 0) {
-    NW = nw;
-    while (NW > 1 && K / NW < 128) NW >>= 1;
-  }
-  if (NW > bs_max_waves(p.MT, p.R, p.U)) NW = bs_max_waves(p.MT, p.R, p.U);
-  p.NW = NW;
-  int ks = (K + NW - 1) / NW;
-  p.kslice = (ks + 63) / 64 * 64;
-  p.rows_per_block = rows > 0 ? rows : 16 * p.R;
+  while (nw > 1 && K / nw < 128) nw >>= 1;
+  if (u * (r + 1) > 4 && nw > 8) nw = 8;
+  p.NA = r, p.S = u > 1 ? 2 : 1, p.NW = nw;
+  p.units = ((K + nw - 1) / nw + 63) / 64;
+  p.turn = 2 * u;
+  p.rows_per_block = rows > 0 ? rows : 16 * r;
   return p;
 }
 
 // Workgroups (= partial sums of squares per row) the residual epilogue of this product gives.
 extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
   if (M <= 0 || M > HE_BLOCKSPLIT_MAX_M || N <= 0 || K <= 0) return 0;
-  const BlockSplitPlan p = blocksplit_plan(M, N, K, 0, 0, 0, 0);
+  const BlockSplitPlan p = blocksplit_plan(M, N, K, 0, 0, 0);
   return (N + p.rows_per_block - 1) / p.rows_per_block;
 }
 
@@ -119,7 +122,7 @@ extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
 // bias or gate); resid: the residual epilogue (C is not written; gain, xg, sq_out needed). unary: an activation of one input
 // (he_unary's kinds) of the bf16 results, -1: none: a feed-forward without a gate writes its activations at once (a launch of its
 // own for 18944 of them took 4.7 us beside the product's 26). used: groups of the weight that no row uses are not read (BsFusion):
-// the experts of a routed step that nobody chose.
+// the experts of a routed step that nobody chose. ordered: see ordered_plan.
 extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W,
                                              const void* bias, int M, int N, int K, int out_dtype,
                                              int bias_dtype, int gated, int R, int U, int NW,
@@ -130,7 +133,7 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
                                              float act_alpha, float act_limit, float act_shift, float act_cubic,
                                              float resid_scale, const void* dyt_bias,
                                              const void* dyt_alpha, int unary, const void* used, int used_ld,
-                                             int used_count, int used_rows, int used_k, void* stream) {
+                                             int used_count, int used_rows, int used_k, int ordered, void* stream) {
   HE_REQUIRE((dyt_alpha == nullptr) == (dyt_bias == nullptr), "he_gemm_blocksplit_bf16: Dynamic Tanh needs alpha and bias");
   HE_REQUIRE(M > 0 && M <= HE_BLOCKSPLIT_MAX_M, "he_gemm_blocksplit_bf16: M=%d outside [1, %d]", M,
              HE_BLOCKSPLIT_MAX_M);
@@ -153,7 +156,9 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
                                  (used_rows > 0) != (used_k > 0) && (used_k == 0 || used_k >= 512) &&
                                  (resid == nullptr || used_rows == 0) && (resid != nullptr || out_dtype == HE_BF16)),
              "he_gemm_blocksplit_bf16: groups that are used: up to 16 rows, bf16 results, along the rows or in stretches of 512 k and more");
-  const BlockSplitPlan p = blocksplit_plan(M, N, K, gated, R, U, NW);
+  HE_REQUIRE(!ordered || (M <= 16 && resid == nullptr && R <= 0 && U <= 0 && NW <= 0),
+             "he_gemm_blocksplit_bf16: ordered sums are for up to 16 rows, plan themselves and leave no residual");
+  const BlockSplitPlan p = ordered ? ordered_plan(M, N, K) : blocksplit_plan(M, N, K, R, U, NW);
   HE_REQUIRE(p.NW >= 1 && p.NW <= 16, "he_gemm_blocksplit_bf16: %d wavefronts outside [1, 16]",
              p.NW);
   const int blocks = (N + p.rows_per_block - 1) / p.rows_per_block;
@@ -190,11 +195,12 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
   fu.dyt_bias = dyt_bias;
   fu.dyt_alpha = dyt_alpha;
   hipStream_t s = (hipStream_t)stream;
-  int rc;
-  static int (*const tiles[2][2])(HE_BS_DISPATCH_ARGS) = {
-      {he_blocksplit_tiles_bf16, he_blocksplit_tiles_f32},
-      {he_blocksplit_tiles_gated_bf16, he_blocksplit_tiles_gated_f32}};
-  rc = (used ? he_blocksplit_tiles_used_bf16 : tiles[gated != 0][out_dtype != HE_BF16])(p, C, A, W, bias, bias_dtype, M, N, K, fu, x_pieces != 0, s);
+  const bool f32 = out_dtype != HE_BF16;
+  const int rc = (resid != nullptr ? (used ? he_blocksplit_tiles_used_resid : he_blocksplit_tiles_resid)
+                  : used           ? he_blocksplit_tiles_used_bf16
+                  : gated          ? (f32 ? he_blocksplit_tiles_gated_f32 : he_blocksplit_tiles_gated_bf16)
+                                   : (f32 ? he_blocksplit_tiles_f32 : he_blocksplit_tiles_bf16))(p, C, A, W, bias, bias_dtype, M, N, K, fu,
+                                                                                                  x_pieces != 0, s);
   if (rc) return rc;
   return he_check_launch("he_gemm_blocksplit_bf16");
 }
@@ -204,5 +210,5 @@ extern "C" int he_gemm_blocksplit_bf16(void* C, const void* A, const void* W, co
                                        int gated, int R, int U, int NW, void* stream) {
   return he_gemm_blocksplit_fused_bf16(C, A, W, bias, M, N, K, out_dtype, bias_dtype, gated, R, U,
                                        NW, nullptr, 0, 0.f, nullptr, nullptr, HE_F32, nullptr,
-                                       nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, -1, nullptr, 0, 0, 0, 0, stream);
+                                       nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, -1, nullptr, 0, 0, 0, 0, 0, stream);
 }

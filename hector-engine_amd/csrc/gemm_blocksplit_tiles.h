@@ -8,12 +8,8 @@
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-template <bool CHECKED>
-__device__ __forceinline__ bf16x8 bs_load8(const uint16_t* p, bool ok) {
-  if (!CHECKED) return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
-  uint4 v = make_uint4(0, 0, 0, 0);
-  if (ok) v = *reinterpret_cast<const uint4*>(p);
-  return __builtin_bit_cast(bf16x8, v);
+__device__ __forceinline__ bf16x8 bs_load8(const char* p) {
+  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
 }
 
 // Four neighbouring outputs. align: how many elements the address is a multiple of (4, 2 or 1).
@@ -89,57 +85,40 @@ __device__ __forceinline__ void bs_store_pieces(uint16_t* base, int M, int m, in
   for (int i = 0; i < valid; ++i) *at(col + i) = float_to_bf16_bits(v[i]);
 }
 
-// Registers hold the operands of two steps (the loads of the next step are issued before
-// the products of this one), 16 U (R + MT) of them; above 4 tile pairs the workgroup is
-// limited to 8 wavefronts so that each may use 256 registers.
-constexpr int bs_max_waves(int MT, int R, int U) { return U * (R + MT) <= 4 ? 16 : 8; }
-
-template <int MT, int R, int U>
-struct BsFrags {
-  bf16x8 a[U][R][2], b[U][MT][2];
+// How a wavefront lays its lanes over the weight. An instruction of 16 x 16 outputs over 32 k has 16 columns for rows of X, of which
+// a step of few rows would leave most empty. SP spreads the columns: column c is row c >> SP of X at the k chunk c & (2^SP - 1), and
+// likewise tile row r is weight row r >> SP at chunk r & (2^SP - 1). Only outputs whose two chunks agree are sums of matching k; they
+// lie in neighbouring lanes and are added at the end (bs_spread_sum). What it buys is the loads: an instruction's operand is
+// 16 >> SP weight rows of 64 << SP bytes each, whole lines from SP = 1 on with neighbouring lanes side by side, where 16 rows are half a
+// line each. Whole lines can be asked for past the caches (he_load16_once), which half lines cannot: the other half would be
+// fetched twice. 37888 x 3584 at 1 row 50.8 -> 42 us (6.4 TB/s), at 8 rows 52.5 -> 42, 3584 x 3584 at 1 row 9.6 -> 6.2.
+// SP = 0 keeps each sum in the order this product had before: a unit of 64 k is two instructions, whose lanes take the halves of 16
+// neighbouring k. For 17 to 32 rows, and where a caller asks for that order (`ordered`; also the K slices and, by workgroup, the
+// turn each wavefront begins at are then those it had).
+template <int SP>
+struct BsLanes {
+  static constexpr int RT = 16 >> SP;              // weight rows, and rows of X, of an instruction
+  static constexpr int PARTS = 1 << SP;
+  static constexpr int H = SP == 0 ? 2 : 1;        // instructions of a unit
+  static constexpr int KM = SP == 0 ? 64 : 32 << SP;   // k of a unit
 };
 
-// CHECKED: the step may reach past k_end (it then loads nothing there and adds zeros). Unchecked
-// loads carry no branch, so the compiler counts them and waits for the older fragments only,
-// not for all that are in flight.
-template <int MT, int R, int U, bool PIECES, bool CHECKED>
-__device__ __forceinline__ void bs_load(BsFrags<MT, R, U>& f, const uint16_t* const* wp,
-                                        const uint16_t* const* xp, int k, int lg, int k_end, int M) {
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int kk = k + 64 * u + lg * 16;   // this lane's 16 k values of the step
-    const bool ok0 = !CHECKED || kk + 8 <= k_end, ok1 = !CHECKED || kk + 16 <= k_end;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      f.a[u][r][0] = bs_load8<CHECKED>(wp[r] + k + 64 * u, ok0);
-      f.a[u][r][1] = bs_load8<CHECKED>(wp[r] + k + 64 * u + 8, ok1);
-    }
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      if (PIECES) {   // piece-major X: the piece of 8 k values from kk on lies at kk M (+ 8 row)
-        f.b[u][t][0] = bs_load8<CHECKED>(xp[t] + (k + 64 * u) * M, ok0);
-        f.b[u][t][1] = bs_load8<CHECKED>(xp[t] + (k + 64 * u + 8) * M, ok1);
-      } else {
-        f.b[u][t][0] = bs_load8<CHECKED>(xp[t] + k + 64 * u, ok0);
-        f.b[u][t][1] = bs_load8<CHECKED>(xp[t] + k + 64 * u + 8, ok1);
-      }
-    }
-  }
+template <int SP>
+__device__ __forceinline__ float bs_spread_sum(float v) {      // over the 2^SP neighbouring lanes, the same in each
+  if (SP >= 1) v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0xB1, 0xf, 0xf, true));      // lanes 1 0 3 2
+  if (SP >= 2) v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x4E, 0xf, 0xf, true));      // lanes 2 3 0 1
+  return v;
 }
 
-template <int MT, int R, int U>
-__device__ __forceinline__ void bs_multiply(const BsFrags<MT, R, U>& f, floatx4 (&acc)[R][MT]) {
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[u][r][h], f.b[u][t][h], acc[r][t],
-                                                              0, 0, 0);
-}
+// Registers hold the operands of two steps (the loads of the next step are issued before
+// the products of this one), 8 S (NA + MT) of them (16 with SP = 0); above 4 operands a step the workgroup is
+// limited to 8 wavefronts so that each may use 256 registers.
+constexpr int bs_max_waves(int MT, int NA, int S) { return S * (NA + MT) <= 4 ? 16 : 8; }
+
+template <int MT, int NA, int S, int H>
+struct BsFrags {
+  bf16x8 a[S][H][NA], b[S][H][MT];
+};
 
 struct BsFusion {
   const float* scale_partials;   // [M][scale_count] or null: sums of squares of the input rows
@@ -165,35 +144,17 @@ struct BsFusion {
   const void* dyt_alpha;         // gain's dtype; alpha one stored number), and sq_out = 0: nothing is owed
 };
 
-// The residual values and gains of output item (tile, lane) of a non-gated product:
-// row m = 16 t + lane % 16, columns n0 + 16 r + 4 (lane / 16) .. + 4.
-// With few rows the 16 columns of the activation tile hold each row several times: column c
-// is row c >> spread (spread 2 up to 4 rows, 1 up to 8), so that the four lanes the memory
-// pipeline takes together read one or two rows, not four (1-4 % of a product's time). The
-// first column of a row owns its outputs.
-template <int MT>
-__device__ __forceinline__ int bs_spread(int M) {
-  return MT == 1 ? (M <= 4 ? 2 : (M <= 8 ? 1 : 0)) : 0;
-}
-
-template <int MT>
-__device__ __forceinline__ void bs_load_resid(const BsFusion& fu, int item, int n0, int n_end, int M,
-                                              int N, float res[4], float gain[4]) {
-  const int spread = bs_spread<MT>(M);
-  const int ot = item >> 6, ol = item & 63;
-  const int col = 16 * (ot % MT) + (ol & 15);
-  const int m = col >> spread;
-  const int n = n0 + 16 * (ot / MT) + 4 * (ol >> 4);
-  const int valid = (m < M && (m << spread) == col) ? max(0, min(4, n_end - n)) : 0;
-  if (valid == 4 && ((N | n0) & 3) == 0) {
-    const float4 r4 = *reinterpret_cast<const float4*>(fu.resid + (int64_t)m * N + n);
+// The residual values, gains and bias of an output item: row m, columns n .. n + valid.
+__device__ __forceinline__ void bs_load_resid(const BsFusion& fu, int m, int n, int valid, int N, int align, float res[4], float gain[4]) {
+  const float* p = fu.resid + (int64_t)m * N + n;
+  if (valid == 4 && align >= 4) {
+    const float4 r4 = *reinterpret_cast<const float4*>(p);
     res[0] = r4.x, res[1] = r4.y, res[2] = r4.z, res[3] = r4.w;
-  } else if (valid == 4 && ((N | n0) & 1) == 0) {
-    const float2 a = *reinterpret_cast<const float2*>(fu.resid + (int64_t)m * N + n);
-    const float2 b = *reinterpret_cast<const float2*>(fu.resid + (int64_t)m * N + n + 2);
+  } else if (valid == 4 && align >= 2) {
+    const float2 a = *reinterpret_cast<const float2*>(p), b = *reinterpret_cast<const float2*>(p + 2);
     res[0] = a.x, res[1] = a.y, res[2] = b.x, res[3] = b.y;
   } else {
-    for (int i = 0; i < 4; ++i) res[i] = i < valid ? fu.resid[(int64_t)m * N + n + i] : 0.f;
+    for (int i = 0; i < 4; ++i) res[i] = i < valid ? p[i] : 0.f;
   }
   if (valid == 4 && fu.gain_dtype == HE_BF16 && (n & 1) == 0 && (((uintptr_t)fu.gain) & 3) == 0) {
     const uint32_t* g = reinterpret_cast<const uint32_t*>((const uint16_t*)fu.gain + n);
@@ -215,193 +176,250 @@ __device__ __forceinline__ bool bs_used(const BsFusion& fu, int M, int e) {
   return any;
 }
 
-// grid: one workgroup per 16*R weight rows; block: 64 * NW threads.
+enum BsOut { BS_PLAIN, BS_GATED, BS_RESID };
+
+// grid: one workgroup per rows_per_block weight rows, at most RT NA; block: 64 * NW threads, each wavefront `units_per_wave`
+// units' k; turn: units that are walked together (ORDERED: the turns of a wavefront begin at one that depends on its workgroup). The
+// arguments that the first loads need come first.
 // USED (of a routed feed-forward in a step of a few rows: the experts that nobody chose, a third of 16 at 4 rows of 4 choices): a
-// workgroup of rows nobody uses leaves before it asks for weights; along K a wavefront walks the turns of the groups that are
-// used in the order it walks all of them, so its sums are the same bits. (4 rows, 4 choices of 16 experts of 2048 over 2048: first product 49.3 us
-// with all weights, 44.6 with the check behind the first loads, 41.5 ahead of them; the second 33.5 and 29.9.)
-template <int MT, int R, int U, bool GATED, bool PIECES, bool USED, typename TC>
-__global__ __launch_bounds__(64 * bs_max_waves(MT, R, U)) void gemm_blocksplit_kernel(
-    TC* __restrict__ C, const uint16_t* __restrict__ X, const uint16_t* __restrict__ W,
-    const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int kslice, int rows_per_block,
-    BsFusion fu) {
-  extern __shared__ float4 tiles[];   // [NW][R*MT][64]
-  __shared__ float row_scale[16 * MT];
-  __shared__ float row_sq[R * MT][16];
+// workgroup of rows nobody uses leaves before it asks for weights; along K a wavefront walks the steps of the groups that are
+// used in the order it walks all of them, so its sums are the same bits.
+template <int SP, int MT, int NA, int S, BsOut OUT, bool PIECES, bool USED, typename TC>
+__global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_kernel(
+    const uint16_t* __restrict__ W, const uint16_t* __restrict__ X, int M, int N, int K, int rows_per_block, int units_per_wave,
+    int turn, int bias_dtype, TC* __restrict__ C, const void* __restrict__ bias, BsFusion fu) {
+  using L = BsLanes<SP>;
+  constexpr bool ORDERED = SP == 0 && MT == 1;
+  constexpr int ROWS = L::RT * NA;              // weight rows a workgroup can hold
+  constexpr int MX = L::RT * MT;                // rows of X
+  extern __shared__ float4 tiles[];             // [NW][MX][ROWS] floats
+  __shared__ float row_scale[MX];
+  float* const red = reinterpret_cast<float*>(tiles);
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;
-  // the workgroup's weight rows [n0, n_end): at most 16 R, fewer when the rows are dealt out evenly
   const int n0 = blockIdx.x * rows_per_block;
   const int n_end = min(N, n0 + rows_per_block);
-  const int k_begin = wave * kslice;
-  const int k_end = min(K, k_begin + kslice);
   const int lr = lane & 15, lg = lane >> 4;
-  const int spread = bs_spread<MT>(M);
-
-  const uint16_t* wp[R];
-  const uint16_t* xp[MT];
-#pragma unroll
-  for (int r = 0; r < R; ++r) wp[r] = W + (int64_t)min(n0 + 16 * r + lr, n_end - 1) * K + lg * 16;
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-    xp[t] = PIECES ? X + (2 * lg * M + min((16 * t + lr) >> spread, M - 1)) * 8
-                   : X + (int64_t)min((16 * t + lr) >> spread, M - 1) * K + lg * 16;
-
-  floatx4 acc[R][MT];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[r][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  // Loads the epilogue needs are issued here, ahead of the weight stream, so that their
-  // latency is not added at the end: the partial sums of squares of the input rows
-  // (wavefront w takes the rows w, w + nw, ... up to four; lanes hold strided partials) and, for the
-  // residual epilogue (a little further down, behind the first weight loads), the residual
-  // values and gains of this thread's first outputs.
-  constexpr int OUT_TILES = R * MT;
-  const int out_align = ((N | n0) & 3) == 0 ? 4 : (((N | n0) & 1) == 0 ? 2 : 1);
-  const bool scaled = fu.scale_partials != nullptr;
-  const bool to_resid = !GATED && fu.resid != nullptr;
-  const bool dyt = fu.dyt_alpha != nullptr;
-  const float dyt_a = dyt ? load_param(fu.dyt_alpha, 0, fu.gain_dtype) : 0.f;
-  constexpr int SCALE_ROWS = 4;           // rows a wavefront takes: 16 rows with 4 wavefronts
-  const bool scale_early = scaled && fu.scale_count <= 256 && M <= SCALE_ROWS * nw;
-  float pv[SCALE_ROWS][4];
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);   // in a scalar register: rows beyond M cost a scalar branch
-  if (scale_early) {
-#pragma unroll
-    for (int j = 0; j < SCALE_ROWS; ++j) {
-      const int m = wave_s + j * nw;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) pv[j][q] = 0.f;
-      if (m < M) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int i = lane + 64 * q;
-          if (i < fu.scale_count) pv[j][q] = fu.scale_partials[(int64_t)m * fu.scale_count + i];
-        }
-      }
-    }
-  }
-  float res0[4] = {0.f, 0.f, 0.f, 0.f}, gain0[4] = {0.f, 0.f, 0.f, 0.f};
-
-  // Two steps of 64 U k values per turn. The whole turns of a wavefront's slice run without
-  // bounds checks, two fragments in flight: the loads of one are waited for while the other's
-  // are on their way. They start at a point of the slice that differs from workgroup to
-  // workgroup and wrap around: workgroups that run in step then read addresses that do not
-  // all sit at the same offset of their (equally spaced) weight rows. What is left of the
-  // slice is one checked turn at the end (a step past k_end loads nothing and adds zeros).
-  BsFrags<MT, R, U> f0, f1;
-  constexpr int TURN = 128 * U;
-  const int span = max(k_end - k_begin, 0);
-  int full = span / TURN;
-  const int k_full = k_begin + full * TURN;
-  const bool tail = span > full * TURN;
-  int k = full > 0 ? k_begin + (int)((blockIdx.x * 3u) % (unsigned)full) * TURN : k_begin;
+  const int row = lr >> SP;                                       // of an instruction's weight rows
+  // columns that a row of X takes (with SP = 0 and few rows they repeat it, so that neighbouring lanes read few rows)
+  const int spread = ORDERED ? (M <= 4 ? 2 : M <= 8 ? 1 : 0) : SP;
+  const int xrow = lr >> spread;
+  const int units = (K + L::KM - 1) / L::KM;
+  const int u0 = min(wave * units_per_wave, units), u1 = min(units, u0 + units_per_wave);
   if (USED && fu.used_rows > 0) {
     const int e0 = n0 / fu.used_rows, e1 = (n_end - 1) / fu.used_rows;
     if (e1 - e0 < 64 && __ballot(lane <= e1 - e0 && bs_used(fu, M, e0 + lane)) == 0) return;      // (the whole workgroup)
   }
-  // USED along K: bit t says that turn t of this wavefront's slice meets a group that is used (of more than 64 turns: all do)
-  uint64_t turns = 0;
-  auto advance = [&]() {
-    if (USED && turns != 0) {
-      const int t = (k - k_begin) / TURN;
-      const uint64_t behind = t < 63 ? turns >> (t + 1) : 0;
-      k = k_begin + TURN * (behind != 0 ? t + 1 + __builtin_ctzll(behind) : __builtin_ctzll(turns));
-    } else {
-      k += TURN;
-      if (k >= k_full) k = k_begin;
-    }
+
+  // a lane's weight rows are neighbours (row NA + a), so that the sums it ends with are neighbouring columns
+  const char* const wb = reinterpret_cast<const char*>(W + (int64_t)n0 * K);
+  const char* const xb = reinterpret_cast<const char*>(X);
+  const int k_lane = SP == 0 ? 16 * lg : 8 * ((lg << SP) | (lr & (L::PARTS - 1)));    // this lane's first k of a unit
+  uint32_t wo[NA], xo[MT];
+#pragma unroll
+  for (int a = 0; a < NA; ++a) wo[a] = 2u * (uint32_t)(min(row * NA + a, n_end - n0 - 1) * K);
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xo[t] = 2u * (uint32_t)(min(t * L::RT + xrow, M - 1) * (PIECES ? 8 : K));
+  const uint32_t xk = PIECES ? 2 * M : 2;                         // piece-major X: the piece of 8 k from k on lies at k M (+ 8 row)
+
+  floatx4 acc[NA][MT];
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[a][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // Steps of S units, the operands of two steps in registers: the loads of one go out together, ahead of the products of
+  // the other. Of a last step that is not whole the last k are loaded again in place of what lies beyond (no branch, no second
+  // trip to memory), and those products are left out, or of zeros where only some lanes lie beyond K.
+  BsFrags<MT, NA, S, L::H> f0, f1;
+  auto load = [&](BsFrags<MT, NA, S, L::H>& f, int u) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int h = 0; h < L::H; ++h) {
+        const uint32_t k = min(min(u + s, u1 - 1) * L::KM + k_lane + 8 * h, K - 8);
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+          f.a[s][h][a] = SP > 0 ? he_load16_once<bf16x8>(wb + (wo[a] + 2 * k)) : bs_load8(wb + (wo[a] + 2 * k));
+#pragma unroll
+        for (int t = 0; t < MT; ++t) f.b[s][h][t] = bs_load8(xb + (xo[t] + k * xk));
+      }
   };
-  if (USED && fu.used_k > 0 && full > 0 && full <= 64) {
-    const int at = k_begin + min(lane, full - 1) * TURN, first = at / fu.used_k, last = (at + TURN - 1) / fu.used_k;
-    bool any = bs_used(fu, M, first);
-    if (last != first) any = any || bs_used(fu, M, last);      // (groups are no shorter than a turn)
-    turns = __ballot(any && lane < full);
-    full = __popcll(turns);
-    if (full > 0 && ((turns >> ((k - k_begin) / TURN)) & 1) == 0) advance();
+  auto multiply_unit = [&](const BsFrags<MT, NA, S, L::H>& f, int s) {
+#pragma unroll
+    for (int h = 0; h < L::H; ++h)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[s][h][a], f.b[s][h][t], acc[a][t], 0, 0, 0);
+  };
+  auto multiply = [&](const BsFrags<MT, NA, S, L::H>& f) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) multiply_unit(f, s);
+  };
+  auto multiply_last = [&](BsFrags<MT, NA, S, L::H>& f, int u) {
+    const bf16x8 zero = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (u + s < u1) {
+        if ((u + s + 1) * L::KM > K) {
+#pragma unroll
+          for (int h = 0; h < L::H; ++h) {
+            const bool beyond = (u + s) * L::KM + k_lane + 8 * h >= K;
+#pragma unroll
+            for (int a = 0; a < NA; ++a) f.a[s][h][a] = beyond ? zero : f.a[s][h][a];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) f.b[s][h][t] = beyond ? zero : f.b[s][h][t];
+          }
+        }
+        multiply_unit(f, s);
+      }
+  };
+
+  // The order of the units: whole turns from turn `first` on, around, then what is left. USED along K: bit t of `turns` says that
+  // turn t meets a group that is used (of more than 64 turns: all do).
+  const int n = u1 - u0, whole = max(min(u1, K / L::KM) - u0, 0) / turn * turn;
+  const int first = ORDERED && whole > 0 ? (int)((blockIdx.x * 3u) % (unsigned)(whole / turn)) * turn : 0;
+  int left = (n + S - 1) / S, j = 0;
+  uint64_t turns = ~0ull;
+  auto unit = [&](int j) { return u0 + (!ORDERED || j >= whole ? j : j + first < whole ? j + first : j + first - whole); };
+  auto skip = [&]() {
+    if (USED)
+      while (j < whole && ((turns >> (((unit(j) - u0) / turn) & 63)) & 1) == 0) j += turn;
+  };
+  if (USED && fu.used_k > 0 && whole > 0 && whole <= 64 * turn) {
+    const int at = (u0 + min(lane * turn, whole - turn)) * L::KM, e0 = at / fu.used_k, e1 = min(at + turn * L::KM - 1, K - 1) / fu.used_k;
+    bool any = bs_used(fu, M, e0);
+    if (e1 != e0) any = any || bs_used(fu, M, e1);      // (groups are no shorter than a turn)
+    turns = __ballot(any && lane * turn < whole);
+    left = __popcll(turns) * (turn / S) + (n - whole + S - 1) / S;
+    skip();
   }
-  if (full > 0) bs_load<MT, R, U, PIECES, false>(f0, wp, xp, k, lg, k_end, M);
-  else if (tail) bs_load<MT, R, U, PIECES, true>(f0, wp, xp, k_full, lg, k_end, M);
-  if (to_resid && threadIdx.x < OUT_TILES * 64)   // behind the first weights, ahead of the rest
-    bs_load_resid<MT>(fu, threadIdx.x, n0, n_end, M, N, res0, gain0);
-  if (full > 0) {
-    for (int j = 0; j + 1 < full; ++j) {
-      bs_load<MT, R, U, PIECES, false>(f1, wp, xp, k + 64 * U, lg, k_end, M);
-      __builtin_amdgcn_sched_barrier(0);   // the loads of a fragment go out together, ahead of the products
-      bs_multiply<MT, R, U>(f0, acc);
-      advance();
+  int u = unit(j);
+  auto next = [&]() {
+    j += S;
+    if (USED && turns != ~0ull && j < whole && j % turn == 0) skip();
+    return u = unit(j);
+  };
+  if (left > 0) load(f0, u);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // Loads the epilogue needs go out behind the first weights, so that their latency is not added at the end: the partial sums of
+  // squares of the input rows (wavefront w takes the rows w, w + nw, ...; lanes hold strided partials), and the residual
+  // values, gains and bias of this thread's first outputs.
+  const bool scaled = fu.scale_partials != nullptr;
+  constexpr int SCALE_ROWS = (MX + 3) / 4;      // rows a wavefront takes: all of them with 4 wavefronts
+  constexpr int SCALE_LOADS = SCALE_ROWS <= 2 ? 8 : 4;
+  const bool scale_early = scaled && fu.scale_count <= 64 * SCALE_LOADS && M <= SCALE_ROWS * nw;
+  float pv[SCALE_ROWS][SCALE_LOADS];
+  if (scale_early) {
+#pragma unroll
+    for (int j = 0; j < SCALE_ROWS; ++j) {
+      const float* p = fu.scale_partials + (int64_t)min(wave + j * nw, M - 1) * fu.scale_count;
+#pragma unroll
+      for (int q = 0; q < SCALE_LOADS; ++q) pv[j][q] = p[min(lane + 64 * q, fu.scale_count - 1)];
+    }
+  }
+  constexpr int G = ROWS / 4;                   // items of four columns a row
+  const int items = M * G;
+  const int out_align = ((N | n0) & 3) == 0 ? 4 : (((N | n0) & 1) == 0 ? 2 : 1);
+  float res0[4] = {0.f, 0.f, 0.f, 0.f}, gain0[4] = {0.f, 0.f, 0.f, 0.f}, bias0[4] = {0.f, 0.f, 0.f, 0.f};
+  auto ahead = [&](int item) {
+    const int m = item / G, at = n0 + 4 * (item % G), valid = max(0, min(4, n_end - at));
+    if (OUT == BS_RESID) bs_load_resid(fu, m, at, valid, N, out_align, res0, gain0);
+    if (OUT != BS_GATED && bias != nullptr)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bias0[i] = load_param(bias, min(at + i, N - 1), bias_dtype);
+  };
+  if (OUT != BS_GATED && (int)threadIdx.x < items) ahead(threadIdx.x);
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (left > 0) {
+    for (; left > 2; left -= 2) {
+      load(f1, next());
+      __builtin_amdgcn_sched_barrier(0);   // the loads of a step go out together, ahead of the products
+      multiply(f0);
       __builtin_amdgcn_sched_barrier(0);
-      bs_load<MT, R, U, PIECES, false>(f0, wp, xp, k, lg, k_end, M);
+      load(f0, next());
       __builtin_amdgcn_sched_barrier(0);
-      bs_multiply<MT, R, U>(f1, acc);
+      multiply(f1);
       __builtin_amdgcn_sched_barrier(0);
     }
-    bs_load<MT, R, U, PIECES, false>(f1, wp, xp, k + 64 * U, lg, k_end, M);
-    bs_multiply<MT, R, U>(f0, acc);
-    if (tail) bs_load<MT, R, U, PIECES, true>(f0, wp, xp, k_full, lg, k_end, M);
-    bs_multiply<MT, R, U>(f1, acc);
-  }
-  if (tail) {
-    bs_load<MT, R, U, PIECES, true>(f1, wp, xp, k_full + 64 * U, lg, k_end, M);
-    bs_multiply<MT, R, U>(f0, acc);
-    bs_multiply<MT, R, U>(f1, acc);
+    if (left == 2) {
+      load(f1, next());
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(f0);
+      multiply_last(f1, u);
+    } else {
+      multiply_last(f0, u);
+    }
   }
 
   if (scaled) {
     if (scale_early) {
 #pragma unroll
       for (int j = 0; j < SCALE_ROWS; ++j) {
-        const int m = wave_s + j * nw;
-        if (m < M) {
-          const float total = wave_sum(((pv[j][0] + pv[j][1]) + pv[j][2]) + pv[j][3]);
-          if (lane == 0) row_scale[m] = 1.0f / sqrtf(total / (float)fu.scale_dim + fu.scale_eps);
-        }
+        float part = 0.f;
+#pragma unroll
+        for (int q = 0; q < SCALE_LOADS; ++q) part += lane + 64 * q < fu.scale_count ? pv[j][q] : 0.f;
+        const float total = wave_sum(part);
+        if (lane == 0 && wave + j * nw < M) row_scale[wave + j * nw] = 1.0f / sqrtf(total / (float)fu.scale_dim + fu.scale_eps);
       }
     } else {
       for (int m = wave; m < M; m += nw) {
         float part = 0.f;
-        for (int i = lane; i < fu.scale_count; i += 64)
-          part += fu.scale_partials[(int64_t)m * fu.scale_count + i];
+        for (int i = lane; i < fu.scale_count; i += 64) part += fu.scale_partials[(int64_t)m * fu.scale_count + i];
         const float total = wave_sum(part);
         if (lane == 0) row_scale[m] = 1.0f / sqrtf(total / (float)fu.scale_dim + fu.scale_eps);
       }
     }
   }
 
-  // every wavefront leaves its tiles; acc[r][t][i] = D[n0 + 16r + 4lg + i][16t + lr]
+  // every wavefront leaves its sums: tile row 4 lg + i of an instruction is weight row (4 lg + i) >> SP at chunk (4 lg + i) % 2^SP
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+  for (int t = 0; t < MT; ++t) {
+    const int m = t * L::RT + xrow, part = lr & ((1 << spread) - 1);
+    constexpr int J = 4 >> SP;
+    float v[J * NA];
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
-      tiles[(wave * (R * MT) + r * MT + t) * 64 + lane] =
-          make_float4(acc[r][t][0], acc[r][t][1], acc[r][t][2], acc[r][t][3]);
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        float x = acc[a][t][j * L::PARTS];
+#pragma unroll
+        for (int i = 1; i < L::PARTS; ++i) x = part == i ? acc[a][t][j * L::PARTS + i] : x;
+        v[j * NA + a] = bs_spread_sum<SP>(x);
+      }
+    if (part == 0 && m < M) {
+      float* at = red + (wave * MX + m) * ROWS + lg * J * NA;
+      if constexpr (J * NA % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < J * NA; i += 4) *reinterpret_cast<float4*>(at + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < J * NA; ++i) at[i] = v[i];
+      }
+    }
+  }
   __syncthreads();
 
-  // thread (tile, lane) adds the slices in wavefront order and writes 4 outputs; a
-  // wavefront works on one tile at a time (item >> 6 is the same in all its lanes)
-  for (int item = threadIdx.x; item < OUT_TILES * 64; item += blockDim.x) {
-    const int ot = item >> 6, ol = item & 63;
-    const int olr = ol & 15, olg = ol >> 4;
-    const int t = ot % MT;
-    const int r = ot / MT;
-    const int col = 16 * t + olr, m = col >> spread;
-    const bool owner = m < M && (m << spread) == col;
+  // a thread adds four neighbouring columns of a row over the wavefronts in their order and writes them
+  for (int item = threadIdx.x; item < items; item += blockDim.x) {
+    const int m = item / G, n = n0 + 4 * (item % G);
+    const int valid = max(0, min(4, n_end - n));
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int w = 0; w < nw; ++w) {
-      const float4 v = tiles[(w * (R * MT) + r * MT + t) * 64 + ol];
+      const float4 v = *reinterpret_cast<const float4*>(red + (w * MX + m) * ROWS + 4 * (item % G));
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
     float v[4] = {s.x, s.y, s.z, s.w};
-    const float rs = (scaled && m < M) ? row_scale[m] : 1.f;
-    if (GATED) {
+    const float rs = scaled ? row_scale[m] : 1.f;
+    if (OUT == BS_GATED) {
       // the thread's four weight rows are two (gate, up) pairs: two outputs
-      const int NO = N >> 1;
-      const int n = n0 + 16 * r + 4 * olg;
-      const int valid = owner ? max(0, min(4, n_end - n)) >> 1 : 0;
-      if (valid <= 0) continue;
+      const int NO = N >> 1, pairs = valid >> 1;
+      if (pairs <= 0) continue;
       float y[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -410,17 +428,14 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, R, U)) void gemm_blocksplit_k
                               : g / (1.f + expf(-g)) * (v[2 * i + 1] * rs);
       }
       if (fu.out_pieces)
-        bs_store_pieces(reinterpret_cast<uint16_t*>(C), M, m, n >> 1, y, 2, valid);
+        bs_store_pieces(reinterpret_cast<uint16_t*>(C), M, m, n >> 1, y, 2, pairs);
       else
-        bs_store2<TC>(C + (int64_t)m * NO + (n >> 1), y, ((NO | (n0 >> 1)) & 1) == 0, valid);
+        bs_store2<TC>(C + (int64_t)m * NO + (n >> 1), y, ((NO | (n0 >> 1)) & 1) == 0, pairs);
     } else {
-      const int n = n0 + 16 * r + 4 * olg;
-      const int valid = owner ? max(0, min(4, n_end - n)) : 0;
+      if (item != (int)threadIdx.x) ahead(item);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] *= rs;
-      if (bias != nullptr)
-        for (int i = 0; i < valid; ++i) v[i] += load_param(bias, n + i, bias_dtype);
-      if (!to_resid) {
+      for (int i = 0; i < 4; ++i) v[i] = v[i] * rs + bias0[i];
+      if (OUT == BS_PLAIN) {
         if (fu.unary >= 0)
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[i] = he_unary(bf16_bits_to_float(float_to_bf16_bits(v[i])), fu.unary);
@@ -432,7 +447,8 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, R, U)) void gemm_blocksplit_k
         }
         continue;
       }
-      if (item != threadIdx.x) bs_load_resid<MT>(fu, item, n0, n_end, M, N, res0, gain0);
+      const bool dyt = fu.dyt_alpha != nullptr;
+      const float dyt_a = dyt ? load_param(fu.dyt_alpha, 0, fu.gain_dtype) : 0.f;
       float sq = 0.f, x[4], xgv[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -448,46 +464,35 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, R, U)) void gemm_blocksplit_k
         else
           bs_store4<bf16_t>(reinterpret_cast<bf16_t*>(fu.xg) + at, xgv, out_align, valid);
       }
-      // the four lane groups hold the row's other columns of this tile
-      sq = xor16_sum(sq);     // lane swaps, not the LDS crossbar: the same sums
-      sq = xor32_sum(sq);
-      if (olg == 0) row_sq[ot][olr] = sq;
-    }
-  }
-  if (to_resid) {
-    __syncthreads();
-    const int m = threadIdx.x;
-    if (m < M && m < 16 * MT) {
-      float sq = 0.f;
-      const int col = m << spread;
-      for (int r = 0; r < R; ++r) sq += row_sq[r * MT + col / 16][col % 16];
-      fu.sq_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
+      // a row's items are neighbouring lanes (G of them, a power of two)
+#pragma unroll
+      for (int step = 1; step < G; step <<= 1) sq += __shfl_xor(sq, step, HE_WAVE);
+      if (item % G == 0) fu.sq_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
     }
   }
 }
 
 struct BlockSplitPlan {
-  int MT, R, U, NW, kslice;
-  int rows_per_block;   // weight rows of a workgroup, at most 16 R
+  int SP, MT, NA, S, NW, units;      // units: of a wavefront
+  int turn;                          // units walked together, a multiple of S
+  int rows_per_block;                // weight rows of a workgroup, at most (16 >> SP) NA
 };
 
-template <int MT, int R, int U, bool GATED, bool USED, typename TC>
+template <int SP, int MT, int NA, int S, BsOut OUT, bool USED, typename TC>
 static inline void launch_blocksplit(const BlockSplitPlan& p, void* C, const void* X, const void* W,
                               const void* bias, int bias_dtype, int M, int N, int K,
                               const BsFusion& fu, bool x_pieces, hipStream_t s) {
   const int blocks = (N + p.rows_per_block - 1) / p.rows_per_block;
-  const size_t lds = (size_t)p.NW * R * MT * 64 * sizeof(float4);
-  if constexpr (MT == 1) {   // piece-major activations are for up to 16 rows
+  const size_t lds = (size_t)p.NW * BsLanes<SP>::RT * MT * BsLanes<SP>::RT * NA * sizeof(float);
+  if constexpr (SP > 0 || MT == 1) {   // piece-major activations are for up to 16 rows
     if (x_pieces) {
-      gemm_blocksplit_kernel<MT, R, U, GATED, true, USED, TC><<<blocks, 64 * p.NW, lds, s>>>(
-          (TC*)C, (const uint16_t*)X, (const uint16_t*)W, bias, bias_dtype, M, N, K, p.kslice,
-          p.rows_per_block, fu);
+      gemm_blocksplit_kernel<SP, MT, NA, S, OUT, true, USED, TC><<<blocks, 64 * p.NW, lds, s>>>(
+          (const uint16_t*)W, (const uint16_t*)X, M, N, K, p.rows_per_block, p.units, p.turn, bias_dtype, (TC*)C, bias, fu);
       return;
     }
   }
-  gemm_blocksplit_kernel<MT, R, U, GATED, false, USED, TC><<<blocks, 64 * p.NW, lds, s>>>(
-      (TC*)C, (const uint16_t*)X, (const uint16_t*)W, bias, bias_dtype, M, N, K, p.kslice,
-      p.rows_per_block, fu);
+  gemm_blocksplit_kernel<SP, MT, NA, S, OUT, false, USED, TC><<<blocks, 64 * p.NW, lds, s>>>(
+      (const uint16_t*)W, (const uint16_t*)X, M, N, K, p.rows_per_block, p.units, p.turn, bias_dtype, (TC*)C, bias, fu);
 }
 
 // Every tiling with one epilogue and output type: a function per file of
@@ -497,23 +502,34 @@ static inline void launch_blocksplit(const BlockSplitPlan& p, void* C, const voi
   const BlockSplitPlan &p, void *C, const void *X, const void *W, const void *bias, int bias_dtype, \
       int M, int N, int K, const BsFusion &fu, bool x_pieces, hipStream_t s
 int he_blocksplit_tiles_bf16(HE_BS_DISPATCH_ARGS);
+int he_blocksplit_tiles_resid(HE_BS_DISPATCH_ARGS);
 int he_blocksplit_tiles_f32(HE_BS_DISPATCH_ARGS);
 int he_blocksplit_tiles_gated_bf16(HE_BS_DISPATCH_ARGS);
 int he_blocksplit_tiles_gated_f32(HE_BS_DISPATCH_ARGS);
-int he_blocksplit_tiles_used_bf16(HE_BS_DISPATCH_ARGS);      // (up to 16 rows)
+int he_blocksplit_tiles_used_bf16(HE_BS_DISPATCH_ARGS);
+int he_blocksplit_tiles_used_resid(HE_BS_DISPATCH_ARGS);      // (up to 16 rows)
 
-#define HE_BS_TILING(MT_, R_, U_, GATED_, TC_) HE_BS_TILING_OF(MT_, R_, U_, GATED_, false, TC_)
-#define HE_BS_TILING_OF(MT_, R_, U_, GATED_, USED_, TC_)                                            \
-  if (p.MT == MT_ && p.R == R_ && p.U == U_) {                                                      \
-    launch_blocksplit<MT_, R_, U_, GATED_, USED_, TC_>(p, C, X, W, bias, bias_dtype, M, N, K, fu, x_pieces, s); \
+#define HE_BS_TILING(SP_, MT_, NA_, S_, OUT_, USED_, TC_)                                         \
+  if (p.SP == SP_ && p.MT == MT_ && p.NA == NA_ && p.S == S_) {                                     \
+    launch_blocksplit<SP_, MT_, NA_, S_, OUT_, USED_, TC_>(p, C, X, W, bias, bias_dtype, M, N, K, fu, x_pieces, s); \
     return 0;                                                                                       \
   }
-#define HE_BS_ALL_TILINGS(GATED_, TC_)                                                              \
-  HE_BS_TILING(1, 1, 1, GATED_, TC_) HE_BS_TILING(1, 1, 2, GATED_, TC_)                             \
-  HE_BS_TILING(1, 1, 4, GATED_, TC_) HE_BS_TILING(2, 1, 1, GATED_, TC_)                             \
-  HE_BS_TILING(2, 1, 2, GATED_, TC_) HE_BS_TILING(1, 2, 1, GATED_, TC_)                             \
-  HE_BS_TILING(1, 2, 2, GATED_, TC_) HE_BS_TILING(1, 2, 4, GATED_, TC_)                             \
-  HE_BS_TILING(2, 2, 1, GATED_, TC_) HE_BS_TILING(2, 2, 2, GATED_, TC_)                             \
-  HE_BS_TILING(1, 4, 1, GATED_, TC_) HE_BS_TILING(1, 4, 2, GATED_, TC_)                             \
-  he_set_error("he_gemm_blocksplit_bf16: no kernel for MT=%d R=%d U=%d", p.MT, p.R, p.U);           \
+#define HE_BS_SIXTEEN_ROWS(OUT_, USED_, TC_)                                                      \
+  HE_BS_TILING(2, 1, 1, 1, OUT_, USED_, TC_) HE_BS_TILING(2, 1, 1, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(2, 1, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(2, 1, 2, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(2, 1, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(2, 1, 4, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(1, 1, 1, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 1, 1, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(1, 1, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 1, 2, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(1, 1, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 1, 4, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(1, 2, 1, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 1, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(1, 2, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 2, 2, OUT_, USED_, TC_)         \
+  HE_BS_TILING(1, 2, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 4, 2, OUT_, USED_, TC_)             \
+  HE_BS_TILING(0, 1, 1, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 1, 2, OUT_, USED_, TC_)             \
+  HE_BS_TILING(0, 1, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 2, 2, OUT_, USED_, TC_)             \
+  HE_BS_TILING(0, 1, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 4, 2, OUT_, USED_, TC_)
+#define HE_BS_ALL_TILINGS(OUT_, TC_)                                                              \
+  HE_BS_SIXTEEN_ROWS(OUT_, false, TC_)                                                            \
+  HE_BS_TILING(0, 2, 1, 1, OUT_, false, TC_) HE_BS_TILING(0, 2, 1, 2, OUT_, false, TC_)         \
+  HE_BS_TILING(0, 2, 2, 1, OUT_, false, TC_) HE_BS_TILING(0, 2, 2, 2, OUT_, false, TC_)         \
+  he_set_error("he_gemm_blocksplit_bf16: no kernel for SP=%d MT=%d NA=%d S=%d", p.SP, p.MT, p.NA, p.S); \
   return -1

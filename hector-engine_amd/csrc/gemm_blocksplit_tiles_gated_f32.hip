@@ -2,5 +2,5 @@
 #include "gemm_blocksplit_tiles.h"
 
 int he_blocksplit_tiles_gated_f32(HE_BS_DISPATCH_ARGS) {
-  HE_BS_ALL_TILINGS(true, float);
+  HE_BS_ALL_TILINGS(BS_GATED, float);
 }

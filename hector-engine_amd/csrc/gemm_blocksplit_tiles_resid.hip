@@ -1,0 +1,6 @@
+// Tilings of the few-rows product (gemm_blocksplit_tiles.h): the residual epilogue.
+#include "gemm_blocksplit_tiles.h"
+
+int he_blocksplit_tiles_resid(HE_BS_DISPATCH_ARGS) {
+  HE_BS_ALL_TILINGS(BS_RESID, bf16_t);
+}

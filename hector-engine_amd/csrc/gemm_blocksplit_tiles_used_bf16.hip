@@ -2,8 +2,7 @@
 #include "gemm_blocksplit_tiles.h"
 
 int he_blocksplit_tiles_used_bf16(HE_BS_DISPATCH_ARGS) {
-#define HE_BS_USED(R_, U_) HE_BS_TILING_OF(1, R_, U_, false, true, bf16_t)
-  HE_BS_USED(1, 1) HE_BS_USED(1, 2) HE_BS_USED(1, 4) HE_BS_USED(2, 1) HE_BS_USED(2, 2) HE_BS_USED(2, 4) HE_BS_USED(4, 1) HE_BS_USED(4, 2)
-  he_set_error("he_gemm_blocksplit_bf16: no kernel for R=%d U=%d", p.R, p.U);
+  HE_BS_SIXTEEN_ROWS(BS_PLAIN, true, bf16_t)
+  he_set_error("he_gemm_blocksplit_bf16: no kernel for SP=%d MT=%d NA=%d S=%d", p.SP, p.MT, p.NA, p.S);
   return -1;
 }

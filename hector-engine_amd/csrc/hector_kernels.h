@@ -95,7 +95,9 @@ int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W, const v
                                   void* xg, void* sq_out, int sq_count, int x_pieces, int out_pieces,
                                   float act_alpha, float act_limit, float act_shift, float act_cubic, float resid_scale,
                                   const void* dyt_bias, const void* dyt_alpha, int unary, const void* used, int used_ld,
-                                  int used_count, int used_rows, int used_k, void* stream);
+                                  int used_count, int used_rows, int used_k, int ordered, void* stream);
+// ordered (M <= 16, no plan, no residual epilogue): every sum in tiles of 16 weight rows, K slices and turns of an older tiling of this
+// product, for results that feed a choice which another rounding turns over.
 // resid_scale: the residual epilogue adds resid_scale * result. dyt_alpha, dyt_bias (both null, or both
 // of gain's dtype; alpha one stored number): the norm that follows is Dynamic Tanh, and the epilogue
 // leaves it finished, xg = tanh(alpha * resid) * gain + dyt_bias, with sq_out = 0 (a reader that

@@ -44,7 +44,7 @@ _SIGNATURES = {
     "he_gemm_blocksplit_fused_bf16": [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_int,
                                       c_int, c_int, c_int, c_ptr, c_int, c_f32, c_ptr, c_ptr, c_int,
                                       c_ptr, c_ptr, c_int, c_int, c_int, c_f32, c_f32, c_f32, c_f32, c_f32, c_ptr, c_ptr,
-                                      c_int, c_ptr, c_int, c_int, c_int, c_int, c_ptr],
+                                      c_int, c_ptr, c_int, c_int, c_int, c_int, c_int, c_ptr],
     "he_scale_rows_bf16": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_f32, c_int, c_ptr],
     "he_splitk_reduce": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_ptr],
     "he_compute_units": [],

@@ -298,7 +298,7 @@ def _act4(act) -> tuple:
 @_op("gemm_blocksplit")
 def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0), *,
                     row_scale=None, residual=None, x_pieces: bool = False, out_pieces: bool = False,
-                    act=(1.0, 0.0, 0.0), unary: str | None = None, used=None) -> None:
+                    act=(1.0, 0.0, 0.0), unary: str | None = None, used=None, ordered: bool = False) -> None:
     """bf16 MFMA product for M <= 32 with K cut inside the workgroup; one launch, complete
     result (bf16 or fp32), with bias or, gated, as [M, N/2] = silu(gate) * up for a weight
     that alternates gate and up rows (gate i at row 2i, its up at 2i + 1). plan = (R, U, NW),
@@ -318,7 +318,9 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
     unary: an activation (ACT_KINDS) of the bf16 results, as unary_act gives it.
     used = (weights fp32 [M, count + 1 or more], count, size, along_k): the weight's rows, or its k, come in groups of `size`, and of the
     first `count` of them those are left out that no row has a weight for: their outputs are not written, or their products,
-    with zeros in `a`, not added (up to 16 rows)."""
+    with zeros in `a`, not added (up to 16 rows).
+    ordered: the order of sums this product had before its lanes read whole lines (up to 16 rows, no plan, no residual): for
+    results that reach a router over rows no norm has evened out."""
     N, K = w.shape
     NO = N // 2 if gated else N
     _need(a, "a", torch.bfloat16)
@@ -383,7 +385,7 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
         dtype_code(bias.dtype) if bias is not None else F32, int(gated),
         int(plan[0]), int(plan[1]), int(plan[2]), sp, sc, float(se), rp, gp, gdt, xp, qp, qc,
         int(x_pieces), int(out_pieces), *_act4(act), float(rscale),
-        _ptr(dyt_bias), _ptr(dyt_alpha), -1 if unary is None else ACT_KINDS[unary], *uargs, _stream()))
+        _ptr(dyt_bias), _ptr(dyt_alpha), -1 if unary is None else ACT_KINDS[unary], *uargs, int(ordered), _stream()))
 
 
 def gemm_rows_plan(M: int, N: int, K: int) -> tuple[int, int]:

@@ -219,6 +219,10 @@ class Part:
     # (parts that name the same function share the call), runs steps with different values as
     # different graphs, and hands the values over as ctx.hints[function]. None: no such wish.
     step_hint = None
+    # True for a part that chooses what a row is multiplied with by comparing numbers (a router), and for a block whose
+    # parts read the stream as it is, without a norm
+    routes = False
+    reads_stream = False
 
     def __init__(self, prefix: str, env: BuildEnv):
         self.prefix = prefix

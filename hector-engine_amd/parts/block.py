@@ -256,6 +256,8 @@ class PostNormBlock(Block):
     branch that reads them next. Other norms go through their own add_norm on a 32-bit copy of the branch output.
     names: mixer_norm, mixer, feed_forward_norm, feed_forward (suffixes of the parts' prefixes)."""
 
+    reads_stream = True
+
     def __init__(self, params: dict, prefix: str, env: BuildEnv):
         super().__init__(prefix, env)
         names = param(params, "names", dict)

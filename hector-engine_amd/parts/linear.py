@@ -70,6 +70,7 @@ class Linear:
         self.bias = bias
         self.out_features, self.in_features = weight.shape
         self.one_round_tiles = False        # set by a part: _long's, gated_tile's and K slices' products may run in tiles of this library's own
+        self.ordered = False                # set by the model: the few-rows product keeps an older order of sums (ops.gemm_blocksplit)
         self._plans: dict[bool, tuple[int, int]] = {}
         self._chosen: dict[tuple, routes.Route] = {}     # (rows, activations, fast) -> route, for one version of the table
         self._chosen_version = -1
@@ -151,7 +152,7 @@ class Linear:
         if out is None:
             out = ctx.alloc((rows, N), out_dtype)
         if rows <= ops.BLOCKSPLIT_PIECES_MAX_M:
-            ops.gemm_blocksplit(out, a, w, bias, rows, row_scale=scale, x_pieces=pieces, used=used)
+            ops.gemm_blocksplit(out, a, w, bias, rows, row_scale=scale, x_pieces=pieces, used=used, ordered=self.ordered)
             return out
         splits = self._plan(rows)[1]
         if splits == 1:
@@ -374,7 +375,7 @@ class Linear:
             raise ValueError("Linear.gated_silu: not for these rows (ask gated_silu_rows)")
         if rows <= ops.BLOCKSPLIT_PIECES_MAX_M:
             ops.gemm_blocksplit(out, a, self.weight, None, rows, gated=True, row_scale=scale,
-                                x_pieces=pieces, out_pieces=out_pieces, act=consts)
+                                x_pieces=pieces, out_pieces=out_pieces, act=consts, ordered=self.ordered)
             return
         splits = self._plan(rows)[1]
         if splits == 1:
@@ -432,7 +433,7 @@ class Linear:
             return None
         if 0 < rows <= ops.BLOCKSPLIT_PIECES_MAX_M and self.route(rows, ctx, act).run is Linear._run_mfma:
             out = ctx.alloc((rows, self.weight.shape[0]), act)
-            ops.gemm_blocksplit(out, a, self.weight, self.bias, rows, row_scale=scale, x_pieces=pieces, unary=kind)
+            ops.gemm_blocksplit(out, a, self.weight, self.bias, rows, row_scale=scale, x_pieces=pieces, unary=kind, ordered=self.ordered)
             return out
         tile = self.gated_tile(rows, ctx, x) if kind in ("relu2", "relu") else None
         if tile is None:

@@ -50,6 +50,8 @@ def _linears(part) -> list[Linear]:
 
 @register_part("feed_forward", "routed_experts")
 class RoutedExperts(FeedForward):
+    routes = True
+
     def __init__(self, params: dict, prefix: str, env: BuildEnv):
         super().__init__(prefix, env)
         self.hidden = param(params, "hidden_size", int)

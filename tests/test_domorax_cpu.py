@@ -218,3 +218,22 @@ def test_prefix_logits_do_not_depend_on_what_follows():
     whole = P.forward(MODELS["C"], w, ids)
     assert torch.allclose(P.forward(MODELS["C"], w, ids[:6]), whole[:6], atol=1e-9)
     assert P.greedy(MODELS["C"], w, ids[:4], 3) == P.greedy(MODELS["C"], w, ids[:4], 5)[:3]
+
+
+@pytest.mark.parametrize("name", ["A", "B", "C"])
+def test_layers_beside_a_router_of_unnormed_rows_keep_their_order_of_sums(name):
+    """All products of the layers, where some layer routes; the head's stay free."""
+    from hector_engine_amd.parts.base import BuildEnv
+    from hector_engine_amd.parts.linear import Linear
+    from hector_engine_amd.registry import build_model
+    cfg = config_of(MODELS[name])
+    m = build_model(cfg, BuildEnv(torch.device("cpu"), torch.bfloat16))
+    m.bind({n: torch.zeros(s.random_shape(), dtype=torch.int32 if s.integer else torch.bfloat16) for n, s in m.tensor_specs().items()})
+    parts, todo = [], list(m.blocks)
+    while todo:
+        parts.append(todo.pop())
+        todo += parts[-1].children()
+    linears = [v for p in parts for v in vars(p).values() if isinstance(v, Linear)]
+    routed = any((l.get("mlp") or {}).get("kind") == "moe" for l in MODELS[name]["layers"])
+    assert linears and all(lin.ordered == routed for lin in linears)
+    assert not any(v.ordered for v in vars(m.head).values() if isinstance(v, Linear))

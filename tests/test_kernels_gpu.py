@@ -937,6 +937,38 @@ def test_attention_far_key_stands_out(ops):
         assert torch.allclose(got.reshape(H, hd)[0], v[far, 0].double(), atol=0.05), kind
 
 
+# (rows of X on both sides of each layout of the lanes; one chunk of k, K around an instruction's 64 and 128 k and around eight wavefronts'
+# slices of them; weight rows around the tiles of 4, 8, 16 and 32, few and more than two a compute unit)
+@pytest.mark.parametrize("ordered", [False, True])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("K", [8, 56, 136, 264, 1016, 1032, 2112])
+def test_gemm_blocksplit_at_the_edges_of_its_tiles(ops, M, K, ordered):
+    x = rnd(M, K, seed=1).to(torch.bfloat16)
+    for N in (2, 4, 6, 18, 34, 514, 1026, 4356):
+        w, b = rnd(N, K, seed=2, scale=0.05).to(torch.bfloat16), rnd(N, seed=3)
+        want = x.double() @ w.double().T
+        off = (K + 20) * 2 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30      # so many roundings of the sum of magnitudes
+        out = torch.full((M + 1, N), 7.0, device="cuda")
+        ops.gemm_blocksplit(out, dev(x), dev(w), dev(b), M, ordered=ordered)
+        got = out.cpu()
+        assert ((got[:M].double() - want - b.double()).abs() <= off + 2 ** -23 * (want.abs() + b.double().abs())).all(), N
+        assert (got[M] == 7).all()
+        pieces = torch.empty(M, N, device="cuda")
+        ops.gemm_blocksplit(pieces, to_pieces(dev(x)), dev(w), dev(b), M, x_pieces=True, ordered=ordered)
+        assert torch.equal(pieces.cpu(), got[:M]), N
+        g, u = want[:, 0::2], want[:, 1::2]
+        half = torch.empty(M, N // 2, device="cuda")
+        ops.gemm_blocksplit(half, dev(x), dev(w), None, M, gated=True, ordered=ordered)
+        assert ((half.cpu().double() - P.silu(g) * u).abs() <= 2 * (off[:, 0::2] * u.abs() + off[:, 1::2] * g.abs() + 2 ** -21 * (g * u).abs()) + 1e-12).all(), N
+        if ordered:
+            continue
+        resid, gain, xg = torch.ones(M, N, device="cuda"), torch.full((N,), 2.0, device="cuda"), torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        sq = torch.full((M, ops.gemm_blocksplit_blocks(M, N, K)), float("nan"), device="cuda")
+        ops.gemm_blocksplit(None, dev(x), dev(w), dev(b), M, residual=(resid, gain, xg, sq))
+        assert torch.equal(resid.cpu(), got[:M] + 1) and torch.equal(xg.cpu(), (2 * resid.cpu()).to(torch.bfloat16)), N
+        assert torch.allclose(sq.cpu().double().sum(1), (resid.cpu().double() ** 2).sum(1), rtol=(N + 3) * 2 ** -24), N
+
+
 # ------------------------------------------------------------------ random sizes
 def test_gemm_blocksplit_at_random_sizes(ops):
     """300 products of random sizes (1 to 32 rows, any N up to 6000, K in steps of 8 up to 20000), plain and gated,
