@@ -304,7 +304,7 @@ __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
   float angle = (float)p * freq;
   asm volatile("" : "+v"(angle));
   __builtin_amdgcn_sched_barrier(0);
-  if (early) attend_first<NT>(cursor, kpool, vpool, num_pages, KVH, kvh, kb_begin, lr, lg);
+  if (early) attend_first<NT, true>(cursor, kpool, vpool, num_pages, KVH, kvh, kb_begin, lr, lg);
   if (SLICED) {
     // The workgroup adds the slices of its heads' q once, four neighbouring values a thread, and hands
     // the sums round through LDS (the buffer the join uses at the end); every wavefront then takes its
@@ -408,8 +408,8 @@ __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
   if (has_keys) {
     bf16x8 qf[KS];
     rotate_q<NT>(qf, qx, lg, sn, c);
-    if (!early) attend_start<NT>(cursor, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin, lr, lg);
-    attend_walk<NT, false>(st, qf, cursor, pt, max_blocks, num_pages, kb_begin, (kb_end + 31) & ~31,
+    if (!early) attend_start<NT, true>(cursor, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin, lr, lg);
+    attend_walk<NT, false, true>(st, qf, cursor, pt, max_blocks, num_pages, kb_begin, (kb_end + 31) & ~31,
                            first, p, first, p, scale * 1.4426950408889634f, lr, lg);
   }
   float l = st.l;

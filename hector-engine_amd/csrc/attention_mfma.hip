@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(
   const bool full_tile = q0 + 15 < q_len;
   const int clear_lo = attn_first(last_pos, window, ex.chunk);
   const int clear_hi = full_tile ? first_pos : -1;
-  attend_range<NT, true, MODE>(st, qf, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, tile_lo & ~31,
+  attend_range<NT, true, false, MODE>(st, qf, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, tile_lo & ~31,
                    (last_pos & ~31) + 32, lo, hi, clear_lo, clear_hi, MODE == ATTN_SHAPED ? 1.f : scale * 1.4426950408889634f,
                    lr, lg);
   float l = st.l;
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(64) void attention_decode_kernel(
   if (MODE == ATTN_SHAPED) st.sh = attn_shape_of(ex, h, scale);
   st.pos = n_keys - 1;
   const int hi = n_keys - 1;
-  attend_range<NT, false, MODE>(st, qf, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin,
+  attend_range<NT, false, true, MODE>(st, qf, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin,
                    (kb_end + 31) & ~31, first, hi, first, hi, MODE == ATTN_SHAPED ? 1.f : scale * 1.4426950408889634f, lr, lg);
   float l = st.l;
   l = xor32_sum(xor16_sum(l));

@@ -26,7 +26,9 @@ struct bf16_t {
   uint16_t v;
 };
 
-// 16 bytes that nothing else of the launch reads, in loads of whole lines: the caches may drop them first.
+// 16 bytes that nothing else of the launch reads, in loads of whole lines: the caches may drop them first. (A plain read of 128 MB by 256
+// workgroups 23.7 us, so 21.7, and the small kernels behind it 0.2 to 0.6 us shorter, their code and arguments still at hand; in loads of
+// half lines 1.1 to 1.27 of the time, the other half being fetched again.)
 typedef uint32_t he_uint4v __attribute__((ext_vector_type(4)));
 template <typename T>
 __device__ __forceinline__ T he_load16_once(const void* p) {

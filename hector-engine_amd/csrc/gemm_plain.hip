@@ -227,7 +227,8 @@ __global__ __launch_bounds__(256, 2) void gemm_plain_mfma_kernel(
 // weight rows of 18,944, 2479 where this takes 53.) A wavefront fetches a stage of KS k
 // of its 16 weight rows (and activation rows) whole lines at a time, two stages ahead, into its own LDS region, the
 // 16-byte pieces of row r at their index xor r, from which the operand of lane (row, k mod 4) is read a float at a
-// time without bank conflicts. For weights of whole segments in aligned rows.
+// time without bank conflicts; the weights past the caches (he_load16_once; at 4 rows the 543 MB 98 -> 87 us). For weights of whole
+// segments in aligned rows.
 #define GP_MROWS_MAX_M 64
 template <int MT, int NW, int KS>
 __global__ __launch_bounds__(NW * 64) void gemm_plain_stream_kernel(
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_plain_stream_kernel(
     const int seg_ = wave + NW * ((ST_) / SPS);                                                      \
     if (seg_ < segments) {                                                                           \
       const int64_t k_ = (int64_t)seg_ * GP_SEG + ((ST_) % SPS) * KS;                                \
-      _Pragma("unroll") for (int t = 0; t < LD; ++t) wv[B_][t] = *reinterpret_cast<const gp_f32x4*>(wsrc[t] + k_); \
+      _Pragma("unroll") for (int t = 0; t < LD; ++t) wv[B_][t] = he_load16_once<gp_f32x4>(wsrc[t] + k_); \
       _Pragma("unroll") for (int i = 0; i < MT; ++i)                                                 \
         _Pragma("unroll") for (int t = 0; t < LD; ++t)                                               \
           if (real[i][t]) av[B_][i][t] = *reinterpret_cast<const gp_f32x4*>(asrc[i][t] + k_);        \
@@ -437,9 +438,9 @@ __global__ __launch_bounds__(256) void gemm_plain_rows_turned_kernel(
   for (int i = 0; i < 8; ++i) src[i] = W + (int64_t)min(n0 + 8 * i + lrow, N - 1) * ldw + k_begin + 4 * piece;
   float4 w0[8], w1[8];   // two chunks of 32 k on their way while a third is multiplied
 #pragma unroll
-  for (int i = 0; i < 8; ++i) w0[i] = *reinterpret_cast<const float4*>(src[i]);
+  for (int i = 0; i < 8; ++i) w0[i] = he_load16_once<float4>(src[i]);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) w1[i] = *reinterpret_cast<const float4*>(src[i] + 32);
+  for (int i = 0; i < 8; ++i) w1[i] = he_load16_once<float4>(src[i] + 32);
   float acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = 0.f;
@@ -466,12 +467,12 @@ __global__ __launch_bounds__(256) void gemm_plain_rows_turned_kernel(
   GP_TURN(w0, 0)
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) w0[i] = *reinterpret_cast<const float4*>(src[i] + 64);
+  for (int i = 0; i < 8; ++i) w0[i] = he_load16_once<float4>(src[i] + 64);
   __builtin_amdgcn_sched_barrier(0);
   GP_TURN(w1, 1)
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) w1[i] = *reinterpret_cast<const float4*>(src[i] + 96);
+  for (int i = 0; i < 8; ++i) w1[i] = he_load16_once<float4>(src[i] + 96);
   __builtin_amdgcn_sched_barrier(0);
   GP_TURN(w0, 2)
   GP_TURN(w1, 3)

@@ -450,7 +450,8 @@ extern "C" int he_routed_act(void* out, const void* gate_up, const void* dense_f
 // ---- the chosen experts alone, for steps of very few rows ---------------------------------------
 // Where a step's rows choose fewer experts than there are, the two products over all experts read weights
 // nobody asked for. These two kernels walk only the chosen experts' rows of the same fused matrices (bf16):
-// a wavefront an output, the lanes along K with 16-byte loads, sums in fp32.
+// a wavefront an output, the lanes along K with 16-byte loads (the weights' past the caches: 2 rows of 4 choices among experts of 2048 over
+// 2048 24.9 -> 23.3 us and 16.6 -> 15.7), sums in fp32.
 __device__ __forceinline__ float dot8_bf16(const uint4& a, const uint4& b, float acc) {
   const uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -486,8 +487,8 @@ __global__ __launch_bounds__(256) void chosen_gate_up_kernel(uint16_t* __restric
 #pragma unroll 4
     for (int c = lane * 8; c < D; c += 512) {
       const uint4 xv = *reinterpret_cast<const uint4*>(xr + c * x_step);
-      g = dot8_bf16(*reinterpret_cast<const uint4*>(wg + c), xv, g);
-      u = dot8_bf16(*reinterpret_cast<const uint4*>(wg + D + c), xv, u);
+      g = dot8_bf16(he_load16_once<uint4>(wg + c), xv, g);
+      u = dot8_bf16(he_load16_once<uint4>(wg + D + c), xv, u);
     }
   }
   g = wave_sum(g);
@@ -518,12 +519,12 @@ __global__ __launch_bounds__(256) void chosen_down_kernel(uint16_t* __restrict__
     const uint16_t* hr = h + (row * top + k) * I;
 #pragma unroll 4
     for (int c = lane * 8; c < I; c += 512)
-      acc = dot8_bf16(*reinterpret_cast<const uint4*>(w + c), *reinterpret_cast<const uint4*>(hr + c), acc);
+      acc = dot8_bf16(he_load16_once<uint4>(w + c), *reinterpret_cast<const uint4*>(hr + c), acc);
   }
   const uint16_t* ws = down + (int64_t)d * ldw + (int64_t)real * I;
   const uint16_t* hs = h + (int64_t)gridDim.y * top * I + row * shared;
   for (int c = lane * 8; c < shared; c += 512)
-    acc = dot8_bf16(*reinterpret_cast<const uint4*>(ws + c), *reinterpret_cast<const uint4*>(hs + c), acc);
+    acc = dot8_bf16(he_load16_once<uint4>(ws + c), *reinterpret_cast<const uint4*>(hs + c), acc);
   acc = wave_sum(acc);
   if (lane == 0)
     out[row * D + d] = float_to_bf16_bits(
