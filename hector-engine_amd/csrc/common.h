@@ -48,6 +48,22 @@ __device__ __forceinline__ uint16_t float_to_bf16_bits(float f) {
   return (uint16_t)(u >> 16);
 }
 
+// A matrix instruction's operand of 16 weight rows has a row a lane of each group of 16, so loading it as it lies takes half a line
+// of 16 rows. Loaded instead as whole lines of 8 rows, the lanes 8 .. 15 the other half of the rows of the lanes 0 .. 7 (x), and of the
+// next 8 rows (y), it takes its place by this exchange: x of the upper lanes with y of the lower ones.
+template <typename T>
+__device__ __forceinline__ void he_halves_to_rows(T& x, T& y, bool upper) {
+  static_assert(sizeof(T) == 16, "16 bytes");
+  he_uint4v a = __builtin_bit_cast(he_uint4v, x), b = __builtin_bit_cast(he_uint4v, y);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(upper ? a[i] : b[i]), 0x128, 0xf, 0xf, true);   // lane l + 8 of 16
+    a[i] = upper ? other : a[i];
+    b[i] = upper ? b[i] : other;
+  }
+  x = __builtin_bit_cast(T, a), y = __builtin_bit_cast(T, b);
+}
+
 // two floats to two bf16 in one register, round to nearest even (v_cvt_pk_bf16_f32)
 typedef __bf16 he_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float he_float2 __attribute__((ext_vector_type(2)));

@@ -93,7 +93,7 @@ __device__ __forceinline__ void bs_store_pieces(uint16_t* base, int M, int m, in
 // line each. Whole lines can be asked for past the caches (he_load16_once), which half lines cannot: the other half would be
 // fetched twice. 37888 x 3584 at 1 row 50.8 -> 42 us (6.4 TB/s), at 8 rows 52.5 -> 42, 3584 x 3584 at 1 row 9.6 -> 6.2.
 // SP = 0 keeps each sum in the order this product had before: a unit of 64 k is two instructions, whose lanes take the halves of 16
-// neighbouring k. For 17 to 32 rows, and where a caller asks for that order (`ordered`; also the K slices and, by workgroup, the
+// neighbouring k (loaded as whole lines all the same, see he_halves_to_rows). For 17 to 32 rows, and where a caller asks for that order (`ordered`; also the K slices and, by workgroup, the
 // turn each wavefront begins at are then those it had).
 template <int SP>
 struct BsLanes {
@@ -216,9 +216,12 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_
   const char* const wb = reinterpret_cast<const char*>(W + (int64_t)n0 * K);
   const char* const xb = reinterpret_cast<const char*>(X);
   const int k_lane = SP == 0 ? 16 * lg : 8 * ((lg << SP) | (lr & (L::PARTS - 1)));    // this lane's first k of a unit
-  uint32_t wo[NA], xo[MT];
+  uint32_t wo[L::H][NA], xo[MT];
+  const bool upper = (lr & 8) != 0;
 #pragma unroll
-  for (int a = 0; a < NA; ++a) wo[a] = 2u * (uint32_t)(min(row * NA + a, n_end - n0 - 1) * K);
+  for (int h = 0; h < L::H; ++h)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) wo[h][a] = 2u * (uint32_t)(min((SP == 0 ? (lr & 7) + 8 * h : row) * NA + a, n_end - n0 - 1) * K);
 #pragma unroll
   for (int t = 0; t < MT; ++t) xo[t] = 2u * (uint32_t)(min(t * L::RT + xrow, M - 1) * (PIECES ? 8 : K));
   const uint32_t xk = PIECES ? 2 * M : 2;                         // piece-major X: the piece of 8 k from k on lies at k M (+ 8 row)
@@ -239,12 +242,17 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_
 #pragma unroll
       for (int h = 0; h < L::H; ++h) {
         const uint32_t k = min(min(u + s, u1 - 1) * L::KM + k_lane + 8 * h, K - 8);
+        const uint32_t kw = SP == 0 ? min(min(u + s, u1 - 1) * L::KM + k_lane + (lr & 8), K - 8) : k;      // (see he_halves_to_rows)
 #pragma unroll
-        for (int a = 0; a < NA; ++a)
-          f.a[s][h][a] = SP > 0 ? he_load16_once<bf16x8>(wb + (wo[a] + 2 * k)) : bs_load8(wb + (wo[a] + 2 * k));
+        for (int a = 0; a < NA; ++a) f.a[s][h][a] = he_load16_once<bf16x8>(wb + (wo[h][a] + 2 * kw));
 #pragma unroll
         for (int t = 0; t < MT; ++t) f.b[s][h][t] = bs_load8(xb + (xo[t] + k * xk));
       }
+  };
+  auto in_place = [&](BsFrags<MT, NA, S, L::H>& f, int s) {
+    if constexpr (SP == 0)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) he_halves_to_rows(f.a[s][0][a], f.a[s][1][a], upper);
   };
   auto multiply_unit = [&](const BsFrags<MT, NA, S, L::H>& f, int s) {
 #pragma unroll
@@ -255,15 +263,16 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_
         for (int t = 0; t < MT; ++t)
           acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[s][h][a], f.b[s][h][t], acc[a][t], 0, 0, 0);
   };
-  auto multiply = [&](const BsFrags<MT, NA, S, L::H>& f) {
+  auto multiply = [&](BsFrags<MT, NA, S, L::H>& f) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) multiply_unit(f, s);
+    for (int s = 0; s < S; ++s) in_place(f, s), multiply_unit(f, s);
   };
   auto multiply_last = [&](BsFrags<MT, NA, S, L::H>& f, int u) {
     const bf16x8 zero = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
 #pragma unroll
     for (int s = 0; s < S; ++s)
       if (u + s < u1) {
+        in_place(f, s);
         if ((u + s + 1) * L::KM > K) {
 #pragma unroll
           for (int h = 0; h < L::H; ++h) {

@@ -34,20 +34,21 @@ struct RowsA {
   bf16x8 a[2][R][2];
 };
 
+// Whole lines of 8 rows a load, past the caches: lanes 8 .. 15 of a group have the second half of the 16 k of the rows of the lanes
+// 0 .. 7 (wp[r][0]) and of the 8 rows behind them (wp[r][1]); rows_multiply exchanges them into place.
 // TAIL: the chunk may reach past k_end (such loads read a safe address and give zeros).
 template <int R, bool TAIL>
-__device__ __forceinline__ void rows_load_a(RowsA<R>& f, const uint16_t* const* wp, const uint16_t* safe,
-                                            int k, int lg, int k_end) {
+__device__ __forceinline__ void rows_load_a(RowsA<R>& f, const uint16_t* const (*wp)[2], const uint16_t* safe,
+                                            int k, int kl, int k_end) {
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int kk = k + 64 * u + 16 * lg + 8 * h;
-      const bool ok = !TAIL || kk + 8 <= k_end;
+      const bool ok = !TAIL || k + 64 * u + kl + 8 <= k_end;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const uint16_t* p = ok ? wp[r] + k + 64 * u + 8 * h : safe;
-        uint4 v = *reinterpret_cast<const uint4*>(p);
+        const uint16_t* p = ok ? wp[r][h] + k + 64 * u : safe;
+        uint4 v = he_load16_once<uint4>(p);
         if (TAIL && !ok) v = make_uint4(0, 0, 0, 0);
         f.a[u][r][h] = __builtin_bit_cast(bf16x8, v);
       }
@@ -92,10 +93,12 @@ __device__ __forceinline__ void rows_store_b(const uint4 (&st)[(MT * 256 + NT - 
 }
 
 template <int MT, int R>
-__device__ __forceinline__ void rows_multiply(const RowsA<R>& f, const unsigned char* buf, int lane,
+__device__ __forceinline__ void rows_multiply(RowsA<R>& f, const unsigned char* buf, int lane,
                                               floatx4 (&acc)[R][MT]) {
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < 2; ++u) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) he_halves_to_rows(f.a[u][r][0], f.a[u][r][1], (lane & 8) != 0);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       bf16x8 b[MT];
@@ -109,6 +112,7 @@ __device__ __forceinline__ void rows_multiply(const RowsA<R>& f, const unsigned 
         for (int t = 0; t < MT; ++t)
           acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[u][r][h], b[t], acc[r][t], 0, 0, 0);
     }
+  }
 }
 
 template <typename TC>
@@ -173,9 +177,12 @@ __global__ __launch_bounds__(64 * NWV) void gemm_rows_kernel(
   const int k_end = min(K, k_begin + kslice);
   const int nchunks = k_end > k_begin ? (k_end - k_begin + ROWS_KC - 1) / ROWS_KC : 0;
 
-  const uint16_t* wp[R];
+  const int kl = 16 * lg + (lr & 8);       // this lane's k of a load
+  const uint16_t* wp[R][2];
 #pragma unroll
-  for (int r = 0; r < R; ++r) wp[r] = W + (int64_t)min(n_wave + 16 * r + lr, n_end - 1) * K + lg * 16;
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) wp[r][h] = W + (int64_t)min(n_wave + 16 * r + 8 * h + (lr & 7), n_end - 1) * K + kl;
 
   floatx4 acc[R][MT];
 #pragma unroll
@@ -219,7 +226,7 @@ __global__ __launch_bounds__(64 * NWV) void gemm_rows_kernel(
     if (WORK_) rows_multiply<MT, R>(A_, xs[B_], lane, acc);                                        \
     if (!(GUARD_) || jj + 1 < nchunks) rows_store_b<MT, NT>(N_, xs[(B_) ^ 1]);                     \
     if (!(GUARD_) || jj + 3 < nchunks) rows_load_b<MT, NT, XP, TAIL>(N_, X, M, K, kof(jj + 3), k_end); \
-    if ((WORK_) && (!(GUARD_) || jj + 2 < nchunks)) rows_load_a<R, TAIL>(A_, wp, W, kof(jj + 2), lg, k_end); \
+    if ((WORK_) && (!(GUARD_) || jj + 2 < nchunks)) rows_load_a<R, TAIL>(A_, wp, W, kof(jj + 2), kl, k_end); \
     __syncthreads();                                                                               \
   }
   int j = 0;
@@ -235,12 +242,12 @@ __global__ __launch_bounds__(64 * NWV) void gemm_rows_kernel(
     __builtin_amdgcn_sched_barrier(0);
     rows_load_b<MT, NT, XP, TAIL>(bst1, X, M, K, kof(1), k_end);
     __builtin_amdgcn_sched_barrier(0);
-    rows_load_a<R, TAIL>(a0, wp, W, kof(0), lg, k_end);
+    rows_load_a<R, TAIL>(a0, wp, W, kof(0), kl, k_end);
     __builtin_amdgcn_sched_barrier(0);
     rows_store_b<MT, NT>(bst0, xs[0]);
     rows_load_b<MT, NT, XP, TAIL>(bst0, X, M, K, kof(2), k_end);
     __builtin_amdgcn_sched_barrier(0);
-    rows_load_a<R, TAIL>(a1, wp, W, kof(1), lg, k_end);
+    rows_load_a<R, TAIL>(a1, wp, W, kof(1), kl, k_end);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     for (; j + 4 < nchunks; j += 2) {
@@ -256,10 +263,10 @@ __global__ __launch_bounds__(64 * NWV) void gemm_rows_kernel(
     if (nchunks > 0) {
       rows_load_b<MT, NT, XP, TAIL>(bst0, X, M, K, kof(0), k_end);
       if (nchunks > 1) rows_load_b<MT, NT, XP, TAIL>(bst1, X, M, K, kof(1), k_end);
-      if (n_wave < n_end) rows_load_a<R, TAIL>(a0, wp, W, kof(0), lg, k_end);
+      if (n_wave < n_end) rows_load_a<R, TAIL>(a0, wp, W, kof(0), kl, k_end);
       rows_store_b<MT, NT>(bst0, xs[0]);
       if (nchunks > 2) rows_load_b<MT, NT, XP, TAIL>(bst0, X, M, K, kof(2), k_end);
-      if (n_wave < n_end && nchunks > 1) rows_load_a<R, TAIL>(a1, wp, W, kof(1), lg, k_end);
+      if (n_wave < n_end && nchunks > 1) rows_load_a<R, TAIL>(a1, wp, W, kof(1), kl, k_end);
     }
     __syncthreads();
     if (n_wave < n_end) {
