@@ -21,6 +21,7 @@ import dataclasses
 import numpy as np
 import torch
 
+from ..kernels import ops
 from ..parts.base import KVNeed, LayerCache
 from .pages import PAGE_TOKENS, CacheError, CacheFull, GroupPages, SlotBook, blocks_for  # noqa: F401
 
@@ -35,8 +36,7 @@ class RunPlan:
 
 
 class _Group:
-    def __init__(self, need: KVNeed, runs: list[int], num_pages: int, max_slots: int,
-                 max_blocks: int, dtype, device):
+    def __init__(self, need: KVNeed, runs: list[int], num_pages: int, dtype, device, tables: "_Tables", index: int):
         self.need = need
         self.runs = runs
         # zero-filled once (as the reference's cache is: src/kv_cache.hpp:161-203): a masked
@@ -44,9 +44,60 @@ class _Group:
         # a page is as large as the mixers of the group say; what lies where inside it is theirs
         self.kpool = torch.zeros((len(runs), num_pages, need.kv_heads, need.k_elems), dtype=dtype, device=device)
         self.vpool = torch.zeros((len(runs), num_pages, need.kv_heads, need.v_elems), dtype=dtype, device=device)
-        self.page_table = torch.full((max_slots, max_blocks), -1, dtype=torch.int32, device=device)
+        self._tables = tables
+        self._table = tables.device[index]
         # the same table on the host: a step can take its sequences' rows along with its metadata
-        self.host_table = np.full((max_slots, max_blocks), -1, dtype=np.int32)
+        self.host_table = tables.host[index]
+
+    @property
+    def page_table(self) -> torch.Tensor:
+        self._tables.flush()
+        return self._table
+
+
+class _Tables:
+    """The groups' page tables [groups][slots][blocks], on the host and on the device. Entries change on the host at once and
+    on the device all together before the next step (flush): one copy from pinned memory and one launch behind what is
+    queued. (Written slot by slot, from pageable memory, every release, truncation and new page made the host wait for
+    all queued steps and left the GPU idle for 60 us behind them: 64 sequences cut back after eight steps, 21 of them by a
+    page, 1.3 ms of 17.2.)"""
+
+    def __init__(self, groups: int, max_slots: int, max_blocks: int, device):
+        self.host = np.full((groups, max_slots, max_blocks), -1, dtype=np.int32)
+        self.device = torch.full((groups, max_slots, max_blocks), -1, dtype=torch.int32, device=device)
+        self._flat = self.host.reshape(-1)
+        self._dirty: set[int] = set()
+        self._pinned: list[torch.Tensor | None] = [None] * 4       # in turn, each free again when its event has passed
+        self._events: list[torch.cuda.Event | None] = [None] * 4
+        self._next = 0
+
+    def write(self, index: int, page: int) -> None:
+        self._flat[index] = page
+        self._dirty.add(index)
+
+    def flush(self) -> None:
+        n = len(self._dirty)
+        if n == 0:
+            return
+        idx = np.fromiter(self._dirty, dtype=np.int32, count=n)
+        self._dirty.clear()
+        if self.device.device.type == "cpu":
+            self.device.view(-1)[torch.from_numpy(idx).long()] = torch.from_numpy(self._flat[idx])
+            return
+        i = self._next
+        self._next = (i + 1) % len(self._pinned)
+        if self._events[i] is not None:
+            self._events[i].synchronize()
+        if self._pinned[i] is None or self._pinned[i].numel() < 2 * n:
+            self._pinned[i] = torch.empty(max(256, 1 << (2 * n - 1).bit_length()), dtype=torch.int32, pin_memory=True)
+        staged = self._pinned[i][:2 * n]
+        staged.numpy()[:n] = idx
+        staged.numpy()[n:] = self._flat[idx]
+        entries = torch.empty(2 * n, dtype=torch.int32, device=self.device.device)
+        entries.copy_(staged, non_blocking=True)
+        self._events[i] = torch.cuda.Event()
+        self._events[i].record()
+        ops.scatter_i32(self.device, entries, n)
 
 
 class PagedCache:
@@ -80,8 +131,8 @@ class PagedCache:
                 if plan.cache_from not in self.run_group or plan.cache_from >= r:
                     raise CacheError(f"run {r} reads the cache of run {plan.cache_from}, "
                                      "which is not an earlier run with a cache of its own")
-        self.groups = [_Group(k, m, self.num_pages, self.max_slots, self.max_blocks, dtype, device)
-                       for k, m in zip(keys, members)]
+        self.tables = _Tables(len(keys), self.max_slots, self.max_blocks, device)
+        self.groups = [_Group(k, m, self.num_pages, dtype, device, self.tables, i) for i, (k, m) in enumerate(zip(keys, members))]
         self.book = SlotBook(self.max_slots, self.max_blocks,
                              [GroupPages(self.num_pages, k.window, f"{i}", k.chunk) for i, k in enumerate(keys)])
 
@@ -139,11 +190,12 @@ class PagedCache:
             for s, n in growth:
                 if n < self.book.length[s]:
                     raise CacheError(f"slot {s}: cannot shrink from {self.book.length[s]} to {n}")
-            return
-        added = []
-        for s, n in growth:
-            added += self.book.reserve(s, n)
-        self._write(added)
+        else:
+            added = []
+            for s, n in growth:
+                added += self.book.reserve(s, n)
+            self._write(added)
+        self.tables.flush()
 
     def commit(self, growth: list[tuple[int, int]]) -> None:
         cleared = []
@@ -152,15 +204,8 @@ class PagedCache:
         self._clear(cleared)
 
     def _write(self, entries) -> None:
-        by_group: dict[int, tuple[list, list]] = {}
         for gi, slot, block, page in entries:
-            idx, val = by_group.setdefault(gi, ([], []))
-            idx.append(slot * self.max_blocks + block)
-            val.append(page)
-        for gi, (idx, val) in by_group.items():
-            self.groups[gi].host_table.reshape(-1)[idx] = val
-            packed = torch.tensor([idx, val], dtype=torch.int64).to(self.device)
-            self.groups[gi].page_table.view(-1).index_copy_(0, packed[0], packed[1].to(torch.int32))
+            self.tables.write((gi * self.max_slots + slot) * self.max_blocks + block, page)
 
     def _clear(self, entries) -> None:
         self._write([(gi, slot, block, -1) for gi, slot, block in entries])

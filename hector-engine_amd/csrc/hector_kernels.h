@@ -426,6 +426,8 @@ int he_qk_head_norm(void* out, int64_t out_stride, const void* in, int64_t in_st
 
 // ---- whole rows of the stream (stream_ops.hip) ---------------------------------------------------------
 // kept_f32 plane n - 1 = resid; resid = sum_{j < n} coeffs[j] * plane j
+// table[entries[i]] = entries[n + i] for i < n (distinct indexes; those outside [0, size) are passed over).
+int he_scatter_i32(void* table_i32, const void* entries_i32, int n, int64_t size, void* stream);
 int he_depth_mix(void* resid_f32, void* kept_f32, int64_t plane, const void* coeffs, int c_dtype, int n, int64_t count,
                  void* stream);
 // out = a + sigmoid(x . g) * b, row by row

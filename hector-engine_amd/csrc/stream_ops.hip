@@ -1,9 +1,27 @@
-// Two small operations on whole rows of the residual stream's width:
+// Small operations around the layers. On whole rows of the residual stream's width:
 //   he_depth_mix   the stream that goes on after a layer as a weighted sum of the embedding's output and
 //                  of every layer's result so far
 //   he_gated_add   out = a + sigmoid(x . g) * b, one number a row in front of b
+// and on the page tables:
+//   he_scatter_i32 table[index] = value
 #include "common.h"
 #include "hector_kernels.h"
+
+// entries: n indexes, then n values. Bound by its launch: a step's new and given-back pages are some tens of entries.
+__global__ __launch_bounds__(256) void scatter_i32_kernel(int32_t* __restrict__ table, const int32_t* __restrict__ entries, int n,
+                                                          int64_t size) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int at = entries[i];
+  if (at >= 0 && at < size) table[at] = entries[n + i];
+}
+
+extern "C" int he_scatter_i32(void* table_i32, const void* entries_i32, int n, int64_t size, void* stream) {
+  HE_REQUIRE(n >= 0 && size >= 0 && n <= (1 << 30), "he_scatter_i32: bad sizes n=%d", n);
+  if (n == 0) return 0;
+  scatter_i32_kernel<<<(n + 255) / 256, 256, 0, (hipStream_t)stream>>>((int32_t*)table_i32, (const int32_t*)entries_i32, n, size);
+  return he_check_launch("he_scatter_i32");
+}
 
 // kept: fp32 [n or more][count] (plane j at j * plane elements): planes 0 .. n - 2 hold the earlier results.
 // resid (fp32 [count]) holds the newest result: it is stored as plane n - 1, and resid becomes

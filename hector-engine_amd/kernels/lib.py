@@ -95,6 +95,7 @@ _SIGNATURES = {
                             c_int, c_int, c_ptr],
     "he_polynorm": [c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_f32, c_int, c_ptr],
     "he_qk_head_norm": [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_f32, c_int, c_int, c_int, c_ptr],
+    "he_scatter_i32": [c_ptr, c_ptr, c_int, c_i64, c_ptr],
     "he_depth_mix": [c_ptr, c_ptr, c_i64, c_ptr, c_int, c_int, c_i64, c_ptr],
     "he_gated_add": [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_int, c_int, c_int, c_int, c_ptr],
     "he_head_product": [c_ptr, c_i64, c_i64, c_ptr, c_i64, c_i64, c_ptr, c_int, c_int, c_int, c_int, c_int, c_ptr, c_i64,

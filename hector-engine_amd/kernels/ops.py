@@ -104,6 +104,16 @@ def gather_rows_f32(out, src, rows_idx, n_out: int, n_src: int) -> None:
                                     n_src, _stream()))
 
 
+@_op("scatter_i32")
+def scatter_i32(table, entries, n: int) -> None:
+    """table.view(-1)[entries[i]] = entries[n + i] for i < n (distinct indexes)."""
+    _need(table, "table", torch.int32)
+    _need(entries, "entries", torch.int32)
+    if entries.numel() < 2 * n or table.numel() > 2 ** 31 - 1:
+        raise ValueError("scatter_i32: fewer entries than n indexes and n values, or a table beyond 32-bit indexes")
+    _lib.check(_lib.load().he_scatter_i32(table.data_ptr(), entries.data_ptr(), n, table.numel(), _stream()))
+
+
 @_op("residual_add")
 def residual_add(resid_f32, delta, rows: int, scale: float = 1.0, delta2=None) -> None:
     """resid += scale * (delta + delta2) (delta2 None: delta alone)."""

@@ -861,3 +861,19 @@ def test_state_of_fixed_size_under_graph_replay(fw, toys, tmp_path, dtype):
     mixer = type(eng.model.blocks[1].mixer)
     assert mixer.seen_hints == {False, True}
     assert {hints[-1] for _, hints in eng._buckets} == {False, True}
+
+
+@pytest.mark.parametrize("count", [1, 2, 255, 256, 257, 5000])
+def test_page_table_entries_written_together(fw, count):
+    """Entries over three groups, some of them twice before the device hears of them, more than the staging buffer held before
+    and fewer again: the device's table is the host's, and every other entry stays."""
+    from hector_engine_amd.cache.paged import _Tables
+    t = _Tables(3, 40, 50, torch.device("cuda:0"))
+    g = torch.Generator().manual_seed(count)
+    for n in (count, 1, 2 * count, 7):
+        for i in torch.randperm(6000, generator=g)[:min(n, 6000)].tolist():
+            t.write(i, 1)
+            t.write(i, int(i % 97) - 1)
+        t.flush()
+        t.flush()
+    assert (t.device.cpu().numpy() == t.host).all() and (t.host.max() > 0 or count < 3)
