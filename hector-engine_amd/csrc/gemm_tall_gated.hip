@@ -2,7 +2,5 @@
 #include "gemm_tall_tiles.h"
 
 int gt_run_gated(const GtCase& c, int tile, int mtiles, hipStream_t s) {
-#define GT_CASE(BM, BN, NX, NW) if (tile == ((BM) << 16 | (BN))) return gt_run<BM, BN, NX, NW, GT_GATED, false>(c, mtiles, s);
-  GT_TILES(GT_CASE)
-  return -1;
+  return gt_run_tile<GT_GATED, false>(c, tile, mtiles, s);
 }

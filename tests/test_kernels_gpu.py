@@ -1319,3 +1319,34 @@ def test_plain_products_in_whole_rounds_give_the_bits_of_the_other_kernels(ops, 
     size = a.double().abs() @ w.double().abs().T + b.double().abs()
     # chains of 128 and the sums of segments: so many roundings of at most the sum of magnitudes
     assert ((out[:M].double() - want).abs() <= (128 + K / 128 + 2) * 2 ** -24 * size).all()
+
+
+# ------------------------------------------------------------------ single rows of tiles
+@pytest.mark.parametrize("tile", [(256, 160), (256, 224), (256, 256), (256, 192), (128, 288), (128, 256), (128, 224), (128, 160)])
+@pytest.mark.parametrize("N,K", [(1500, 192), (4100, 640), (452, 64)])
+def test_a_single_row_of_tiles_gives_the_bits_of_many(ops, tile, N, K):
+    """Rows on both sides of every height a single row of tiles is made in, more than one round of columns and columns that end inside
+    a tile; a taller product runs the same tile's kernel for several rows of tiles."""
+    kw = dict(bm=tile[0], bn=tile[1])
+    w, x = dev(rnd(N, K, seed=1).to(torch.bfloat16)), dev(rnd(520, K, seed=2).to(torch.bfloat16))
+    whole = torch.empty(520, N, dtype=torch.bfloat16, device="cuda")
+    ops.gemm_tall(whole, x, w, None, 520, **kw)
+    # sums of K products in 32 bits, then a rounding to bf16
+    want = x.double() @ w.double().T
+    assert ((whole.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -24 * K * (x.double().abs() @ w.double().abs().T)).all()
+    gated = torch.empty(520, N // 2, dtype=torch.bfloat16, device="cuda")
+    ops.gemm_tall(gated, x, w, None, 520, act=(1.0, 0.0, 0.0, 0.0), **kw)
+    sliced = torch.empty(2, 520, N, device="cuda") if K % 128 == 0 else None
+    if sliced is not None:
+        ops.gemm_tall(sliced, x, w, None, 520, slices=2, **kw)
+    for M in (1, 65, 128, 129, 160, 161, 192, 193, 224, 225, 256):
+        out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_tall(out, x, w, None, M, **kw)
+        assert torch.equal(out[:M], whole[:M]) and (out[M] == 7).all(), M
+        act = torch.full((M + 1, N // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_tall(act, x, w, None, M, act=(1.0, 0.0, 0.0, 0.0), **kw)
+        assert torch.equal(act[:M], gated[:M]) and (act[M] == 7).all(), M
+        if sliced is not None:
+            part = torch.full((2, M, N), 7.0, device="cuda")
+            ops.gemm_tall(part, x, w, None, M, slices=2, **kw)
+            assert torch.equal(part, sliced[:, :M]), M
