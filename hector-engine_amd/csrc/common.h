@@ -147,7 +147,7 @@ __device__ __forceinline__ float xor16_sum(float x) {
 // permutations inside a quad. All 64 lanes must be active.
 template <int CTRL>
 __device__ __forceinline__ unsigned dpp_bits(unsigned x) {
-  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);      // (true: no register is cleared for it first)
 }
 // OFF: 8, 4, 2 or 1
 template <int OFF>

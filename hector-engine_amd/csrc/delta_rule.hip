@@ -16,7 +16,12 @@
 //     u = beta (v - g a),   o = g b + u (k . q),   S <- g S + k u^T,
 // which is the recurrence above with the read-out written in terms of the old S: the write is off the path
 // from one token's sums to its output. The rows' k, q and scalars are staged in LDS a block of 8 rows at a
-// time, the next block's loads in flight while this block is walked. Every token's sums are formed in one
+// time, the next block's loads in flight while this block is walked. What bounds it is the chain and
+// the vector instructions of the two wavefronts a SIMD has, some 45 each a row: a row's operands are read from LDS while the row
+// before is walked, no branch stands inside a block, one lane a row stores its result, the two butterflies go on in one register
+// after their first step (16 lanes), and the workgroups of a sequence lie together in the grid, so that a SIMD has
+// wavefronts of different sequences (with the sequence as the first index an XCD had one sequence, both wavefronts of a
+// SIMD the longest). Four sequences of 3001 rows in all, 16 heads of 128 x 128: 390 -> 305 us, the same bits. Every token's sums are formed in one
 // order however the rows were cut into steps, so a sequence's results do not depend on the cut. A
 // sequence's S lies in its row of the state area as [head][value dim][NG * KPT]: each lane's share is
 // contiguous.
@@ -108,45 +113,28 @@ __device__ __forceinline__ float dr_group_sum(float v, int NG) {
   return v;
 }
 
-// What a lane moves of the block that begins at row T0: its float4 of the rows' k | q, a row's scalars (lanes below
-// DR_ROWS; rows beyond the sequence get beta 0, g 1: they leave S as it is), and its own value dim of every row.
-// Rows beyond the sequence read its last row.
-#define DR_FETCH(T0)                                                                                     \
-  {                                                                                                      \
-    _Pragma("unroll") for (int i = 0; i < NLD; ++i) {                                                    \
-      const int f = min(lane + 64 * i, BLOCK_F4 - 1);                                                    \
-      const int t = f / ROW_F4, c = f - t * ROW_F4;                                                      \
-      const float4 w = kq4[((int64_t)min((T0) + t, r1 - 1) * G + kv) * ROW_F4 + c];                      \
-      ld[4 * i] = w.x, ld[4 * i + 1] = w.y, ld[4 * i + 2] = w.z, ld[4 * i + 3] = w.w;                    \
-    }                                                                                                    \
-    const int tr = (T0) + min(lane, DR_ROWS - 1);                                                        \
-    const float4 w = head4[(int64_t)min(tr, r1 - 1) * H + h];                                            \
-    sc_beta = tr >= r1 ? 0.f : w.x, sc_g = tr >= r1 ? 1.f : w.y, sc_kq = tr >= r1 ? 0.f : w.z;           \
-    _Pragma("unroll") for (int t = 0; t < DR_ROWS; ++t)                                                  \
-        ld_v[t] = to_float(vp[(int64_t)min((T0) + t, r1 - 1) * in_stride]);                              \
-  }
-
 template <typename T, int KPT, int NG>
 __global__ __launch_bounds__(64) void delta_scan_kernel(
     float* __restrict__ y, const float* __restrict__ kq_in, const float* __restrict__ head_in,
     const T* __restrict__ v_in, int64_t in_stride, uint8_t* __restrict__ state, int64_t state_stride,
     int64_t state_offset, const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_slot, int H, int G,
-    int e) {
+    int e, int tiles) {
   constexpr int DP = NG * KPT;
   constexpr int ROW_F4 = DP / 2;                       // float4 of one row's k | q
   constexpr int BLOCK_F4 = DR_ROWS * ROW_F4;
   constexpr int NLD = (BLOCK_F4 + 63) / 64;            // float4 a lane moves per block
   constexpr int PER_BLOCK = 64 / NG;                   // value dims of this wavefront
+  constexpr bool PAIRED = NG == 16;                    // (16 = 2 DR_ROWS lanes store 8 rows)
   __shared__ float4 kq_s[BLOCK_F4];
   __shared__ float4 sc_s[DR_ROWS];
-  const int seq = blockIdx.x, h = blockIdx.y;
+  const int tile = blockIdx.x % tiles, h = blockIdx.x / tiles % H, seq = blockIdx.x / (tiles * H);
   const int slot = seq_slot[seq];
   if (slot < 0) return;
   const int r0 = cu_seqlens[seq], r1 = cu_seqlens[seq + 1];
   if (r1 <= r0) return;
   const int lane = threadIdx.x;
   const int g_lane = lane & (NG - 1);
-  const int j = blockIdx.z * PER_BLOCK + lane / NG;    // this lane's value dim
+  const int j = tile * PER_BLOCK + lane / NG;    // this lane's value dim
   const bool has = j < e;
   const int kv = h / (H / G);                          // the head's q/k group
   float* S_row = reinterpret_cast<float*>(state + (int64_t)slot * state_stride + state_offset) +
@@ -154,7 +142,8 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(
   float S[KPT];
 #pragma unroll
   for (int i = 0; i < KPT; ++i) S[i] = has ? S_row[i] : 0.f;
-  const T* vp = v_in + (int64_t)h * e + (has ? j : 0);
+  const T* vp = v_in + (int64_t)h * e;
+  const uint32_t j_lane = has ? j : 0;
   const float4* kq4 = reinterpret_cast<const float4*>(kq_in);
   const float4* head4 = reinterpret_cast<const float4*>(head_in);
   float* yp = y + (int64_t)h * e + (has ? j : 0);
@@ -162,7 +151,31 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(
 
   float ld[4 * NLD], sc_beta, sc_g, sc_kq;
   float ld_v[DR_ROWS];
-  DR_FETCH(r0)
+  // What a lane moves of the block that begins at row t0: its float4 of the rows' k | q, a row's scalars (lanes below
+  // DR_ROWS; rows beyond the sequence get beta 0, g 1: they leave S as it is), and its own value dim of every row.
+  // Rows beyond the sequence read its last row. (A row's address is the wavefront's, a lane adds 32 bits.)
+  auto fetch = [&](int t0) {
+    auto row = [&](int t) { return (int64_t)min(t0 + t, r1 - 1); };
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      float4 w;
+      if constexpr (ROW_F4 % 64 == 0) {
+        w = (kq4 + (row(64 * i / ROW_F4) * G + kv) * ROW_F4 + 64 * i % ROW_F4)[lane];
+      } else {
+        const int f = min(lane + 64 * i, BLOCK_F4 - 1);
+        const int t = f / ROW_F4, c = f - t * ROW_F4;
+        w = kq4[(row(t) * G + kv) * ROW_F4 + c];
+      }
+      ld[4 * i] = w.x, ld[4 * i + 1] = w.y, ld[4 * i + 2] = w.z, ld[4 * i + 3] = w.w;
+    }
+    const int tr = min(lane, DR_ROWS - 1);
+    const float4 w = head4[row(tr) * H + h];
+    const bool beyond = t0 + tr >= r1;
+    sc_beta = beyond ? 0.f : w.x, sc_g = beyond ? 1.f : w.y, sc_kq = beyond ? 0.f : w.z;
+#pragma unroll
+    for (int t = 0; t < DR_ROWS; ++t) ld_v[t] = to_float((vp + row(t) * in_stride)[j_lane]);
+  };
+  fetch(r0);
   for (int t0 = r0; t0 < r1; t0 += DR_ROWS) {
     __syncthreads();        // the block before has been walked
 #pragma unroll
@@ -174,33 +187,61 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(
 #pragma unroll
     for (int t = 0; t < DR_ROWS; ++t) vs[t] = ld_v[t];
     __syncthreads();
-    if (t0 + DR_ROWS < r1) DR_FETCH(t0 + DR_ROWS)
+    if (t0 + DR_ROWS < r1) fetch(t0 + DR_ROWS);
     const int n = r1 - t0;
-#pragma unroll
-    for (int t = 0; t < DR_ROWS; ++t) {
-      const float4 sc = sc_s[t];                       // beta, g, k . q
+    // a row's operands are read while the row before is walked
+    float o[DR_ROWS], k[2][KPT], q[2][KPT];
+    float4 sc_row[2];
+    auto operands = [&](int t) {
+      sc_row[t & 1] = sc_s[t];                         // beta, g, k . q
       const float4* kr = kq_s + t * ROW_F4 + g_lane * (KPT / 4);
       const float4* qr = kr + ROW_F4 / 2;
-      float k[KPT], q[KPT];
 #pragma unroll
       for (int i = 0; i < KPT / 4; ++i) {
         const float4 a = kr[i], b = qr[i];
-        k[4 * i] = a.x, k[4 * i + 1] = a.y, k[4 * i + 2] = a.z, k[4 * i + 3] = a.w;
-        q[4 * i] = b.x, q[4 * i + 1] = b.y, q[4 * i + 2] = b.z, q[4 * i + 3] = b.w;
+        k[t & 1][4 * i] = a.x, k[t & 1][4 * i + 1] = a.y, k[t & 1][4 * i + 2] = a.z, k[t & 1][4 * i + 3] = a.w;
+        q[t & 1][4 * i] = b.x, q[t & 1][4 * i + 1] = b.y, q[t & 1][4 * i + 2] = b.z, q[t & 1][4 * i + 3] = b.w;
       }
+    };
+    operands(0);
+#pragma unroll
+    for (int t = 0; t < DR_ROWS; ++t) {
+      if (t + 1 < DR_ROWS) operands(t + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const float4 sc = sc_row[t & 1];
       float sk = 0.f, sq = 0.f;
 #pragma unroll
       for (int i = 0; i < KPT; ++i) {
-        sk = fmaf(S[i], k[i], sk);
-        sq = fmaf(S[i], q[i], sq);
+        sk = fmaf(S[i], k[t & 1][i], sk);
+        sq = fmaf(S[i], q[t & 1][i], sq);
       }
-      sk = dr_group_sum(sk, NG);
-      sq = dr_group_sum(sq, NG);
+      if constexpr (PAIRED) {       // even lanes go on with sk, odd ones with sq: the sums of the two butterflies
+        sk += lane_xor1(sk), sq += lane_xor1(sq);
+        sq = (lane & 1) ? sq : sk;
+        sq += lane_xor2(sq);
+        sq += lane_xor4(sq);
+        sq += lane_xor8(sq);
+        sk = __uint_as_float(dpp_bits<0xA0>(__float_as_uint(sq)));      // lanes 0 0 2 2
+      } else {
+        sk = dr_group_sum(sk, NG);
+        sq = dr_group_sum(sq, NG);
+      }
       const float u = sc.x * (vs[t] - sc.y * sk);
-      const float o = fmaf(sc.y, sq, u * sc.z);
+      o[t] = fmaf(sc.y, sq, u * sc.z);
 #pragma unroll
-      for (int i = 0; i < KPT; ++i) S[i] = fmaf(k[i], u, sc.y * S[i]);
-      if (has && g_lane == 0 && t < n) yp[(int64_t)(t0 + t) * y_stride] = o;
+      for (int i = 0; i < KPT; ++i) S[i] = fmaf(k[t & 1][i], u, sc.y * S[i]);
+    }
+    // the lanes of a value dim hold its results (PAIRED: the odd ones): one of them stores each row
+    if constexpr (NG >= DR_ROWS) {
+      const int at = PAIRED ? g_lane >> 1 : g_lane;
+      float mine = o[0];
+#pragma unroll
+      for (int t = 1; t < DR_ROWS; ++t) mine = at == t ? o[t] : mine;
+      if (has && at < min(n, DR_ROWS) && (!PAIRED || (lane & 1))) yp[(int64_t)(t0 + at) * y_stride] = mine;
+    } else {
+#pragma unroll
+      for (int t = 0; t < DR_ROWS; ++t)
+        if (has && g_lane == 0 && t < n) yp[(int64_t)(t0 + t) * y_stride] = o[t];
     }
   }
   if (has) {
@@ -208,7 +249,6 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(
     for (int i = 0; i < KPT; ++i) S_row[i] = S[i];
   }
 }
-#undef DR_FETCH
 
 // The same walk without staging, for key widths beyond DR_MAX_DP: a lane reads its own share of a row's prepared
 // k and q, one row ahead.
@@ -316,12 +356,14 @@ extern "C" int he_delta_scan(void* y_f32, const void* q, const void* k, const vo
   const int per_block = 64 / ng;
   const dim3 grid(num_seqs, H, (e + per_block - 1) / per_block);
   HE_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "he_delta_scan: too many heads or value tiles for one launch");
+  const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
+  HE_REQUIRE(blocks <= INT32_MAX, "he_delta_scan: too many sequences, heads and value tiles for one launch");
 #define DR_ARGS(T)                                                                                          \
   (float*)y_f32, kq_ws, head_ws, (const T*)v, in_stride, (uint8_t*)state, state_stride, state_offset,       \
       (const int32_t*)cu_seqlens, (const int32_t*)seq_slot, H, G, e
 #define DR_STAGED(T, KPT, NG)           \
   if (kpt == KPT && ng == NG) {         \
-    delta_scan_kernel<T, KPT, NG><<<grid, 64, 0, s>>>(DR_ARGS(T)); \
+    delta_scan_kernel<T, KPT, NG><<<(unsigned)blocks, 64, 0, s>>>(DR_ARGS(T), (int)grid.z); \
     launched = true;                    \
   }
 #define DR_STAGED_ALL(T)                                                                                         \

@@ -124,6 +124,24 @@ def test_delta_rule_in_portions_and_batches_equals_the_whole(ops, dtype, H, G, d
     assert bool((state[[1, 3, 5]][:, offset:offset + nbytes] == 0).all())          # other slots' matrices stay zero
 
 
+@pytest.mark.parametrize("d,e", [(128, 128), (121, 6), (200, 9), (64, 5)])
+def test_delta_rule_at_the_edges_of_its_blocks(ops, d, e):
+    """Sequences around whole blocks of eight rows side by side, at key widths of 16 lanes (whose two sums share a register) and
+    below: each as the plain recurrence has it, nothing stored beyond the rows."""
+    H, G, lengths = 4, 2, [1, 7, 8, 9, 15, 16, 17, 33]
+    xs = [rnd(n, 2 * G * d + H * e, seed=40 + i) for i, n in enumerate(lengths)]
+    bas = [rnd(n, 2 * H, seed=60 + i, scale=2.0) for i, n in enumerate(lengths)]
+    a_log, dt_bias = rnd(H, seed=30, scale=0.5), rnd(H, seed=31) - 1.0
+    x, rows = dev(torch.cat(xs)), sum(lengths)
+    y = torch.full((rows + 1, H * e), 3.0, device="cuda")
+    state = torch.zeros(len(lengths), 4 * ops.delta_state_floats(H, d, e), dtype=torch.uint8, device="cuda")
+    ops.delta_scan(y[:rows], x[:, :G * d], x[:, G * d:2 * G * d], x[:, 2 * G * d:], dev(torch.cat(bas)), dev(a_log), dev(dt_bias),
+                   state, 0, cu_of(lengths), i32(range(len(lengths))), rows, len(lengths), H, G, d, e, d ** -0.5, 1e-6)
+    want = torch.cat([plain_delta(x, ba, a_log, dt_bias, H, G, d, e, d ** -0.5) for x, ba in zip(xs, bas)])
+    assert torch.allclose(y[:rows].cpu().double(), want, rtol=1e-4, atol=2e-5 * max(1.0, want.abs().max().item()))
+    assert bool((y[rows] == 3.0).all())
+
+
 @pytest.mark.parametrize("feed", ["whole", "ones", "pairs"])
 def test_a_value_written_early_is_read_back_far_later(ops, feed):
     """Token 3 writes a large value under a key of its own with full strength; no later token's key meets it and
