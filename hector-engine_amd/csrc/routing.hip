@@ -20,9 +20,11 @@
 //
 // A step of many rows is bound by the reads of the router's matrix from L2, D * E * 4 bytes a workgroup: two rows share them.
 // What bounds a step of few rows is the chain: the router's rows come from memory, so a wavefront asks for those of up to four
-// outputs together; the choice is made by the first wavefront alone, PL outputs a lane in registers, without a barrier or a
-// walk through LDS a choice. (2 rows of 2048, 18 outputs in 3 groups, 4 chosen: 14.5 us with eight wavefronts that meet at two barriers a choice and
-// ask for one output at a time, 9 so; 2048 rows 41 us and 31; one row of 300 outputs in 5 groups, 8 chosen, 89 and 36.)
+// outputs, with the row, its scale's parts, the biases and corrections, all at the start; the choice is made by the first wavefront alone, PL
+// outputs a lane in registers, without a barrier or a walk through LDS a choice, while the others write the scaled row. (2 rows of 2048, 18
+// outputs in 3 groups, 4 chosen: 14.5 us with eight wavefronts that meet at two barriers a choice and ask for one output at a time, 9 so; 2048 rows 41 us and 31; one
+// row of 300 outputs in 5 groups, 8 chosen, 89 and 36. The loads in two turns, the scale, the corrections and the scaled row one after the other in front of
+// the choice: the same 2 rows within a step 10.4 us, so 7.3.)
 #define ROUTE_WAVES 8
 
 // Rows x whose norm's scale is still owed (partials null: none is): the rows are bf16(x * inv) with inv as scale_rows_kernel forms it, and
@@ -46,11 +48,33 @@ __device__ __forceinline__ uint2 route_scaled(const uint2 b, float inv) {
                     float_to_bf16_bits(v.z * inv) | (uint32_t)float_to_bf16_bits(v.w * inv) << 16);
 }
 
+// The scale a row still owes, from its parts in the order lane, lane + 64, ...: the first ROUTE_PARTS of a lane are asked for ahead.
+#define ROUTE_PARTS 4
+struct RouteParts {
+  float v[ROUTE_PARTS];
+};
+__device__ __forceinline__ RouteParts route_parts(const RouteOwed& owed, int64_t row) {
+  RouteParts p;
+#pragma unroll
+  for (int j = 0; j < ROUTE_PARTS; ++j) p.v[j] = owed.partials[row * owed.count + min((int)(threadIdx.x & 63) + 64 * j, owed.count - 1)];
+  return p;
+}
+__device__ __forceinline__ float route_inv(const RouteParts& p, const RouteOwed& owed, int64_t row, int D) {
+  const int lane = threadIdx.x & 63;
+  float part = 0.f;
+#pragma unroll
+  for (int j = 0; j < ROUTE_PARTS; ++j)
+    if (lane + 64 * j < owed.count) part += p.v[j];
+  for (int i = lane + 64 * ROUTE_PARTS; i < owed.count; i += 64) part += owed.partials[row * owed.count + i];
+  return 1.0f / sqrtf(wave_sum(part) / (float)D + owed.eps);
+}
+
 // The dot products of row x with the router's rows e0, e0 + ROUTE_WAVES, ... (OUT of them, those beyond E repeat the last): four elements
-// a lane and turn, four sums a lane that meet in index order.
+// a lane and turn, four sums a lane that meet in index order. The loads of up to eight turns (rows of 2048 elements) are
+// asked for together, ahead of what the row's scale is made of: one trip to memory.
 template <int OUT, bool OWED>
 __device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x_dtype, const float* router, int64_t row, int rows, int D, int E,
-                                           int e0, int x_pieces, float inv) {
+                                           int e0, int x_pieces, const RouteParts& parts, const RouteOwed& owed) {
   const int lane = threadIdx.x & 63;
   const bool vec = (D & 3) == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)router & 15) == 0;
   const float* w[OUT];
@@ -62,28 +86,43 @@ __device__ __forceinline__ void route_dots(float (&z)[OUT], const void* x, int x
     for (int j = 0; j < 4; ++j) a[o][j] = 0.f;
   }
   if (vec) {
+    constexpr int TURNS = OUT > 2 ? 4 : 8;
     // row-major: four elements i at 4 i; piece-major [D / 8][rows][8]: half i & 1 of the row's piece i / 2
     const uint2* xh = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * row : row * (D >> 2));
     const float4* xf = reinterpret_cast<const float4*>((const float*)x + row * D);
     const int64_t piece = 2 * (int64_t)rows;
-#pragma unroll 4
-    for (int i = lane; i < (D >> 2); i += 64) {
-      float4 xv;
-      if (OWED || x_dtype == HE_BF16) {
-        const uint2 b = x_pieces ? xh[(i >> 1) * piece + (i & 1)] : xh[i];
-        xv = route_four(OWED ? route_scaled(b, inv) : b);
-      } else {
-        xv = xf[i];
-      }
+    const int n = D >> 2;
+    float inv = 1.f;
+    const auto walk = [&](auto bf) {         // one loop a type, without a branch around its loads
+      for (int i0 = 0; i0 < n; i0 += 64 * TURNS) {
+        uint2 xb[TURNS];
+        float4 xv[TURNS], wv[TURNS][OUT];
 #pragma unroll
-      for (int o = 0; o < OUT; ++o) {
-        const float4 wv = reinterpret_cast<const float4*>(w[o])[i];
-        a[o][0] = fmaf(xv.x, wv.x, a[o][0]);
-        a[o][1] = fmaf(xv.y, wv.y, a[o][1]);
-        a[o][2] = fmaf(xv.z, wv.z, a[o][2]);
-        a[o][3] = fmaf(xv.w, wv.w, a[o][3]);
+        for (int t = 0; t < TURNS; ++t) {
+          const int i = min(i0 + 64 * t + lane, n - 1);
+          if constexpr (decltype(bf)::value) xb[t] = xh[x_pieces ? (i >> 1) * piece + (i & 1) : i];
+          else xv[t] = xf[i];
+#pragma unroll
+          for (int o = 0; o < OUT; ++o) wv[t][o] = reinterpret_cast<const float4*>(w[o])[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (OWED && i0 == 0) inv = route_inv(parts, owed, row, D);
+#pragma unroll
+        for (int t = 0; t < TURNS; ++t) {
+          if (i0 + 64 * t + lane >= n) continue;
+          if constexpr (decltype(bf)::value) xv[t] = route_four(OWED ? route_scaled(xb[t], inv) : xb[t]);
+#pragma unroll
+          for (int o = 0; o < OUT; ++o) {
+            a[o][0] = fmaf(xv[t].x, wv[t][o].x, a[o][0]);
+            a[o][1] = fmaf(xv[t].y, wv[t][o].y, a[o][1]);
+            a[o][2] = fmaf(xv[t].z, wv[t][o].z, a[o][2]);
+            a[o][3] = fmaf(xv[t].w, wv[t][o].w, a[o][3]);
+          }
+        }
       }
-    }
+    };
+    if (OWED || x_dtype == HE_BF16) walk(std::true_type{});
+    else walk(std::false_type{});
   } else {
     for (int i = lane; i < D; i += 64) {
       const float xv = x_dtype == HE_BF16 ? bf16_bits_to_float(((const uint16_t*)x)[row * D + i])
@@ -171,17 +210,20 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
   const int row0 = blockIdx.x * RW;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+  // what the choosing wavefronts need at the end, asked for at the start (each lane its first output's)
+  const bool chooses = wave < RW && row0 + wave < rows;
+  float bias0 = 0.f, correction0 = 0.f;
+  if (chooses && lane < E) {
+    if (bias) bias0 = load_param(bias, lane, bias_dtype);
+    if (correction) correction0 = load_param(correction, lane, c_dtype);
+  }
+  RouteParts parts = {};
+  if (OWED) parts = route_parts(owed, row0);
   if (x != nullptr) {
-    float inv = 1.f;
-    if (OWED) {
-      float part = 0.f;
-      for (int i = lane; i < owed.count; i += 64) part += owed.partials[(int64_t)row0 * owed.count + i];
-      inv = 1.0f / sqrtf(wave_sum(part) / (float)D + owed.eps);
-    }
     for (int e0 = wave; e0 < E; e0 += 4 * ROUTE_WAVES) {
       if (e0 + 2 * ROUTE_WAVES < E) {
         float z[RW][4];
-        if constexpr (RW == 1) route_dots<4, OWED>(z[0], x, x_dtype, router, row0, rows, D, E, e0, x_pieces, inv);
+        if constexpr (RW == 1) route_dots<4, OWED>(z[0], x, x_dtype, router, row0, rows, D, E, e0, x_pieces, parts, owed);
         else route_dots_rows<4, RW>(z, x, x_dtype, router, row0, rows, D, E, e0);
 #pragma unroll
         for (int r = 0; r < RW; ++r)
@@ -190,7 +232,7 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
             if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_all[r][e0 + o * ROUTE_WAVES] = z[r][o];
       } else {
         float z[RW][2];
-        if constexpr (RW == 1) route_dots<2, OWED>(z[0], x, x_dtype, router, row0, rows, D, E, e0, x_pieces, inv);
+        if constexpr (RW == 1) route_dots<2, OWED>(z[0], x, x_dtype, router, row0, rows, D, E, e0, x_pieces, parts, owed);
         else route_dots_rows<2, RW>(z, x, x_dtype, router, row0, rows, D, E, e0);
 #pragma unroll
         for (int r = 0; r < RW; ++r)
@@ -199,13 +241,14 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
             if (lane == 0 && e0 + o * ROUTE_WAVES < E) z_all[r][e0 + o * ROUTE_WAVES] = z[r][o];
       }
     }
-    if (OWED) {
-      const uint2* xh = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * (int64_t)row0 : (int64_t)row0 * (D >> 2));
-      uint2* to = reinterpret_cast<uint2*>(owed.out) + (int64_t)row0 * (D >> 2);
-      for (int i = threadIdx.x; i < (D >> 2); i += 64 * ROUTE_WAVES)
-        to[i] = route_scaled(x_pieces ? xh[(i >> 1) * (2 * (int64_t)rows) + (i & 1)] : xh[i], inv);
-    }
     __syncthreads();
+  }
+  if (OWED && wave >= RW) {      // the scaled row, by the wavefronts that don't choose
+    const float inv = route_inv(parts, owed, row0, D);
+    const uint2* xh = reinterpret_cast<const uint2*>((const uint16_t*)x) + (x_pieces ? 2 * (int64_t)row0 : (int64_t)row0 * (D >> 2));
+    uint2* to = reinterpret_cast<uint2*>(owed.out) + (int64_t)row0 * (D >> 2);
+    for (int i = threadIdx.x - 64 * RW; i < (D >> 2); i += 64 * (ROUTE_WAVES - RW))
+      to[i] = route_scaled(x_pieces ? xh[(i >> 1) * (2 * (int64_t)rows) + (i & 1)] : xh[i], inv);
   }
   const int64_t row = row0 + wave;
   if (wave >= RW || row >= rows) return;
@@ -219,7 +262,7 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
     const int e = lane + 64 * j;
     z[j] = s[j] = d[j] = 0.f;
     if (e >= E) continue;
-    z[j] = (x != nullptr ? z_sh[e] : logits[row * E + e]) + (bias ? load_param(bias, e, bias_dtype) : 0.f);
+    z[j] = (x != nullptr ? z_sh[e] : logits[row * E + e]) + (bias ? j == 0 ? bias0 : load_param(bias, e, bias_dtype) : 0.f);
     mx = fmaxf(mx, z[j]);
   }
   mx = wave_max(mx);
@@ -237,7 +280,7 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
     const int e = lane + 64 * j;
     s[j] *= inv;
     // (without a correction the choice is made on the logits themselves: the same order, and no two meet at zero)
-    c[j] = e >= E ? NAN : correction ? s[j] + load_param(correction, e, c_dtype) : z[j];
+    c[j] = e >= E ? NAN : correction ? s[j] + (j == 0 ? correction0 : load_param(correction, e, c_dtype)) : z[j];
   }
   if (keep < groups) {
     // a lane ranks whole groups; the kept ones are marked by NaN, then the others' outputs are masked
@@ -252,6 +295,7 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
       g[j] = NAN;
       if (group >= groups) continue;
       float best = -INFINITY;
+#pragma unroll 4
       for (int i = 0; i < size; ++i) best = fmaxf(best, c_sh[group * size + i]);
       g[j] = best == INFINITY ? NAN : best;      // (such a group is kept beside the `keep` best)
     }

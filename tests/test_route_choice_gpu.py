@@ -103,3 +103,29 @@ def test_the_norms_scale_with_the_choice(rows, E, D, count, pieces):
     with pytest.raises(RuntimeError):
         ops.route_tokens(*want, None, None, rows, E - 2, 1, 1, 3, 1.5, x=given, router=torch.randn(65, D, device="cuda"), x_pieces=pieces,
                          owed=(partials, 1e-6, got_rows))
+
+
+@pytest.mark.parametrize("E,D,count", [(3, 2040, 257), (18, 2048, 255), (17, 2056, 600), (41, 1032, 256), (9, 4104, 1)])
+@pytest.mark.parametrize("pieces", [False, True])
+def test_a_routers_turns_and_parts_at_their_edges(E, D, count, pieces):
+    """Rows around whole turns of loads, scales of more parts than are asked for ahead, biases and corrections: the bits of the same
+    rows scaled beforehand and routed two a workgroup."""
+    from hector_engine_amd.kernels import ops
+    g, rows = torch.Generator().manual_seed(D + E), 2
+    x = torch.randn(rows, D, generator=g).bfloat16().cuda()
+    partials = (torch.rand(rows, count, generator=g) * D / count).cuda()
+    router, bias, correction = (torch.randn(*s, generator=g).cuda() for s in ((E, D), (E,), (E,)))
+    given = x.view(rows, D // 8, 8).transpose(0, 1).contiguous() if pieces else x
+    scaled, got_rows = torch.empty_like(x), torch.full_like(x, math.nan)
+    ops.scale_rows(scaled, given, partials, 1e-6, rows, pieces)
+
+    def route(x, n, **more):
+        dense, ids = torch.full((n, E + 1), math.nan, device="cuda"), torch.full((n, 3), 77, dtype=torch.int32, device="cuda")
+        weights = torch.full((n, 3), math.nan, device="cuda")
+        ops.route_tokens(dense, ids, weights, None, correction, n, E, 1, 1, 3, 1.5, x=x, router=router, bias=bias, **more)
+        return dense, ids, weights
+    want = route(scaled.repeat(150, 1), 150 * rows)
+    got = route(given, rows, x_pieces=pieces, owed=(partials, 1e-6, got_rows))
+    assert torch.equal(got_rows, scaled)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b[:rows]) and torch.equal(a, b[-rows:])
