@@ -162,29 +162,43 @@ __device__ __forceinline__ void fused_join(const float* ws_o, const float* ws_ml
   constexpr int HD = 16 * NT, PER = 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float* inv = lds + 64 * GT;
-  for (int hg = wave; hg < GT; hg += 4) {
-    const float2 ml = lane < Z ? shared_load2(ws_ml + 2 * ((head0 + hg) * Z + lane)) : make_float2(-INFINITY, 0.f);
-    const float M = wave_max(ml.x);
-    const float w = ml.x > -INFINITY ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
-    const float L = wave_sum(ml.y * w);
+  const int items = GT * (HD / 4), mine = min((int)threadIdx.x, items - 1);
+  auto ask = [&](int item, int s) {
+    const float* at = ws_o + ((head0 + item / (HD / 4)) * Z + min(s, Z - 1)) * HD + 4 * (item % (HD / 4));
+    const float2 lo = shared_load2(at), hi = shared_load2(at + 2);
+    return make_float4(lo.x, lo.y, hi.x, hi.y);
+  };
+  // everything a thread reads first goes out together, in one trip to memory: the (m, l) of its wavefront's heads (at most 16 heads a
+  // tile), then the first parts of its first item (head after head, and eight parts behind them, it was three to five trips:
+  // one sequence of 2,048 keys, 28 heads of 128, 10.9 -> 10.6 us a layer; of 512 keys, 14 heads of 64, 8.7 -> 7.5)
+  float2 ml[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ml[j] = shared_load2(ws_ml + 2 * ((head0 + min(wave + 4 * j, GT - 1)) * Z + min(lane, Z - 1)));
+  float4 first[PER], second[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) first[i] = ask(mine, i);
+  if (Z > PER) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) second[i] = ask(mine, PER + i);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int hg = wave + 4 * j;
+    if (hg >= GT) break;
+    const float m = lane < Z ? ml[j].x : -INFINITY;
+    const float M = wave_max(m);
+    const float w = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+    const float L = wave_sum((lane < Z ? ml[j].y : 0.f) * w);
     lds[64 * hg + lane] = w;
     if (lane == 0) inv[hg] = L > 0.f ? 1.f / L : 0.f;
   }
   __syncthreads();
-  for (int item = threadIdx.x; item < GT * (HD / 4); item += 256) {
+  for (int item = threadIdx.x; item < items; item += 256) {
     const int hg = item / (HD / 4), d = 4 * (item % (HD / 4));
-    const float* o = ws_o + (head0 + hg) * Z * HD + d;
     float4 acc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = 0; s0 < Z; s0 += PER) {
-      float4 v[PER];
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const float* at = o + (int64_t)min(s0 + i, Z - 1) * HD;
-        const float2 lo = shared_load2(at), hi = shared_load2(at + 2);
-        v[i] = make_float4(lo.x, lo.y, hi.x, hi.y);
-      }
+    auto add = [&](const float4 (&v)[PER], int s0) {
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         if (s0 + i >= Z) break;
@@ -192,6 +206,18 @@ __device__ __forceinline__ void fused_join(const float* ws_o, const float* ws_ml
         float4& a = acc[i & 3];
         a.x = fmaf(v[i].x, w, a.x), a.y = fmaf(v[i].y, w, a.y), a.z = fmaf(v[i].z, w, a.z), a.w = fmaf(v[i].w, w, a.w);
       }
+    };
+    int s0 = 0;
+    if (item == (int)threadIdx.x) {
+      add(first, 0);
+      if (Z > PER) add(second, PER);
+      s0 = 2 * PER;
+    }
+    for (; s0 < Z; s0 += PER) {
+      float4 v[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) v[i] = ask(item, s0 + i);
+      add(v, s0);
     }
     const float f = inv[hg];
     store(hg, d, make_float4((((acc[0].x + acc[1].x) + acc[2].x) + acc[3].x) * f, (((acc[0].y + acc[1].y) + acc[2].y) + acc[3].y) * f,
