@@ -409,7 +409,7 @@ class Engine:
             ctx = self._context(bucket.views, size, size, 1, True, bucket.pool)
             ctx.want_all = True
             ctx.hints = dict(zip(self._hint_fns, hints))
-            ctx.padded = True
+            ctx.padded = size > 2            # (a bucket of 1 or 2 rows has no other count of sequences)
             if by_row:
                 dev_tables = bucket.views["row_tables"].view(groups, size, blocks)
                 ctx.row_tables = {g.page_table.data_ptr(): dev_tables[gi] for gi, g in enumerate(self.cache.groups)}
@@ -493,7 +493,7 @@ class Engine:
             ctx = self._context(bucket.views, R, S, Q, all_single, bucket.pool)
             ctx.want_all = want_all
             ctx.most_keys = keys
-            ctx.padded = True
+            ctx.padded = R <= self.graph_step_rows      # (a whole chunk has no padding rows)
             if bucket.uses == 1 or bucket.capture_failed is not None:
                 bucket.pool.reset()          # first use: eagerly; it also sizes the bucket's scratch pool
                 self.stats["eager_steps"] += 1

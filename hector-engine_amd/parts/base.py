@@ -167,8 +167,10 @@ class StepContext:
         self.host = host                  # {"q_lens", "starts", "slots"}: lists per sequence, eager steps only
         self.hints: dict = {}             # what the parts' step_hint functions said of this step (function -> value)
         self.want_all = False             # the wanted rows are all rows, in order
-        self.padded = False               # the step may hold padding rows and sequences (row_seq -1, slot -1: a step that
-                                          # runs as a graph of its bucket of sizes); a part leaves such rows finite
+        self.padded = False               # the step may hold padding rows (row_seq -1: a step that runs as a graph of its
+                                          # bucket of sizes); a part leaves such rows finite. Without them no launch clears
+                                          # rows: 6 us a layer of a 2,048-token prompt, 4 a layer of a one-token step. (Padding
+                                          # sequences, slot -1, come in any such step.)
         self.row_tables: dict = {}        # a cache group's page table (its data_ptr) -> int32 [rows, blocks]: the table
                                           # rows of the step's rows, gathered by the host into the step's metadata
                                           # (one-token steps that replay a graph; a mixer may read it in place of

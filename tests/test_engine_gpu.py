@@ -779,3 +779,37 @@ def test_step_graphs_are_kept_least_recently_used_first_out(model_dirs, plain_mo
     again = [run(1, 20, [19]) for _ in range(3)]
     assert eng.stats["step_graph_captures"] == captures + 1
     assert all(torch.equal(a, first[0]) for a in again + first)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_steps_without_padding_rows_clear_none(model_dirs, dtype, monkeypatch):
+    """A whole chunk of 768 rows dealt to four sequences and then to three (a padding sequence, no padding row), and one-token steps of one
+    and two sequences: graphs whose launches clear no rows, three uses each, as an engine without graphs has them. Three one-token
+    sequences run in a bucket of four, whose rows are still cleared."""
+    import hector_engine_amd as he
+    opts = dict(max_tokens=4096, max_slots=8, max_seq_len=1024, beyond_max_positions=True)
+    eng = he.Engine(model_dirs[NAMES[0]], dtype=dtype, **opts)
+    plain_eng = he.Engine(model_dirs[NAMES[0]], dtype=dtype, graph_step_rows=0, **opts)
+    padded, context = [], type(eng)._context
+
+    def noted(self, *a, **k):
+        ctx = context(self, *a, **k)
+        if self is eng:
+            padded.append(ctx)
+        return ctx
+    monkeypatch.setattr(type(eng), "_context", noted)
+    for use, lengths in enumerate(([192, 210, 183, 183], [300, 276, 192], [195, 189, 192, 192])):
+        ids = [rand_ids(100, n + 4, 900 + 10 * use + i) for i, n in enumerate(lengths)]
+        held = {e: [e.acquire() for _ in lengths] for e in (eng, plain_eng)}
+        a, b = (e.step([entry(s, r[:n], [n - 1]) for s, r, n in zip(held[e], ids, lengths)]).clone() for e in (eng, plain_eng))
+        assert torch.equal(a, b) if dtype == "float32" else torch.isfinite(a).all() and torch.allclose(a, b, atol=0.05 * float(b.abs().max()))
+        for count in (1, 2, 3):
+            first = len(padded)
+            a, b = (e.step([entry(s, [r[n + count]], [0]) for s, r, n in zip(held[e][:count], ids, lengths)]).clone() for e in (eng, plain_eng))
+            assert torch.equal(a, b) if dtype == "float32" else torch.allclose(a, b, atol=0.05 * float(b.abs().max()))
+            assert all(c.padded == (count == 3) for c in padded[first:])
+        for e, slots in held.items():
+            for s in slots:
+                e.release(s)
+    chunks = [c for c in padded if c.rows == 768]
+    assert chunks and not any(c.padded for c in chunks)
