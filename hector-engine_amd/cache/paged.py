@@ -80,9 +80,9 @@ class _Tables:
         if n == 0:
             return
         idx = np.fromiter(self._dirty, dtype=np.int32, count=n)
-        self._dirty.clear()
         if self.device.device.type == "cpu":
             self.device.view(-1)[torch.from_numpy(idx).long()] = torch.from_numpy(self._flat[idx])
+            self._dirty.clear()
             return
         i = self._next
         self._next = (i + 1) % len(self._pinned)
@@ -98,6 +98,7 @@ class _Tables:
         self._events[i] = torch.cuda.Event()
         self._events[i].record()
         ops.scatter_i32(self.device, entries, n)
+        self._dirty.clear()              # (only now: entries that an error kept from the device go with the next flush)
 
 
 class PagedCache:

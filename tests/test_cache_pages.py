@@ -276,3 +276,24 @@ def test_chunked_group_frees_the_blocks_before_the_running_chunk(chunk):
     b.check_invariants()
     b.release(s)
     assert all(g.pool.available == 32 for g in b.groups)
+
+
+def test_entries_an_error_kept_from_the_device_go_with_the_next_flush():
+    import torch
+
+    from hector_engine_amd.cache.paged import _Tables
+
+    class Broken:
+        device = torch.device("cpu")
+
+        def view(self, *_):
+            raise RuntimeError("no room")
+    t = _Tables(2, 3, 4, torch.device("cpu"))
+    t.write(5, 9)
+    table, t.device = t.device, Broken()
+    with pytest.raises(RuntimeError):
+        t.flush()
+    t.device = table
+    t.write(17, 2)
+    t.flush()
+    assert (t.device.numpy() == t.host).all() and t.device[0, 1, 1] == 9 and t.device[1, 1, 1] == 2
