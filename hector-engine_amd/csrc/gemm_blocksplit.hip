@@ -103,7 +103,7 @@ static BlockSplitPlan ordered_plan(int M, int N, int K) {
   }
   while (nw > 1 && K / nw < 128) nw >>= 1;
   if (u * (r + 1) > 4 && nw > 8) nw = 8;
-  p.NA = r, p.S = u > 1 ? 2 : 1, p.NW = nw;
+  p.NA = r, p.S = u > 1 || r == 1 ? 2 : 1, p.NW = nw;      // (two units a step where a wavefront has one accumulator: the same turns)
   p.units = ((K + nw - 1) / nw + 63) / 64;
   p.turn = 2 * u;
   p.rows_per_block = rows > 0 ? rows : 16 * r;
