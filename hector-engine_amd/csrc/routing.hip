@@ -277,6 +277,9 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(
   const float inv = 1.f / sum;
 #pragma unroll
   for (int j = 0; j < PL; ++j) {
+    // a score is rounded, then its sum with the correction: as one multiply-add, for the outputs whose correction is at hand, two outputs of equal
+    // scores and corrections on both sides of 64 would no longer tie
+#pragma clang fp contract(off)
     const int e = lane + 64 * j;
     s[j] *= inv;
     // (without a correction the choice is made on the logits themselves: the same order, and no two meet at zero)

@@ -129,3 +129,19 @@ def test_a_routers_turns_and_parts_at_their_edges(E, D, count, pieces):
     assert torch.equal(got_rows, scaled)
     for a, b in zip(got, want):
         assert torch.equal(a, b[:rows]) and torch.equal(a, b[-rows:])
+
+
+@pytest.mark.parametrize("copies", [2, 4, 12])
+@pytest.mark.parametrize("rows", [40, 300])
+def test_equal_outputs_tie_wherever_they_stand(copies, rows):
+    """Outputs with one score and one correction, 64 apart: a lane's first output among them, whose correction is asked for ahead. The scores meet
+    the corrections in two roundings, so that the copies tie and are chosen in the order of their numbers; from logits and from rows."""
+    from hector_engine_amd.kernels import ops
+    g, E, D, top = torch.Generator().manual_seed(copies), 64 * copies, 256, 3 * copies
+    correction = (0.1 * torch.randn(64, generator=g)).repeat(copies).cuda()
+    x, router = torch.randn(rows, D, generator=g).bfloat16().cuda(), (0.1 * torch.randn(64, D, generator=g)).repeat(copies, 1).cuda()
+    logits = torch.randn(rows, 64, generator=g).repeat(1, copies).cuda()
+    for given in (dict(logits=logits), dict(logits=None, x=x, router=router)):
+        dense, ids = torch.empty(rows, E + 1, device="cuda"), torch.full((rows, top), 77, dtype=torch.int32, device="cuda")
+        ops.route_tokens(dense, ids, torch.empty(rows, top, device="cuda"), given.pop("logits"), correction, rows, E, 1, 1, top, 1.0, **given)
+        assert torch.equal(ids, torch.cat([ids[:, i * copies:i * copies + 1] + 64 * torch.arange(copies, device="cuda", dtype=torch.int32) for i in range(3)], 1))
