@@ -60,15 +60,22 @@ class _Tables:
     on the device all together before the next step (flush): one copy from pinned memory and one launch behind what is
     queued. (Written slot by slot, from pageable memory, every release, truncation and new page made the host wait for
     all queued steps and left the GPU idle for 60 us behind them: 64 sequences cut back after eight steps, 21 of them by a
-    page, 1.3 ms of 17.2.)"""
+    page, 1.3 ms of 17.2.) The pinned memory is there from the start: TURNS parts of TURN entries, used in turn, each free again when its
+    event has passed; more entries than a part holds go in several launches. (Made by the steps that first wanted it, each of the
+    first four and every one with more entries than before had a host allocation in its path.)"""
+
+    TURNS, TURN = 4, 4096
 
     def __init__(self, groups: int, max_slots: int, max_blocks: int, device):
         self.host = np.full((groups, max_slots, max_blocks), -1, dtype=np.int32)
         self.device = torch.full((groups, max_slots, max_blocks), -1, dtype=torch.int32, device=device)
         self._flat = self.host.reshape(-1)
         self._dirty: set[int] = set()
-        self._pinned: list[torch.Tensor | None] = [None] * 4       # in turn, each free again when its event has passed
-        self._events: list[torch.cuda.Event | None] = [None] * 4
+        self._turn = max(1, min(self.TURN, self._flat.size))
+        self._pinned: list[torch.Tensor] = []
+        if self.device.device.type != "cpu":
+            self._pinned = list(torch.empty((self.TURNS, 2 * self._turn), dtype=torch.int32, pin_memory=True))
+        self._events: list[torch.cuda.Event | None] = [None] * self.TURNS
         self._next = 0
 
     def write(self, index: int, page: int) -> None:
@@ -84,12 +91,15 @@ class _Tables:
             self.device.view(-1)[torch.from_numpy(idx).long()] = torch.from_numpy(self._flat[idx])
             self._dirty.clear()
             return
-        i = self._next
-        self._next = (i + 1) % len(self._pinned)
+        for at in range(0, n, self._turn):
+            self._send(idx[at:at + self._turn])
+        self._dirty.clear()              # (only now: entries that an error kept from the device go with the next flush)
+
+    def _send(self, idx: np.ndarray) -> None:
+        i, n = self._next, len(idx)
+        self._next = (i + 1) % self.TURNS
         if self._events[i] is not None:
             self._events[i].synchronize()
-        if self._pinned[i] is None or self._pinned[i].numel() < 2 * n:
-            self._pinned[i] = torch.empty(max(256, 1 << (2 * n - 1).bit_length()), dtype=torch.int32, pin_memory=True)
         staged = self._pinned[i][:2 * n]
         staged.numpy()[:n] = idx
         staged.numpy()[n:] = self._flat[idx]
@@ -98,7 +108,6 @@ class _Tables:
         self._events[i] = torch.cuda.Event()
         self._events[i].record()
         ops.scatter_i32(self.device, entries, n)
-        self._dirty.clear()              # (only now: entries that an error kept from the device go with the next flush)
 
 
 class PagedCache:

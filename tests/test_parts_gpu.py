@@ -877,3 +877,19 @@ def test_page_table_entries_written_together(fw, count):
         t.flush()
         t.flush()
     assert (t.device.cpu().numpy() == t.host).all() and (t.host.max() > 0 or count < 3)
+
+
+def test_page_table_entries_need_no_new_pinned_memory(fw, monkeypatch):
+    """From the first flush on, and for more entries than one part of the pinned memory holds (several launches, the parts in turn)."""
+    from hector_engine_amd.cache.paged import _Tables
+    t, made = _Tables(2, 100, 100, torch.device("cuda:0")), torch.empty
+
+    def empty(*size, **kw):
+        assert not kw.get("pin_memory")
+        return made(*size, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+    for round_, n in enumerate((1, 300, 4096, 4097, 20000, 2, 9000)):
+        for i in torch.randperm(20000, generator=torch.Generator().manual_seed(n))[:n].tolist():
+            t.write(i, (i + round_) % 97 - 1)
+        t.flush()
+    assert (t.device.cpu().numpy() == t.host).all()
