@@ -43,7 +43,7 @@
 // 9.8; 37888 x 3584 at 16 rows in thirty-twos 49, in eights 86.
 // NW = 8 wavefronts take a K slice each; 4 where that leaves a slice one instruction and the chip has other workgroups to run
 // (151936 x 896 at 4 rows 43 us, with eight 52). A wavefront with a single accumulator asks for two units a step (896 x 4864 at 8 rows 6.0 us, 6.8).
-// plan arguments NA, S, NW <= 0: this choice.
+// plan arguments NA, S, NW <= 0: this choice; NA: instructions' weight rows a wavefront holds (1, 2 or 4; 1 or 2 above 16 rows), S: units a step.
 static BlockSplitPlan blocksplit_plan(int M, int N, int K, int NA, int S, int NW) {
   BlockSplitPlan p;
   const int cus = he_cus();
@@ -101,10 +101,9 @@ static BlockSplitPlan ordered_plan(int M, int N, int K) {
     rows = ((N + cus * rounds - 1) / (cus * rounds) + 1) & ~1;
     r = rows > 16 ? 2 : 1;
   }
-  while (nw > 1 && K / nw < 128) nw >>= 1;
+  while (nw > 1 && K / nw < 128) nw >>= 1;      // (at most 8: bs_max_waves for any of these)
   // (Two units of a turn a step also where a wavefront has one accumulator and turns of two: 2048 x 32768 in sixteen groups, 4 rows, 31.7 -> 28.5 us;
   // with two accumulators 65536 x 2048 so 36.7 -> 41.9.)
-  if (u * (r + 1) > 4 && nw > 8) nw = 8;
   p.NA = r, p.S = u > 1 || r == 1 ? 2 : 1, p.NW = nw;
   p.units = ((K + nw - 1) / nw + 63) / 64;
   p.turn = 2 * u;
@@ -119,7 +118,8 @@ extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
   return (N + p.rows_per_block - 1) / p.rows_per_block;
 }
 
-// R, U, NW <= 0 choose the heuristic tiling (NW wavefronts = K slices per workgroup).
+// NA, S, NW: the tiling asked for, <= 0 the one blocksplit_plan chooses (NW wavefronts = K slices per workgroup). S = 4 asks for two units, as 2 does
+// (not beside NA = 4).
 // scale_partials: sums of squares of the input rows (the rows are then scaled before
 // bias or gate); resid: the residual epilogue (C is not written; gain, xg, sq_out needed). unary: an activation of one input
 // (he_unary's kinds) of the bf16 results, -1: none: a feed-forward without a gate writes its activations at once (a launch of its
@@ -127,7 +127,7 @@ extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
 // the experts of a routed step that nobody chose. ordered: see ordered_plan.
 extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W,
                                              const void* bias, int M, int N, int K, int out_dtype,
-                                             int bias_dtype, int gated, int R, int U, int NW,
+                                             int bias_dtype, int gated, int NA, int S, int NW,
                                              const void* scale_partials, int scale_count,
                                              float scale_eps, void* resid, const void* gain,
                                              int gain_dtype, void* xg, void* sq_out,
@@ -158,9 +158,14 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
                                  (used_rows > 0) != (used_k > 0) && (used_k == 0 || used_k >= 512) &&
                                  (resid == nullptr || used_rows == 0) && (resid != nullptr || out_dtype == HE_BF16)),
              "he_gemm_blocksplit_bf16: groups that are used: up to 16 rows, bf16 results, along the rows or in stretches of 512 k and more");
-  HE_REQUIRE(!ordered || (M <= 16 && resid == nullptr && R <= 0 && U <= 0 && NW <= 0),
+  HE_REQUIRE(!ordered || (M <= 16 && resid == nullptr && NA <= 0 && S <= 0 && NW <= 0),
              "he_gemm_blocksplit_bf16: ordered sums are for up to 16 rows, plan themselves and leave no residual");
-  const BlockSplitPlan p = ordered ? ordered_plan(M, N, K) : blocksplit_plan(M, N, K, R, U, NW);
+  HE_REQUIRE(NA <= (M <= 16 ? 4 : 2) && NA != 3 && S <= (M <= 16 && NA != 4 ? 4 : 2) && S != 3,
+             "he_gemm_blocksplit_bf16: no tiling NA=%d S=%d at M=%d", NA, S, M);
+  const BlockSplitPlan p = ordered ? ordered_plan(M, N, K) : blocksplit_plan(M, N, K, NA, S, NW);
+  // (a lane's offsets into X and into its workgroup's weight rows are 32 bits of bytes)
+  const int most_rows = N < p.rows_per_block ? N : p.rows_per_block;
+  HE_REQUIRE((int64_t)(M > most_rows ? M : most_rows) * K < (1ll << 31), "he_gemm_blocksplit_bf16: K=%d: rows too long", K);
   HE_REQUIRE(p.NW >= 1 && p.NW <= 16, "he_gemm_blocksplit_bf16: %d wavefronts outside [1, 16]",
              p.NW);
   const int blocks = (N + p.rows_per_block - 1) / p.rows_per_block;
@@ -209,8 +214,8 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
 
 extern "C" int he_gemm_blocksplit_bf16(void* C, const void* A, const void* W, const void* bias,
                                        int M, int N, int K, int out_dtype, int bias_dtype,
-                                       int gated, int R, int U, int NW, void* stream) {
-  return he_gemm_blocksplit_fused_bf16(C, A, W, bias, M, N, K, out_dtype, bias_dtype, gated, R, U,
+                                       int gated, int NA, int S, int NW, void* stream) {
+  return he_gemm_blocksplit_fused_bf16(C, A, W, bias, M, N, K, out_dtype, bias_dtype, gated, NA, S,
                                        NW, nullptr, 0, 0.f, nullptr, nullptr, HE_F32, nullptr,
                                        nullptr, 0, 0, 0, 1.f, 0.f, 0.f, 0.f, 1.f, nullptr, nullptr, -1, nullptr, 0, 0, 0, 0, 0, stream);
 }

@@ -532,13 +532,15 @@ int he_blocksplit_tiles_used_resid(HE_BS_DISPATCH_ARGS);      // (up to 16 rows)
   HE_BS_TILING(1, 1, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 1, 4, 2, OUT_, USED_, TC_)         \
   HE_BS_TILING(1, 2, 1, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 1, 2, OUT_, USED_, TC_)         \
   HE_BS_TILING(1, 2, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 2, 2, OUT_, USED_, TC_)         \
-  HE_BS_TILING(1, 2, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 4, 2, OUT_, USED_, TC_)             \
-  HE_BS_TILING(0, 1, 1, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 1, 2, OUT_, USED_, TC_)             \
-  HE_BS_TILING(0, 1, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 2, 2, OUT_, USED_, TC_)             \
+  HE_BS_TILING(1, 2, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(1, 2, 4, 2, OUT_, USED_, TC_)
+// (what ordered_plan gives; no residual epilogue goes with it)
+#define HE_BS_ORDERED(OUT_, USED_, TC_)                                                           \
+  HE_BS_TILING(0, 1, 1, 2, OUT_, USED_, TC_)                                                      \
+  HE_BS_TILING(0, 1, 2, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 2, 2, OUT_, USED_, TC_)         \
   HE_BS_TILING(0, 1, 4, 1, OUT_, USED_, TC_) HE_BS_TILING(0, 1, 4, 2, OUT_, USED_, TC_)
-#define HE_BS_ALL_TILINGS(OUT_, TC_)                                                              \
-  HE_BS_SIXTEEN_ROWS(OUT_, false, TC_)                                                            \
+#define HE_BS_THIRTY_TWO_ROWS(OUT_, TC_)                                                          \
   HE_BS_TILING(0, 2, 1, 1, OUT_, false, TC_) HE_BS_TILING(0, 2, 1, 2, OUT_, false, TC_)         \
-  HE_BS_TILING(0, 2, 2, 1, OUT_, false, TC_) HE_BS_TILING(0, 2, 2, 2, OUT_, false, TC_)         \
+  HE_BS_TILING(0, 2, 2, 1, OUT_, false, TC_) HE_BS_TILING(0, 2, 2, 2, OUT_, false, TC_)
+#define HE_BS_NO_TILING                                                                           \
   he_set_error("he_gemm_blocksplit_bf16: no kernel for SP=%d MT=%d NA=%d S=%d", p.SP, p.MT, p.NA, p.S); \
   return -1

@@ -2,5 +2,8 @@
 #include "gemm_blocksplit_tiles.h"
 
 int he_blocksplit_tiles_gated_bf16(HE_BS_DISPATCH_ARGS) {
-  HE_BS_ALL_TILINGS(BS_GATED, bf16_t);
+  HE_BS_SIXTEEN_ROWS(BS_GATED, false, bf16_t)
+  HE_BS_ORDERED(BS_GATED, false, bf16_t)
+  HE_BS_THIRTY_TWO_ROWS(BS_GATED, bf16_t)
+  HE_BS_NO_TILING;
 }

@@ -79,7 +79,7 @@ int he_gemm_plain(void* C, const void* A, const void* W, const void* bias, int M
 // wavefronts, one slice each, added in LDS): complete in one launch.
 #define HE_BLOCKSPLIT_MAX_M 32
 int he_gemm_blocksplit_bf16(void* C, const void* A, const void* W, const void* bias, int M, int N,
-                            int K, int out_dtype, int bias_dtype, int gated, int R, int U, int NW,
+                            int K, int out_dtype, int bias_dtype, int gated, int NA, int S, int NW,
                             void* stream);
 // The same with an RMS norm carried across a pair of products. resid != null: the residual
 // epilogue (resid[M,N] fp32 += result in place, xg[M,N] bf16 = resid * gain, sq_out[M, sq_count]
@@ -89,8 +89,8 @@ int he_gemm_blocksplit_bf16(void* C, const void* A, const void* W, const void* b
 // 16-byte pieces [D / 8][M][8], element (m, d) at ((d / 8) M + m) 8 + d % 8.
 int he_gemm_blocksplit_blocks(int M, int N, int K);
 int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void* W, const void* bias, int M,
-                                  int N, int K, int out_dtype, int bias_dtype, int gated, int R,
-                                  int U, int NW, const void* scale_partials, int scale_count,
+                                  int N, int K, int out_dtype, int bias_dtype, int gated, int NA,
+                                  int S, int NW, const void* scale_partials, int scale_count,
                                   float scale_eps, void* resid, const void* gain, int gain_dtype,
                                   void* xg, void* sq_out, int sq_count, int x_pieces, int out_pieces,
                                   float act_alpha, float act_limit, float act_shift, float act_cubic, float resid_scale,

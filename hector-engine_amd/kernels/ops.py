@@ -311,8 +311,9 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
                     act=(1.0, 0.0, 0.0), unary: str | None = None, used=None, ordered: bool = False) -> None:
     """bf16 MFMA product for M <= 32 with K cut inside the workgroup; one launch, complete
     result (bf16 or fp32), with bias or, gated, as [M, N/2] = silu(gate) * up for a weight
-    that alternates gate and up rows (gate i at row 2i, its up at 2i + 1). plan = (R, U, NW),
-    zeros = heuristic. act = (alpha, limit, up_shift[, cubic]): the gated epilogue's
+    that alternates gate and up rows (gate i at row 2i, its up at 2i + 1). plan = (NA, S, NW): the instructions' weight
+    rows a wavefront holds (1, 2 or 4; above 16 rows 1 or 2), its units of k a step (1 or 2; up to 16 rows 4 means 2, not with
+    NA = 4) and the wavefronts; zeros: as the sizes say. act = (alpha, limit, up_shift[, cubic]): the gated epilogue's
     constants as silu_mul takes them.
 
     row_scale = (partials fp32 [M, count], eps): the rows of `a` are r * gain of an RMS norm
