@@ -146,7 +146,8 @@ class Linear:
         w = self.weight
         N = w.shape[0]
         act, a, scale, pieces = _operand(x)
-        if sink is not None and out is None and out_dtype == act \
+        # (up to 16 rows the residual epilogue has one order of sums, not the kept one)
+        if sink is not None and out is None and out_dtype == act and not (self.ordered and rows <= ops.BLOCKSPLIT_PIECES_MAX_M) \
                 and sink.stream.rows == rows and sink.stream.resid.shape[-1] == N:
             return self._into_residual(x, bias, rows, ctx, sink, used)
         if out is None:

@@ -2,10 +2,15 @@
 
 The order is told with the tile kernel, which adds in the order of k: K is laid out anew in the order of units of 64 k that is stated for the kernel under
 test, 16 of a unit's k to a lane group as that has them, and the results are the same bits, which another order's are not."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
+from hector_engine_amd.engine.scratch import ScratchPool
 from hector_engine_amd.kernels import ops
+from hector_engine_amd.parts.base import BuildEnv
+from hector_engine_amd.parts.linear import Linear
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -204,3 +209,25 @@ def test_rows_beyond_32_bit_offsets_are_refused():
     x, w = torch.empty(16, K, dtype=BF16, device="cuda"), torch.empty(2, K, dtype=BF16, device="cuda")
     with pytest.raises(RuntimeError):
         ops.gemm_blocksplit(torch.empty(16, 2, device="cuda"), x, w, None, 16)
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17])
+def test_an_ordered_product_leaves_no_residual(rows):
+    """A layer whose products keep their order gives its results as they are, also where the caller's stream would take them (above 16 rows
+    there is one order)."""
+    x, w = operands(rows, 512, 2048)
+    lin = Linear(w)
+    lin.ordered = True
+    scratch = ScratchPool(torch.device("cuda:0"))
+    ctx = SimpleNamespace(rows=rows, env=BuildEnv(torch.device("cuda:0"), BF16, True), scratch=scratch,
+                          alloc=lambda shape, dtype=BF16: scratch.alloc(shape, dtype or BF16))
+    resid = torch.zeros(rows, 512, device="cuda")
+    norm = SimpleNamespace(carried=lambda: (torch.ones(512, dtype=BF16, device="cuda"), 1e-6))
+    sink = SimpleNamespace(stream=SimpleNamespace(rows=rows, resid=resid, prepared=None), norm=norm, scale=1.0)
+    out = lin(x, rows, ctx, sink=sink)
+    if rows > 16:
+        assert out is None and sink.stream.prepared is not None
+        return
+    want = torch.empty(rows, 512, dtype=BF16, device="cuda")
+    ops.gemm_blocksplit(want, x, w, None, rows, ordered=True)
+    assert torch.equal(out, want) and (resid == 0).all() and sink.stream.prepared is None
