@@ -70,30 +70,32 @@ static BlockSplitPlan blocksplit_plan(int M, int N, int K, int NA, int S, int NW
   return p;
 }
 
-// The tiling of the ordered sums of up to 16 rows: tiles, K slices and turns of 128 u k as this product had them before its lanes
-// were spread. For weights whose results reach a router over rows that no norm has evened out: there another order of sums turns
-// near ties over.
+// The tiling of the ordered sums: tiles, K slices and turns of 128 u k as this product had them before its lanes were spread. For weights of up
+// to 16 rows whose results reach a router over rows that no norm has evened out (there another order of sums turns near ties over), and for
+// 17 to 32 rows.
 static BlockSplitPlan ordered_plan(int M, int N, int K) {
   BlockSplitPlan p;
   const int cus = he_cus();
-  p.SP = 0, p.MT = 1;
+  p.SP = 0, p.MT = M <= 16 ? 1 : 2;
   int r, u, nw;
   if (N >= 256 * cus) {             // 256 rows or more a unit
     if (M <= 8) r = 2, u = 1, nw = 8;
-    else r = 4, u = 2, nw = 4;
+    else r = p.MT == 1 ? 4 : 2, u = 2, nw = 4;
   } else if (K >= 8192) {           // long K
     const int groups = (N + 31) / 32, last_round = groups % cus;   // with two tiles a workgroup
-    if (N < 16 * cus) r = 1, u = 1, nw = 8;
+    if (N < 16 * cus) r = 1, u = 1, nw = p.MT == 1 ? 8 : 4;
+    else if (p.MT == 2) r = 2, u = 2, nw = 4;
     else if (M > 8 && N >= 40 * cus) r = 4, u = 2, nw = 4;
     else if (groups < cus) r = 2, u = 1, nw = 8;
     else if (groups < 4 * cus && last_round > 0 && last_round <= cus / 2) r = 1, u = 1, nw = 8;
     else if (K >= 16384) r = 2, u = 2, nw = 8;
     else r = 2, u = 4, nw = 4;
   } else if (N >= 64 * cus) {       // wide N
-    r = M > 8 ? 4 : 2, u = 1, nw = 8;
-    if (K < 5120) r = 2, u = 2, nw = 4;
+    r = M > 8 && p.MT == 1 ? 4 : 2, u = 1, nw = 8;
+    if (K < 5120) r = 2;
+    if (p.MT == 2 || K < 5120) u = 2, nw = 4;
   } else {                          // small products
-    r = N >= 16 * cus ? 2 : 1, u = K < 5120 ? 4 : 1, nw = 8;
+    r = N >= 16 * cus ? 2 : 1, u = p.MT == 1 && K < 5120 ? 4 : 1, nw = 8;
   }
   int rows = 0;
   if (r <= 2 && N >= 2 * cus && N < 256 * cus) {      // dealt out evenly over the compute units, an even number each
@@ -103,8 +105,8 @@ static BlockSplitPlan ordered_plan(int M, int N, int K) {
   }
   while (nw > 1 && K / nw < 128) nw >>= 1;      // (at most 8: bs_max_waves for any of these)
   // (Two units of a turn a step also where a wavefront has one accumulator and turns of two: 2048 x 32768 in sixteen groups, 4 rows, 31.7 -> 28.5 us;
-  // with two accumulators 65536 x 2048 so 36.7 -> 41.9.)
-  p.NA = r, p.S = u > 1 || r == 1 ? 2 : 1, p.NW = nw;
+  // with two accumulators 65536 x 2048 so 36.7 -> 41.9; above 16 rows 3584 x 18944 39.5 -> 38.0, but 3584 x 3584 11.3 -> 12.1.)
+  p.NA = r, p.S = u > 1 || (r == 1 && (p.MT == 1 || K >= 8192)) ? 2 : 1, p.NW = nw;
   p.units = ((K + nw - 1) / nw + 63) / 64;
   p.turn = 2 * u;
   p.rows_per_block = rows > 0 ? rows : 16 * r;
@@ -114,7 +116,7 @@ static BlockSplitPlan ordered_plan(int M, int N, int K) {
 // Workgroups (= partial sums of squares per row) the residual epilogue of this product gives.
 extern "C" int he_gemm_blocksplit_blocks(int M, int N, int K) {
   if (M <= 0 || M > HE_BLOCKSPLIT_MAX_M || N <= 0 || K <= 0) return 0;
-  const BlockSplitPlan p = blocksplit_plan(M, N, K, 0, 0, 0);
+  const BlockSplitPlan p = M > 16 ? ordered_plan(M, N, K) : blocksplit_plan(M, N, K, 0, 0, 0);
   return (N + p.rows_per_block - 1) / p.rows_per_block;
 }
 
@@ -162,7 +164,8 @@ extern "C" int he_gemm_blocksplit_fused_bf16(void* C, const void* A, const void*
              "he_gemm_blocksplit_bf16: ordered sums are for up to 16 rows, plan themselves and leave no residual");
   HE_REQUIRE(NA <= (M <= 16 ? 4 : 2) && NA != 3 && S <= (M <= 16 && NA != 4 ? 4 : 2) && S != 3,
              "he_gemm_blocksplit_bf16: no tiling NA=%d S=%d at M=%d", NA, S, M);
-  const BlockSplitPlan p = ordered ? ordered_plan(M, N, K) : blocksplit_plan(M, N, K, NA, S, NW);
+  const bool planned = NA <= 0 && S <= 0 && NW <= 0;
+  const BlockSplitPlan p = ordered || (planned && M > 16) ? ordered_plan(M, N, K) : blocksplit_plan(M, N, K, NA, S, NW);
   // (a lane's offsets into X and into its workgroup's weight rows are 32 bits of bytes)
   const int most_rows = N < p.rows_per_block ? N : p.rows_per_block;
   HE_REQUIRE((int64_t)(M > most_rows ? M : most_rows) * K < (1ll << 31), "he_gemm_blocksplit_bf16: K=%d: rows too long", K);

@@ -93,8 +93,9 @@ __device__ __forceinline__ void bs_store_pieces(uint16_t* base, int M, int m, in
 // line each. Whole lines can be asked for past the caches (he_load16_once), which half lines cannot: the other half would be
 // fetched twice. 37888 x 3584 at 1 row 50.8 -> 42 us (6.4 TB/s), at 8 rows 52.5 -> 42, 3584 x 3584 at 1 row 9.6 -> 6.2.
 // SP = 0 keeps each sum in the order this product had before: a unit of 64 k is two instructions, whose lanes take the halves of 16
-// neighbouring k (loaded as whole lines all the same, see he_halves_to_rows). For 17 to 32 rows, and where a caller asks for that order (`ordered`; also the K slices and, by workgroup, the
-// turn each wavefront begins at are then those it had).
+// neighbouring k (loaded as whole lines all the same, see he_halves_to_rows), and the K slices and, by workgroup, the turn each
+// wavefront begins at are those it had. For 17 to 32 rows, whose rows of X are loaded in whole lines too (37888 x 3584 at 17, 24 and 32 rows 60.8, 67.3
+// and 72.4 us with half lines of both, so 54.6, 60.5 and 67.0; half lines of X alone 56.7, 65.6 and 75.0), and where a caller asks for that order (`ordered`).
 template <int SP>
 struct BsLanes {
   static constexpr int RT = 16 >> SP;              // weight rows, and rows of X, of an instruction
@@ -189,7 +190,8 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_
     const uint16_t* __restrict__ W, const uint16_t* __restrict__ X, int M, int N, int K, int rows_per_block, int units_per_wave,
     int turn, int bias_dtype, TC* __restrict__ C, const void* __restrict__ bias, BsFusion fu) {
   using L = BsLanes<SP>;
-  constexpr bool ORDERED = SP == 0 && MT == 1;
+  constexpr bool ORDERED = SP == 0;
+  constexpr bool X_LINES = ORDERED && MT == 2;  // rows of X in whole lines too, where there are enough of them
   constexpr int ROWS = L::RT * NA;              // weight rows a workgroup can hold
   constexpr int MX = L::RT * MT;                // rows of X
   extern __shared__ float4 tiles[];             // [NW][MX][ROWS] floats
@@ -216,14 +218,16 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_
   const char* const wb = reinterpret_cast<const char*>(W + (int64_t)n0 * K);
   const char* const xb = reinterpret_cast<const char*>(X);
   const int k_lane = SP == 0 ? 16 * lg : 8 * ((lg << SP) | (lr & (L::PARTS - 1)));    // this lane's first k of a unit
-  uint32_t wo[L::H][NA], xo[MT];
+  uint32_t wo[L::H][NA], xo[L::H][MT];
   const bool upper = (lr & 8) != 0;
 #pragma unroll
   for (int h = 0; h < L::H; ++h)
 #pragma unroll
     for (int a = 0; a < NA; ++a) wo[h][a] = 2u * (uint32_t)(min((SP == 0 ? (lr & 7) + 8 * h : row) * NA + a, n_end - n0 - 1) * K);
 #pragma unroll
-  for (int t = 0; t < MT; ++t) xo[t] = 2u * (uint32_t)(min(t * L::RT + xrow, M - 1) * (PIECES ? 8 : K));
+  for (int h = 0; h < L::H; ++h)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xo[h][t] = 2u * (uint32_t)(min(t * L::RT + (X_LINES ? (lr & 7) + 8 * h : xrow), M - 1) * (PIECES ? 8 : K));
   const uint32_t xk = PIECES ? 2 * M : 2;                         // piece-major X: the piece of 8 k from k on lies at k M (+ 8 row)
 
   floatx4 acc[NA][MT];
@@ -246,13 +250,16 @@ __global__ __launch_bounds__(64 * bs_max_waves(MT, NA, S)) void gemm_blocksplit_
 #pragma unroll
         for (int a = 0; a < NA; ++a) f.a[s][h][a] = he_load16_once<bf16x8>(wb + (wo[h][a] + 2 * kw));
 #pragma unroll
-        for (int t = 0; t < MT; ++t) f.b[s][h][t] = bs_load8(xb + (xo[t] + k * xk));
+        for (int t = 0; t < MT; ++t) f.b[s][h][t] = bs_load8(xb + (xo[h][t] + (X_LINES ? kw : k) * xk));
       }
   };
   auto in_place = [&](BsFrags<MT, NA, S, L::H>& f, int s) {
     if constexpr (SP == 0)
 #pragma unroll
       for (int a = 0; a < NA; ++a) he_halves_to_rows(f.a[s][0][a], f.a[s][1][a], upper);
+    if constexpr (X_LINES)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) he_halves_to_rows(f.b[s][0][t], f.b[s][1][t], upper);
   };
   auto multiply_unit = [&](const BsFrags<MT, NA, S, L::H>& f, int s) {
 #pragma unroll

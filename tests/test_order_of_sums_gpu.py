@@ -55,13 +55,15 @@ def operands(M, N, K):
 # (a shape for each branch of the ordered tiling, on 256 units: weight rows a workgroup has, its wavefronts, units of a turn)
 ORDERED = [(3, 65536, 2048, 32, 8, 2), (12, 65537, 2048, 64, 4, 4), (5, 896, 8192, 4, 8, 2), (4, 300, 8256, 16, 8, 2), (16, 10240, 8192, 64, 4, 4),
            (8, 4608, 8192, 18, 8, 2), (2, 10240, 8192, 20, 8, 2), (4, 8192, 16384, 32, 8, 4), (1, 8192, 8192, 32, 4, 8), (7, 16384, 3584, 32, 4, 4),
-           (4, 16384, 5120, 32, 8, 2), (9, 16500, 5120, 64, 8, 2), (4, 4608, 3584, 18, 8, 8), (1, 3584, 5128, 14, 8, 2), (4, 512, 520, 2, 4, 8)]
+           (4, 16384, 5120, 32, 8, 2), (9, 16500, 5120, 64, 8, 2), (4, 4608, 3584, 18, 8, 8), (1, 3584, 5128, 14, 8, 2), (4, 512, 520, 2, 4, 8),
+           (20, 4608, 3584, 18, 8, 2), (17, 3584, 18944, 14, 4, 2), (32, 16384, 3584, 32, 4, 4), (24, 65537, 2048, 32, 4, 4), (31, 4104, 8200, 18, 4, 4),
+           (29, 300, 1032, 16, 8, 2)]
 
 
 @pytest.mark.parametrize("M,N,K,rows,waves,turn", ORDERED)
 def test_ordered_sums_are_added_as_they_always_were(M, N, K, rows, waves, turn):
     """Wavefronts with a K slice each, whose walk begins at a turn of the workgroup's own and goes around, and which are added in their order; an
-    activation and a gated product walk the same way."""
+    activation walks the same way. Above 16 rows that is the only order."""
     if ops.compute_units() != 256:
         pytest.skip("the tilings of 256 compute units")
     x, w = operands(M, N, K)
@@ -75,16 +77,18 @@ def test_ordered_sums_are_added_as_they_always_were(M, N, K, rows, waves, turn):
         starts = (3 * torch.arange(-(-N // rows), device="cuda")) % max(whole // turn, 1) * turn
         want = want + chained(xu, wu, block, lambda f: [u0 + (f + j) % whole for j in range(whole)] + list(range(u0 + whole, u1)), starts)
     pieces = x.view(M, K // 8, 8).transpose(0, 1).contiguous()
-    for given, more in ((x, {}), (pieces, dict(x_pieces=True))):
+    for given, more in ((x, {}), (pieces, dict(x_pieces=True)))[:2 if M <= 16 else 1]:
         out = torch.empty(M, N, device="cuda")
-        ops.gemm_blocksplit(out, given, w, None, M, ordered=True, **more)
+        ops.gemm_blocksplit(out, given, w, None, M, ordered=M <= 16, **more)
         assert torch.equal(out, want)
+    half = torch.empty(M, N, dtype=BF16, device="cuda")
+    ops.gemm_blocksplit(half, x, w, None, M, ordered=M <= 16, unary="relu")
+    assert torch.equal(half, want.to(BF16).relu())
+    if M > 16:
+        return
     free = torch.empty(M, N, device="cuda")
     ops.gemm_blocksplit(free, x, w, None, M)
     assert not torch.equal(free, want)                        # (another order does give other bits)
-    half = torch.empty(M, N, dtype=BF16, device="cuda")
-    ops.gemm_blocksplit(half, x, w, None, M, ordered=True, unary="relu")
-    assert torch.equal(half, want.to(BF16).relu())
 
 
 @pytest.mark.parametrize("M,N,K,R,NWV", [(17, 4608, 3584, 1, 8), (64, 4608, 3584, 1, 8), (33, 3584, 18944, 1, 8), (20, 900, 1032, 1, 4), (64, 16400, 1096, 1, 16),
