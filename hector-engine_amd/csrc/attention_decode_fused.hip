@@ -226,8 +226,8 @@ __device__ __forceinline__ void fused_join(const float* ws_o, const float* ws_ml
 }
 
 // SLICED: qkv is null and the projection row comes as the fp32 sums of its K slices,
-// qkv_part [qkv_slices][.][qkv_stride], slice_stride elements from slice to slice.
-template <int NT, bool SLICED>
+// qkv_part [qkv_slices][.][qkv_stride], slice_stride elements from slice to slice. ONCE: see ld8 (a single tile of heads a group).
+template <int NT, bool SLICED, bool ONCE>
 __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
     uint16_t* __restrict__ out, float* ws_o, float* ws_ml,      // (other workgroups' parts are read back: no __restrict__)
     const uint16_t* __restrict__ qkv, const float* __restrict__ qkv_part, int qkv_slices,
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
   float angle = (float)p * freq;
   asm volatile("" : "+v"(angle));
   __builtin_amdgcn_sched_barrier(0);
-  if (early) attend_first<NT, true>(cursor, kpool, vpool, num_pages, KVH, kvh, kb_begin, lr, lg);
+  if (early) attend_first<NT, ONCE>(cursor, kpool, vpool, num_pages, KVH, kvh, kb_begin, lr, lg);
   if (SLICED) {
     // The workgroup adds the slices of its heads' q once, four neighbouring values a thread, and hands
     // the sums round through LDS (the buffer the join uses at the end); every wavefront then takes its
@@ -434,8 +434,8 @@ __global__ __launch_bounds__(512) void attention_decode_fused_kernel(
   if (has_keys) {
     bf16x8 qf[KS];
     rotate_q<NT>(qf, qx, lg, sn, c);
-    if (!early) attend_start<NT, true>(cursor, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin, lr, lg);
-    attend_walk<NT, false, true>(st, qf, cursor, pt, max_blocks, num_pages, kb_begin, (kb_end + 31) & ~31,
+    if (!early) attend_start<NT, ONCE>(cursor, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin, lr, lg);
+    attend_walk<NT, false, ONCE>(st, qf, cursor, pt, max_blocks, num_pages, kb_begin, (kb_end + 31) & ~31,
                            first, p, first, p, scale * 1.4426950408889634f, lr, lg);
   }
   float l = st.l;
@@ -617,8 +617,8 @@ extern "C" int he_attention_decode_fused_bf16(void* out, const void* qkv, const 
   int32_t* counters = Z > 1 && nw == 4 && (int64_t)rows * KVH * head_tiles <= num_counters ? (int32_t*)counters_i32 : nullptr;
   hipStream_t s = (hipStream_t)stream;
   dim3 grid(KVH * head_tiles, rows, Z);
-#define FUSED_LAUNCH(NTV, SL)                                                                   \
-    attention_decode_fused_kernel<NTV, SL><<<grid, 64 * nw, lds, s>>>(                          \
+#define FUSED_LAUNCH(NTV, SL, ONCE)                                                             \
+    attention_decode_fused_kernel<NTV, SL, ONCE><<<grid, 64 * nw, lds, s>>>(                          \
         (uint16_t*)out, ws_o, ws_ml, (const uint16_t*)qkv, (const float*)qkv_part, qkv_slices,  \
         qkv_slice_stride, qkv_stride, bias, bias_dtype,                                         \
         (uint16_t*)kpool,                                                                       \
@@ -628,7 +628,10 @@ extern "C" int he_attention_decode_fused_bf16(void* out, const void* qkv, const 
         out_pieces, counters)
 #define FUSED(NTV)                                                                              \
   case NTV:                                                                                     \
-    if (qkv_part != nullptr) FUSED_LAUNCH(NTV, true); else FUSED_LAUNCH(NTV, false);            \
+    if (qkv_part != nullptr && head_tiles == 1) FUSED_LAUNCH(NTV, true, true);                  \
+    else if (qkv_part != nullptr) FUSED_LAUNCH(NTV, true, false);                               \
+    else if (head_tiles == 1) FUSED_LAUNCH(NTV, false, true);                                   \
+    else FUSED_LAUNCH(NTV, false, false);                                                       \
     break;
   switch (hd / 16) {
     FUSED(4) FUSED(8)

@@ -105,7 +105,8 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(
 // With a single slice in the grid the result is written directly.
 #define DECODE_MIN_CHUNK 64
 
-template <int NT, int MODE>
+// ONCE: see ld8 (a single tile of heads a group).
+template <int NT, int MODE, bool ONCE>
 __global__ __launch_bounds__(64) void attention_decode_kernel(
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml,
     const uint16_t* __restrict__ q,
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(64) void attention_decode_kernel(
   if (MODE == ATTN_SHAPED) st.sh = attn_shape_of(ex, h, scale);
   st.pos = n_keys - 1;
   const int hi = n_keys - 1;
-  attend_range<NT, false, true, MODE>(st, qf, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin,
+  attend_range<NT, false, ONCE, MODE>(st, qf, kpool, vpool, pt, max_blocks, num_pages, KVH, kvh, kb_begin,
                    (kb_end + 31) & ~31, first, hi, first, hi, MODE == ATTN_SHAPED ? 1.f : scale * 1.4426950408889634f, lr, lg);
   float l = st.l;
   l = xor32_sum(xor16_sum(l));
@@ -285,20 +286,20 @@ extern "C" int64_t he_attention_decode_workspace_floats(int rows, int H, int KVH
   return (int64_t)rows * H * decode_splits(rows, KVH, head_tiles, max_keys) * (hd + 2);
 }
 
-#define ATTN_DISPATCH(NTV, CALL) \
+#define ATTN_DISPATCH(NTV, ...)  \
   case NTV: {                    \
     constexpr int NT = NTV;      \
-    CALL;                        \
+    __VA_ARGS__;                 \
     break;                       \
   }
-#define ATTN_SWITCH(nt, CALL)                                                              \
+#define ATTN_SWITCH(nt, ...)                                                               \
   switch (nt) {                                                                            \
-    ATTN_DISPATCH(1, CALL) ATTN_DISPATCH(2, CALL) ATTN_DISPATCH(3, CALL)                   \
-    ATTN_DISPATCH(4, CALL) ATTN_DISPATCH(5, CALL) ATTN_DISPATCH(6, CALL)                   \
-    ATTN_DISPATCH(7, CALL) ATTN_DISPATCH(8, CALL) ATTN_DISPATCH(9, CALL)                   \
-    ATTN_DISPATCH(10, CALL) ATTN_DISPATCH(11, CALL) ATTN_DISPATCH(12, CALL)                \
-    ATTN_DISPATCH(13, CALL) ATTN_DISPATCH(14, CALL) ATTN_DISPATCH(15, CALL)                \
-    ATTN_DISPATCH(16, CALL)                                                                \
+    ATTN_DISPATCH(1, __VA_ARGS__) ATTN_DISPATCH(2, __VA_ARGS__) ATTN_DISPATCH(3, __VA_ARGS__)                   \
+    ATTN_DISPATCH(4, __VA_ARGS__) ATTN_DISPATCH(5, __VA_ARGS__) ATTN_DISPATCH(6, __VA_ARGS__)                   \
+    ATTN_DISPATCH(7, __VA_ARGS__) ATTN_DISPATCH(8, __VA_ARGS__) ATTN_DISPATCH(9, __VA_ARGS__)                   \
+    ATTN_DISPATCH(10, __VA_ARGS__) ATTN_DISPATCH(11, __VA_ARGS__) ATTN_DISPATCH(12, __VA_ARGS__)                \
+    ATTN_DISPATCH(13, __VA_ARGS__) ATTN_DISPATCH(14, __VA_ARGS__) ATTN_DISPATCH(15, __VA_ARGS__)                \
+    ATTN_DISPATCH(16, __VA_ARGS__)                                                                \
     default:                                                                               \
       he_set_error("attention: head_dim %d is not a multiple of 16 up to 256", 16 * (nt)); \
       return -1;                                                                           \
@@ -347,11 +348,17 @@ extern "C" int he_attention_decode_bf16(void* out, const void* q, const void* kp
   (uint16_t*)out, ws_o, ws_ml, (const uint16_t*)q, (const uint16_t*)kpool, (const uint16_t*)vpool,     \
       (const int32_t*)positions, (const int32_t*)row_seq, (const int32_t*)seq_slot,                    \
       (const int32_t*)page_table, max_blocks, num_pages, H, KVH, head_tiles, window, scale, ex
+#define DECODE_LAUNCH(MODE_)                                                            \
+  do {                                                                                  \
+    if (head_tiles == 1) attention_decode_kernel<NT, MODE_, true><<<grid, 64, 0, s>>>(DECODE_ARGS); \
+    else attention_decode_kernel<NT, MODE_, false><<<grid, 64, 0, s>>>(DECODE_ARGS);    \
+  } while (0)
   switch (attn_mode(ex)) {
-    case ATTN_SLOPES: ATTN_SWITCH(hd / 16, (attention_decode_kernel<NT, ATTN_SLOPES><<<grid, 64, 0, s>>>(DECODE_ARGS))); break;
-    case ATTN_SHAPED: ATTN_SWITCH(hd / 16, (attention_decode_kernel<NT, ATTN_SHAPED><<<grid, 64, 0, s>>>(DECODE_ARGS))); break;
-    default: ATTN_SWITCH(hd / 16, (attention_decode_kernel<NT, ATTN_RAW><<<grid, 64, 0, s>>>(DECODE_ARGS)));
+    case ATTN_SLOPES: ATTN_SWITCH(hd / 16, DECODE_LAUNCH(ATTN_SLOPES)); break;
+    case ATTN_SHAPED: ATTN_SWITCH(hd / 16, DECODE_LAUNCH(ATTN_SHAPED)); break;
+    default: ATTN_SWITCH(hd / 16, DECODE_LAUNCH(ATTN_RAW));
   }
+#undef DECODE_LAUNCH
 #undef DECODE_ARGS
   int rc = he_check_launch("he_attention_decode_bf16");
   if (rc || nsplit == 1) return rc;

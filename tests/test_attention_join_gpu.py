@@ -46,3 +46,40 @@ def test_the_last_workgroup_joins_with_the_same_bits(ops, H, KVH, hd, lengths, m
     if groups > 1:
         few = torch.full((groups - 1,), 77, dtype=torch.int32, device="cuda")      # too few: not used
         assert torch.equal(run(False, few), want) and bool((few == 77).all())
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("G", [17, 20, 33])
+def test_tiles_of_heads_give_the_bits_of_groups_of_their_own(ops, hd, G):
+    """A group of more than 16 query heads, whose tiles walk the same keys by way of the caches, beside groups of 16 heads and fewer, whose keys are read
+    past them: in one launch and in two, 1 to 250 keys."""
+    KVH, lengths, max_keys = 2, [1, 33, 64, 250], 256
+    B, H = len(lengths), 2 * G
+    slots, table, kpool, vpool = paged_setup(lengths, KVH, hd, torch.bfloat16, 40)
+    fill_cache(table, slots, kpool, vpool, [rnd(n, KVH, hd, seed=61 + i).bfloat16() for i, n in enumerate(lengths)],
+               [rnd(n, KVH, hd, seed=171 + i).bfloat16() for i, n in enumerate(lengths)])
+    qkv = dev(rnd(B, (H + 2 * KVH) * hd, seed=81, scale=1.5).bfloat16())
+    inv, table = dev(P.rope_inv_freq(hd, 50000.0)), dev(table)
+    i32 = lambda v: dev(torch.tensor(v, dtype=torch.int32))
+    positions, row_seq, seq_slot = i32([n - 1 for n in lengths]), i32(range(B)), i32(slots)
+
+    def run(first, count, fused):
+        """The heads first .. first + count of both groups as groups of their own."""
+        q = qkv[:, :H * hd].view(B, KVH, G, hd)[:, :, first:first + count].reshape(B, -1)
+        if fused:
+            out = torch.empty(B, KVH * count * hd, dtype=torch.bfloat16, device="cuda")
+            floats = ops.attention_decode_fused_workspace_floats(B, KVH * count, KVH, hd, max_keys, False)
+            assert floats == 0
+            ops.attention_decode_fused(out, torch.cat([q, qkv[:, H * hd:]], 1).contiguous(), None, dev(kpool), dev(vpool), positions, row_seq, seq_slot, table,
+                                       inv, hd, B, KVH * count, KVH, hd, 0, hd ** -0.5, max_keys, True, None)
+        else:
+            out = torch.empty(B, KVH * count, hd, dtype=torch.bfloat16, device="cuda")
+            ws = torch.empty(ops.attention_decode_workspace_floats(B, KVH * count, KVH, hd, max_keys), device="cuda")
+            ops.attention_decode(out, q.reshape(B, -1, hd).contiguous(), dev(kpool), dev(vpool), positions, row_seq, seq_slot, table, B, KVH * count, KVH, hd, 0,
+                                 hd ** -0.5, max_keys, ws)
+        return out.view(B, KVH, count, hd)
+    for fused in (True, False):
+        whole = run(0, G, fused)
+        assert bool(torch.isfinite(whole.float()).all()) and whole.abs().max() > 0
+        for first in range(0, G, 16):
+            assert torch.equal(whole[:, :, first:first + 16], run(first, min(16, G - first), fused))
