@@ -221,16 +221,16 @@ __global__ __launch_bounds__(256, 2) void gemm_plain_mfma_kernel(
 // workgroup owns 16 weight rows and all activation rows (MT tiles of 16) and walks K with NW wavefronts, each
 // a segment of its own at a time: v_mfma_f32_16x16x4_f32 chains, whose sums go to LDS; after FLUSH rounds of
 // segments the workgroup adds them to its totals in segment order. So a weight of 3,584 rows still has 224 workgroups
-// with 16 wavefronts' loads in flight, and nothing goes through a workspace. (7B gate||up, 543 MB: 1 row 97 us, 4 rows
+// with 16 wavefronts' loads in flight, and nothing goes through a workspace. (7B gate||up, 543 MB, by way of the caches: 1 row 97 us, 4 rows
 // 98, 16 rows 128, 64 rows 308; a lane a weight row on the vector ALU and a second kernel for the segment sums, up to 8
 // rows, 104 and 114; 64 x 64 tiles, which more rows went through, 657 at 16 rows and, for the down projection's 3,584
 // weight rows of 18,944, 2479 where this takes 53.) A wavefront fetches a stage of KS k
 // of its 16 weight rows (and activation rows) whole lines at a time, two stages ahead, into its own LDS region, the
 // 16-byte pieces of row r at their index xor r, from which the operand of lane (row, k mod 4) is read a float at a
-// time without bank conflicts; the weights past the caches (he_load16_once; at 4 rows the 543 MB 98 -> 87 us). For weights of whole
-// segments in aligned rows.
+// time without bank conflicts; up to 64 rows the weights past the caches (ONCE: he_load16_once; at 4 rows the 543 MB 98 -> 87 us; more rows are two
+// workgroups' of the same weights, 2048 x 8192 at 65 rows 61.9 and 62.6 so). For weights of whole segments in aligned rows.
 #define GP_MROWS_MAX_M 64
-template <int MT, int NW, int KS>
+template <int MT, int NW, int KS, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void gemm_plain_stream_kernel(
     float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, const void* __restrict__ bias,
     int bias_dtype, int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc) {
@@ -278,7 +278,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_plain_stream_kernel(
     const int seg_ = wave + NW * ((ST_) / SPS);                                                      \
     if (seg_ < segments) {                                                                           \
       const int64_t k_ = (int64_t)seg_ * GP_SEG + ((ST_) % SPS) * KS;                                \
-      _Pragma("unroll") for (int t = 0; t < LD; ++t) wv[B_][t] = he_load16_once<gp_f32x4>(wsrc[t] + k_); \
+      _Pragma("unroll") for (int t = 0; t < LD; ++t) wv[B_][t] =                          \
+          ONCE ? he_load16_once<gp_f32x4>(wsrc[t] + k_) : *reinterpret_cast<const gp_f32x4*>(wsrc[t] + k_); \
       _Pragma("unroll") for (int i = 0; i < MT; ++i)                                                 \
         _Pragma("unroll") for (int t = 0; t < LD; ++t)                                               \
           if (real[i][t]) av[B_][i][t] = *reinterpret_cast<const gp_f32x4*>(asrc[i][t] + k_);        \
@@ -574,15 +575,17 @@ static int launch_rows(void* C, const void* A, const void* W, const void* bias, 
 static int launch_stream(float* C, const float* A, const float* W, const void* bias, int bias_dtype, int M, int N, int K,
                          int64_t lda, int64_t ldw, int64_t ldc, hipStream_t s) {
   const dim3 grid((N + 15) / 16, (M + GP_MROWS_MAX_M - 1) / GP_MROWS_MAX_M);
-#define GP_STREAM(MT_, NW_, KS_) \
-  gemm_plain_stream_kernel<MT_, NW_, KS_><<<grid, NW_ * 64, 0, s>>>(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc)
+#define GP_STREAM(MT_, NW_, KS_, ONCE_) \
+  gemm_plain_stream_kernel<MT_, NW_, KS_, ONCE_><<<grid, NW_ * 64, 0, s>>>(C, A, W, bias, bias_dtype, M, N, K, lda, ldw, ldc)
   if (M <= 16) {
-    if ((int)grid.x <= he_cus()) GP_STREAM(1, 16, 64);
-    else GP_STREAM(1, 8, 64);
+    if ((int)grid.x <= he_cus()) GP_STREAM(1, 16, 64, true);
+    else GP_STREAM(1, 8, 64, true);
   } else if (M <= 32) {
-    GP_STREAM(2, 8, 32);
+    GP_STREAM(2, 8, 32, true);
+  } else if (M <= GP_MROWS_MAX_M) {
+    GP_STREAM(4, 8, 32, true);
   } else {
-    GP_STREAM(4, 8, 32);
+    GP_STREAM(4, 8, 32, false);
   }
 #undef GP_STREAM
   return he_check_launch("he_gemm_plain");
