@@ -497,8 +497,10 @@ extern "C" int he_routed_act(void* out, const void* gate_up, const void* dense_f
 // ---- the chosen experts alone, for steps of very few rows ---------------------------------------
 // Where a step's rows choose fewer experts than there are, the two products over all experts read weights
 // nobody asked for. These two kernels walk only the chosen experts' rows of the same fused matrices (bf16):
-// a wavefront an output, the lanes along K with 16-byte loads (the weights' past the caches: 2 rows of 4 choices among experts of 2048 over
-// 2048 24.9 -> 23.3 us and 16.6 -> 15.7), sums in fp32.
+// a wavefront an output, the lanes along K with 16-byte loads, sums in fp32. Weights that one row of the step alone reads come past the caches, those
+// of an expert that several rows chose, and of the shared columns, by way of them: 8 rows of 4 choices among 64 experts of 1024 over 2048 and 2048 shared
+// columns, weights from memory, 80 us all by way of the caches, 86 all past them, 75 so; where all rows choose the same experts 47, 70 and 49. (One row of 4 choices
+// among 16 experts of 2048 over 2048 28.2 and 25.5.)
 __device__ __forceinline__ float dot8_bf16(const uint4& a, const uint4& b, float acc) {
   const uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -508,6 +510,27 @@ __device__ __forceinline__ float dot8_bf16(const uint4& a, const uint4& b, float
   }
   return acc;
 }
+
+// ONCE: past the caches (he_load16_once).
+template <bool ONCE>
+__device__ __forceinline__ uint4 chosen_load(const uint16_t* p) {
+  return ONCE ? he_load16_once<uint4>(p) : *reinterpret_cast<const uint4*>(p);
+}
+
+// The ids of a step of several rows, a lane each (up to 64: one trip to memory for all that a wavefront asks of them).
+struct ChosenIds {
+  int rows, n, mine;
+  bool held;
+  __device__ __forceinline__ ChosenIds(const int32_t* __restrict__ ids, int rows, int top)
+      : rows(rows), n(rows * top), mine(0), held(rows > 1 && n <= 64) {
+    if (held) mine = ids[min((int)(threadIdx.x & 63), n - 1)];
+  }
+  __device__ __forceinline__ int at(const int32_t* __restrict__ ids, int i) const { return held ? __builtin_amdgcn_readlane(mine, i) : ids[i]; }
+  // whether one row alone chose expert e (of more than 64 ids: not said)
+  __device__ __forceinline__ bool alone(int e) const {
+    return rows == 1 || (held && __popcll(__ballot((int)(threadIdx.x & 63) < n && mine == e)) == 1);
+  }
+};
 
 // Grid y: the rows * top (row, choice) pairs, then, with shared columns, the rows once more: those write h_shared[row][i].
 // h[(row, k), i] = weight[row, k] * act(gate . x[row], up . x[row]) with gate and up the rows 2 (e I + i) and
@@ -523,7 +546,8 @@ __global__ __launch_bounds__(256) void chosen_gate_up_kernel(uint16_t* __restric
   const bool common = (int)blockIdx.y >= rows * top;   // the columns every row uses
   const int64_t rk = blockIdx.y;                 // row * top + k
   if (i >= (common ? shared : I)) return;
-  const int e = common ? real : ids[rk];
+  const ChosenIds chosen(ids, rows, top);
+  const int e = common ? real : chosen.at(ids, (int)rk);
   const int64_t row = common ? rk - (int64_t)rows * top : rk / top;
   float g = 0.f, u = 0.f;
   if (common || (e >= 0 && e < real)) {
@@ -531,12 +555,17 @@ __global__ __launch_bounds__(256) void chosen_gate_up_kernel(uint16_t* __restric
     // row-major rows, or piece-major [D / 8][rows][8]
     const uint16_t* xr = x + (x_pieces ? 8 * row : row * D);
     const int64_t x_step = x_pieces ? rows : 1;
+    const auto walk = [&](auto once) {
+      constexpr bool ONCE = decltype(once)::value;
 #pragma unroll 4
-    for (int c = lane * 8; c < D; c += 512) {
-      const uint4 xv = *reinterpret_cast<const uint4*>(xr + c * x_step);
-      g = dot8_bf16(he_load16_once<uint4>(wg + c), xv, g);
-      u = dot8_bf16(he_load16_once<uint4>(wg + D + c), xv, u);
-    }
+      for (int c = lane * 8; c < D; c += 512) {
+        const uint4 xv = *reinterpret_cast<const uint4*>(xr + c * x_step);
+        g = dot8_bf16(chosen_load<ONCE>(wg + c), xv, g);
+        u = dot8_bf16(chosen_load<ONCE>(wg + D + c), xv, u);
+      }
+    };
+    if (common ? rows == 1 : chosen.alone(e)) walk(std::true_type{});
+    else walk(std::false_type{});
   }
   g = wave_sum(g);
   u = wave_sum(u);
@@ -558,20 +587,26 @@ __global__ __launch_bounds__(256) void chosen_down_kernel(uint16_t* __restrict__
   const int d = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t row = blockIdx.y;
   if (d >= D) return;
+  const int rows = gridDim.y;
   float acc = 0.f;
+  const auto walk = [&](const uint16_t* w, const uint16_t* hr, int n, auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+#pragma unroll 4
+    for (int c = lane * 8; c < n; c += 512) acc = dot8_bf16(chosen_load<ONCE>(w + c), *reinterpret_cast<const uint4*>(hr + c), acc);
+  };
+  const ChosenIds chosen(ids, rows, top);
   for (int k = 0; k < top; ++k) {
-    const int e = ids[row * top + k];
+    const int e = chosen.at(ids, (int)row * top + k);
     if (e < 0 || e >= real) continue;
     const uint16_t* w = down + (int64_t)d * ldw + (int64_t)e * I;
     const uint16_t* hr = h + (row * top + k) * I;
-#pragma unroll 4
-    for (int c = lane * 8; c < I; c += 512)
-      acc = dot8_bf16(he_load16_once<uint4>(w + c), *reinterpret_cast<const uint4*>(hr + c), acc);
+    if (chosen.alone(e)) walk(w, hr, I, std::true_type{});
+    else walk(w, hr, I, std::false_type{});
   }
   const uint16_t* ws = down + (int64_t)d * ldw + (int64_t)real * I;
-  const uint16_t* hs = h + (int64_t)gridDim.y * top * I + row * shared;
-  for (int c = lane * 8; c < shared; c += 512)
-    acc = dot8_bf16(he_load16_once<uint4>(ws + c), *reinterpret_cast<const uint4*>(hs + c), acc);
+  const uint16_t* hs = h + (int64_t)rows * top * I + row * shared;
+  if (rows == 1) walk(ws, hs, shared, std::true_type{});
+  else walk(ws, hs, shared, std::false_type{});
   acc = wave_sum(acc);
   if (lane == 0)
     out[row * D + d] = float_to_bf16_bits(

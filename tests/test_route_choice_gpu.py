@@ -145,3 +145,33 @@ def test_equal_outputs_tie_wherever_they_stand(copies, rows):
         dense, ids = torch.empty(rows, E + 1, device="cuda"), torch.full((rows, top), 77, dtype=torch.int32, device="cuda")
         ops.route_tokens(dense, ids, torch.empty(rows, top, device="cuda"), given.pop("logits"), correction, rows, E, 1, 1, top, 1.0, **given)
         assert torch.equal(ids, torch.cat([ids[:, i * copies:i * copies + 1] + 64 * torch.arange(copies, device="cuda", dtype=torch.int32) for i in range(3)], 1))
+
+
+@pytest.mark.parametrize("rows,top,real,I,D,shared", [(1, 4, 16, 64, 128, 32), (2, 4, 16, 520, 264, 0), (5, 3, 30, 72, 1032, 40), (16, 4, 128, 24, 64, 8), (17, 4, 140, 24, 64, 8), (33, 2, 140, 16, 72, 16)])
+@pytest.mark.parametrize("kind", ["apart", "same", "some", "none"])
+def test_chosen_experts_of_a_row_do_not_depend_on_the_others(rows, top, real, I, D, shared, kind):
+    """Experts that one row chose, several, or all, ids that name no expert, up to 64 ids and more of them: each row has the bits it has alone,
+    whichever way its weights come."""
+    from hector_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + I)
+    ids = torch.stack([torch.randperm(real, generator=g)[:top] for _ in range(rows)])
+    if kind == "apart":
+        ids = torch.randperm(real, generator=g)[:rows * top].view(rows, top)
+    elif kind == "same":
+        ids[:] = ids[0].clone()
+    elif kind == "none":
+        ids[::2, 0], ids[1::3, top - 1] = real, -1
+    ids, weights = ids.int().contiguous().cuda(), torch.rand(rows, top, generator=g).cuda()
+    x, dense = torch.randn(rows, D, generator=g).bfloat16().cuda(), torch.zeros(rows, real + 1, device="cuda")
+    gate_up, down = ((0.1 * torch.randn(*s, generator=g)).bfloat16().cuda() for s in ((2 * (real * I + shared), D), (D, real * I + shared)))
+
+    def run(at):
+        n = at.stop - at.start
+        out, h = torch.full((n + 1, D), 7.0, dtype=torch.bfloat16, device="cuda"), torch.empty(n * (top * I + shared), dtype=torch.bfloat16, device="cuda")
+        ops.chosen_experts(out, h, x[at].contiguous(), gate_up, down, ids[at].contiguous(), weights[at].contiguous(), dense[at].contiguous(), n, real, I, shared=shared)
+        assert (out[n] == 7).all()
+        return out[:n]
+    whole = run(slice(0, rows))
+    assert whole.abs().max() > 0
+    for r in range(rows):
+        assert torch.equal(run(slice(r, r + 1))[0], whole[r])
