@@ -1,11 +1,11 @@
 // bf16 matrix product for few rows (M <= 32) with K cut inside the workgroup:
 // C[M,N] = X[M,K] * W[N,K]^T (+ bias), or the gated activation of a gate||up
-// weight. One workgroup owns up to 32 weight rows (blocksplit_plan); its NW wavefronts take one K slice
+// weight. One workgroup owns up to 32 weight rows (blocksplit_plan; 64 in ordered_plan); its NW wavefronts take one K slice
 // each (operands straight from global memory into the MFMA registers, laid out so that the weight is read in whole lines, see
 // BsLanes), leave their fp32 sums in LDS, and the workgroup adds the slices in wavefront order and writes
 // the result. The sum is complete inside one launch: no partial sums in global
 // memory, no second kernel, no atomics, and the order of the additions is fixed.
-// What bounds it: the weight's way from memory (6.1 to 6.8 TB/s at 37888 x 3584 and more), and for small products the launch and one
+// What bounds it: the weight's way from memory (6.3 to 6.6 TB/s at 37888 x 3584 up to 8 rows), and for small products the launch and one
 // trip to memory: nothing is read ahead of the first weights, and what the epilogue reads is asked for behind them.
 //
 // Gated epilogue: the weight alternates gate and up rows (gate i at row 2i, its up at
@@ -44,6 +44,7 @@
 // NW = 8 wavefronts take a K slice each; 4 where that leaves a slice one instruction and the chip has other workgroups to run
 // (151936 x 896 at 4 rows 43 us, with eight 52). A wavefront with a single accumulator asks for two units a step (896 x 4864 at 8 rows 6.0 us, 6.8).
 // plan arguments NA, S, NW <= 0: this choice; NA: instructions' weight rows a wavefront holds (1, 2 or 4; 1 or 2 above 16 rows), S: units a step.
+// (More than 16 rows come here with plan arguments alone: see ordered_plan.)
 static BlockSplitPlan blocksplit_plan(int M, int N, int K, int NA, int S, int NW) {
   BlockSplitPlan p;
   const int cus = he_cus();

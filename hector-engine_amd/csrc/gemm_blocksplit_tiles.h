@@ -91,7 +91,7 @@ __device__ __forceinline__ void bs_store_pieces(uint16_t* base, int M, int m, in
 // lie in neighbouring lanes and are added at the end (bs_spread_sum). What it buys is the loads: an instruction's operand is
 // 16 >> SP weight rows of 64 << SP bytes each, whole lines from SP = 1 on with neighbouring lanes side by side, where 16 rows are half a
 // line each. Whole lines can be asked for past the caches (he_load16_once), which half lines cannot: the other half would be
-// fetched twice. 37888 x 3584 at 1 row 50.8 -> 42 us (6.4 TB/s), at 8 rows 52.5 -> 42, 3584 x 3584 at 1 row 9.6 -> 6.2.
+// fetched twice. Alone, weights from memory: 37888 x 3584 at 1 row 49.0 -> 42.9 us (6.3 TB/s), at 8 rows 51.2 -> 41.4, 3584 x 3584 at 1 row 7.7 -> 6.7.
 // SP = 0 keeps each sum in the order this product had before: a unit of 64 k is two instructions, whose lanes take the halves of 16
 // neighbouring k (loaded as whole lines all the same, see he_halves_to_rows), and the K slices and, by workgroup, the turn each
 // wavefront begins at are those it had. For 17 to 32 rows, whose rows of X are loaded in whole lines too (37888 x 3584 at 17, 24 and 32 rows 60.8, 67.3

@@ -221,13 +221,13 @@ __global__ __launch_bounds__(256, 2) void gemm_plain_mfma_kernel(
 // workgroup owns 16 weight rows and all activation rows (MT tiles of 16) and walks K with NW wavefronts, each
 // a segment of its own at a time: v_mfma_f32_16x16x4_f32 chains, whose sums go to LDS; after FLUSH rounds of
 // segments the workgroup adds them to its totals in segment order. So a weight of 3,584 rows still has 224 workgroups
-// with 16 wavefronts' loads in flight, and nothing goes through a workspace. (7B gate||up, 543 MB, by way of the caches: 1 row 97 us, 4 rows
-// 98, 16 rows 128, 64 rows 308; a lane a weight row on the vector ALU and a second kernel for the segment sums, up to 8
+// with 16 wavefronts' loads in flight, and nothing goes through a workspace. (7B gate||up, 543 MB: 1 row 88 us, 4 rows 86,
+// 16 rows 101, 64 rows 288; a lane a weight row on the vector ALU and a second kernel for the segment sums, up to 8
 // rows, 104 and 114; 64 x 64 tiles, which more rows went through, 657 at 16 rows and, for the down projection's 3,584
 // weight rows of 18,944, 2479 where this takes 53.) A wavefront fetches a stage of KS k
 // of its 16 weight rows (and activation rows) whole lines at a time, two stages ahead, into its own LDS region, the
 // 16-byte pieces of row r at their index xor r, from which the operand of lane (row, k mod 4) is read a float at a
-// time without bank conflicts; up to 64 rows the weights past the caches (ONCE: he_load16_once; at 4 rows the 543 MB 98 -> 87 us; more rows are two
+// time without bank conflicts; up to 64 rows the weights past the caches (ONCE: he_load16_once; at 4 rows the 543 MB 95 -> 86 us; more rows are two
 // workgroups' of the same weights, 2048 x 8192 at 65 rows 61.9 and 62.6 so). For weights of whole segments in aligned rows.
 #define GP_MROWS_MAX_M 64
 template <int MT, int NW, int KS, bool ONCE>

@@ -375,8 +375,9 @@ __global__ __launch_bounds__(GT_THREADS, 1) void gemm_tall_kernel(GtCase c) {
   F(256, 256, 3, 2) F(256, 224, 3, 2) F(256, 192, 3, 2) F(256, 160, 3, 3) F(128, 288, 3, 3) F(128, 256, 4, 3) F(128, 224, 4, 3) F(128, 160, 4, 4)
 
 // A product with a single row of tiles runs in one no taller than it needs, its weights read past the caches: F(tile's BM, BN, BM, NX, NW), the
-// lowest first. (37888 x 3584: 203 rows in 224 of 256 77 -> 67 us, 5 of them for the lower tile, 150 in 160 73 -> 64, 100 of 128 66 -> 61; two
-// rows of tiles past the caches 1.01 to 1.08 of the time without.)
+// lowest first. (Gate||up of 37888 x 3584 alone, weights from memory: 256 rows 76.7 -> 72.8 us, 203 in a tile of 224 75.3 -> 66, 150 in one of 160 71.6 -> 59,
+// 100 of 128 59.1 -> 54.4; two rows of tiles past the caches 1.01 to 1.08 of the time without.) The heights between 128 and 256 are for steps that run as
+// they are and for what is left of a long step behind turns of 8192 rows: steps of up to 512 rows that run as graphs are padded to powers of two.
 #define GT_ONE_TILES(F)                                                                                                      \
   F(256, 160, 160, 4, 4) F(256, 160, 192, 4, 3) F(256, 160, 224, 3, 3) F(256, 160, 256, 3, 3)                                \
   F(256, 224, 160, 3, 3) F(256, 224, 192, 3, 3) F(256, 224, 224, 3, 2) F(256, 224, 256, 3, 2)                                \

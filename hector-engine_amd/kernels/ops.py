@@ -330,8 +330,8 @@ def gemm_blocksplit(out, a, w, bias, M: int, gated: bool = False, plan=(0, 0, 0)
     used = (weights fp32 [M, count + 1 or more], count, size, along_k): the weight's rows, or its k, come in groups of `size`, and of the
     first `count` of them those are left out that no row has a weight for: their outputs are not written, or their products,
     with zeros in `a`, not added (up to 16 rows).
-    ordered: the order of sums this product had before its lanes read whole lines (up to 16 rows, no plan, no residual): for
-    results that reach a router over rows no norm has evened out."""
+    ordered: the order of sums this product had before its lanes read whole lines (up to 16 rows, no plan, no residual; above 16 rows there
+    is no other): for results that reach a router over rows no norm has evened out."""
     N, K = w.shape
     NO = N // 2 if gated else N
     _need(a, "a", torch.bfloat16)
