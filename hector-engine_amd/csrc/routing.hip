@@ -500,7 +500,10 @@ extern "C" int he_routed_act(void* out, const void* gate_up, const void* dense_f
 // a wavefront an output, the lanes along K with 16-byte loads, sums in fp32. Weights that one row of the step alone reads come past the caches, those
 // of an expert that several rows chose, and of the shared columns, by way of them: 8 rows of 4 choices among 64 experts of 1024 over 2048 and 2048 shared
 // columns, weights from memory, 80 us all by way of the caches, 86 all past them, 75 so; where all rows choose the same experts 47, 70 and 49. (One row of 4 choices
-// among 16 experts of 2048 over 2048 28.2 and 25.5.)
+// among 16 experts of 2048 over 2048 28.2 and 25.5.) Two rows' experts come past the caches whoever chose them: by way of them where both did, 2 rows of 4
+// among those 16 take 37.3 us instead of 39.6 when alone, but within a step the small kernels behind them find their code and arguments gone, 0.2 to 0.4 us
+// each, and a request of eight such steps takes 0.6 % longer (5284 and 5255 us). (Read past the caches by two rows, those of 3 rows and more are slower by more than that: 4 rows
+// of 2 among 16 of 1024 over 2048 20.6 us instead of 19.4.)
 __device__ __forceinline__ float dot8_bf16(const uint4& a, const uint4& b, float acc) {
   const uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -522,13 +525,13 @@ struct ChosenIds {
   int rows, n, mine;
   bool held;
   __device__ __forceinline__ ChosenIds(const int32_t* __restrict__ ids, int rows, int top)
-      : rows(rows), n(rows * top), mine(0), held(rows > 1 && n <= 64) {
+      : rows(rows), n(rows * top), mine(0), held(rows > 2 && n <= 64) {
     if (held) mine = ids[min((int)(threadIdx.x & 63), n - 1)];
   }
   __device__ __forceinline__ int at(const int32_t* __restrict__ ids, int i) const { return held ? __builtin_amdgcn_readlane(mine, i) : ids[i]; }
-  // whether one row alone chose expert e (of more than 64 ids: not said)
+  // whether one row alone chose expert e (of more than 64 ids: not said; of one or two rows: taken so)
   __device__ __forceinline__ bool alone(int e) const {
-    return rows == 1 || (held && __popcll(__ballot((int)(threadIdx.x & 63) < n && mine == e)) == 1);
+    return rows <= 2 || (held && __popcll(__ballot((int)(threadIdx.x & 63) < n && mine == e)) == 1);
   }
 };
 
